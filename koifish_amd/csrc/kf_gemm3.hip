@@ -202,9 +202,8 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_kerne
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int nbx = (a.M + C::BM - 1) / C::BM, nby = (a.n + C::BN - 1) / C::BN, nwg = nbx * nby;
     const int wg = g3_remap(blockIdx.x, nwg);
-    // (round 4: the other orientation -- row tiles slow, so that an XCD's L2 fetches all of x and an eighth of W when W is the larger operand -- measured on the 2047-token
-    // prompt: gate | up 41.5 us either way, Q | K | V 34.1 vs 32.5: not the fabric traffic that bounds these launches)
-    const int bx = wg % nbx, by = wg / nbx;
+    int bx, by;
+    g3_tile(wg, nbx, nby, bx, by);
     const int m0 = bx * C::BM, t0 = by * C::BN;
     f32x4 acc[C::MT][C::NT];
 #pragma unroll
@@ -212,7 +211,8 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_kerne
 #pragma unroll
         for (int j = 0; j < C::NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     g3_mainloop<AKM, BKM, BK, C>(a, m0, t0, 0, a.K / BK, acc, smem_raw, wid, lane);
-    g3_epilogue<AKM, C>(a, m0, t0, acc, wid, lane, smem_raw);
+    const int e = g3_opaque(tid);
+    g3_epilogue<AKM, C>(a, m0, t0, acc, e >> 6, e & 63, smem_raw);
 }
 
 // SPLIT-K forms for launches with fewer tiles than CUs (a weight gradient [OC, IC] is 49 .. 175 tiles, its contraction 8192 token rows long).  The pieces are cut so
@@ -231,7 +231,6 @@ struct G3SkArgs {
     int P, S, kp, R;
     uint32_t epoch; /* the value a raised flag holds in THIS launch (g3_sk_epoch): no memset between launches */
 };
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t g3_rsrc(const void* p, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000); }
 template <class C>
 __device__ __forceinline__ void g3_publish(const G3SkArgs& s, int slot, const f32x4 (&acc)[C::MT][C::NT], int tid) {
     const __amdgpu_buffer_rsrc_t rs = g3_rsrc(s.ws + (size_t)slot * (C::BM * C::BN), C::BM * C::BN * 4);
@@ -269,8 +268,8 @@ __device__ __forceinline__ void g3_collect(const G3SkArgs& s, int slot, f32x4 (&
 template <bool AKM, bool BKM, int BK, class C>
 __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_sk_kernel(const GemmArgs a, const G3SkArgs s) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int nbx = (a.M + C::BM - 1) / C::BM, nkt = a.K / BK;
+    const int tid = threadIdx.x;
+    const int nbx = (a.M + C::BM - 1) / C::BM, nby = (a.n + C::BN - 1) / C::BN, nkt = a.K / BK;
     // Roles by DISPATCH order: every non-owner piece of a tile has a smaller blockIdx than the tile's owner, and non-owners wait for nobody -- so when an owner runs, the
     // pieces it waits for have at least started, whatever else occupies the chip (a collective on another stream): the waits end, no residency assumption.
     // S >= 2: blockIdx group g = blockIdx / P holds piece S - 1 - g of every tile (the owners, piece 0, are the last group); S == 1: the helpers first, then the owners.
@@ -300,18 +299,22 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_sk_ke
             k0 = s.kp + o, k1 = k0 + len, owner = false, slot = (w - s.P) + tile; /* pieces in range order: one slot each, < P + helpers */
         }
         c0 = __builtin_amdgcn_readfirstlane(c0), c1 = __builtin_amdgcn_readfirstlane(c1), slot = __builtin_amdgcn_readfirstlane(slot);
-        const int bx = tile % nbx, by = tile / nbx, m0 = bx * C::BM, t0 = by * C::BN;
+        int bx, by;
+        g3_tile(tile, nbx, nby, bx, by);
+        const int m0 = bx * C::BM, t0 = by * C::BN;
         f32x4 acc[C::MT][C::NT];
 #pragma unroll
         for (int i = 0; i < C::MT; i++)
 #pragma unroll
             for (int j = 0; j < C::NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        g3_mainloop<AKM, BKM, BK, C>(a, m0, t0, k0, k1, acc, smem_raw, wid, lane);
+        const int b = g3_opaque(tid);
+        g3_mainloop<AKM, BKM, BK, C>(a, m0, t0, k0, k1, acc, smem_raw, b >> 6, b & 63);
+        const int e = g3_opaque(tid);
         if (!owner) {
-            g3_publish<C>(s, slot, acc, tid);
+            g3_publish<C>(s, slot, acc, e);
         } else {
-            for (int c = c0; c < c1; c++) g3_collect<C>(s, c, acc, tid);
-            g3_epilogue<AKM, C>(a, m0, t0, acc, wid, lane, smem_raw);
+            for (int c = c0; c < c1; c++) g3_collect<C>(s, c, acc, e);
+            g3_epilogue<AKM, C>(a, m0, t0, acc, e >> 6, e & 63, smem_raw);
         }
         it += helper ? k1 - k0 : 1;
     }

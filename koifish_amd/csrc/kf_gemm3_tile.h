@@ -26,22 +26,37 @@ using G3Tiny = G3Cfg<64, 64, 4>;
 // 192 x 256: a product whose 256 x 256 tiles number 160-255 (gate | up of a 0.6B model at 2047 tokens: 24 x 8 = 192 tiles on 256 CUs) becomes 32 x 8 = 256 tiles of 3/4 the work
 using G3Wide = G3Cfg<192, 256, 8>;
 
-// one operand tile (256 rows x 2 BK bytes) = BK / 2 wave instructions of 1 KiB; wave `wid` issues BK / 16 of them.  BK = 64: 8 rows per instruction, chunk c of row r
-// at position c ^ ((r >> 1) & 7); BK = 32: 16 rows per instruction (64-byte rows), chunk c at position c ^ ((r >> 2) & 3) -- either way a fragment read
-// (16 rows x one 16-byte chunk) touches all 64 banks once.
-template <int BK, int NI>
-__device__ __forceinline__ const uint16_t* g3_src(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int i, int wid, int lane) {
-    constexpr int CPR = BK / 8, RPI = 64 / CPR; /* chunks per row, rows per instruction */
-    const int j = wid * NI + i;
-    const int r = j * RPI + lane / CPR, p = lane % CPR, c = BK == 64 ? p ^ ((r >> 1) & 7) : p ^ ((r >> 2) & 3);
-    int gr = row0 + r;
-    gr = gr < nrows ? gr : nrows - 1; /* rows past the end re-read the last row: their outputs are not stored */
-    return src + (size_t)gr * ld + c * 8; /* + k0 per step */
+// x, which the compiler cannot trace: addresses formed from it are formed behind this point and take no registers in front of it
+__device__ __forceinline__ int g3_opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
-template <int BK>
+// One operand tile (256 rows x 128 bytes) = 32 wave instructions of 1 KiB; wave `wid` issues NI of them.  8 rows per instruction, chunk c of row r at position
+// c ^ ((r >> 1) & 7): a fragment read (16 rows x one 16-byte chunk) touches all 64 banks once.
+// An instruction's address is a scalar part (the tile's origin, the k-step, whole groups of rows) and a lane's part, which the swizzle makes one of two: even and odd
+// instructions.  Rows past the operand's end lie past the descriptor's end: the load writes zeros (their outputs are not stored).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t g3_rsrc(const void* p, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000); }
+constexpr uint32_t G3_ALL = 0x7FFFFFF0u; /* a descriptor's size that no lane part reaches */
+struct G3Src {
+    const unsigned char* base; /* uniform: the tile's origin at k-step 0 */
+    long long left, step, inst; /* bytes from there to the operand's end (< 0: no row past the end); bytes per k-step; bytes per instruction */
+    uint32_t lane[2];
+};
+template <int NI>
+__device__ __forceinline__ G3Src g3_src(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int wid, int lane) {
+    G3Src s;
+    s.base = reinterpret_cast<const unsigned char*>(src + ((size_t)row0 + (size_t)wid * NI * 8) * ld);
+    s.left = ((long long)nrows - row0 - (long long)wid * NI * 8) * ld * 2, s.step = G3_BK * 2, s.inst = ld * 16;
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+        const int r = (wid * NI + v) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        s.lane[v] = (uint32_t)(lane >> 3) * (uint32_t)(ld * 2) + c * 16;
+    }
+    return s;
+}
 __device__ __forceinline__ bf16x8 g3_frag(const unsigned char* tile, int row, int c) {
-    const int p = BK == 64 ? c ^ ((row >> 1) & 7) : c ^ ((row >> 2) & 3);
-    return *reinterpret_cast<const bf16x8*>(tile + row * (2 * BK) + (p << 4));
+    const int p = c ^ ((row >> 1) & 7);
+    return *reinterpret_cast<const bf16x8*>(tile + row * (2 * G3_BK) + (p << 4));
 }
 
 // the same tile from a K-MAJOR operand (src[k][row], `row` contiguous: an activation or a weight as it lies in memory when the contraction runs over its ROWS --
@@ -50,36 +65,40 @@ __device__ __forceinline__ bf16x8 g3_frag(const unsigned char* tile, int row, in
 // banks once (without the second term the two 16-lane halves meet in the same 32 banks: SQ_LDS_BANK_CONFLICT = 50 % of the LDS cycles, measured).
 // ROWS = the tile's rows (256 or 128): a k-row of the image is 2 ROWS bytes = CPK chunks of 16 bytes, one wave instruction covers 64 / CPK k-rows, wave `wid` issues
 // instructions NI wid .. NI wid + NI - 1 of the ROWS / 8
-template <int BK, int ROWS, int NI>
-__device__ __forceinline__ const uint16_t* g3_src_km(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int i, int wid, int lane) {
-    constexpr int CPK = ROWS / 8, KPI = 64 / CPK;
-    const int j = wid * NI + i;
-    const int kr = j * KPI + lane / CPK, p = lane % CPK, c = p ^ ((kr & 3) << 1) ^ (((kr >> 3) & 1) << 3);
-    int col = row0 + c * 8;
-    col = col + 8 <= nrows ? col : (nrows - 8 > 0 ? nrows - 8 : 0); /* chunks past the end re-read the last whole chunk: their outputs are not stored (rows % 8 == 0) */
-    return src + (size_t)kr * ld + col; /* + k0 * ld per step */
+template <int ROWS, int NI>
+__device__ __forceinline__ G3Src g3_src_km(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int wid, int lane) {
+    constexpr int CPK = ROWS / 8, KPI = 64 / CPK, UNIT = ROWS == 256 ? 1 : 2; /* 256: the swizzle tells even from odd instructions, 128: pairs of them */
+    static_assert((ROWS == 256 || ROWS == 128) && NI == 4, "two lane parts per wave");
+    G3Src s;
+    s.base = reinterpret_cast<const unsigned char*>(src + (size_t)wid * NI * KPI * ld);
+    s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = (long long)KPI * ld * 2; /* every k-row of the steps exists; chunks past a row's end are clamped here */
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+        const int kr = (wid * NI + v * UNIT) * KPI + lane / CPK, p = lane % CPK, c = p ^ ((kr & 3) << 1) ^ (((kr >> 3) & 1) << 3);
+        int col = row0 + c * 8;
+        col = col + 8 <= nrows ? col : (nrows - 8 > 0 ? nrows - 8 : 0); /* chunks past the end re-read the last whole chunk: their outputs are not stored (rows % 8 == 0) */
+        s.lane[v] = (uint32_t)(lane / CPK) * (uint32_t)(ld * 2) + col * 2;
+    }
+    return s;
 }
 // fragment (8 consecutive k of row `row`, k = kbase .. kbase + 7) of a k-major tile: two ds_read_b64_tr_b16, each a 4 (k) x 16 (rows) block transposed across 16 lanes
 // (lane i of the 16 receives D[(i >> 2) + 4 j][i & 3], scratch/dbg/ds_read_tr_probe.hip): lane l16 reads k-row kbase + (l16 >> 2), 8-byte piece l16 & 3 of the 16-row block
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+// The row block only flips three bits of a lane's offset (the swizzle's), so one register serves all blocks.
+__device__ __forceinline__ int g3_km_lane(int rows, int l16, int q4) { /* the lane's offset in a tile at row block 0, k 0 */
+    const int k = 8 * q4 + (l16 >> 2), swz = ((k & 3) << 1) ^ (((k >> 3) & 1) << 3);
+    return k * (2 * rows) + ((((l16 & 3) >> 1) ^ swz) << 4) + 8 * (l16 & 1);
+}
 template <int ROWS>
-__device__ __forceinline__ bf16x8 g3_frag_km(const unsigned char* tile, int rowblk16, int kbase, int l16) {
+__device__ __forceinline__ bf16x8 g3_frag_km(const unsigned char* tile, int km_lane, int rowblk16, int kk) {
     bf16x4 h[2];
+    const unsigned char* const at = tile + ((km_lane ^ ((rowblk16 & 7) << 5)) + ((rowblk16 >> 3) << 8));
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int k = kbase + 4 * t + (l16 >> 2);
-        const int byte_in_row = (rowblk16 * 16 + 4 * (l16 & 3)) * 2, c = byte_in_row >> 4, p = c ^ ((k & 3) << 1) ^ (((k >> 3) & 1) << 3);
-        h[t] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(tile + k * (2 * ROWS) + p * 16 + (byte_in_row & 8)));
-    }
+    for (int t = 0; t < 2; t++) h[t] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(at + (kk * 32 + 4 * t) * (2 * ROWS)));
     return bf16x8{h[0][0], h[0][1], h[0][2], h[0][3], h[1][0], h[1][1], h[1][2], h[1][3]};
 }
 
-// k-steps kt0 .. kt1 - 1 (of BK) of the output tile at (m0, t0) accumulated into acc (the caller zeroes it).  NST = 128 KiB / stage LDS buffers: the loads of step
-// kt + NST - 1 are issued while step kt is multiplied and drained with a COUNTED s_waitcnt vmcnt + one raw s_barrier per step (a __syncthreads() would drain the loads
-// in flight): BK = 64 -> 2 buffers; BK = 32 -> 4 buffers, three steps in flight (measured slower, see g3_go).  Also measured and dropped: the barrier moved into
-// the middle of the step's MFMA stream (the last 16 MFMAs of a step held back behind it, the first fragments of the next step read under them): 979 TFLOP/s against
-// 1000 on the forward shapes at 246 VGPRs, and the k-major forms spill; four waves of 128 x 128 outputs each (256 accumulator AGPRs, a third less LDS traffic per MFMA,
-// the vendor library's shape): the compiler fills all 512 registers and still spills inside the loop, 228 TFLOP/s -- that form needs a hand-scheduled loop.
+// k-steps kt0 .. kt1 - 1 (of BK) of the output tile at (m0, t0) accumulated into acc (the caller zeroes it).  See g3_mainloop below for the schedule.
 // `rows` (G3Rows: plain; G3Gather: row r of the token tile is row map[r] of x) says where the tile's token rows lie.
 // TILED: w is stored in MFMA tiles (kf_rb.h: 16 rows x 32 columns, piece (r, q) at number 16 q + r) instead of rows: a load
 // instruction moves one tile, contiguous in memory and in LDS, and a fragment read is lane-linear -- no swizzle on this operand.
@@ -93,93 +112,183 @@ struct G3GatherTiled {
     static constexpr bool GATHER = true, TILED = true;
     const int32_t* map; /* [BN] rows of x, every entry valid */
 };
+// The schedule.  A wave's outputs are four quadrants (row half x token half); the fragments of a quadrant are read from LDS under the MFMAs of the quadrant before it:
+//   quadrant (0,0): read token half 1          (0,1): read row half 1          -- step kt + 1 has landed, every wave holds its last fragments of step kt: ONE barrier --
+//   loads of step kt + 2 into the buffer of step kt          (1,1): read row half 0 of step kt + 1          (1,0): read token half 0 of step kt + 1
+// so neither the LDS reads (1.5 k of the 2 k cycles that a 256 x 256 x 64 step's MFMAs take) nor the barrier leave the matrix pipe without issued work, and a load has a
+// whole step to arrive.  The form before it read a step's fragments right behind the barrier, two at a time in front of the four MFMAs that use them, and waited there for the
+// loads it had issued one barrier earlier.  Same products in the same order: same bits.
 template <bool AKM, bool BKM, int BK, class C, class ROWS = G3Rows>
-__device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, int kt0, int kt1, f32x4 (&acc)[C::MT][C::NT], unsigned char* smem_raw, int wid, int lane, ROWS rows = ROWS()) {
-    static_assert(BK == G3_BK, "two k-halves of 32 per step");
-    constexpr int NST = 2, LPW = C::NIA + C::NIB; /* loads per wave and step */
-    const int wm = wid / C::WN, wn = wid % C::WN;
-    const uint16_t* const W = reinterpret_cast<const uint16_t*>(a.w);
-    auto bufA = [&](int b) { return smem_raw + (size_t)b * C::STAGE; };
-    auto bufB = [&](int b) { return smem_raw + (size_t)b * C::STAGE + C::BM * BK * 2; };
+__device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, int kt0, int kt1, f32x4 (&acc)[C::MT][C::NT], unsigned char* smem_raw, int wid_, int lane, ROWS rows = ROWS()) {
+    static_assert(BK == G3_BK && C::MT % 2 == 0 && C::NT % 2 == 0, "two k-halves of 32 per step, two halves of rows and of tokens per wave");
+    constexpr int LPW = C::NIA + C::NIB, HM = C::MT / 2, HN = C::NT / 2; /* loads per wave and step; MFMA blocks per half */
+    constexpr int BYTES_A = C::BM * BK * 2, BYTES_B = C::BN * BK * 2;
+    const int wid = __builtin_amdgcn_readfirstlane(wid_), wm = wid / C::WN, wn = wid % C::WN;
+    auto bufA = [&](int b) { return smem_raw + b * BYTES_A; }; /* an operand's two buffers side by side: both in reach of an LDS instruction's 16-bit offset */
+    auto bufB = [&](int b) { return smem_raw + 2 * BYTES_A + b * BYTES_B; };
     // AKM: W is [K][M] with row stride a.ldr (re-used field: the residual is not served by the k-major forms); BKM: x is [K][n] with row stride a.ldx.
-    // Per-lane source pointers are set up once; a step adds a uniform offset (a 64-bit multiply per load and step was a tenth of the loop's issue slots).
-    const uint16_t *pa[C::NIA], *pb[C::NIB];
+    G3Src sa, sb;
+    const uint16_t* gat[ROWS::GATHER ? C::NIB : 1];
+    const uint16_t* const W = reinterpret_cast<const uint16_t*>(a.w);
+    if constexpr (ROWS::TILED) {
+        static_assert(!AKM && C::NIA % 2 == 0, "an instruction is a tile, two tiles per row block and step");
+        const long long rb = (m0 >> 4) + wid * (C::NIA / 2), row = (long long)(a.K / 32) * 1024; /* row block of the wave's first tile; bytes of a row block */
+        sa.base = a.w + rb * row, sa.left = ((a.M + 15) / 16 - rb) * row, sa.step = 2048, sa.inst = row;
+        sa.lane[0] = lane * 16, sa.lane[1] = lane * 16;
+    } else if constexpr (AKM)
+        sa = g3_src_km<C::BM, C::NIA>(W, a.ldr, m0, a.M, wid, lane);
+    else
+        sa = g3_src<C::NIA>(W, a.K, m0, a.M, wid, lane);
+    if constexpr (ROWS::GATHER) {
+        static_assert(!BKM, "gathered rows: K-contiguous operands");
 #pragma unroll
-    for (int i = 0; i < C::NIA; i++) {
-        if constexpr (ROWS::TILED) {
-            static_assert(!AKM && BK == 64, "two tiles per row block and step");
-            const int j = wid * C::NIA + i, last = (a.M - 1) >> 4, rb = (m0 >> 4) + (j >> 1); /* tile (row block j / 2, k-half j % 2) */
-            pa[i] = W + ((size_t)(rb < last ? rb : last) * (a.K / 32) + (j & 1)) * 512 + lane * 8;
-            continue;
-        }
-        pa[i] = AKM ? g3_src_km<BK, C::BM, C::NIA>(W, a.ldr, m0, a.M, i, wid, lane) : g3_src<BK, C::NIA>(W, a.K, m0, a.M, i, wid, lane);
-    }
-#pragma unroll
-    for (int i = 0; i < C::NIB; i++) {
-        if constexpr (ROWS::GATHER) {
-            static_assert(!BKM && BK == 64, "gathered rows: K-contiguous operands");
+        for (int i = 0; i < C::NIB; i++) {
             const int r = (wid * C::NIB + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-            pb[i] = a.x + (size_t)rows.map[r] * a.ldx + c * 8;
-        } else {
-            pb[i] = BKM ? g3_src_km<BK, C::BN, C::NIB>(a.x, a.ldx, t0, a.n, i, wid, lane) : g3_src<BK, C::NIB>(a.x, a.ldx, t0, a.n, i, wid, lane);
+            gat[i] = a.x + (size_t)rows.map[r] * a.ldx + c * 8;
         }
-    }
-    const long long stepA = ROWS::TILED ? 1024 : (AKM ? (long long)BK * a.ldr : BK), stepB = BKM ? (long long)BK * a.ldx : BK;
-    auto stage = [&](int kt, int b) {
-        const long long oa = stepA * kt, ob = stepB * kt;
+    } else if constexpr (BKM)
+        sb = g3_src_km<C::BN, C::NIB>(a.x, a.ldx, t0, a.n, wid, lane);
+    else
+        sb = g3_src<C::NIB>(a.x, a.ldx, t0, a.n, wid, lane);
+    // K-contiguous operands: one descriptor per instruction for the whole tile, a step is the scalar offset (a row past the end lies past the descriptor's end at every
+    // step, whether or not the check counts that offset; a row inside never does).  k-major: every step has a base of its own, of any size.
+    // Past the last step the descriptors are empty: the load moves nothing and puts zeros where nobody reads, and the steps need no branch.
+    uint32_t restA[C::NIA], restB[C::NIB];
+    auto rest = [](long long left) { return (uint32_t)(left < 0 ? 0 : (left > 0xFFFFFFFFll ? 0xFFFFFFFFll : left)); };
+    auto atA = [&](int i) { return ROWS::TILED ? sa.inst * (i >> 1) + (i & 1) * 1024 : sa.inst * i; };
 #pragma unroll
-        for (int i = 0; i < C::NIA; i++)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pa[i] + oa),
-                                             (__attribute__((address_space(3))) void*)(bufA(b) + (wid * C::NIA + i) * 1024), 16, 0, 0);
+    for (int i = 0; i < C::NIA; i++) restA[i] = AKM ? G3_ALL : rest(sa.left - atA(i));
 #pragma unroll
-        for (int i = 0; i < C::NIB; i++)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pb[i] + ob),
-                                             (__attribute__((address_space(3))) void*)(bufB(b) + (wid * C::NIB + i) * 1024), 16, 0, 0);
+    for (int i = 0; i < C::NIB; i++) restB[i] = BKM || ROWS::GATHER ? G3_ALL : rest(sb.left - sb.inst * i);
+    [[maybe_unused]] const unsigned char *nextA = sa.base + (AKM ? sa.step * kt0 : 0), *nextB = BKM ? sb.base + sb.step * kt0 : nullptr; /* k-major: the base of the step staged next */
+    auto stageA = [&](int kt, int b) {
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int i = 0; i < C::NIA; i++) {
+            const auto to = (__attribute__((address_space(3))) void*)(bufA(b) + (wid * C::NIA + i) * 1024);
+            const uint32_t n = kt < kt1 ? restA[i] : 0;
+            if constexpr (AKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextA + sa.inst * i, n), to, 16, sa.lane[C::BM == 128 ? i >> 1 : i & 1], 0, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sa.base + atA(i), n), to, 16, sa.lane[ROWS::TILED ? 0 : i & 1], (int)sa.step * kt, 0, 0);
+        }
+        if constexpr (AKM) nextA += sa.step;
+#endif
     };
+    auto stageB = [&](int kt, int b) {
+#ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
-    for (int st = 0; st < NST - 1; st++)
-        if (kt0 + st < kt1) stage(kt0 + st, st);
-    const int r16 = lane & 15, q4 = lane >> 4;
-    // the steps are unrolled by the NST buffers so that every LDS address of a step is base + an immediate
-    auto step = [&](int kt, auto cur_c) {
+        for (int i = 0; i < C::NIB; i++) {
+            const auto to = (__attribute__((address_space(3))) void*)(bufB(b) + (wid * C::NIB + i) * 1024);
+            const uint32_t n = kt < kt1 ? restB[i] : 0;
+            if constexpr (ROWS::GATHER) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gat[i] + (size_t)(kt < kt1 ? kt : kt1 - 1) * BK), to, 16, 0, 0); /* (past the end: the last step again) */
+            else if constexpr (BKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextB + sb.inst * i, n), to, 16, sb.lane[C::BN == 128 ? i >> 1 : i & 1], 0, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sb.base + sb.inst * i, n), to, 16, sb.lane[i & 1], (int)sb.step * kt, 0, 0);
+        }
+        if constexpr (BKM) nextB += sb.step;
+#endif
+    };
+    auto stage = [&](int kt, int b) { stageA(kt, b), stageB(kt, b); };
+    const int r16 = lane & 15, q4 = lane >> 4, kmA = g3_km_lane(C::BM, r16, q4), kmB = g3_km_lane(C::BN, r16, q4);
+    auto readA = [&](int b, int half, bf16x8 (&f)[HM][2]) {
+        const int km = AKM ? g3_opaque(kmA) : 0;
+#pragma unroll
+        for (int mh = 0; mh < HM; mh++)
+#pragma unroll
+            for (int kk = 0; kk < 2; kk++) {
+                const int mt = half * HM + mh;
+                if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(bufA(b) + ((wm * C::MT + mt) * 2 + kk) * 1024 + lane * 16);
+                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(bufA(b), km, wm * C::MT + mt, kk);
+                else f[mh][kk] = g3_frag(bufA(b), wm * (16 * C::MT) + mt * 16 + r16, kk * 4 + q4);
+            }
+    };
+    auto readB = [&](int b, int half, bf16x8 (&f)[HN][2]) {
+        const int km = BKM ? g3_opaque(kmB) : 0;
+#pragma unroll
+        for (int nh = 0; nh < HN; nh++)
+#pragma unroll
+            for (int kk = 0; kk < 2; kk++) {
+                const int nt = half * HN + nh;
+                if constexpr (BKM) f[nh][kk] = g3_frag_km<C::BN>(bufB(b), km, wn * C::NT + nt, kk);
+                else f[nh][kk] = g3_frag(bufB(b), wn * (16 * C::NT) + nt * 16 + r16, kk * 4 + q4);
+            }
+    };
+    auto mul = [&](int mh0, int nh0, const bf16x8 (&fa)[HM][2], const bf16x8 (&fb)[HN][2]) {
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+            for (int i = 0; i < HM; i++)
+#pragma unroll
+                for (int j = 0; j < HN; j++)
+                    acc[mh0 * HM + i][nh0 * HN + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][kk], fb[j][kk], acc[mh0 * HM + i][nh0 * HN + j], 0, 0, 0);
+    };
+    // a quadrant's issue order: its LDS reads and its loads one by one among its first MFMAs, the rest of the MFMAs behind them
+    auto order = [&](auto n_reads, auto n_loads) {
+        constexpr int N = decltype(n_reads)::value, V = decltype(n_loads)::value, M = HM * HN * 2, P = N < M ? N : M, Q = V < M - 1 ? V : M - 1, X = P > Q ? P : Q;
+#pragma unroll
+        for (int i = 0; i < X; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (i < P) __builtin_amdgcn_sched_group_barrier(0x100, N / P, 0);
+            if (i < Q) __builtin_amdgcn_sched_group_barrier(0x010, V / (Q ? Q : 1), 0);
+        }
+        if (M > X) __builtin_amdgcn_sched_group_barrier(0x008, M - X, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr std::integral_constant<int, HM * 2 * (AKM ? 2 : 1)> ra{};
+    constexpr std::integral_constant<int, HN * 2 * (BKM ? 2 : 1)> rb{};
+    bf16x8 a0[HM][2], a1[HM][2], b0[HN][2], b1[HN][2];
+    if (kt0 >= kt1) return;
+    stage(kt0, 0), stage(kt0 + 1, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory"); /* no read moves up */
+    readA(0, 0, a0), readB(0, 0, b0);
+    // the steps are unrolled by the two buffers (every LDS address of a step is base + an immediate); the two token halves' registers swap roles with them.  Behind the last
+    // step the reads of "step kt + 1" take what lies in the other buffer: never used
+    constexpr std::integral_constant<int, 0> none{};
+    constexpr std::integral_constant<int, C::NIA> la{};
+    constexpr std::integral_constant<int, C::NIB> lb{};
+    auto step = [&](int kt, auto cur_c, bf16x8 (&bx)[HN][2], bf16x8 (&by)[HN][2]) {
         constexpr int cur = decltype(cur_c)::value;
-        const int left = kt1 - 1 - kt; /* steps issued after kt that may stay in flight */
-        if (NST >= 4 && left >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
-        else if (NST >= 3 && left >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier(); /* step kt has landed for every wave, and every wave is done reading the buffer of step kt - 1: the next loads overwrite that one */
-        if (kt + NST - 1 < kt1) stage(kt + NST - 1, (cur + NST - 1) % NST);
-#pragma unroll
-        for (int kk = 0; kk < BK / 32; kk++) {
-            bf16x8 af[C::MT], bfr[C::NT];
-#pragma unroll
-            for (int nt = 0; nt < C::NT; nt++) {
-                if constexpr (BKM) bfr[nt] = g3_frag_km<C::BN>(bufB(cur), wn * C::NT + nt, kk * 32 + 8 * q4, r16);
-                else bfr[nt] = g3_frag<BK>(bufB(cur), wn * (16 * C::NT) + nt * 16 + r16, kk * 4 + q4);
-            }
-#pragma unroll
-            for (int mt = 0; mt < C::MT; mt++) {
-                if constexpr (ROWS::TILED) af[mt] = *reinterpret_cast<const bf16x8*>(bufA(cur) + ((wm * C::MT + mt) * 2 + kk) * 1024 + lane * 16);
-                else if constexpr (AKM) af[mt] = g3_frag_km<C::BM>(bufA(cur), wm * C::MT + mt, kk * 32 + 8 * q4, r16);
-                else af[mt] = g3_frag<BK>(bufA(cur), wm * (16 * C::MT) + mt * 16 + r16, kk * 4 + q4);
-            }
-#pragma unroll
-            for (int mt = 0; mt < C::MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < C::NT; nt++) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mt], bfr[nt], acc[mt][nt], 0, 0, 0);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        readB(cur, 1, by);
+        mul(0, 0, a0, bx);
+        order(rb, none);
+        readA(cur, 1, a1);
+        mul(0, 1, a0, by);
+        order(ra, none);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier(); /* step kt + 1 has landed for every wave, and every wave has read all of step kt: its buffer may be filled again */
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        stageA(kt + 2, cur);
+        readA(cur ^ 1, 0, a0);
+        mul(1, 1, a1, by);
+        order(ra, la);
+        stageB(kt + 2, cur);
+        readB(cur ^ 1, 0, by);
+        mul(1, 0, a1, bx);
+        order(rb, lb);
     };
-    for (int kt = kt0; kt < kt1; kt += NST) {
-        step(kt, std::integral_constant<int, 0>{});
-        if (kt + 1 < kt1) step(kt + 1, std::integral_constant<int, 1>{});
+    for (int kt = kt0; kt < kt1; kt += 2) {
+        step(kt, std::integral_constant<int, 0>{}, b0, b1);
+        if (kt + 1 < kt1) step(kt + 1, std::integral_constant<int, 1>{}, b1, b0);
     }
-    __builtin_amdgcn_s_barrier(); /* a following segment's first loads must not overtake the last reads */
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier(); /* the buffers are free: for a following segment's first loads, for an epilogue's exchange */
+    asm volatile("" ::: "memory");
 }
 
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {
     const int q = nwg / 8, rr = nwg % 8, xcd = orig % 8;
     return (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + orig / 8;
+}
+// tile number -> (row tile, token tile): bands of at most 8 row tiles, token tile after token tile inside a band, so that the 32 tiles an XCD multiplies at a time are a block of about
+// 8 x 4.  What a step of those 32 brings into that XCD's L2 is 12 operand tiles; numbered row tile by row tile through all of M it was 33, and the link of an XCD (1.1 TB/s) was what the main loop
+// waited for: 8192 x 8192 x 8192 with its MFMAs left out took as long as with them.
+__device__ __forceinline__ void g3_tile(int t, int nbx, int nby, int& bx, int& by) {
+    const int nb = (nbx + 7) / 8, h = nbx / nb, tall = nbx % nb, cut = tall * (h + 1) * nby; /* the first `tall` bands have h + 1 row tiles, the others h */
+    const bool up = t < cut;
+    const int r = up ? t : t - cut, w = up ? h + 1 : h, band = r / (w * nby), in = r - band * (w * nby);
+    by = in / w, bx = (up ? band * (h + 1) : tall * (h + 1) + band * h) + in % w;
 }
 }  // namespace kf

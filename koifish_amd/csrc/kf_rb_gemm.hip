@@ -20,7 +20,9 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     __shared__ int32_t s_src[EXPERTS ? C::BN : 1], s_dst[EXPERTS ? C::BN : 1];
     const kf_rb_product& p = q.p;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int nbx = (p.m + C::BM - 1) / C::BM, wg = g3_remap(blockIdx.x, gridDim.x), bx = wg % nbx, by = wg / nbx;
+    const int nbx = (p.m + C::BM - 1) / C::BM;
+    int bx, by;
+    g3_tile(g3_remap(blockIdx.x, gridDim.x), nbx, (int)gridDim.x / nbx, bx, by);
     const int m0 = bx * C::BM, t0 = by * C::BN;
     GemmArgs a; /* what the main loop reads */
     a.w = reinterpret_cast<const unsigned char*>(p.w), a.M = p.m, a.K = p.k, a.x = reinterpret_cast<const uint16_t*>(p.x), a.ldx = p.ldx, a.n = p.n, a.ldr = 0;
