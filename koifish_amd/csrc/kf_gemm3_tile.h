@@ -189,7 +189,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     auto stage = [&](int kt, int b) { stageA(kt, b), stageB(kt, b); };
     const int r16 = lane & 15, q4 = lane >> 4, kmA = g3_km_lane(C::BM, r16, q4), kmB = g3_km_lane(C::BN, r16, q4);
     auto readA = [&](int b, int half, bf16x8 (&f)[HM][2]) {
-        const int km = AKM ? g3_opaque(kmA) : 0;
+        const int km = AKM && HM > 2 ? g3_opaque(kmA) : kmA; /* eight blocks' addresses kept would not leave room for the fragments */
 #pragma unroll
         for (int mh = 0; mh < HM; mh++)
 #pragma unroll
@@ -201,7 +201,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
             }
     };
     auto readB = [&](int b, int half, bf16x8 (&f)[HN][2]) {
-        const int km = BKM ? g3_opaque(kmB) : 0;
+        const int km = BKM && C::BN > 128 ? g3_opaque(kmB) : kmB;
 #pragma unroll
         for (int nh = 0; nh < HN; nh++)
 #pragma unroll
