@@ -360,3 +360,25 @@ def test_resident_dequantised_copies_give_the_scratch_routes_results(ctx, O, t):
     finally:
         ctx.sync()
         L.check(ctx.hip.kf_set_dequant_arena(ctx.h, None, 0), "kf_set_dequant_arena")
+
+
+@pytest.mark.parametrize("M,K,n", [(1024, 2048, 320), (1024, 2048, 512), (1024, 3072, 384), (1024, 3072, 1024), (2048, 2048, 520)])
+def test_resident_copies_with_a_lent_workspace_sum_every_k_piece(ctx, M, K, n):
+    """short token batches on resident copies go in k-pieces when a workspace is lent (64 x 64, 64 x 128 and 128 x 128 tiles): every piece reaches the output.  fp32 sums of K products of the same bf16
+    values in another order and one bf16 rounding: 2^-8 of the result's scale"""
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4)
+    ref_w, x, d = ctx.dequant(w).float(), torch.randn(n, K, device=ctx.device).bfloat16(), w.desc()
+    arena = torch.zeros(M * K * 2 + 4096, dtype=torch.uint8, device=ctx.device)
+    ws = torch.full((ctx.hip.kf_resident_scratch_bytes(),), 0x5A, dtype=torch.uint8, device=ctx.device)
+    ref = x.float() @ ref_w.t()
+    try:
+        assert ctx.hip.kf_set_dequant_arena(ctx.h, C.c_void_p(arena.data_ptr()), C.c_size_t(arena.numel())) == 0
+        assert ctx.hip.kf_set_scratch(ctx.h, C.c_void_p(ws.data_ptr()), C.c_size_t(ws.numel())) == 0
+        for _ in range(3):
+            y = torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
+            assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
+            assert float((y.float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
