@@ -158,6 +158,13 @@ int kf_set_scratch(kf_ctx* ctx, void* scratch, size_t bytes);
 int kf_set_dequant_arena(kf_ctx* ctx, void* arena, size_t bytes);
 size_t kf_dequant_arena_used(kf_ctx* ctx);
 size_t kf_resident_scratch_bytes(void); /* a kf_set_scratch workspace of at least this size lets kf_linear's resident-copy route cut short token batches into k-pieces */
+/* bf16 copies of ONE layer's seven matrices for the token-batch calls that follow: kf_layer_copies dequantises them with one launch into the front of the kf_set_scratch workspace
+ * (kf_layer_copies_bytes: how large it has to be, 0: not for this layer or batch) when they are 4-bit in groups of 128, the batch has >= 320 rows and no arena is lent; the routes of
+ * kf_linear, kf_qkv_rope_batch / _seqs, kf_linear_multi and kf_gateup_swiglu_batch then multiply the copies.  Returns 1 when it does nothing.  The copies hold until kf_layer_copies_end,
+ * the next kf_layer_copies or kf_set_scratch; the caller does not change these weights in between. */
+size_t kf_layer_copies_bytes(const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok);
+int kf_layer_copies(kf_ctx* ctx, const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok);
+int kf_layer_copies_end(kf_ctx* ctx);
 int kf_linear(kf_ctx* ctx, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const kf_bf16* bias, int nTok, float alpha, float beta,
               uint32_t epilogue, const kf_bf16* residual);
 

@@ -101,10 +101,15 @@ int kf_init(int device, void* stream, kf_ctx** out) {
     HIPCHK(hipMalloc(&c->amax_val, sizeof(float) * kf::KF_MAX_ARGMAX_PARTIALS));
     HIPCHK(hipMalloc(&c->amax_idx, sizeof(int) * kf::KF_MAX_ARGMAX_PARTIALS));
     c->scratch = nullptr, c->scratch_bytes = 0;
-    c->arena = nullptr, c->arena_bytes = c->arena_used = 0;
+    c->arena = nullptr, c->arena_bytes = c->arena_used = 0, c->call_used = 0;
     c->canonical = 1;
     *out = c;
     return KF_OK;
+}
+// `bytes` of a copy are about to be written at dst in the scratch: where they reach the split-K flags, the next launch that waits for these clears them first
+static void scratch_written(kf_ctx* c, const void* dst, size_t bytes) {
+    const char* const slots = (const char*)c->scratch_end(kf::gemm3_sk_ws_bytes());
+    if (slots && (const char*)dst >= (const char*)c->scratch && (const char*)dst < (const char*)c->scratch + c->scratch_bytes && (const char*)dst + bytes > slots) kf::gemm3_sk_forget((void*)slots);
 }
 // bf16 view of a weight: the data itself (bf16 storage) or its dequantisation into the caller's scratch (kf_set_scratch)
 static int lib_weight_bf16(kf_ctx* c, const kf_weight* w, const uint16_t** out) {
@@ -113,10 +118,11 @@ static int lib_weight_bf16(kf_ctx* c, const kf_weight* w, const uint16_t** out) 
         return KF_OK;
     }
     const size_t need = (size_t)w->ne0 * w->ne1 * 2;
-    if (need > c->scratch_bytes || !c->scratch)
-        return fail(KF_INVALID_ARGS, "kf_linear: this weight needs %zu bytes of scratch (kf_linear_scratch_bytes), kf_set_scratch gave %zu", need, c->scratch_bytes);
-    const int r = kf::dequant_launch(c->stream, w, (uint16_t*)c->scratch);
-    *out = (const uint16_t*)c->scratch;
+    if (need > c->scratch_left() || !c->scratch)
+        return fail(KF_INVALID_ARGS, "kf_linear: this weight needs %zu bytes of scratch (kf_linear_scratch_bytes), kf_set_scratch gave %zu", need, c->scratch_left());
+    scratch_written(c, c->scratch_tail(), need);
+    const int r = kf::dequant_launch(c->stream, w, (uint16_t*)c->scratch_tail());
+    *out = (const uint16_t*)c->scratch_tail();
     return r;
 }
 static size_t up256z(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -126,6 +132,14 @@ static int deq_copies(kf_ctx* c, int n_w, const kf_weight* const* w, int form, c
     size_t need = 0;
     for (int i = 0; i < n_w; i++) need += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
     if (resident) *resident = false;
+    for (const kf_ctx::DeqCopy& e : c->call) {
+        bool same = e.form == form;
+        for (int i = 0; i < 3; i++) same = same && e.key[i] == (i < n_w ? w[i]->data : nullptr);
+        if (same) {
+            *out = (const uint16_t*)((const char*)c->scratch + e.off);
+            return KF_OK;
+        }
+    }
     if (c->arena) {
         for (const kf_ctx::DeqCopy& e : c->copies) {
             bool same = e.form == form;
@@ -138,9 +152,10 @@ static int deq_copies(kf_ctx* c, int n_w, const kf_weight* const* w, int form, c
         }
     }
     const bool keep = c->arena && !c->capturing && c->arena_used + need <= c->arena_bytes; /* a captured launch would replay the fill with every replay: those use the scratch */
-    char* dst = keep ? (char*)c->arena + c->arena_used : (char*)c->scratch;
-    if (!keep && (arena_only || !c->scratch || c->scratch_bytes < need)) return 1;
+    char* dst = keep ? (char*)c->arena + c->arena_used : c->scratch_tail();
+    if (!keep && (arena_only || !c->scratch || c->scratch_left() < need)) return 1;
     size_t off = 0;
+    if (!keep) scratch_written(c, dst, need);
     for (int i = 0; i < n_w; i++) {
         const int r = form == DEQ_ILV ? kf::dequant_launch(c->stream, w[i], (uint16_t*)dst, n_w, i) : kf::dequant_launch(c->stream, w[i], (uint16_t*)(dst + off));
         if (r != KF_OK) return r < 0 ? r : KF_HIP_CHECK;
@@ -331,7 +346,11 @@ int kf_quantize(kf_ctx* c, const kf_weight* w, const kf_bf16* src, int symmetric
 
 static void init_args(kf_ctx* c, kf::GemvLaunch& L) { memset(&L, 0, sizeof(L)); L.args.alpha = 1.0f; L.canon = c->canonical; }
 
-static const int KF_DEQ_GEMM_MIN = 2048; /* token rows from which a quantised weight is dequantised once and multiplied by the bf16 tile kernel (when scratch was handed over) */
+// token rows from which a layer's seven matrices are dequantised by one launch (kf_layer_copies) for the bf16 tile kernels.  One product in registers | on a copy that is there, us: 1024 x 2048 at 256
+// tokens 9.8 | 10.8, at 320 16.3 | 10.8, at 2047 30.5 | 16.8;  1024 x 3072 at 256 12.6 | 14.3, at 320 20.5 | 19.0, at 2047 43.9 | 30.2;  4096 x 1024 at 320 17.5 | 10.0;  6144 x 1024 at 320 20.5 | 12.4;
+// the launch itself 10 us for those.  A launch per matrix gives that back: 2047 tokens 1024 x 2048 30.5 | 26.8, 512 tokens 16.5 | 22.5.
+static const int KF_LAYER_COPIES_MIN = 320;
+static const int KF_DEQ_GEMM_MIN = 2048; /* token rows from which a quantised weight is dequantised by a launch of its own and multiplied by the bf16 tile kernel (when scratch was handed over) */
 size_t kf_linear_scratch_bytes(const kf_weight* w, int nTok) {
     if (!w || nTok < 1) return 0;
     if (w->qzeros) return kf::awq_scratch_bytes(w);
@@ -356,12 +375,14 @@ int kf_set_dequant_arena(kf_ctx* c, void* arena, size_t bytes) {
     return KF_OK;
 }
 size_t kf_dequant_arena_used(kf_ctx* c) { return c ? c->arena_used : 0; }
-size_t kf_resident_scratch_bytes(void) { return kf::gemm3_sk_ws_bytes(); }
+size_t kf_resident_scratch_bytes(void) { return kf::gemm3_sk_ws_bytes() + 512; }
 int kf_set_scratch(kf_ctx* c, void* scratch, size_t bytes) {
     CHKCTX(c);
     if (scratch && !al16(scratch)) return fail(KF_BLAS_UNALIGN, "kf_set_scratch: unaligned");
     if (c->capturing) return fail(KF_INVALID_ARGS, "kf_set_scratch: not while capturing (captured launches hold the old pointer)");
     c->scratch = scratch, c->scratch_bytes = scratch ? bytes : 0;
+    c->call.clear(), c->call_used = 0;
+    if (void* slots = c->scratch_end(kf::gemm3_sk_ws_bytes())) kf::gemm3_sk_forget(slots); /* whatever lay there before */
     return KF_OK;
 }
 
@@ -378,11 +399,12 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
     // up when the shape is covered (K a multiple of 128, 16-byte aligned rows), otherwise one mat-vec launch per token row.
     if (w->qzeros) { /* AutoAWQ layout: its own transposed mat-vec */
         const size_t need = kf::awq_scratch_bytes(w);
-        if (need > c->scratch_bytes || !c->scratch)
-            return fail(KF_INVALID_ARGS, "kf_linear: the AWQ mat-vec needs %zu bytes of scratch (kf_linear_scratch_bytes), kf_set_scratch gave %zu", need, c->scratch_bytes);
+        if (need > c->scratch_left() || !c->scratch)
+            return fail(KF_INVALID_ARGS, "kf_linear: the AWQ mat-vec needs %zu bytes of scratch (kf_linear_scratch_bytes), kf_set_scratch gave %zu", need, c->scratch_left());
+        scratch_written(c, c->scratch_tail(), need);
         for (int t = 0; t < nTok; t++) {
             int rc = kf::awq_linear_launch(c->stream, w, x + (size_t)t * w->ne1, y + (size_t)t * w->ne0, bias, alpha, beta,
-                                           (epilogue & KF_EPI_RESIDUAL) ? residual + (size_t)t * w->ne0 : nullptr, (float*)c->scratch);
+                                           (epilogue & KF_EPI_RESIDUAL) ? residual + (size_t)t * w->ne0 : nullptr, (float*)c->scratch_tail());
             if (rc != KF_OK) return fail(rc, "kf_linear (AWQ) failed with %d", rc);
         }
         return KF_OK;
@@ -398,6 +420,16 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         wb.data = Wd, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
         return kf_linear(c, &wb, x, y, bias, nTok, alpha, beta, epilogue, residual);
     }
+    for (const kf_ctx::DeqCopy& e : c->call) {
+        if (e.form != DEQ_STACK || e.key[0] != w->data || e.key[1] || nTok < KF_LAYER_COPIES_MIN) continue; /* a copy of this matrix alone (kf_layer_copies) */
+        kf_weight wb;
+        memset(&wb, 0, sizeof(wb));
+        wb.data = (char*)c->scratch + e.off, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
+        const size_t slots = kf::gemm3_sk_ws_bytes(); /* split-K slots behind the copies */
+        const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, c->scratch_end(slots), slots);
+        if (rc < 0) return fail(rc, "kf_linear (bf16 tile GEMM on the layer's copy) failed with %d", rc);
+        if (rc == KF_OK) return KF_OK;
+    }
     if (c->arena && nTok >= kf::g_knobs.resident_min && w->type != KF_BF16 && w->quant == KF_QUANT_GROUP && w->ne0 >= 128 && (w->ne1 % 64) == 0) {
         // a resident copy (kf_set_dequant_arena): nothing to dequantise -- the bf16 tile kernels of kf_gemm3.hip from g_knobs.resident_min token rows (the 1024-row o_proj / down_proj of a
         // long prompt as 256 tiles of 64 x 128 or 64 x 64)
@@ -409,22 +441,22 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
             kf_weight wb;
             memset(&wb, 0, sizeof(wb));
             wb.data = W, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
-            const bool lend = c->scratch && c->scratch_bytes >= kf::gemm3_sk_ws_bytes() && al16(c->scratch); /* the scratch holds no copy on this route: split-K slots */
-            const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, lend ? c->scratch : nullptr,
-                                           lend ? c->scratch_bytes : 0);
+            const size_t slots = kf::gemm3_sk_ws_bytes(); /* the scratch holds no copy on this route: split-K slots */
+            const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, c->scratch_end(slots), slots);
             if (rc < 0) return fail(rc, "kf_linear (bf16 tile GEMM on the resident copy) failed with %d", rc);
             if (rc == KF_OK) return KF_OK;
         }
     }
     if (nTok >= KF_DEQ_GEMM_MIN && w->type != KF_BF16 && w->quant == KF_QUANT_GROUP && w->ne0 >= 256 && (w->ne1 % 64) == 0 && c->scratch &&
-        c->scratch_bytes >= (size_t)w->ne0 * w->ne1 * 2 &&
+        c->scratch_left() >= (size_t)w->ne0 * w->ne1 * 2 &&
         ((long)((w->ne0 + 255) / 256) * ((nTok + 255) / 256) >= 128 || (long)((w->ne0 + 127) / 128) * ((nTok + 127) / 128) >= 256 /* the 128 x 128 form: M 1024 from 4096 rows */)) {
         // GetDataX into the caller's scratch, then the 256 x 256 bf16 tile kernel: the reference's own order, on our own kernels
-        r = kf::dequant_launch(c->stream, w, (uint16_t*)c->scratch);
+        scratch_written(c, c->scratch_tail(), (size_t)w->ne0 * w->ne1 * 2);
+        r = kf::dequant_launch(c->stream, w, (uint16_t*)c->scratch_tail());
         if (r != KF_OK) return fail(r, "kf_linear (dequantise for the large-batch tile kernel) failed with %d", r);
         kf_weight wb;
         memset(&wb, 0, sizeof(wb));
-        wb.data = c->scratch, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
+        wb.data = c->scratch_tail(), wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
         const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0);
         if (rc < 0) return fail(rc, "kf_linear (large-batch bf16 tile GEMM) failed with %d", rc);
         if (rc == KF_OK) return KF_OK;
@@ -434,7 +466,7 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         if (rc < 0) return fail(rc, "kf_linear (token-batch GEMM) failed with %d", rc);
         if (rc == KF_OK) return KF_OK;
     }
-    if (nTok >= gemm_min && w->quant == KF_QUANT_ROW_LUT && c->scratch && c->scratch_bytes >= (size_t)w->ne0 * w->ne1 * 2) {
+    if (nTok >= gemm_min && w->quant == KF_QUANT_ROW_LUT && c->scratch && c->scratch_left() >= (size_t)w->ne0 * w->ne1 * 2) {
         // row-codebook storage whose shape the in-register-unpack tile kernels do not cover: the reference's own order -- GetDataX into the scratch,
         // then the bf16 product on the dequantised copy.  Mat-vecs (below) read the nibble stream directly.
         const uint16_t* Wd = nullptr;
@@ -758,8 +790,13 @@ int kf_embed_batch(kf_ctx* c, const kf_weight* w, const int32_t* d_tokens, int n
 // Large token batches of matrices that share their input (Q | K | V, gate | up): GetDataX of each into the caller's scratch, back to back, then ONE launch of the
 // 256 x 256 bf16 tile kernel over the stacked rows (each matrix a multiple of 256 rows; its rows go to its own output).  A 1024-row K or V projection alone is 4 x 8
 // tiles at 2048 tokens -- an eighth of the chip -- and took 32 us on the in-register-unpack kernels; stacked with Q it is 128 tiles.
-static const int KF_MULTI_DEQ_MIN = 1024; /* token rows from which the stacked route is taken (with a dequantise per call; resident copies: g_knobs.resident_min) */
-static int multi_min(const kf_ctx* c) { return c && c->arena && kf::g_knobs.resident_min < KF_MULTI_DEQ_MIN ? kf::g_knobs.resident_min : KF_MULTI_DEQ_MIN; }
+static const int KF_MULTI_DEQ_MIN = 1024; /* token rows from which the stacked route is taken with a dequantise launch per matrix and call; resident copies: g_knobs.resident_min; the layer's: KF_LAYER_COPIES_MIN */
+static int multi_min(const kf_ctx* c) {
+    int n = KF_MULTI_DEQ_MIN;
+    if (c && c->arena && kf::g_knobs.resident_min < n) n = kf::g_knobs.resident_min;
+    if (c && !c->call.empty() && KF_LAYER_COPIES_MIN < n) n = KF_LAYER_COPIES_MIN;
+    return n;
+}
 /* up256z: a no-op on these sizes (multiples of 256 rows x 64 columns): the stacked rows are contiguous */
 static bool multi_deq_ok(int n_w, const kf_weight* const* w, int nTok, size_t* need, const kf_ctx* c = nullptr) {
     size_t tot = 0;
@@ -779,6 +816,70 @@ size_t kf_linear_multi_scratch_bytes(int n_w, const kf_weight* const* w, int nTo
     for (int i = 0; i < n_w; i++)
         if (!w[i]) return 0;
     return multi_deq_ok(n_w, w, nTok, &need) ? need : 0;
+}
+// The copies of a layer: groups of matrices as the routes look for them.  false: this weight is not one the one-launch dequantiser serves
+static bool layer_groups(const kf_weight* const w[7], int nTok, int n_w[4], int form[4], size_t* need) {
+    static const int first[4] = {0, 3, 4, 6};
+    size_t tot = 0;
+    for (int i = 0; i < 7; i++) {
+        if (!w[i] || w[i]->qzeros || w[i]->quant != KF_QUANT_GROUP || w[i]->type != KF_Q4 || w[i]->lGroup != 128 || !w[i]->gama || !w[i]->data || !al16(w[i]->data)) return false;
+        if (w[i]->ne0 < 128 || w[i]->ne0 % 16 || w[i]->ne1 % 128) return false;
+        tot += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
+    }
+    n_w[0] = 3, n_w[1] = 1, n_w[2] = 2, n_w[3] = 1;
+    for (int g = 0; g < 4; g++) form[g] = g == 2 ? DEQ_ILV : DEQ_STACK;
+    for (int g = 0; g < 4; g += 2) { /* stacked sets: the stacked routes' own conditions */
+        long rows = 0;
+        for (int i = first[g]; i < first[g] + n_w[g]; i++) {
+            if (w[i]->ne0 % 256 || w[i]->ne1 != w[first[g]]->ne1 || (g == 2 && w[i]->ne0 != w[first[g]]->ne0)) return false;
+            rows += w[i]->ne0;
+        }
+        if ((rows / 256) * ((nTok + 255) / 256) < 64 && (rows / 128) * ((nTok + 127) / 128) < 64) return false;
+    }
+    *need = tot;
+    return true;
+}
+size_t kf_layer_copies_bytes(const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok) {
+    const kf_weight* const w[7] = {wq, wk, wv, wo, gate, up, down};
+    int n_w[4], form[4];
+    size_t need = 0;
+    return nTok >= KF_LAYER_COPIES_MIN && layer_groups(w, nTok, n_w, form, &need) ? need + kf::gemm3_sk_ws_bytes() + 512 : 0;
+}
+int kf_layer_copies(kf_ctx* c, const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok) {
+    CHKCTX(c);
+    const kf_weight* const w[7] = {wq, wk, wv, wo, gate, up, down};
+    int n_w[4], form[4];
+    size_t need = 0;
+    c->call.clear(), c->call_used = 0;
+    if (c->capturing || c->arena || nTok < KF_LAYER_COPIES_MIN || !layer_groups(w, nTok, n_w, form, &need) || !c->scratch || c->scratch_bytes < need) return 1;
+    uint16_t* out[7];
+    int ilv_n[7], ilv_i[7];
+    size_t off = 0;
+    for (int g = 0, i = 0; g < 4; g++) {
+        kf_ctx::DeqCopy e;
+        e.form = form[g], e.off = off;
+        for (int j = 0; j < 3; j++) e.key[j] = j < n_w[g] ? w[i + j]->data : nullptr;
+        uint16_t* const group = (uint16_t*)((char*)c->scratch + off);
+        for (int j = 0; j < n_w[g]; j++, i++) {
+            ilv_n[i] = form[g] == DEQ_ILV ? n_w[g] : 1, ilv_i[i] = form[g] == DEQ_ILV ? j : 0;
+            out[i] = form[g] == DEQ_ILV ? group : (uint16_t*)((char*)c->scratch + off);
+            off += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
+        }
+        c->call.push_back(e);
+    }
+    scratch_written(c, c->scratch, need);
+    const int r = kf::dequant4_layer_launch(c->stream, 7, w, out, ilv_n, ilv_i);
+    if (r != KF_OK) {
+        c->call.clear();
+        return fail(r, "kf_layer_copies failed with %d", r);
+    }
+    c->call_used = off;
+    return KF_OK;
+}
+int kf_layer_copies_end(kf_ctx* c) {
+    CHKCTX(c);
+    c->call.clear(), c->call_used = 0;
+    return KF_OK;
 }
 // KF_OK done, 1 not this route, < 0 error
 static int multi_deq_route(kf_ctx* c, int n_w, const kf_weight* const* w, const kf_bf16* x, kf_bf16* const* y, int nTok, const kf::G3Rope* rope = nullptr) {

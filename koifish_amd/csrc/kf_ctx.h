@@ -26,6 +26,13 @@ struct kf_ctx {
     void* arena;
     size_t arena_bytes, arena_used;
     std::vector<DeqCopy> copies;
+    // bf16 copies of one layer's matrices for the calls between kf_layer_copies and kf_layer_copies_end, at the front of the scratch (call_used bytes of it)
+    std::vector<DeqCopy> call;
+    size_t call_used;
+    char* scratch_tail() const { return scratch ? (char*)scratch + call_used : nullptr; } /* what the copies leave: 256-byte steps */
+    size_t scratch_left() const { return scratch_bytes > call_used ? scratch_bytes - call_used : 0; }
+    /* the split-K slots lent to the tile kernels lie at the scratch's END, so their flags stay where they were as long as no copy reaches them (scratch_written) */
+    void* scratch_end(size_t bytes) const { return scratch && scratch_left() >= bytes + 256 ? (void*)(((uintptr_t)scratch + scratch_bytes - bytes) & ~(uintptr_t)255) : nullptr; }
 };
 enum { DEQ_STACK = 0, DEQ_ILV = 1 };
 

@@ -375,6 +375,13 @@ static int g3_sk_epoch(hipStream_t st, uint32_t* flags, int n, uint32_t* epoch) 
     return KF_OK;
 }
 
+void gemm3_sk_forget(void* ws) { /* something else was (or will be) written where this workspace's flags lie: its next launch clears them */
+    const void* const flags = (char*)ws + gemm3_sk_ws_bytes() - G3_SK_FLAG_BYTES;
+    std::lock_guard<std::mutex> lk(g_sk_mu);
+    for (const void*& p : g_sk_seen)
+        if (p == flags) p = nullptr;
+}
+
 // KF_OK launched, 1 = not for this kernel (the caller's other tile kernels take the shape), < 0 error.  bf16 "weights" only: quantised ones are dequantised first.
 // BK = 32 (4 LDS buffers, three steps in flight) was measured 8-10 % slower than BK = 64 (2 buffers) on every shape, forward and backward: the per-step costs
 // (barrier, counted wait, loop) double, and the loop is not waiting for memory.  Only BK = 64 is instantiated.
@@ -387,9 +394,10 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
         if (hipFuncSetAttribute((const void*)gemm3_sk_kernel<AKM, BKM, BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
-    // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k
+    // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; K-contiguous products from K = 3072 (plain | split, us:
+    // 1024 x 2048 at 512 tokens 11.2 | 12.6, at 2047 17.3 | 20.5;  2048 x 2048 at 512 11.0 | 15.2;  1024 x 3072 at 320 21.3 | 15.3, at 512 15.5 | 16.3, at 2047 30.0 | 25.5;  2048 x 6144 at 512 44.5 | 32.6)
     const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
-    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G) {
+    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || nkt >= 48)) {
         G3SkArgs s;
         // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they moved with it,
         // and another configuration's fp32 partials could overwrite words already marked "seen" with values that pass for an epoch)

@@ -738,6 +738,25 @@ int Fish::RunSteps(int pos, int n, bool use_graph) {
     return KF_OK;
 }
 
+// the bf16 copies of a layer's 4-bit matrices for the launches of its token batch (kf_layer_copies), for the life of this object
+struct LayerCopies {
+    kf_ctx* ctx = nullptr;
+    int rc = KF_OK;
+    LayerCopies(Fish* f, int l, int n) {
+        const kf_weight q = f->attn[l]->Q.w->desc(), k = f->attn[l]->K.w->desc(), v = f->attn[l]->V.w->desc(), o = f->attn[l]->proj_cat.w->desc();
+        const kf_weight g = f->ffn[l]->gate.w->desc(), u = f->ffn[l]->up.w->desc(), d = f->ffn[l]->down.w->desc();
+        if (!kf_layer_copies_bytes(&q, &k, &v, &o, &g, &u, &d, n)) return;
+        rc = kf_layer_copies(f->ctx, &q, &k, &v, &o, &g, &u, &d, n);
+        if (rc == KF_OK) ctx = f->ctx;
+        else if (rc == 1) rc = KF_OK; /* no workspace, or resident copies: the routes do without */
+    }
+    ~LayerCopies() {
+        if (ctx) kf_layer_copies_end(ctx);
+    }
+    LayerCopies(const LayerCopies&) = delete;
+    LayerCopies& operator=(const LayerCopies&) = delete;
+};
+
 int Fish::Prefill(const int* tokens, int n, int pos0) {
     if (n < 1 || pos0 < 0 || pos0 + n > config.n_ctx) return KF_INVALID_ARGS;
     for (int i = 0; i < n; i++)
@@ -752,6 +771,8 @@ int Fish::Prefill(const int* tokens, int n, int pos0) {
         KF_TRY(kf_h2d(ctx, gBUFF.d_ptok, tokens + c0, (size_t)m * 4));
         KF_TRY(kf_embed_batch(ctx, &we, gBUFF.d_ptok, m, bx));
         for (int l = 0; l < config.nLayer; l++) {
+            LayerCopies copies(this, l, m);
+            KF_TRY(copies.rc);
             KF_TRY(attn[l]->cuFlow(bx, pos0 + c0, m));
             KF_TRY(ffn[l]->cuFlow(bx, m));
         }
@@ -791,8 +812,10 @@ int Fish::PrefillReady(int min_rows) {
             kf_weight wq = attn[l]->Q.w->desc(), wk = attn[l]->K.w->desc(), wv = attn[l]->V.w->desc(), wg = ffn[l]->gate.w->desc(), wu = ffn[l]->up.w->desc();
             const kf_weight* qkv[3] = {&wq, &wk, &wv};
             const kf_weight* gu[2] = {&wg, &wu};
-            size_t need = kf_linear_multi_scratch_bytes(3, qkv, PC), need2 = kf_linear_multi_scratch_bytes(2, gu, PC);
-            need = need > need2 ? need : need2;
+            kf_weight wo = attn[l]->proj_cat.w->desc(), wd = ffn[l]->down.w->desc();
+            size_t need = 0;
+            for (size_t n : {kf_linear_multi_scratch_bytes(3, qkv, PC), kf_linear_multi_scratch_bytes(2, gu, PC), kf_linear_scratch_bytes(&wo, PC), kf_linear_scratch_bytes(&wd, PC),
+                             kf_layer_copies_bytes(&wq, &wk, &wv, &wo, &wg, &wu, &wd, PC)}) need = n > need ? n : need;
             if (need > lin_scratch_bytes) {
                 KF_TRY(kf_sync(ctx));
                 void* p = nullptr;
@@ -1150,6 +1173,8 @@ int XcdReplicas::PrefillBatch(const int* slots, const int32_t* tokens, const int
     for (int l = 0; l < c.nLayer; l++) {
         SelfAttention& a = *f->attn[l];
         kf_weight wq = a.Q.w->desc(), wk = a.K.w->desc(), wv = a.V.w->desc(), wo = a.proj_cat.w->desc();
+        LayerCopies copies(f, l, R);
+        KF_TRY(copies.rc);
         KF_TRY(kf_rmsnorm(ctx, bx, ToX(a.norm.w), bn, R, C, a.norm.rms_eps, nullptr));
         KF_TRY(kf_qkv_rope_seqs(ctx, &wq, &wk, &wv, bn, bq, bk, bv, R, T, a.normQ.w ? ToX(a.normQ.w) : nullptr, a.normK.w ? ToX(a.normK.w) : nullptr, f->rope_table, 0, c.n_head,
                                 c.n_head_kv, c.head_dim, a.normQ.rms_eps)); /* positions restart with every prompt */

@@ -1,0 +1,77 @@
+"""kf_layer_copies: one launch's bf16 copies are kf_dequant's, bit for bit, in every layout (rows back to back, gate | up interleaved in blocks of 16), and the routes that find them give what the
+same products give on bf16 weights; what is not served is left to the routes as they were."""
+import ctypes as C
+
+import pytest
+import torch
+
+from koifish_amd import lib as L
+from koifish_amd import runtime as R
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(ctx, dim, q, kv, ffn, types=(L.Q4,) * 7):
+    g = torch.Generator(device=ctx.device)
+    g.manual_seed(dim + ffn)
+    shapes = [(q, dim), (kv, dim), (kv, dim), (dim, q), (ffn, dim), (ffn, dim), (dim, ffn)]
+    ws = [ctx.quantize((torch.randn(*s, device=ctx.device, generator=g) * 0.05).bfloat16(), t) for s, t in zip(shapes, types)]
+    return ws, [w.desc() for w in ws]
+
+
+def _copies(ctx, descs, n):
+    need = ctx.hip.kf_layer_copies_bytes(*[C.byref(d) for d in descs], n)
+    if not need:
+        return 0, None
+    scratch = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=ctx.device)
+    assert ctx.hip.kf_set_scratch(ctx.h, C.c_void_p(scratch.data_ptr()), C.c_size_t(need)) == 0
+    assert ctx.hip.kf_layer_copies(ctx.h, *[C.byref(d) for d in descs], n) == 0
+    ctx.sync()
+    assert bool((scratch[need:] == 0x5A).all())   # nothing past the workspace
+    return need, scratch
+
+
+@pytest.mark.parametrize("dim,q,kv,ffn,n", [(1024, 2048, 1024, 3072, 320), (256, 512, 256, 512, 2047), (2560, 4096, 1024, 9728, 321)])
+def test_copies_and_routes(ctx, dim, q, kv, ffn, n):
+    ws, descs = _layer(ctx, dim, q, kv, ffn)
+    try:
+        need, scratch = _copies(ctx, descs, n)
+        assert need
+        bf = [ctx.dequant(w) for w in ws]
+        out, off = scratch.view(torch.bfloat16), 0
+        for i in (0, 1, 2, 3):
+            assert torch.equal(out[off:off + bf[i].numel()].view_as(bf[i]), bf[i])
+            off += bf[i].numel()
+        both = torch.stack([bf[4].view(ffn // 16, 16, dim), bf[5].view(ffn // 16, 16, dim)], 1).reshape(2 * ffn, dim)
+        assert torch.equal(out[off:off + both.numel()].view_as(both), both)
+        off += both.numel()
+        assert torch.equal(out[off:off + bf[6].numel()].view_as(bf[6]), bf[6])
+        # o and down through kf_linear: the product on the copy, against fp32 on the dequantised values (sums of K bf16 products in fp32, one bf16 rounding: 2^-8 of a value, 2^-8 of the sum's scale)
+        for i in (3, 6):
+            x = torch.randn(n, ws[i].ne1, device=ctx.device).bfloat16()
+            y = torch.zeros(n, ws[i].ne0, device=ctx.device, dtype=torch.bfloat16)
+            assert ctx.hip.kf_linear(ctx.h, C.byref(descs[i]), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
+            ref = x.float() @ bf[i].float().t()
+            assert float((y.float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+            assert torch.equal(out[:bf[0].numel()].view_as(bf[0]), bf[0])   # the split-K slots do not touch the copies
+        x = torch.randn(n, dim, device=ctx.device).bfloat16()
+        act, up = (torch.zeros(n, ffn, device=ctx.device, dtype=torch.bfloat16) for _ in range(2))
+        assert ctx.hip.kf_gateup_swiglu_batch(ctx.h, C.byref(descs[4]), C.byref(descs[5]), x.data_ptr(), act.data_ptr(), up.data_ptr(), n) == 0
+        g, u = x.float() @ bf[4].float().t(), x.float() @ bf[5].float().t()
+        ref = torch.nn.functional.silu(g) * u
+        assert float((act.float() - ref).abs().max()) <= 2.0 ** -6 * float(ref.abs().max())
+        # other uses of the scratch stay behind the copies; after the end the routes are the ones without copies
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+def test_not_served_is_left_alone(ctx):
+    _, descs = _layer(ctx, 256, 512, 256, 512)
+    p = [C.byref(d) for d in descs]
+    assert ctx.hip.kf_layer_copies_bytes(*p, 319) == 0 and ctx.hip.kf_layer_copies(ctx.h, *p, 2047) == 1   # too few rows; no workspace
+    mixed = [C.byref(d) for d in _layer(ctx, 256, 512, 256, 512, (L.Q4,) * 6 + (L.F8E5M2,))[1]]
+    assert ctx.hip.kf_layer_copies_bytes(*mixed, 2047) == 0
+    odd = [C.byref(d) for d in _layer(ctx, 256, 384, 128, 512)[1]]   # rows no multiple of 256: the stacked route does not take them
+    assert ctx.hip.kf_layer_copies_bytes(*odd, 2047) == 0
