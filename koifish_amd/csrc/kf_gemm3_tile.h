@@ -102,15 +102,24 @@ __device__ __forceinline__ bf16x8 g3_frag_km(const unsigned char* tile, int km_l
 // `rows` (G3Rows: plain; G3Gather: row r of the token tile is row map[r] of x) says where the tile's token rows lie.
 // TILED: w is stored in MFMA tiles (kf_rb.h: 16 rows x 32 columns, piece (r, q) at number 16 q + r) instead of rows: a load
 // instruction moves one tile, contiguous in memory and in LDS, and a fragment read is lane-linear -- no swizzle on this operand.
+// F32: both operands are 32-bit floats, their strides counted in 16-bit units like the others' (K = twice the floats): a step is 32 of them, the tile's bytes, chunks and swizzle are
+// the same, and a lane's 16-byte chunk is the operand of four v_mfma_f32_16x16x4_f32 (lane group q, float i: k = 4 q + i on both sides).
 struct G3Rows {
-    static constexpr bool GATHER = false, TILED = false;
+    static constexpr bool GATHER = false, TILED = false, F32 = false;
 };
 struct G3Tiled {
-    static constexpr bool GATHER = false, TILED = true;
+    static constexpr bool GATHER = false, TILED = true, F32 = false;
 };
 struct G3GatherTiled {
-    static constexpr bool GATHER = true, TILED = true;
+    static constexpr bool GATHER = true, TILED = true, F32 = false;
     const int32_t* map; /* [BN] rows of x, every entry valid */
+};
+struct G3RowsF32 {
+    static constexpr bool GATHER = false, TILED = false, F32 = true;
+};
+struct G3GatherF32 {
+    static constexpr bool GATHER = true, TILED = false, F32 = true;
+    const int32_t* map;
 };
 // The schedule.  A wave's outputs are four quadrants (row half x token half); the fragments of a quadrant are read from LDS under the MFMAs of the quadrant before it:
 //   quadrant (0,0): read token half 1          (0,1): read row half 1          -- step kt + 1 has landed, every wave holds its last fragments of step kt: ONE barrier --
@@ -211,18 +220,24 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
                 else f[nh][kk] = g3_frag(bufB(b), wn * (16 * C::NT) + nt * 16 + r16, kk * 4 + q4);
             }
     };
+    constexpr int PIECES = ROWS::F32 ? 4 : 1; /* MFMAs per pair of fragments */
     auto mul = [&](int mh0, int nh0, const bf16x8 (&fa)[HM][2], const bf16x8 (&fb)[HN][2]) {
 #pragma unroll
         for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int i = 0; i < HM; i++)
+            for (int e = 0; e < PIECES; e++)
 #pragma unroll
-                for (int j = 0; j < HN; j++)
-                    acc[mh0 * HM + i][nh0 * HN + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][kk], fb[j][kk], acc[mh0 * HM + i][nh0 * HN + j], 0, 0, 0);
+                for (int i = 0; i < HM; i++)
+#pragma unroll
+                    for (int j = 0; j < HN; j++) {
+                        f32x4& d = acc[mh0 * HM + i][nh0 * HN + j];
+                        if constexpr (ROWS::F32) d = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4, fa[i][kk])[e], __builtin_bit_cast(f32x4, fb[j][kk])[e], d, 0, 0, 0);
+                        else d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][kk], fb[j][kk], d, 0, 0, 0);
+                    }
     };
     // a quadrant's issue order: its LDS reads and its loads one by one among its first MFMAs, the rest of the MFMAs behind them
     auto order = [&](auto n_reads, auto n_loads) {
-        constexpr int N = decltype(n_reads)::value, V = decltype(n_loads)::value, M = HM * HN * 2, P = N < M ? N : M, Q = V < M - 1 ? V : M - 1, X = P > Q ? P : Q;
+        constexpr int N = decltype(n_reads)::value, V = decltype(n_loads)::value, M = HM * HN * 2 * PIECES, P = N < M ? N : M, Q = V < M - 1 ? V : M - 1, X = P > Q ? P : Q;
 #pragma unroll
         for (int i = 0; i < X; i++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);

@@ -31,7 +31,7 @@ struct RbProduct {
     kf_rb_product p;
     kf_rb_experts e;
 };
-// kf_rb_gemm.hip: bf16 tile kernels (any number of rows); kf_rb_linear.hip: streaming form (<= KF_RB_DECODE_MAX rows) and the fp32 product
+// kf_rb_gemm.hip: tile kernels in both storages (any number of rows); kf_rb_linear.hip: streaming form (bf16, <= KF_RB_DECODE_MAX rows)
 int rb_gemm_launch(hipStream_t st, const RbProduct& a);
 int rb_stream_launch(hipStream_t st, const RbProduct& a);
 int rb_f32_launch(hipStream_t st, const RbProduct& a);

@@ -14,7 +14,8 @@ using RbMid = G3Cfg<64, 128, 4>;
 using RbTiny = G3Cfg<64, 64, 4>;
 using RbPairs = G3Cfg<128, 64, 4>; /* experts of about a hundred pairs: half the padding of 128-pair tiles, each weight tile read about once */
 
-template <class C, bool EXPERTS>
+// T: the storage, uint16_t (bf16: weights in MFMA tiles) or float (true 32-bit: weights in rows)
+template <class C, bool EXPERTS, class T>
 __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_kernel(const RbProduct q) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ int32_t s_src[EXPERTS ? C::BN : 1], s_dst[EXPERTS ? C::BN : 1];
@@ -25,7 +26,8 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     g3_tile(g3_remap(blockIdx.x, gridDim.x), nbx, (int)gridDim.x / nbx, bx, by);
     const int m0 = bx * C::BM, t0 = by * C::BN;
     GemmArgs a; /* what the main loop reads */
-    a.w = reinterpret_cast<const unsigned char*>(p.w), a.M = p.m, a.K = p.k, a.x = reinterpret_cast<const uint16_t*>(p.x), a.ldx = p.ldx, a.n = p.n, a.ldr = 0;
+    constexpr int U = sizeof(T) / 2, KT = G3_BK / U; /* 16-bit units of an element, elements of a step */
+    a.w = reinterpret_cast<const unsigned char*>(p.w), a.M = p.m, a.K = p.k * U, a.x = reinterpret_cast<const uint16_t*>(p.x), a.ldx = p.ldx * U, a.n = p.n, a.ldr = 0;
     f32x4 acc[C::MT][C::NT];
 #pragma unroll
     for (int i = 0; i < C::MT; i++)
@@ -34,15 +36,16 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     if constexpr (EXPERTS) {
         const int ex = q.e.tile_expert[by];
         if (ex < 0) return; /* workgroup-uniform */
-        a.w += (size_t)ex * q.e.w_stride * 2;
+        a.w += (size_t)ex * q.e.w_stride * sizeof(T);
         for (int i = tid; i < C::BN; i += C::NTH) {
             const int pair = q.e.list[(size_t)by * C::BN + i];
             s_dst[i] = pair, s_src[i] = pair < 0 ? 0 : (p.mode == KF_RB_UP ? pair / q.e.top : pair);
         }
         __syncthreads();
-        g3_mainloop<false, false, G3_BK, C, G3GatherTiled>(a, m0, 0, 0, p.k / G3_BK, acc, smem_raw, wid, lane, G3GatherTiled{s_src});
+        using Rows = std::conditional_t<U == 2, G3GatherF32, G3GatherTiled>;
+        g3_mainloop<false, false, G3_BK, C, Rows>(a, m0, 0, 0, p.k / KT, acc, smem_raw, wid, lane, Rows{s_src});
     } else {
-        g3_mainloop<false, false, G3_BK, C, G3Tiled>(a, m0, t0, 0, p.k / G3_BK, acc, smem_raw, wid, lane);
+        g3_mainloop<false, false, G3_BK, C, std::conditional_t<U == 2, G3RowsF32, G3Tiled>>(a, m0, t0, 0, p.k / KT, acc, smem_raw, wid, lane);
     }
     const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
 #pragma unroll
@@ -66,7 +69,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
                 f32x4 o;
 #pragma unroll
                 for (int j = 0; j < 4; j++) o[j] = scale * (rb_activate(p.act, g[j]) * u[j]);
-                rb_st4(reinterpret_cast<uint16_t*>(p.y) + (size_t)row * p.ldy + (m >> 1) + 4 * q4, o);
+                rb_st4(reinterpret_cast<T*>(p.y) + (size_t)row * p.ldy + (m >> 1) + 4 * q4, o);
             }
         } else {
 #pragma unroll
@@ -80,7 +83,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
                         for (int j = 0; j < 4; j++)
                             if (m + j >= p.act_lo && m + j < p.act_hi) d[j] = rb_activate(p.act, d[j]);
                     }
-                    rb_st4(reinterpret_cast<uint16_t*>(p.y) + (size_t)row * p.ldy + m, d);
+                    rb_st4(reinterpret_cast<T*>(p.y) + (size_t)row * p.ldy + m, d);
                 } else {
                     if (p.epilogue == KF_RB_RESIDUAL) {
                         const f32x4 r = rb_ld4(p.res + (size_t)row * p.ldr + m);
@@ -93,30 +96,38 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
         }
     }
 }
-template <class C, bool EXPERTS>
+template <class C, bool EXPERTS, class T = uint16_t>
 static int rb_go(hipStream_t st, const RbProduct& q, long nwg) {
     constexpr int SMEM = 2 * C::STAGE;
     static int attr_set = 0;
     if (!attr_set && SMEM + 2 * 4 * C::BN > 64 * 1024) { /* the pair rows of the experts form sit in static LDS */
-        if (hipFuncSetAttribute((const void*)rb_gemm_kernel<C, EXPERTS>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
+        if (hipFuncSetAttribute((const void*)rb_gemm_kernel<C, EXPERTS, T>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
-    hipLaunchKernelGGL((rb_gemm_kernel<C, EXPERTS>), dim3((unsigned)nwg), dim3(C::NTH), SMEM, st, q);
+    hipLaunchKernelGGL((rb_gemm_kernel<C, EXPERTS, T>), dim3((unsigned)nwg), dim3(C::NTH), SMEM, st, q);
     return KF_OK;
 }
+static long rb_tiles(const kf_rb_product& p, int bm, int bn) { return (long)((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); }
 int rb_gemm_launch(hipStream_t st, const RbProduct& q) {
     const kf_rb_product& p = q.p;
-    auto tiles = [&](int bm, int bn) { return (long)((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
     if (p.mode != KF_RB_ALL) {
         if (q.e.tile == 128) return rb_go<RbSmall, true>(st, q, (long)((p.m + 127) / 128) * q.e.n_tile);
         if (q.e.tile == 64) return rb_go<RbPairs, true>(st, q, (long)((p.m + 127) / 128) * q.e.n_tile);
         return 1;
     }
     // the measured thresholds of gemm3_launch: big tiles from 160 of them, then smaller ones that fill the chip
-    if (p.m >= 256 && p.n >= 256 && tiles(256, 256) >= 160) return rb_go<RbBig, false>(st, q, tiles(256, 256));
-    if (tiles(128, 128) >= 256) return rb_go<RbSmall, false>(st, q, tiles(128, 128));
-    if (tiles(64, 128) >= 192) return rb_go<RbMid, false>(st, q, tiles(64, 128));
-    return rb_go<RbTiny, false>(st, q, tiles(64, 64));
+    if (p.m >= 256 && p.n >= 256 && rb_tiles(p, 256, 256) >= 160) return rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
+    if (rb_tiles(p, 128, 128) >= 256) return rb_go<RbSmall, false>(st, q, rb_tiles(p, 128, 128));
+    if (rb_tiles(p, 64, 128) >= 192) return rb_go<RbMid, false>(st, q, rb_tiles(p, 64, 128));
+    return rb_go<RbTiny, false>(st, q, rb_tiles(p, 64, 64));
+}
+// The 32-bit product on v_mfma_f32_16x16x4_f32 (157 TFLOP/s; the vector pipe without packed instructions: 78).  It is bound by the MFMAs, 16 x slower than bf16's, so the tile only has to share them
+// out evenly: 64 x 64 tiles, five to a CU.
+int rb_f32_launch(hipStream_t st, const RbProduct& q) {
+    const kf_rb_product& p = q.p;
+    if (p.mode == KF_RB_SUM || (p.mode != KF_RB_ALL && q.e.tile != 64)) return 1;
+    if (p.mode != KF_RB_ALL) return rb_go<RbTiny, true, float>(st, q, (long)(p.m / 64) * q.e.n_tile);
+    return rb_go<RbTiny, false, float>(st, q, rb_tiles(p, 64, 64));
 }
 
 }  // namespace kf

@@ -279,98 +279,6 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     return KF_OK;
 }
 
-// ---- the 32-bit product: 64 x 64 outputs per workgroup, k in steps of 16 through LDS, 4 x 4 outputs per thread, fp32 fma chains in k order
-__global__ void __launch_bounds__(256) rb_f32_kernel(const RbProduct q) {
-    const kf_rb_product& p = q.p;
-    constexpr int KT = 16;
-    __shared__ float sw[KT][68], sx[KT][68];
-    __shared__ int srow[64], sdst[64];
-    const int tid = threadIdx.x, m0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
-    const float* W = reinterpret_cast<const float*>(p.w);
-    const float* X = reinterpret_cast<const float*>(p.x);
-    const bool ex_mode = p.mode != KF_RB_ALL;
-    if (ex_mode) {
-        const int ex = q.e.tile_expert[blockIdx.y];
-        if (ex < 0) return;
-        W += (size_t)ex * q.e.w_stride;
-    }
-    if (tid < 64) {
-        int src, dst;
-        if (ex_mode) {
-            dst = q.e.list[(size_t)blockIdx.y * 64 + tid];
-            src = dst < 0 ? -1 : (p.mode == KF_RB_UP ? dst / q.e.top : dst);
-        } else {
-            dst = src = c0 + tid < p.n ? c0 + tid : -1;
-        }
-        srow[tid] = src, sdst[tid] = dst;
-    }
-    __syncthreads();
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = 0.f;
-    const int lr = tid >> 2, lk = (tid & 3) * 4; /* staging: row lr, four k */
-    const int tm = (tid & 15) * 4, tc = (tid >> 4) * 4;
-    const int xr = srow[lr];
-    for (int k0 = 0; k0 < p.k; k0 += KT) {
-        const f32x4 wv = *reinterpret_cast<const f32x4*>(W + (size_t)(m0 + lr) * p.k + k0 + lk);
-        f32x4 xv = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (xr >= 0) xv = *reinterpret_cast<const f32x4*>(X + (size_t)xr * p.ldx + k0 + lk);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 4; j++) sw[lk + j][lr] = wv[j], sx[lk + j][lr] = xv[j];
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < KT; kk++) {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(&sw[kk][tm]), b = *reinterpret_cast<const f32x4*>(&sx[kk][tc]);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-    }
-    __shared__ float sout[64][65]; /* [column][row]: GATED pairs rows 16 apart */
-    if (p.epilogue == KF_RB_GATED) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) sout[tc + j][tm + i] = acc[i][j];
-        __syncthreads();
-        for (int i = tid; i < 64 * 32; i += 256) {
-            const int f = i & 31, col = i >> 5, yr = sdst[col];
-            if (yr < 0) continue;
-            const int row = (f >> 4) * 32 + (f & 15);
-            const float scale = p.mode == KF_RB_UP ? q.e.weight[yr] : 1.f;
-            reinterpret_cast<float*>(p.y)[(size_t)yr * p.ldy + (m0 >> 1) + f] = scale * (rb_activate(p.act, sout[col][row]) * sout[col][row + 16]);
-        }
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int yr = sdst[tc + j];
-        if (yr < 0) continue;
-        f32x4 d = f32x4{acc[0][j], acc[1][j], acc[2][j], acc[3][j]};
-        if (p.epilogue == KF_RB_RESIDUAL) {
-            const f32x4 r = *reinterpret_cast<const f32x4*>(p.res + (size_t)yr * p.ldr + m0 + tm);
-#pragma unroll
-            for (int i = 0; i < 4; i++) d[i] = fmaf(p.alpha, r[i], d[i]);
-        } else if (p.epilogue == KF_RB_STORE && m0 + tm + 3 >= p.act_lo && m0 + tm < p.act_hi) {
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (m0 + tm + i >= p.act_lo && m0 + tm + i < p.act_hi) d[i] = rb_activate(p.act, d[i]);
-        }
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.y) + (size_t)yr * p.ldy + m0 + tm) = d;
-    }
-}
-int rb_f32_launch(hipStream_t st, const RbProduct& q) {
-    const kf_rb_product& p = q.p;
-    if (p.mode == KF_RB_SUM || (p.mode != KF_RB_ALL && q.e.tile != 64)) return 1;
-    dim3 grid(p.m / 64, p.mode == KF_RB_ALL ? (p.n + 63) / 64 : q.e.n_tile);
-    hipLaunchKernelGGL(rb_f32_kernel, grid, dim3(256), 0, st, q);
-    return KF_OK;
-}
-
 }  // namespace kf
 
 using namespace kf;
