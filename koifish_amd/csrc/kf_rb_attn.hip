@@ -8,7 +8,7 @@
 //   * only the tiles between a wave's first chunk start and its last position.
 // A decode row is one workgroup per (kv-head, key range): q and the new key are prepared in LDS, each of its four waves walks its own 32-key tiles (staged into LDS of its
 // own, no barrier in the walk) and the four partial softmaxes meet at the end.
-// fp32 storage (and other head sizes): a plain form, one wave per (row, head), 32-bit throughout.
+// fp32 storage, prompts with heads of multiples of 16 up to 128: the same scheme on 32-bit MFMAs.  Everything else: a plain form, one wave per (row, head), 32-bit throughout.
 #include <algorithm>
 
 #include "kf_ctx.h"
@@ -216,6 +216,166 @@ __global__ void __launch_bounds__(64) rb_attn_plain_kernel(const kf_rb_attention
     for (int j = 0; j < ND; j++) {
         const int d = lane + 64 * j;
         if (d < a.vdim) rb_st(out + d, o[j] * f / l * (a.gated ? rb_sigmoid(rb_ld(gate + d)) : 1.f));
+    }
+}
+
+// ---- 32-bit prompts on v_mfma_f32_16x16x4_f32: 32 columns ((token, query head) pairs of a kv-head) per workgroup, waves as 2 column groups x 2 key halves, 32 keys per tile.  S^T = K Q^T leaves a lane
+// with four keys (4 q + i) of its column, which is how the MFMA takes its second operand, so the weights go into O^T = V^T P as they are; operands are read four k at a time (see kf_rb_recur.hip).
+// K and V rows are HD + 4 floats apart: a fragment's reads of V (16 dimensions of four keys) touch every bank once.  Everything the plain form keeps in 32 bits stays so: scores, expf, sums.
+// 512 tokens, 16 heads of 128 on 8: 373 us in the plain form (a wave per row and head), 50 us here; the MFMAs alone would take 7.
+template <int HD>
+__global__ void __launch_bounds__(256, 2) rb_attn_prefill_f32_kernel(const kf_rb_attention a, const int32_t* __restrict__ seqs) {
+    constexpr int LD = HD + 4, NC = HD / 16, CPT = 32 * HD / 4 / 256; /* row stride, blocks of 16 dimensions, 16-byte pieces per thread and operand */
+    extern __shared__ __attribute__((aligned(16))) float s_kv[]; /* two buffers of K [32][LD], V [32][LD] */
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, cg = wid & 1, kh = wid >> 1, r16 = lane & 15, q4 = lane >> 4, kvd = a.n_kv * a.dim;
+    const int row0 = seqs[4 * blockIdx.z], n = seqs[4 * blockIdx.z + 1], pos0 = seqs[4 * blockIdx.z + 2], slot = seqs[4 * blockIdx.z + 3];
+    const int wg = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y, g = wg % a.n_kv, bx = (int)gridDim.x - 1 - wg / a.n_kv; /* a kv-head's workgroups on the same XCDs, long walks first */
+    const int GQ = a.n_head / a.n_kv, ncol = n * GQ;
+    if (bx * 32 >= ncol) return; /* workgroup-uniform */
+    const float* raw = reinterpret_cast<const float*>(a.raw) + (size_t)row0 * a.ldraw;
+    const float *k_new = reinterpret_cast<const float*>(a.k_new) + (size_t)row0 * kvd + (size_t)g * a.dim, *v_new = raw + a.v_col + (size_t)g * a.vdim;
+    const float* k_ring = reinterpret_cast<const float*>(a.k_cache) + (size_t)slot * a.slot_stride + (size_t)g * a.head_stride;
+    const float* v_ring = reinterpret_cast<const float*>(a.v_cache) + (size_t)slot * a.slot_stride + (size_t)g * a.head_stride;
+    int c = bx * 32 + cg * 16 + r16;
+    const bool col_ok = c < ncol;
+    c = col_ok ? c : ncol - 1; /* columns past the end repeat the last one and are not stored */
+    const int tok = c / GQ, head = g * GQ + (c - tok * GQ), pos = pos0 + tok, lo = rb_first_key(pos, a);
+    auto tok_of = [&](int cc) { return (cc < ncol ? cc : ncol - 1) / GQ; };
+    const int wlo = rb_first_key(pos0 + tok_of(bx * 32 + cg * 16), a), w1 = pos0 + tok_of(bx * 32 + cg * 16 + 15);
+    const int klo = rb_first_key(pos0 + tok_of(bx * 32), a), khi = pos0 + tok_of(bx * 32 + 31);
+    f32x4 qf[NC], o[NC], kr[CPT], vr[CPT];
+    {
+        const float* q = raw + (size_t)tok * a.ldraw + (size_t)head * a.dim;
+#pragma unroll
+        for (int s = 0; s < NC; s++) {
+            o[s] = qf[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (16 * s < a.dim) qf[s] = *reinterpret_cast<const f32x4*>(q + 16 * s + 4 * q4);
+        }
+    }
+    auto tload = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < CPT; i++) {
+            const int ch = tid + 256 * i, key = ch / (HD / 4), d = (ch - key * (HD / 4)) * 4;
+            const int kk = k0 + key < khi ? k0 + key : khi; /* past the last key: masked, never read past it */
+            const float *kb = k_new, *vb = v_new;
+            size_t ok, ov;
+            if (kk >= pos0) {
+                ok = (size_t)(kk - pos0) * kvd, ov = (size_t)(kk - pos0) * a.ldraw;
+            } else {
+                const uint32_t row = (uint32_t)kk % (uint32_t)a.cache_rows;
+                kb = k_ring, vb = v_ring, ok = (size_t)row * a.dim, ov = (size_t)row * a.vdim;
+            }
+            kr[i] = vr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (d < a.dim) kr[i] = *reinterpret_cast<const f32x4*>(kb + ok + d);
+            if (d < a.vdim) vr[i] = *reinterpret_cast<const f32x4*>(vb + ov + d);
+        }
+    };
+    __shared__ int s_odd[2]; /* the tile (+ 1) whose values hold an infinity or a NaN, per buffer */
+    auto tstore = [&](int t) {
+        const int b = t & 1;
+        bool odd = false;
+#pragma unroll
+        for (int i = 0; i < CPT; i++) {
+            const int ch = tid + 256 * i, key = ch / (HD / 4), d = (ch - key * (HD / 4)) * 4;
+            *reinterpret_cast<f32x4*>(s_kv + (size_t)(b * 64 + key) * LD + d) = kr[i];
+            *reinterpret_cast<f32x4*>(s_kv + (size_t)(b * 64 + 32 + key) * LD + d) = vr[i];
+#pragma unroll
+            for (int j = 0; j < 4; j++) odd = odd || (__float_as_uint(vr[i][j]) & 0x7F800000u) == 0x7F800000u;
+        }
+        if (odd) s_odd[b] = t + 1;
+    };
+    float M = -__builtin_inff(), l = 0.f;
+    const int ntile = (khi - klo) / 32 + 1;
+    if (tid < 2) s_odd[tid] = 0;
+    __syncthreads();
+    tload(klo);
+    tstore(0);
+    __syncthreads();
+    for (int t = 0; t < ntile; t++) {
+        const int k0 = klo + 32 * t, b = t & 1;
+        if (t + 1 < ntile) tload(k0 + 32);
+        if (k0 + kh * 16 + 15 >= wlo && k0 + kh * 16 <= w1) { /* wave-uniform: some column of the wave sees some of its 16 keys */
+            const float *ks = s_kv + (size_t)(b * 64 + kh * 16 + r16) * LD + 4 * q4, *vs = s_kv + (size_t)(b * 64 + 32 + kh * 16 + 4 * q4) * LD + r16;
+            f32x4 S0 = f32x4{0.f, 0.f, 0.f, 0.f}, S1 = S0;
+#pragma unroll
+            for (int s = 0; s < NC; s++) {
+                const f32x4 kf = *reinterpret_cast<const f32x4*>(ks + 16 * s);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    f32x4& d = (s & 1) ? S1 : S0;
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[s][e], d, 0, 0, 0);
+                }
+            }
+            float p[4], mt = -__builtin_inff();
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int kk = k0 + kh * 16 + 4 * q4 + j;
+                p[j] = kk >= lo && kk <= pos ? (S0[j] + S1[j]) * a.scale : -__builtin_inff();
+                mt = fmaxf(mt, p[j]);
+            }
+            mt = fmaxf(mt, __shfl_xor(mt, 16, 64)), mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+            const float Mn = fmaxf(M, mt), base = Mn == -__builtin_inff() ? 0.f : Mn; /* a column may have seen no key yet */
+            const float f = expf(M - base);
+            float sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) p[j] = expf(p[j] - base), sum += p[j];
+            l = fmaf(l, f, sum), M = Mn;
+#pragma unroll
+            for (int s = 0; s < NC; s++) o[s] *= f;
+            if (s_odd[b] != t + 1) { /* workgroup-uniform */
+#pragma unroll
+                for (int s = 0; s < NC; s++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[e * LD + 16 * s], p[e], o[s], 0, 0, 0);
+            } else { /* 0 x infinity: a value that a column does not see must not reach it, so key by key */
+                const float* const v0 = s_kv + (size_t)(b * 64 + 32 + kh * 16) * LD + 4 * q4;
+                for (int i = 0; i < 16; i++) {
+                    const float pi = __shfl(i & 2 ? (i & 1 ? p[3] : p[2]) : (i & 1 ? p[1] : p[0]), (i >> 2) * 16 + r16, 64);
+                    const int kk = k0 + kh * 16 + i;
+                    if (kk < lo || kk > pos) continue;
+#pragma unroll
+                    for (int s = 0; s < NC; s++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) o[s][j] = fmaf(pi, v0[(size_t)i * LD + 16 * s + j], o[s][j]);
+                }
+            }
+        }
+        if (t + 1 < ntile) tstore(t + 1);
+        __syncthreads();
+    }
+    // the second key half hands its part over: [group][NC * 4 + 2][64 lanes]
+    float* const ex = s_kv + (size_t)cg * (NC * 4 + 2) * 64 + lane;
+    if (kh) {
+#pragma unroll
+        for (int s = 0; s < NC; s++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) ex[(s * 4 + j) * 64] = o[s][j];
+        ex[NC * 4 * 64] = M, ex[(NC * 4 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (kh) return;
+    const float M1 = ex[NC * 4 * 64], Mm = fmaxf(M, M1), f0 = expf(M - Mm), f1 = expf(M1 - Mm); /* one of the halves has seen a key of the column: its own position's */
+    l = l * f0 + ex[(NC * 4 + 1) * 64] * f1;
+    l += __shfl_xor(l, 16, 64), l += __shfl_xor(l, 32, 64);
+    if (!col_ok) return;
+    float f = a.out_scale;
+    if (a.sink) {
+        const float Ms = fmaxf(Mm, 0.f), fs = expf(Mm - Ms);
+        l = l * fs + expf(-Ms), f *= fs;
+    }
+    const float* gate = raw + (size_t)tok * a.ldraw + a.gate_col + (size_t)head * a.vdim;
+    float* out = reinterpret_cast<float*>(a.out) + (size_t)(row0 + tok) * a.ldout + (size_t)head * a.vdim;
+#pragma unroll
+    for (int s = 0; s < NC; s++) {
+        const int d = 16 * s + 4 * q4;
+        if (16 * s >= a.vdim) break;
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            v[j] = (o[s][j] * f0 + ex[(s * 4 + j) * 64] * f1) * f / l;
+            if (a.gated) v[j] *= rb_sigmoid(gate[d + j]);
+        }
+        rb_st4(out + d, v);
     }
 }
 
@@ -664,6 +824,16 @@ static int decode_go(hipStream_t st, const kf_rb_attention& a, const kf_rb_decay
 static bool mfma_served(const kf_rb_attention& a, int n_rows) {
     return a.type == KF_BF16 && (int64_t)n_rows * a.ldraw < ((int64_t)1 << 30) && (int64_t)a.cache_rows * a.n_kv * std::max(a.dim, a.vdim) < ((int64_t)1 << 30) && a.dim % 8 == 0 && a.dim <= 256 && a.vdim % 8 == 0 && a.vdim <= 256 && a.v_col % 8 == 0 && a.gate_col % 4 == 0 && a.ldraw % 8 == 0 && a.ldout % 4 == 0 && a.slot_stride % 8 == 0 && a.head_stride % 8 == 0;
 }
+static bool f32_served(const kf_rb_attention& a) { return a.dim % 16 == 0 && a.vdim % 16 == 0 && a.dim <= 128 && a.vdim <= 128 && a.v_col % 4 == 0 && a.gate_col % 4 == 0 && a.ldraw % 4 == 0 && a.ldout % 4 == 0 && a.slot_stride % 4 == 0 && a.head_stride % 4 == 0; }
+template <int HD>
+static int f32_go(hipStream_t st, const kf_rb_attention& a, const int32_t* seqs, int n_seq, int max_n) {
+    constexpr size_t smem = (size_t)4 * 32 * (HD + 4) * 4;
+    static_assert(smem >= (size_t)2 * (HD / 4 + 2) * 64 * 4, "the hand-over in the tiles' place");
+    static int done = 0;
+    if (big_lds(rb_attn_prefill_f32_kernel<HD>, smem, done)) return KF_HIP_CHECK;
+    hipLaunchKernelGGL(rb_attn_prefill_f32_kernel<HD>, dim3((unsigned)(((long long)max_n * (a.n_head / a.n_kv) + 31) / 32), a.n_kv, n_seq), dim3(256), smem, st, a, seqs);
+    return KF_OK;
+}
 #define RB_BY_DIM(call)                                 \
     (std::max(a.dim, a.vdim) <= 32    ? call(32)        \
      : std::max(a.dim, a.vdim) <= 64  ? call(64)        \
@@ -779,7 +949,8 @@ int kf_rb_attention_prefill(kf_ctx* c, const kf_rb_attention* ap, const int32_t*
         store_go<uint16_t>(st, a, meta, n_rows);
     } else {
         prep_go<float>(st, a, meta, n_rows, false);
-        plain_go<float>(st, a, meta, n_rows, 0);
+        if (f32_served(a)) r = std::max(a.dim, a.vdim) <= 64 ? f32_go<64>(st, a, seqs, n_seq, max_n) : f32_go<128>(st, a, seqs, n_seq, max_n);
+        else plain_go<float>(st, a, meta, n_rows, 0);
         store_go<float>(st, a, meta, n_rows);
     }
     if (r != KF_OK || hipGetLastError() != hipSuccess) return abi_fail(KF_HIP_CHECK, "kf_rb_attention_prefill: launch failed");

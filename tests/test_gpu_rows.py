@@ -363,6 +363,30 @@ def test_attention_sees_exactly_its_chunk(ctx, kind, shape, how):
             assert np.abs((ref / gate)[away[0], D - 1] - 8.0) > 1.0
 
 
+@pytest.mark.parametrize("shape", [(4, 2, 64, 0, 32), (6, 1, 128, 50, 32), (2, 2, 16, 31, 8), (3, 1, 112, 0, 0)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("odd", [float("inf"), float("nan")])
+def test_f32_prompts_at_tile_edges_and_values_that_are_not_numbers(ctx, shape, odd):
+    """32-bit prompts of lengths around the 32-column, 32-key tiles, in one go and behind a ring; one token whose key and value are not numbers stays invisible to every row that does not see it
+    (a product with a weight of zero would not hide it)"""
+    H, G, D, chunk, rot = shape
+    for n in (1, 15, 31, 32, 33, 64, 97):
+        a = Attn(ctx, mix(*shape), TYPES["f32"], seed=n)
+        a.new(0), a.new(2)
+        a.check({0: a.rows(n), 2: a.rows(n + 1)})
+        a.check({0: a.rows(17), 2: a.rows(2)})
+    a, n, bad = Attn(ctx, mix(*shape), TYPES["f32"], seed=5), 75, 20
+    a.new(0)
+    x = a.rows(n)
+    clean = x.copy()
+    x[bad, H * D:(H + G) * D] = odd
+    got = a.feed({0: x})[0][0]
+    a.hist[0] = clean
+    ref = a.reference(0)
+    blind = [t for t in range(n) if t < bad or (chunk and t // chunk != bad // chunk)]
+    assert np.abs(got[blind] - ref[blind]).max() < 2e-5
+    assert not np.isfinite(got[bad]).any()
+
+
 def test_attention_long_range_in_key_ranges(ctx):
     """a decode row whose keys are cut into ranges for several workgroups (and no chunks)"""
     kind = TYPES["bf16"]
