@@ -140,8 +140,8 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     const uint16_t* gat[ROWS::GATHER ? C::NIB : 1];
     const uint16_t* const W = reinterpret_cast<const uint16_t*>(a.w);
     if constexpr (ROWS::TILED) {
-        static_assert(!AKM && C::NIA % 2 == 0, "an instruction is a tile, two tiles per row block and step");
-        const long long rb = (m0 >> 4) + wid * (C::NIA / 2), row = (long long)(a.K / 32) * 1024; /* row block of the wave's first tile; bytes of a row block */
+        static_assert(!AKM, "an instruction is a tile, two tiles per row block and step");
+        const long long rb = m0 >> 4, row = (long long)(a.K / 32) * 1024; /* row block of the first tile; bytes of a row block */
         sa.base = a.w + rb * row, sa.left = ((a.M + 15) / 16 - rb) * row, sa.step = 2048, sa.inst = row;
         sa.lane[0] = lane * 16, sa.lane[1] = lane * 16;
     } else if constexpr (AKM)
@@ -164,7 +164,10 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     // Past the last step the descriptors are empty: the load moves nothing and puts zeros where nobody reads, and the steps need no branch.
     uint32_t restA[C::NIA], restB[C::NIB];
     auto rest = [](long long left) { return (uint32_t)(left < 0 ? 0 : (left > 0xFFFFFFFFll ? 0xFFFFFFFFll : left)); };
-    auto atA = [&](int i) { return ROWS::TILED ? sa.inst * (i >> 1) + (i & 1) * 1024 : sa.inst * i; };
+    auto atA = [&](int i) {
+        const int j = wid * C::NIA + i; /* tile (row block j / 2, k-half j % 2) of the workgroup's */
+        return ROWS::TILED ? sa.inst * (j >> 1) + (j & 1) * 1024 : sa.inst * i;
+    };
 #pragma unroll
     for (int i = 0; i < C::NIA; i++) restA[i] = AKM ? G3_ALL : rest(sa.left - atA(i));
 #pragma unroll
@@ -292,6 +295,12 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     asm volatile("" ::: "memory");
 }
 
+// 256 x 256 or 192 x 256: with one big workgroup per CU a launch takes whole rounds of 256 tiles, and a round of the smaller ones takes 0.79 of a round (measured at K = 1024 - 2048), so the last
+// round's emptiness decides: 6144 x 1024 at 2608 rows 264 tiles in two rounds 66.8 us, 352 of 192 x 256 in two 53; 8704 x 2048 at 1971 rows (272 | 368) 108 | 86
+static inline bool g3_prefer_wide(int M, int n) {
+    const long by = (n + 255) / 256, rb = ((M + 255) / 256 * by + 255) / 256, rw = ((M + 191) / 192 * by + 255) / 256;
+    return 79 * rw < 97 * rb;
+}
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {
     const int q = nwg / 8, rr = nwg % 8, xcd = orig % 8;

@@ -9,6 +9,7 @@
 namespace kf {
 
 using RbBig = G3Cfg<256, 256, 8>;
+using RbWide = G3Cfg<192, 256, 8>;
 using RbSmall = G3Cfg<128, 128, 4>;
 using RbMid = G3Cfg<64, 128, 4>;
 using RbTiny = G3Cfg<64, 64, 4>;
@@ -116,7 +117,8 @@ int rb_gemm_launch(hipStream_t st, const RbProduct& q) {
         return 1;
     }
     // the measured thresholds of gemm3_launch: big tiles from 160 of them, then smaller ones that fill the chip
-    if (p.m >= 256 && p.n >= 256 && rb_tiles(p, 256, 256) >= 160) return rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
+    if (p.m >= 256 && p.n >= 256 && rb_tiles(p, 256, 256) >= 160)
+        return g3_prefer_wide(p.m, p.n) ? rb_go<RbWide, false>(st, q, rb_tiles(p, 192, 256)) : rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
     if (rb_tiles(p, 128, 128) >= 256) return rb_go<RbSmall, false>(st, q, rb_tiles(p, 128, 128));
     if (rb_tiles(p, 64, 128) >= 192) return rb_go<RbMid, false>(st, q, rb_tiles(p, 64, 128));
     return rb_go<RbTiny, false>(st, q, rb_tiles(p, 64, 64));
