@@ -1,8 +1,8 @@
 // kf_rb_linear.hip -- row-batch products y[t][m] = W[m] . x[t] for few rows (decode batches) and in 32-bit, and the ABI entry that picks the form.
 //
 // Decode batches stream the weights: a workgroup owns 16 weight rows (GATED: 16 gate and the 16 up rows that follow them), its waves take runs of 32-deep k-steps -- a
-// step's 16 x 32 weights are one stored tile, a contiguous kilobyte -- and multiply them against up to 64 token columns by v_mfma_f32_16x16x32_bf16 (A = weight rows, B = token rows, straight
-// from global memory: the activations of a decode batch are a few KB and stay in L2), the next run's weights in flight.  The waves' partial tiles meet in LDS, one thread
+// step's 16 x 32 weights are one stored tile, a contiguous kilobyte -- and multiply them against up to 64 token columns by v_mfma_f32_16x16x32_bf16 (A = weight rows, B = token rows from
+// L2, where the activations of a decode batch stay: more than 8 rows by way of RbTokens), the next run's weights in flight.  The waves' partial tiles meet in LDS, one thread
 // per output finishes it.  The RMS norm in front of a product (NORM: few rows of the 32-bit residual sum) costs no pass: the product that formed the sum left its squares
 // per 16 columns, every wave adds them up for itself and norms its token fragments as it reads them.  With experts a workgroup's columns are the pairs of one expert (UP, DOWN), or it walks all chosen experts' k-steps as one list dealt to its waves,
 // columns that did not choose an expert held at zero (SUM): an expert's rows are read once per workgroup whoever chose them.
@@ -104,11 +104,46 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
     }
 }
 
-template <int NT, bool GATED, int NW, bool NORM>
+// A run's token rows on their way to the fragments: loaded in whole lines (a row's U x 64 bytes by neighbouring lanes) a run ahead, turned round in this wave's own LDS, no barrier.  A fragment read
+// straight from memory takes half a line of each of 16 rows, and a workgroup of 32 rows reads twice as many token bytes as weight bytes: the CU's way to its L2 was the bound, not HBM.  32 rows,
+// 2048 x 6144 (128 workgroups): 16.9 -> 12.4 us; gate and up 12288 x 2048: 17.8 -> 15.5; 32768 x 2048: 43.2 -> 32.6 (134 MB: 4.1 TB/s).  Prefetching alone, without the lines, gave 1 %, and 16 waves
+// instead of 8 where workgroups are few cost 10 %.
+template <int NT, int U>
+struct RbTokens {
+    static constexpr int CH = 4 * U, ROW = 8 * CH + 8; /* 16-byte pieces of a row, a row's LDS stride in elements (16 bytes of padding: 16 rows' equal pieces lie in different banks) */
+    static constexpr int LDS = 16 * NT * ROW;
+    const uint16_t* x;
+    uint16_t* lds;
+    uint32_t off[NT * U]; /* load i's row */
+    u32x4 v[NT * U];
+    int lane;
+    __device__ __forceinline__ void load(int s, int s_end) {
+        const int c = lane % CH, st = s + c / 4 < s_end ? s + c / 4 : s_end - 1; /* steps past the end meet zero weights */
+        const uint16_t* at = x + 32 * st + 8 * (c % 4);
+#pragma unroll
+        for (int i = 0; i < NT * U; i++) v[i] = *reinterpret_cast<const u32x4*>(at + off[i]);
+    }
+    __device__ __forceinline__ int row(int i) const { return i * (64 / CH) + lane / CH; }
+    __device__ __forceinline__ void turn(u32x4 (&b)[U][NT]) {
+#pragma unroll
+        for (int i = 0; i < NT * U; i++) *reinterpret_cast<u32x4*>(lds + row(i) * ROW + 8 * (lane % CH)) = v[i];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) b[u][t] = *reinterpret_cast<const u32x4*>(lds + (16 * t + (lane & 15)) * ROW + 32 * u + 8 * (lane >> 4));
+    }
+};
+
+// TURN: the token rows go through RbTokens (rows in order, no experts); else every lane reads its fragments itself
+template <int NT, bool GATED, int NW, bool NORM, bool TURN>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
     constexpr int MG = GATED ? 2 : 1, U = NT >= 4 ? 2 : 4;
-    __shared__ float red[NW][MG][16 * NT][17]; /* [wave][block][column][row], padded */
+    static_assert(!(NORM && TURN), "normed fragments are made from the residual sum");
+    using Tokens = RbTokens<NT, U>;
+    constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * Tokens::LDS * 2 : 0;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[RED > STAGE ? RED : STAGE];
+    auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
     const int m0 = blockIdx.x * (16 * MG), nstep = p.k / 32;
     const uint16_t* W = reinterpret_cast<const uint16_t*>(p.w);
@@ -125,6 +160,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     int s = wid * U;
     rb_load_w<MG, U>(a, wr, p.k, s, nstep);
     const uint16_t* xp[NT];
+    Tokens tok;
     const float* zp = nullptr;   /* NORM: this lane's row of the residual sum, and 1 / its root mean square */
     const uint16_t* gp = nullptr;
     float rs = 0.f;
@@ -139,6 +175,14 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
             if (row == t) rs = 1.0f / sqrtf(ss / (float)p.norm_dim + p.norm_eps);
         }
         xp[0] = nullptr;
+    } else if constexpr (TURN) {
+        tok.x = X, tok.lds = reinterpret_cast<uint16_t*>(smem) + wid * Tokens::LDS, tok.lane = lane;
+#pragma unroll
+        for (int i = 0; i < NT * U; i++) {
+            const int row = tok.row(i);
+            tok.off[i] = (uint32_t)(row < p.n ? row : p.n - 1) * (uint32_t)p.ldx; /* <= 64 rows: below 2^32 (the launch sees to it) */
+        }
+        tok.load(s < nstep ? s : nstep - 1, nstep);
     } else {
 #pragma unroll
         for (int t = 0; t < NT; t++) { /* columns past the end repeat a row: their outputs are not stored */
@@ -178,6 +222,10 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
                     *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(const_cast<void*>(p.x)) + at) = b[u][0];
                 }
             }
+        } else if constexpr (TURN) {
+            tok.turn(b);
+            if (s + NW * U < nstep) tok.load(s + NW * U, nstep); /* wave-uniform */
+            rb_load_w<MG, U>(an, wr, p.k, s + NW * U, nstep);
         } else {
             rb_load_x<NT, U, false>(b, xp, s, nstep);
             rb_load_w<MG, U>(an, wr, p.k, s + NW * U, nstep);
@@ -188,6 +236,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
 #pragma unroll
             for (int g = 0; g < MG; g++) a[u][g] = an[u][g];
     }
+    if constexpr (TURN) __syncthreads(); /* the token rows make way */
     rb_stream_finish<NT, MG, NW>(q, acc, red, list, m0, tid);
 }
 
@@ -249,14 +298,20 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
 }
 template <int NT, int NW>
 static void stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
-    if (q.p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
-    else if (q.p.epilogue == KF_RB_GATED) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false>), grid, dim3(64 * NW), 0, st, q);
-    else hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false>), grid, dim3(64 * NW), 0, st, q);
+    const kf_rb_product& p = q.p;
+    // whole lines for more than 8 rows in order: below, a fragment's 16 half lines are few distinct ones and the way round costs more than it saves (one token of a 2048-wide model: 1.79 -> 1.87 ms
+    // over four steps; 6 rows 2.04 -> 2.08; 14 rows 2.42 -> 2.35; 32 rows 4.62 -> 4.23); experts' tiles are mostly padding, which repeats row 0 (32 rows of 64 experts: 10.15 -> 10.36)
+    const bool turn = p.mode == KF_RB_ALL && p.n > 8 && p.ldx <= (1 << 24), gated = p.epilogue == KF_RB_GATED;
+    if (p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
+    else if (gated && turn) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
+    else if (gated) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
+    else if (turn) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
+    else hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
 }
 template <int NW>
 static void norm_stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
-    if (q.p.epilogue == KF_RB_GATED) hipLaunchKernelGGL((rb_stream_kernel<1, true, 4, true>), grid, dim3(256), 0, st, q);
-    else hipLaunchKernelGGL((rb_stream_kernel<1, false, NW, true>), grid, dim3(64 * NW), 0, st, q);
+    if (q.p.epilogue == KF_RB_GATED) hipLaunchKernelGGL((rb_stream_kernel<1, true, 4, true, false>), grid, dim3(256), 0, st, q);
+    else hipLaunchKernelGGL((rb_stream_kernel<1, false, NW, true, false>), grid, dim3(64 * NW), 0, st, q);
 }
 int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const kf_rb_product& p = q.p;

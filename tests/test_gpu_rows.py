@@ -148,6 +148,19 @@ def test_product_many_tiles(ctx):
         assert (y - x.float() @ w.float().T).abs().max().item() < 1e-4
 
 
+@pytest.mark.parametrize("n", [8, 9, 16, 25, 33, 49, 64])
+@pytest.mark.parametrize("k", [576, 1088, 2112])
+def test_decode_product_of_several_runs(ctx, n, k):
+    """rows read in whole lines and turned round: several runs of steps a wave, a ragged last one, rows past the last; the bound is that of a k-term fp32 sum"""
+    g = torch.Generator().manual_seed(n + k)
+    m, w, x = 128, dev(torch.randn(128, k, generator=g) / k ** 0.5, torch.bfloat16), dev(torch.randn(n, k + 8, generator=g), torch.bfloat16)
+    y, ws = torch.full((n + 1, m), 7.0, device="cuda"), stored(w)
+    p = L.RbProduct(ws.data_ptr(), x.data_ptr(), y.data_ptr(), None, k + 8, m, 0, L.BF16, m, k, n, L.RB_STORE_F32, 0, L.RB_ALL, 0.0, None)
+    L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+    a, b = f64(x)[:, :k], f64(w)
+    assert (np.abs(f64(y)[:n] - a @ b.T) <= k * 2.0 ** -24 * (np.abs(a) @ np.abs(b).T)).all() and (y[n] == 7.0).all()
+
+
 def test_product_refuses_what_it_cannot_do(ctx):
     t = torch.zeros(64, 64, device="cuda")
     ok = dict(w=t.data_ptr(), x=t.data_ptr(), y=t.data_ptr(), res=t.data_ptr(), ldx=64, ldy=64, ldr=64, type=L.F32, m=64, k=64, n=2, epilogue=L.RB_STORE, act=0, mode=L.RB_ALL, alpha=1.0)
