@@ -588,22 +588,26 @@ __global__ void __launch_bounds__(256 * KH, HD <= 128 ? 2 : 1) rb_attn_prefill_k
         }
 }
 
-// decode: grid (n_kv * column blocks of 32 query heads, key ranges of `span` keys, rows).  raw is not prepared: q and the new key are normed and rotated here while the first
+// decode: grid (n_kv * column blocks of 32 query heads, key ranges, rows).  A row's keys are dealt to the ranges evenly by its own position: the launch only knows a bound that holds for the graph it
+// is captured in, up to twice the keys there are, and with ranges cut from the bound 32 rows at position 1024 had all their keys in the first of two ranges and half the workgroups
+// returned at once.  A second range costs about 10 us wherever it is cheap to avoid (256 -> 257 keys of 32 rows: 15.2 -> 25.4 us: parts written through, an arrival counter, three trips to memory in a
+// chain), so a workgroup has eight waves, whose parts meet in LDS, before a row is cut into ranges.
+// raw is not prepared: q and the new key are normed and rotated here while the first
 // tiles are on their way; the workgroup whose range holds the row's position patches the new key and value into its tile and puts them into the ring.
-template <int HD>
-__device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const int32_t* __restrict__ meta, int span, int n_range, int block, int range, int rr, int n_rows, unsigned char* smem_raw) {
+template <int HD, int NW>
+__device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const int32_t* __restrict__ meta, int n_range, int block, int range, int rr, int n_rows, unsigned char* smem_raw) {
     using Tile = RbTile<HD>;
     constexpr int KS = Tile::KS, VS = Tile::VS, CH = HD / 8, WAVE_EL = 32 * (KS + VS), NREG = Tile::NDB * 16;
     const int pos = meta[KF_RB_META * rr], slot = meta[KF_RB_META * rr + 1];
     if (pos < 0) return; /* workgroup-uniform, like the next */
-    const int first = rb_first_key(pos, a), k_lo = first + range * span, k_hi = k_lo + span - 1 < pos ? k_lo + span - 1 : pos;
+    const int first = rb_first_key(pos, a), even = (pos - first + n_range) / n_range, span = even <= 64 * NW ? 64 * NW : (even + 31) & ~31, k_lo = first + range * span, k_hi = k_lo + span - 1 < pos ? k_lo + span - 1 : pos;
     if (k_lo > pos) return;
     const int GQ = a.n_head / a.n_kv, ncb = (GQ + 31) / 32, g = block / ncb, cb = block % ncb, col0 = cb * 32, ncol = GQ - col0 < 32 ? GQ - col0 : 32;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r = lane & 31, h = lane >> 5;
     uint16_t* s_new = reinterpret_cast<uint16_t*>(smem_raw);             /* the new key, the new value: [2][HD] */
-    uint16_t* s_kv = s_new + 2 * HD;                                     /* [4 waves] [32][KS] + [32][VS]; before the walk: */
+    uint16_t* s_kv = s_new + 2 * HD;                                     /* [NW waves] [32][KS] + [32][VS]; before the walk: */
     uint16_t* s_q = s_kv;                                                /* [32][KS] */
-    float* s_buf = reinterpret_cast<float*>(s_q + 32 * KS);              /* [4][HD] */
+    float* s_buf = reinterpret_cast<float*>(s_q + 32 * KS);              /* [NW][HD] */
     __shared__ int s_last;
     const uint16_t* raw = reinterpret_cast<const uint16_t*>(a.raw) + (size_t)rr * a.ldraw;
     const size_t base = (size_t)slot * a.slot_stride + (size_t)g * a.head_stride;
@@ -623,9 +627,9 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
     };
     int k0 = k_lo + wid * 32;
     if (k0 <= k_hi) tload(k0);
-    for (int i = tid; i < 32 * KS / 8; i += 256) reinterpret_cast<u32x4*>(s_q)[i] = u32x4{0, 0, 0, 0};
+    for (int i = tid; i < 32 * KS / 8; i += 64 * NW) reinterpret_cast<u32x4*>(s_q)[i] = u32x4{0, 0, 0, 0};
     __syncthreads();
-    for (int u = wid; u <= ncol; u += 4) {
+    for (int u = wid; u <= ncol; u += NW) {
         if (u < ncol) {
             rb_prep_head(raw + (size_t)(g * GQ + col0 + u) * a.dim, s_q + u * KS, reinterpret_cast<const uint16_t*>(a.q_norm), a.unit, a.rope, a.rot_dims, a.dim, pos, a.eps, s_buf + wid * HD, lane);
         } else if (k_hi == pos) {
@@ -651,7 +655,7 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
     Tile T;
     T.init();
     const float sc2 = a.scale * RB_LOG2E;
-    for (; k0 <= k_hi; k0 += 128) {
+    for (; k0 <= k_hi; k0 += 32 * NW) {
         __builtin_amdgcn_wave_barrier(); /* the tile is this wave's own: its LDS accesses are in order, only the compiler has to be told */
 #pragma unroll
         for (int i = 0; i < CPT; i++) {
@@ -660,7 +664,7 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
             *reinterpret_cast<u32x4*>(ks + key * KS + d) = own ? *reinterpret_cast<const u32x4*>(s_new + d) : kr[i];
             *reinterpret_cast<u32x4*>(vs + key * VS + d) = own ? *reinterpret_cast<const u32x4*>(s_new + HD + d) : vr[i];
         }
-        if (k0 + 128 <= k_hi) tload(k0 + 128);
+        if (k0 + 32 * NW <= k_hi) tload(k0 + 32 * NW);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -668,9 +672,9 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
-    // the four waves' partial softmaxes: registers lane-major per wave, every wave finishes a quarter of them
+    // the waves' partial softmaxes: registers lane-major per wave, every wave finishes its share of them
     __syncthreads();
-    float* ex = reinterpret_cast<float*>(s_kv); /* [4][NREG + 2][64] */
+    float* ex = reinterpret_cast<float*>(s_kv); /* [NW][NREG + 2][64] */
 #pragma unroll
     for (int db = 0; db < Tile::NDB; db++)
 #pragma unroll
@@ -678,11 +682,11 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
     ex[((size_t)wid * (NREG + 2) + NREG) * 64 + lane] = T.M;
     ex[((size_t)wid * (NREG + 2) + NREG + 1) * 64 + lane] = xsum32(T.l);
     __syncthreads();
-    float f[4], M = -__builtin_inff(), L = 0.f;
+    float f[NW], M = -__builtin_inff(), L = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; w++) M = fmaxf(M, ex[((size_t)w * (NREG + 2) + NREG) * 64 + lane]); /* wave 0 has seen a key: finite */
+    for (int w = 0; w < NW; w++) M = fmaxf(M, ex[((size_t)w * (NREG + 2) + NREG) * 64 + lane]); /* wave 0 has seen a key: finite */
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
+    for (int w = 0; w < NW; w++) {
         f[w] = rb_exp2(ex[((size_t)w * (NREG + 2) + NREG) * 64 + lane] - M);
         L += f[w] * ex[((size_t)w * (NREG + 2) + NREG + 1) * 64 + lane];
     }
@@ -693,12 +697,12 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
     float* parts = reinterpret_cast<float*>(a.scratch) + RB_CNT_STRIDE * (size_t)n_rows * a.n_head; /* behind the arrival counters: [row][head][range][vdim + 2] */
     float* part = parts + (((size_t)rr * a.n_head + head) * n_range + range) * (a.vdim + 2);
     const float inv = a.out_scale * rb_softmax_factor(M, L, a.sink);
-    for (int q = wid; q < Tile::NDB * 4 && r < ncol; q += 4) { /* a quad of registers = four consecutive d */
+    for (int q = wid; q < Tile::NDB * 4 && r < ncol; q += NW) { /* a quad of registers = four consecutive d */
         const int d = 8 * q + 4 * h;
         if (d >= a.vdim) continue;
         f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < 4; w++)
+        for (int w = 0; w < NW; w++)
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = fmaf(f[w], ex[((size_t)w * (NREG + 2) + 4 * q + j) * 64 + lane], v[j]);
         if (n_used > 1) {
@@ -722,7 +726,7 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
     __syncthreads();
     if (!s_last) return;
     if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int c = wid; c < ncol; c += 4) {
+    for (int c = wid; c < ncol; c += NW) {
         const int hd = g * GQ + col0 + c;
         const float* p = parts + ((size_t)rr * a.n_head + hd) * n_range * (a.vdim + 2);
         const bool mine = lane < n_used;
@@ -754,26 +758,27 @@ __device__ __forceinline__ void rb_attn_decode(const kf_rb_attention& a, const i
         }
     }
 }
-template <int HD>
-__global__ void __launch_bounds__(256) rb_attn_decode_kernel(const kf_rb_attention a, const int32_t* __restrict__ meta, int span, int n_range) {
+template <int HD, int NW>
+__global__ void __launch_bounds__(64 * NW, HD <= 128 ? 2 : 1) rb_attn_decode_kernel(const kf_rb_attention a, const int32_t* __restrict__ meta, int n_range) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    rb_attn_decode<HD>(a, meta, span, n_range, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, smem_raw);
+    rb_attn_decode<HD, NW>(a, meta, n_range, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, smem_raw);
 }
 // a layer's decayed sum (its heads first) and its attention in one launch: neither waits for the other
 template <int HD>
-__global__ void __launch_bounds__(256) rb_attn_decay_decode_kernel(const kf_rb_attention a, const kf_rb_decay d, const int32_t* __restrict__ meta, int span, int n_range) {
+__global__ void __launch_bounds__(256, HD <= 128 ? 2 : 1) rb_attn_decay_decode_kernel(const kf_rb_attention a, const kf_rb_decay d, const int32_t* __restrict__ meta, int n_range) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int block = (int)blockIdx.x - d.n_head, blocks = ((int)gridDim.x - d.n_head) / n_range;
     if (block < 0) rc_decay_step<uint16_t, 256, 16>(d, meta, blockIdx.x, blockIdx.y, gridDim.y, reinterpret_cast<float*>(smem_raw));
-    else rb_attn_decode<HD>(a, meta, span, n_range, block % blocks, block / blocks, blockIdx.y, gridDim.y, smem_raw);
+    else rb_attn_decode<HD, 4>(a, meta, n_range, block % blocks, block / blocks, blockIdx.y, gridDim.y, smem_raw);
 }
 constexpr int RB_MAX_RANGES = 32;
-static void decode_ranges(int n_rows, int n_kv, int keys, int& span, int& n_range) {
-    n_range = (keys + 255) / 256; /* a range is at least two tiles per wave */
-    const int want = (512 + n_rows * n_kv - 1) / (n_rows * n_kv); /* two workgroups per CU: one round */
-    n_range = std::max(1, std::min(n_range, std::min(want, RB_MAX_RANGES)));
-    span = ((keys + n_range - 1) / n_range + 127) / 128 * 128;
-    n_range = (keys + span - 1) / span;
+// Eight waves a workgroup (one per CU) where four-wave ranges would lie two to a CU; a few rows' ranges have a CU each and stay four waves (one row of 16 heads, 1024 keys: 13.1 us against 14.6), and from
+// 512 workgroups on two of four waves share a CU.  16 heads of 128 on 8, before -> now: 16 rows of 1024 keys 27.7 -> 20.7 us, 32 rows of 257 24.3 -> 15.2, of 1024 41.7 -> 32.1 (4.2 TB/s), 48 rows of 512
+// 43.3 -> 34.6 (two of four waves a CU: 26.4, but a long row among short ones would be walked by four waves instead of eight), 64 rows of 2048 104.9 -> 98.0 (5.5 TB/s): besides the ranges, the register bound that lets eight waves into a CU (328 registers let in four).
+static bool decode_wide(int hd, int wgs, int keys) { return hd <= 128 && wgs < 512 && keys > 256 && (long)wgs * ((keys + 255) / 256) > 256; }
+static int decode_ranges(int wgs, int keys, bool wide) {
+    const int least = wide ? 512 : 256, want = ((wide ? 256 : 512) + wgs - 1) / wgs; /* least: two tiles per wave; want: the chip filled once */
+    return std::max(1, std::min((keys + least - 1) / least, std::min(want, RB_MAX_RANGES)));
 }
 template <class K>
 static int big_lds(K kernel, size_t smem, int& done) {
@@ -800,26 +805,41 @@ static int prefill_go(hipStream_t st, const kf_rb_attention& a, const int32_t* s
     }
     return prefill_kh<HD, 1>(st, a, seqs, grid);
 }
-template <int HD>
-static int decode_go(hipStream_t st, const kf_rb_attention& a, const kf_rb_decay* d, const int32_t* meta, int n_rows, int span, int n_range) {
-    constexpr size_t tiles = 4 * 2 * 32 * (size_t)(RbTile<HD>::KS + RbTile<HD>::VS), merge = 4 * (size_t)(RbTile<HD>::NDB * 16 + 2) * 256;
-    constexpr size_t smem = 4 * HD + (tiles > merge ? tiles : merge);
-    static_assert(32 * RbTile<HD>::KS * 2 + 16 * HD <= tiles, "queries in the tiles' place");
+template <int HD, int NW>
+constexpr size_t decode_lds() {
+    constexpr size_t tiles = NW * 2 * 32 * (size_t)(RbTile<HD>::KS + RbTile<HD>::VS), merge = NW * (size_t)(RbTile<HD>::NDB * 16 + 2) * 256;
+    static_assert(32 * RbTile<HD>::KS * 2 + 4 * NW * HD <= tiles, "queries in the tiles' place");
+    return 4 * HD + (tiles > merge ? tiles : merge);
+}
+template <int HD, int NW>
+static int decode_nw(hipStream_t st, const kf_rb_attention& a, const int32_t* meta, dim3 grid) {
+    constexpr size_t smem = decode_lds<HD, NW>();
     static_assert(smem <= 160 * 1024, "LDS");
+    static int done = 0;
+    if (big_lds(rb_attn_decode_kernel<HD, NW>, smem, done)) return KF_HIP_CHECK;
+    hipLaunchKernelGGL((rb_attn_decode_kernel<HD, NW>), grid, dim3(64 * NW), smem, st, a, meta, (int)grid.y);
+    return KF_OK;
+}
+template <int HD>
+static int decode_go(hipStream_t st, const kf_rb_attention& a, const kf_rb_decay* d, const int32_t* meta, int n_rows, int keys) {
     const int blocks = a.n_kv * ((a.n_head / a.n_kv + 31) / 32);
+    const bool wide = !d && decode_wide(HD, (int)std::min((long)n_rows * blocks, 1l << 20), keys);
+    const int n_range = decode_ranges((int)std::min((long)n_rows * blocks, 1l << 20), keys, wide);
+    if (n_range > 1 && !a.scratch) return KF_INVALID_ARGS;
     if (d) {
         static int done = 0;
-        const size_t both = std::max(smem, rc_decay_step_lds(d->dim, d->vdim, 256));
+        const size_t both = std::max(decode_lds<HD, 4>(), rc_decay_step_lds(d->dim, d->vdim, 256));
         if (both > 150 * 1024) return 1;
         if (!done && hipFuncSetAttribute((const void*)rb_attn_decay_decode_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess) return KF_HIP_CHECK;
         done = 1;
-        hipLaunchKernelGGL(rb_attn_decay_decode_kernel<HD>, dim3(d->n_head + blocks * n_range, n_rows), dim3(256), both, st, a, *d, meta, span, n_range);
+        hipLaunchKernelGGL(rb_attn_decay_decode_kernel<HD>, dim3(d->n_head + blocks * n_range, n_rows), dim3(256), both, st, a, *d, meta, n_range);
         return KF_OK;
     }
-    static int done = 0;
-    if (big_lds(rb_attn_decode_kernel<HD>, smem, done)) return KF_HIP_CHECK;
-    hipLaunchKernelGGL(rb_attn_decode_kernel<HD>, dim3(blocks, n_range, n_rows), dim3(256), smem, st, a, meta, span, n_range);
-    return KF_OK;
+    const dim3 grid(blocks, n_range, n_rows);
+    if constexpr (HD <= 128) {
+        if (wide) return decode_nw<HD, 8>(st, a, meta, grid);
+    }
+    return decode_nw<HD, 4>(st, a, meta, grid);
 }
 static bool mfma_served(const kf_rb_attention& a, int n_rows) {
     return a.type == KF_BF16 && (int64_t)n_rows * a.ldraw < ((int64_t)1 << 30) && (int64_t)a.cache_rows * a.n_kv * std::max(a.dim, a.vdim) < ((int64_t)1 << 30) && a.dim % 8 == 0 && a.dim <= 256 && a.vdim % 8 == 0 && a.vdim <= 256 && a.v_col % 8 == 0 && a.gate_col % 4 == 0 && a.ldraw % 8 == 0 && a.ldout % 4 == 0 && a.slot_stride % 8 == 0 && a.head_stride % 8 == 0;
@@ -905,14 +925,13 @@ static int attention_decode(kf_ctx* c, const kf_rb_attention* ap, const kf_rb_de
     hipStream_t st = c->stream;
     int r = KF_OK;
     if (mfma_served(a, n_rows)) {
-        int keys = max_pos + 1, span, n_range;
+        int keys = max_pos + 1;
         const int seen = a.window > 0 ? a.window : a.chunk;
         if (seen > 0 && keys > seen) keys = seen;
-        decode_ranges(n_rows, a.n_kv * ((a.n_head / a.n_kv + 31) / 32), keys, span, n_range);
-        if (n_range > 1 && !a.scratch) return abi_fail(KF_INVALID_ARGS, "%s: null scratch", who);
-#define RB_CALL(HD) decode_go<HD>(st, a, d, meta, n_rows, span, n_range)
+#define RB_CALL(HD) decode_go<HD>(st, a, d, meta, n_rows, keys)
         r = RB_BY_DIM(RB_CALL);
 #undef RB_CALL
+        if (r == KF_INVALID_ARGS) return abi_fail(KF_INVALID_ARGS, "%s: null scratch", who);
     } else if (a.type == KF_BF16) {
         prep_go<uint16_t>(st, a, meta, n_rows, true);
         plain_go<uint16_t>(st, a, meta, n_rows, 1);

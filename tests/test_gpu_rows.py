@@ -410,6 +410,40 @@ def test_attention_long_range_in_key_ranges(ctx):
         a.check({0: a.rows(1), 1: a.rows(1)}, decode=True)
 
 
+@pytest.mark.parametrize("n,G,D,top", [(2, 2, 128, 600), (130, 2, 128, 300), (70, 2, 64, 1100), (128, 2, 128, 2047), (260, 2, 64, 257), (140, 2, 192, 300)])
+@pytest.mark.parametrize("window", [0, 290])
+def test_decode_deals_each_row_its_own_keys(ctx, n, G, D, top, window):
+    """ragged rows under one bound: key ranges of four and of eight waves, cut by the row's own position; inputs are exact in bf16, the weights are held to 2^-16, so only the result's rounding is left"""
+    g = torch.Generator().manual_seed(n + D)
+    H, rows = 2 * G, top + 1
+    kc, vc = (torch.randn(n, G, rows, D, generator=g).bfloat16().cuda() for _ in range(2))
+    ld = (H + 2 * G) * D
+    raw, out = torch.randn(n, ld, generator=g).bfloat16().cuda(), torch.full((n, H * D), 7.0, dtype=torch.bfloat16, device="cuda")
+    pos = torch.randint(0, top + 1, (n,), generator=g)
+    edge = [top, 0, 31, 32, 255, 256, 257, -1][:min(n, 8)]
+    pos[:len(edge)] = torch.tensor(edge)
+    meta = torch.stack([pos, torch.arange(n), pos, pos], 1).int().cuda()
+    sc = torch.zeros(ctx.hip.kf_rb_attention_scratch(n, H, D) // 4, device="cuda")
+    a = L.RbAttention(type=L.BF16, n_head=H, n_kv=G, dim=D, cache_rows=rows, scale=D ** -0.5, eps=1e-5, v_col=(H + G) * D, window=window, k_cache=kc.data_ptr(), v_cache=vc.data_ptr(), ldraw=ld, ldout=H * D, slot_stride=G * rows * D,
+                      head_stride=rows * D, raw=raw.data_ptr(), out=out.data_ptr(), scratch=sc.data_ptr())
+    k64, v64 = kc.double(), vc.double()
+    for bound in (top, 2 * top + 1):
+        L.check(ctx.hip.kf_rb_attention_decode(ctx.h, C.byref(a), meta.data_ptr(), n, bound))
+        torch.cuda.synchronize()
+        for i, at in enumerate(pos.tolist()):
+            if at < 0:
+                assert (out[i] == 7.0).all()
+                continue
+            lo = max(0, at + 1 - window) if window else 0
+            k, v = k64[i, :, lo:at + 1].clone(), v64[i, :, lo:at + 1].clone()
+            new = raw[i].double()
+            k[:, -1], v[:, -1] = new[H * D:(H + G) * D].view(G, D), new[(H + G) * D:].view(G, D)
+            w = torch.softmax((new[:H * D].view(G, 2, 1, D) * k[:, None]).sum(-1) * D ** -0.5, -1)
+            want, size = (w[..., None] * v[:, None]).sum(2), (w[..., None] * v[:, None].abs()).sum(2)
+            assert ((out[i].double().view(G, 2, D) - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * size).all(), (i, at, bound)
+    assert not sc[:32].any()
+
+
 def test_attention_refuses(ctx):
     a = Attn(ctx, mix(4, 2, 64, 24, 32), TYPES["bf16"])
     t = torch.zeros(4096, device="cuda")
