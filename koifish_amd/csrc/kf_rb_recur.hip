@@ -932,9 +932,10 @@ __global__ void __launch_bounds__(256) rb_decay_states_kernel(const kf_rb_decay 
     for (int j = 0; j < 4; j++)
         if (v < vs && d + j < dim) S1[(size_t)(d + j) * vs + v] = S[j];
 }
-// 128 queries of a head: a wave 32 of them, one per lane pair
+// 128 queries of a head: a wave 32 of them, one per lane pair.  Two waves a SIMD: left alone the compiler takes 320 registers and one wave waits out every LDS and memory latency (16 heads of 128, 8190
+// tokens: 119 -> 78 us at 254 registers, nothing spilled).
 template <int HD>
-__global__ void __launch_bounds__(256) rb_decay_out_kernel(const kf_rb_decay a, const uint16_t* __restrict__ planes, float* __restrict__ o, const int32_t* __restrict__ seqs) {
+__global__ void __launch_bounds__(256, 2) rb_decay_out_kernel(const kf_rb_decay a, const uint16_t* __restrict__ planes, float* __restrict__ o, const int32_t* __restrict__ seqs) {
     using Stage = RcStage<HD>;
     constexpr int NS = HD / 16, NB = HD / 32;
     __shared__ __attribute__((aligned(16))) uint16_t lds[2][32 * (Stage::KS + Stage::VS)];
