@@ -823,9 +823,10 @@ static int decode_nw(hipStream_t st, const kf_rb_attention& a, const int32_t* me
 template <int HD>
 static int decode_go(hipStream_t st, const kf_rb_attention& a, const kf_rb_decay* d, const int32_t* meta, int n_rows, int keys) {
     const int blocks = a.n_kv * ((a.n_head / a.n_kv + 31) / 32);
-    const bool wide = !d && decode_wide(HD, (int)std::min((long)n_rows * blocks, 1l << 20), keys);
-    const int n_range = decode_ranges((int)std::min((long)n_rows * blocks, 1l << 20), keys, wide);
-    if (n_range > 1 && !a.scratch) return KF_INVALID_ARGS;
+    const int wgs = (int)std::min((long)n_rows * blocks, 1l << 20);
+    if (!a.scratch && decode_ranges(wgs, keys, false) > 1) return KF_INVALID_ARGS; /* whichever form it takes: a caller lends the scratch by the four-wave rule */
+    const bool wide = !d && decode_wide(HD, wgs, keys);
+    const int n_range = decode_ranges(wgs, keys, wide);
     if (d) {
         static int done = 0;
         const size_t both = std::max(decode_lds<HD, 4>(), rc_decay_step_lds(d->dim, d->vdim, 256));
