@@ -152,7 +152,7 @@ int kf_set_scratch(kf_ctx* ctx, void* scratch, size_t bytes);
  * time they meet a weight (or a stacked Q | K | V / interleaved gate | up set) and find it there afterwards -- same values, same tile kernels, no dequantise
  * launches, and kf_linear takes the bf16 tile kernels from 320 rows (o_proj / down_proj of a prompt: 64 x 128 / 64 x 64 tiles of kf_gemm3.hip, in k-pieces when a
  * kf_set_scratch workspace of kf_resident_scratch_bytes() is lent).
- * Copies are keyed by the weights' data pointers: the caller promises the weights do not change while the arena holds them (inference; after a weight update
+ * Copies are keyed by the weights' data pointers and shapes: the caller promises the weights do not change while the arena holds them (inference; after a weight update
  * call kf_set_dequant_arena again -- it forgets every copy).  arena: device memory, 16-byte aligned, the caller's; NULL switches the feature off; when it is
  * full, further weights go through the scratch as before.  kf_dequant_arena_used: bytes filled so far.  Not while capturing. */
 int kf_set_dequant_arena(kf_ctx* ctx, void* arena, size_t bytes);

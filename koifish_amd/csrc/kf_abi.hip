@@ -132,24 +132,18 @@ static int deq_copies(kf_ctx* c, int n_w, const kf_weight* const* w, int form, c
     size_t need = 0;
     for (int i = 0; i < n_w; i++) need += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
     if (resident) *resident = false;
-    for (const kf_ctx::DeqCopy& e : c->call) {
-        bool same = e.form == form;
-        for (int i = 0; i < 3; i++) same = same && e.key[i] == (i < n_w ? w[i]->data : nullptr);
-        if (same) {
+    for (const kf_ctx::DeqCopy& e : c->call)
+        if (e.of(n_w, w, form)) {
             *out = (const uint16_t*)((const char*)c->scratch + e.off);
             return KF_OK;
         }
-    }
     if (c->arena) {
-        for (const kf_ctx::DeqCopy& e : c->copies) {
-            bool same = e.form == form;
-            for (int i = 0; i < 3; i++) same = same && e.key[i] == (i < n_w ? w[i]->data : nullptr);
-            if (same) {
+        for (const kf_ctx::DeqCopy& e : c->copies)
+            if (e.of(n_w, w, form)) {
                 *out = (const uint16_t*)((const char*)c->arena + e.off);
                 if (resident) *resident = true;
                 return KF_OK;
             }
-        }
     }
     const bool keep = c->arena && !c->capturing && c->arena_used + need <= c->arena_bytes; /* a captured launch would replay the fill with every replay: those use the scratch */
     char* dst = keep ? (char*)c->arena + c->arena_used : c->scratch_tail();
@@ -162,10 +156,7 @@ static int deq_copies(kf_ctx* c, int n_w, const kf_weight* const* w, int form, c
         off += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
     }
     if (keep) {
-        kf_ctx::DeqCopy e;
-        for (int i = 0; i < 3; i++) e.key[i] = i < n_w ? w[i]->data : nullptr;
-        e.form = form, e.off = c->arena_used;
-        c->copies.push_back(e);
+        c->copies.emplace_back(n_w, w, form, c->arena_used);
         c->arena_used += need;
         if (resident) *resident = true;
     }
@@ -421,7 +412,7 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         return kf_linear(c, &wb, x, y, bias, nTok, alpha, beta, epilogue, residual);
     }
     for (const kf_ctx::DeqCopy& e : c->call) {
-        if (e.form != DEQ_STACK || e.key[0] != w->data || e.key[1] || nTok < KF_LAYER_COPIES_MIN) continue; /* a copy of this matrix alone (kf_layer_copies) */
+        if (!e.of(1, &w, DEQ_STACK) || nTok < KF_LAYER_COPIES_MIN) continue; /* a copy of this matrix alone (kf_layer_copies) */
         kf_weight wb;
         memset(&wb, 0, sizeof(wb));
         wb.data = (char*)c->scratch + e.off, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
@@ -856,9 +847,7 @@ int kf_layer_copies(kf_ctx* c, const kf_weight* wq, const kf_weight* wk, const k
     int ilv_n[7], ilv_i[7];
     size_t off = 0;
     for (int g = 0, i = 0; g < 4; g++) {
-        kf_ctx::DeqCopy e;
-        e.form = form[g], e.off = off;
-        for (int j = 0; j < 3; j++) e.key[j] = j < n_w[g] ? w[i + j]->data : nullptr;
+        const kf_ctx::DeqCopy e(n_w[g], w + i, form[g], off);
         uint16_t* const group = (uint16_t*)((char*)c->scratch + off);
         for (int j = 0; j < n_w[g]; j++, i++) {
             ilv_n[i] = form[g] == DEQ_ILV ? n_w[g] : 1, ilv_i[i] = form[g] == DEQ_ILV ? j : 0;

@@ -16,12 +16,21 @@ struct kf_ctx {
     int canonical;    /* 1: the decode kernels sum in the canonical order of oracle/kf_oracle.c sections 4c / 6 (bit-exact against the oracle; the default); 0: v_dot2c / fp32 forms */
     void* scratch;    /* caller-owned workspace of kf_linear (kf_set_scratch): AWQ slice partials, or a weight dequantised to bf16 */
     size_t scratch_bytes;
-    // resident GetDataX copies for token batches (kf_set_dequant_arena): caller-owned memory, filled on first use, keyed by the data pointers of the matrices a route
-    // multiplies in one launch and the form they are laid out in (DEQ_STACK: back to back; DEQ_ILV: gate | up interleaved in blocks of 16 rows)
+    // resident GetDataX copies for token batches (kf_set_dequant_arena): caller-owned memory, filled on first use, keyed by the data pointers and shapes of the matrices a route
+    // multiplies in one launch and the form they are laid out in (DEQ_STACK: back to back; DEQ_ILV: gate | up interleaved in blocks of 16 rows).  A descriptor of a matrix's
+    // first rows has the matrix's pointer, but the rows behind its own lie elsewhere in a set: another key.
     struct DeqCopy {
         const void* key[3];
-        int form;
+        int rows[3], cols, form;
         size_t off;
+        DeqCopy(int n_w, const kf_weight* const* w, int form_, size_t off_) : cols(w[0]->ne1), form(form_), off(off_) {
+            for (int i = 0; i < 3; i++) key[i] = i < n_w ? w[i]->data : nullptr, rows[i] = i < n_w ? w[i]->ne0 : 0;
+        }
+        bool of(int n_w, const kf_weight* const* w, int form_) const {
+            bool same = form == form_;
+            for (int i = 0; i < 3; i++) same = same && key[i] == (i < n_w ? w[i]->data : nullptr) && (i >= n_w || (rows[i] == w[i]->ne0 && cols == w[i]->ne1));
+            return same;
+        }
     };
     void* arena;
     size_t arena_bytes, arena_used;

@@ -75,3 +75,26 @@ def test_not_served_is_left_alone(ctx):
     assert ctx.hip.kf_layer_copies_bytes(*mixed, 2047) == 0
     odd = [C.byref(d) for d in _layer(ctx, 256, 384, 128, 512)[1]]   # rows no multiple of 256: the stacked route does not take them
     assert ctx.hip.kf_layer_copies_bytes(*odd, 2047) == 0
+
+
+
+def test_a_set_with_a_matrix_of_fewer_rows_is_another_set(ctx):
+    """the first 256 rows of q have q's pointer: stacked with k and v they are not the set that resident copies hold"""
+    n, dim = 2047, 256
+    ws = [ctx.quantize((torch.randn(m, dim, device=ctx.device) * 0.05).bfloat16(), L.F8E5M2) for m in (2048, 1024, 1024)]
+    x = torch.randn(n, dim, device=ctx.device).bfloat16()
+    arena = torch.zeros((4096 + 2304) * dim * 2 + 4096, dtype=torch.uint8, device=ctx.device)
+    try:
+        assert ctx.hip.kf_set_dequant_arena(ctx.h, C.c_void_p(arena.data_ptr()), C.c_size_t(arena.numel())) == 0
+        for rows in (2048, 256):
+            descs = [w.desc() for w in ws]
+            descs[0].ne0 = rows
+            y = [torch.zeros(n, m, device=ctx.device, dtype=torch.bfloat16) for m in (rows, 1024, 1024)]
+            w3, y3 = (C.POINTER(L.Weight) * 3)(*[C.pointer(d) for d in descs]), (C.c_void_p * 3)(*[t.data_ptr() for t in y])
+            assert ctx.hip.kf_linear_multi(ctx.h, 3, w3, x.data_ptr(), y3, n) == 0, ctx.hip.kf_last_error()
+            for out, w in zip(y, ws):
+                want = x.float() @ ctx.dequant(w).float()[: out.shape[1]].t()
+                assert float((out.float() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())   # fp32 sums, one bf16 rounding
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
