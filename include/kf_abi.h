@@ -161,7 +161,7 @@ size_t kf_resident_scratch_bytes(void); /* a kf_set_scratch workspace of at leas
 /* bf16 copies of ONE layer's seven matrices for the token-batch calls that follow: kf_layer_copies dequantises them with one launch into the front of the kf_set_scratch workspace
  * (kf_layer_copies_bytes: how large it has to be, 0: not for this layer or batch) when they are 4-bit in groups of 128, the batch has >= 320 rows and no arena is lent; the routes of
  * kf_linear, kf_qkv_rope_batch / _seqs, kf_linear_multi and kf_gateup_swiglu_batch then multiply the copies.  Returns 1 when it does nothing.  The copies hold until kf_layer_copies_end,
- * the next kf_layer_copies or kf_set_scratch; the caller does not change these weights in between. */
+ * the next kf_layer_copies or kf_set_scratch; the caller does not change these weights in between.  Launches captured meanwhile (kf_graph_begin) do without the copies. */
 size_t kf_layer_copies_bytes(const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok);
 int kf_layer_copies(kf_ctx* ctx, const kf_weight* wq, const kf_weight* wk, const kf_weight* wv, const kf_weight* wo, const kf_weight* gate, const kf_weight* up, const kf_weight* down, int nTok);
 int kf_layer_copies_end(kf_ctx* ctx);

@@ -133,7 +133,7 @@ static int deq_copies(kf_ctx* c, int n_w, const kf_weight* const* w, int form, c
     for (int i = 0; i < n_w; i++) need += up256z((size_t)w[i]->ne0 * w[i]->ne1 * 2);
     if (resident) *resident = false;
     for (const kf_ctx::DeqCopy& e : c->call)
-        if (e.of(n_w, w, form)) {
+        if (c->call_live() && e.of(n_w, w, form)) {
             *out = (const uint16_t*)((const char*)c->scratch + e.off);
             return KF_OK;
         }
@@ -412,7 +412,7 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         return kf_linear(c, &wb, x, y, bias, nTok, alpha, beta, epilogue, residual);
     }
     for (const kf_ctx::DeqCopy& e : c->call) {
-        if (!e.of(1, &w, DEQ_STACK) || nTok < KF_LAYER_COPIES_MIN) continue; /* a copy of this matrix alone (kf_layer_copies) */
+        if (!c->call_live() || !e.of(1, &w, DEQ_STACK) || nTok < KF_LAYER_COPIES_MIN) continue; /* a copy of this matrix alone (kf_layer_copies) */
         kf_weight wb;
         memset(&wb, 0, sizeof(wb));
         wb.data = (char*)c->scratch + e.off, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
@@ -785,7 +785,7 @@ static const int KF_MULTI_DEQ_MIN = 1024; /* token rows from which the stacked r
 static int multi_min(const kf_ctx* c) {
     int n = KF_MULTI_DEQ_MIN;
     if (c && c->arena && kf::g_knobs.resident_min < n) n = kf::g_knobs.resident_min;
-    if (c && !c->call.empty() && KF_LAYER_COPIES_MIN < n) n = KF_LAYER_COPIES_MIN;
+    if (c && c->call_live() && KF_LAYER_COPIES_MIN < n) n = KF_LAYER_COPIES_MIN;
     return n;
 }
 /* up256z: a no-op on these sizes (multiples of 256 rows x 64 columns): the stacked rows are contiguous */

@@ -38,6 +38,7 @@ struct kf_ctx {
     // bf16 copies of one layer's matrices for the calls between kf_layer_copies and kf_layer_copies_end, at the front of the scratch (call_used bytes of it)
     std::vector<DeqCopy> call;
     size_t call_used;
+    bool call_live() const { return !call.empty() && !capturing; } /* a captured launch is replayed after the copies are gone: it does without them */
     char* scratch_tail() const { return scratch ? (char*)scratch + call_used : nullptr; } /* what the copies leave: 256-byte steps */
     size_t scratch_left() const { return scratch_bytes > call_used ? scratch_bytes - call_used : 0; }
     /* the split-K slots lent to the tile kernels lie at the scratch's END, so their flags stay where they were as long as no copy reaches them (scratch_written) */

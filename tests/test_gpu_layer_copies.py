@@ -98,3 +98,30 @@ def test_a_set_with_a_matrix_of_fewer_rows_is_another_set(ctx):
     finally:
         ctx.sync()
         ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
+
+
+def test_captured_launches_do_without_the_copies(ctx):
+    """a product captured between kf_layer_copies and _end is replayed when the copies are gone and their place holds something else"""
+    n = 320
+    ws, descs = _layer(ctx, 1024, 2048, 1024, 3072)
+    x = torch.randn(n, 2048, device=ctx.device).bfloat16()
+    y, g = torch.zeros(n, 1024, device=ctx.device, dtype=torch.bfloat16), C.c_void_p()
+    want = x.float() @ ctx.dequant(ws[3]).float().t()
+    try:
+        _, scratch = _copies(ctx, descs, n)
+        assert ctx.hip.kf_graph_begin(ctx.h) == 0
+        rc = ctx.hip.kf_linear(ctx.h, C.byref(descs[3]), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None)
+        assert ctx.hip.kf_graph_end(ctx.h, C.byref(g)) == 0 and rc == 0
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+        ctx.sync()
+        for fill in (0, 0x3C):
+            scratch.fill_(fill)
+            y.zero_()
+            assert ctx.hip.kf_graph_launch(ctx.h, g) == 0
+            ctx.sync()
+            assert float((y.float() - want).abs().max()) <= 2.0 ** -7 * float(want.abs().max())   # the in-register product: 2^-7 as in the tests of that kernel
+    finally:
+        ctx.sync()
+        if g:
+            ctx.hip.kf_graph_destroy(g)
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
