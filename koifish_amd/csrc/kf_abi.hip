@@ -108,7 +108,7 @@ int kf_init(int device, void* stream, kf_ctx** out) {
 }
 // `bytes` of a copy are about to be written at dst in the scratch: where they reach the split-K flags, the next launch that waits for these clears them first
 static void scratch_written(kf_ctx* c, const void* dst, size_t bytes) {
-    const char* const slots = (const char*)c->scratch_end(kf::gemm3_sk_ws_bytes());
+    const char* const slots = (const char*)c->slots_at(kf::gemm3_sk_ws_bytes());
     if (slots && (const char*)dst >= (const char*)c->scratch && (const char*)dst < (const char*)c->scratch + c->scratch_bytes && (const char*)dst + bytes > slots) kf::gemm3_sk_forget((void*)slots);
 }
 // bf16 view of a weight: the data itself (bf16 storage) or its dequantisation into the caller's scratch (kf_set_scratch)
@@ -373,7 +373,7 @@ int kf_set_scratch(kf_ctx* c, void* scratch, size_t bytes) {
     if (c->capturing) return fail(KF_INVALID_ARGS, "kf_set_scratch: not while capturing (captured launches hold the old pointer)");
     c->scratch = scratch, c->scratch_bytes = scratch ? bytes : 0;
     c->call.clear(), c->call_used = 0;
-    if (void* slots = c->scratch_end(kf::gemm3_sk_ws_bytes())) kf::gemm3_sk_forget(slots); /* whatever lay there before */
+    if (void* slots = c->slots_at(kf::gemm3_sk_ws_bytes())) kf::gemm3_sk_forget(slots); /* whatever lay there before */
     return KF_OK;
 }
 

@@ -41,8 +41,9 @@ struct kf_ctx {
     bool call_live() const { return !call.empty() && !capturing; } /* a captured launch is replayed after the copies are gone: it does without them */
     char* scratch_tail() const { return scratch ? (char*)scratch + call_used : nullptr; } /* what the copies leave: 256-byte steps */
     size_t scratch_left() const { return scratch_bytes > call_used ? scratch_bytes - call_used : 0; }
-    /* the split-K slots lent to the tile kernels lie at the scratch's END, so their flags stay where they were as long as no copy reaches them (scratch_written) */
-    void* scratch_end(size_t bytes) const { return scratch && scratch_left() >= bytes + 256 ? (void*)(((uintptr_t)scratch + scratch_bytes - bytes) & ~(uintptr_t)255) : nullptr; }
+    /* the split-K slots of the tile kernels lie at the scratch's END, whether or not copies leave room to lend them now: their flags stay where they were as long as nothing is written there (scratch_written) */
+    void* slots_at(size_t bytes) const { return scratch && scratch_bytes >= bytes + 256 ? (void*)(((uintptr_t)scratch + scratch_bytes - bytes) & ~(uintptr_t)255) : nullptr; }
+    void* scratch_end(size_t bytes) const { return scratch_left() >= bytes + 256 ? slots_at(bytes) : nullptr; }
 };
 enum { DEQ_STACK = 0, DEQ_ILV = 1 };
 

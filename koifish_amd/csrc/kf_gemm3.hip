@@ -359,7 +359,7 @@ static int g3_sk_epoch(hipStream_t st, uint32_t* flags, int n, uint32_t* epoch) 
     bool seen = false;
     for (int i = 0; i < 8; i++) seen = seen || g_sk_seen[i] == flags;
     if (cs != hipStreamCaptureStatusNone || !seen) {
-        if (hipMemsetAsync(flags, 0, n * sizeof(uint32_t), st) != hipSuccess) return KF_HIP_CHECK;
+        if (hipMemsetAsync(flags, 0, seen ? n * sizeof(uint32_t) : G3_SK_FLAG_BYTES, st) != hipSuccess) return KF_HIP_CHECK; /* (the whole area: the next launch may be of smaller tiles, with more flags) */
     }
     if (cs != hipStreamCaptureStatusNone) {
         *epoch = 1;

@@ -125,3 +125,42 @@ def test_captured_launches_do_without_the_copies(ctx):
         if g:
             ctx.hip.kf_graph_destroy(g)
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+def test_flags_written_over_behind_the_copies_are_cleared(ctx):
+    """copies that end just below the split-K slots leave too little to lend them; a matrix dequantised there meanwhile lies on their flags, and the next product in k-pieces clears them first"""
+    M, K, n, words = 1024, 3072, 384, 2048   # the flags: the last 8 KiB of the slots
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4)
+    x, y, d = torch.randn(n, K, device=ctx.device).bfloat16(), torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16), w.desc()
+    want = x.float() @ ctx.dequant(w).float().t()
+    _, descs = _layer(ctx, 256, 512, 256, 512)
+    slots, need = ctx.hip.kf_resident_scratch_bytes() - 512, ctx.hip.kf_layer_copies_bytes(*[C.byref(e) for e in descs], 2047)
+    copies = need - slots - 512
+    rows = (slots + 128) // 4096   # of 2048 values: as much as lies behind the copies
+    other = ctx.quantize_nf4((torch.randn(rows, 2048, device=ctx.device) * 0.05).bfloat16(), 3)
+    xo, yo, do = torch.randn(8, 2048, device=ctx.device).bfloat16(), torch.zeros(8, rows, device=ctx.device, dtype=torch.bfloat16), other.desc()
+    arena = torch.zeros(M * K * 2 + 4096, dtype=torch.uint8, device=ctx.device)
+    scratch = torch.zeros(copies + slots + 128, dtype=torch.uint8, device=ctx.device)
+    assert scratch.data_ptr() % 256 == 0 and copies % 256 == 0 and slots % 256 == 0 and rows * 4096 > slots - 4 * words
+
+    def product():
+        assert ctx.hip.kf_set_dequant_arena(ctx.h, C.c_void_p(arena.data_ptr()), C.c_size_t(arena.numel())) == 0
+        y.zero_()
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
+        assert float((y.float() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())
+        assert ctx.hip.kf_set_dequant_arena(ctx.h, None, 0) == 0
+    try:
+        assert ctx.hip.kf_set_scratch(ctx.h, C.c_void_p(scratch.data_ptr()), C.c_size_t(scratch.numel())) == 0
+        product()
+        flags = scratch[copies + slots - 4 * words:copies + slots].view(torch.int32)
+        assert len(flags.unique()) == 2   # raised ones and zeros
+        assert ctx.hip.kf_layer_copies(ctx.h, *[C.byref(e) for e in descs], 2047) == 0
+        assert ctx.hip.kf_linear(ctx.h, C.byref(do), xo.data_ptr(), yo.data_ptr(), None, 8, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+        assert len(flags.unique()) > 2
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+        product()
+        assert len(flags.unique()) == 2
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
