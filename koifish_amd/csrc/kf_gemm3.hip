@@ -346,12 +346,15 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_sk_ke
 }
 
 // The flag value of one split-K launch.  Launches outside a capture take a fresh value each (a process-wide counter from 2 up), so the flags of the launch before need
-// no clearing -- the memset was a dependent 2-3 us node in front of every such product; a flag area seen for the first time is cleared once.  A launch that is being
+// no clearing -- that was a dependent 2-3 us node in front of every such product; a flag area seen for the first time is cleared once.  A launch that is being
 // CAPTURED is replayed with the arguments it was recorded with: it keeps the clearing node and the value 1.
 constexpr size_t G3_SK_FLAG_BYTES = 8192; /* up to 2048 resident workgroups (64 x 64 tiles, eight per CU) */
 static std::mutex g_sk_mu;
 static uint32_t g_sk_epoch = 1;
 static const void* g_sk_seen[8] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+__global__ void __launch_bounds__(256) g3_clear_kernel(u32x4* flags, int n4) {
+    for (int i = threadIdx.x; i < n4; i += 256) flags[i] = u32x4{0, 0, 0, 0};
+}
 static int g3_sk_epoch(hipStream_t st, uint32_t* flags, int n, uint32_t* epoch) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess) return KF_HIP_CHECK;
@@ -359,7 +362,9 @@ static int g3_sk_epoch(hipStream_t st, uint32_t* flags, int n, uint32_t* epoch) 
     bool seen = false;
     for (int i = 0; i < 8; i++) seen = seen || g_sk_seen[i] == flags;
     if (cs != hipStreamCaptureStatusNone || !seen) {
-        if (hipMemsetAsync(flags, 0, seen ? n * sizeof(uint32_t) : G3_SK_FLAG_BYTES, st) != hipSuccess) return KF_HIP_CHECK; /* (the whole area: the next launch may be of smaller tiles, with more flags) */
+        const int n4 = seen ? n / 4 : (int)(G3_SK_FLAG_BYTES / 16); /* first seen: the whole area (the next launch may be of smaller tiles, with more flags) */
+        hipLaunchKernelGGL(g3_clear_kernel, dim3(1), dim3(256), 0, st, (u32x4*)flags, n4); /* a kernel: memset nodes of a replayed graph have left their memory as it was on this part */
+        if (hipGetLastError() != hipSuccess) return KF_HIP_CHECK;
     }
     if (cs != hipStreamCaptureStatusNone) {
         *epoch = 1;

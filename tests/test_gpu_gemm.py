@@ -382,3 +382,42 @@ def test_resident_copies_with_a_lent_workspace_sum_every_k_piece(ctx, M, K, n):
         ctx.sync()
         ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+def test_a_captured_product_in_k_pieces_is_right_at_every_replay(ctx):
+    """replays wait for their own pieces: the flags are cleared by a node that works at each of them, with eager launches (which raise other values in the same flags) in between.  Every replay has the
+    eager result's bits -- the pieces are added in order -- and the graph holds no memset node"""
+    M, K, n = 1024, 3072, 384
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4)
+    x, d = torch.randn(n, K, device=ctx.device).bfloat16(), w.desc()
+    y, out = torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16), torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
+    arena = torch.zeros(M * K * 2 + 4096, dtype=torch.uint8, device=ctx.device)
+    ws = torch.full((ctx.hip.kf_resident_scratch_bytes(),), 0x5A, dtype=torch.uint8, device=ctx.device)
+    run = lambda to: ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), to.data_ptr(), None, n, 1.0, 0.0, 0, None)
+    g = C.c_void_p()
+    try:
+        assert ctx.hip.kf_set_dequant_arena(ctx.h, C.c_void_p(arena.data_ptr()), C.c_size_t(arena.numel())) == 0
+        assert ctx.hip.kf_set_scratch(ctx.h, C.c_void_p(ws.data_ptr()), C.c_size_t(ws.numel())) == 0
+        assert run(y) == 0
+        assert ctx.hip.kf_graph_begin(ctx.h) == 0
+        rc = run(out)
+        assert ctx.hip.kf_graph_end(ctx.h, C.byref(g)) == 0 and rc == 0
+        rt, graph, count = C.CDLL("libamdhip64.so"), C.c_void_p.from_address(g.value), C.c_size_t(0)   # kf_graph begins with its hipGraph_t
+        assert rt.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+        nodes, kind = (C.c_void_p * count.value)(), C.c_int()
+        assert rt.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0
+        for node in nodes:
+            assert rt.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0 and kind.value == 0   # hipGraphNodeTypeKernel
+        for i in range(6):
+            x.copy_(torch.randn(n, K, device=ctx.device).bfloat16())
+            out.zero_()
+            assert ctx.hip.kf_graph_launch(ctx.h, g) == 0
+            assert run(y) == 0
+            ctx.sync()
+            assert torch.equal(out, y)
+    finally:
+        ctx.sync()
+        if g:
+            ctx.hip.kf_graph_destroy(g)
+        ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
