@@ -124,9 +124,17 @@ struct RbTokens {
         for (int i = 0; i < NT * U; i++) v[i] = *reinterpret_cast<const u32x4*>(at + off[i]);
     }
     __device__ __forceinline__ int row(int i) const { return i * (64 / CH) + lane / CH; }
+    // Other lanes read what a lane stores, and store over what it has read.  A wave's LDS accesses are in order; only the compiler has to be told, which sees one lane's addresses and could swap them.
+    static __device__ __forceinline__ void in_order() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
     __device__ __forceinline__ void turn(u32x4 (&b)[U][NT]) {
+        in_order();
 #pragma unroll
         for (int i = 0; i < NT * U; i++) *reinterpret_cast<u32x4*>(lds + row(i) * ROW + 8 * (lane % CH)) = v[i];
+        in_order();
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
