@@ -182,7 +182,10 @@ int kf_malloc(kf_ctx* c, size_t bytes, void** out) {
     CHKCTX(c);
     if (!out) return fail(KF_INVALID_ARGS, "kf_malloc: out is null");
     hipError_t e = hipMalloc(out, bytes ? bytes : 16);
-    if (e != hipSuccess) return fail(KF_OUTOF_GPUMEMORY, "kf_malloc(%zu): %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError(); /* reported here: the next launch's check must not find it */
+        return fail(KF_OUTOF_GPUMEMORY, "kf_malloc(%zu): %s", bytes, hipGetErrorString(e));
+    }
     return KF_OK;
 }
 int kf_free(kf_ctx* c, void* p) {

@@ -129,3 +129,13 @@ def test_tp_reduce_rank_order(ctx):
     assert ctx.hip.kf_linear_f32(ctx.h, C.byref(desc_), x_d.data_ptr(), y.data_ptr()) == 0
     ref32 = O.linear_f32(ow, x)
     assert np.abs(y.cpu().numpy() - ref32).max() <= 1e-5 * np.abs(ref32).max() + 1e-6
+
+
+def test_a_refused_allocation_leaves_no_error_behind(ctx):
+    """more memory than any card has: the refusal is kf_malloc's own result, and the launches that follow do without the block"""
+    p, x = C.c_void_p(), torch.ones(4, 256, device=ctx.device).bfloat16()
+    y = torch.zeros_like(x)
+    assert ctx.hip.kf_malloc(ctx.h, C.c_size_t(1 << 50), C.byref(p)) < 0
+    assert ctx.hip.kf_add(ctx.h, x.data_ptr(), x.data_ptr(), y.data_ptr(), x.numel()) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    assert bool((y == 2).all())
