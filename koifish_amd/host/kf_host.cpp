@@ -464,7 +464,7 @@ void Fish::DropResident() {
         kf_set_dequant_arena(ctx, nullptr, 0);
         kf_free(ctx, deq_arena), deq_arena = nullptr, deq_arena_bytes = 0;
     }
-    resident_tried = false;
+    resident_tried = false, scratch_rows = 0;
 }
 // Resident bf16 copies of the layers' quantised matrices for long prompts (kf_set_dequant_arena): 2 bytes per weight -- 0.9 GB for Qwen3-0.6B, 62 GB for Qwen3-32B -- of a
 // 288 GB part, instead of five dequantise launches per layer and prompt.  Sized and allocated by the first Prefill after the weights were set (never inside a launch
@@ -806,27 +806,41 @@ int Fish::PrefillReady(int min_rows) {
         gBUFF.bUp = GT(ctx, "bUp", typNUMBER::BF16, config.n_ff, PC);
         if (!gBUFF.bX || !gBUFF.bNorm || !gBUFF.bQ || !gBUFF.bAttn || !gBUFF.bGate || !gBUFF.bUp) return KF_OUTOF_GPUMEMORY;
         KF_TRY(kf_malloc(ctx, (size_t)PC * 4, (void**)&gBUFF.d_ptok));
-        // the stacked large-batch routes (Q | K | V and gate | up dequantised back to back, one tile-GEMM launch each): their workspace, sized here -- the first
-        // Prefill allocates the batch buffers anyway; the launches themselves never allocate
-        for (int l = 0; l < config.nLayer; l++) {
-            kf_weight wq = attn[l]->Q.w->desc(), wk = attn[l]->K.w->desc(), wv = attn[l]->V.w->desc(), wg = ffn[l]->gate.w->desc(), wu = ffn[l]->up.w->desc();
-            const kf_weight* qkv[3] = {&wq, &wk, &wv};
-            const kf_weight* gu[2] = {&wg, &wu};
-            kf_weight wo = attn[l]->proj_cat.w->desc(), wd = ffn[l]->down.w->desc();
-            size_t need = 0;
-            for (size_t n : {kf_linear_multi_scratch_bytes(3, qkv, PC), kf_linear_multi_scratch_bytes(2, gu, PC), kf_linear_scratch_bytes(&wo, PC), kf_linear_scratch_bytes(&wd, PC),
-                             kf_layer_copies_bytes(&wq, &wk, &wv, &wo, &wg, &wu, &wd, PC)}) need = n > need ? n : need;
-            if (need > lin_scratch_bytes) {
-                KF_TRY(kf_sync(ctx));
-                void* p = nullptr;
-                KF_TRY(kf_malloc(ctx, need, &p));
-                KF_TRY(kf_set_scratch(ctx, p, need));
-                if (lin_scratch) kf_free(ctx, lin_scratch);
-                lin_scratch = p, lin_scratch_bytes = need;
-            }
-        }
     }
-    return EnsureResident(gBUFF.rows);
+    KF_TRY(EnsureResident(gBUFF.rows));
+    return PrefillScratch(gBUFF.rows);
+}
+
+// The workspace of the token-batch launches: what the stacked routes (Q | K | V and gate | up dequantised back to back, one tile-GEMM launch each) and o / down ask for has to be there.  Room for one layer's
+// bf16 copies (kf_layer_copies: 98 MB for a 0.6B model, 1.04 GB for a 32B one) only saves time: a card that has not that much left does without, and resident copies make it needless.
+int Fish::PrefillScratch(int rows) {
+    if (scratch_rows >= rows) return KF_OK;
+    scratch_rows = rows;
+    size_t need = lin_scratch_bytes, want = 0;
+    for (int l = 0; l < config.nLayer; l++) {
+        const kf_weight wq = attn[l]->Q.w->desc(), wk = attn[l]->K.w->desc(), wv = attn[l]->V.w->desc(), wo = attn[l]->proj_cat.w->desc();
+        const kf_weight wg = ffn[l]->gate.w->desc(), wu = ffn[l]->up.w->desc(), wd = ffn[l]->down.w->desc();
+        const kf_weight *qkv[3] = {&wq, &wk, &wv}, *gu[2] = {&wg, &wu};
+        for (size_t n : {kf_linear_multi_scratch_bytes(3, qkv, rows), kf_linear_multi_scratch_bytes(2, gu, rows), kf_linear_scratch_bytes(&wo, rows), kf_linear_scratch_bytes(&wd, rows)}) need = std::max(need, n);
+        if (!deq_arena) want = std::max(want, kf_layer_copies_bytes(&wq, &wk, &wv, &wo, &wg, &wu, &wd, rows));
+    }
+    want = std::max(want, need);
+    if (want <= lin_scratch_bytes) return KF_OK;
+    KF_TRY(kf_sync(ctx));
+    for (auto& g : graphs) /* captured steps may hold the block that goes */
+        if (g) kf_graph_destroy(g), g = nullptr;
+    KF_TRY(kf_set_scratch(ctx, nullptr, 0)); /* the old block goes first: the card need not hold both */
+    if (lin_scratch) kf_free(ctx, lin_scratch);
+    lin_scratch = nullptr, lin_scratch_bytes = 0;
+    for (size_t bytes : {want, need}) {
+        void* p = nullptr;
+        if (bytes == 0) return KF_OK;
+        if (kf_malloc(ctx, bytes, &p) != KF_OK) continue;
+        lin_scratch = p, lin_scratch_bytes = bytes;
+        return kf_set_scratch(ctx, p, bytes);
+    }
+    scratch_rows = 0;
+    return KF_OUTOF_GPUMEMORY;
 }
 
 int Fish::HeadAndPick(const floatX* x_last) {

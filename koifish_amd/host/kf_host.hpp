@@ -239,8 +239,9 @@ struct Fish {
     int fuse_level = 1;  // 0: one launch per reference kernel; 1: fused launches (5 per layer)
     // the layer loop of a decode step as one persistent launch (kf_engine_*): used by EnqueueStep when fuse_level >= 1, the model's shapes and
     // storage are served and the position bound is; otherwise the per-layer launches run.  Same arithmetic, bit for bit.
-    void* lin_scratch = nullptr;  // kf_set_scratch: workspace of the dequantise-then-multiply storages (AutoAWQ, row forms), sized when weights are set
+    void* lin_scratch = nullptr;  // kf_set_scratch: workspace of the dequantise-then-multiply storages (AutoAWQ, row forms), sized when weights are set, and of the token-batch launches
     size_t lin_scratch_bytes = 0;
+    int scratch_rows = 0;  // token rows that PrefillScratch has sized it for (0: again at the next prefill)
     void* deq_arena = nullptr;  // kf_set_dequant_arena: resident bf16 copies of the layers' quantised matrices for long prompts (EnsureResident)
     size_t deq_arena_bytes = 0, resident_max_bytes = (size_t)16 << 30;
     // OFF by default: the copies are keyed by the blobs' addresses, so a caller that hands weights over as device pointers (kfh_set_weight is_device = 1) and later
@@ -251,6 +252,7 @@ struct Fish {
     int EnsureResident(int PC);
     void DropResident();
     int EnsureLinearScratch(const kf_weight& w, int nTok);
+    int PrefillScratch(int rows);
     bool use_engine = true;
     kf_engine* engine = nullptr;
     void* engine_ws = nullptr;
