@@ -398,10 +398,12 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
         if (hipFuncSetAttribute((const void*)gemm3_sk_kernel<AKM, BKM, BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
-    // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; K-contiguous products from K = 3072 (plain | split, us:
-    // 1024 x 2048 at 512 tokens 11.2 | 12.6, at 2047 17.3 | 20.5;  2048 x 2048 at 512 11.0 | 15.2;  1024 x 3072 at 320 21.3 | 15.3, at 512 15.5 | 16.3, at 2047 30.0 | 25.5;  2048 x 6144 at 512 44.5 | 32.6)
+    // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; a K-contiguous product of K < 3072 only where three pieces of
+    // every tile find room.  us per layer of prompts, never | from K = 3072 | three pieces: 0.6B, resident copies, 320 rows 134 | 116 | 106, 1024 rows 149 | 143 | 137, 2047 rows 198 | 190 | 187; a layer's
+    // copies 119 | 111 | 105, 136 | 134 | 130, 190 | 187 | 185;  1.7B resident 320 rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800
+    // rows 325 -> 332 us.  (One product by itself on operands that are in the L2 already shows the opposite: 1024 x 2048 at 512 rows 11.2 whole, 12.6 in four pieces.)
     const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
-    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || nkt >= 48)) {
+    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || nkt >= 48)) {
         G3SkArgs s;
         // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they moved with it,
         // and another configuration's fp32 partials could overwrite words already marked "seen" with values that pass for an epoch)
@@ -451,7 +453,7 @@ int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws
     if (a.n < 128 || a.M < 128) return 1;
     const long nwg = (long)((a.M + 127) / 128) * ((a.n + 127) / 128);
     if (nwg < 32 && (g_knobs.g3_tiles < 3 || (long)((a.M + 63) / 64) * ((a.n + 63) / 64) < 64)) return 1;
-    if (nwg < 256 && g_knobs.g3_tiles >= 1 && !a.swiglu && !a.qkrope) { /* fewer 128 x 128 tiles than CUs: twice or four times as many smaller ones, no k-pieces */
+    if (nwg < 256 && g_knobs.g3_tiles >= 1 && !a.swiglu && !a.qkrope) { /* fewer 128 x 128 tiles than CUs: twice or four times as many smaller ones */
         // with the caller's workspace these go in k-pieces when even the small tiles leave CUs idle (1024 rows x K 2048-3072 at 512 tokens: 128 tiles of 64 x 64, each a
         // 32-48 step k-loop of ~0.7 us per step on its own CU: 31 us; a 16 KiB partial per piece is cheap where the 64 KiB ones of the 128 x 128 tile were not)
         const long nmid = (long)((a.M + 63) / 64) * ((a.n + 127) / 128);

@@ -362,9 +362,11 @@ def test_resident_dequantised_copies_give_the_scratch_routes_results(ctx, O, t):
         L.check(ctx.hip.kf_set_dequant_arena(ctx.h, None, 0), "kf_set_dequant_arena")
 
 
-@pytest.mark.parametrize("M,K,n", [(1024, 2048, 320), (1024, 2048, 512), (1024, 3072, 384), (1024, 3072, 1024), (2048, 2048, 520)])
-def test_resident_copies_with_a_lent_workspace_sum_every_k_piece(ctx, M, K, n):
-    """short token batches on resident copies go in k-pieces when a workspace is lent (64 x 64, 64 x 128 and 128 x 128 tiles): every piece reaches the output.  fp32 sums of K products of the same bf16
+@pytest.mark.parametrize("M,K,n,pieces", [(1024, 2048, 320, True), (1024, 2048, 512, True), (1024, 3072, 384, True), (1024, 3072, 1024, True), (2048, 2048, 520, True),   # 64 x 64 tiles
+                                          (1024, 3072, 2047, True), (1024, 3200, 1537, True), (1024, 2048, 2047, True),                                            # 64 x 128: three pieces, uneven ones
+                                          (2048, 3200, 1800, True), (2048, 2048, 1800, False), (1024, 2048, 2608, False)])                                         # 480 of 768 residents: a piece and tails, or whole
+def test_resident_copies_with_a_lent_workspace_sum_every_k_piece(ctx, M, K, n, pieces):
+    """short token batches on resident copies go in k-pieces when a workspace is lent (64 x 64 and 64 x 128 tiles): every piece reaches the output.  fp32 sums of K products of the same bf16
     values in another order and one bf16 rounding: 2^-8 of the result's scale"""
     w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4)
     ref_w, x, d = ctx.dequant(w).float(), torch.randn(n, K, device=ctx.device).bfloat16(), w.desc()
@@ -378,6 +380,7 @@ def test_resident_copies_with_a_lent_workspace_sum_every_k_piece(ctx, M, K, n):
             y = torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
             assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
             assert float((y.float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+        assert bool((ws[:-16384] != 0x5A).any()) == pieces   # partials were written (or none)
     finally:
         ctx.sync()
         ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
