@@ -443,7 +443,7 @@ int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws
         const long nwg = (long)((a.M + G3_BM - 1) / G3_BM) * ((a.n + G3_BN - 1) / G3_BN);
         // (M 1024 x K 3072 at 8192 rows, 128 big tiles: 83 -> 57 us = 890 TFLOP/s on the small ones; from 400 big tiles up the big tile is 8-12 % faster)
         if (nwg >= 160) { /* fewer big tiles than that: four times as many small ones fill the chip better */
-            if (g_knobs.g3_wide && g3_prefer_wide(a.M, a.n)) return g3_go_c<false, false, G3Wide>(st, a, (long)((a.M + 191) / 192) * ((a.n + 255) / 256), nullptr, 0, 1);
+            if (g_knobs.g3_wide && g3_prefer_wide(a.M, a.n, a.K)) return g3_go_c<false, false, G3Wide>(st, a, (long)((a.M + 191) / 192) * ((a.n + 255) / 256), nullptr, 0, 1);
             return g3_go<false, false>(st, a, nwg, nullptr, 0);
         }
     }
@@ -537,7 +537,7 @@ int gemm3_swiglu_launch(hipStream_t st, const uint16_t* Wilv, int ffn, int K, co
     const bool wide_ok = g_knobs.g3_wide && M % 192 == 0 && nww <= 256;
     // fewer than 160 big tiles: four times as many 128 x 128 ones -- unless those spill into a second round of the 512 resident workgroups and the 192 x 256 ones make one round
     if (nwg < 160 && !(wide_ok && nws > 512 && nww >= 160)) return g3_go_c<false, false, G3Small>(st, a, nws, nullptr, 0, 1);
-    if (g_knobs.g3_wide && g3_prefer_wide(M, n)) return g3_go_c<false, false, G3Wide>(st, a, (long)((M + 191) / 192) * ((n + G3_BN - 1) / G3_BN), nullptr, 0, 1);
+    if (g_knobs.g3_wide && g3_prefer_wide(M, n, K)) return g3_go_c<false, false, G3Wide>(st, a, (long)((M + 191) / 192) * ((n + G3_BN - 1) / G3_BN), nullptr, 0, 1);
     return g3_go<false, false>(st, a, nwg, nullptr, 0);
 }
 

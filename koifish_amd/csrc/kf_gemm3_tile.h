@@ -295,11 +295,13 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     asm volatile("" ::: "memory");
 }
 
-// 256 x 256 or 192 x 256: with one big workgroup per CU a launch takes whole rounds of 256 tiles, and a round of the smaller ones takes 0.79 of a round (measured at K = 1024 - 2048), so the last
-// round's emptiness decides: 6144 x 1024 at 2608 rows 264 tiles in two rounds 66.8 us, 352 of 192 x 256 in two 53; 8704 x 2048 at 1971 rows (272 | 368) 108 | 86
-static inline bool g3_prefer_wide(int M, int n) {
+// 256 x 256 or 192 x 256: with one big workgroup per CU a launch takes whole rounds of 256 tiles, and a round of the smaller ones takes 0.79 to 0.95 of a round, so the smaller tile pays where it needs no
+// more rounds.  us, big | wide: 6144 x 1024 at 2608 rows (264 | 352 tiles) 66.7 | 54.3, x 4096 176 | 143, x 25600 1230 | 1036; 5120 x 12288 at 4096 rows (320 | 432) 543 | 518; 10240 x 8192 at 3500 rows
+// (560 | 756) 522 | 449.  One round more pays for 5 and 6 of them at K <= 2048, where the round is shortest against its start: 12288 x 2048 at 5888 rows (1104 | 1472) 280 | 269, at 6912 (1296 | 1728) 332 |
+// 312; at K 4096 486 | 498 and 585 | 606.  Two more never: 12288 x 2048 at 11008 rows (2064 | 2752) 515 | 562.
+static constexpr bool g3_prefer_wide(int M, int n, int K) {
     const long by = (n + 255) / 256, rb = ((M + 255) / 256 * by + 255) / 256, rw = ((M + 191) / 192 * by + 255) / 256;
-    return 79 * rw < 97 * rb;
+    return rw <= rb || (rw == rb + 1 && (rb == 5 || rb == 6) && K <= 2048);
 }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {

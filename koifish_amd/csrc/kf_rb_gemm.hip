@@ -118,7 +118,7 @@ int rb_gemm_launch(hipStream_t st, const RbProduct& q) {
     }
     // the measured thresholds of gemm3_launch: big tiles from 160 of them, then smaller ones that fill the chip
     if (p.m >= 256 && p.n >= 256 && rb_tiles(p, 256, 256) >= 160)
-        return g3_prefer_wide(p.m, p.n) ? rb_go<RbWide, false>(st, q, rb_tiles(p, 192, 256)) : rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
+        return g3_prefer_wide(p.m, p.n, p.k) ? rb_go<RbWide, false>(st, q, rb_tiles(p, 192, 256)) : rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
     if (rb_tiles(p, 128, 128) >= 256) return rb_go<RbSmall, false>(st, q, rb_tiles(p, 128, 128));
     if (rb_tiles(p, 64, 128) >= 192) return rb_go<RbMid, false>(st, q, rb_tiles(p, 64, 128));
     return rb_go<RbTiny, false>(st, q, rb_tiles(p, 64, 64));
