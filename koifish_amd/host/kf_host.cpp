@@ -1233,7 +1233,9 @@ int XcdReplicas::RunSteps(int n) {
 // A queue of prompts answered through the sequences' slots: what Fish::Chat does round by round over DEBUG.prompts (GoPT.cpp:1111-1180: prefill the prompt, then sample
 // until the tokenizer's EOS or the context is full, then the next prompt), with n_seq rounds in flight at once.  A free slot takes the next prompt (Prefill), the launches
 // decode every occupied slot, a finished round's slot is parked until the queue refills it; an answer ends at `eos` (eos < 0: never), at max_new ids, or at the last cache
-// row.  out [n_req][max_new] (-1 behind an answer's end), out_len [n_req]; every answer equals Fish::Generate's on the same prompt (same prefill, same decode arithmetic).
+// row.  out [n_req][max_new] (-1 behind an answer's end), out_len [n_req]; with one prompt read at a time (prefill_batch 1, the default) every answer equals Fish::Generate's on the
+// same prompt (same prefill, same decode arithmetic).  Prompts read together agree to the token-batch tolerance only: the batch's rows choose the kernels (from 320 rows the bf16 tiles, which sum in another
+// order), so a near-tie id can depend on who shares the batch.
 // With eos >= 0 the ids of each launch are read back (one sync per launch) and a sequence may run up to steps_per_launch - 1 ids past its EOS before its slot is freed --
 // those ids are dropped; stats [4] = {launches, steps, prefills, sequence-steps decoded and dropped}.
 //

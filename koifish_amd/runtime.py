@@ -778,7 +778,8 @@ class XcdReplicas:
         L.check(self.host.kfh_xr_prefill_batch(self.h, sl.ctypes.data_as(C.c_void_p), flat.ctypes.data_as(C.c_void_p), lens.ctypes.data_as(C.c_void_p), n, stride), "kfh_xr_prefill_batch")
 
     def set_prefill_batch(self, n):
-        """chat(): up to n waiting prompts are prefilled together when as many slots are free (1, the default: one by one -- the bits of the model's own prefill)"""
+        """chat(): up to n waiting prompts are prefilled together when as many slots are free (1, the default: one by one -- the bits of the model's own prefill).  Together the batch's rows choose the
+        kernels (320 rows and more: bf16 tiles, another order of summation): the token-batch tolerance, and a near-tie id can depend on who shares the batch"""
         L.check(self.host.kfh_xr_set_prefill_batch(self.h, int(n)), "kfh_xr_set_prefill_batch")
 
     def set_sampler(self, temperature=0.0, top_p=0.95, top_k=50, seed=42, true_topk=False):

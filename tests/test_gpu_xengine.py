@@ -699,3 +699,24 @@ def test_prefill_batch_vs_the_oracle(lens, slots):
         xr.prefill_batch((0,), [prompt_ids(cfg, cfg["max_seq"], seed=1)])   # no row left behind the prompt
     xr.close()
     m.close()
+
+
+@pytest.mark.parametrize("n,tokens", [(11, 29), (10, 32)])   # 319 and 320 rows: the products of a layer change kernels in between
+def test_a_prompt_in_a_batch_and_alone(n, tokens):
+    """who shares a batch decides the batch's rows, and these the kernels, which sum in other orders: K / V rows and logits of a prompt read with others and alone agree to the token-batch
+    tolerance (2^-6 of scale, as against the oracle)"""
+    cfg = dict(synth.CONFIGS["small"], max_seq=64)
+    m = synth.build_from_raw(cfg, synth.raw_weights_numpy(cfg, 99, w_std=0.1), L.Q4, L.BF16)
+    xr, f = XcdReplicas(m, n), O.bf16_to_f32
+    prompts = [prompt_ids(cfg, tokens, seed=500 + i) for i in range(n)]
+    xr.prefill_batch(list(range(n)), prompts)
+    m.sync()
+    together = [[f(a[:, :tokens]) for a in xr.kv_to_host(s)] + [f(xr.logits(s))] for s in (0, n - 1)]
+    for s, got in zip((0, n - 1), together):
+        xr.prefill(s, prompts[s])
+        m.sync()
+        alone = [f(a[:, :tokens]) for a in xr.kv_to_host(s)] + [f(xr.logits(s))]
+        for a, b in zip(got, alone):
+            assert np.abs(a - b).max() <= 2.0 ** -6 * np.abs(b).max()
+    xr.close()
+    m.close()
