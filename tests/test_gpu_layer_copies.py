@@ -60,10 +60,74 @@ def test_copies_and_routes(ctx, dim, q, kv, ffn, n):
         g, u = x.float() @ bf[4].float().t(), x.float() @ bf[5].float().t()
         ref = torch.nn.functional.silu(g) * u
         assert float((act.float() - ref).abs().max()) <= 2.0 ** -6 * float(ref.abs().max())
-        # other uses of the scratch stay behind the copies; after the end the routes are the ones without copies
         assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
     finally:
         ctx.sync()
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+def _routes(ctx, ws, descs, dim, q, kv, ffn, n):
+    """(first and last matrix of the set, call that returns the outputs, their values from the seven matrices) of every route that looks for copies"""
+    x, xo, xd = (torch.randn(n, k, device=ctx.device).bfloat16() for k in (dim, q, ffn))
+    res = torch.randn(n, dim, device=ctx.device).bfloat16()
+    out = lambda *cols: [torch.zeros(n, c, device=ctx.device, dtype=torch.bfloat16) for c in cols]
+    h, p = ctx.hip, [C.byref(d) for d in descs]
+
+    def single(i, xi, residual):
+        y, = out(dim)
+        assert h.kf_linear(ctx.h, p[i], xi.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, int(residual), res.data_ptr() if residual else None) == 0
+        return [y]
+
+    def stacked(rope):
+        y = out(q, kv, kv)
+        if rope:   # neither norms nor a table: the products themselves, by the launch that would norm and rotate them
+            assert h.kf_qkv_rope_batch(ctx.h, p[0], p[1], p[2], x.data_ptr(), *[t.data_ptr() for t in y], n, None, None, None, 0, q // 128, kv // 128, 128, 1e-6) == 0
+        else:
+            assert h.kf_linear_multi(ctx.h, 3, (C.POINTER(L.Weight) * 3)(*[C.pointer(d) for d in descs[:3]]), x.data_ptr(), (C.c_void_p * 3)(*[t.data_ptr() for t in y]), n) == 0
+        return y
+
+    def gated():
+        act, up = out(ffn, ffn)
+        assert h.kf_gateup_swiglu_batch(ctx.h, p[4], p[5], x.data_ptr(), act.data_ptr(), up.data_ptr(), n) == 0
+        return [act]
+    mm = lambda a, w: a.float() @ w.float().t()
+    silu = torch.nn.functional.silu
+    return [(0, 2, lambda: stacked(True), lambda w: [mm(x, w[i]) for i in range(3)]), (0, 2, lambda: stacked(False), lambda w: [mm(x, w[i]) for i in range(3)]),
+            (3, 3, lambda: single(3, xo, False), lambda w: [mm(xo, w[3])]), (3, 3, lambda: single(3, xo, True), lambda w: [mm(xo, w[3]) + res.float()]),
+            (4, 5, gated, lambda w: [silu(mm(x, w[4])) * mm(x, w[5])]), (6, 6, lambda: single(6, xd, True), lambda w: [mm(xd, w[6]) + res.float()])]
+
+
+@pytest.mark.parametrize("dim,q,kv,ffn,n", [(1024, 2048, 1024, 3072, 320), (1024, 2048, 1024, 3072, 2047), (256, 512, 256, 512, 2047), (2560, 4096, 1024, 9728, 321)])
+def test_every_route_multiplies_the_copies_until_the_end(ctx, dim, q, kv, ffn, n):
+    """with a set's copies halved its products are those of halved matrices, with the copies ended those of the matrices; what another matrix is dequantised to meanwhile lies behind the copies.  2^-6 of
+    the result's scale covers every route's roundings (gate and up: each rounded to 2^-9, then their product; behind a residual two roundings); a half would be off by 2^-1"""
+    ws, descs = _layer(ctx, dim, q, kv, ffn)
+    real = [ctx.dequant(w) for w in ws]
+    off = [0]
+    for w in real:
+        off.append(off[-1] + w.numel())
+    near = lambda got, want, tol: all(float((a.float() - b).abs().max()) <= tol * float(b.abs().max()) for a, b in zip(got, want))
+    try:
+        need, scratch = _copies(ctx, descs, n)
+        copies = scratch.view(torch.bfloat16)[:off[-1]]
+        before = copies.clone()
+        routes = _routes(ctx, ws, descs, dim, q, kv, ffn, n)
+        for first, last, call, ref in routes:
+            halved = [w * 0.5 if first <= i <= last else w for i, w in enumerate(real)]
+            assert near(call(), ref(real), 2.0 ** -6)
+            copies[off[first]:off[last + 1]] *= 0.5   # exact
+            assert near(call(), ref(halved), 2.0 ** -6)
+            copies[off[first]:off[last + 1]] *= 2.0
+        other = ctx.quantize_nf4((torch.randn(1024, 1024, device=ctx.device) * 0.05).bfloat16(), 3)   # a row form: dequantised into the scratch
+        xs, ys, do = torch.randn(8, 1024, device=ctx.device).bfloat16(), torch.zeros(8, 1024, device=ctx.device, dtype=torch.bfloat16), other.desc()
+        assert ctx.hip.kf_linear(ctx.h, C.byref(do), xs.data_ptr(), ys.data_ptr(), None, 8, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+        assert near([ys], [xs.float() @ ctx.dequant(other).float().t()], 2.0 ** -7) and torch.equal(copies, before)
+        copies *= 0.5
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+        assert all(near(call(), ref(real), 2.0 ** -6) for _, _, call, ref in routes)
+    finally:
+        ctx.sync()
+        ctx.hip.kf_layer_copies_end(ctx.h)
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
 
 
