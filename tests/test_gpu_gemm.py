@@ -187,9 +187,11 @@ def test_gemm_many_token_tiles_vs_exact(ctx, O, t):
     assert close_bf16(O.f32_to_bf16(y[-100:].astype(np.float32)), y2).all()
 
 
-@pytest.mark.parametrize("m,k,nt", [(4096, 1024, 2048), (4100, 512, 2050), (8192, 64, 4096), (1024, 2048, 2048), (1032, 3072, 2000), (3072, 1024, 1500)])
+@pytest.mark.parametrize("m,k,nt", [(4096, 1024, 2048), (4100, 512, 2050), (8192, 64, 4096), (1024, 2048, 2048), (1032, 3072, 2000), (3072, 1024, 1500),
+                                    (8192, 192, 4096), (8192, 256, 4096), (8188, 448, 4090), (8190, 128, 4090),   # 512 tiles of 256 x 256: odd and even numbers of k-steps, ragged ends, rows no multiple of 4
+                                    (2560, 192, 4096), (2564, 256, 4090)])                                        # 192 x 256, rows no multiple of 192
 def test_large_batch_bf16_tile_kernel(ctx, O, m, k, nt):
-    """the global_load_lds tile kernels (kf_gemm3.hip: bf16 operands; 256 x 256 tiles from 128 tiles up, else 128 x 128 tiles on four waves -- the last three shapes)
+    """the tile kernels of kf_gemm3.hip (bf16 operands; 256 x 256 tiles from 160 of them up, 192 x 256 where those fill the chip's rounds better, else 128 x 128, 64 x 128 or 64 x 64 on four waves)
     against the fp32 product of the same bf16 values: ragged last tiles in both dimensions, and the epilogue (alpha, beta, bias, residual) in gemm_epilogue's order"""
     g = torch.Generator(device=ctx.device)
     g.manual_seed(m + k + nt)

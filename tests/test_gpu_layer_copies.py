@@ -97,7 +97,9 @@ def _routes(ctx, ws, descs, dim, q, kv, ffn, n):
             (4, 5, gated, lambda w: [silu(mm(x, w[4])) * mm(x, w[5])]), (6, 6, lambda: single(6, xd, True), lambda w: [mm(xd, w[6]) + res.float()])]
 
 
-@pytest.mark.parametrize("dim,q,kv,ffn,n", [(1024, 2048, 1024, 3072, 320), (1024, 2048, 1024, 3072, 2047), (256, 512, 256, 512, 2047), (2560, 4096, 1024, 9728, 321)])
+@pytest.mark.parametrize("dim,q,kv,ffn,n", [(1024, 2048, 1024, 3072, 320), (1024, 2048, 1024, 3072, 2047), (256, 512, 256, 512, 2047), (2560, 4096, 1024, 9728, 321),
+                                             (256, 512, 256, 2560, 2047),      # gate | up on 192 x 256 tiles, 5120 rows: no multiple of 192
+                                             (512, 4096, 1024, 9728, 2047)])   # q | k | v and gate | up on 256 x 256 tiles
 def test_every_route_multiplies_the_copies_until_the_end(ctx, dim, q, kv, ffn, n):
     """with a set's copies halved its products are those of halved matrices, with the copies ended those of the matrices; what another matrix is dequantised to meanwhile lies behind the copies.  2^-6 of
     the result's scale covers every route's roundings (gate and up: each rounded to 2^-9, then their product; behind a residual two roundings); a half would be off by 2^-1"""

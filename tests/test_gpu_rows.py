@@ -139,13 +139,20 @@ def test_norm_in_front_of_a_product(ctx, n, m, k, dim):
 
 
 def test_product_many_tiles(ctx):
-    """the larger tiles of the bf16 product (256 x 256, 128 x 128, 64 x 128)"""
-    for m, n, k in ((2560, 4096, 128), (2048, 2048, 64), (1024, 1500, 192)):
+    """the larger tiles of the bf16 product (192 x 256, 128 x 128, 64 x 128; 256 x 256 with even and odd numbers of k-steps, rows no multiple of 256, tokens past the last tile)"""
+    for m, n, k in ((2560, 4096, 128), (2048, 2048, 64), (1024, 1500, 192), (8192, 4096, 192), (8192, 4096, 256), (8128, 4090, 320), (2624, 4090, 192)):
         w, x = (torch.randn(m, k, device="cuda") / k ** 0.5).bfloat16(), torch.randn(n, k, device="cuda").bfloat16()
         y, ws = torch.zeros(n, m, device="cuda"), stored(w)
         p = L.RbProduct(ws.data_ptr(), x.data_ptr(), y.data_ptr(), None, k, m, m, L.BF16, m, k, n, L.RB_STORE_F32, 0, L.RB_ALL, 0.0, None)
         L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
-        assert (y - x.float() @ w.float().T).abs().max().item() < 1e-4
+        full = x.float() @ w.float().T
+        assert (y - full).abs().max().item() < 1e-4
+        z = torch.zeros(n, m // 2, dtype=torch.bfloat16, device="cuda")   # gate and up in blocks of 16 rows: one bf16 rounding of silu(gate) * up
+        p = L.RbProduct(ws.data_ptr(), x.data_ptr(), z.data_ptr(), None, k, m // 2, 0, L.BF16, m, k, n, L.RB_GATED, L.RB_SILU, L.RB_ALL, 0.0, None)
+        L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+        pair = full.reshape(n, m // 32, 2, 16)
+        want = (torch.nn.functional.silu(pair[:, :, 0]) * pair[:, :, 1]).reshape(n, m // 2)
+        assert ((z.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
 @pytest.mark.parametrize("n", [8, 9, 16, 25, 33, 49, 64])
