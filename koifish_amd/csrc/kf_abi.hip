@@ -340,9 +340,9 @@ int kf_quantize(kf_ctx* c, const kf_weight* w, const kf_bf16* src, int symmetric
 
 static void init_args(kf_ctx* c, kf::GemvLaunch& L) { memset(&L, 0, sizeof(L)); L.args.alpha = 1.0f; L.canon = c->canonical; }
 
-// token rows from which a layer's seven matrices are dequantised by one launch (kf_layer_copies) for the bf16 tile kernels.  One product in registers | on a copy that is there, us: 1024 x 2048 at 256
-// tokens 9.8 | 10.8, at 320 16.3 | 10.8, at 2047 30.5 | 16.8;  1024 x 3072 at 256 12.6 | 14.3, at 320 20.5 | 19.0, at 2047 43.9 | 30.2;  4096 x 1024 at 320 17.5 | 10.0;  6144 x 1024 at 320 20.5 | 12.4;
-// the launch itself 10 us for those.  A launch per matrix gives that back: 2047 tokens 1024 x 2048 30.5 | 26.8, 512 tokens 16.5 | 22.5.
+// token rows from which a layer's seven matrices are dequantised by one launch (kf_layer_copies) for the bf16 tile kernels.  ms per layer of a prompt in registers at 319 rows | on copies at 320: 0.6B
+// 0.128 | 0.118, 1.7B 0.289 | 0.179, 4B 0.445 | 0.254, 8B 0.661 | 0.418, 32B 1.135 | 0.873 (the launch itself 8 us for a 0.6B layer's 31 MB of copies); at 1023 rows 0.234 | 0.141 to 2.08 | 1.52.  A launch per
+// matrix gives part of that back: 0.6B, 1024 rows 0.190.  At 256 rows one product in registers is the faster one (1024 x 2048 9.8 | 10.8 us, 1024 x 3072 12.6 | 14.3).
 static const int KF_LAYER_COPIES_MIN = 320;
 static const int KF_DEQ_GEMM_MIN = 2048; /* token rows from which a quantised weight is dequantised by a launch of its own and multiplied by the bf16 tile kernel (when scratch was handed over) */
 size_t kf_linear_scratch_bytes(const kf_weight* w, int nTok) {

@@ -4,10 +4,10 @@
 //     such a load is lane-linear, so the bank-conflict-free layout is produced on the SOURCE side: a tile row is 128 bytes = 8 chunks of 16 bytes, chunk c of row r
 //     is stored at position c ^ ((r >> 1) & 7); a fragment read (16 rows x one chunk, ds_read_b128) then touches all 64 banks exactly once;
 //     a k-major operand's image is [64 k][rows], two-term swizzle, fragments by the transposing ds_read_b64_tr_b16 (g3_frag_km);
-//   * two LDS buffers: the loads of a later k-step are issued among the MFMAs of this one, the fragments of a quadrant are read while the one before is multiplied, a COUNTED s_waitcnt vmcnt and
-//     raw s_barriers (a __syncthreads() would drain the loads in flight);
-//   * 256 x 256: 8 waves as 2 (rows) x 4 (tokens), 128 x 64 outputs per wave = 32 accumulator tiles of v_mfma_f32_16x16x32_bf16, one workgroup per CU; 192 x 256 where the last round of those would be
-//     nearly empty; 128 x 128: 4 waves as 2 x 2, 64 x 64 outputs per wave, two workgroups per CU -- for products with too few big tiles to fill the chip; 64 x 128 and 64 x 64 below that;
+//   * two LDS buffers: the loads of a later k-step are issued among the MFMAs of this one, the fragments of a quadrant are read while the one before is multiplied, and ONE raw s_barrier per
+//     step, behind a wait for everything that was issued a step earlier (in front of the loop only the first step's loads are waited for, by count);
+//   * 256 x 256: 8 waves as 2 (rows) x 4 (tokens), 128 x 64 outputs per wave = 32 accumulator tiles of v_mfma_f32_16x16x32_bf16, one workgroup per CU; 192 x 256 where those fill the chip's
+//     rounds better; 128 x 128: 4 waves as 2 x 2, 64 x 64 outputs per wave, two workgroups per CU -- for products with too few big tiles to fill the chip; 64 x 128 and 64 x 64 below that;
 //   * workgroup order remapped so that the blocks an XCD runs back to back share their W row-tile in that XCD's L2;
 //   * split-K forms (gemm3_sk_kernel) with an ordered in-kernel fix-up for launches with fewer tiles than resident workgroups: deterministic, no atomics on data;
 //   * up to three matrices stacked along M (Q | K | V, gate | up) in one launch, each tile's rows routed to its matrix's output (gemm3_multi_launch).
@@ -405,7 +405,7 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
     const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
     if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || nkt >= 48)) {
         G3SkArgs s;
-        // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they moved with it,
+        // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they would move with it,
         // and another configuration's fp32 partials could overwrite words already marked "seen" with values that pass for an epoch)
         static_assert((size_t)256 * C::WGS_PER_CU * C::BM * C::BN * 4 <= (size_t)256 * G3_BM * G3_BN * 4 && 256 * C::WGS_PER_CU * 4 <= G3_SK_FLAG_BYTES, "partials and flags fit the lent workspace");
         s.ws = (float*)ws, s.flags = (uint32_t*)((char*)ws + gemm3_sk_ws_bytes() - G3_SK_FLAG_BYTES);
@@ -448,14 +448,13 @@ int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws
         }
     }
     // 128 x 128 tiles, two workgroups per CU: bf16 products of 1-4 k rows whose M is 1024-3072 (M 1024 x K 2048 at 2048 rows: 36.9 -> 27.4 us, 3072 x 1024: 35.6 -> 23.9;
-    // 4096 rows: 583-656 TFLOP/s).  For QUANTISED weights of that size dequantise + this kernel only ties with the in-register-unpack kernels (the 5 us dequantise pass
-    // and, with split-K, the flag memset eat the gain): kf_linear keeps those on kf_gemm.hip.
+    // 4096 rows: 583-656 TFLOP/s); a quantised weight of that size reaches them as a layer's or a resident copy (a dequantise pass of its own gives the gain back).
     if (a.n < 128 || a.M < 128) return 1;
     const long nwg = (long)((a.M + 127) / 128) * ((a.n + 127) / 128);
     if (nwg < 32 && (g_knobs.g3_tiles < 3 || (long)((a.M + 63) / 64) * ((a.n + 63) / 64) < 64)) return 1;
     if (nwg < 256 && g_knobs.g3_tiles >= 1 && !a.swiglu && !a.qkrope) { /* fewer 128 x 128 tiles than CUs: twice or four times as many smaller ones */
-        // with the caller's workspace these go in k-pieces when even the small tiles leave CUs idle (1024 rows x K 2048-3072 at 512 tokens: 128 tiles of 64 x 64, each a
-        // 32-48 step k-loop of ~0.7 us per step on its own CU: 31 us; a 16 KiB partial per piece is cheap where the 64 KiB ones of the 128 x 128 tile were not)
+        // with the caller's workspace these go in k-pieces (g3_go_c says when): 1024 rows x K 2048-3072 at 512 tokens are 128 tiles of 64 x 64, each a 32-48 step k-loop on its own CU.  A partial
+        // is 16 or 32 KiB; the 64 KiB ones of the 128 x 128 tile cost more than they gave (37.8 us against 27 whole)
         const long nmid = (long)((a.M + 63) / 64) * ((a.n + 127) / 128);
         if (nmid >= g_knobs.g3_mid_min || g_knobs.g3_tiles < 3) return nmid >= 64 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 64) : 1;
         return g3_go_c<false, false, G3Tiny>(st, a, (long)((a.M + 63) / 64) * ((a.n + 63) / 64), ws, ws_bytes, 64);

@@ -19,8 +19,8 @@ struct G3Cfg {
 };
 using G3Big = G3Cfg<256, 256, 8>;
 using G3Small = G3Cfg<128, 128, 4>;
-// round 4: products whose 128 x 128 tiles do not fill the chip either (M = 1024 at 1-2 k tokens: 64-128 of them; split-K S = 4 measured 37.8 us against 27 plain: three
-// 64 KiB partials per tile through memory) get MORE, SMALLER tiles instead of k-pieces: 64 x 128 (48 KiB of LDS: three workgroups per CU) and 64 x 64 (32 KiB: five)
+// products whose 128 x 128 tiles do not fill the chip either (M = 1024 at 1-2 k tokens: 64-128 of them; four k-pieces of those measured 37.8 us against 27 plain: three
+// 64 KiB partials per tile through memory) get MORE, SMALLER tiles, these in k-pieces where a workspace is lent: 64 x 128 (48 KiB of LDS: three workgroups per CU) and 64 x 64 (32 KiB: five)
 using G3Mid = G3Cfg<64, 128, 4>;
 using G3Tiny = G3Cfg<64, 64, 4>;
 // 192 x 256: a product whose 256 x 256 tiles number 160-255 (gate | up of a 0.6B model at 2047 tokens: 24 x 8 = 192 tiles on 256 CUs) becomes 32 x 8 = 256 tiles of 3/4 the work
