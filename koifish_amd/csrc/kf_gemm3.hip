@@ -399,9 +399,9 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
         attr_set = 1;
     }
     // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; a K-contiguous product of K < 3072 only where three pieces of
-    // every tile find room.  us per layer of prompts, never | from K = 3072 | three pieces: 0.6B, resident copies, 320 rows 134 | 116 | 106, 1024 rows 149 | 143 | 137, 2047 rows 198 | 190 | 187; a layer's
-    // copies 119 | 111 | 105, 136 | 134 | 130, 190 | 187 | 185;  1.7B resident 320 rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800
-    // rows 325 -> 332 us.  (One product by itself on operands that are in the L2 already shows the opposite: 1024 x 2048 at 512 rows 11.2 whole, 12.6 in four pieces.)
+    // every tile find room.  us per layer of prompts on resident copies, never | from K = 3072 | three pieces: 0.6B 320 rows 134 | 116 | 106, 1024 rows 149 | 143 | 137, 2047 rows 198 | 190 | 187; 1.7B 320
+    // rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800 rows 325 -> 332 us.  (One product by itself on operands that are in the L2
+    // already shows the opposite: 1024 x 2048 at 512 rows 11.2 whole, 12.6 in four pieces.)
     const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
     if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || nkt >= 48)) {
         G3SkArgs s;
