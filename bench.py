@@ -139,7 +139,7 @@ def main():
     layer_type = {"q4": L.Q4, "bf16": L.BF16, "f8": L.F8E5M2, "ternary": L.T_SIGN, "1bit": L.BOOL1, "nf4": L.NF4}[args.layers]
     m = synth.build_on_gpu(cfg, seed=1234 + rank, layer_type=layer_type, head_type=head_type, device=dev)
     _lap("model built")
-    m.set_prefill_resident(True, 96 << 30)   # opt-in (library default: off): this run never changes a weight in place, so long prompts may keep bf16 copies of the layer matrices in HBM
+    m.set_prefill_resident(True, 96 << 30)   # opt-in (library default: off, a layer's copies written anew by every prompt): this run never changes a weight in place, so long prompts may keep bf16 copies of the layer matrices in HBM
     ctx = m._ctx
     hots = {}
     if args.sparse > 0.0:
@@ -917,7 +917,7 @@ def prefill_rate(m, prompt, decode_ms_per_step, reps=5, bound=None):
     nbytes = sum(w.algorithmic_bytes() for (layer, slot), w in m.weights.items() if layer >= 0) + m.weights[(-1, 1)].algorithmic_bytes() + n * cfg["dim"] * 2 \
         + cfg["n_layer"] * n * kvd * 2 * 2 * 2
     tf, gbs = flops / (ms * 1e-3) / 1e12, nbytes / (ms * 1e-3) / 1e9
-    return {"prompt_tokens": n, "ms": round(ms, 3), "tokens_per_s": round(n / ms * 1e3, 1), "mode": "token batches: < 320 rows MFMA 32x32x16 bf16 on 4-bit tiles unpacked in registers; >= 320 rows the 256x256 / 128x128 bf16 tile kernels (MFMA 16x16x32; SwiGLU and q/k-norm + RoPE in their epilogues) on RESIDENT bf16 copies of the layer matrices (dequantised by the first such prompt, kept in HBM); flash attention tile",
+    return {"prompt_tokens": n, "ms": round(ms, 3), "tokens_per_s": round(n / ms * 1e3, 1), "mode": "token batches: < 320 rows MFMA 32x32x16 bf16 on 4-bit tiles unpacked in registers; >= 320 rows the 256x256 / 128x128 bf16 tile kernels (MFMA 16x16x32; SwiGLU and q/k-norm + RoPE in their epilogues) on bf16 copies of the layer matrices: resident ones where resident_copy_bytes > 0 (dequantised by the first such prompt, kept in HBM), else a layer's own, written by one launch per layer and prompt; flash attention tile",
             "first_call_ms": round(first_ms, 3), "resident_copy_bytes": m.resident_bytes(),
             "token_serial_ms": round(decode_ms_per_step * n, 3),
             "roofline": {"flops": int(flops), "bytes": int(nbytes), "achieved_TFLOPs": round(tf, 2), "mfma_peak_TFLOPs": MFMA_BF16_PEAK_TFLOPS, "mfma_frac": round(tf / MFMA_BF16_PEAK_TFLOPS, 4),
