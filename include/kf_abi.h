@@ -4,7 +4,7 @@
  * its name starts with h_.  All functions return 0 (KF_OK) or a negative KOIFISH_* code
  * (src/g_def_x.hpp:21-83) and never exit(); kf_last_error() returns the text.
  *
- * Each entry point replaces one seam of the reference (SURVEY.md section 8b); the seam is cited as
+ * Each entry point replaces one seam of the reference; the seam is cited as
  * file:line into gruai/koifish.  A kf_ctx is single-threaded by contract (the reference drives one
  * stream from one host thread, NeuronFuse.cu:29); kernels never allocate (GTensor owns memory).
  * bf16 is carried as uint16_t bit patterns (floatX = floatGama = __nv_bfloat16, g_float.hpp:246-262).
@@ -134,7 +134,7 @@ int kf_quantize(kf_ctx* ctx, const kf_weight* w, const kf_bf16* src, int symmetr
  * much a weight needs (0 for every PackedQ / bf16 / f8 weight), kf_set_scratch hands the context a buffer (device memory, 16-byte aligned, the caller's
  * to free after the last call that used it; not while capturing, since captured launches hold the pointer).  Too small or missing: KF_INVALID_ARGS. */
 /* Summation order of the decode kernels (mat-vecs, LM head, decode attention, the persistent engine's mat-vec phases).
- *   1 (the default since round 4): the CANONICAL order kernels and the CPU oracle share (oracle/kf_oracle.c sections 4c and 6 "CANON"): every lane keeps two fused
+ *   1 (the default): the CANONICAL order kernels and the CPU oracle share (oracle/kf_oracle.c sections 4c and 6 "CANON"): every lane keeps two fused
  *     multiply-add chains (even / odd elements: one v_pk_fma_f32 per weight pair) joined by a balanced tree, the softmax works on exact power-of-two scalings with
  *     fp64 sums -- logits, greedy ids and KV rows equal the oracle's BIT FOR BIT (tests/test_gpu_canonical.py, bench.py cpu_baseline parity pass).  It is the order
  *     bench.py times.  (The persistent engine follows the switch in every phase: mat-vecs, attention slice, head.)
@@ -168,7 +168,7 @@ int kf_layer_copies_end(kf_ctx* ctx);
 int kf_linear(kf_ctx* ctx, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const kf_bf16* bias, int nTok, float alpha, float beta,
               uint32_t epilogue, const kf_bf16* residual);
 
-/* ---- tensor parallel (no counterpart in the reference, which is single-GPU: QKV.cu:503; SURVEY.md section 8e) ----
+/* ---- tensor parallel (no counterpart in the reference, which is single-GPU: QKV.cu:503) ----
  * column-split projections (o_proj, down_proj) give un-rounded fp32 partial row dots per rank ... */
 int kf_linear_f32(kf_ctx* ctx, const kf_weight* w_shard, const kf_bf16* x_shard, float* y_partial);
 /* ... that are combined in rank order after an all-gather: out = bf16(residual + bf16(sum_r partials[r][:])) */
@@ -274,7 +274,7 @@ int kf_set_state(kf_ctx* ctx, int32_t* d_state, int token, int pos);
 int kf_embed_state(kf_ctx* ctx, const kf_weight* w, const int32_t* d_state, const int32_t* d_forced, kf_bf16* out);
 
 /* GeneratOnPrompt::Sample, non-greedy branch (GoPT.cpp:614-630; LogitsInfo::TopK / UpdateLogits / TopP / Qu_FlipCoin, GoPT.cpp:632-790):
- * picks the next token from bf16 logits[n] on the device -- candidate set exactly as TOPK_heap::Select builds it (see DESIGN.md: indices
+ * picks the next token from bf16 logits[n] on the device -- candidate set exactly as TOPK_heap::Select builds it (indices
  * 0..k-2 plus the first maximum over i >= k-1), softmax with temperature, top-p cut, xorshift64* coin.  d_rng_state: one uint64 in device
  * memory (LogitsInfo::rng_state, seeded with config.common.seed), advanced once per call.  Writes *d_token (when non-NULL) and, when
  * d_state is non-NULL, the decode-state update of kf_norm_lm_head.  temperature == 0 or top_k == 1 is the greedy path: use kf_lm_head.
@@ -290,7 +290,7 @@ int kf_sample(kf_ctx* ctx, const kf_bf16* logits, int n, int top_k, float temper
 int kf_sample_topk(kf_ctx* ctx, const kf_bf16* logits, int n, int top_k, float temperature, float top_p, uint64_t* d_rng_state, int32_t* d_token,
                    int32_t* d_state, int32_t* d_tokens_out, const int32_t* d_forced, int n_forced);
 
-/* ---- GPT-2 family forward pieces (BASELINE config 3) */
+/* ---- GPT-2 family forward pieces */
 /* LayerNorm forward with affine weight and bias (LayerNormal::cuFlow for the GPT-2 family -> CU_lm_forward, layernorm.cuh:226-300):
  * y = bf16((x - mean) * rstd * w + b), rstd = 1/sqrtf(var + eps); bias may be NULL; mean / rstd [rows] fp32 are optional outputs. */
 int kf_layernorm(kf_ctx* ctx, const kf_bf16* x, const kf_bf16* w, const kf_bf16* bias_or_null, kf_bf16* y, int rows, int dim, float eps, float* mean_or_null,
@@ -387,7 +387,7 @@ int kf_swiglu_backward(kf_ctx* ctx, kf_bf16* delta_in_out, kf_bf16* delta_gate, 
 int kf_fused_classifier(kf_ctx* ctx, kf_bf16* logits, float* losses, kf_bf16* probs_or_null, float dloss, const int32_t* targets, int B, int T, int V, int P,
                         const int32_t* mask_or_null, int write_dlogits);
 
-/* ---- training kernel path (BASELINE config 3), first piece: the AdamW parameter update CU_adamw_p (src/Device/CUDA/Optimizer.cu:393-442)
+/* ---- training kernel path, first piece: the AdamW parameter update CU_adamw_p (src/Device/CUDA/Optimizer.cu:393-442)
  * as PIPE_Adamw::Update launches it (Optimizer.cu:630-646; TASKA_1p1, packedN.cuh:612-643: 512 threads x 8 bf16 per thread).
  * params / grads bf16 [n] (grads are zeroed), gm / gv: first and second moments, mv_type KF_BF16 (floatMV = bf16) or KF_F32.
  * g = grad_scale*grad; m = sAtB(g, m, beta1); v = sAtB(g*g, v, beta2); step = (m/beta1_correction) / (sqrtf(v/beta2_correction) + eps);
@@ -500,7 +500,7 @@ int kf_engine_check(kf_ctx* ctx, kf_engine* e); /* synchronises; KF_INTERNAL_ERR
 int kf_engine_reset(kf_ctx* ctx, kf_engine* e);
 int kf_engine_destroy(kf_engine* e);
 
-/* ---- EIGHT decoders per GPU, one per XCD, for up to 32 independent sequences (kf_xengine.hip; rounds 5 - 6).  The reference decodes ONE sequence per process (Fish::Chat, GoPT.cpp:1139-1180) and
+/* ---- EIGHT decoders per GPU, one per XCD, for up to 32 independent sequences (kf_xengine.hip).  The reference decodes ONE sequence per process (Fish::Chat, GoPT.cpp:1139-1180) and
  * scales a small model by running more processes; on this part a single sequence cannot keep the HBM busy (its step is a chain of hand-offs), so the replicas move
  * INSIDE the package: the 32 workgroups of XCD s are the decoder of sequence s, every hand-off stays in that XCD's L2, and the chip streams eight sequences' bytes at
  * once.  The sequences share the weights (the kf_engine_desc's layer table, the embedding, the head) and nothing else; per sequence: a K/V cache (sequence s at
@@ -508,12 +508,12 @@ int kf_engine_destroy(kf_engine* e);
  * (logits + s * vocab), the residual stream out (x_out + s * dim).  Each sequence's ids, logits and K/V rows are bit for bit those kf_engine_steps_head, the per-layer
  * calls and the oracle give for that sequence alone (canonical order only: kf_set_canonical(ctx, 0) is refused).  One workgroup per CU, 32 per XCD: the launch must have
  * the GPU to itself (bounded polls, error word, kf_xengine_check / _reset as for kf_engine).  Sequences may stand at different positions.
- * n_seq <= 8: sequence s on XCD s, one workgroup per CU.  More (round 6): still ONE decoder per XCD, each decoding 2 (n_seq <= 16) or 4 (n_seq <= 32) sequences -- XCD x takes
+ * n_seq <= 8: sequence s on XCD s, one workgroup per CU.  More: still ONE decoder per XCD, each decoding 2 (n_seq <= 16) or 4 (n_seq <= 32) sequences -- XCD x takes
  * sequences x, x + 8, x + 16, x + 24.  Every 4-bit block a decoder streams is unpacked ONCE (the exact bf16-stepwise dequantisation, T.cu:274, is what bounds these engines) and
  * multiplied against the activations of all its sequences; each sequence keeps its own canonical chains, attention, K / V cache and state, so its bits do not change.
  * Served: 4-bit PackedQ (RTN, groups of 128) layers of the Qwen3-0.6B, 1.7B, 4B and 8B shapes (and two small test shapes), bf16 embedding / head; more than 8
- * sequences for the 0.6B / 1.7B shapes (1.7B: at most 16), more than 16 for the 0.6B shape.  Round 6: 1-bit and 2-bit PackedQ (YinYang) layers for the 0.6B shape and the 256-wide
- * test shape (1-bit: BASELINE config 5's storage), and FFNs with a hot-row mask (kf_engine_layer::hot_ffn: a cold gate / up row publishes a zero, D_matmul_sparse).  Weights are read in place and must not
+ * sequences for the 0.6B / 1.7B shapes (1.7B: at most 16), more than 16 for the 0.6B shape.  1-bit and 2-bit PackedQ (YinYang) layers for the 0.6B shape and the 256-wide
+ * test shape, and FFNs with a hot-row mask (kf_engine_layer::hot_ffn: a cold gate / up row publishes a zero, D_matmul_sparse).  Weights are read in place and must not
  * change while an engine built on them lives; for the GQA-4 shapes (and the TP form below) the engine keeps a fused COPY of every layer's q | k | v rows in its workspace, made at
  * create time: after a weight update destroy the engine and create it again.
  * d_state [n_seq][4] = {token, pos, parked, status}.  parked != 0: the launch skips the sequence (the other sequences of its decoder go on).  A launch one of whose positions
@@ -534,7 +534,7 @@ int kf_xengine_steps(kf_ctx* ctx, kf_xengine* e, kf_bf16* x_out, int32_t* d_stat
 int kf_xengine_check(kf_ctx* ctx, kf_xengine* e); /* synchronises; KF_INTERNAL_ERR when a hand-off poll has timed out since creation or the last kf_xengine_reset */
 int kf_xengine_reset(kf_ctx* ctx, kf_xengine* e);
 int kf_xengine_destroy(kf_xengine* e);
-/* Tensor parallel over the XCDs (round 5): ONE sequence of a model whose TP = 8 ranks (koifish_amd/tp.py TPPlan; the partitioning of SURVEY 8e) run as the eight XCDs of one
+/* Tensor parallel over the XCDs: ONE sequence of a model whose TP = 8 ranks (koifish_amd/tp.py TPPlan) run as the eight XCDs of one
  * launch -- rank r's 32 workgroups stream rank r's shards; q | k | v, the attention of the rank's kv-head and gate | up stay inside the XCD; the column shards (o_proj, down_proj)
  * leave as fp32 partials into every rank's receive area (the {value | generation} protocol of kf_tp_*, inside the launch), summed in rank order: the bits of kf_tp_reduce_recv.
  * Served: the ranks of Qwen3-32B (per rank: dim 5120, 8 / 1 heads of 128, ffn 3200), 4-bit PackedQ layers, bf16 embedding (replicated) and head (vocabulary shards).

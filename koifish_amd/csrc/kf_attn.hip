@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(const AttnArgs a) {
     if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// ---- the fp32 form of rounds 1-2 (kf_set_canonical(ctx, 0), the default): scores by v_dot2c_f32_bf16, exp by v_exp_f32(x * log2 e), a workgroup-wide running
+// ---- the fp32 form (kf_set_canonical(ctx, 0), the default): scores by v_dot2c_f32_bf16, exp by v_exp_f32(x * log2 e), a workgroup-wide running
 // maximum, fp32 sums, slices merged with fp32 exponentials.  <= 1 bf16 ulp / 2^-10 of the scale from the oracle's FUSED mode; about half the vector work of the
 // canonical form above (no fp64).  Partials: [n_head][n_splits][hd + 4] floats in the same scratch.
 template <int GQ, int NW, int HD>
@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(64) qknorm_rope_kernel(uint16_t* q, uint16_t* 
 int attn_splits(int pos_bound, int n_kv) {
     // keys per slice: one workgroup streams a slice in batches of 64 keys (hd 128, 4 waves); short contexts stay in ONE slice per
     // kv-head (no cross-workgroup hand-off at all), long ones are cut so that the chip is covered.
-    constexpr int slice = 64, single = 192; /* keys per slice / longest context served by one slice (settled by the round-1 sweeps) */
+    constexpr int slice = 64, single = 192; /* keys per slice / longest context served by one slice (settled by sweeps of both) */
     const int len = pos_bound + 1;
     if (len <= single) return 1;
     int nsp = (len + slice - 1) / slice;

@@ -171,7 +171,7 @@ __device__ __forceinline__ void canon_apply_items(CanonAcc<GQ>& A, double p, con
         canon_apply_items<GQ, U, I + 1>(A, p, vd);
     }
 }
-// (Round 6, measured and removed: two query heads per v_pk_fma_f32 / v_pk_mul_f32 / v_pk_add_f32 in the score chain and in the exponential's polynomial -- bit-identical (179
+// (Measured and removed: two query heads per v_pk_fma_f32 / v_pk_mul_f32 / v_pk_add_f32 in the score chain and in the exponential's polynomial -- bit-identical (179
 //  canonical tests), half the vector instructions of those two parts, and slower: the single-sequence engine 2304 -> 2103 tokens/s, 32 batched sequences 7770 -> 7410: the operand
 //  pairs have to be assembled in even-aligned register pairs per use.)
 #ifndef KF_CANON_ITEMS
@@ -180,7 +180,7 @@ __device__ __forceinline__ void canon_apply_items(CanonAcc<GQ>& A, double p, con
                             broadcast is a DPP move with its wait states in front of a dependent fp64 chain; the replicated form keeps sixteen independent lanes busy instead).  Off. */
 #endif
 // one batch of U key tiles of this lane's key group: k / v tiles (8 elements of this lane), validity per tile; q as 8 floats per head
-// KF_CANON_ITEMS (round 6, measured and left off): hd = 128, a key group is a row of 16 lanes -- the U * GQ dots of a group stand in all of its 16 lanes after the tree; the
+// KF_CANON_ITEMS (measured and left off): hd = 128, a key group is a row of 16 lanes -- the U * GQ dots of a group stand in all of its 16 lanes after the tree; the
 // score's scale and rounding, the exponential's parts and the exact power-of-two weight p worked out ONCE, item i = u * GQ + hq in lane i of the group, p_i handed to the
 // group's lanes by a row broadcast: the same operations on the same values as the per-lane form.
 template <int GQ, int LPK, int U = ATTN_U>

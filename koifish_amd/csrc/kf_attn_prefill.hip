@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256 * KH) attn_prefill_kernel(const AttnPrefil
         for (int s = 0; s < NS; s++) qf[s] = *reinterpret_cast<const u32x4*>(qrow + 16 * s + 8 * h);
     }
 
-    // K / V tiles travel global -> registers -> LDS.  Round 4: TWO register sets, a tile's loads are issued two steps before it is multiplied (the step that follows the issue
+    // K / V tiles travel global -> registers -> LDS.  TWO register sets, a tile's loads are issued two steps before it is multiplied (the step that follows the issue
     // stores the OTHER set): with one set the loads of step j + 1 had only step j's arithmetic (~0.4 us) to land in, and a step took what the load took (~2 us from the
     // fabric at one workgroup per CU: 67 us for 32 steps at 2047 tokens).
     // (KH = 1 -- more workgroups than CUs, two resident per CU hide each other's loads -- keeps one set: a second one takes it past 256 registers.)

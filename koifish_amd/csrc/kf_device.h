@@ -242,7 +242,7 @@ __device__ __forceinline__ float perm_dot_dword(uint32_t D, u32x4 X, const PermL
 // order -- so that the fp32 sum is formed in exactly the order of dot_q4_dword (kf_gemv.hip): two extra v_perm_b32 per dword gather the index bytes
 // (low nibble of a byte of D >> 4 = an even element, of D = an odd element; the lookup ignores the high nibbles).
 // (the pair product of kf_gemv_blocks.h, stated here for the lookup below)
-// ---- the accumulator of one lane's mat-vec chain.  Default order: one float fed by v_dot2c_f32_bf16.  Canonical order (oracle/kf_oracle.c section 4c, round 4):
+// ---- the accumulator of one lane's mat-vec chain.  Default order: one float fed by v_dot2c_f32_bf16.  Canonical order (oracle/kf_oracle.c section 4c):
 // TWO fused multiply-add chains per lane -- the even-indexed elements of the lane's blocks into .x, the odd-indexed into .y, both through one v_pk_fma_f32 per
 // weight pair (each half is an IEEE fma: fmaf on the host) -- joined as x + y in front of the lane tree.
 template <bool CANON>

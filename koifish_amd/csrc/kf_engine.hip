@@ -8,7 +8,7 @@
 //   P5 [RMSNorm + gate/up + SwiGLU]  P6 [down_proj + residual]
 //
 // because on this chip a dependent launch boundary plus the setup and first HBM miss of the next kernel costs ~3 us while a layer's
-// 8.4 MB of weights stream in ~1.3 us (DESIGN.md, scratch/ub_overlap.hip).  One workgroup of 8 waves per CU:
+// 8.4 MB of weights stream in ~1.3 us (scratch/ub_overlap.hip).  One workgroup of 8 waves per CU:
 //
 //   * wave 7 ("poller") waits for the phase's input vector and stages it into LDS.  Producers publish every output as a tagged
 //     granule -- one aligned 4-byte {bf16 value, 16-bit generation} (attention partials: 8-byte {fp32, 32-bit generation}) written by
@@ -217,7 +217,7 @@ __device__ __forceinline__ void mv_prefetch(const EngMat m, const EngMat m2, int
 #ifndef ENG_COOP
 #define ENG_COOP 1 /* the norm-free vectors (ao, act) are swept by all eight waves */
 #endif
-// the wave's blocks as bf16 pair words (BlockPrep): formed while the wave waits for the phase's activations.  (Round 4 also widened them to the fp32 operand pairs of the
+// the wave's blocks as bf16 pair words (BlockPrep): formed while the wave waits for the phase's activations.  (Widening them to the fp32 operand pairs of the
 // canonical v_pk_fma_f32 in front of the barrier: 32 registers per block -- the kernel spilled 30 - 180 registers and ran 20 % slower; the two conversions per pair stay behind
 // the barrier, where they fill the bubbles of the dependent fma chains.)
 template <bool PAIRED, int MAXS>
@@ -701,7 +701,7 @@ __device__ __forceinline__ void eng_poller_main(const EngArgs& a, const EngLds& 
                 mv_prefetch<P1, NCW1, FMT, S1>(mat1(ln), mat1(ln), S.s1, NWV - 1, lane, S.M1, r1);
             }
             eng_attn_phase<C>(a, L, S, ly, gen, tag, NWV - 1, lane, T, l, wg);
-            /* the next layer's tiles (the last layer asks for its own again).  Round 4 moved this request of the poller behind the merge's sweep (loads return in order: the sweep's
+            /* the next layer's tiles (the last layer asks for its own again).  Moving this request of the poller behind the merge's sweep (loads return in order: the sweep's
                answer might wait for these sixteen HBM lines) and, with a second register set, in front of the attention phase: 387 / 392 us per launch against 383 / 390 here --
                the ao store then queues behind the tile requests, and the earlier sweep mostly comes too early */
             if (!S.empty) eng_attn_issue<C>(a, L.lay[l + 1 < a.n_layer ? l + 1 : l], S, NWV - 1, lane, T, 0);
@@ -1289,7 +1289,7 @@ struct EngineHost {
 
 // the instantiated model shapes: {GQA group, head_dim, dim, q_dim, ffn}
 static int engine_shape_class(int GQ, int hd, int dim, int q_dim, int ffn) { /* kv_dim = q_dim / GQ */
-    if (GQ == 2 && hd == 128 && dim == 1024 && q_dim == 2048 && ffn == 3072) return 1; /* Qwen3-0.6B (BASELINE config 2) */
+    if (GQ == 2 && hd == 128 && dim == 1024 && q_dim == 2048 && ffn == 3072) return 1; /* Qwen3-0.6B */
     if (GQ == 2 && hd == 64 && dim == 256 && q_dim == 256 && ffn == 512) return 2;     /* the small parity-test shape */
     if (GQ == 2 && hd == 128 && dim == 2048 && q_dim == 2048 && ffn == 6144) return 3;  /* Qwen3-1.7B: the 0.6B head geometry on a 2048-wide stream (4-bit register-table storage only) */
     return 0;
@@ -1403,7 +1403,7 @@ int engine_build(const kf_engine_desc* d, void* ws, size_t ws_bytes, hipStream_t
     const kf_engine_layer& L0 = d->layers[0];
     int fmt = gemv_fmt_of(&L0.w[0]);
     *why = "layer storage not served: the engine is instantiated for 4-bit (RTN), 2-bit and 1-bit PackedQ layers in groups of 128; other storages keep the per-layer launches";
-    if (fmt != FMT_Q4 && fmt != FMT_Q1 && fmt != FMT_Q2) { /* the engine is instantiated for the 4-bit PackedQ storage (BASELINE config 2); other storages keep the per-layer launches */
+    if (fmt != FMT_Q4 && fmt != FMT_Q1 && fmt != FMT_Q2) { /* the engine is instantiated for the 4-bit PackedQ storage; other storages keep the per-layer launches */
         delete E;
         return KF_UNSUPPORTED_DATATYPE;
     }
@@ -1652,7 +1652,7 @@ int engine_error_word(EngineHost* E, hipStream_t st, int* h_err) {
 }
 void engine_set_canonical(EngineHost* E, int on) { E->canon = on ? 1 : 0; }
 
-// ---- self-calibration of the first-sweep delays (VERDICT r03 item 1c).  The hand-off protocol is correct for ANY delay -- a sweep that comes too early is repeated -- but a
+// ---- self-calibration of the first-sweep delays.  The hand-off protocol is correct for ANY delay -- a sweep that comes too early is repeated -- but a
 // repeated sweep costs its whole round trip on the critical path and a late one its lateness, and the best values depend on the device (clocks, fabric) and on how many
 // slices the context is cut into.  engine_tune times the layers-only launch at the position the decode state holds (it reads the state's token and writes that position's
 // K / V rows, as the real step is about to: idempotent, nothing advances) and walks the six delays by coordinate descent, smallest mean launch time wins.

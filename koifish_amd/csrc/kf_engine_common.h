@@ -1,5 +1,5 @@
 // kf_engine_common.h -- what the two persistent decode engines share: kf_engine.hip (one sequence on all 256 CUs, weights in registers ahead of every hand-off) and
-// kf_xengine.hip (round 5: eight independent sequences, one per XCD, every hand-off through that XCD's L2, weights streamed): the device tables, the tagged-granule
+// kf_xengine.hip (eight independent sequences, one per XCD, every hand-off through that XCD's L2, weights streamed): the device tables, the tagged-granule
 // accessors, and the mat-vec phase geometry as compile-time types (the lanes per row, rows per wave step and steps per row gemv_launch picks for the same matrices: the
 // canonical summation order is a property of the matrix shape, not of how many workgroups share the rows).
 #pragma once

@@ -6,7 +6,7 @@
 // per lane in registers with the reference's bf16-stepwise arithmetic (T.cu:274) straight into an MFMA A-fragment, and contracts on
 // v_mfma_f32_32x32x16_bf16 against x fragments staged through LDS.
 //
-// Fragment mapping (cdna_hip_programming.md section 3): for the 32x32x16 bf16 MFMA lane l (r = l & 31, h = l >> 5) holds
+// Fragment mapping: for the 32x32x16 bf16 MFMA lane l (r = l & 31, h = l >> 5) holds
 // A[row r][k = 8h + j] and B[k = 8h + j][col r], j = 0..7; D has col = l & 31, row = (reg & 3) + 8 (reg >> 2) + 4 h.
 // A = weights (rows = output features), B = x^T (cols = tokens).  The contraction index may be visited in any order as long as A and B
 // agree, so the two lane halves do not take k and k+8 of one 16-wide step: over a staged tile of 128 k, half h owns whole 16-byte

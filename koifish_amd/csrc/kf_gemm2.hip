@@ -2,7 +2,7 @@
 //
 // Same contract as kf_gemm.hip (y[n, M] = x[n, K] . W[M, K]^T, fp32 accumulate in the MFMA, one bf16 store, the mat-vec's epilogue
 // order); used when a batch has at least 256 token rows and the grid fills the chip.  What the PMC passes on the first tile kernel
-// showed (DESIGN.md section 8: 58 % of the wave cycles parked on waits, MFMA busy 18 %, one wave per SIMD) is answered structurally:
+// showed (58 % of the wave cycles parked on waits, MFMA busy 18 %, one wave per SIMD) is answered structurally:
 //
 //   * 8 waves per workgroup = 2 per SIMD, specialised.  Waves 0..3 PRODUCE: they stream the packed weight tile (coalesced: consecutive
 //     lanes read consecutive 16-byte blocks of a row) and the x tile, unpack every weight ONCE per workgroup with the reference's

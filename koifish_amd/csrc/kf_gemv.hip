@@ -45,7 +45,7 @@ struct Batch {
 // Each wave keeps two batches of G blocks in flight: the first batch is issued BEFORE the x prologue so that the
 // weight stream's HBM latency overlaps the (dependent) activation load + norm.
 // ONEJOB: a launch with a single matrix (o_proj, down_proj, LM head, sparse rows) never reads the descriptors of jobs 1 and 2: kernel arguments are fetched ahead of the
-// first load, and every one a launch touches is on its critical path (DESIGN.md section 0)
+// first load, and every one a launch touches is on its critical path
 // XF (canonical 4-bit forms only, chosen by the launcher when K * 4 bytes of LDS leave the occupancy alone): x is staged as fp32 chunks [8][nBlk] and multiplied through
 // BlockDotF (the engine's form): a product is two conversions of the weight pair + one v_pk_fma_f32 instead of four conversions + one -- same chains, same bits
 // XF2 (XF of a row too long for that: the 25600-wide down_proj of Qwen3-32B, one row slot per wave): the fp32 chunks of HALF the block columns at a time -- the iterations

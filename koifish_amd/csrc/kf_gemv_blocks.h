@@ -339,7 +339,7 @@ struct BlockDot<FMT_Q2T, CANON> {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x2_t perm_fma_dword(uint32_t D, f32x4 X0, f32x4 X1, const PermLut& t, f32x2_t acc) {
     // the even-indexed elements (low nibbles of D >> 4, element 0 in byte 3) and the odd-indexed ones (low nibbles of D) are looked up as they lie: a pair's two fp32
-    // operands come from the two lookups at the same byte position, so the index bytes need no gather (round 3 gathered elements 0..3 / 4..7 first: 2 perms more per dword)
+    // operands come from the two lookups at the same byte position, so the index bytes need no gather (gathering elements 0..3 / 4..7 first is 2 perms more per dword)
     uint32_t le, he, lo, ho;
     perm_lookup4(D >> 4, t, le, he);
     perm_lookup4(D, t, lo, ho);

@@ -226,7 +226,7 @@ int gelu_backward_launch(hipStream_t st, uint16_t* d_in_out, const uint16_t* x, 
 }
 // SwiGLU backward (CU_swiglu_back_v0, Activation.cu:245-260): sig = 1 / (1 + exp(-gate));
 // delta_gate = bf16(delta * up * sig * (1 + gate * (1 - sig))); delta_in_out = bf16(delta * gate * sig)   (the gradient of the up projection).
-// The reference rounds both stores stochastically (seed 42); round-to-nearest here, as everywhere (SURVEY fact 5).
+// The reference rounds both stores stochastically (seed 42); round-to-nearest here, as everywhere.
 __device__ __forceinline__ void swiglu_grad(float xiW, float xiV, float delta, float& d_gate, float& d_up) {
     const float sigW = 1.0f / (1.0f + kf_expf(-xiW));
     d_gate = delta * xiV * sigW * (1.0f + xiW * (1.0f - sigW));
@@ -1008,7 +1008,7 @@ int adamw_launch(hipStream_t st, uint16_t* params, uint16_t* grads, void* gm, vo
 }
 
 // Tensor-parallel combine: out = bf16(residual + bf16(sum_r partial[r])) with the partial sums added in rank order 0..R-1
-// (fixed order: every rank computes the same bits; SURVEY.md section 8e).  residual may be NULL.
+// (fixed order: every rank computes the same bits).  residual may be NULL.
 __global__ void tp_reduce_kernel(const float* __restrict__ partials, int R, int n, const uint16_t* __restrict__ residual, uint16_t* __restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;

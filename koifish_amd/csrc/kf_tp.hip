@@ -1,4 +1,4 @@
-// kf_tp.hip -- the exchange step of tensor-parallel decode (Qwen3-32B over 8 MI355X, SURVEY.md section 8e): one-shot writes into every peer's
+// kf_tp.hip -- the exchange step of tensor-parallel decode (Qwen3-32B over 8 MI355X): one-shot writes into every peer's
 // receive area over xGMI peer-to-peer mappings, then a local rank-ordered sum.  No collective library call, no host involvement: the whole TP
 // step is a chain of kernels that a hipGraph replays.
 //

@@ -15,7 +15,7 @@ namespace kf {
 int xengine_go_lowbit(XEngineHost* E, hipStream_t st);
 size_t xe_smem_lowbit(int fmt, int shape_class, int n_seq, int n_layer);
 static int xe_shape_class(int GQ, int hd, int dim, int q_dim, int ffn) {
-    if (GQ == 2 && hd == 128 && dim == 1024 && q_dim == 2048 && ffn == 3072) return 1; /* Qwen3-0.6B (BASELINE config 2) */
+    if (GQ == 2 && hd == 128 && dim == 1024 && q_dim == 2048 && ffn == 3072) return 1; /* Qwen3-0.6B */
     if (GQ == 2 && hd == 64 && dim == 256 && q_dim == 256 && ffn == 512) return 2;     /* the small parity-test shape */
     if (GQ == 2 && hd == 128 && dim == 2048 && q_dim == 2048 && ffn == 6144) return 3;  /* Qwen3-1.7B: the streaming phases do not care how many blocks a lane walks */
     if (GQ == 4 && hd == 128 && dim == 2560 && q_dim == 4096 && ffn == 9728) return 4;  /* Qwen3-4B (32 / 8 heads; cases/tutorial/history.md:4-6) */
@@ -106,7 +106,7 @@ void xengine_free(XEngineHost* E) {
     delete E;
 }
 // one model's (one TP rank's) layer table out of its descriptor; qbias: the seven matrices' zero points of layer 0 (every layer, every rank: the same)
-// *fmt_io: the storage every matrix of the model carries (0 on entry = not known yet): FMT_Q4P (4-bit PackedQ) or FMT_Q1T (1-bit, round 6)
+// *fmt_io: the storage every matrix of the model carries (0 on entry = not known yet): FMT_Q4P (4-bit PackedQ) or FMT_Q1T (1-bit)
 static int xe_fill_layers(const kf_engine_desc* d, EngLayer* tab, float* qbias, bool qbias_set, bool& q4p_ok, int* fmt_io = nullptr, bool allow_hot = false) {
     const int hd = d->head_dim, q_dim = d->n_head * hd, kv_dim = d->n_kv * hd;
     const int Ks[7] = {d->dim, d->dim, d->dim, q_dim, d->dim, d->dim, d->ffn}, Ms[7] = {q_dim, kv_dim, kv_dim, d->dim, d->ffn, d->ffn, d->dim};
@@ -226,7 +226,7 @@ int xengine_build(const kf_engine_desc* d, int n_seq, long long kv_seq_stride, v
 using XC7 = XCfg<FMT_Q4P, 8, 128, 12, 5120, 1024, 128, 3200, 6, false, 1, 1, true>;
 using XC7D = XCfg<FMT_Q4P, 8, 128, 12, 5120, 1024, 128, 3200, 6, true, 1, 1, true>; /* + the per-phase stamps of one workgroup of one rank */
 static size_t xe_smem_class3_two(int n_layer) { return xe_smem<XC3<8, 4, false, 2, 1>>(n_layer); }
-// a rank of Qwen3-8B under TP = 8 (round 6: ONE sequence of a GQA-4 model on the eight XCDs): 4 query heads on 1 kv-head, q_dim 512, ffn 1536 (12 groups of 128)
+// a rank of Qwen3-8B under TP = 8 (ONE sequence of a GQA-4 model on the eight XCDs): 4 query heads on 1 kv-head, q_dim 512, ffn 1536 (12 groups of 128)
 using XC8 = XCfg<FMT_Q4P, 4, 128, 12, 4096, 512, 128, 1536, 6, false, 1, 1, true>;
 // a rank of Qwen3-4B under TP = 8: ffn 9728 = 76 groups of 128 does not split into eight whole-group column shards -- the model is run with its FFN padded to 80 groups (512
 // zero rows of gate / up, 512 zero columns of down_proj: exact zeros in every sum), 1280 per rank
@@ -346,8 +346,8 @@ int xengine_set_head_tp(XEngineHost* E, const kf_weight* const* ws, const int* r
 #define XE_VARIANTS 1 /* the tuning instantiations (waves per workgroup x ring depth) beside the defaults.  Measured and dropped (ms per step of eight sequences at 2 k keys, default
                          12 x 6: 1.89): 13 x 6 2.22, 16 x 4 2.17 (128 registers: spills), four key tiles per attention batch 2.29 - 2.37 (spills) */
 #endif
-// n_seq <= 8: one decoder per XCD (12 waves, 168 registers), one sequence each.  More: the BATCHED form (round 6) -- still one decoder per XCD, every unpacked block multiplied
-// against the activations of 2 (n_seq <= 16) or 4 (n_seq <= 32) sequences.  The round-5 form of 9 .. 16 sequences (two decoders per XCD, two workgroups of 8 waves per CU,
+// n_seq <= 8: one decoder per XCD (12 waves, 168 registers), one sequence each.  More: the BATCHED form -- still one decoder per XCD, every unpacked block multiplied
+// against the activations of 2 (n_seq <= 16) or 4 (n_seq <= 32) sequences.  The other form of 9 .. 16 sequences (two decoders per XCD, two workgroups of 8 waves per CU,
 // 128 registers) stays behind XEngineHost::two_wpc as the A/B reference.
 template <template <int, int, bool, int, int, int, int> class XC, int NWV, int DEPTH, bool DBG, int WPC, int AU, int NB, int NP = 0>
 using XF = XC<NWV, DEPTH, DBG, WPC, AU, NB, NP>; /* (a template template parameter carries no default arguments) */
@@ -398,7 +398,7 @@ static int xengine_go_shape(XEngineHost* E, hipStream_t st) {
     if (!two && E->variant_set && E->nwv == 9) return xengine_go<XF<XC, 9, 8, false, 1, 2, 1>>(E, st);
     return two ? xengine_go<XF<XC, 8, 4, false, 2, 1, 1>>(E, st) : xengine_go<XF<XC, 12, 2, false, 1, 2, 1>>(E, st); /* (8 sequences: depth 6 4370, 4 4570, 2 4630 tokens/s) */
 }
-// the LDS the chosen form needs (classes 1 and 2), so that create / served can refuse a model too deep for it (ADVICE r05) instead of the first step
+// the LDS the chosen form needs (classes 1 and 2), so that create / served can refuse a model too deep for it instead of the first step
 template <template <int, int, bool, int, int, int, int> class XC>
 static size_t xe_shape_smem(int n_seq, int n_layer, bool two_wpc) {
     if (n_seq <= XE_NXCD) return xe_smem<XF<XC, 12, 2, false, 1, 2, 1>>(n_layer);
@@ -437,7 +437,7 @@ int xengine_steps(XEngineHost* E, hipStream_t st, int32_t* d_state, uint16_t* x_
         else
 #endif
         // two sequences per decoder: 6 compute waves + 2 pollers at 256 registers (measured at 2 k keys, 16 sequences: 2180 tokens/s; 12 waves at 168 registers spill in the
-        // streaming loops: 1650 - 1690; round 5's two decoders per XCD 1600; eight sequences, one per decoder: 1940)
+        // streaming loops: 1650 - 1690; two decoders per XCD 1600; eight sequences, one per decoder: 1940)
         if (a.n_seq > XE_NXCD && !E->two_wpc && xe_smem<XC3<8, 8, false, 1, 2, 2>>(a.n_layer) <= 160 * 1024) rc = xengine_go<XC3<8, 8, false, 1, 2, 2>>(E, st); /* (ring depth 4 / 6 / 8: 2180 / 2230 / 2240) */
         else rc = a.n_seq > XE_NXCD ? xengine_go<XC3<8, 4, false, 2, 1>>(E, st) : xengine_go<XC3<12, 6, false, 1>>(E, st);
     }
@@ -521,7 +521,7 @@ void xengine_set_variant(XEngineHost* E, int nwv, int depth) {
         E->deal_wl = depth;
         return;
     }
-    if (nwv == -2) { /* A/B hook: depth != 0 = 9 .. 16 sequences through the round-5 form (two decoders per XCD) instead of the batched one */
+    if (nwv == -2) { /* A/B hook: depth != 0 = 9 .. 16 sequences through the other form (two decoders per XCD) instead of the batched one */
         E->two_wpc = depth != 0;
         return;
     }

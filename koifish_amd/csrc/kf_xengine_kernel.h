@@ -1,9 +1,9 @@
-// kf_xengine_kernel.h (the device code of kf_xengine.hip; round 6: a header, so that the storages' instantiations compile as separate translation units) -- EIGHT independent decoders per GPU, one per XCD: the decode step of kf_engine.hip re-shaped so that the CHIP streams bytes while each SEQUENCE
-// waits on its hand-offs (round 5).
+// kf_xengine_kernel.h (the device code of kf_xengine.hip, a header so that the storages' instantiations compile as separate translation units) -- EIGHT independent decoders per GPU, one per XCD: the decode step of kf_engine.hip re-shaped so that the CHIP streams bytes while each SEQUENCE
+// waits on its hand-offs.
 //
 // kf_engine.hip gives one sequence all 256 CUs: a layer's 8.4 MB of weights sit in registers before the activations arrive, and the step is bound by its six all-to-all
-// hand-offs per layer across 8 XCDs (0.22 of the HBM roofline, measured to be the floor of that design: DESIGN.md section 8.1).  The reference decodes one sequence per
-// process (GoPT.cpp:1139-1180) and SURVEY section 8e scales the 0.6B model as independent replicas; this file puts the replicas INSIDE the package:
+// hand-offs per layer across 8 XCDs (0.22 of the HBM roofline, measured to be the floor of that design).  The reference decodes one sequence per
+// process (GoPT.cpp:1139-1180) and a larger load is served by independent replicas; this file puts them INSIDE the package:
 //
 //   * 256 workgroups, one per CU.  A workgroup reads its XCD from HW_REG_XCC_ID and takes a ticket there: the 32 workgroups of XCD s are the decoder of sequence s
 //     (placement-independent: nothing assumes which CU a block lands on, only that all 256 are resident).  The sequences share the weights and nothing else: own
@@ -61,7 +61,7 @@ struct XArgs {
     int vocab, pick; /* pick: the greedy pick and the state update run inside (needed for n_steps > 1) */
     char* loc;       /* XCD-local exchange areas, loc_stride bytes each */
     size_t loc_stride;
-    int* ws;         /* [0] (unused since round 6: the epoch is XArgs::epoch0), [1] error word, [16 + 32 x] ticket of XCD x, [17 + 32 x] its workgroups that have left */
+    int* ws;         /* [0] (unused: the epoch is XArgs::epoch0), [1] error word, [16 + 32 x] ticket of XCD x, [17 + 32 x] its workgroups that have left */
     unsigned long long* dbg; /* diagnostic instantiation: [step][layer][16] stamps of (sequence dbg_seq, workgroup rank dbg_wg) */
     int dbg_seq, dbg_wg, dbg_steps;
     int deal_wl;    /* weight (x 8) of the compute waves that share the poller's SIMD: see xe_deal */
@@ -87,7 +87,7 @@ constexpr int xe_p1_wgs(int dim, int epb, int qd, int kvd) { /* the most workgro
 }
 template <int FMT_, int GQ_, int HD_, int NWV_, int DIM_, int QD_, int KVD_, int FFN_, int DEPTH_, bool DBG_, int WPC_ = 1, int AU_ = 2, bool TP_ = false, int NB_ = 1, int NP_ = 0>
 struct XCfg {
-    // NB: sequences per decoder (round 6).  The decoders of a launch unpack the SAME 4-bit blocks; with NB > 1 a decoder multiplies every unpacked block against the
+    // NB: sequences per decoder.  The decoders of a launch unpack the SAME 4-bit blocks; with NB > 1 a decoder multiplies every unpacked block against the
     // activations of NB sequences (xcc + 8 b, b = 0 .. NB - 1) staged side by side in LDS -- the exact bf16-stepwise unpack (7 vector instructions per weight with its
     // bookkeeping) is paid once, each sequence adds its half-instruction per weight (v_pk_fma_f32) and keeps its own canonical chain, lane tree and rounding: every id, logit
     // and K / V row of every sequence stays bit for bit what the sequence alone produces.  Hand-offs carry NB vectors (one wait, NB sweeps), the attention, the K / V caches
@@ -119,7 +119,7 @@ struct XCfg {
     static constexpr int FMT = FMT_, GQ = GQ_, HD = HD_, NWV = NWV_, NCW = NWV_ - NP, DIM = DIM_, QD = QD_, KVD = KVD_, FFN = FFN_, DEPTH = DEPTH_, NWG = XE_NWG;
     static constexpr bool DBG = DBG_;
     static_assert(FMT_ == FMT_Q4 || FMT_ == FMT_Q4P || FMT_ == FMT_Q1T || FMT_ == FMT_Q2T,
-                  "4-bit PackedQ layers (arithmetic or register-table unpack), or -- round 6 -- 1-bit / 2-bit: one dword of a 128-element block, resp. one 8-byte half of a 64-element block per lane");
+                  "4-bit PackedQ layers (arithmetic or register-table unpack), or 1-bit / 2-bit: one dword of a 128-element block, resp. one 8-byte half of a 64-element block per lane");
     static constexpr int VBYTES = FMT_ == FMT_Q1T ? 4 : (FMT_ == FMT_Q2T ? 8 : 16); /* bytes of a lane's 32-weight piece of the packed stream */
     static constexpr bool PREP = FMT_ == FMT_Q1T || FMT_ == FMT_Q2T;                  /* unpacked through BlockPrep<FMT> and the LDS selector table */
     static constexpr int n_head = QD_ / HD_, n_kv = KVD_ / HD_;
@@ -1487,7 +1487,7 @@ __global__ void __launch_bounds__(C::NWV * 64, (C::NWV * C::WPC + 3) / 4 /* wave
     }
     // ---- the decoder's sequences: which exist, are not parked ({token, pos, parked, status}: d_state[s][2] != 0) and stand inside their cache rows for every step of this launch.
     // A sequence that does not is INACTIVE for the launch -- it touches nothing outside its own exchange area and says why in its own status word (d_state[s][3]: 64 = a
-    // position of the launch lies beyond the cache; ADVICE r05: one finished sequence must not stop the others) -- and a decoder without an active sequence leaves.
+    // position of the launch lies beyond the cache: one finished sequence must not stop the others) -- and a decoder without an active sequence leaves.
     const int nst = a.n_steps > 1 ? a.n_steps : 1;
     int pos0[NB];
     bool any_act = false;
@@ -1600,7 +1600,7 @@ struct XEngineHost {
     int epoch;       /* the generation the next launch starts at (XArgs::epoch0) */
     int batch;       /* sequences per decoder of the form in use (XCfg::NB): 1, 2 or 4 */
     int variant_set; /* xengine_set_variant was called with a waves x depth pair (tuning runs) */
-    int two_wpc;     /* n_seq 9 .. 16 through the round-5 form (two decoders per XCD, two workgroups per CU) instead of the batched one: A/B hook */
+    int two_wpc;     /* n_seq 9 .. 16 through the other form (two decoders per XCD, two workgroups per CU) instead of the batched one: A/B hook */
 };
 
 template <class C>
@@ -1609,7 +1609,7 @@ static size_t xe_smem(int n_layer) {
 }
 template <class C>
 static int xengine_go(XEngineHost* E, hipStream_t st) {
-    static unsigned long long ready = 0; /* bit d: the attribute is set on device d (it is per device: ADVICE r05) */
+    static unsigned long long ready = 0; /* bit d: the attribute is set on device d (it is per device) */
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return KF_HIP_CHECK;
     if (dev < 0 || dev >= 64 || !((ready >> dev) & 1ull)) {

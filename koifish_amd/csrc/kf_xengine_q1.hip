@@ -1,4 +1,4 @@
-// kf_xengine_q1.hip -- the XCD-confined decode engines on 1-bit and 2-bit PackedQ layers (round 6; 1-bit: BASELINE config 5's storage): the kernel of kf_xengine_kernel.h
+// kf_xengine_q1.hip -- the XCD-confined decode engines on 1-bit and 2-bit PackedQ layers: the kernel of kf_xengine_kernel.h
 // instantiated for FMT_Q1T / FMT_Q2T -- a lane takes ONE DWORD of a 128-element 1-bit block, resp. one 8-byte half of a 64-element 2-bit block (32 weights either way: the
 // lanes, slots and canonical chains of a 4-bit matrix, kf_engine.hip's dealing), BlockPrep<FMT> turns it into 16 bf16 pair words through the 256-entry LDS selector table, and
 // every sequence of the decoder takes its chain pair over them.  A translation unit of its own, so that the storages' instantiations compile side by side.

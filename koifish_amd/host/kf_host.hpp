@@ -208,7 +208,7 @@ struct CHAT_SAMPLER {
     bool greedy() const { return temperature == 0.0f || top_k == 1; }
 };
 
-// Tensor-parallel decode (no counterpart in the single-GPU reference, QKV.cu:503; SURVEY.md section 8e): this Fish holds ONE rank's shard -- the
+// Tensor-parallel decode (no counterpart in the single-GPU reference, QKV.cu:503): this Fish holds ONE rank's shard -- the
 // card carries the LOCAL head / ffn / vocab counts and the full nEmbed -- and exchanges fp32 partials through peer-mapped receive areas
 // (kf_tp_* of the ABI).  q/k/v/gate/up are row shards, o_proj / down_proj column shards, the head a vocabulary shard, the embedding replicated.
 struct TPState {
@@ -244,7 +244,7 @@ struct Fish {
     int scratch_rows = 0;  // token rows that PrefillScratch has sized it for (0: again at the next prefill)
     void* deq_arena = nullptr;  // kf_set_dequant_arena: resident bf16 copies of the layers' quantised matrices for long prompts (EnsureResident)
     size_t deq_arena_bytes = 0, resident_max_bytes = (size_t)16 << 30;
-    // OFF by default (ADVICE r04): the copies are keyed by the blobs' addresses, so a caller that hands weights over as device pointers (kfh_set_weight is_device = 1) and later
+    // OFF by default: the copies are keyed by the blobs' addresses, so a caller that hands weights over as device pointers (kfh_set_weight is_device = 1) and later
     // re-quantises or updates them IN PLACE would prefill on stale bf16 copies while the decode reads the live data.  kfh_set_prefill_resident opts in and takes that promise
     // ("the quantised data does not change under me"); kfh_weights_changed drops the copies (and the engine's table) after an in-place update.
     int prefill_resident = 0;
@@ -318,7 +318,7 @@ struct Fish {
     int prefill_mode = 0;  // Generate: 0 token-serial prefill like the reference, 1 batched
 };
 
-// Eight independent decoders on ONE GPU, one per XCD, sharing a Fish's weights (kf_xengine_* of the ABI; round 5).  The reference decodes one sequence per process
+// Eight independent decoders on ONE GPU, one per XCD, sharing a Fish's weights (kf_xengine_* of the ABI).  The reference decodes one sequence per process
 // (Fish::Chat, GoPT.cpp:1139-1180) and scales a small model by running more processes; here the "processes" are the 32-workgroup halves of one launch: sequence s has its own
 // KVCache (Cache.cpp:14-57, one per sequence), decode state, forced ids, ids out and logits -- everything the reference's per-process Fish owns except the weights.
 // Every sequence's ids / logits / K / V rows are those Fish::RunSteps produces for it alone (canonical order), bit for bit.

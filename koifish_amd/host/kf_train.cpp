@@ -1,6 +1,6 @@
-// kf_train.cpp -- ONE whole training step of the hybrid-precision GPT-2 of BASELINE config 3, sequenced in C++ behind the C ABI (part of libkf_host.so).
+// kf_train.cpp -- ONE whole training step of the hybrid-precision GPT-2 (1558M shapes, f8e5m2 and 4-bit layers), sequenced in C++ behind the C ABI (part of libkf_host.so).
 //
-// The reference's step ("training"):  Fish::Train -> Optimizer loop -> Fish::ForwardOnRLS (gLLM.cpp:722-787: the neurons in graph order) ->
+// The reference's step:  Fish::Train -> Optimizer loop -> Fish::ForwardOnRLS (gLLM.cpp:722-787: the neurons in graph order) ->
 // BackwardOnRLS (gLLM.cpp:656-686: the reverse walk, SLP::Back NeuronFuse.cu:495-563) -> Optimizer::UpdateTensorParam -> CU_adamw_ (Optimizer.cu:135-160) ->
 // the re-quantisation of every updated matrix (CU_XtoQ128_ / Float2T<f8e5>, T.cu:105-175).  Here the same order as three straight loops over a TABLE of device
 // pointers: the caller (Python owns the buffers: koifish_amd/train_step.py; a C++ host would kf_malloc them) registers every trained tensor {master, gradient, two

@@ -602,7 +602,7 @@ class Qwen3:
         return self.host.kfh_num_graphs(self.h)
 
     def step_bytes(self, pos):
-        """Algorithmic HBM bytes of one decode step at position `pos` (SURVEY.md section 8d): every weight's packed data +
+        """Algorithmic HBM bytes of one decode step at position `pos`: every weight's packed data +
         zero/step once, the norm vectors, and the KV rows 0..pos read once plus the new row written."""
         c = self.cfg
         kvd = c["n_kv"] * c["head_dim"]

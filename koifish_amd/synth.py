@@ -1,5 +1,5 @@
-"""Synthetic Qwen3-shaped models (there is no network for checkpoints): shapes of SURVEY.md section 8 and the
-weight recipe of section 8d -- weights ~ N(0, 0.02) rounded to bf16, norm weights 1 + N(0, 0.01).
+"""Synthetic Qwen3-shaped models (there is no network for checkpoints): the shapes below and the
+weight recipe of the benchmarks -- weights ~ N(0, 0.02) rounded to bf16, norm weights 1 + N(0, 0.01).
 
 numpy (PCG64) generation is used where a CPU checker must see the very same weights (tests, smoke); the
 full-size benchmark model is drawn on the GPU with torch's generator.  Quantisation is always done by the

@@ -1,7 +1,7 @@
 """Tensor-parallel decode for models that do not fit (or should not sit on) one GPU: Qwen3-32B, TP = 8 over xGMI.
 
 The reference is single-GPU (`cudaSetDevice(0)`, src/Device/CUDA/QKV.cu:503); this is the one place where the path shards
-naturally (SURVEY.md section 8e): Megatron-style
+naturally: Megatron-style
     q / k / v / gate / up : split by OUTPUT rows  (whole heads; ffn rows)      -> no exchange
     o_proj / down_proj    : split by INPUT columns (multiples of the 128 group) -> fp32 partial row dots per rank,
                             all-gather, summed in rank order 0..R-1, one bf16 store, + residual (kf_tp_reduce)

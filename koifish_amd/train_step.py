@@ -1,4 +1,4 @@
-"""One WHOLE training step of the hybrid-precision GPT-2 of BASELINE config 3, every operator through the C ABI -- the host-side order of the reference's step:
+"""One WHOLE training step of the hybrid-precision GPT-2 (1558M shapes, f8e5m2 and 4-bit layers), every operator through the C ABI -- the host-side order of the reference's step:
 
   forward  (TokenEmbed, 48 x [LayerNorm, SLP qkv, causal attention, SLP proj + residual, LayerNorm, SLP fc, GELU, SLP proj2 + residual], LayerNorm, tied head)
            on the QUANTISED blobs (attention matrices f8e5m2, MLP matrices 4-bit PackedQ): SLP::Forw, NeuronFuse.cu:305-381
