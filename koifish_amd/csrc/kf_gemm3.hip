@@ -24,93 +24,71 @@
 
 namespace kf {
 
-// epilogue (gemm_epilogue's order): lane holds rows m .. m+3 of a 16 x 16 tile for token column r16
 // ROPE::cuInfer on a 128-row tile that is one head (hd 128) of Q or K, in the epilogue of the stacked Q | K | V launch (the arithmetic of prep_head_cs, kf_attn_common.h: the
 // projection rounded to bf16 as the plain epilogue stores it, fp64 sum of squares, s rounded to bf16, (x s) w rounded, rotate-half pairs (j, j + 64) with every product and the
-// sum rounded once).  Wave (wm, wn) holds rows 64 wm .. + 63 x tokens 64 wn .. + 63: a token's 128 squares are summed over the 4 lanes of a column (row swaps) and the two wm
-// waves (LDS), and a rotation pair's other element sits in the other wm wave at the SAME lane and register: one exchange through the (now free) stage buffers.
+// sum rounded once).  A wave holds rows 32 wm .. + 31 and 64 + 32 wm .. + 31 (row_block): both elements of a pair, so a (cos, sin) is read once for the two and nothing is exchanged but the sums of
+// squares: over the 4 lanes of a column (row swaps) and the two wm waves (LDS).
 template <class C>
 __device__ __forceinline__ void g3_epilogue_qkrope(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int wid, int lane, unsigned char* smem_raw, uint16_t* ybase, long long ldy,
                                                    int mshift, const uint16_t* nw) {
-    static_assert(C::BM == 128 && C::MT == 4 && C::WN == 2, "one head per tile: 2 x 2 waves of 64 rows x 64 tokens");
-    const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
-    float x[C::MT][C::NT][4];
-    double ss[C::NT];
-#pragma unroll
-    for (int nt = 0; nt < C::NT; nt++) {
-        ss[nt] = 0.0;
-#pragma unroll
-        for (int mt = 0; mt < C::MT; mt++) {
-            const float vv[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                x[mt][nt][j] = round_bf16(vv[j]); /* the value the plain epilogue stores (alpha 1, no bias) */
-                ss[nt] = fma((double)x[mt][nt][j], (double)x[mt][nt][j], ss[nt]);
-            }
-        }
-        ss[nt] = xsum32_d(xsum16_d(ss[nt])); /* the column's 4 lanes (l ^ 16, l ^ 32): this wave's 64 rows */
-    }
-    double* red = reinterpret_cast<double*>(smem_raw);                                  /* [2 wm][128 tokens] */
-    uint32_t* xch = reinterpret_cast<uint32_t*>(smem_raw + 2 * 128 * sizeof(double));   /* [4 waves][32 bf16 pairs][64 lanes] */
-    if (q4 == 0) {
-#pragma unroll
-        for (int nt = 0; nt < C::NT; nt++) red[wm * 128 + wn * 64 + nt * 16 + r16] = ss[nt];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int nt = 0; nt < C::NT; nt++) {
-        const int tl = wn * 64 + nt * 16 + r16;
-        float s = 1.0f;
-        if (nw) s = round_bf16(1.0f / sqrtf((float)(red[tl] + red[128 + tl]) / 128.0f + a.qk_eps));
-#pragma unroll
-        for (int mt = 0; mt < C::MT; mt++) {
-            if (nw) {
-                const u32x2 w4 = *reinterpret_cast<const u32x2*>(nw + wm * 64 + mt * 16 + 4 * q4); /* this lane's four norm weights */
-                x[mt][nt][0] = round_bf16(x[mt][nt][0] * s * bf_lo(w4.x)), x[mt][nt][1] = round_bf16(x[mt][nt][1] * s * bf_hi(w4.x));
-                x[mt][nt][2] = round_bf16(x[mt][nt][2] * s * bf_lo(w4.y)), x[mt][nt][3] = round_bf16(x[mt][nt][3] * s * bf_hi(w4.y));
-            }
-            xch[((size_t)wid * 32 + (mt * C::NT + nt) * 2) * 64 + lane] = pack_bf16x2(x[mt][nt][0], x[mt][nt][1]);
-            xch[((size_t)wid * 32 + (mt * C::NT + nt) * 2 + 1) * 64 + lane] = pack_bf16x2(x[mt][nt][2], x[mt][nt][3]);
-        }
-    }
-    __syncthreads();
-    const int pw = (1 - wm) * C::WN + wn; /* the wave that holds the other element of every pair */
-#pragma unroll
-    for (int mt = 0; mt < C::MT; mt++)
+    static_assert(C::BM == 128 && C::MT == 4, "one head per tile");
+    const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4, tok0 = wn * 16 * C::NT + r16;
+    double* red = reinterpret_cast<double*>(smem_raw); /* [2 wm][BN tokens] */
+    if (nw) {
 #pragma unroll
         for (int nt = 0; nt < C::NT; nt++) {
-            const int tok = t0 + wn * 64 + nt * 16 + r16, jj = mt * 16 + 4 * q4; /* pair index 0 .. 63 of this lane's first row */
-            if (tok >= a.n) continue;
-            uint16_t o[4];
-            const uint32_t op0 = xch[((size_t)pw * 32 + (mt * C::NT + nt) * 2) * 64 + lane], op1 = xch[((size_t)pw * 32 + (mt * C::NT + nt) * 2 + 1) * 64 + lane];
-            const float oth[4] = {bf_lo(op0), bf_hi(op0), bf_lo(op1), bf_hi(op1)};
-            f32x4 cs01 = f32x4{1.f, 0.f, 1.f, 0.f}, cs23 = cs01; /* (cos, sin) of the lane's four pairs jj .. jj + 3: 32 contiguous bytes of the table */
-            if (a.rope_table) {
-                const f32x4* tp = reinterpret_cast<const f32x4*>(a.rope_table + (size_t)(a.rope_pos0 + (a.rope_seq > 0 ? tok % a.rope_seq : tok)) * 128 + 2 * jj);
-                cs01 = tp[0], cs23 = tp[1];
-            }
-            const float csv[8] = {cs01.x, cs01.y, cs01.z, cs01.w, cs23.x, cs23.y, cs23.z, cs23.w};
+            double ss = 0.0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float other = oth[j], own = x[mt][nt][j];
-                float v = own;
-                if (a.rope_table) {
-                    const float2 cs = float2{csv[2 * j], csv[2 * j + 1]};
-                    if (wm == 0) { /* x_j c - x_{j+64} s */
-                        const float p0 = own * cs.x, p1 = other * cs.y;
-                        v = p0 - p1;
-                    } else { /* x_j s + x_{j+64} c */
-                        const float p0 = other * cs.y, p1 = own * cs.x;
-                        v = p0 + p1;
-                    }
+            for (int mt = 0; mt < C::MT; mt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const double v = (double)round_bf16(acc[mt][nt][j]); /* the value the plain epilogue stores (alpha 1, no bias) */
+                    ss = fma(v, v, ss);
                 }
-                o[j] = f2bf(v);
-            }
-            uint16_t* yp = ybase + (size_t)tok * ldy + (m0 - mshift) + wm * 64 + jj;
-            *reinterpret_cast<u32x2*>(yp) = u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+            ss = xsum32_d(xsum16_d(ss)); /* the column's 4 lanes (l ^ 16, l ^ 32): this wave's 64 rows */
+            if (q4 == 0) red[wm * C::BN + tok0 + nt * 16] = ss;
         }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int nt = 0; nt < C::NT; nt++) {
+        const int tl = tok0 + nt * 16, tok = t0 + tl;
+        if (tok >= a.n) continue;
+        float s = 1.0f;
+        if (nw) s = round_bf16(1.0f / sqrtf((float)(red[tl] + red[C::BN + tl]) / 128.0f + a.qk_eps));
+        const f32x4* const table = reinterpret_cast<const f32x4*>(a.rope_table + (size_t)(a.rope_pos0 + (a.rope_seq > 0 ? tok % a.rope_seq : tok)) * 128);
+        uint16_t* const yt = ybase + (size_t)tok * ldy + (m0 - mshift);
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+            const int jj = C::row_block(wm, mt) * 16 + 4 * q4; /* pair index 0 .. 63 of this lane's first row */
+            float x[2][4]; /* rows jj .. jj + 3 and 64 + jj .. */
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                u32x2 w4 = u32x2{0, 0};
+                if (nw) w4 = *reinterpret_cast<const u32x2*>(nw + 64 * e + jj);
+                const float w[4] = {bf_lo(w4.x), bf_hi(w4.x), bf_lo(w4.y), bf_hi(w4.y)};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    x[e][j] = round_bf16(acc[2 * e + mt][nt][j]);
+                    if (nw) x[e][j] = round_bf16(x[e][j] * s * w[j]);
+                }
+            }
+            if (a.rope_table) {
+                const f32x4 cs01 = table[jj / 2], cs23 = table[jj / 2 + 1]; /* (cos, sin) of the lane's four pairs: 32 contiguous bytes of the table */
+                const float csv[8] = {cs01.x, cs01.y, cs01.z, cs01.w, cs23.x, cs23.y, cs23.z, cs23.w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float c = csv[2 * j], sn = csv[2 * j + 1], lo = x[0][j], hi = x[1][j], p0 = lo * c, p1 = hi * sn, p2 = lo * sn, p3 = hi * c;
+                    x[0][j] = p0 - p1, x[1][j] = p2 + p3;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++) *reinterpret_cast<u32x2*>(yt + 64 * e + jj) = u32x2{pack_bf16x2(x[e][0], x[e][1]), pack_bf16x2(x[e][2], x[e][3])};
+        }
+    }
 }
 
+// epilogue (gemm_epilogue's order): lane holds rows m .. m + 3 of a 16 x 16 tile for token column r16
 template <bool AKM, class C>
 __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int wid, int lane, unsigned char* smem_raw = nullptr) {
     const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
@@ -121,7 +99,7 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
         for (int mt = 0; mt < C::MT; mt += 2)
 #pragma unroll
             for (int nt = 0; nt < C::NT; nt++) {
-                const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, f = ((m0 + wm * (16 * C::MT)) >> 1) + (mt >> 1) * 16 + 4 * q4;
+                const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, f = (m0 >> 1) + C::row_block(wm, mt) * 8 + 4 * q4;
                 if (tok >= a.n || f >= F) continue;
                 const float gv[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w}, uv[4] = {acc[mt + 1][nt].x, acc[mt + 1][nt].y, acc[mt + 1][nt].z, acc[mt + 1][nt].w};
                 uint16_t o[4];
@@ -169,7 +147,7 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
     if (wide) {
 #pragma unroll
         for (int mt = 0; mt < C::MT; mt++) {
-            const int m = m0 + wm * (16 * C::MT) + mt * 16 + 4 * q4;
+            const int m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
             if (m >= Mlim) continue;
             u32x2 b4 = u32x2{0, 0};
             if (a.bias) b4 = *reinterpret_cast<const u32x2*>(a.bias + m);
@@ -200,7 +178,7 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
     for (int mt = 0; mt < C::MT; mt++)
 #pragma unroll
         for (int nt = 0; nt < C::NT; nt++) {
-            const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, m = m0 + wm * (16 * C::MT) + mt * 16 + 4 * q4;
+            const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
             if (tok >= a.n || m >= Mlim) continue;
             uint16_t* yp = ybase + (size_t)tok * ldy + (m - mshift);
             const float vv[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w};
@@ -391,7 +369,7 @@ void gemm3_sk_forget(void* ws) { /* something else was (or will be) written wher
 // (barrier, counted wait, loop) double, and the loop is not waiting for memory.  Only BK = 64 is instantiated.
 template <bool AKM, bool BKM, class C>
 static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t ws_bytes, long min_plain) {
-    constexpr int BK = G3_BK, SMEM = 2 * C::STAGE;
+    constexpr int BK = G3_BK, SMEM = C::SMEM;
     static int attr_set = 0;
     if (!attr_set && SMEM > 64 * 1024) {
         if (hipFuncSetAttribute((const void*)gemm3_kernel<AKM, BKM, BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
@@ -400,10 +378,10 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
     }
     // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; a K-contiguous product of K < 3072 only where three pieces of
     // every tile find room.  us per layer of prompts on resident copies, never | from K = 3072 | three pieces: 0.6B 320 rows 134 | 116 | 106, 1024 rows 149 | 143 | 137, 2047 rows 198 | 190 | 187; 1.7B 320
-    // rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800 rows 325 -> 332 us.  (One product by itself on operands that are in the L2
-    // already shows the opposite: 1024 x 2048 at 512 rows 11.2 whole, 12.6 in four pieces.)
+    // rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800 rows 325 -> 332 us.  Of one 128 x 128 tile to a CU a piece and tails pay up to two
+    // thirds of the CUs (K 6144: 144 tiles 64.9 -> 50.5 us; K 8192: 200 tiles 68.6 -> 78.9), beyond at K >= 16384 (25600: 200 tiles 227 -> 208)
     const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
-    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || nkt >= 48)) {
+    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || (nkt >= 48 && (C::WGS_PER_CU > 1 || 3 * nwg < 2 * G || nkt >= 256)))) {
         G3SkArgs s;
         // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they would move with it,
         // and another configuration's fp32 partials could overwrite words already marked "seen" with values that pass for an epoch)
@@ -436,30 +414,46 @@ static int g3_go(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t w
     return g3_go_c<AKM, BKM, G3Big>(st, a, nwg, ws, ws_bytes, 64);
 }
 size_t gemm3_sk_ws_bytes() { return (size_t)256 * G3_BM * G3_BN * 4 + G3_SK_FLAG_BYTES; }
+static long g3_tiles_of(int M, int n, int bm, int bn) { return (long)((M + bm - 1) / bm) * ((n + bn - 1) / bn); }
+template <class C>
+static int g3_whole(hipStream_t st, const GemmArgs& a) { /* one workgroup per tile */
+    static int attr_set = 0;
+    if (!attr_set && C::SMEM > 64 * 1024) {
+        if (hipFuncSetAttribute((const void*)gemm3_kernel<false, false, G3_BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::SMEM) != hipSuccess) return KF_HIP_CHECK;
+        attr_set = 1;
+    }
+    hipLaunchKernelGGL((gemm3_kernel<false, false, G3_BK, C>), dim3((unsigned)g3_tiles_of(a.M, a.n, C::BM, C::BN)), dim3(C::NTH), C::SMEM, st, a);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+static int g3_picked(hipStream_t st, const GemmArgs& a, bool wide) {
+    switch (g3_pick(a.M, a.n, a.K, wide && g_knobs.g3_wide)) {
+        case G3_DUO: return g3_whole<G3Duo>(st, a);
+        case G3_HALF: return g3_whole<G3Half>(st, a);
+        case G3_SMALL: return g3_whole<G3Small>(st, a);
+        case G3_WIDE: return g3_whole<G3Wide>(st, a);
+        default: return g3_whole<G3Big>(st, a);
+    }
+}
 int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws_bytes) {
     if (fmt != FMT_BF16 || a.K % G3_BK != 0 || a.K < G3_BK) return 1;
     if ((a.ldx & 7) != 0 || (reinterpret_cast<uintptr_t>(a.x) & 15) != 0 || (reinterpret_cast<uintptr_t>(a.w) & 15) != 0 || (a.K & 7) != 0) return 1;
-    if (a.n >= G3_BN && a.M >= G3_BM) {
-        const long nwg = (long)((a.M + G3_BM - 1) / G3_BM) * ((a.n + G3_BN - 1) / G3_BN);
-        // (M 1024 x K 3072 at 8192 rows, 128 big tiles: 83 -> 57 us = 890 TFLOP/s on the small ones; from 400 big tiles up the big tile is 8-12 % faster)
-        if (nwg >= 160) { /* fewer big tiles than that: four times as many small ones fill the chip better */
-            if (g_knobs.g3_wide && g3_prefer_wide(a.M, a.n, a.K)) return g3_go_c<false, false, G3Wide>(st, a, (long)((a.M + 191) / 192) * ((a.n + 255) / 256), nullptr, 0, 1);
-            return g3_go<false, false>(st, a, nwg, nullptr, 0);
-        }
-    }
-    // 128 x 128 tiles, two workgroups per CU: bf16 products of 1-4 k rows whose M is 1024-3072 (M 1024 x K 2048 at 2048 rows: 36.9 -> 27.4 us, 3072 x 1024: 35.6 -> 23.9;
-    // 4096 rows: 583-656 TFLOP/s); a quantised weight of that size reaches them as a layer's or a resident copy (a dequantise pass of its own gives the gain back).
     if (a.n < 128 || a.M < 128) return 1;
-    const long nwg = (long)((a.M + 127) / 128) * ((a.n + 127) / 128);
-    if (nwg < 32 && (g_knobs.g3_tiles < 3 || (long)((a.M + 63) / 64) * ((a.n + 63) / 64) < 64)) return 1;
-    if (nwg < 256 && g_knobs.g3_tiles >= 1 && !a.swiglu && !a.qkrope) { /* fewer 128 x 128 tiles than CUs: twice or four times as many smaller ones */
-        // with the caller's workspace these go in k-pieces (g3_go_c says when): 1024 rows x K 2048-3072 at 512 tokens are 128 tiles of 64 x 64, each a 32-48 step k-loop on its own CU.  A partial
-        // is 16 or 32 KiB; the 64 KiB ones of the 128 x 128 tile cost more than they gave (37.8 us against 27 whole)
-        const long nmid = (long)((a.M + 63) / 64) * ((a.n + 127) / 128);
-        if (nmid >= g_knobs.g3_mid_min || g_knobs.g3_tiles < 3) return nmid >= 64 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 64) : 1;
-        return g3_go_c<false, false, G3Tiny>(st, a, (long)((a.M + 63) / 64) * ((a.n + 63) / 64), ws, ws_bytes, 64);
+    const int nkt = a.K / G3_BK;
+    const long n128 = g3_tiles_of(a.M, a.n, 128, 128), n64 = g3_tiles_of(a.M, a.n, 64, 64);
+    if (n128 < 32 && n64 < 64) return 1;
+    // resident copies lend the workspace at every K: k-pieces of 64 x 64 and 64 x 128 tiles (g3_go_c says when; a partial is 16 or 32 KiB -- the 64 KiB ones of a 128 x 128 tile cost what they give at these K)
+    if (ws && nkt < 96 && n128 < 256) {
+        const long nmid = g3_tiles_of(a.M, a.n, 64, 128);
+        return nmid >= 192 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 64) : g3_go_c<false, false, G3Tiny>(st, a, n64, ws, ws_bytes, 64);
     }
-    return g3_go_c<false, false, G3Small>(st, a, nwg, nullptr, 0, 128);
+    // Otherwise the smallest tile that makes ONE round of the CUs (g3_pick; in front of it 64 x 64: up to two side by side, from K = 6144 one, or k-pieces).  us with a residual, 64 x 64 | 64 x 128 (three buffers) | 128 x 128 on 8 waves |
+    // 128 x 256 | 128 x 128 on 4 waves:  M 1024 x K 2048 at 515 rows 12.5 | 17.4 | 20.7 | 31.0 | 28.3, at 2047 rows 18.0 | 18.5 | 21.4 | 32.0 | 29.2, at 2608 rows (656 tiles) 22.8 | 23.9 | 21.8 | 32.3 | 29.4;
+    // M 2048 x K 6144 at 1540 rows 99 | 87 | 66 | 100 | 90, at 2608 rows (1312 | 672 | 336 | 176) 146 | 133 | 132 | 102 | 122.  K-pieces where the workspace is lent (K >= 6144), whole | pieces, 128 x 128 on 8 waves:
+    // M 2048 x K 6144 at 515 rows 60.6 | 36.0, at 1030 64.9 | 50.5 (a piece and tails), M 5120 x K 25600 at 330 rows 220 | 135; 64 x 64 tiles of M 2048 x K 6144 at 330 rows 32.9 | 27.3.  At K = 3072 pieces lose (2608
+    // rows 32.6 | 36.8)
+    if (n64 <= (nkt < 96 ? 512 : 256)) return g3_go_c<false, false, G3Few>(st, a, n64, ws, ws_bytes, 1);
+    if (n128 <= 256) return g3_go_c<false, false, G3Duo>(st, a, n128, ws, ws_bytes, 1);
+    return g3_picked(st, a, true);
 }
 // y[n, M] = alpha * sum_k B(k, tok) A(k, m) + beta * y (+ bias) with either operand stored K-MAJOR: akm: A = w[K][lda] (element (k, m) at k * lda + m), else w[M][K];
 // bkm: B = x[K][ldb], else x[n][ldb].  The two GEMMs of SLP::Back without a transpose of anything:  delta[n, IC] = deltaIn[n, OC] . W[OC, IC]  (A = W k-major),
@@ -508,15 +502,13 @@ int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int*
     a.w = reinterpret_cast<const unsigned char*>(Wcat), a.M = tot, a.K = K, a.x = x, a.ldx = ldx, a.n = n, a.y = y[0], a.ldy = M[0], a.alpha = 1.0f, a.beta = 0.0f;
     const long nwg = (long)(tot / G3_BM) * ((n + G3_BN - 1) / G3_BN);
     if (nwg < 64 && (long)(tot / 128) * ((n + 127) / 128) < 64) return 1;
-    // fewer than 160 big tiles (Q | K | V of a 0.6B model at 2047 tokens: 128): four times as many 128 x 128 tiles fill the chip better (2047-token prompt 8.20 -> 7.84 ms;
-    // gate | up, 192 big tiles, is better left on them: 7.93 ms with both small)
-    if (rope) {
+    const long n128 = g3_tiles_of(tot, n, 128, 128);
+    if (rope) { /* a head-sized tile: one round of the wider or the deeper one where it is one */
         if (n_w != 3 || M[0] % 128 != 0 || M[1] % 128 != 0 || ((M[0] | M[1] | M[2]) & 3) || (reinterpret_cast<uintptr_t>(y[0]) & 7) || (reinterpret_cast<uintptr_t>(y[1]) & 7)) return 1;
         a.qkrope = 1, a.qk_norm[0] = rope->wq, a.qk_norm[1] = rope->wk, a.rope_table = rope->table, a.rope_pos0 = rope->pos0, a.rope_seq = rope->seq_len, a.qk_eps = rope->eps;
-        return g3_go_c<false, false, G3Small>(st, a, (long)(tot / 128) * ((n + 127) / 128), nullptr, 0, 1); /* always the head-sized tile */
     }
-    if (nwg < 160) return g3_go_c<false, false, G3Small>(st, a, (long)(tot / 128) * ((n + 127) / 128), nullptr, 0, 1);
-    return g3_go<false, false>(st, a, nwg, nullptr, 0);
+    if (rope) return n128 <= 256 ? g3_whole<G3Duo>(st, a) : g3_tiles_of(tot, n, 128, 256) <= 256 ? g3_whole<G3Half>(st, a) : g3_whole<G3Small>(st, a);
+    return g3_picked(st, a, false); /* a tile's rows are one matrix's: no 192-row ones */
 }
 
 // gate | up dequantised INTERLEAVED in blocks of 16 rows (dequant_launch ilv_n = 2) x the same x, SwiGLU in the epilogue: act[n, ffn] in one launch (the stacked route
@@ -532,12 +524,7 @@ int gemm3_swiglu_launch(hipStream_t st, const uint16_t* Wilv, int ffn, int K, co
     a.w = reinterpret_cast<const unsigned char*>(Wilv), a.M = M, a.K = K, a.x = x, a.ldx = ldx, a.n = n, a.y = act, a.ldy = ffn, a.alpha = 1.0f, a.beta = 0.0f;
     const long nwg = (long)(M / G3_BM) * ((n + G3_BN - 1) / G3_BN);
     if (nwg < 64 && (long)(M / 128) * ((n + 127) / 128) < 64) return 1;
-    const long nws = (long)(M / 128) * ((n + 127) / 128), nww = (long)(M / 192) * ((n + G3_BN - 1) / G3_BN);
-    const bool wide_ok = g_knobs.g3_wide && M % 192 == 0 && nww <= 256;
-    // fewer than 160 big tiles: four times as many 128 x 128 ones -- unless those spill into a second round of the 512 resident workgroups and the 192 x 256 ones make one round
-    if (nwg < 160 && !(wide_ok && nws > 512 && nww >= 160)) return g3_go_c<false, false, G3Small>(st, a, nws, nullptr, 0, 1);
-    if (g_knobs.g3_wide && g3_prefer_wide(M, n, K)) return g3_go_c<false, false, G3Wide>(st, a, (long)((M + 191) / 192) * ((n + G3_BN - 1) / G3_BN), nullptr, 0, 1);
-    return g3_go<false, false>(st, a, nwg, nullptr, 0);
+    return g3_picked(st, a, true);
 }
 
 }  // namespace kf

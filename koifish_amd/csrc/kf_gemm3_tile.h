@@ -8,23 +8,26 @@
 namespace kf {
 
 constexpr int G3_BM = 256, G3_BN = 256, G3_BK = 64;
-// the workgroup tile: BM rows x BN tokens, NW waves as 2 (rows) x NW / 2 (tokens).  Big = the 256 x 256 tile of the header (8 waves, 128 x 64 outputs each, 128 KiB of
-// LDS: one workgroup per CU); Small = 128 x 128 on 4 waves (64 x 64 outputs each, 64 KiB: two workgroups per CU) for products with too few 256 x 256 tiles to fill the
-// chip -- the o_proj / down projections of a 1-2 k token prompt (M = 1024: 32 big tiles), with the split-K form below on top.  K-contiguous operands only.
-template <int BM_, int BN_, int NW_>
+// the workgroup tile: BM rows x BN tokens, NW waves as 2 (rows) x NW / 2 (tokens), NBUF LDS buffers: the loads of NBUF - 1 later k-steps are in flight under the step that is multiplied.
+// A step is bound by those loads, not by its MFMAs (loads alone take 85 - 95 % of every configuration's time), and with two buffers a lone workgroup of a CU waits out their latency: us per
+// step with one workgroup on every CU, two buffers | more: 64 x 64 0.41 | 0.23 (3), 128 x 128 on 8 waves 0.89 | 0.58 (3), 128 x 256 0.82 (3) against 1.26 of 192 x 256 (2: three do not fit).
+template <int BM_, int BN_, int NW_, int NBUF_ = 2>
 struct G3Cfg {
-    static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = NW_ / 2, MT = BM_ / 32, NT = BN_ / (16 * (NW_ / 2));
+    static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = NW_ / 2, MT = BM_ / 32, NT = BN_ / (16 * (NW_ / 2)), NBUF = NBUF_;
     static constexpr int NIA = BM_ / (8 * NW_), NIB = BN_ / (8 * NW_); /* global_load_lds instructions per wave, operand and k-step (8 rows of 128 bytes each) */
-    static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, WGS_PER_CU = (160 * 1024) / (2 * STAGE);
+    /* the 16-row block of the tile that is block mt of the waves wm: in order, but for 128 rows, which may be one head -- there a wave holds both elements of its rotation pairs (rows j and j + 64) */
+    static constexpr __host__ __device__ int row_block(int wm, int mt) { return BM == 128 ? 4 * (mt >> 1) + 2 * wm + (mt & 1) : wm * MT + mt; }
+    static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, SMEM = NBUF_ * STAGE, WGS_PER_CU = (160 * 1024) / SMEM;
 };
-using G3Big = G3Cfg<256, 256, 8>;
-using G3Small = G3Cfg<128, 128, 4>;
-// products whose 128 x 128 tiles do not fill the chip either (M = 1024 at 1-2 k tokens: 64-128 of them; four k-pieces of those measured 37.8 us against 27 plain: three
-// 64 KiB partials per tile through memory) get MORE, SMALLER tiles, these in k-pieces where a workspace is lent: 64 x 128 (48 KiB of LDS: three workgroups per CU) and 64 x 64 (32 KiB: five)
+using G3Big = G3Cfg<256, 256, 8>;      /* 128 KiB of LDS: one workgroup per CU */
+using G3Wide = G3Cfg<192, 256, 8>;
+using G3Half = G3Cfg<128, 256, 8, 3>;  /* 144 KiB */
+using G3Duo = G3Cfg<128, 128, 8, 3>;   /* 96 KiB */
+using G3Small = G3Cfg<128, 128, 4>;    /* 64 KiB: two workgroups per CU; the split-K tile of the k-major products */
+using G3Few = G3Cfg<64, 64, 4, 3>;     /* 48 KiB: three */
+// k-pieces of resident copies (gemm3_launch)
 using G3Mid = G3Cfg<64, 128, 4>;
 using G3Tiny = G3Cfg<64, 64, 4>;
-// 192 x 256: a product whose 256 x 256 tiles number 160-255 (gate | up of a 0.6B model at 2047 tokens: 24 x 8 = 192 tiles on 256 CUs) becomes 32 x 8 = 256 tiles of 3/4 the work
-using G3Wide = G3Cfg<192, 256, 8>;
 
 // x, which the compiler cannot trace: addresses formed from it are formed behind this point and take no registers in front of it
 __device__ __forceinline__ int g3_opaque(int x) {
@@ -134,7 +137,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     constexpr int BYTES_A = C::BM * BK * 2, BYTES_B = C::BN * BK * 2;
     const int wid = __builtin_amdgcn_readfirstlane(wid_), wm = wid / C::WN, wn = wid % C::WN;
     auto bufA = [&](int b) { return smem_raw + b * BYTES_A; }; /* an operand's two buffers side by side: both in reach of an LDS instruction's 16-bit offset */
-    auto bufB = [&](int b) { return smem_raw + 2 * BYTES_A + b * BYTES_B; };
+    auto bufB = [&](int b) { return smem_raw + C::NBUF * BYTES_A + b * BYTES_B; };
     // AKM: W is [K][M] with row stride a.ldr (re-used field: the residual is not served by the k-major forms); BKM: x is [K][n] with row stride a.ldx.
     G3Src sa, sb;
     const uint16_t* gat[ROWS::GATHER ? C::NIB : 1];
@@ -207,9 +210,9 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
                 const int mt = half * HM + mh;
-                if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(bufA(b) + ((wm * C::MT + mt) * 2 + kk) * 1024 + lane * 16);
-                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(bufA(b), km, wm * C::MT + mt, kk);
-                else f[mh][kk] = g3_frag(bufA(b), wm * (16 * C::MT) + mt * 16 + r16, kk * 4 + q4);
+                if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(bufA(b) + (C::row_block(wm, mt) * 2 + kk) * 1024 + lane * 16);
+                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(bufA(b), km, C::row_block(wm, mt), kk);
+                else f[mh][kk] = g3_frag(bufA(b), C::row_block(wm, mt) * 16 + r16, kk * 4 + q4);
             }
     };
     auto readB = [&](int b, int half, bf16x8 (&f)[HN][2]) {
@@ -254,8 +257,9 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     constexpr std::integral_constant<int, HN * 2 * (BKM ? 2 : 1)> rb{};
     bf16x8 a0[HM][2], a1[HM][2], b0[HN][2], b1[HN][2];
     if (kt0 >= kt1) return;
-    stage(kt0, 0), stage(kt0 + 1, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
+#pragma unroll
+    for (int b = 0; b < C::NBUF; b++) stage(kt0 + b, b);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((C::NBUF - 1) * LPW) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory"); /* no read moves up */
     readA(0, 0, a0), readB(0, 0, b0);
@@ -264,8 +268,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     constexpr std::integral_constant<int, 0> none{};
     constexpr std::integral_constant<int, C::NIA> la{};
     constexpr std::integral_constant<int, C::NIB> lb{};
-    auto step = [&](int kt, auto cur_c, bf16x8 (&bx)[HN][2], bf16x8 (&by)[HN][2]) {
-        constexpr int cur = decltype(cur_c)::value;
+    auto step = [&](int kt, auto cur, auto nxt, bf16x8 (&bx)[HN][2], bf16x8 (&by)[HN][2]) {
         __builtin_amdgcn_sched_barrier(0);
         readB(cur, 1, by);
         mul(0, 0, a0, bx);
@@ -273,22 +276,35 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         readA(cur, 1, a1);
         mul(0, 1, a0, by);
         order(ra, none);
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((C::NBUF - 2) * LPW) : "memory");
         __builtin_amdgcn_s_barrier(); /* step kt + 1 has landed for every wave, and every wave has read all of step kt: its buffer may be filled again */
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        stageA(kt + 2, cur);
-        readA(cur ^ 1, 0, a0);
+        stageA(kt + C::NBUF, cur);
+        readA(nxt, 0, a0);
         mul(1, 1, a1, by);
         order(ra, la);
-        stageB(kt + 2, cur);
-        readB(cur ^ 1, 0, by);
+        stageB(kt + C::NBUF, cur);
+        readB(nxt, 0, by);
         mul(1, 0, a1, bx);
         order(rb, lb);
     };
-    for (int kt = kt0; kt < kt1; kt += 2) {
-        step(kt, std::integral_constant<int, 0>{}, b0, b1);
-        if (kt + 1 < kt1) step(kt + 1, std::integral_constant<int, 1>{}, b1, b0);
+    if constexpr (C::NBUF == 2) {
+        constexpr std::integral_constant<int, 0> even{};
+        constexpr std::integral_constant<int, 1> odd{};
+        for (int kt = kt0; kt < kt1; kt += 2) {
+            step(kt, even, odd, b0, b1);
+            if (kt + 1 < kt1) step(kt + 1, odd, even, b1, b0);
+        }
+    } else {
+        int cur = 0;
+        auto behind = [](int b) { return b + 1 < C::NBUF ? b + 1 : 0; };
+        for (int kt = kt0; kt < kt1; kt += 2) {
+            const int one = behind(cur), two = behind(one);
+            step(kt, cur, one, b0, b1);
+            if (kt + 1 < kt1) step(kt + 1, one, two, b1, b0);
+            cur = two;
+        }
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier(); /* the buffers are free: for a following segment's first loads, for an epilogue's exchange */
@@ -302,6 +318,24 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
 static constexpr bool g3_prefer_wide(int M, int n, int K) {
     const long by = (n + 255) / 256, rb = ((M + 255) / 256 * by + 255) / 256, rw = ((M + 191) / 192 * by + 255) / 256;
     return rw <= rb || (rw == rb + 1 && (rb == 5 || rb == 6) && K <= 2048);
+}
+// The tile of a product whose rows are whole tiles of any of them (`wide` = 192-row ones may be taken): the smallest that makes ONE round of the CUs; of several rounds the cheaper of the big
+// tiles and 128 x 128 on 4 waves (512 at a time), a round of R us taking R (ceil r + 0.8 r + 0.55) / 2 for r rounds (the last one is dealt out early and finds the caches warm) --
+// R = E + S (K / 64): 23.1 us at K = 1024 (128 x 128), 33.5 (192 x 256), 42.2 (256 x 256).  us with SwiGLU, 128 x 128 on 8 | 128 x 256 | 128 x 128 on 4 | 192 x 256 | 256 x 256:
+//   6144 x 1024   at 515 rows 14.7 | 20.6 | 17.8 | 26.1 | 32.4, at 1030 25.4 | 22.3 | 22.9 | 27.5 | 33.5, at 2047 39.3 | 41.0 | 36.9 | 31.1 | 36.0, at 2608 51.8 | 62.3 | 45.8 | 56.6 | 68.1
+//   12288 x 2048  at 515 rows 44.1 | 56.9 | 39.1 | 47.6 | 53.3, at 1030 81.7 | 67.6 | 68.3 | 87.0 | 58.3, at 2608 167 | 163 | 141 | 149 | 161, at 6000 373 | 315 | 313 | 298 | 277
+enum G3Pick { G3_DUO, G3_HALF, G3_SMALL, G3_WIDE, G3_BIG };
+static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
+    const long r128 = (M + 127) / 128, c128 = (n + 127) / 128, c256 = (n + 255) / 256, n128 = r128 * c128, nw = (M + 191) / 192 * c256, nb = (M + 255) / 256 * c256;
+    if (n128 <= 256) return G3_DUO;
+    if (r128 * c256 <= 256) return G3_HALF;
+    if (n128 <= 512 || n < 256 || M < 256) return G3_SMALL;
+    if (wide && nw <= 256) return G3_WIDE;
+    if (nb <= 256) return G3_BIG;
+    const bool w = wide && g3_prefer_wide(M, n, K);
+    const double k = K / 64, rs = n128 / 512.0, rb = (w ? nw : nb) / 256.0, Rs = 7.1 + k, Rb = w ? 13.3 + 1.26 * k : 19.0 + 1.45 * k;
+    const double ts = Rs * ((n128 + 511) / 512 + 0.8 * rs + 0.55), tb = Rb * (((w ? nw : nb) + 255) / 256 + 0.8 * rb + 0.55);
+    return ts < 0.97 * tb ? G3_SMALL : w ? G3_WIDE : G3_BIG;
 }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {

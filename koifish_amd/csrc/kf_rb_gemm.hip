@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
         if (p.epilogue == KF_RB_GATED) {
 #pragma unroll
             for (int mt = 0; mt < C::MT; mt += 2) {
-                const int m = m0 + wm * (16 * C::MT) + mt * 16;
+                const int m = m0 + C::row_block(wm, mt) * 16;
                 if (m >= p.m) continue;
                 const f32x4 g = acc[mt][nt], u = acc[mt + 1][nt];
                 f32x4 o;
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
         } else {
 #pragma unroll
             for (int mt = 0; mt < C::MT; mt++) {
-                const int m = m0 + wm * (16 * C::MT) + mt * 16 + 4 * q4;
+                const int m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
                 if (m >= p.m) continue;
                 f32x4 d = acc[mt][nt];
                 if (p.epilogue == KF_RB_STORE) {
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
 }
 template <class C, bool EXPERTS, class T = uint16_t>
 static int rb_go(hipStream_t st, const RbProduct& q, long nwg) {
-    constexpr int SMEM = 2 * C::STAGE;
+    constexpr int SMEM = C::SMEM;
     static int attr_set = 0;
     if (!attr_set && SMEM + 2 * 4 * C::BN > 64 * 1024) { /* the pair rows of the experts form sit in static LDS */
         if (hipFuncSetAttribute((const void*)rb_gemm_kernel<C, EXPERTS, T>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;

@@ -426,3 +426,20 @@ def test_a_captured_product_in_k_pieces_is_right_at_every_replay(ctx):
             ctx.hip.kf_graph_destroy(g)
         ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+@pytest.mark.parametrize("M,K,n", [(1000, 128, 257), (1024, 192, 2047), (512, 8192, 300),                  # 64 x 64, fewer k-steps than LDS buffers and more
+                                   (1032, 128, 2600), (2048, 192, 1541), (2056, 6400, 515),                # 128 x 128 on eight waves
+                                   (2048, 128, 2608), (1608, 320, 4001), (5120, 448, 1031),                # 128 x 256
+                                   (6144, 256, 1290), (6152, 256, 2608), (12288, 128, 1300)])              # 192 x 256; several rounds
+def test_tiles_of_one_round_and_more_against_fp32(ctx, M, K, n):
+    """bf16 weights over every tile that a product's size picks, ragged rows and tokens, with bias and residual: fp32 sums of K products and one bf16 rounding (2^-8 of a value, 2^-8 of the sums' scale)"""
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.BF16)
+    x, bias, res = torch.randn(n, K, device=ctx.device).bfloat16(), torch.randn(M, device=ctx.device).bfloat16(), torch.randn(n, M, device=ctx.device).bfloat16()
+    buf = torch.full((n + 2, M), 7.0, device=ctx.device, dtype=torch.bfloat16)
+    d, y = w.desc(), buf[1:n + 1]
+    assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), bias.data_ptr(), n, 1.0, 0.0, L.KF_EPI_RESIDUAL, res.data_ptr()) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    s = x.float() @ ctx.dequant(w).float().reshape(M, K).t() + bias.float()
+    assert float((y.float() - s - res.float()).abs().max()) <= 2.0 ** -8 * (float(s.abs().max()) + float((s + res.float()).abs().max()))
+    assert bool((buf[0] == 7).all()) and bool((buf[n + 1] == 7).all())

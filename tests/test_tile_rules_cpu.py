@@ -18,3 +18,16 @@ def test_the_faster_of_the_big_tiles_is_taken(tmp_path):
     src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_prefer_wide(%d, %d, %d) == %s);\n" % (m, n, k, "true" if wide < big else "false") for m, n, k, big, wide in TIMED))
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
+
+
+# (rows of the weight, token rows, K, a tile within a tenth of the fastest of the five as timed; the last: fewer than 256 tokens take no 256-token tile)
+PICKED = [(6144, 515, 1024, "DUO"), (6144, 1030, 1024, "HALF"), (6144, 2047, 1024, "WIDE"), (6144, 2608, 1024, "SMALL"), (12288, 515, 2048, "SMALL"), (12288, 1030, 2048, "BIG"), (12288, 6000, 2048, "WIDE"),
+          (24576, 700, 5120, "WIDE"), (24576, 2047, 5120, "BIG"), (2048, 2608, 6144, "HALF"), (5120, 2608, 8192, "BIG"), (1600, 8192, 1600, "BIG"), (6400, 8192, 1600, "BIG"), (151936, 200, 1024, "SMALL")]
+
+
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_one_round_of_tiles_is_taken_where_there_is_one(tmp_path):
+    src = tmp_path / "rules.hip"
+    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_pick(%d, %d, %d, true) == kf::G3_%s);\n" % (m, n, k, t) for m, n, k, t in PICKED))
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
