@@ -1,0 +1,121 @@
+// kf_flash.h -- a wave's walk over key tiles of flash attention on MFMA (32 columns, 32 keys at a time), shared by the prompt kernels of kf_attn_prefill.hip and kf_rb_attn.hip.
+//   S^T[key][col] = sum_d K[key][d] Q[col][d]      v_mfma_f32_32x32x16_bf16, A = K rows (ds_read_b128), B = Q rows (registers): a column's 32 scores sit in ONE lane pair (lane l and l ^ 32)
+//   O^T[d][col]  += sum_key V^T[d][key] P^T[key][col]   the S^T registers, packed to bf16, ARE the B operand (slot (step s, half h, j) <-> key 16 s + (j & 3) + 8 (j >> 2) + 4 h on both operands);
+//      A = V^T fragments straight from the row-major V tile (ds_read_b64_tr_b16).  p enters as a bf16 pair (high part + remainder, ~16 significant bits), its sum stays fp32.
+// What bounds it: a tile's MFMAs take 768 cycles of a SIMD at dim 128, its vector instructions about as many, and one after the other they leave both pipes idle half the time -- a SIMD has two
+// waves at most here, often one.  So the walk is a pipeline: beside the exponentials of tile t run the MFMAs of the scores of tile t + 1, beside the P.V of tile t the scaling and the maximum of
+// tile t + 1 (order() below).  And the running maximum of a column is moved only when a tile's exceeds it by 8 (log2): up to there p just grows to 2^8, which costs no precision in
+// fp32 and bf16 pairs, and the accumulator is rescaled a few times per column instead of at nearly every early tile.
+#pragma once
+#include "kf_device.h"
+
+namespace kf {
+
+typedef __bf16 fl_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 fl_bf16x4 __attribute__((ext_vector_type(4)));
+typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr float FL_SLACK = 8.0f; /* log2 */
+
+template <int HD>
+struct FlashWave {
+    static constexpr int NS = HD / 16, NDB = HD / 32; /* MFMA steps over d of S^T; 32-row blocks of O^T */
+    fl_f32x16 o[NDB];
+    float M, l; /* the column's reference exponent (log2 units; -inf: nothing seen) and this lane's half of the sum of p */
+    u32x4 qf[NS];
+    __device__ __forceinline__ void init() {
+#pragma unroll
+        for (int db = 0; db < NDB; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+        M = -__builtin_inff(), l = 0.f;
+    }
+    // scores of a tile: kfrag(s) = this lane's K fragment of MFMA step s
+    template <class KF>
+    __device__ __forceinline__ void scores(fl_f32x16& st, KF&& kfrag) const {
+        fl_f32x16 z;
+#pragma unroll
+        for (int i = 0; i < 16; i++) z[i] = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; s++) st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fl_bf16x8, kfrag(s)), __builtin_bit_cast(fl_bf16x8, qf[s]), s ? st : z, 0, 0, 0);
+    }
+    // scaled scores and their maximum over this lane's 16 keys.  ROUND: the score is stored in bf16 on its way (the reference's store)
+    template <bool ROUND>
+    static __device__ __forceinline__ float scale(fl_f32x16& st, float by) {
+        float mt = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            st[i] *= by, st[i + 1] *= by;
+            if (ROUND) {
+                const uint32_t w = pack_bf16x2(st[i], st[i + 1]);
+                st[i] = bf_lo(w), st[i + 1] = bf_hi(w);
+            }
+            mt = fmaxf(mt, fmaxf(st[i], st[i + 1]));
+        }
+        return mt;
+    }
+    // keys of the tile that the column does not see: first key k0, it sees lo .. hi
+    static __device__ __forceinline__ float mask(fl_f32x16& st, int k0, int lo, int hi, int h) {
+        float mt = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int key = k0 + 4 * h + (i & 3) + 8 * (i >> 2);
+            st[i] = key >= lo && key <= hi ? st[i] : -__builtin_inff();
+            mt = fmaxf(mt, st[i]);
+        }
+        return mt;
+    }
+    // mt: the column's maximum over the tile in log2 units (both lanes of the pair)
+    __device__ __forceinline__ void move(float mt) {
+        if (mt > M + FL_SLACK) {
+            const float alpha = __builtin_amdgcn_exp2f(M - mt); /* M = -inf on the first tile: 0 */
+            l *= alpha;
+#pragma unroll
+            for (int db = 0; db < NDB; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+            M = mt;
+        }
+    }
+    // p = 2^(LOG2E score - M) as bf16 pairs; scores in natural units where NAT, in log2 units otherwise.  A column that has seen nothing (M = -inf): p = 0
+    template <bool NAT>
+    __device__ __forceinline__ void weights(const fl_f32x16& st, uint32_t (&ph)[8], uint32_t (&pl)[8]) {
+        const float ref = M == -__builtin_inff() ? 0.f : M;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float a = st[2 * i], b = st[2 * i + 1];
+            const float p0 = __builtin_amdgcn_exp2f(NAT ? fmaf(a, 1.44269502162933349609375f, -ref) : a - ref), p1 = __builtin_amdgcn_exp2f(NAT ? fmaf(b, 1.44269502162933349609375f, -ref) : b - ref);
+            l += p0;
+            l += p1;
+            ph[i] = pack_bf16x2(p0, p1);
+            pl[i] = pack_bf16x2(p0 - bf_lo(ph[i]), p1 - bf_hi(ph[i]));
+        }
+    }
+    // O^T += V^T P^T: vfrag(s2, db) = this lane's V^T fragment of keys 16 s2 .. + 15, d 32 db .. + 31
+    template <class VF>
+    __device__ __forceinline__ void accumulate(const uint32_t (&ph)[8], const uint32_t (&pl)[8], VF&& vfrag) {
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++) {
+            const u32x4 B = u32x4{ph[4 * s2], ph[4 * s2 + 1], ph[4 * s2 + 2], ph[4 * s2 + 3]}, B2 = u32x4{pl[4 * s2], pl[4 * s2 + 1], pl[4 * s2 + 2], pl[4 * s2 + 3]};
+#pragma unroll
+            for (int db = 0; db < NDB; db++) {
+                const fl_bf16x8 A = vfrag(s2, db);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(fl_bf16x8, B), o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(fl_bf16x8, B2), o[db], 0, 0, 0);
+            }
+        }
+    }
+    // one tile of the pipeline: its scores are in `cur` (scaled, masked; mt their maximum in log2 units), those of the tile behind it come out in `nxt` (scaled; the result: this lane's maximum)
+    template <bool ROUND, bool NAT, class KF, class VF>
+    __device__ __forceinline__ float tile(fl_f32x16& cur, float mt, fl_f32x16& nxt, float by, KF&& kfrag, VF&& vfrag) {
+        move(mt);
+        uint32_t ph[8], pl[8];
+        scores(nxt, kfrag);
+        weights<NAT>(cur, ph, pl);
+        accumulate(ph, pl, vfrag);
+        const float m = scale<ROUND>(nxt, by);
+        return m;
+    }
+};
+
+}  // namespace kf

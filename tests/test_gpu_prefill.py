@@ -153,3 +153,37 @@ def test_attn_prefill_long_prompt_form_vs_oracle(ctx, nh, nkv, hd, pos0, n):
     _check_attn_rows(q, kc, vc, out, pos0, sorted(t for t in rows if 0 <= t < n), nh, nkv, hd)
     # every row was written (the fill value 3.0 cannot survive: outputs are convex combinations of N(0, 1) values rounded to bf16 -- |.| = 3.0 exactly in all of a row has probability 0)
     assert not (out == 0x4040).all(axis=1).any()
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,n", [(4, 2, 128, 0, 8), (4, 2, 128, 100, 33), (2, 2, 64, 90, 65), (8, 1, 128, 129, 127), (16, 4, 64, 0, 513), (4, 2, 128, 511, 130), (16, 2, 128, 3, 640)])
+@pytest.mark.parametrize("form", ["all keys", "halves", "quarters"])
+def test_every_split_of_the_keys_against_64_bits(ctx, form, nh, nkv, hd, pos0, n):
+    """Keys whose scores climb with the position, so that a column's running maximum moves past its slack again and again, some far below it; every dot is exact in fp32 (small multiples of 1/8), so the bf16
+    scores are the reference's own and only p (a bf16 pair, 2^-16), the sums (fp32) and one bf16 store of out differ: 2^-8 of a value, and half of that again for the sums"""
+    import ctypes as C
+    import torch
+    g = torch.Generator().manual_seed(7 * n + hd)
+    tot, GQ = pos0 + n, nh // nkv
+    q = torch.randint(-1, 2, (n, nh, hd), generator=g).float()
+    k = torch.randint(-1, 2, (tot, nkv, hd), generator=g).float() * 2
+    q[..., 0], k[..., 0] = 8.0, ((torch.arange(tot) % 251) / 8)[:, None]   # multiples of 1/8 below 32: eight bits
+    v = torch.randn(tot, nkv, hd, generator=g).bfloat16()
+    dots = torch.einsum("thd,skd->thsk", q.double(), k.double())
+    dots = torch.stack([dots[:, h, :, h // GQ] for h in range(nh)], 1)                            # [n, nh, tot]
+    s = (dots.float() * torch.tensor(1.0 / hd ** 0.5, dtype=torch.float32)).bfloat16().double()
+    s.masked_fill_(torch.arange(tot)[None, None] > (pos0 + torch.arange(n))[:, None, None], -float("inf"))
+    ref = torch.einsum("ths,shd->thd", torch.softmax(s, -1), v.double().repeat_interleave(GQ, 1))
+    wgs = (n * GQ + 127) // 128 * nkv
+    knob = {"all keys": 0, "halves": wgs // 2 if wgs > 1 else 0, "quarters": 4096}[form]
+    qd, kd, vd = (t.bfloat16().reshape(t.shape[0], -1).to(ctx.device) for t in (q, k, v))
+    buf = torch.full((n + 2, nh * hd), 3.0, dtype=torch.bfloat16, device=ctx.device)
+    try:
+        assert ctx.hip.kfdbg_set_knob(b"attn_parts_max", knob) == 0
+        rc = ctx.hip.kf_attn_prefill(ctx.h, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), buf[1:].data_ptr(), pos0, n, nh * hd, nh, nkv, hd, nkv * hd)
+        assert rc == 0, ctx.hip.kf_last_error()
+        ctx.sync()
+    finally:
+        ctx.hip.kfdbg_set_knob(b"attn_parts_max", 256)
+    got = buf[1:n + 1].cpu().double().reshape(n, nh, hd)
+    assert float((got - ref).abs().max()) <= 1.5 * 2.0 ** -8 * float(ref.abs().max())
+    assert bool((buf[0] == 3).all()) and bool((buf[n + 1] == 3).all())
