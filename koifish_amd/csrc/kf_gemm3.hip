@@ -26,97 +26,75 @@ namespace kf {
 
 // ROPE::cuInfer on a 128-row tile that is one head (hd 128) of Q or K, in the epilogue of the stacked Q | K | V launch (the arithmetic of prep_head_cs, kf_attn_common.h: the
 // projection rounded to bf16 as the plain epilogue stores it, fp64 sum of squares, s rounded to bf16, (x s) w rounded, rotate-half pairs (j, j + 64) with every product and the
-// sum rounded once).  A wave holds rows 32 wm .. + 31 and 64 + 32 wm .. + 31 (row_block): both elements of a pair, so a (cos, sin) is read once for the two and nothing is exchanged but the sums of
-// squares: over the 4 lanes of a column (row swaps) and the two wm waves (LDS).
+// sum rounded once).  A thread has eight pairs of a token, the eight threads of a token are neighbours.
 template <class C>
-__device__ __forceinline__ void g3_epilogue_qkrope(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int wid, int lane, unsigned char* smem_raw, uint16_t* ybase, long long ldy,
-                                                   int mshift, const uint16_t* nw) {
-    static_assert(C::BM == 128 && C::MT == 4, "one head per tile");
-    const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4, tok0 = wn * 16 * C::NT + r16;
-    double* red = reinterpret_cast<double*>(smem_raw); /* [2 wm][BN tokens] */
-    if (nw) {
+__device__ __forceinline__ void g3_epilogue_qkrope(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int tid, unsigned char* smem_raw, uint16_t* ybase, long long ldy, int mshift,
+                                                   const uint16_t* nw) {
+    static_assert(C::BM == 128, "one head per tile");
+    using Out = G3Out<C>;
+    static_assert(Out::TN * 8 % C::NTH == 0, "the eight threads of a token run the loop together");
+    Out::template all<8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+        const int tok = t0 + tk < a.n ? t0 + tk : a.n - 1; /* (a token past the end: the last one's angles, not stored) */
+        float x[2][8]; /* rows 8 u .. and 64 + 8 u .. */
 #pragma unroll
-        for (int nt = 0; nt < C::NT; nt++) {
+        for (int e = 0; e < 2; e++) {
+            Out::rows8(smem_raw, lt, 8 * e + u, tid, x[e]);
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[e][j] = round_bf16(x[e][j]); /* the value the plain epilogue stores (alpha 1, no bias) */
+        }
+        if (nw) {
             double ss = 0.0;
 #pragma unroll
-            for (int mt = 0; mt < C::MT; mt++)
+            for (int e = 0; e < 2; e++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const double v = (double)round_bf16(acc[mt][nt][j]); /* the value the plain epilogue stores (alpha 1, no bias) */
-                    ss = fma(v, v, ss);
-                }
-            ss = xsum32_d(xsum16_d(ss)); /* the column's 4 lanes (l ^ 16, l ^ 32): this wave's 64 rows */
-            if (q4 == 0) red[wm * C::BN + tok0 + nt * 16] = ss;
-        }
-        __syncthreads();
-    }
+                for (int j = 0; j < 8; j++) ss = fma((double)x[e][j], (double)x[e][j], ss);
 #pragma unroll
-    for (int nt = 0; nt < C::NT; nt++) {
-        const int tl = tok0 + nt * 16, tok = t0 + tl;
-        if (tok >= a.n) continue;
-        float s = 1.0f;
-        if (nw) s = round_bf16(1.0f / sqrtf((float)(red[tl] + red[C::BN + tl]) / 128.0f + a.qk_eps));
-        const f32x4* const table = reinterpret_cast<const f32x4*>(a.rope_table + (size_t)(a.rope_pos0 + (a.rope_seq > 0 ? tok % a.rope_seq : tok)) * 128);
-        uint16_t* const yt = ybase + (size_t)tok * ldy + (m0 - mshift);
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            const int jj = C::row_block(wm, mt) * 16 + 4 * q4; /* pair index 0 .. 63 of this lane's first row */
-            float x[2][4]; /* rows jj .. jj + 3 and 64 + jj .. */
+            for (int d = 1; d < 8; d *= 2) ss += __shfl_xor(ss, d, 64);
+            const float s = round_bf16(1.0f / sqrtf((float)ss / 128.0f + a.qk_eps));
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                u32x2 w4 = u32x2{0, 0};
-                if (nw) w4 = *reinterpret_cast<const u32x2*>(nw + 64 * e + jj);
-                const float w[4] = {bf_lo(w4.x), bf_hi(w4.x), bf_lo(w4.y), bf_hi(w4.y)};
+                float w[8];
+                g3_unpack8(*reinterpret_cast<const u32x4*>(nw + 64 * e + 8 * u), w);
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    x[e][j] = round_bf16(acc[2 * e + mt][nt][j]);
-                    if (nw) x[e][j] = round_bf16(x[e][j] * s * w[j]);
-                }
+                for (int j = 0; j < 8; j++) x[e][j] = round_bf16(x[e][j] * s * w[j]);
             }
-            if (a.rope_table) {
-                const f32x4 cs01 = table[jj / 2], cs23 = table[jj / 2 + 1]; /* (cos, sin) of the lane's four pairs: 32 contiguous bytes of the table */
-                const float csv[8] = {cs01.x, cs01.y, cs01.z, cs01.w, cs23.x, cs23.y, cs23.z, cs23.w};
+        }
+        if (a.rope_table) { /* (cos, sin) of the eight pairs: 64 contiguous bytes of the table */
+            const f32x4* const table = reinterpret_cast<const f32x4*>(a.rope_table + (size_t)(a.rope_pos0 + (a.rope_seq > 0 ? tok % a.rope_seq : tok)) * 128 + 16 * u);
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float c = csv[2 * j], sn = csv[2 * j + 1], lo = x[0][j], hi = x[1][j], p0 = lo * c, p1 = hi * sn, p2 = lo * sn, p3 = hi * c;
+            for (int p = 0; p < 4; p++) {
+                const f32x4 cs = table[p];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int j = 2 * p + e;
+                    const float c = cs[2 * e], sn = cs[2 * e + 1], lo = x[0][j], hi = x[1][j], p0 = lo * c, p1 = hi * sn, p2 = lo * sn, p3 = hi * c;
                     x[0][j] = p0 - p1, x[1][j] = p2 + p3;
                 }
             }
-#pragma unroll
-            for (int e = 0; e < 2; e++) *reinterpret_cast<u32x2*>(yt + 64 * e + jj) = u32x2{pack_bf16x2(x[e][0], x[e][1]), pack_bf16x2(x[e][2], x[e][3])};
         }
-    }
+        if (t0 + tk < a.n) {
+#pragma unroll
+            for (int e = 0; e < 2; e++) g3_store16(ybase + (size_t)t0 * ldy + (m0 - mshift), (uint32_t)tk * (uint32_t)(2 * ldy) + 128 * e + 16 * u, g3_pack8(x[e]));
+        }
+    });
 }
 
-// epilogue (gemm_epilogue's order): lane holds rows m .. m + 3 of a 16 x 16 tile for token column r16
+// epilogue (gemm_epilogue's order) of the tile at (m0, t0)
 template <bool AKM, class C>
-__device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int wid, int lane, unsigned char* smem_raw = nullptr) {
-    const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
-    if (a.swiglu) { /* Relu::Forw (CU_swiglu_v0, Activation.cu:85-93) on the two bf16-rounded projections, as swiglu_kernel: accumulator block 2i holds gate rows, block 2i + 1 the up rows of
-                       the same 16 FFN rows (the operand was dequantised interleaved), same lane, same register */
-        const int F = a.M >> 1;
+__device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int tid, unsigned char* smem_raw) {
+    using Out = G3Out<C>;
+    if (!AKM && a.swiglu) { /* Relu::Forw (CU_swiglu_v0, Activation.cu:85-93) on the two bf16-rounded projections, as swiglu_kernel: 16-row block 2i holds gate rows, block 2i + 1 the up rows of
+                               the same 16 FFN rows (the operand was dequantised interleaved) */
+        const int F = a.M >> 1; /* a multiple of 16 (gemm3_swiglu_launch) */
+        Out::template all<C::BM / 16>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+            const int tok = t0 + tk, f = (m0 >> 1) + 8 * u, c = (u >> 1) * 4 + (u & 1);
+            if (tok >= a.n || f >= F) return;
+            float g[8], p[8];
+            Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, p);
 #pragma unroll
-        for (int mt = 0; mt < C::MT; mt += 2)
-#pragma unroll
-            for (int nt = 0; nt < C::NT; nt++) {
-                const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, f = (m0 >> 1) + C::row_block(wm, mt) * 8 + 4 * q4;
-                if (tok >= a.n || f >= F) continue;
-                const float gv[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w}, uv[4] = {acc[mt + 1][nt].x, acc[mt + 1][nt].y, acc[mt + 1][nt].z, acc[mt + 1][nt].w};
-                uint16_t o[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float g = round_bf16(gv[j]), u = round_bf16(uv[j]);
-                    o[j] = f2bf((g * u) / (1.0f + kf_expf(-g)));
-                }
-                uint16_t* yp = a.y + (size_t)tok * a.ldy + f;
-                if (f + 3 < F && ((a.ldy & 3) == 0)) {
-                    *reinterpret_cast<u32x2*>(yp) = u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        if (f + j < F) yp[j] = o[j];
-                }
-            }
+            for (int j = 0; j < 8; j++) g[j] = round_bf16(g[j]), p[j] = round_bf16(p[j]), g[j] = (g[j] * p[j]) / (1.0f + kf_expf(-g[j]));
+            g3_store16(a.y + (size_t)t0 * a.ldy + (m0 >> 1), (uint32_t)tk * (uint32_t)(2 * a.ldy) + 16 * u, g3_pack8(g));
+        });
         return;
     }
     // up to three matrices stacked along M (Q | K | V or gate | up, each a multiple of the 256-row tile: a.rb_end[j] = cumulative rows / 32): the tile's rows go to
@@ -131,71 +109,61 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
         else Mlim = e0;
     }
     if constexpr (!AKM && C::BM == 128) {
-        if (a.qkrope && smem_raw) { /* workgroup-uniform: a tile lies inside one job */
+        if (a.qkrope) { /* workgroup-uniform: a tile lies inside one job */
             const int job = a.njobs > 1 ? (m0 >= a.rb_end[1] * 32 ? 2 : (m0 >= a.rb_end[0] * 32 ? 1 : 0)) : 0;
             if (job < 2) {
-                g3_epilogue_qkrope<C>(a, m0, t0, acc, wid, lane, smem_raw, ybase, ldy, mshift, a.qk_norm[job]);
+                g3_epilogue_qkrope<C>(a, m0, t0, acc, tid, smem_raw, ybase, ldy, mshift, a.qk_norm[job]);
                 return;
             }
         }
     }
-    const bool vec_ok = ((ldy & 3) == 0) && ((reinterpret_cast<uintptr_t>(ybase) & 7) == 0);
     const uint16_t* const res = AKM ? nullptr : a.residual;
-    // four rows of a token at a time, every operand of theirs 8 aligned bytes (bias and residual were 2-byte loads, 256 of them per lane: the forward products of a training step
-    // took 1.3 x what they take without a bias)
-    const bool wide = vec_ok && ((reinterpret_cast<uintptr_t>(a.bias) | reinterpret_cast<uintptr_t>(res)) & 7) == 0 && (!res || (a.ldr & 3) == 0) && (Mlim & 3) == 0;
-    if (wide) {
+    // eight rows of a token, every operand of theirs 16 aligned bytes; else one row
+    const bool whole = ((ldy | Mlim) & 7) == 0 && ldy < (1 << 22) && ((reinterpret_cast<uintptr_t>(ybase) | reinterpret_cast<uintptr_t>(res) | reinterpret_cast<uintptr_t>(a.bias)) & 15) == 0 && (!res || (a.ldr & 7) == 0);
+    if (whole) {
+        Out::template all<C::BM / 8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+            const int tok = t0 + tk, m = m0 + 8 * u;
+            if (tok >= a.n || m >= Mlim) return;
+            u32x4 r4 = u32x4{0, 0, 0, 0};
+            if (res) r4 = *reinterpret_cast<const u32x4*>(res + (size_t)tok * a.ldr + m);
+            float v[8], o[8];
+            Out::rows8(smem_raw, lt, u, tid, v);
+            if (a.alpha != 1.0f) {
 #pragma unroll
-        for (int mt = 0; mt < C::MT; mt++) {
-            const int m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
-            if (m >= Mlim) continue;
-            u32x2 b4 = u32x2{0, 0};
-            if (a.bias) b4 = *reinterpret_cast<const u32x2*>(a.bias + m);
-            const float bv[4] = {bf_lo(b4.x), bf_hi(b4.x), bf_lo(b4.y), bf_hi(b4.y)};
-#pragma unroll
-            for (int nt = 0; nt < C::NT; nt++) {
-                const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16;
-                if (tok >= a.n) continue;
-                u32x2* const yp = reinterpret_cast<u32x2*>(ybase + (size_t)tok * ldy + (m - mshift));
-                u32x2 r4 = u32x2{0, 0}, y4 = u32x2{0, 0};
-                if (res) r4 = *reinterpret_cast<const u32x2*>(res + (size_t)tok * a.ldr + m);
-                if (a.beta != 0.0f) y4 = *yp;
-                const float rv[4] = {bf_lo(r4.x), bf_hi(r4.x), bf_lo(r4.y), bf_hi(r4.y)}, yv[4] = {bf_lo(y4.x), bf_hi(y4.x), bf_lo(y4.y), bf_hi(y4.y)};
-                float v[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w};
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (a.alpha != 1.0f) v[j] = a.alpha * v[j];
-                    if (a.beta != 0.0f) v[j] = v[j] + a.beta * yv[j];
-                    if (a.bias) v[j] = v[j] + bv[j];
-                    if (res) v[j] = rv[j] + round_bf16(v[j]);
-                }
-                *yp = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                for (int j = 0; j < 8; j++) v[j] = a.alpha * v[j];
             }
-        }
+            if (a.beta != 0.0f) {
+                g3_unpack8(*reinterpret_cast<const u32x4*>(ybase + (size_t)tok * ldy + (m - mshift)), o);
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = v[j] + a.beta * o[j];
+            }
+            if (a.bias) {
+                g3_unpack8(*reinterpret_cast<const u32x4*>(a.bias + m), o);
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = v[j] + o[j];
+            }
+            if (res) {
+                g3_unpack8(r4, o);
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = o[j] + round_bf16(v[j]);
+            }
+            g3_store16(ybase + (size_t)t0 * ldy + (m0 - mshift), (uint32_t)tk * (uint32_t)(2 * ldy) + 16 * u, g3_pack8(v));
+        });
         return;
     }
-#pragma unroll
-    for (int mt = 0; mt < C::MT; mt++)
-#pragma unroll
-        for (int nt = 0; nt < C::NT; nt++) {
-            const int tok = t0 + wn * (16 * C::NT) + nt * 16 + r16, m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
-            if (tok >= a.n || m >= Mlim) continue;
-            uint16_t* yp = ybase + (size_t)tok * ldy + (m - mshift);
-            const float vv[4] = {acc[mt][nt].x, acc[mt][nt].y, acc[mt][nt].z, acc[mt][nt].w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (m + j >= Mlim) continue;
-                float v = vv[j];
-                if (a.alpha != 1.0f) v = a.alpha * v;
-                if (a.beta != 0.0f) v = v + a.beta * bf2f(yp[j]);
-                if (a.bias) v = v + bf2f(a.bias[m + j]);
-                uint16_t qv = f2bf(v);
-                if (res) qv = f2bf(bf2f(res[(size_t)tok * a.ldr + m + j]) + bf2f(qv));
-                yp[j] = qv;
-            }
-        }
+    Out::template all<C::BM>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+        const int tok = t0 + tk, m = m0 + u;
+        if (tok >= a.n || m >= Mlim) return;
+        uint16_t* const yp = ybase + (size_t)tok * ldy + (m - mshift);
+        float v = *reinterpret_cast<const float*>(smem_raw + Out::at(lt, u >> 2) + 4 * (u & 3));
+        if (a.alpha != 1.0f) v = a.alpha * v;
+        if (a.beta != 0.0f) v = v + a.beta * bf2f(*yp);
+        if (a.bias) v = v + bf2f(a.bias[m]);
+        uint16_t q = f2bf(v);
+        if (res) q = f2bf(bf2f(res[(size_t)tok * a.ldr + m]) + bf2f(q));
+        *yp = q;
+    });
 }
-// bijective XCD remap: the blocks with equal blockIdx % 8 (one XCD under round-robin placement) get consecutive logical indices
 
 template <bool AKM, bool BKM, int BK, class C>
 __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_kernel(const GemmArgs a) {
@@ -213,7 +181,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_kerne
         for (int j = 0; j < C::NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     g3_mainloop<AKM, BKM, BK, C>(a, m0, t0, 0, a.K / BK, acc, smem_raw, wid, lane);
     const int e = g3_opaque(tid);
-    g3_epilogue<AKM, C>(a, m0, t0, acc, e >> 6, e & 63, smem_raw);
+    g3_epilogue<AKM, C>(a, m0, t0, acc, e, smem_raw);
 }
 
 // SPLIT-K forms for launches with fewer tiles than CUs (a weight gradient [OC, IC] is 49 .. 175 tiles, its contraction 8192 token rows long).  The pieces are cut so
@@ -317,7 +285,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_sk_ke
             g3_publish<C>(s, slot, acc, e);
         } else {
             for (int c = c0; c < c1; c++) g3_collect<C>(s, c, acc, e);
-            g3_epilogue<AKM, C>(a, m0, t0, acc, e >> 6, e & 63, smem_raw);
+            g3_epilogue<AKM, C>(a, m0, t0, acc, e, smem_raw);
         }
         it += helper ? k1 - k0 : 1;
     }
@@ -504,7 +472,7 @@ int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int*
     if (nwg < 64 && (long)(tot / 128) * ((n + 127) / 128) < 64) return 1;
     const long n128 = g3_tiles_of(tot, n, 128, 128);
     if (rope) { /* a head-sized tile: one round of the wider or the deeper one where it is one */
-        if (n_w != 3 || M[0] % 128 != 0 || M[1] % 128 != 0 || ((M[0] | M[1] | M[2]) & 3) || (reinterpret_cast<uintptr_t>(y[0]) & 7) || (reinterpret_cast<uintptr_t>(y[1]) & 7)) return 1;
+        if (n_w != 3 || M[0] % 128 != 0 || M[1] % 128 != 0 || ((reinterpret_cast<uintptr_t>(y[0]) | reinterpret_cast<uintptr_t>(y[1]) | reinterpret_cast<uintptr_t>(rope->wq) | reinterpret_cast<uintptr_t>(rope->wk) | reinterpret_cast<uintptr_t>(rope->table)) & 15)) return 1;
         a.qkrope = 1, a.qk_norm[0] = rope->wq, a.qk_norm[1] = rope->wk, a.rope_table = rope->table, a.rope_pos0 = rope->pos0, a.rope_seq = rope->seq_len, a.qk_eps = rope->eps;
     }
     if (rope) return n128 <= 256 ? g3_whole<G3Duo>(st, a) : g3_tiles_of(tot, n, 128, 256) <= 256 ? g3_whole<G3Half>(st, a) : g3_whole<G3Small>(st, a);
@@ -516,7 +484,7 @@ int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int*
 int gemm3_swiglu_launch(hipStream_t st, const uint16_t* Wilv, int ffn, int K, const uint16_t* x, long long ldx, int n, uint16_t* act) {
     const int M = 2 * ffn;
     if (ffn % 16 != 0 || M % G3_BM != 0 || K % G3_BK != 0 || K < G3_BK || n < G3_BN || (ldx & 7) || (ffn & 3) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(Wilv) & 15) ||
-        (reinterpret_cast<uintptr_t>(act) & 7))
+        (reinterpret_cast<uintptr_t>(act) & 15))
         return 1;
     GemmArgs a;
     memset(&a, 0, sizeof(a));

@@ -15,8 +15,7 @@ template <int BM_, int BN_, int NW_, int NBUF_ = 2>
 struct G3Cfg {
     static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = NW_ / 2, MT = BM_ / 32, NT = BN_ / (16 * (NW_ / 2)), NBUF = NBUF_;
     static constexpr int NIA = BM_ / (8 * NW_), NIB = BN_ / (8 * NW_); /* global_load_lds instructions per wave, operand and k-step (8 rows of 128 bytes each) */
-    /* the 16-row block of the tile that is block mt of the waves wm: in order, but for 128 rows, which may be one head -- there a wave holds both elements of its rotation pairs (rows j and j + 64) */
-    static constexpr __host__ __device__ int row_block(int wm, int mt) { return BM == 128 ? 4 * (mt >> 1) + 2 * wm + (mt & 1) : wm * MT + mt; }
+    static constexpr __host__ __device__ int row_block(int wm, int mt) { return wm * MT + mt; } /* the 16-row block of the tile that is block mt of the waves wm */
     static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, SMEM = NBUF_ * STAGE, WGS_PER_CU = (160 * 1024) / SMEM;
 };
 using G3Big = G3Cfg<256, 256, 8>;      /* 128 KiB of LDS: one workgroup per CU */
@@ -318,6 +317,59 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     asm volatile("" ::: "memory");
 }
 
+// The output tile on its way out: the accumulators go to LDS as they are, where the operands' buffers were, and a LOOP over eight rows of a token applies the epilogue and stores 16 bytes a lane, whole rows of the
+// tile at a time.  What bounds an epilogue is its CODE: it runs once, so every line of it is an instruction-cache miss (two CUs share 64 KiB), and unrolled over the 32 MFMA tiles of a wave it was 40 - 60 KB:
+// a 256 x 256 tile took 14.4 us to store (4096 x 4096 in one round), from this loop it takes 8.4 (writing as much alone: 4).  Storing rows instead of 32-byte pieces from code as long changed nothing.
+// PASSES: the tile in 32 bits may be more than the buffers hold; then half of every wave's tokens at a time.  16-byte chunks of a token are XOR-swizzled by the token: a wave's writes (16 tokens x one chunk) and its
+// reads (consecutive chunks) touch all banks once.
+template <class C>
+struct G3Out {
+    static constexpr int PASSES = (C::BM * C::BN * 4 + C::SMEM - 1) / C::SMEM, TN = C::BN / PASSES, HT = C::NT / PASSES; /* tokens, and 16-token blocks of a wave, per pass */
+    static_assert(PASSES <= 2 && C::NT % PASSES == 0 && C::BM % 64 == 0, "a token is whole turns of the banks");
+    static __device__ __forceinline__ int at(int lt, int chunk) { return lt * (4 * C::BM) + ((chunk ^ (lt & 15)) << 4); } /* rows 4 chunk .. + 3 of the pass's token lt */
+    static __device__ __forceinline__ int token(int pass, int lt) { return PASSES == 1 ? lt : lt / (16 * HT) * (16 * C::NT) + pass * (16 * HT) + lt % (16 * HT); } /* its place in the tile */
+    static __device__ __forceinline__ void spill(const f32x4 (&acc)[C::MT][C::NT], unsigned char* smem, int pass, int wid, int lane) {
+        const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
+        unsigned char* const to = smem + (wn * (16 * HT) + r16) * (4 * C::BM); /* (16 tokens further the swizzle is the same) */
+#pragma unroll
+        for (int mt = 0; mt < C::MT; mt++) {
+            unsigned char* const b = to + (((C::row_block(wm, mt) * 4 + q4) ^ r16) << 4);
+#pragma unroll
+            for (int nt = 0; nt < HT; nt++) *reinterpret_cast<f32x4*>(b + nt * 16 * (4 * C::BM)) = PASSES == 2 && pass ? acc[mt][nt + C::NT - HT] : acc[mt][nt];
+        }
+    }
+    /* rows 8 c .. 8 c + 7 of token lt; which of the two chunks is read first alternates every eight lanes, so that sixteen lanes in a row meet in no bank */
+    static __device__ __forceinline__ void rows8(const unsigned char* smem, int lt, int c, int lane, float (&v)[8]) {
+        const bool odd = (lane >> 3) & 1;
+        const f32x4 p = *reinterpret_cast<const f32x4*>(smem + at(lt, 2 * c + (odd ? 1 : 0))), q = *reinterpret_cast<const f32x4*>(smem + at(lt, 2 * c + (odd ? 0 : 1)));
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = odd ? q[j] : p[j], v[4 + j] = odd ? p[j] : q[j];
+    }
+    /* f(token of the tile, token of the pass, unit) for this thread's share of TN tokens x U units, after a barrier */
+    template <int U, class F>
+    static __device__ __forceinline__ void each(int pass, int tid, F&& f) {
+        __syncthreads();
+#pragma unroll 1
+        for (int id = tid; id < TN * U; id += C::NTH) f(token(pass, id / U), id / U, id % U);
+    }
+    /* PASSES times: the accumulators to LDS, then each<U> */
+    template <int U, class F>
+    static __device__ __forceinline__ void all(const f32x4 (&acc)[C::MT][C::NT], unsigned char* smem, int tid, F&& f) {
+#pragma unroll
+        for (int pass = 0; pass < PASSES; pass++) {
+            if (pass) __syncthreads();
+            spill(acc, smem, pass, tid >> 6, tid & 63);
+            each<U>(pass, tid, f);
+        }
+    }
+};
+// 16 bytes to base + off (base: uniform), written through: left to the write-back of the XCDs' L2s at the launch's end a one-round product is 1.5 - 2.5 us longer
+__device__ __forceinline__ void g3_store16(void* base, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, g3_rsrc(base, G3_ALL), off, 0, 16 /* sc1 */); }
+__device__ __forceinline__ u32x4 g3_pack8(const float (&v)[8]) { return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])}; }
+__device__ __forceinline__ void g3_unpack8(u32x4 p, float (&v)[8]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[2 * j] = bf_lo(p[j]), v[2 * j + 1] = bf_hi(p[j]);
+}
 // 256 x 256 or 192 x 256: with one big workgroup per CU a launch takes whole rounds of 256 tiles, and a round of the smaller ones takes 0.79 to 0.95 of a round, so the smaller tile pays where it needs no
 // more rounds.  us, big | wide: 6144 x 1024 at 2608 rows (264 | 352 tiles) 66.7 | 54.3, x 4096 176 | 143, x 25600 1230 | 1036; 5120 x 12288 at 4096 rows (320 | 432) 543 | 518; 10240 x 8192 at 3500 rows
 // (560 | 756) 522 | 449.  One round more pays for 5 and 6 of them at K <= 2048, where the round is shortest against its start: 12288 x 2048 at 5888 rows (1104 | 1472) 280 | 269, at 6912 (1296 | 1728) 332 |
@@ -328,9 +380,10 @@ static constexpr bool g3_prefer_wide(int M, int n, int K) {
 }
 // The tile of a product whose rows are whole tiles of any of them (`wide` = 192-row ones may be taken): the smallest that makes ONE round of the CUs; of several rounds the cheaper of the big
 // tiles and 128 x 128 on 4 waves (512 at a time), a round of R us taking R (ceil r + 0.8 r + 0.55) / 2 for r rounds (the last one is dealt out early and finds the caches warm) --
-// R = E + S (K / 64): 23.1 us at K = 1024 (128 x 128), 33.5 (192 x 256), 42.2 (256 x 256).  us with SwiGLU, 128 x 128 on 8 | 128 x 256 | 128 x 128 on 4 | 192 x 256 | 256 x 256:
-//   6144 x 1024   at 515 rows 14.7 | 20.6 | 17.8 | 26.1 | 32.4, at 1030 25.4 | 22.3 | 22.9 | 27.5 | 33.5, at 2047 39.3 | 41.0 | 36.9 | 31.1 | 36.0, at 2608 51.8 | 62.3 | 45.8 | 56.6 | 68.1
-//   12288 x 2048  at 515 rows 44.1 | 56.9 | 39.1 | 47.6 | 53.3, at 1030 81.7 | 67.6 | 68.3 | 87.0 | 58.3, at 2608 167 | 163 | 141 | 149 | 161, at 6000 373 | 315 | 313 | 298 | 277
+// R = E + S (K / 64): 19.7 us at K = 1024 (128 x 128), 29.2 (192 x 256), 33.3 (256 x 256).  us, 128 x 128 on 8 | 128 x 256 | 128 x 128 on 4 | 192 x 256 | 256 x 256:
+//   4096 x 1024   at 2047 rows 22.6 | 18.9 | 19.7 | 22.9 | 28.3, at 2608 32.6 | 34.5 | 31.1 | 24.6 | 30.1, at 4096 48.0 | 39.3 | 38.5 | 48.1 | 33.3
+//   6144 x 1024 with SwiGLU at 2047 rows 36.9 | 40.0 | 35.1 | 29.2 | 36.0, at 2608 47.5 | 58.3 | 39.9 | 53.5 | 67.9
+//   6400 x 1600 at 8192 rows 191 | 174 | 169 | 164 | 169, 12288 x 2048 with SwiGLU at 8190 rows 448 | 372 | 368 | 339 | 327
 enum G3Pick { G3_DUO, G3_HALF, G3_SMALL, G3_WIDE, G3_BIG };
 static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
     const long r128 = (M + 127) / 128, c128 = (n + 127) / 128, c256 = (n + 255) / 256, n128 = r128 * c128, nw = (M + 191) / 192 * c256, nb = (M + 255) / 256 * c256;
@@ -340,7 +393,7 @@ static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
     if (wide && nw <= 256) return G3_WIDE;
     if (nb <= 256) return G3_BIG;
     const bool w = wide && g3_prefer_wide(M, n, K);
-    const double k = K / 64, rs = n128 / 512.0, rb = (w ? nw : nb) / 256.0, Rs = 7.1 + k, Rb = w ? 13.3 + 1.26 * k : 19.0 + 1.45 * k;
+    const double k = K / 64, rs = n128 / 512.0, rb = (w ? nw : nb) / 256.0, Rs = 3.7 + k, Rb = w ? 9.0 + 1.26 * k : 10.1 + 1.45 * k;
     const double ts = Rs * ((n128 + 511) / 512 + 0.8 * rs + 0.55), tb = Rb * (((w ? nw : nb) + 255) / 256 + 0.8 * rb + 0.55);
     return ts < 0.97 * tb ? G3_SMALL : w ? G3_WIDE : G3_BIG;
 }

@@ -15,6 +15,16 @@ using RbMid = G3Cfg<64, 128, 4>;
 using RbTiny = G3Cfg<64, 64, 4>;
 using RbPairs = G3Cfg<128, 64, 4>; /* experts of about a hundred pairs: half the padding of 128-pair tiles, each weight tile read about once */
 
+// eight values from a multiple of 8 columns; rows of 16-bit values are at least 8-byte aligned
+__device__ __forceinline__ void rb_st8(uint16_t* p, const float (&v)[8], int64_t ld) {
+    const u32x4 o = g3_pack8(v);
+    if ((ld & 7) == 0) *reinterpret_cast<u32x4*>(p) = o;
+    else reinterpret_cast<u32x2*>(p)[0] = u32x2{o.x, o.y}, reinterpret_cast<u32x2*>(p)[1] = u32x2{o.z, o.w};
+}
+__device__ __forceinline__ void rb_st8(float* p, const float (&v)[8], int64_t) {
+    reinterpret_cast<f32x4*>(p)[0] = f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p)[1] = f32x4{v[4], v[5], v[6], v[7]};
+}
+
 // T: the storage, uint16_t (bf16: weights in MFMA tiles) or float (true 32-bit: weights in rows)
 template <class C, bool EXPERTS, class T>
 __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_kernel(const RbProduct q) {
@@ -48,53 +58,53 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     } else {
         g3_mainloop<false, false, G3_BK, C, std::conditional_t<U == 2, G3RowsF32, G3Tiled>>(a, m0, t0, 0, p.k / KT, acc, smem_raw, wid, lane);
     }
-    const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
+    // the tile by way of LDS (G3Out); rows of y: the token itself, or the pair in the token tile's place
+    using Out = G3Out<C>;
+    T* const y = reinterpret_cast<T*>(p.y);
+    auto row_of = [&](int tk) { return EXPERTS ? s_dst[EXPERTS ? tk : 0] : (t0 + tk < p.n ? t0 + tk : -1); };
+    if (p.epilogue == KF_RB_GATED) {
+        Out::template all<C::BM / 16>(acc, smem_raw, tid, [&](int tk, int lt, int u) { /* rows of 16 gates and of the 16 ups behind them: eight outputs */
+            const int row = row_of(tk), f = (m0 >> 1) + 8 * u, c = (u >> 1) * 4 + (u & 1);
+            if (row < 0 || 2 * f >= p.m) return;
+            const float scale = EXPERTS && p.mode == KF_RB_UP ? q.e.weight[row] : 1.f;
+            float g[8], v[8];
+            Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, v);
 #pragma unroll
-    for (int nt = 0; nt < C::NT; nt++) {
-        const int col = wn * (16 * C::NT) + nt * 16 + r16;
-        int row = t0 + col;
-        float scale = 1.f;
-        if constexpr (EXPERTS) {
-            row = s_dst[col];
-            if (row < 0) continue;
-            if (p.mode == KF_RB_UP) scale = q.e.weight[row];
-        } else {
-            if (row >= p.n) continue;
-        }
-        if (p.epilogue == KF_RB_GATED) {
+            for (int j = 0; j < 8; j++) g[j] = scale * (rb_activate(p.act, g[j]) * v[j]);
+            rb_st8(y + (size_t)row * p.ldy + f, g, p.ldy);
+        });
+    } else if (p.epilogue == KF_RB_STORE && U == 1) {
+        Out::template all<C::BM / 8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+            const int row = row_of(tk), m = m0 + 8 * u;
+            if (row < 0 || m >= p.m) return;
+            float v[8];
+            Out::rows8(smem_raw, lt, u, tid, v);
+            if (m + 7 >= p.act_lo && m < p.act_hi) {
 #pragma unroll
-            for (int mt = 0; mt < C::MT; mt += 2) {
-                const int m = m0 + C::row_block(wm, mt) * 16;
-                if (m >= p.m) continue;
-                const f32x4 g = acc[mt][nt], u = acc[mt + 1][nt];
-                f32x4 o;
-#pragma unroll
-                for (int j = 0; j < 4; j++) o[j] = scale * (rb_activate(p.act, g[j]) * u[j]);
-                rb_st4(reinterpret_cast<T*>(p.y) + (size_t)row * p.ldy + (m >> 1) + 4 * q4, o);
-            }
-        } else {
-#pragma unroll
-            for (int mt = 0; mt < C::MT; mt++) {
-                const int m = m0 + C::row_block(wm, mt) * 16 + 4 * q4;
-                if (m >= p.m) continue;
-                f32x4 d = acc[mt][nt];
-                if (p.epilogue == KF_RB_STORE) {
-                    if (m + 3 >= p.act_lo && m < p.act_hi) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++)
-                            if (m + j >= p.act_lo && m + j < p.act_hi) d[j] = rb_activate(p.act, d[j]);
-                    }
-                    rb_st4(reinterpret_cast<T*>(p.y) + (size_t)row * p.ldy + m, d);
-                } else {
-                    if (p.epilogue == KF_RB_RESIDUAL) {
-                        const f32x4 r = rb_ld4(p.res + (size_t)row * p.ldr + m);
-#pragma unroll
-                        for (int j = 0; j < 4; j++) d[j] = fmaf(p.alpha, r[j], d[j]);
-                    }
-                    rb_st4(reinterpret_cast<float*>(p.y) + (size_t)row * p.ldy + m, d);
+                for (int j = 0; j < 8; j++) {
+                    const float w = rb_activate(p.act, v[j]);
+                    v[j] = m + j >= p.act_lo && m + j < p.act_hi ? w : v[j];
                 }
             }
-        }
+            rb_st8(y + (size_t)row * p.ldy + m, v, p.ldy);
+        });
+    } else {
+        Out::template all<C::BM / 4>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+            const int row = row_of(tk), m = m0 + 4 * u;
+            if (row < 0 || m >= p.m) return;
+            f32x4 d = *reinterpret_cast<const f32x4*>(smem_raw + Out::at(lt, u));
+            if (U == 2 && p.epilogue == KF_RB_STORE && m + 3 >= p.act_lo && m < p.act_hi) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (m + j >= p.act_lo && m + j < p.act_hi) d[j] = rb_activate(p.act, d[j]);
+            }
+            if (p.epilogue == KF_RB_RESIDUAL) {
+                const f32x4 r = rb_ld4(p.res + (size_t)row * p.ldr + m);
+#pragma unroll
+                for (int j = 0; j < 4; j++) d[j] = fmaf(p.alpha, r[j], d[j]);
+            }
+            rb_st4(reinterpret_cast<float*>(p.y) + (size_t)row * p.ldy + m, d);
+        });
     }
 }
 template <class C, bool EXPERTS, class T = uint16_t>
