@@ -1,26 +1,30 @@
 // kf_attn_bwd_mfma.hip -- causal multi-head attention backward on MFMA (flash form), gfx950 / wave64.  Same contract as kf_attn_bwd.hip (its
-// header has the mathematics and the reference), same two-launch split, the tile algebra of the forward kernel (kf_attn_prefill.hip):
+// header has the mathematics and the reference), same two-launch split, the tile algebra of the forward kernel (kf_flash.h):
 //
-//   dQ launch, workgroup = 128 query columns (32 per wave), key tiles of 32 staged in LDS (K and V row-major, K a second time with the row stride the transposing reads want):
-//     pass A   S^T[key][col] = K . Q^T                      -> the column's log-sum-exp L (and D = dO . O from registers), kept for launch 2
-//     pass B   S^T again, dP^T[key][col] = V . dO^T         A = K / V rows (ds_read_b128), B = Q / dO rows (registers, loaded once)
-//              dS^T = exp(scale S^T - L) o (dP^T - D)       element-wise on the accumulators: a column lives in one lane pair
-//              dQ^T[d][col] += K^T[d][key] . dS^T[key][col] the dS^T registers, packed to bf16, ARE the B operand (free contraction order)
-//   dK/dV launch, workgroup = 128 key columns, query tiles of 32 from the diagonal down (Q and dO row-major, twice: row reads / transposing reads; L and D of the tile):
+//   dQ launch, workgroup = 128 query columns (32 per wave), ONE walk over key tiles of 32:
+//              S^T[key][col] = K . Q^T, dP^T[key][col] = V . dO^T     A = K / V rows (ds_read_b128), B = Q / dO rows (registers, loaded once)
+//              p = exp(scale S^T - M), dS^T = p o (dP^T - D)          element-wise on the accumulators: a column lives in one lane pair; M the column's running reference as in the forward kernel
+//              dQ^T[d][col] += K^T[d][key] . dS^T[key][col]           the dS^T registers, packed to bf16, ARE the B operand (free contraction order)
+//              dQ is linear in p, so it is divided by the sum of p at the end; the column's log-sum-exp L and D = dO . O go to launch 2, side by side
+//   dK/dV launch, workgroup = 128 key columns, query tiles of 32 from the diagonal down (Q, dO, and L | D of the tile's queries):
 //              S[q][key] = Q . K^T, dP[q][key] = dO . V^T   A = Q / dO rows, B = K / V rows of the column (registers)
-//              P = exp(scale S - L_q), dS = P o (dP - D_q)  L, D per accumulator ROW: four ds_read_b128 each
+//              P = exp(scale S - L_q), dS = P o (dP - D_q)  L, D per accumulator ROW: two ds_read_b128 per four rows
 //              dV^T[d][key] += dO^T[d][q] . P[q][key],  dK^T[d][key] += Q^T[d][q] . dS[q][key]
 // P and dS enter their products as single bf16 values (gradients are compared at 2^-7 of scale); everything else fp32.
+//
+// What bounds it: per 32 x 32 tile the two launches' MFMAs take 384 + 512 cycles of a SIMD at dim 64 and their vector instructions about as many.  A tile goes global -> LDS by buffer loads, AB_NB buffers, ONE barrier per
+// tile; it lies there once, under a swizzle that suits the row reads and the transposing reads of the same rows (ab_swz); two or three waves to a SIMD do the rest.  25 heads x 64, 8 x 1024 tokens: 430 us with tiles staged through
+// registers, twice each, two barriers a tile and a walk of its own for L; 164 (76 + 88) so.
 #include "kf_kernels.h"
 
 namespace kf {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int AB_T = 32;        /* tile of keys (dQ launch) / queries (dK/dV launch) */
-constexpr int AB_PAD2 = 32;     /* row padding (elements, 64 B) of the second row-major copy that the transposing reads use: 4 rows of a 32-lane pass -> distinct 16-bank groups */
-constexpr float AB_LOG2E = 1.44269502162933349609375f;
+constexpr int AB_T = 32, AB_NB = 4; /* rows of a tile; buffers: two to three tiles are on their way */
+constexpr float AB_LOG2E = 1.44269502162933349609375f, AB_SLACK = 8.0f; /* the running reference of a column moves only past 2^8 (kf_flash.h) */
 
 __device__ __forceinline__ f32x16 ab_zero() {
     f32x16 z;
@@ -31,74 +35,85 @@ __device__ __forceinline__ f32x16 ab_zero() {
 __device__ __forceinline__ f32x16 ab_mfma(u32x4 A, u32x4 B, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A), __builtin_bit_cast(bf16x8, B), c, 0, 0, 0);
 }
-// stage a [32][HD] tile of rows (row index clamped to T - 1) row-major (padded rows) and, optionally, a second time with AB_PAD2 row padding (ab_tfrag's operand)
-template <int HD, bool TRANSPOSE>
-__device__ __forceinline__ void ab_stage(const uint16_t* __restrict__ src, long long ld, size_t hoff, int row0, int T, uint16_t* rows, uint16_t* tr) {
-    constexpr int KS = HD + 8, CH = AB_T * HD / 8;
-    for (int c = threadIdx.x; c < CH; c += 256) {
-        const int row = c / (HD / 8), dc = c - row * (HD / 8);
-        int rr = row0 + row;
-        rr = rr < T ? rr : T - 1;
-        const u32x4 x = *reinterpret_cast<const u32x4*>(src + (size_t)rr * ld + hoff + dc * 8);
-        *reinterpret_cast<u32x4*>(rows + row * KS + dc * 8) = x;
-        if (TRANSPOSE) *reinterpret_cast<u32x4*>(tr + row * (HD + AB_PAD2) + dc * 8) = x;
-    }
-}
-// the same in two halves, so that a tile's global loads can be in flight while the previous tile is multiplied: registers <- global, LDS <- registers
+// the place of 16-byte chunk c of row r: 16 rows of a chunk (row reads) and four rows, from a multiple of four, of four chunks (transposing reads) touch all 64 banks once
 template <int HD>
-__device__ __forceinline__ void ab_load(const uint16_t* __restrict__ src, long long ld, size_t hoff, int row0, int T, u32x4* regs) {
-    constexpr int CH = AB_T * HD / 8;
-#pragma unroll
-    for (int i = 0; i < CH / 256; i++) {
-        const int c = threadIdx.x + 256 * i, row = c / (HD / 8), dc = c - row * (HD / 8);
-        int rr = row0 + row;
-        rr = rr < T ? rr : T - 1;
-        regs[i] = *reinterpret_cast<const u32x4*>(src + (size_t)rr * ld + hoff + dc * 8);
-    }
+__device__ __forceinline__ int ab_swz(int r, int c) {
+    return HD == 128 ? c ^ (((r & 3) << 2) | ((r >> 2) & 3)) : c ^ ((((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1));
 }
-template <int HD, bool TRANSPOSE>
-__device__ __forceinline__ void ab_store(const u32x4* regs, uint16_t* rows, uint16_t* tr) {
-    constexpr int KS = HD + 8, CH = AB_T * HD / 8;
-#pragma unroll
-    for (int i = 0; i < CH / 256; i++) {
-        const int c = threadIdx.x + 256 * i, row = c / (HD / 8), dc = c - row * (HD / 8);
-        *reinterpret_cast<u32x4*>(rows + row * KS + dc * 8) = regs[i];
-        if (TRANSPOSE) *reinterpret_cast<u32x4*>(tr + row * (HD + AB_PAD2) + dc * 8) = regs[i];
-    }
-}
-// A fragment of X^T (row d = 32 db + (lane & 31), contraction slots j <-> tile rows 16 s2 + (j & 3) + 8 (j >> 2) + 4 h) read straight from the second row-major
-// copy of the tile with two transposing ds_read_b64_tr_b16: lane l16 of a 16-lane group addresses tile row (l16 >> 2) of its 4 and d-piece 4 (l16 & 3) of the
-// group's 16 d, and receives the 4 rows' values of d = l16 (scratch/dbg/ds_read_tr_probe.hip).  No transposed copy, no 16-bit scatter stores.
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 template <int HD>
-__device__ __forceinline__ u32x4 ab_tfrag(const uint16_t* rows2, int db, int s2, int lane) {
-    constexpr int VS = HD + AB_PAD2;
-    const uint16_t* p = rows2 + (16 * s2 + 4 * (lane >> 5) + ((lane & 15) >> 2)) * VS + db * 32 + (lane & 16) + 4 * (lane & 3);
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(p));
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(p + 8 * VS));
-    return __builtin_bit_cast(u32x4, bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+struct AbTile {
+    static constexpr int RB = 2 * HD, PART = AB_T * RB, RPI = 1024 / RB, NI = PART / 4096; /* bytes of a row, of a tile; rows per load instruction; instructions per wave (four to a workgroup) */
+    int rf[HD / 16], tl[HD / 32], th[HD / 32]; /* this lane's offsets: row fragments per MFMA step, transposing reads per 32 columns (tile rows 4 h + (l16 >> 2), and 8 further) */
+    int off_row[NI], off_chunk[NI];
+    __device__ __forceinline__ void init(int lane, int wave) {
+        const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+        for (int s = 0; s < HD / 16; s++) rf[s] = r * RB + ab_swz<HD>(r, 2 * s + h) * 16;
+#pragma unroll
+        for (int db = 0; db < HD / 32; db++) { /* lane l16 of a 16-lane group addresses row (l16 >> 2) of its 4, piece 4 (l16 & 3) of the group's 16 columns; it receives the 4 rows' values of column l16 */
+            const int row = 4 * h + ((lane & 15) >> 2), c = 4 * db + ((lane & 16) >> 3) + ((lane & 3) >> 1);
+            tl[db] = row * RB + ab_swz<HD>(row, c) * 16 + 8 * (lane & 1);
+            th[db] = (row + 8) * RB + ab_swz<HD>(row + 8, c) * 16 + 8 * (lane & 1);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; i++) off_row[i] = (wave * NI + i) * RPI + lane / (HD / 8), off_chunk[i] = ab_swz<HD>(off_row[i], lane % (HD / 8)) * 16;
+    }
+    __device__ __forceinline__ u32x4 rows(const unsigned char* tile, int s) const { return *reinterpret_cast<const u32x4*>(tile + rf[s]); }
+    // contraction slots j <-> tile rows 16 s2 + (j & 3) + 8 (j >> 2) + 4 h
+    __device__ __forceinline__ u32x4 turned(const unsigned char* tile, int db, int s2) const {
+        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(tile + tl[db] + 16 * s2 * RB));
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(tile + th[db] + 16 * s2 * RB));
+        return __builtin_bit_cast(u32x4, bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+    }
+    // 32 rows from `base` (rows `row_bytes` apart, `left` of them exist: the others become zeros) into LDS, this wave's share
+    __device__ __forceinline__ void load(const uint16_t* base, uint32_t row_bytes, int left, unsigned char* to, int wave) const {
+#ifdef __HIP_DEVICE_COMPILE__
+        const long long n = left <= 0 ? 0 : (long long)(left < AB_T ? left : AB_T) * row_bytes;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (int)n, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < NI; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(to + (wave * NI + i) * 1024), 16, (uint32_t)off_row[i] * row_bytes + off_chunk[i], 0, 0, 0);
+#endif
+    }
+};
+template <int N>
+__device__ __forceinline__ void ab_landed() { /* all but the wave's N latest loads have landed, for every wave, and every wave has read what it wanted */
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// f over a tile and the place that the loads set out for meanwhile, told apart (restrict): the compiler otherwise puts a wait for those loads in front of every transposing read
+template <class F>
+__device__ __forceinline__ void ab_apart(const unsigned char* __restrict__ tile, unsigned char* __restrict__ to, F&& f) {
+    f(tile, to);
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256) attn_bwd_dq_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o,
-                                                               uint16_t* dq, long long ld_d, float* Lbuf, float* Dbuf, int T, float scale, int gq, long long ld_kv) {
-    constexpr int NS = HD / 16, NDB = HD / 32, KS = HD + 8;
-    __shared__ __attribute__((aligned(16))) uint16_t ks[AB_T * KS], vs[AB_T * KS], kt[AB_T * (HD + AB_PAD2)];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-    const int head = blockIdx.y, tok0 = (gridDim.x - 1 - blockIdx.x) * 128; /* the longest columns first */
+__global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o,
+                                                                                 uint16_t* dq, long long ld_d, float* LD, int T, float scale, int gq, long long ld_kv) {
+    using Tile = AbTile<HD>;
+    constexpr int NS = HD / 16, NDB = HD / 32, SET = 2 * Tile::PART, LPS = 2 * Tile::NI; /* K and V of a tile; loads per wave and tile */
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+    /* consecutive workgroups go to consecutive XCDs: a head's blocks stay on the same one(s); the longest columns first */
+    const int wg = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y, head = wg % (int)gridDim.y, tok0 = ((int)gridDim.x - 1 - wg / (int)gridDim.y) * 128;
     const size_t hoff = (size_t)head * HD, hoff_kv = (size_t)(head / gq) * HD; /* GQA: gq query heads share a kv head */
     { /* sequence blockIdx.z: T rows further on in every tensor */
         const size_t ro = (size_t)blockIdx.z * T;
-        q += ro * ld_qkv, k += ro * ld_kv, v += ro * ld_kv, o += ro * ld_o, dO += ro * ld_o, dq += ro * ld_d;
-        Lbuf += (size_t)blockIdx.z * gridDim.y * T, Dbuf += (size_t)blockIdx.z * gridDim.y * T;
+        q += ro * ld_qkv, k += ro * ld_kv + hoff_kv, v += ro * ld_kv + hoff_kv, o += ro * ld_o, dO += ro * ld_o, dq += ro * ld_d;
+        LD += (size_t)blockIdx.z * gridDim.y * T * 2;
     }
-    int tok = tok0 + wave * 32 + r;
+    const int tok_last = tok0 + 127 < T ? tok0 + 127 : T - 1, ntile = tok_last / AB_T + 1, first = tok0 + wave * 32; /* first: this wave's first column */
+    Tile W;
+    W.init(lane, wave);
+    const uint32_t rb = (uint32_t)(ld_kv * 2);
+    auto load = [&](int t, unsigned char* to) {
+        const int left = t < ntile ? T - t * AB_T : 0;
+        W.load(k + (size_t)t * AB_T * ld_kv, rb, left, to, wave);
+        W.load(v + (size_t)t * AB_T * ld_kv, rb, left, to + Tile::PART, wave);
+    };
+    int tok = first + r;
     const bool col_ok = tok < T;
     if (!col_ok) tok = T - 1;
-    int tok_last = tok0 + 127;
-    tok_last = tok_last < T ? tok_last : T - 1;
-    const int ntile = tok_last / AB_T + 1;
-
     u32x4 qf[NS], dof[NS];
     float Dp = 0.f;
     {
@@ -116,118 +131,108 @@ __global__ void __launch_bounds__(256) attn_bwd_dq_mfma_kernel(const uint16_t* q
         }
     }
     const float D = Dp + __shfl_xor(Dp, 32, 64);
+#pragma unroll
+    for (int b = 0; b < AB_NB - 1; b++) load(b, smem_raw + b * SET);
 
-    // ---- pass A: log-sum-exp of every column
-    float M = -__builtin_inff(), l = 0.f;
-    for (int t = 0; t < ntile; t++) {
-        __syncthreads();
-        ab_stage<HD, false>(k, ld_kv, hoff_kv, t * AB_T, T, ks, nullptr);
-        __syncthreads();
-        f32x16 st = ab_zero();
-#pragma unroll
-        for (int s = 0; s < NS; s++) st = ab_mfma(*reinterpret_cast<const u32x4*>(ks + r * KS + 16 * s + 8 * h), qf[s], st);
-        // scores in log2 units (scale * log2 e folded in): M, l are the running maximum / sum of 2^(s - M)
-        float sc[16], mt = -__builtin_inff();
-        const bool full = t * AB_T + AB_T - 1 <= tok0 + wave * 32;
-        const float c1 = scale * AB_LOG2E;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int key = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2);
-            sc[i] = st[i] * c1;
-            if (!full) sc[i] = key <= tok ? sc[i] : -__builtin_inff();
-            mt = fmaxf(mt, sc[i]);
-        }
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        if (mt > M) l *= __builtin_amdgcn_exp2f(M - mt), M = mt;
-#pragma unroll
-        for (int i = 0; i < 16; i++) l += __builtin_amdgcn_exp2f(sc[i] - M);
-    }
-    l += __shfl_xor(l, 32, 64);
-    const float L = (M + __log2f(l)) * 0.693147182464599609375f; /* back to natural units: log-sum-exp of the scaled scores */
-    if (col_ok && h == 0) Lbuf[(size_t)head * T + tok] = L, Dbuf[(size_t)head * T + tok] = D;
-
-    // ---- pass B: dQ^T
     f32x16 acc[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; db++) acc[db] = ab_zero();
-    constexpr int CPT = AB_T * HD / 8 / 256;
-    u32x4 kreg[CPT], vreg[CPT];
-    __syncthreads(); /* pass A's last readers of ks are done */
-    ab_load<HD>(k, ld_kv, hoff_kv, 0, T, kreg);
-    ab_load<HD>(v, ld_kv, hoff_kv, 0, T, vreg);
-    ab_store<HD, true>(kreg, ks, kt);
-    ab_store<HD, false>(vreg, vs, nullptr);
-    __syncthreads();
+    float M = -__builtin_inff(), l = 0.f; /* log2 units; this lane's half of the sum */
+    const float c1 = scale * AB_LOG2E;
+    int b = 0;
     for (int t = 0; t < ntile; t++) {
-        const bool more = t + 1 < ntile;
-        if (more) { /* the next tile's rows travel while this one is multiplied */
-            ab_load<HD>(k, ld_kv, hoff_kv, (t + 1) * AB_T, T, kreg);
-            ab_load<HD>(v, ld_kv, hoff_kv, (t + 1) * AB_T, T, vreg);
-        }
-        f32x16 st = ab_zero(), dpt = ab_zero();
+        ab_landed<(AB_NB - 2) * LPS>(); /* tile t; tile t + NB - 1 goes where tile t - 1 was */
+        ab_apart(smem_raw + b * SET, smem_raw + (b ? b - 1 : AB_NB - 1) * SET, [&](const unsigned char* tile, unsigned char* to) __attribute__((always_inline)) {
+            load(t + AB_NB - 1, to);
+            if (t * AB_T > first + 31) return; /* every key of the tile follows this wave's columns */
+            f32x16 st = ab_zero(), dpt = ab_zero();
 #pragma unroll
-        for (int s = 0; s < NS; s++) {
-            st = ab_mfma(*reinterpret_cast<const u32x4*>(ks + r * KS + 16 * s + 8 * h), qf[s], st);
-            dpt = ab_mfma(*reinterpret_cast<const u32x4*>(vs + r * KS + 16 * s + 8 * h), dof[s], dpt);
-        }
-        uint32_t dw[8];
-        const bool full = t * AB_T + AB_T - 1 <= tok0 + wave * 32; /* every key of the tile precedes every column of this wave: no mask */
-        const float c1 = scale * AB_LOG2E, L2 = L * AB_LOG2E;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            float ds[2];
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int ii = 2 * i + e, key = t * AB_T + 4 * h + (ii & 3) + 8 * (ii >> 2);
-                float p = __builtin_amdgcn_exp2f(fmaf(st[ii], c1, -L2));
-                if (!full) p = key <= tok ? p : 0.f;
-                ds[e] = p * (dpt[ii] - D);
+            for (int s = 0; s < NS; s++) {
+                st = ab_mfma(W.rows(tile, s), qf[s], st);
+                dpt = ab_mfma(W.rows(tile + Tile::PART, s), dof[s], dpt);
             }
-            dw[i] = pack_bf16x2(ds[0], ds[1]);
-        }
+            if (t * AB_T + AB_T - 1 > first) { /* else every key of the tile precedes every column of this wave */
 #pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
-            const u32x4 B = u32x4{dw[4 * s2], dw[4 * s2 + 1], dw[4 * s2 + 2], dw[4 * s2 + 3]};
+                for (int i = 0; i < 16; i++) st[i] = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2) <= tok ? st[i] : -__builtin_inff();
+            }
+            float mt = st[0];
 #pragma unroll
-            for (int db = 0; db < NDB; db++) acc[db] = ab_mfma(ab_tfrag<HD>(kt, db, s2, lane), B, acc[db]);
-        }
-        __syncthreads(); /* everyone has read this tile */
-        if (more) {
-            ab_store<HD, true>(kreg, ks, kt);
-            ab_store<HD, false>(vreg, vs, nullptr);
-        }
-        __syncthreads();
+            for (int i = 1; i < 16; i++) mt = fmaxf(mt, st[i]);
+            mt = xmax32(mt) * c1;
+            if (mt > M + AB_SLACK) {
+                const float alpha = __builtin_amdgcn_exp2f(M - mt); /* M = -inf on the first tile: 0 */
+                l *= alpha;
+#pragma unroll
+                for (int db = 0; db < NDB; db++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[db][i] *= alpha;
+                M = mt;
+            }
+            uint32_t dw[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(st[2 * i], c1, -M)), p1 = __builtin_amdgcn_exp2f(fmaf(st[2 * i + 1], c1, -M));
+                l += p0;
+                l += p1;
+                dw[i] = pack_bf16x2(p0 * (dpt[2 * i] - D), p1 * (dpt[2 * i + 1] - D));
+            }
+#pragma unroll
+            for (int s2 = 0; s2 < 2; s2++) {
+                const u32x4 B = u32x4{dw[4 * s2], dw[4 * s2 + 1], dw[4 * s2 + 2], dw[4 * s2 + 3]};
+#pragma unroll
+                for (int db = 0; db < NDB; db++) acc[db] = ab_mfma(W.turned(tile, db, s2), B, acc[db]);
+            }
+        });
+        b = b + 1 < AB_NB ? b + 1 : 0;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* loads past the last tile write zeros: none may be on its way when the workgroup's LDS goes to another */
+    l = xsum32(l);
     if (!col_ok) return;
+    if (h == 0) LD[((size_t)head * T + tok) * 2] = M + __log2f(l), LD[((size_t)head * T + tok) * 2 + 1] = D; /* log-sum-exp of the scaled scores, log2 units */
+    const float by = scale / l;
     uint16_t* out = dq + (size_t)tok * ld_d + hoff;
 #pragma unroll
     for (int db = 0; db < NDB; db++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const int d = 32 * db + 8 * g + 4 * h;
-            *reinterpret_cast<u32x2*>(out + d) = u32x2{pack_bf16x2(acc[db][4 * g] * scale, acc[db][4 * g + 1] * scale), pack_bf16x2(acc[db][4 * g + 2] * scale, acc[db][4 * g + 3] * scale)};
+            *reinterpret_cast<u32x2*>(out + d) = u32x2{pack_bf16x2(acc[db][4 * g] * by, acc[db][4 * g + 1] * by), pack_bf16x2(acc[db][4 * g + 2] * by, acc[db][4 * g + 3] * by)};
         }
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256) attn_bwd_dkv_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* dO, long long ld_o, uint16_t* dk,
-                                                                uint16_t* dv, long long ld_d, const float* Lbuf, const float* Dbuf, int T, float scale, int gq, long long ld_kv, long long ld_dkv) {
-    constexpr int NS = HD / 16, NDB = HD / 32, KS = HD + 8;
-    __shared__ __attribute__((aligned(16))) uint16_t qs[AB_T * KS], os[AB_T * KS], qt[AB_T * (HD + AB_PAD2)], ot[AB_T * (HD + AB_PAD2)];
-    __shared__ __attribute__((aligned(16))) float Ls[AB_T], Ds[AB_T];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-    const int kvh = blockIdx.y, key0 = blockIdx.x * 128; /* blockIdx.y = kv head; the first key columns see the most query tiles: already first */
+__global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dkv_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* dO, long long ld_o, uint16_t* dk,
+                                                                                  uint16_t* dv, long long ld_d, const float* LD, int T, float scale, int gq, long long ld_kv, long long ld_dkv) {
+    using Tile = AbTile<HD>;
+    constexpr int NS = HD / 16, NDB = HD / 32, SET = 2 * Tile::PART + 1024, LPS = 2 * Tile::NI + 1; /* Q and dO of a tile, and each wave's own copy of its L | D; loads per wave and tile */
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+    const int wg = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y, kvh = wg % (int)gridDim.y, key0 = wg / (int)gridDim.y * 128; /* the first key columns see the most query tiles: first */
     const size_t hoff = (size_t)kvh * HD;
     {
         const size_t ro = (size_t)blockIdx.z * T;
         q += ro * ld_qkv, k += ro * ld_kv, v += ro * ld_kv, dO += ro * ld_o, dk += ro * ld_dkv, dv += ro * ld_dkv;
-        Lbuf += (size_t)blockIdx.z * gridDim.y * gq * T, Dbuf += (size_t)blockIdx.z * gridDim.y * gq * T;
+        LD += (size_t)blockIdx.z * gridDim.y * gq * T * 2;
     }
-    int key = key0 + wave * 32 + r;
+    const int ntq = (T + AB_T - 1) / AB_T, tg0 = (key0 / AB_T) * gq, tg1 = ntq * gq; /* (query tile, query head of the group) pairs */
+    Tile W;
+    W.init(lane, wave);
+    const uint32_t rbq = (uint32_t)(ld_qkv * 2), rbo = (uint32_t)(ld_o * 2);
+    int lt = tg0 / gq, lh = 0; /* the pair loaded next */
+    auto load = [&](unsigned char* to) {
+        const int left = lt < ntq ? T - lt * AB_T : 0, head = kvh * gq + lh;
+        W.load(q + (size_t)lt * AB_T * ld_qkv + (size_t)head * HD, rbq, left, to, wave);
+        W.load(dO + (size_t)lt * AB_T * ld_o + (size_t)head * HD, rbo, left, to + Tile::PART, wave);
+#ifdef __HIP_DEVICE_COMPILE__
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(LD + ((size_t)head * T + lt * AB_T) * 2), 0, left < 0 ? 0 : left * 8, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(to + 2 * Tile::PART + wave * 256), 4, lane * 4, 0, 0, 0);
+#endif
+        if (++lh == gq) lh = 0, lt++;
+    };
+    const int wave_key0 = key0 + wave * 32;
+    int key = wave_key0 + r;
     const bool key_ok = key < T;
     if (!key_ok) key = T - 1;
-    const int wave_key0 = key0 + wave * 32;
-
     u32x4 kf_[NS], vf[NS];
     {
         const uint16_t* krow = k + (size_t)key * ld_kv + hoff;
@@ -235,74 +240,54 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_mfma_kernel(const uint16_t* 
 #pragma unroll
         for (int s = 0; s < NS; s++) kf_[s] = *reinterpret_cast<const u32x4*>(krow + 16 * s + 8 * h), vf[s] = *reinterpret_cast<const u32x4*>(vrow + 16 * s + 8 * h);
     }
+#pragma unroll
+    for (int b = 0; b < AB_NB - 1; b++) load(smem_raw + b * SET);
     f32x16 dka[NDB], dva[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; db++) dka[db] = ab_zero(), dva[db] = ab_zero();
-    const int ntq = (T + AB_T - 1) / AB_T;
-    constexpr int CPT = AB_T * HD / 8 / 256;
-    u32x4 qreg[CPT], oreg[CPT];
-    float lreg = 0.f, dreg = 0.f;
-    const int tg0 = (key0 / AB_T) * gq, tg1 = ntq * gq;
-    auto fetch = [&](int tg) { /* (query tile, query head of the group) pair tg: rows of Q and dO, L and D of the tile's queries */
-        const int t = tg / gq, head = kvh * gq + (tg - t * gq);
-        ab_load<HD>(q, ld_qkv, (size_t)head * HD, t * AB_T, T, qreg);
-        ab_load<HD>(dO, ld_o, (size_t)head * HD, t * AB_T, T, oreg);
-        if (tid < AB_T) {
-            const int qi = t * AB_T + tid;
-            lreg = qi < T ? Lbuf[(size_t)head * T + qi] * AB_LOG2E : 0.f, dreg = qi < T ? Dbuf[(size_t)head * T + qi] : 0.f;
-        }
-    };
-    auto put = [&]() {
-        ab_store<HD, true>(qreg, qs, qt);
-        ab_store<HD, true>(oreg, os, ot);
-        if (tid < AB_T) Ls[tid] = lreg, Ds[tid] = dreg;
-    };
-    if (tg0 < tg1) fetch(tg0);
-    put();
-    __syncthreads();
+    const float c1 = scale * AB_LOG2E;
+    int b = 0, t = tg0 / gq, th = 0;
     for (int tg = tg0; tg < tg1; tg++) {
-        const int t = tg / gq;
-        const bool more = tg + 1 < tg1;
-        if (more) fetch(tg + 1);
-        if (t * AB_T + AB_T - 1 >= wave_key0) { /* else: every query of the tile precedes this wave's keys */
-        f32x16 st = ab_zero(), dpt = ab_zero();
+        ab_landed<(AB_NB - 2) * LPS>();
+        ab_apart(smem_raw + b * SET, smem_raw + (b ? b - 1 : AB_NB - 1) * SET, [&](const unsigned char* tile, unsigned char* to) __attribute__((always_inline)) {
+            load(to);
+            if (t * AB_T + AB_T - 1 < wave_key0) return; /* every query of the tile precedes this wave's keys */
+            f32x16 st = ab_zero(), dpt = ab_zero();
 #pragma unroll
-        for (int s = 0; s < NS; s++) {
-            st = ab_mfma(*reinterpret_cast<const u32x4*>(qs + r * KS + 16 * s + 8 * h), kf_[s], st);
-            dpt = ab_mfma(*reinterpret_cast<const u32x4*>(os + r * KS + 16 * s + 8 * h), vf[s], dpt);
-        }
-        uint32_t pw[8], dw[8];
-        /* every query of the tile follows every key of this wave and lies inside the sequence: no mask */
-        const bool full = t * AB_T >= wave_key0 + 31 && t * AB_T + AB_T <= T && wave_key0 + 31 < T;
-        const float c1 = scale * AB_LOG2E;
-#pragma unroll
-        for (int g = 0; g < 4; g++) { /* accumulator rows 8 g + 4 h + {0..3}: one 16-byte read of L and of D */
-            const f32x4 Lq = *reinterpret_cast<const f32x4*>(Ls + 8 * g + 4 * h), Dq = *reinterpret_cast<const f32x4*>(Ds + 8 * g + 4 * h);
-            float p[4], ds[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int qi = t * AB_T + 8 * g + 4 * h + e;
-                p[e] = __builtin_amdgcn_exp2f(fmaf(st[4 * g + e], c1, -Lq[e])); /* Ls holds L * log2 e */
-                if (!full) p[e] = (key_ok && qi < T && qi >= key) ? p[e] : 0.f;
-                ds[e] = p[e] * (dpt[4 * g + e] - Dq[e]);
+            for (int s = 0; s < NS; s++) {
+                st = ab_mfma(W.rows(tile, s), kf_[s], st);
+                dpt = ab_mfma(W.rows(tile + Tile::PART, s), vf[s], dpt);
             }
-            pw[2 * g] = pack_bf16x2(p[0], p[1]), pw[2 * g + 1] = pack_bf16x2(p[2], p[3]);
-            dw[2 * g] = pack_bf16x2(ds[0], ds[1]), dw[2 * g + 1] = pack_bf16x2(ds[2], ds[3]);
-        }
+            if (t * AB_T < wave_key0 + 31) { /* else every query of the tile follows every key of this wave; rows past the sequence's end are zeros in Q, dO, L and D and add nothing */
 #pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
-            const u32x4 BP = u32x4{pw[4 * s2], pw[4 * s2 + 1], pw[4 * s2 + 2], pw[4 * s2 + 3]}, BS = u32x4{dw[4 * s2], dw[4 * s2 + 1], dw[4 * s2 + 2], dw[4 * s2 + 3]};
-#pragma unroll
-            for (int db = 0; db < NDB; db++) {
-                dva[db] = ab_mfma(ab_tfrag<HD>(ot, db, s2, lane), BP, dva[db]);
-                dka[db] = ab_mfma(ab_tfrag<HD>(qt, db, s2, lane), BS, dka[db]);
+                for (int i = 0; i < 16; i++) st[i] = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2) >= key ? st[i] : -__builtin_inff();
             }
-        }
-        } /* wave has work on this tile */
-        __syncthreads();
-        if (more) put();
-        __syncthreads();
+            uint32_t pw[8], dw[8];
+            const f32x4* const ld = reinterpret_cast<const f32x4*>(tile + 2 * Tile::PART + wave * 256);
+#pragma unroll
+            for (int g = 0; g < 4; g++) /* accumulator rows 8 g + 4 h + {0..3} */
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const f32x4 w = ld[4 * g + 2 * h + e]; /* L, D of two queries */
+                    const int i = 4 * g + 2 * e;
+                    const float p0 = __builtin_amdgcn_exp2f(fmaf(st[i], c1, -w[0])), p1 = __builtin_amdgcn_exp2f(fmaf(st[i + 1], c1, -w[2]));
+                    pw[2 * g + e] = pack_bf16x2(p0, p1);
+                    dw[2 * g + e] = pack_bf16x2(p0 * (dpt[i] - w[1]), p1 * (dpt[i + 1] - w[3]));
+                }
+#pragma unroll
+            for (int s2 = 0; s2 < 2; s2++) {
+                const u32x4 BP = u32x4{pw[4 * s2], pw[4 * s2 + 1], pw[4 * s2 + 2], pw[4 * s2 + 3]}, BS = u32x4{dw[4 * s2], dw[4 * s2 + 1], dw[4 * s2 + 2], dw[4 * s2 + 3]};
+#pragma unroll
+                for (int db = 0; db < NDB; db++) {
+                    dva[db] = ab_mfma(W.turned(tile + Tile::PART, db, s2), BP, dva[db]);
+                    dka[db] = ab_mfma(W.turned(tile, db, s2), BS, dka[db]);
+                }
+            }
+        });
+        b = b + 1 < AB_NB ? b + 1 : 0;
+        if (++th == gq) th = 0, t++;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!key_ok) return;
     uint16_t* okp = dk + (size_t)key * ld_dkv + hoff;
     uint16_t* ovp = dv + (size_t)key * ld_dkv + hoff;
@@ -316,23 +301,30 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_mfma_kernel(const uint16_t* 
         }
 }
 
+template <int HD>
+static int ab_go(hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o, uint16_t* dq, uint16_t* dk, uint16_t* dv,
+                 long long ld_d, int T, int n_head, int n_seq, float* LD, int n_kv, long long ld_kv, long long ld_dkv) {
+    constexpr int smem_q = AB_NB * 2 * AbTile<HD>::PART, smem_kv = AB_NB * (2 * AbTile<HD>::PART + 1024);
+    static int attr_set = 0;
+    if (!attr_set && smem_kv > 64 * 1024) {
+        if (hipFuncSetAttribute((const void*)attn_bwd_dq_mfma_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q) != hipSuccess) return KF_HIP_CHECK;
+        if (hipFuncSetAttribute((const void*)attn_bwd_dkv_mfma_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv) != hipSuccess) return KF_HIP_CHECK;
+        attr_set = 1;
+    }
+    const float scale = 1.0f / sqrtf((float)HD);
+    const dim3 grid((T + 127) / 128, n_head, n_seq), grid_kv((T + 127) / 128, n_kv, n_seq);
+    hipLaunchKernelGGL((attn_bwd_dq_mfma_kernel<HD>), grid, dim3(256), smem_q, st, q, k, v, ld_qkv, o, dO, ld_o, dq, ld_d, LD, T, scale, n_head / n_kv, ld_kv);
+    hipLaunchKernelGGL((attn_bwd_dkv_mfma_kernel<HD>), grid_kv, dim3(256), smem_kv, st, q, k, v, ld_qkv, dO, ld_o, dk, dv, ld_d, LD, T, scale, n_head / n_kv, ld_kv, ld_dkv);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
 // KF_OK launched; 1 = shape not covered by the MFMA form
 int attn_backward_mfma_launch(hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o,
                               uint16_t* dq, uint16_t* dk, uint16_t* dv, long long ld_d, int T, int n_head, int hd, int n_seq, float* scratch, int n_kv, long long ld_kv, long long ld_dkv) {
     if ((hd != 64 && hd != 128) || n_kv < 1 || n_head % n_kv != 0) return 1;
-    const int gq = n_head / n_kv;
-    const float scale = 1.0f / sqrtf((float)hd);
-    float* Lb = scratch;
-    float* Db = scratch + (size_t)n_seq * n_head * T;
-    const dim3 grid((T + 127) / 128, n_head, n_seq), grid_kv((T + 127) / 128, n_kv, n_seq);
-    if (hd == 64) {
-        hipLaunchKernelGGL((attn_bwd_dq_mfma_kernel<64>), grid, dim3(256), 0, st, q, k, v, ld_qkv, o, dO, ld_o, dq, ld_d, Lb, Db, T, scale, gq, ld_kv);
-        hipLaunchKernelGGL((attn_bwd_dkv_mfma_kernel<64>), grid_kv, dim3(256), 0, st, q, k, v, ld_qkv, dO, ld_o, dk, dv, ld_d, Lb, Db, T, scale, gq, ld_kv, ld_dkv);
-    } else {
-        hipLaunchKernelGGL((attn_bwd_dq_mfma_kernel<128>), grid, dim3(256), 0, st, q, k, v, ld_qkv, o, dO, ld_o, dq, ld_d, Lb, Db, T, scale, gq, ld_kv);
-        hipLaunchKernelGGL((attn_bwd_dkv_mfma_kernel<128>), grid_kv, dim3(256), 0, st, q, k, v, ld_qkv, dO, ld_o, dk, dv, ld_d, Lb, Db, T, scale, gq, ld_kv, ld_dkv);
-    }
-    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+    if ((ld_qkv | ld_o | ld_kv) >= (1 << 24)) return 1; /* 32 rows in reach of a load's 32-bit offset */
+    float* const LD = scratch; /* [n_seq][n_head][T][2]: log-sum-exp and dO . O of a query */
+    return hd == 64 ? ab_go<64>(st, q, k, v, ld_qkv, o, dO, ld_o, dq, dk, dv, ld_d, T, n_head, n_seq, LD, n_kv, ld_kv, ld_dkv)
+                    : ab_go<128>(st, q, k, v, ld_qkv, o, dO, ld_o, dq, dk, dv, ld_d, T, n_head, n_seq, LD, n_kv, ld_kv, ld_dkv);
 }
 
 }  // namespace kf

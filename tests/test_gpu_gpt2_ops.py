@@ -437,3 +437,33 @@ def test_rope_backward_bit_exact(ctx):
     f = lambda a: O.bf16_to_f32(a).astype(np.float64)
     lhs, rhs = float(f(O.rope(x, H, hd, 5, theta)) @ f(g)), float(f(x) @ f(O.rope_backward(g, H, hd, 5, theta)))
     assert abs(lhs - rhs) <= 2.0 ** -6 * (abs(lhs) + 1.0)
+
+
+@pytest.mark.parametrize("T,H,G,hd,std", [(1, 2, 2, 64, 1.0), (31, 1, 1, 64, 1.0), (129, 2, 1, 128, 3.0), (700, 4, 2, 64, 4.0), (1000, 2, 2, 64, 0.1), (515, 2, 2, 128, 4.0)])
+def test_attn_backward_where_references_move(ctx, T, H, G, hd, std):
+    """gradients against fp64: more tiles than LDS buffers, one query, grouped heads, scores that keep growing (a column's reference moves) and hardly differ; two sequences back to back.
+    P and dS enter their products in bf16: 2^-8 of a summand each, and D = dO . O holds the forward's bf16 rounding: 2^-6 of the largest gradient"""
+    g = torch.Generator().manual_seed(T)
+    S, dev = 2, ctx.device
+    r = lambda n, s: (torch.randn(S * T, n, generator=g) * s).bfloat16()
+    q, k, v, dO = r(H * hd, std), r(G * hd, std), r(G * hd, 1.0), r(H * hd, 1.0)
+    k *= torch.linspace(0.2, 1.0, T).repeat(S)[:, None].bfloat16()
+    x = [t.double().requires_grad_() for t in (q, k, v)]
+    heads = lambda t, n: t.reshape(S, T, n, hd).permute(0, 2, 1, 3)
+    qh, kh, vh = heads(x[0], H), heads(x[1], G).repeat_interleave(H // G, 1), heads(x[2], G).repeat_interleave(H // G, 1)
+    s = (qh @ kh.transpose(-1, -2) * hd ** -0.5).masked_fill(~torch.ones(T, T, dtype=torch.bool).tril(), -float("inf"))
+    out = (torch.softmax(s, -1) @ vh).permute(0, 2, 1, 3).reshape(S * T, H * hd)
+    out.backward(dO.double())
+    d = [t.to(dev) for t in (q, k, v, out.detach().bfloat16(), dO)]
+    # rows of K and V as wide as those of Q, gradients alike: columns behind the last kv head stay as they are
+    wide = torch.zeros(3, S * T, H * hd, dtype=torch.bfloat16, device=dev)
+    wide[0, :, :G * hd], wide[1, :, :G * hd] = d[1], d[2]
+    got = torch.zeros(3, S * T, H * hd, dtype=torch.bfloat16, device=dev)
+    sc = torch.zeros(ctx.hip.kf_attn_backward_scratch_bytes(T, H, S) // 4 + 1, dtype=torch.float32, device=dev)
+    assert ctx.hip.kf_attn_backward(ctx.h, d[0].data_ptr(), wide[0].data_ptr(), wide[1].data_ptr(), H * hd, d[3].data_ptr(), d[4].data_ptr(), H * hd, got[0].data_ptr(), got[1].data_ptr(), got[2].data_ptr(),
+                                    H * hd, T, H, G, hd, S, sc.data_ptr()) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    for i, n in enumerate((H, G, G)):
+        ref, y = x[i].grad, got[i].double().cpu()
+        assert float((y[:, :n * hd] - ref).abs().max()) <= 2.0 ** -6 * max(float(ref.abs().max()), 2.0 ** -6 * (i < 2)), i
+        assert bool((y[:, n * hd:] == 0).all())
