@@ -336,6 +336,9 @@ int kf_argmax_rows_state(kf_ctx* ctx, const kf_bf16* logits, long long ld, int n
  * destinations); sizes, strides and the offset multiples of 16 bytes.  One launch scatters the K / V rows of a batch of prompts into the prompts' own caches
  * (the reference re-aims K.out / V.out at the cache rows of ONE sequence, TGraph.cpp:198-207). */
 int kf_copy_blocks(kf_ctx* ctx, void* const* d_dst_table, size_t dst_offset, const void* src, size_t src_stride, size_t block_bytes, int n_blocks);
+/* The ends of a batch of prompts: d_ends [n][4] = {row of x, sequence, token, position}; y row i = that row of x (dim columns, rows dim apart), and the sequence's decode state
+ * d_states [..][4] becomes {token, position, unchanged, 0}. */
+int kf_prompt_ends(kf_ctx* ctx, const kf_bf16* x, int dim, const int32_t* d_ends, int n, kf_bf16* y, int32_t* d_states);
 /* value into `width` bytes of each of `rows` rows `pitch` bytes apart, on the context's stream (the padded logit columns of a step) */
 int kf_memset2d(kf_ctx* ctx, void* p, size_t pitch, int value, size_t width, size_t rows);
 

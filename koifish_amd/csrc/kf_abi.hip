@@ -1203,6 +1203,12 @@ int kf_copy_blocks(kf_ctx* c, void* const* d_dst_table, size_t dst_offset, const
     if (r == KF_INVALID_ARGS) return fail(r, "kf_copy_blocks: 1 .. 65535 blocks, sizes / strides / offset multiples of 16 bytes");
     RET(r);
 }
+int kf_prompt_ends(kf_ctx* c, const kf_bf16* x, int dim, const int32_t* d_ends, int n, kf_bf16* y, int32_t* d_states) {
+    CHKCTX(c);
+    if (!x || !d_ends || !y || !d_states || dim < 1 || n < 1) return fail(KF_INVALID_ARGS, "kf_prompt_ends: null pointer, dim or n < 1");
+    if (!al16(d_ends)) return fail(KF_BLAS_UNALIGN, "kf_prompt_ends: the table must be 16-byte aligned");
+    RET(kf::prompt_ends_launch(c->stream, x, dim, d_ends, n, y, d_states));
+}
 int kf_memset2d(kf_ctx* c, void* p, size_t pitch, int value, size_t width, size_t rows) {
     CHKCTX(c);
     if (!p || width > pitch) return fail(KF_INVALID_ARGS, "kf_memset2d: null pointer or width > pitch");

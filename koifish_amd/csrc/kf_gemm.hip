@@ -627,7 +627,8 @@ int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long
         const int rc3 = gemm3_launch(st, g.fmt, a, ws, ws_bytes);
         if (rc3 != 1) return rc3;
     }
-    if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max) {
+    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide (us, staged | direct: 151936 x 1024 bf16 at 16 rows 157 | 122, at 32 160 | 137; 4-bit 80 | 56, 78 | 66)
+    if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max || n <= 32) {
         KS = 0;
         grid = dim3((M + 31) / 32, (n + 31) / 32);
     } else {

@@ -475,7 +475,8 @@ int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int*
         if (n_w != 3 || M[0] % 128 != 0 || M[1] % 128 != 0 || ((reinterpret_cast<uintptr_t>(y[0]) | reinterpret_cast<uintptr_t>(y[1]) | reinterpret_cast<uintptr_t>(rope->wq) | reinterpret_cast<uintptr_t>(rope->wk) | reinterpret_cast<uintptr_t>(rope->table)) & 15)) return 1;
         a.qkrope = 1, a.qk_norm[0] = rope->wq, a.qk_norm[1] = rope->wk, a.rope_table = rope->table, a.rope_pos0 = rope->pos0, a.rope_seq = rope->seq_len, a.qk_eps = rope->eps;
     }
-    if (rope) return n128 <= 256 ? g3_whole<G3Duo>(st, a) : g3_tiles_of(tot, n, 128, 256) <= 256 ? g3_whole<G3Half>(st, a) : g3_whole<G3Small>(st, a);
+    // us, 16 + 8 + 8 heads x 128, K 1024, at 2608 rows: 128 x 128 on 4 waves (672 tiles) 36.7, 128 x 384 (224) 32.4
+    if (rope) return n128 <= 256 ? g3_whole<G3Duo>(st, a) : g3_tiles_of(tot, n, 128, 256) <= 256 ? g3_whole<G3Half>(st, a) : g3_tiles_of(tot, n, 128, 384) <= 256 ? g3_whole<G3Long>(st, a) : g3_whole<G3Small>(st, a);
     return g3_picked(st, a, false); /* a tile's rows are one matrix's: no 192-row ones */
 }
 

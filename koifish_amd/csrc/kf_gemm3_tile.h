@@ -21,6 +21,7 @@ struct G3Cfg {
 using G3Big = G3Cfg<256, 256, 8>;      /* 128 KiB of LDS: one workgroup per CU */
 using G3Wide = G3Cfg<192, 256, 8>;
 using G3Half = G3Cfg<128, 256, 8, 3>;  /* 144 KiB */
+using G3Long = G3Cfg<128, 384, 8>;     /* 128 KiB: as many outputs as 192 x 256, where a tile is a head */
 using G3Duo = G3Cfg<128, 128, 8, 3>;   /* 96 KiB */
 using G3Small = G3Cfg<128, 128, 4>;    /* 64 KiB: two workgroups per CU; the split-K tile of the k-major products */
 using G3Few = G3Cfg<64, 64, 4, 3>;     /* 48 KiB: three */

@@ -218,6 +218,7 @@ int attn_backward_mfma_launch(hipStream_t st, const uint16_t* q, const uint16_t*
 // embedding backward (kf_embed_bwd.hip)
 int argmax_rows_state_launch(hipStream_t st, const uint16_t* logits, long long ld, int n, int n_rows, const int* d_seq, int32_t* states, int32_t* tokens_out, int tokens_stride);
 int copy_blocks_launch(hipStream_t st, void* const* dst_table, size_t dst_offset, const void* src, size_t src_stride, size_t block_bytes, int n_blocks);
+int prompt_ends_launch(hipStream_t st, const uint16_t* x, int dim, const int32_t* ends, int n, uint16_t* y, int32_t* states);
 int embed_pos_launch(hipStream_t st, const uint16_t* wte, long long ldw, const uint16_t* wpe, const int* tokens, int B, int T, int C, int V, uint16_t* out);
 int embed_backward_launch(hipStream_t st, uint16_t* dwte, long long ldw, uint16_t* dwpe, const uint16_t* dout, const int* tokens, int B, int T, int C, int V);
 // fused classifier (kf_loss.hip): cross-entropy loss per row + logit gradient in place

@@ -830,10 +830,24 @@ __global__ void __launch_bounds__(1024) argmax_rows_state_kernel(const uint16_t*
     const uint16_t* row = logits + (size_t)blockIdx.x * ld;
     float best = -__builtin_inff();
     int bi = 0x7fffffff;
-    for (int i = threadIdx.x; i < n; i += 1024) { /* ascending i per thread: a strict > keeps the thread's first maximum */
-        const float v = bf2f(row[i]);
+    auto take = [&](float v, int i) { /* ascending i per thread: a strict > keeps the thread's first maximum */
         if (v > best || bi == 0x7fffffff) best = v, bi = i;
+    };
+    // few workgroups, each a serial walk: eight 16-byte loads per thread at a time (16 rows of 151936: one 2-byte load at a time 50 us, so 8)
+    const int n8 = (ld & 7) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0 ? n / 8 : 0;
+    for (int c0 = threadIdx.x; c0 < n8; c0 += 8192) {
+        u32x4 w[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (c0 + 1024 * u < n8) w[u] = *reinterpret_cast<const u32x4*>(row + 8 * (size_t)(c0 + 1024 * u));
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (c0 + 1024 * u < n8) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) take(bf_lo(w[u][e]), 8 * (c0 + 1024 * u) + 2 * e), take(bf_hi(w[u][e]), 8 * (c0 + 1024 * u) + 2 * e + 1);
+            }
     }
+    for (int i = 8 * n8 + threadIdx.x; i < n; i += 1024) take(bf2f(row[i]), i);
     auto better = [](float v, int i, float bv, int bi2) { return v > bv || (v == bv && i < bi2); };
     for (int m = 32; m > 0; m >>= 1) {
         const float ov = __shfl_xor(best, m, 64);
@@ -871,6 +885,23 @@ int copy_blocks_launch(hipStream_t st, void* const* dst_table, size_t dst_offset
     if (!block_bytes) return KF_OK;
     hipLaunchKernelGGL(copy_blocks_kernel, dim3((unsigned)((block_bytes / 16 + 255) / 256), n_blocks), dim3(256), 0, st, dst_table, dst_offset, (const unsigned char*)src, src_stride,
                        block_bytes);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+// the ends of a batch of prompts, one launch: row ends[i].x of x (dim columns) -> row i of y, and the decode state of sequence ends[i].y = {ends[i].z, ends[i].w, as it was, 0}
+__global__ void __launch_bounds__(256) prompt_ends_kernel(const uint16_t* __restrict__ x, int dim, const i32x4_t* __restrict__ ends, uint16_t* __restrict__ y, int32_t* __restrict__ states) {
+    const i32x4_t e = ends[blockIdx.x];
+    const uint16_t* const from = x + (size_t)e[0] * dim;
+    uint16_t* const to = y + (size_t)blockIdx.x * dim;
+    for (int i = threadIdx.x; i < dim; i += 256) to[i] = from[i];
+    if (threadIdx.x == 0) {
+        int32_t* const st = states + 4 * (size_t)e[1];
+        st[0] = e[2], st[1] = e[3], st[3] = 0;
+    }
+}
+int prompt_ends_launch(hipStream_t st, const uint16_t* x, int dim, const int32_t* ends, int n, uint16_t* y, int32_t* states) {
+    hipLaunchKernelGGL(prompt_ends_kernel, dim3(n), dim3(256), 0, st, x, dim, reinterpret_cast<const i32x4_t*>(ends), y, states);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 

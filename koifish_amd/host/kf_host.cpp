@@ -1160,28 +1160,33 @@ int XcdReplicas::PrefillBatch(const int* slots, const int32_t* tokens, const int
     if (T >= c.n_ctx || R > f->prefill_chunk) return KF_INVALID_ARGS;
     KF_TRY(Fresh());
     KF_TRY(f->PrefillReady(R));
-    if (!bK || bK->ne[1] < R) {
+    const size_t table = (size_t)3 * n_seq * sizeof(void*), table_bytes = ((table + 15) & ~(size_t)15) + (size_t)n_seq * 20; /* three tables of destinations (K, V, logits), the ends, the slots */
+    if (!bKV || bKV->ne[1] < 2 * R) {
         KF_TRY(kf_sync(ctx));
         const int rows = f->gBUFF.rows;
-        bK = GT(ctx, "xr.bK", typNUMBER::BF16, kvd, rows), bV = GT(ctx, "xr.bV", typNUMBER::BF16, kvd, rows);
-        if (!bK || !bV) return KF_OUTOF_GPUMEMORY;
-        if (!d_dst) KF_TRY(kf_malloc(ctx, (size_t)3 * n_seq * sizeof(void*) + (size_t)n_seq * 4, (void**)&d_dst)); /* three tables of destinations (K, V, logits) + the slots */
+        bKV = GT(ctx, "xr.bKV", typNUMBER::BF16, kvd, 2 * rows);
+        if (!bKV) return KF_OUTOF_GPUMEMORY;
+        if (!d_dst) KF_TRY(kf_malloc(ctx, table_bytes, (void**)&d_dst));
         if (!bL) bL = GT(ctx, "xr.bL", typNUMBER::BF16, c.vocab, n_seq);
-        if (!bL) return KF_OUTOF_GPUMEMORY;
+        if (!bE) bE = GT(ctx, "xr.bE", typNUMBER::BF16, C, n_seq);
+        if (!bL || !bE) return KF_OUTOF_GPUMEMORY;
     }
     std::vector<int32_t> rows((size_t)R, 0);
-    std::vector<void*> dst((size_t)3 * n_seq + (n_seq + 1) / 2, nullptr); /* the slots ride behind the pointer tables as int32 */
-    int32_t* h_slots = reinterpret_cast<int32_t*>(dst.data() + (size_t)3 * n_seq);
+    std::vector<unsigned char> upload(table_bytes, 0);
+    void** const dst = reinterpret_cast<void**>(upload.data());
+    int32_t* const h_ends = reinterpret_cast<int32_t*>(upload.data() + table_bytes - (size_t)n_seq * 20);
+    int32_t* const h_slots = h_ends + 4 * n_seq;
     for (int i = 0; i < S; i++) {
         memcpy(rows.data() + (size_t)i * T, tokens + (size_t)i * stride, (size_t)lens[i] * 4);
-        dst[i] = ToX(key) + (size_t)slots[i] * kv_seq_elems(), dst[n_seq + i] = ToX(val) + (size_t)slots[i] * kv_seq_elems();
+        dst[i] = ToX(key) + (size_t)slots[i] * kv_seq_elems(), dst[S + i] = ToX(val) + (size_t)slots[i] * kv_seq_elems();
         dst[2 * n_seq + i] = ToX(logits) + (size_t)slots[i] * c.vocab;
+        h_ends[4 * i] = i * T + lens[i] - 1, h_ends[4 * i + 1] = slots[i], h_ends[4 * i + 2] = tokens[(size_t)i * stride + lens[i] - 1], h_ends[4 * i + 3] = lens[i] - 1;
         h_slots[i] = slots[i];
     }
-    const int32_t* d_slots = reinterpret_cast<const int32_t*>(d_dst + (size_t)3 * n_seq);
+    const int32_t *d_ends = reinterpret_cast<const int32_t*>(reinterpret_cast<const unsigned char*>(d_dst) + table_bytes - (size_t)n_seq * 20), *d_slots = d_ends + 4 * n_seq;
     KF_TRY(kf_h2d(ctx, f->gBUFF.d_ptok, rows.data(), (size_t)R * 4));
-    KF_TRY(kf_h2d(ctx, d_dst, dst.data(), (size_t)3 * n_seq * sizeof(void*) + (size_t)n_seq * 4));
-    floatX *bx = ToX(f->gBUFF.bX), *bn = ToX(f->gBUFF.bNorm), *bq = ToX(f->gBUFF.bQ), *ba = ToX(f->gBUFF.bAttn), *bk = ToX(bK), *bv = ToX(bV);
+    KF_TRY(kf_h2d(ctx, d_dst, upload.data(), table_bytes));
+    floatX *bx = ToX(f->gBUFF.bX), *bn = ToX(f->gBUFF.bNorm), *bq = ToX(f->gBUFF.bQ), *ba = ToX(f->gBUFF.bAttn), *bk = ToX(bKV), *bv = bk + (size_t)R * kvd;
     kf_weight we = f->embed.w->desc();
     KF_TRY(kf_embed_batch(ctx, &we, f->gBUFF.d_ptok, R, bx));
     for (int l = 0; l < c.nLayer; l++) {
@@ -1194,8 +1199,7 @@ int XcdReplicas::PrefillBatch(const int* slots, const int32_t* tokens, const int
                                 c.n_head_kv, c.head_dim, a.normQ.rms_eps)); /* positions restart with every prompt */
         KF_TRY(kf_attn_prefill_batch(ctx, bq, bk, bv, ba, T, qd, c.n_head, c.n_head_kv, c.head_dim, kvd, S)); /* the rows of a prompt see that prompt's keys only */
         const size_t off = (size_t)l * c.n_ctx * kvd * 2, blk = (size_t)T * kvd * 2;
-        KF_TRY(kf_copy_blocks(ctx, d_dst, off, bk, blk, blk, S));
-        KF_TRY(kf_copy_blocks(ctx, d_dst + n_seq, off, bv, blk, blk, S));
+        KF_TRY(kf_copy_blocks(ctx, d_dst, off, bk, blk, blk, 2 * S)); /* the V blocks lie behind the K blocks, and so do their destinations */
         KF_TRY(kf_linear(ctx, &wo, ba, bx, nullptr, R, 1.0f, 0.0f, KF_EPI_RESIDUAL, bx));
         KF_TRY(f->ffn[l]->cuFlow(bx, R));
     }
@@ -1203,17 +1207,12 @@ int XcdReplicas::PrefillBatch(const int* slots, const int32_t* tokens, const int
     // (the head matrix -- 311 MB on Qwen3-0.6B -- is read ONCE for all prompts: the last rows normed side by side, one product, one pick launch, one scatter of the logits)
     kf_weight wh = f->head.proj.w->desc();
     const bool together = S > 1 && c.vocab % 8 == 0;
-    for (int i = 0; i < S; i++) {
-        const int s = slots[i], n = lens[i];
-        KF_TRY(kf_set_state(ctx, d_state + 4 * s, tokens[(size_t)i * stride + n - 1], n - 1));
-        KF_TRY(kf_memset(ctx, d_state + 4 * s + 3, 0, 4));
-        if (together)
-            KF_TRY(kf_rmsnorm(ctx, bx + ((size_t)i * T + n - 1) * C, ToX(f->final_norm.w), bn + (size_t)i * C, 1, C, f->final_norm.rms_eps, nullptr));
-        else
-            KF_TRY(kf_norm_lm_head(ctx, bx + ((size_t)i * T + n - 1) * C, ToX(f->final_norm.w), f->final_norm.rms_eps, &wh, ToX(logits) + (size_t)s * c.vocab, d_state + 4 * s,
-                                   d_tokens_out + (size_t)s * c.n_ctx, f->gBUFF.head_ws->data));
-    }
+    KF_TRY(kf_prompt_ends(ctx, bx, C, d_ends, S, ToX(bE), d_state));
+    for (int i = 0; i < S && !together; i++)
+        KF_TRY(kf_norm_lm_head(ctx, ToX(bE) + (size_t)i * C, ToX(f->final_norm.w), f->final_norm.rms_eps, &wh, ToX(logits) + (size_t)slots[i] * c.vocab, d_state + 4 * slots[i],
+                               d_tokens_out + (size_t)slots[i] * c.n_ctx, f->gBUFF.head_ws->data));
     if (together) {
+        KF_TRY(kf_rmsnorm(ctx, ToX(bE), ToX(f->final_norm.w), bn, S, C, f->final_norm.rms_eps, nullptr));
         KF_TRY(kf_linear(ctx, &wh, bn, ToX(bL), nullptr, S, 1.0f, 0.0f, 0u, nullptr));
         KF_TRY(kf_argmax_rows_state(ctx, ToX(bL), c.vocab, c.vocab, S, d_slots, d_state, d_tokens_out, c.n_ctx));
         KF_TRY(kf_copy_blocks(ctx, d_dst + 2 * n_seq, 0, ToX(bL), (size_t)c.vocab * 2, (size_t)c.vocab * 2, S));

@@ -401,3 +401,30 @@ def test_argmax_rows_state_copy_blocks_memset32(ctx, O):
     assert hip.kf_memset32(ctx.h, w.data_ptr() + 8, -7, 5) == 0, hip.kf_last_error()
     ctx.sync()
     assert w.cpu().numpy().tolist() == [0, 0, -7, -7, -7, -7, -7, 0, 0, 0]
+
+
+@pytest.mark.parametrize("n,ld", [(1, 8), (7, 7), (8, 8), (1003, 1008), (8192, 8192), (70001, 70008), (151936, 151936)])
+def test_argmax_rows_by_wide_loads_and_the_ends_of_prompts(ctx, n, ld):
+    """the first maximum of a row wherever it stands, rows that 16-byte loads divide and others; kf_prompt_ends: rows gathered, the state's parked word left alone"""
+    rows, dev = 5, ctx.device
+    g = torch.Generator().manual_seed(n)
+    lg = torch.randn(rows, ld, generator=g).bfloat16()
+    lg[:, n:] = 100.0   # behind the row's end: not looked at
+    at = [0, n - 1, n // 2, min(n - 1, 8191), min(n - 1, 65536)]
+    for i, a in enumerate(at):
+        lg[i, a] = 50.0
+        lg[i, min(n - 1, a + 3)] = 50.0   # a tie further on
+    x = torch.randn(40, 72, generator=g).bfloat16().to(dev)
+    ends = torch.tensor([[39 - 7 * i, (3 * i) % rows, 11 + i, 20 + i] for i in range(rows)], dtype=torch.int32, device=dev)
+    st = torch.full((rows, 4), 9, dtype=torch.int32, device=dev)
+    y = torch.zeros(rows, 72, dtype=torch.bfloat16, device=dev)
+    assert ctx.hip.kf_prompt_ends(ctx.h, x.data_ptr(), 72, ends.data_ptr(), rows, y.data_ptr(), st.data_ptr()) == 0
+    seq, d = ends[:, 1].contiguous(), lg.to(dev)
+    out = torch.zeros(rows, 64, dtype=torch.int32, device=dev)
+    ctx.sync()
+    assert torch.equal(y, x[ends[:, 0].long()])
+    assert st[seq.long()].tolist() == [[11 + i, 20 + i, 9, 0] for i in range(rows)]
+    assert ctx.hip.kf_argmax_rows_state(ctx.h, d.data_ptr(), ld, n, rows, seq.data_ptr(), st.data_ptr(), out.data_ptr(), 64) == 0
+    ctx.sync()
+    assert st[seq.long()].tolist() == [[at[i], 21 + i, 9, 0] for i in range(rows)]
+    assert [int(out[int(seq[i]), 20 + i]) for i in range(rows)] == at
