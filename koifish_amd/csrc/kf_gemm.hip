@@ -178,6 +178,13 @@ struct WTile<FMT_Q1, KS> {
     }
 };
 
+// one loaded register of a tile
+__device__ __forceinline__ uint32_t gm_first(const u32x4& v) { return v.x; }
+__device__ __forceinline__ uint32_t gm_first(const u32x2& v) { return v.x; }
+template <int N>
+__device__ __forceinline__ uint32_t gm_first(const u32x4 (&v)[N]) { return v[0].x; }
+template <int N, int M>
+__device__ __forceinline__ uint32_t gm_first(const u32x4 (&v)[N][M]) { return v[0][0].x; }
 template <int FMT, int KS>
 __device__ __forceinline__ u32x4 get_frag(const WTile<FMT, KS>& t, int sl, const GemmArgs& a, int ks) {
     if constexpr (FMT == FMT_Q2 || FMT == FMT_Q1)
@@ -314,15 +321,15 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmArgs a) {
 
 // ---- small token counts: every wave is independent.  Workgroup = one block of 32 output rows x TB*32 tokens; its NW waves split k in
 // groups of UPG consecutive 64-element units (for 2-bit / 1-bit: halves of a 128-element unit): wave w takes groups w, w + NW, ...,
-// reads its x fragments straight from global memory (x is n*K*2 bytes: L2-resident) and meets the others once, at the end, where
+// reads its x fragments straight from global memory (x is n*K*2 bytes: L2-resident) or by way of its own LDS (XL) and meets the others once, at the end, where
 // wave 0 adds the sums in wave order.  All loads of a group are issued before any of its arithmetic and the next group's loads before
 // the current group's arithmetic: the prompt-sized GEMMs of a 0.6B model are latency-bound (a 1024 x 1024 4-bit matrix is 0.5 MB,
 // far fewer waves than SIMDs), so the k loop is kept as short as the register file allows (K = 1024: one group per wave, no loop).
 // PAIRED: the workgroup multiplies the same x fragments against TWO matrices (gate, up) and stores silu(gate) * up: the bf16 stores of
 // gate and up and the SwiGLU expression are the ones of the separate launches (kf_linear x 2 + kf_swiglu), so the result is bit-identical.
 // Otherwise a launch may carry up to three matrices that share x (Q, K, V): blockIdx.x walks their 32-row blocks one job after the other.
-template <int FMT, int TB, int UPG, int NW, bool PAIRED>
-__global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0) {
+template <int FMT, int TB, int UPG, int NW, bool PAIRED, bool XL>
+__global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0, int slots) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     float* red = reinterpret_cast<float*>(smem_raw); /* [PAIRED ? 2 : 1][NW][TB][16][64] */
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -368,9 +375,28 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0)
     struct Group {
         WTile<FMT, 2> w[UPG];
         WTile<FMT, 2> w2[PAIRED ? UPG : 1];
-        u32x4 x[UPG][4][TB];
+        u32x4 x[XL ? 1 : UPG][4][TB];
     };
-    auto gload = [&](int u0, Group& g) { /* units u0 .. u0+UPG-1; units past the end repeat the last one and are skipped in the arithmetic */
+    // XL: a group's 128 columns of the token rows, [tokens][256 bytes] in LDS, 16-byte chunk c of row r at c ^ (r & 15); this wave's own, so no barrier: its loads set out in front of the group's weights, and loads
+    // return in order
+    static_assert(!XL || UPG == 2, "a group is 128 columns");
+    constexpr int XG = TB * 32 * 256;
+    unsigned char* const xs = smem_raw + __builtin_amdgcn_readfirstlane(wave) * slots * XG;
+    [[maybe_unused]] const uint32_t ldb = (uint32_t)a.ldx * 2;
+    auto xload = [&](int u0, int slot) {
+#ifdef __HIP_DEVICE_COMPILE__
+        const long long left = ((long long)a.n - tok0) * ldb - (long long)u0 * 128;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x) + (size_t)tok0 * a.ldx + (size_t)u0 * 64, 0, (int)(left < 0x7FFFFFFFll ? left : 0x7FFFFFFFll), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < TB * 8; i++) {
+            const int row = 4 * i + (lane >> 4);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(xs + slot * XG + i * 1024), 16, (uint32_t)row * ldb + (((lane & 15) ^ (row & 15)) << 4), 0, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+#endif
+    };
+    auto gload = [&](int u0, Group& g, int slot) { /* units u0 .. u0+UPG-1; units past the end repeat the last one and are skipped in the arithmetic */
+        if constexpr (XL) xload(u0, slot);
 #pragma unroll
         for (int j = 0; j < UPG; j++) {
             int u = u0 + j;
@@ -378,40 +404,54 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0)
             const int it = u >> 1, ks = u & 1;
             g.w[j].load(a, row, it, h, ks);
             if (PAIRED) g.w2[j].load(b, row, it, h, ks);
+            if constexpr (!XL) {
 #pragma unroll
-            for (int sl = 0; sl < 4; sl++) {
-                const int ko = it * GM_KT + WTile<FMT, 2>::koff(sl, h, ks);
+                for (int sl = 0; sl < 4; sl++) {
+                    const int ko = it * GM_KT + WTile<FMT, 2>::koff(sl, h, ks);
 #pragma unroll
-                for (int tb = 0; tb < TB; tb++) g.x[j][sl][tb] = *reinterpret_cast<const u32x4*>(xrow[tb] + ko);
+                    for (int tb = 0; tb < TB; tb++) g.x[j][sl][tb] = *reinterpret_cast<const u32x4*>(xrow[tb] + ko);
+                }
             }
         }
     };
+    auto xfrag = [&](const Group& g, int slot, int j, int sl, int tb) {
+        if constexpr (XL) return *reinterpret_cast<const u32x4*>(xs + slot * XG + (tb * 32 + r) * 256 + (((WTile<FMT, 2>::koff(sl, h, j) >> 3) ^ (r & 15)) << 4));
+        else return g.x[j][sl][tb];
+    };
     Group gc, gn;
-    int u0 = wave * UPG;
-    if (u0 < nunit) gload(u0, gc);
+    int u0 = wave * UPG, slot = 0;
+    if (u0 < nunit) gload(u0, gc, 0);
     for (; u0 < nunit; u0 += NW * UPG) {
         const bool more = u0 + NW * UPG < nunit;
-        if (more) gload(u0 + NW * UPG, gn);
+        if (more) gload(u0 + NW * UPG, gn, slot ^ 1);
+        if constexpr (XL) { /* a weight of the group has come: its token rows have */
+            asm volatile("" ::"v"(gm_first(gc.w[0].b)) : "memory");
+        }
 #pragma unroll
         for (int j = 0; j < UPG; j++) {
             if (u0 + j < nunit) {
 #pragma unroll
                 for (int sl = 0; sl < 4; sl++) {
                     const bf16x8 A = __builtin_bit_cast(bf16x8, get_frag<FMT, 2>(gc.w[j], sl, a, (u0 + j) & 1));
+                    u32x4 X[TB];
+#pragma unroll
+                    for (int tb = 0; tb < TB; tb++) X[tb] = xfrag(gc, slot, j, sl, tb);
 #pragma unroll
                     for (int tb = 0; tb < TB; tb++)
-                        acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(bf16x8, gc.x[j][sl][tb]), acc[tb], 0, 0, 0);
+                        acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(bf16x8, X[tb]), acc[tb], 0, 0, 0);
                     if (PAIRED) {
                         const bf16x8 A2 = __builtin_bit_cast(bf16x8, get_frag<FMT, 2>(gc.w2[j], sl, b, (u0 + j) & 1));
 #pragma unroll
                         for (int tb = 0; tb < TB; tb++)
-                            acc2[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A2, __builtin_bit_cast(bf16x8, gc.x[j][sl][tb]), acc2[tb], 0, 0, 0);
+                            acc2[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A2, __builtin_bit_cast(bf16x8, X[tb]), acc2[tb], 0, 0, 0);
                     }
                 }
             }
         }
         if (more) gc = gn;
+        slot ^= 1;
     }
+    if constexpr (XL) __syncthreads(); /* the sums go where the token rows were */
     // fixed-order sum over the k-slices, ((w0 + w1) + w2) + ..., and the epilogue, spread over the waves: every wave leaves its 16 sums per token block in LDS and
     // wave w adds and stores accumulator registers 16 w / NW .. (two adjacent output rows per lane with 8 waves) -- the same additions in the same order as one wave
     // doing all of it, at an eighth of the serial work behind the barrier (measured on the 0.6B shapes at 128 tokens: reduce 0.65 us + epilogue 1.3-1.7 us by wave 0)
@@ -486,14 +526,27 @@ static int gm_fmt_of(int type) {
 
 constexpr int GD_NW = 8, GD_UPG = 2; /* direct kernel: 8 waves, groups of two 64-element units, 32-token tiles */
 
+// Token rows by way of LDS, whole lines, from 17 rows (bf16: always): read as fragments a wave's load touches 64 pieces of 16 bytes.  us at 128 rows, fragments | LDS: 4-bit 1024 x 2048 9.6 | 8.5, 1024 x 3072 12.5 | 11.2,
+// 4096 x 1024 8.6 | 7.5, 2048 x 6144 24.6 | 20.6, gate and up 3072 x 1024 13.8 | 11.6; at 16 rows, where the padding repeats one row's lines, 8.1 | 8.3, 11.2 | 10.9, 5.2 | 5.5 (at 8: 7.7 | 8.4, 10.3 | 10.9, 5.0 | 6.0); bf16
+// 151936 x 1024 at 8 rows 115 | 94, at 32 137 | 108.  Same sums in the same order.
+template <int FMT, int TB, bool PAIRED>
+static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
+    const size_t sums = (size_t)GD_NW * (PAIRED ? 2 : 1) * TB * 16 * 64 * 4;
+    const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1; /* one group of a wave, or two in turn */
+    const size_t rows = (size_t)GD_NW * slots * TB * 32 * 256;
+    if ((a.n > 16 || FMT == FMT_BF16) && rows <= 128 * 1024 && a.ldx < (1 << 24)) {
+        static int attr_set = 0;
+        if (!attr_set) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024), attr_set = 1;
+        hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), grid, dim3(GD_NW * 64), rows > sums ? rows : sums, st, a, slots);
+        return;
+    }
+    hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, false>), grid, dim3(GD_NW * 64), sums, st, a, 0);
+}
 template <int FMT>
 static void gm_launch(const GemmArgs& a, int KS, dim3 grid, size_t smem, hipStream_t st) {
-    if (KS == 0)
-        hipLaunchKernelGGL((gemm_direct_kernel<FMT, 1, GD_UPG, GD_NW, false>), grid, dim3(GD_NW * 64), (size_t)GD_NW * 16 * 64 * 4, st, a);
-    else if (KS == -2) /* 64-token tiles: every weight block is unpacked for two token blocks */
-        hipLaunchKernelGGL((gemm_direct_kernel<FMT, 2, GD_UPG, GD_NW, false>), grid, dim3(GD_NW * 64), (size_t)GD_NW * 2 * 16 * 64 * 4, st, a);
-    else if (KS == -1) /* paired SwiGLU */
-        hipLaunchKernelGGL((gemm_direct_kernel<FMT, 1, GD_UPG, GD_NW, true>), grid, dim3(GD_NW * 64), (size_t)GD_NW * 2 * 16 * 64 * 4, st, a);
+    if (KS == 0) gm_direct<FMT, 1, false>(a, grid, st);
+    else if (KS == -2) gm_direct<FMT, 2, false>(a, grid, st); /* 64-token tiles: every weight block is unpacked for two token blocks */
+    else if (KS == -1) gm_direct<FMT, 1, true>(a, grid, st); /* paired SwiGLU */
     else if (KS == 2)
         hipLaunchKernelGGL((gemm_kernel<FMT, 2>), grid, dim3(256), smem, st, a);
     else
@@ -627,7 +680,7 @@ int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long
         const int rc3 = gemm3_launch(st, g.fmt, a, ws, ws_bytes);
         if (rc3 != 1) return rc3;
     }
-    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide (us, staged | direct: 151936 x 1024 bf16 at 16 rows 157 | 122, at 32 160 | 137; 4-bit 80 | 56, 78 | 66)
+    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide (us, staged | direct: 151936 x 1024 bf16 at 16 rows 157 | 100, at 32 160 | 108; 4-bit 80 | 50, 78 | 56)
     if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max || n <= 32) {
         KS = 0;
         grid = dim3((M + 31) / 32, (n + 31) / 32);
