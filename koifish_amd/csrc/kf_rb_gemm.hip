@@ -8,12 +8,8 @@
 
 namespace kf {
 
-using RbBig = G3Cfg<256, 256, 8>;
-using RbWide = G3Cfg<192, 256, 8>;
-using RbSmall = G3Cfg<128, 128, 4>;
-using RbMid = G3Cfg<64, 128, 4>;
-using RbTiny = G3Cfg<64, 64, 4>;
-using RbPairs = G3Cfg<128, 64, 4>; /* experts of about a hundred pairs: half the padding of 128-pair tiles, each weight tile read about once */
+using RbTiny = G3Cfg<64, 64, 4>;      /* 32-bit storage: five to a CU */
+using RbPairs = G3Cfg<128, 64, 4>;    /* experts of about a hundred pairs: half the padding of 128-pair tiles, each weight tile read about once; three to a CU (with three buffers, two: 64 experts of 3072 x 2048, 7884 pairs 259 -> 268 us) */
 
 // eight values from a multiple of 8 columns; rows of 16-bit values are at least 8-byte aligned
 __device__ __forceinline__ void rb_st8(uint16_t* p, const float (&v)[8], int64_t ld) {
@@ -63,16 +59,20 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     T* const y = reinterpret_cast<T*>(p.y);
     auto row_of = [&](int tk) { return EXPERTS ? s_dst[EXPERTS ? tk : 0] : (t0 + tk < p.n ? t0 + tk : -1); };
     if (p.epilogue == KF_RB_GATED) {
-        Out::template all<C::BM / 16>(acc, smem_raw, tid, [&](int tk, int lt, int u) { /* rows of 16 gates and of the 16 ups behind them: eight outputs */
-            const int row = row_of(tk), f = (m0 >> 1) + 8 * u, c = (u >> 1) * 4 + (u & 1);
-            if (row < 0 || 2 * f >= p.m) return;
-            const float scale = EXPERTS && p.mode == KF_RB_UP ? q.e.weight[row] : 1.f;
-            float g[8], v[8];
-            Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, v);
+        auto gated = [&](auto act) { /* a loop per activation: decided inside it costs a branch per value */
+            Out::template all<C::BM / 16>(acc, smem_raw, tid, [&](int tk, int lt, int u) { /* rows of 16 gates and of the 16 ups behind them: eight outputs */
+                const int row = row_of(tk), f = (m0 >> 1) + 8 * u, c = (u >> 1) * 4 + (u & 1);
+                if (row < 0 || 2 * f >= p.m) return;
+                const float scale = EXPERTS && p.mode == KF_RB_UP ? q.e.weight[row] : 1.f;
+                float g[8], v[8];
+                Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, v);
 #pragma unroll
-            for (int j = 0; j < 8; j++) g[j] = scale * (rb_activate(p.act, g[j]) * v[j]);
-            rb_st8(y + (size_t)row * p.ldy + f, g, p.ldy);
-        });
+                for (int j = 0; j < 8; j++) g[j] = scale * (rb_activate(act, g[j]) * v[j]);
+                rb_st8(y + (size_t)row * p.ldy + f, g, p.ldy);
+            });
+        };
+        if (p.act == KF_RB_SILU) gated(std::integral_constant<int, KF_RB_SILU>());
+        else gated(p.act);
     } else if (p.epilogue == KF_RB_STORE && U == 1) {
         Out::template all<C::BM / 8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
             const int row = row_of(tk), m = m0 + 8 * u;
@@ -122,16 +122,20 @@ static long rb_tiles(const kf_rb_product& p, int bm, int bn) { return (long)((p.
 int rb_gemm_launch(hipStream_t st, const RbProduct& q) {
     const kf_rb_product& p = q.p;
     if (p.mode != KF_RB_ALL) {
-        if (q.e.tile == 128) return rb_go<RbSmall, true>(st, q, (long)((p.m + 127) / 128) * q.e.n_tile);
+        if (q.e.tile == 128) return rb_go<G3Small, true>(st, q, (long)((p.m + 127) / 128) * q.e.n_tile);
         if (q.e.tile == 64) return rb_go<RbPairs, true>(st, q, (long)((p.m + 127) / 128) * q.e.n_tile);
         return 1;
     }
-    // the measured thresholds of gemm3_launch: big tiles from 160 of them, then smaller ones that fill the chip
-    if (p.m >= 256 && p.n >= 256 && rb_tiles(p, 256, 256) >= 160)
-        return g3_prefer_wide(p.m, p.n, p.k) ? rb_go<RbWide, false>(st, q, rb_tiles(p, 192, 256)) : rb_go<RbBig, false>(st, q, rb_tiles(p, 256, 256));
-    if (rb_tiles(p, 128, 128) >= 256) return rb_go<RbSmall, false>(st, q, rb_tiles(p, 128, 128));
-    if (rb_tiles(p, 64, 128) >= 192) return rb_go<RbMid, false>(st, q, rb_tiles(p, 64, 128));
-    return rb_go<RbTiny, false>(st, q, rb_tiles(p, 64, 64));
+    // the smallest tile that makes one round of the CUs, as for the products of kf_gemm3.hip (g3_pick has the figures): same main loop
+    const long n64 = rb_tiles(p, 64, 64);
+    if (n64 <= (p.k < 96 * G3_BK ? 512 : 256)) return rb_go<G3Few, false>(st, q, n64);
+    switch (g3_pick(p.m, p.n, p.k, true)) {
+        case G3_DUO: return rb_go<G3Duo, false>(st, q, rb_tiles(p, 128, 128));
+        case G3_HALF: return rb_go<G3Half, false>(st, q, rb_tiles(p, 128, 256));
+        case G3_SMALL: return rb_go<G3Small, false>(st, q, rb_tiles(p, 128, 128));
+        case G3_WIDE: return rb_go<G3Wide, false>(st, q, rb_tiles(p, 192, 256));
+        default: return rb_go<G3Big, false>(st, q, rb_tiles(p, 256, 256));
+    }
 }
 // The 32-bit product on v_mfma_f32_16x16x4_f32 (157 TFLOP/s; the vector pipe without packed instructions: 78).  It is bound by the MFMAs, 16 x slower than bf16's, so the tile only has to share them
 // out evenly: 64 x 64 tiles, five to a CU.
