@@ -18,13 +18,6 @@
 
 namespace kf {
 
-constexpr int AP_NB = 5;
-// the place of 16-byte chunk c of row r of a tile
-template <int HD>
-__device__ __forceinline__ int ap_swz_k(int r, int c) { return HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7); }
-template <int HD>
-__device__ __forceinline__ int ap_swz_v(int r, int c) { return HD == 128 ? c ^ ((r & 3) << 2) : c ^ (((r >> 1) & 1) << 2); }
-
 struct AttnPrefillArgs {
     const uint16_t* q;
     const uint16_t* kcache;
@@ -37,29 +30,6 @@ struct AttnPrefillArgs {
     float rden;
 };
 
-// one wave of either kernel: where its K and V rows lie in a tile of 32 keys and in LDS
-template <int HD>
-struct ApTile {
-    static constexpr int RB = HD * 2, PART = 32 * RB, RPI = 1024 / RB; /* bytes of a row, of 32 rows; rows per load instruction */
-    int kf[HD / 16], vf[HD / 32]; /* a swizzle flips bits of the chunk, so one offset per MFMA step (K) and per block of d (V) */
-    __device__ __forceinline__ void init(int lane) {
-        const int r = lane & 31, h = lane >> 5;
-#pragma unroll
-        for (int s = 0; s < HD / 16; s++) kf[s] = r * RB + ap_swz_k<HD>(r, 2 * s + h) * 16;
-#pragma unroll
-        for (int db = 0; db < HD / 32; db++) { /* lane l16 of a 16-lane group addresses key-row (l16 >> 2) of its 4, d-piece 4 (l16 & 3) of the group's 16 d; it receives the 4 keys of d = l16 */
-            const int row = 4 * h + ((lane & 15) >> 2);
-            vf[db] = row * RB + ap_swz_v<HD>(row, 4 * db + ((lane & 16) >> 3) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
-        }
-    }
-    __device__ __forceinline__ u32x4 k(const unsigned char* tile, int s) const { return *reinterpret_cast<const u32x4*>(tile + kf[s]); }
-    __device__ __forceinline__ fl_bf16x8 v(const unsigned char* tile, int s2, int db) const {
-        const unsigned char* const at = tile + vf[db] + 16 * s2 * RB;
-        const fl_bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) fl_bf16x4*)(at));
-        const fl_bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) fl_bf16x4*)(at + 8 * RB));
-        return fl_bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    }
-};
 // rows of K or V from memory into LDS: N instructions per wave, from row `first` of those the workgroup loads at a time.  Rows past `left` bytes from `base` become zeros
 template <int HD, int N, bool V>
 struct ApLoad {
@@ -80,12 +50,6 @@ struct ApLoad {
 #endif
     }
 };
-template <int N>
-__device__ __forceinline__ void ap_landed() { /* all but the wave's N latest loads have landed, for every wave, and every wave has read what it wanted */
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 // this lane's column of a workgroup whose first token is `first`
 struct ApCol {
     int tok, head; /* clamped to the last token */

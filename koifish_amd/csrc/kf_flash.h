@@ -118,4 +118,49 @@ struct FlashWave {
     }
 };
 
+// ---- tiles that went global -> LDS by buffer loads: the LDS image of such a load is lane-linear, so rows are unpadded and the swizzle is made at the source: 16 lanes of a K read and 32 of a transposing V read touch
+// all 64 banks once
+constexpr int AP_NB = 5; /* buffers: up to three tiles of 16 KiB are on their way while one is multiplied, which is what a load from another XCD's memory side takes */
+// the place of 16-byte chunk c of row r of a tile
+template <int HD>
+__device__ __forceinline__ int ap_swz_k(int r, int c) { return HD == 128 ? c ^ (r & 15) : c ^ ((r >> 1) & 7); }
+template <int HD>
+__device__ __forceinline__ int ap_swz_v(int r, int c) { return HD == 128 ? c ^ ((r & 3) << 2) : c ^ (((r >> 1) & 1) << 2); }
+
+// where a wave's K and V rows lie in a tile of 32 keys (K, then V, each row-major) in LDS
+template <int HD>
+struct ApTile {
+    static constexpr int RB = HD * 2, PART = 32 * RB, RPI = 1024 / RB; /* bytes of a row, of 32 rows; rows per load instruction */
+    int kf[HD / 16], vf[HD / 32]; /* a swizzle flips bits of the chunk, so one offset per MFMA step (K) and per block of d (V) */
+    __device__ __forceinline__ void init(int lane) {
+        const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+        for (int s = 0; s < HD / 16; s++) kf[s] = r * RB + ap_swz_k<HD>(r, 2 * s + h) * 16;
+#pragma unroll
+        for (int db = 0; db < HD / 32; db++) { /* lane l16 of a 16-lane group addresses key-row (l16 >> 2) of its 4, d-piece 4 (l16 & 3) of the group's 16 d; it receives the 4 keys of d = l16 */
+            const int row = 4 * h + ((lane & 15) >> 2);
+            vf[db] = row * RB + ap_swz_v<HD>(row, 4 * db + ((lane & 16) >> 3) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
+        }
+    }
+    __device__ __forceinline__ u32x4 k(const unsigned char* tile, int s) const { return *reinterpret_cast<const u32x4*>(tile + kf[s]); }
+    __device__ __forceinline__ fl_bf16x8 v(const unsigned char* tile, int s2, int db) const {
+        const unsigned char* const at = tile + vf[db] + 16 * s2 * RB;
+        const fl_bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) fl_bf16x4*)(at));
+        const fl_bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) fl_bf16x4*)(at + 8 * RB));
+        return fl_bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+};
+template <int N>
+__device__ __forceinline__ void ap_landed() { /* all but the wave's N latest loads have landed, for every wave, and every wave has read what it wanted */
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// f while loads set out for to_k, to_v.  The pointers are told apart (restrict): the compiler otherwise takes every transposing LDS read for one that may read what those loads write, and puts a wait for all of them
+// in front of it -- a tile then takes what a load takes.  What has to have landed is waited for by ap_landed.
+template <class F>
+__device__ __forceinline__ void ap_apart(const unsigned char* __restrict__ k, const unsigned char* __restrict__ v, unsigned char* __restrict__ to_k, unsigned char* __restrict__ to_v, F&& f) {
+    f(k, v, to_k, to_v);
+}
+
 }  // namespace kf

@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "kf_ctx.h"
+#include "kf_flash.h"
 #include "kf_rb_recur.h"
 
 namespace kf {
@@ -588,6 +589,158 @@ __global__ void __launch_bounds__(256 * KH, HD <= 128 ? 2 : 1) rb_attn_prefill_k
         }
 }
 
+// The same for heads of exactly HD keys and values columns, four waves over all keys: tiles go global -> LDS by buffer loads, several on their way, and a wave's walk is the pipeline of kf_flash.h.
+// us, staged through registers (keys in two halves up to 512 workgroups) | so, 16 heads on 8 of 128: 300 tokens 22.1 | 20.0, 1500 58.7 | 51.0, 3000 109 | 99.5, windowed 4096, 8190 tokens 443 | 313; four
+// sequences of 300 25.9 | 22.6, of 509 with 20 heads on 4 52.4 | 43.0
+template <int HD>
+__global__ void __launch_bounds__(256, 2) rb_attn_walk_kernel(const kf_rb_attention a, const int32_t* __restrict__ seqs) {
+    using Wave = FlashWave<HD>;
+    using Tile = ApTile<HD>;
+    constexpr int NI = Tile::PART / 4096, SET = 2 * Tile::PART; /* load instructions per wave and part; bytes of a K and a V tile */
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5, kvd = a.n_kv * HD;
+    const int row0 = seqs[4 * blockIdx.z], n = seqs[4 * blockIdx.z + 1], pos0 = seqs[4 * blockIdx.z + 2], slot = seqs[4 * blockIdx.z + 3];
+    const int wg = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y, g = __builtin_amdgcn_readfirstlane(wg % a.n_kv), bx = (int)gridDim.x - 1 - __builtin_amdgcn_readfirstlane(wg / a.n_kv);
+    const int GQ = __builtin_amdgcn_readfirstlane(a.n_head / a.n_kv), ncol = n * GQ;
+    if (bx * 128 >= ncol) return; /* workgroup-uniform */
+    const uint16_t* raw = reinterpret_cast<const uint16_t*>(a.raw) + (size_t)row0 * a.ldraw;
+    [[maybe_unused]] const uint16_t *k_new = reinterpret_cast<const uint16_t*>(a.k_new) + (size_t)row0 * kvd + (size_t)g * HD, *v_new = raw + a.v_col + (size_t)g * HD;
+    [[maybe_unused]] const uint16_t* k_ring = reinterpret_cast<const uint16_t*>(a.k_cache) + (size_t)slot * a.slot_stride + (size_t)g * a.head_stride;
+    [[maybe_unused]] const uint16_t* v_ring = reinterpret_cast<const uint16_t*>(a.v_cache) + (size_t)slot * a.slot_stride + (size_t)g * a.head_stride;
+    int c = bx * 128 + wid * 32 + r;
+    c = c < ncol ? c : ncol - 1; /* columns past the end repeat the last one and are not stored */
+    const int tok = c / GQ, head = g * GQ + (c - tok * GQ), pos = pos0 + tok, lo = rb_first_key(pos, a);
+    auto tok_of = [&](int cc) { return __builtin_amdgcn_readfirstlane((cc < ncol ? cc : ncol - 1) / GQ); }; /* (a division is vector work: what follows from it would count as a lane's own) */
+    auto first_key = [&](int p) { return __builtin_amdgcn_readfirstlane(rb_first_key(p, a)); };
+    const int w0 = pos0 + tok_of(bx * 128 + wid * 32), w1 = pos0 + tok_of(bx * 128 + wid * 32 + 31);
+    const int wlo = first_key(w0), wlo1 = first_key(w1);
+    const int klo = first_key(pos0 + tok_of(bx * 128)), khi = pos0 + tok_of(bx * 128 + 127);
+    Wave W;
+    W.init();
+    const uint16_t* q = raw + (size_t)tok * a.ldraw + (size_t)head * HD;
+#pragma unroll
+    for (int s = 0; s < Wave::NS; s++) W.qf[s] = *reinterpret_cast<const u32x4*>(q + 16 * s + 8 * h);
+    [[maybe_unused]] const uint32_t ldk = (uint32_t)kvd * 2, ldv = (uint32_t)a.ldraw * 2; /* offsets inside a batch or a ring fit 31 bits (checked by the launcher) */
+    [[maybe_unused]] const int turn = __builtin_amdgcn_readfirstlane(klo / a.cache_rows * a.cache_rows); /* the old keys that are seen are in the ring: from the first of them on it turns at most once */
+    uint32_t lk[NI], lv[NI]; /* this lane's offsets in a tile of the batch */
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int row = (wid * NI + i) * Tile::RPI + lane / (HD / 8), p = lane % (HD / 8);
+        lk[i] = (uint32_t)row * ldk + ap_swz_k<HD>(row, p) * 16, lv[i] = (uint32_t)row * ldv + ap_swz_v<HD>(row, p) * 16;
+    }
+    auto load = [&](int t, unsigned char* to_k, unsigned char* to_v) {
+#ifdef __HIP_DEVICE_COMPILE__
+        const int k0 = klo + 32 * t;
+        auto rsrc = [](const uint16_t* p, uint32_t n) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, (int)n, 0x00020000); };
+        auto to = [&](unsigned char* p, int i) { return (__attribute__((address_space(3))) void*)(p + (wid * NI + i) * 1024); };
+        if (k0 >= pos0) { /* workgroup-uniform: a tile of the batch, rows past the last key become zeros */
+            const uint32_t left = khi - k0 < 0 ? 0 : (khi - k0 < 31 ? khi - k0 + 1 : 32);
+            const __amdgpu_buffer_rsrc_t rk = rsrc(k_new + (size_t)(k0 - pos0) * kvd, left * ldk), rv = rsrc(v_new + (size_t)(k0 - pos0) * a.ldraw, left * ldv);
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to(to_k, i), 16, lk[i], 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to(to_v, i), 16, lv[i], 0, 0, 0);
+            }
+            return;
+        }
+#pragma unroll 1
+        for (int i = 0; i < NI; i++) {
+            const int row = (wid * NI + i) * Tile::RPI + lane / (HD / 8), p = lane % (HD / 8);
+            const int kk = k0 + row < khi ? k0 + row : khi; /* past the last key: masked, never read past it */
+            if (kk >= pos0) { /* (a tile of both kinds takes two loads a part: more than the waits count on, which is the safe side) */
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(k_new, 0x7FFFFFF0u), to(to_k, i), 16, (uint32_t)(kk - pos0) * ldk + ap_swz_k<HD>(row, p) * 16, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(v_new, 0x7FFFFFF0u), to(to_v, i), 16, (uint32_t)(kk - pos0) * ldv + ap_swz_v<HD>(row, p) * 16, 0, 0, 0);
+            } else {
+                const int at = (kk - turn < a.cache_rows ? kk - turn : kk - turn - a.cache_rows) * (2 * HD);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(k_ring, 0x7FFFFFF0u), to(to_k, i), 16, at + ap_swz_k<HD>(row, p) * 16, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(v_ring, 0x7FFFFFF0u), to(to_v, i), 16, at + ap_swz_v<HD>(row, p) * 16, 0, 0, 0);
+            }
+        }
+#endif
+    };
+    auto part = [&](int b, bool v) { return smem_raw + b * SET + (v ? Tile::PART : 0); };
+#pragma unroll 1
+    for (int b = 0; b < AP_NB - 1; b++) load(b, part(b, false), part(b, true));
+    Tile T;
+    T.init(lane);
+    const float sc2 = a.scale * RB_LOG2E;
+    const int ntile = (khi - klo) / 32 + 1, ta = (wlo - klo) / 32, tb = (w1 - klo) / 32; /* the workgroup's tiles; this wave's */
+    auto maximum = [&](fl_f32x16& st, int t, float m) {
+        const int k0 = klo + 32 * t;
+        if (!(k0 >= wlo1 && k0 + 31 <= w0)) m = Wave::mask(st, k0, lo, pos, h); /* else every key of the tile is seen by every column of the wave */
+        return xmax32(m);
+    };
+    int b = 0;
+    auto turn_to = [&](int t, auto&& f) { /* K of tile t + 1 and V of tile t are here; tile t + NB - 1 goes where tile t - 1 was */
+        const int b1 = b + 1 < AP_NB ? b + 1 : 0, bl = b ? b - 1 : AP_NB - 1;
+        ap_apart(part(b1, false), part(b, true), part(bl, false), part(bl, true), [&](const unsigned char* k, const unsigned char* v, unsigned char* to_k, unsigned char* to_v) __attribute__((always_inline)) {
+            load(t + AP_NB - 1, to_k, to_v);
+            f(k, v);
+        });
+        ap_landed<(AP_NB - 3) * 2 * NI>(); /* tile t + 2 */
+        b = b1;
+    };
+    auto idle = [](const unsigned char*, const unsigned char*) {};
+    fl_f32x16 sa, sb;
+    float mt;
+    auto first = [&](int t, const unsigned char* k) { /* the scores of this wave's first tile */
+        W.scores(sa, [&](int s) { return T.k(k, s); });
+        mt = maximum(sa, t, Wave::template scale<false>(sa, sc2));
+    };
+    auto step = [&](int t, fl_f32x16& cur, fl_f32x16& nxt) {
+        turn_to(t, [&](const unsigned char* k, const unsigned char* v) __attribute__((always_inline)) {
+            mt = W.template tile<false, false>(cur, mt, nxt, sc2, [&](int s) { return T.k(k, s); }, [&](int s2, int db) { return T.v(v, s2, db); });
+            mt = maximum(nxt, t + 1, mt);
+        });
+    };
+    ap_landed<(AP_NB - 3) * 2 * NI>(); /* tiles 0 and 1 */
+    int t = 0;
+    if (ta == 0) {
+        first(0, part(0, false));
+    } else { /* every wave takes part in the loads and barriers of all tiles */
+#pragma unroll 1
+        for (; t < ta - 1; t++) turn_to(t, idle);
+        turn_to(t, [&](const unsigned char* k, const unsigned char*) __attribute__((always_inline)) { first(ta, k); });
+        t++;
+    }
+    for (; t <= tb; t += 2) {
+        step(t, sa, sb);
+        if (t + 1 <= tb) step(t + 1, sb, sa);
+    }
+#pragma unroll 1
+    for (t = tb + 1; t < ntile; t++) turn_to(t, idle);
+    ap_landed<0>(); /* loads past the last tile too: the tiles' place is free */
+    // out[col][d] = O^T[d][col] times a factor, by way of LDS: a wave's 32 columns [32][HD] in 32 bits, chunk c of a column at c ^ (column & 15); eight d's to a lane and turn
+    unsigned char* const mine = smem_raw + wid * 32 * HD * 4;
+    const float inv = a.out_scale * rb_softmax_factor(W.M, xsum32(W.l), a.sink);
+#pragma unroll
+    for (int db = 0; db < Wave::NDB; db++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            *reinterpret_cast<f32x4*>(mine + r * (HD * 4) + (((8 * db + 2 * e + h) ^ (r & 15)) << 4)) = f32x4{W.o[db][4 * e] * inv, W.o[db][4 * e + 1] * inv, W.o[db][4 * e + 2] * inv, W.o[db][4 * e + 3] * inv};
+    asm volatile("" ::: "memory");
+#pragma unroll 1
+    for (int i = lane; i < 32 * HD / 8; i += 64) {
+        const int col = i / (HD / 8), u = i % (HD / 8), cc = bx * 128 + wid * 32 + col;
+        if (cc >= ncol) break;
+        const int tk = cc / GQ, hd = g * GQ + (cc - tk * GQ);
+        f32x4 v[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) v[e] = *reinterpret_cast<const f32x4*>(mine + col * (HD * 4) + (((2 * u + e) ^ (col & 15)) << 4));
+        if (a.gated) {
+            const uint16_t* const gate = raw + (size_t)tk * a.ldraw + a.gate_col + (size_t)hd * HD + 8 * u;
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const f32x4 gv = rb_ld4(gate + 4 * e);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[e][j] *= rb_sigmoid(gv[j]);
+            }
+        }
+        uint16_t* const out = reinterpret_cast<uint16_t*>(a.out) + (size_t)(row0 + tk) * a.ldout + (size_t)hd * HD + 8 * u;
+        rb_st4(out, v[0]), rb_st4(out + 4, v[1]);
+    }
+}
+
 // decode: grid (n_kv * column blocks of 32 query heads, key ranges, rows).  A row's keys are dealt to the ranges evenly by its own position: the launch only knows a bound that holds for the graph it
 // is captured in, up to twice the keys there are, and with ranges cut from the bound 32 rows at position 1024 had all their keys in the first of two ranges and half the workgroups
 // returned at once.  A second range costs about 10 us wherever it is cheap to avoid (256 -> 257 keys of 32 rows: 15.2 -> 25.4 us: parts written through, an arrival counter, three trips to memory in a
@@ -801,6 +954,15 @@ template <int HD>
 static int prefill_go(hipStream_t st, const kf_rb_attention& a, const int32_t* seqs, int n_seq, int max_n) {
     const dim3 grid((unsigned)(((long long)max_n * (a.n_head / a.n_kv) + 127) / 128), a.n_kv, n_seq);
     if constexpr (HD <= 128) {
+        if constexpr (HD == 64 || HD == 128) {
+            if (a.dim == HD && a.vdim == HD) {
+                constexpr size_t smem = AP_NB * 2 * ApTile<HD>::PART;
+                static int done = 0;
+                if (big_lds(rb_attn_walk_kernel<HD>, smem, done)) return KF_HIP_CHECK;
+                hipLaunchKernelGGL((rb_attn_walk_kernel<HD>), grid, dim3(256), smem, st, a, seqs);
+                return KF_OK;
+            }
+        }
         if ((long)grid.x * grid.y * grid.z <= 512 && max_n >= 256) return prefill_kh<HD, 2>(st, a, seqs, grid);
     }
     return prefill_kh<HD, 1>(st, a, seqs, grid);

@@ -376,7 +376,7 @@ class Window(Layer):
 
 
 WINDOWS = [(4, 2, 64, 64, 24, 0.1), (6, 1, 32, 16, 100, 0.3), (5, 5, 48, 80, 7, 0.2), (40, 1, 16, 32, 40, 0.5), (8, 2, 128, 64, 200, 0.05), (2, 1, 64, 192, 33, 0.1), (2, 2, 256, 256, 1, 0.02),
-           (3, 1, 20, 9, 16, 0.3), (2, 1, 100, 30, 600, 0.1), (4, 1, 128, 128, 400, 0.12)]
+           (3, 1, 20, 9, 16, 0.3), (2, 1, 100, 30, 600, 0.1), (4, 1, 128, 128, 400, 0.12), (6, 2, 128, 128, 250, 0.1), (3, 1, 64, 64, 333, 0.2)]
 
 
 @pytest.mark.parametrize("shape", WINDOWS, ids=lambda s: "x".join(map(str, s[:5])))
