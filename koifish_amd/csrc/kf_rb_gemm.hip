@@ -138,12 +138,14 @@ int rb_gemm_launch(hipStream_t st, const RbProduct& q) {
     }
 }
 // The 32-bit product on v_mfma_f32_16x16x4_f32 (157 TFLOP/s; the vector pipe without packed instructions: 78).  It is bound by the MFMAs, 16 x slower than bf16's, so the tile only has to share them
-// out evenly: 64 x 64 tiles, five to a CU.
+// out evenly: 64 x 64 tiles, five to a CU; a lone one of a CU waits for its loads, so with three buffers.  us at 512 rows, two buffers | three: 2048 x 6144 (256 tiles) 127.6 | 108.6, x 2048 46.3 | 40.9; 5120 x 2048
+// (640) 95.6 | 100.5, 12288 x 2048 190 | 201.
 int rb_f32_launch(hipStream_t st, const RbProduct& q) {
     const kf_rb_product& p = q.p;
     if (p.mode == KF_RB_SUM || (p.mode != KF_RB_ALL && q.e.tile != 64)) return 1;
     if (p.mode != KF_RB_ALL) return rb_go<RbTiny, true, float>(st, q, (long)(p.m / 64) * q.e.n_tile);
-    return rb_go<RbTiny, false, float>(st, q, rb_tiles(p, 64, 64));
+    const long nwg = rb_tiles(p, 64, 64);
+    return nwg <= 256 ? rb_go<G3Few, false, float>(st, q, nwg) : rb_go<RbTiny, false, float>(st, q, nwg);
 }
 
 }  // namespace kf
