@@ -31,17 +31,14 @@ template <class C>
 __device__ __forceinline__ void g3_epilogue_qkrope(const GemmArgs& a, int m0, int t0, const f32x4 (&acc)[C::MT][C::NT], int tid, unsigned char* smem_raw, uint16_t* ybase, long long ldy, int mshift,
                                                    const uint16_t* nw) {
     static_assert(C::BM == 128, "one head per tile");
-    using Out = G3Out<C>;
-    static_assert(Out::TN * 8 % C::NTH == 0, "the eight threads of a token run the loop together");
-    Out::template all<8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+    using Out = G3Out16<C>;
+    static_assert(C::BN * 8 % C::NTH == 0, "the eight threads of a token run the loop together");
+    Out::template spill<false>(acc, smem_raw, tid, nullptr, 0);
+    Out::template each<8>(tid, [&](int tk, int u) {
         const int tok = t0 + tk < a.n ? t0 + tk : a.n - 1; /* (a token past the end: the last one's angles, not stored) */
-        float x[2][8]; /* rows 8 u .. and 64 + 8 u .. */
+        float x[2][8]; /* rows 8 u .. and 64 + 8 u .., as the plain epilogue stores them (alpha 1, no bias) */
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            Out::rows8(smem_raw, lt, 8 * e + u, tid, x[e]);
-#pragma unroll
-            for (int j = 0; j < 8; j++) x[e][j] = round_bf16(x[e][j]); /* the value the plain epilogue stores (alpha 1, no bias) */
-        }
+        for (int e = 0; e < 2; e++) g3_unpack8(Out::rows8(smem_raw, tk, 8 * e + u), x[e]);
         if (nw) {
             double ss = 0.0;
 #pragma unroll
@@ -86,13 +83,15 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
     if (!AKM && a.swiglu) { /* Relu::Forw (CU_swiglu_v0, Activation.cu:85-93) on the two bf16-rounded projections, as swiglu_kernel: 16-row block 2i holds gate rows, block 2i + 1 the up rows of
                                the same 16 FFN rows (the operand was dequantised interleaved) */
         const int F = a.M >> 1; /* a multiple of 16 (gemm3_swiglu_launch) */
-        Out::template all<C::BM / 16>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
+        using Half = G3Out16<C>;
+        Half::template spill<false>(acc, smem_raw, tid, nullptr, 0);
+        Half::template each<C::BM / 16>(tid, [&](int tk, int u) {
             const int tok = t0 + tk, f = (m0 >> 1) + 8 * u, c = (u >> 1) * 4 + (u & 1);
             if (tok >= a.n || f >= F) return;
             float g[8], p[8];
-            Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, p);
+            g3_unpack8(Half::rows8(smem_raw, tk, c), g), g3_unpack8(Half::rows8(smem_raw, tk, c + 2), p);
 #pragma unroll
-            for (int j = 0; j < 8; j++) g[j] = round_bf16(g[j]), p[j] = round_bf16(p[j]), g[j] = (g[j] * p[j]) / (1.0f + kf_expf(-g[j]));
+            for (int j = 0; j < 8; j++) g[j] = (g[j] * p[j]) / (1.0f + kf_expf(-g[j]));
             g3_store16(a.y + (size_t)t0 * a.ldy + (m0 >> 1), (uint32_t)tk * (uint32_t)(2 * a.ldy) + 16 * u, g3_pack8(g));
         });
         return;
@@ -120,6 +119,24 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
     const uint16_t* const res = AKM ? nullptr : a.residual;
     // eight rows of a token, every operand of theirs 16 aligned bytes; else one row
     const bool whole = ((ldy | Mlim) & 7) == 0 && ldy < (1 << 22) && ((reinterpret_cast<uintptr_t>(ybase) | reinterpret_cast<uintptr_t>(res) | reinterpret_cast<uintptr_t>(a.bias)) & 15) == 0 && (!res || (a.ldr & 7) == 0);
+    if (whole && a.alpha == 1.0f && a.beta == 0.0f) {
+        using Half = G3Out16<C>;
+        uint16_t* const yt = ybase + (size_t)t0 * ldy + (m0 - mshift);
+        if (a.bias) Half::template spill<true>(acc, smem_raw, tid, a.bias + m0, Mlim - m0);
+        else Half::template spill<false>(acc, smem_raw, tid, nullptr, 0);
+        Half::template each<C::BM / 8>(tid, [&](int tk, int u) {
+            const int tok = t0 + tk, m = m0 + 8 * u;
+            if (tok >= a.n || m >= Mlim) return;
+            u32x4 v = Half::rows8(smem_raw, tk, u);
+            if (res) {
+                const u32x4 r = *reinterpret_cast<const u32x4*>(res + (size_t)tok * a.ldr + m);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = pack_bf16x2(bf_lo(r[j]) + bf_lo(v[j]), bf_hi(r[j]) + bf_hi(v[j]));
+            }
+            g3_store16(yt, (uint32_t)tk * (uint32_t)(2 * ldy) + 16 * u, v);
+        });
+        return;
+    }
     if (whole) {
         Out::template all<C::BM / 8>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
             const int tok = t0 + tk, m = m0 + 8 * u;

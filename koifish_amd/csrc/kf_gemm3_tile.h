@@ -371,6 +371,45 @@ __device__ __forceinline__ void g3_unpack8(u32x4 p, float (&v)[8]) {
 #pragma unroll
     for (int j = 0; j < 4; j++) v[2 * j] = bf_lo(p[j]), v[2 * j + 1] = bf_hi(p[j]);
 }
+// The same where a result is a bf16 rounding of the sum (plus a bias) and nothing else: it is rounded in front of LDS, half the bytes, never two passes.  us, 32 bits | so, K = 64: 4096 x 4096 in 256 x 256 tiles 13.8 | 11.6, in 192 x 256 20.3 | 15.1; 4800 x 1600
+// at 8192 rows 125.7 | 120.3
+template <class C>
+struct G3Out16 {
+    static constexpr int ROW = (C::BM / 2) % 64, P = ROW == 0 ? 1 : 2; /* tokens whose rows start at different banks */
+    static_assert(C::BM * C::BN * 2 <= C::SMEM && C::BM % 64 == 0, "the tile fits, its chunks of eight rows in eights");
+    static __device__ __forceinline__ int at(int tok, int chunk) { return tok * (2 * C::BM) + ((chunk ^ ((tok / P) & (16 / P - 1))) << 4); } /* rows 8 chunk .. + 7 of a token */
+    template <bool BIAS>
+    static __device__ __forceinline__ void spill(const f32x4 (&acc)[C::MT][C::NT], unsigned char* smem, int tid, const uint16_t* bias, int rows) { /* bias: of the tile's rows, `rows` of them exist */
+        const int wid = tid >> 6, lane = tid & 63, wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
+#pragma unroll
+        for (int mt = 0; mt < C::MT; mt++) {
+            const int blk = C::row_block(wm, mt);
+            float b[4] = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (BIAS) {
+                u32x2 b4 = u32x2{0, 0};
+                if (blk * 16 + 4 * q4 < rows) b4 = *reinterpret_cast<const u32x2*>(bias + blk * 16 + 4 * q4);
+                b[0] = bf_lo(b4.x), b[1] = bf_hi(b4.x), b[2] = bf_lo(b4.y), b[3] = bf_hi(b4.y);
+            }
+            unsigned char* const to = smem + at(wn * (16 * C::NT) + r16, 2 * blk + (q4 >> 1)) + 8 * (q4 & 1); /* (16 tokens further the swizzle is the same) */
+#pragma unroll
+            for (int nt = 0; nt < C::NT; nt++) {
+                f32x4 v = acc[mt][nt];
+                if constexpr (BIAS) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = v[j] + b[j];
+                }
+                *reinterpret_cast<u32x2*>(to + nt * 16 * (2 * C::BM)) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+        }
+    }
+    static __device__ __forceinline__ u32x4 rows8(const unsigned char* smem, int tok, int chunk) { return *reinterpret_cast<const u32x4*>(smem + at(tok, chunk)); }
+    template <int U, class F>
+    static __device__ __forceinline__ void each(int tid, F&& f) { /* f(token of the tile, unit) for this thread's share of BN tokens x U units, after a barrier */
+        __syncthreads();
+#pragma unroll 1
+        for (int id = tid; id < C::BN * U; id += C::NTH) f(id / U, id % U);
+    }
+};
 // 256 x 256 or 192 x 256: with one big workgroup per CU a launch takes whole rounds of 256 tiles, and a round of the smaller ones takes 0.79 to 0.95 of a round, so the smaller tile pays where it needs no
 // more rounds.  us, big | wide: 6144 x 1024 at 2608 rows (264 | 352 tiles) 66.7 | 54.3, x 4096 176 | 143, x 25600 1230 | 1036; 5120 x 12288 at 4096 rows (320 | 432) 543 | 518; 10240 x 8192 at 3500 rows
 // (560 | 756) 522 | 449.  One round more pays for 5 and 6 of them at K <= 2048, where the round is shortest against its start: 12288 x 2048 at 5888 rows (1104 | 1472) 280 | 269, at 6912 (1296 | 1728) 332 |
