@@ -38,10 +38,7 @@ __device__ __forceinline__ u32x4 ld_nt(const u32x4* p) { return __builtin_nontem
 // Fixed fp32 exp: the same operation sequence as oracle/kfo_math.h kfo_expf (independent statement of one
 // recipe: Cody-Waite reduction, degree-7 Taylor/Horner in fma form, two-step power-of-two scaling), so the
 // softmax numerators and SwiGLU agree bit for bit with the CPU oracle.  Needs -ffp-contract=off.
-__device__ __forceinline__ float kf_expf(float x) {
-    if (x > 88.72283f) return __builtin_inff();
-    if (x < -87.33654f) return 0.0f;
-    if (x != x) return x;
+__device__ __forceinline__ float kf_exp_core(float x) { /* x in [-87.33654, 88.72283] */
     float t = x * 1.44269502162933349609375f;
     float n = (t + 12582912.0f) - 12582912.0f;
     float r = fmaf(n, -0.693145751953125f, x);
@@ -57,6 +54,20 @@ __device__ __forceinline__ float kf_expf(float x) {
     // the oracle scales in two exact-then-rounded steps ((p * 2^e1) * 2^e2, e1 = e/2): the first product is exact, so the pair rounds once,
     // exactly like one v_ldexp_f32
     return __builtin_amdgcn_ldexpf(p, (int)n);
+}
+__device__ __forceinline__ float kf_expf(float x) {
+    if (x > 88.72283f) return __builtin_inff();
+    if (x < -87.33654f) return 0.0f;
+    if (x != x) return x;
+    return kf_exp_core(x);
+}
+// n / d, correctly rounded as the compiler's division (reciprocal, one Newton step, two residual steps), for operands and quotients far from the ends of the range: no scaling, no fix-up
+__device__ __forceinline__ float kf_div_mid(float n, float d) {
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    float q = n * r;
+    q = fmaf(fmaf(-d, q, n), r, q);
+    return fmaf(fmaf(-d, q, n), r, q);
 }
 
 // Fixed fp32 natural log (same operation sequence as oracle/kfo_math.h kfo_logf): x = m * 2^e with m in [sqrt(1/2), sqrt(2)),
