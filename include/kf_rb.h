@@ -75,9 +75,14 @@ typedef struct kf_rb_product {
     float norm_eps;
     int32_t norm_dim;
     int32_t act_lo, act_hi; /* STORE: the columns that pass through act; equal: none */
+    int32_t parts;          /* STORE_F32 of a decode batch, kf_rb_linear_parts() of them (0, 1: none): y + j part_stride gets the sum over the j-th part of k; who reads y adds them up (kf_rb_norm_rows) */
+    int64_t part_stride;
 } kf_rb_product;
 int kf_rb_linear(kf_ctx* ctx, const kf_rb_product* p);
 int kf_rb_linear_norms(int type, int n, int k);
+/* into how many parts of k a STORE_F32 product of a decode batch is best cut, 1 .. KF_RB_MAX_PARTS */
+#define KF_RB_MAX_PARTS 2
+int kf_rb_linear_parts(int type, int m, int k, int n);
 
 /* load time: a bf16 matrix src [rows][cols] into rows row0 .. of a padded one (ld columns; columns cols .. ld - 1 are left alone: allocate zeroed) of storage `type`.
  * half < 0: row r goes to row row0 + r; half 0 / 1: to row 32 (r / 16) + 16 half + r % 16, the gate / up halves of a GATED product's weight.  tiled (bf16): a product's
@@ -116,6 +121,8 @@ typedef struct kf_rb_norming {
     int64_t ld;
     int32_t type, kind, dim, n;
     float eps;
+    int32_t parts; /* z is the sum of z + j part_stride, j < parts (0: 1) */
+    int64_t part_stride;
 } kf_rb_norming;
 int kf_rb_norm_rows(kf_ctx* ctx, const kf_rb_norming* a);
 /* host: (sin, cos) of p * base^(-2 i / width) for column pair i, as two factors of the angle: hi [(n_pos + 63) / 64][ld / 2][2] at p = 64 j, lo [64][ld / 2][2]; column 2 i of

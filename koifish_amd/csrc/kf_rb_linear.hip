@@ -56,7 +56,7 @@ __device__ __forceinline__ void rb_multiply(const u32x4 (&a)[U][MG], const u32x4
 }
 // the waves' partial tiles -> outputs; list: the columns are pairs
 template <int NT, int MG, int NW>
-__device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4 (&acc)[MG][NT], float (&red)[NW][MG][16 * NT][17], const int32_t* list, int m0, int tid) {
+__device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4 (&acc)[MG][NT], float (&red)[NW][MG][16 * NT][17], const int32_t* list, int m0, int tid, int part = 0) {
     const kf_rb_product& p = q.p;
     const int lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
 #pragma unroll
@@ -88,7 +88,7 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
             const int m = m0 + row;
             reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + m] = f2bf(m >= p.act_lo && m < p.act_hi ? rb_activate(p.act, d) : d);
         } else if (p.epilogue == KF_RB_STORE_F32) {
-            reinterpret_cast<float*>(p.y)[(size_t)yr * p.ldy + m0 + row] = d;
+            reinterpret_cast<float*>(p.y)[part * (size_t)p.part_stride + (size_t)yr * p.ldy + m0 + row] = d;
         } else {
             const float z = fmaf(p.alpha, p.res[(size_t)yr * p.ldr + m0 + row], d);
             reinterpret_cast<float*>(p.y)[(size_t)yr * p.ldy + m0 + row] = z;
@@ -153,7 +153,8 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[RED > STAGE ? RED : STAGE];
     auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
-    const int m0 = blockIdx.x * (16 * MG), nstep = p.k / 32;
+    const int m0 = blockIdx.x * (16 * MG), part = p.mode == KF_RB_ALL ? (int)blockIdx.y : 0, parts = p.parts > 1 ? p.parts : 1;
+    const int steps = p.k / 32, nstep = parts > 1 ? steps * (part + 1) / parts : steps; /* this part's steps end here */
     const uint16_t* W = reinterpret_cast<const uint16_t*>(p.w);
     const uint16_t* X = reinterpret_cast<const uint16_t*>(p.x);
     const int32_t* list = nullptr;
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     }
     const uint16_t* wr = W + (size_t)m0 * p.k + 8 * lane;
     u32x4 a[U][MG], b[U][NT];
-    int s = wid * U;
+    int s = (parts > 1 ? steps * part / parts : 0) + wid * U;
     rb_load_w<MG, U>(a, wr, p.k, s, nstep);
     const uint16_t* xp[NT];
     Tokens tok;
@@ -245,7 +246,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
             for (int g = 0; g < MG; g++) a[u][g] = an[u][g];
     }
     if constexpr (TURN) __syncthreads(); /* the token rows make way */
-    rb_stream_finish<NT, MG, NW>(q, acc, red, list, m0, tid);
+    rb_stream_finish<NT, MG, NW>(q, acc, red, list, m0, tid, part);
 }
 
 // RESIDUAL with the rows' experts summed: (chosen expert, k-step) pairs as one list, cut evenly over the waves
@@ -327,7 +328,7 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const int cols = tiles ? q.e.tile : p.n, nt = (cols + 15) / 16;
     if (nt > 4 || (tiles && q.e.tile % 16)) return 1;
     if (p.mode == KF_RB_SUM && ((long)p.n * q.e.top > KF_RB_SUM_PAIRS || q.e.tile < p.n)) return 1;
-    dim3 grid(p.m / (p.epilogue == KF_RB_GATED ? 32 : 16), tiles ? q.e.n_tile : 1);
+    dim3 grid(p.m / (p.epilogue == KF_RB_GATED ? 32 : 16), tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
     const bool wide = (long)grid.x * grid.y < 768 && p.k >= 512; /* few workgroups: more waves each, more loads in flight per CU */
     if (p.norm_z) {
         wide ? norm_stream_go<8>(st, q, grid) : norm_stream_go<4>(st, q, grid);
@@ -345,6 +346,9 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
 }  // namespace kf
 
 using namespace kf;
+// Up to half a workgroup per CU: two parts of k, a chip full of workgroups.  us per step of 8 recurrent / windowed layers behind 300 tokens, whole | two | four parts: 2048 wide, 32 rows 867 | 828 | 850, 8 rows 537 | 514 | 523, one
+// 473 | 457 | 467; 4096 wide (256 workgroups) 1 row 969 | 978, 16 rows 1238 | 1252
+extern "C" int kf_rb_linear_parts(int type, int m, int k, int n) { return type == KF_BF16 && n >= 1 && n <= KF_RB_DECODE_MAX && m >= 1 && m / 16 <= 128 && k >= 2048 ? 2 : 1; }
 extern "C" int kf_rb_linear_norms(int type, int n, int k) { return type == KF_BF16 && n >= 1 && n <= KF_RB_NORM_ROWS && k % KF_RB_PAD == 0; }
 extern "C" int kf_rb_linear(kf_ctx* c, const kf_rb_product* p) {
     CHKCTX(c);
@@ -356,6 +360,8 @@ extern "C" int kf_rb_linear(kf_ctx* c, const kf_rb_product* p) {
     if (p->epilogue < KF_RB_STORE || p->epilogue > KF_RB_GATED || p->mode < KF_RB_ALL || p->mode > KF_RB_SUM) return abi_fail(KF_INVALID_ARGS, "kf_rb_linear: epilogue or mode");
     if (p->epilogue == KF_RB_RESIDUAL && (!p->res || !al16(p->res) || p->ldr < p->m || p->ldr % 4)) return abi_fail(KF_INVALID_ARGS, "kf_rb_linear: residual");
     if (p->act_lo < p->act_hi && (p->epilogue != KF_RB_STORE || p->mode != KF_RB_ALL || p->act_lo < 0 || p->act_hi > p->m)) return abi_fail(KF_INVALID_ARGS, "kf_rb_linear: activated columns");
+    if (p->parts > 1 && (p->type != KF_BF16 || p->epilogue != KF_RB_STORE_F32 || p->mode != KF_RB_ALL || p->n > KF_RB_DECODE_MAX || p->parts > KF_RB_MAX_PARTS || p->part_stride < (int64_t)(p->n - 1) * p->ldy + p->m || p->norm_z))
+        return abi_fail(KF_INVALID_ARGS, "kf_rb_linear: %d parts", p->parts);
     if (p->ssq && (!kf_rb_linear_norms(p->type, p->n, p->m) || p->epilogue != KF_RB_RESIDUAL)) return abi_fail(KF_INVALID_ARGS, "kf_rb_linear: sums of squares");
     if (p->norm_z && (!kf_rb_linear_norms(p->type, p->n, p->k) || p->mode != KF_RB_ALL || p->epilogue == KF_RB_RESIDUAL || !p->norm_w || !p->norm_x || !p->norm_ssq || p->norm_dim < 1 || p->norm_dim > p->k || p->ldx != p->k || !al16(p->norm_z) ||
                       !al16(p->norm_w) || !al16(p->norm_x)))

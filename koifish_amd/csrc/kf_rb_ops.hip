@@ -150,7 +150,14 @@ __global__ void __launch_bounds__(256) rb_norm_rows_kernel(const kf_rb_norming a
         const int c = 4 * ((int)threadIdx.x + i * nt);
         v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (c < a.ld) {
-            v[i] = rb_ld4(a.z + (size_t)src * a.ld + c);
+            f32x4 w[KF_RB_MAX_PARTS];
+#pragma unroll
+            for (int j = 0; j < KF_RB_MAX_PARTS; j++) w[j] = j == 0 || j < a.parts ? rb_ld4(a.z + j * (size_t)a.part_stride + (size_t)src * a.ld + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+            v[i] = w[0];
+#pragma unroll
+            for (int j = 1; j < KF_RB_MAX_PARTS; j++) {
+                if (j < a.parts) v[i] += w[j];
+            }
             if (hi) { /* two (sin, cos) pairs of each factor */
                 const f32x4 p = rb_ld4(hi + c), q = rb_ld4(lo + c);
                 v[i].x += p.x * q.y + p.y * q.x, v[i].y += p.y * q.y - p.x * q.x;
@@ -452,6 +459,7 @@ int kf_rb_norm_rows(kf_ctx* c, const kf_rb_norming* a) {
     if (!a || !a->z || !a->w || (!a->x_out && !a->h_out) || a->dim < 1 || a->ld < a->dim || a->ld % KF_RB_PAD || a->n < 1 || a->kind < KF_RB_RMS || a->kind > KF_RB_LAYER)
         return abi_fail(KF_INVALID_ARGS, "kf_rb_norm_rows: bad arguments");
     if (!type_ok(a->type)) return abi_fail(KF_UNSUPPORTED_DATATYPE, "kf_rb_norm_rows: storage %d", a->type);
+    if (a->parts > 1 && (a->parts > KF_RB_MAX_PARTS || a->part_stride < a->ld || a->part_stride % 4)) return abi_fail(KF_INVALID_ARGS, "kf_rb_norm_rows: %d parts", a->parts);
     if (a->pos_hi && (!a->pos_lo || !a->meta || !al16(a->pos_hi) || !al16(a->pos_lo))) return abi_fail(KF_INVALID_ARGS, "kf_rb_norm_rows: positions");
     if (!al16(a->z) || (a->add && !al16(a->add)) || !al16(a->w) || (a->x_out && !al16(a->x_out)) || (a->h_out && !al16(a->h_out))) return abi_fail(KF_BLAS_UNALIGN, "kf_rb_norm_rows: unaligned pointer");
     const int rc = a->type == KF_BF16 ? norm_rows_go<uint16_t>(c->stream, *a) : norm_rows_go<float>(c->stream, *a);

@@ -22,11 +22,12 @@ static hGTensor Mem(kf_ctx* c, const char* name, int type, size_t n) {
 }
 
 // ------------------------------------------------------------------------------------------------ neurons
-int RowProduct::Forw(const void* x, int64_t ldx, int n, void* y, int64_t ldy, int epilogue, int act, const float* res, float alpha, int mode, const kf_rb_experts* ex, float* ssq) {
+int RowProduct::Forw(const void* x, int64_t ldx, int n, void* y, int64_t ldy, int epilogue, int act, const float* res, float alpha, int mode, const kf_rb_experts* ex, float* ssq, int parts) {
     kf_rb_product p;
     std::memset(&p, 0, sizeof(p));
     p.w = w->data, p.x = x, p.y = y, p.res = res, p.ldx = ldx, p.ldy = ldy, p.ldr = ldy;
     p.type = hFish->Seq()->card.type, p.m = m, p.k = k, p.n = n, p.epilogue = epilogue, p.act = act, p.mode = mode, p.alpha = alpha, p.ssq = ssq;
+    p.parts = parts, p.part_stride = (int64_t)n * ldy;
     if (epilogue == KF_RB_STORE && act_lo < act_hi) p.act_lo = act_lo, p.act_hi = act_hi, p.act = col_act;
     kf_rb_experts e;
     if (ex) e = *ex, e.w_stride = (int64_t)m * k, p.experts = &e;
@@ -46,11 +47,12 @@ int RowNorm::Forw(const void* z, int n, float* x_out, void* h_out, const float* 
     const SEQ_CARD& c = hFish->Seq()->card;
     return kf_rb_norm(hFish->ctx, c.type, z, res, alpha, top, w->data, c.eps, dim, ld, n, rows, x_out, h_out);
 }
-int RowNorm::Rows(RowWork& w, const float* z, int n, const float* add, float* x_out, void* h_out, const int32_t* rows, bool positions) {
+int RowNorm::Rows(RowWork& w, const float* z, int n, const float* add, float* x_out, void* h_out, const int32_t* rows, bool positions, int parts) {
     const SeqFish* f = hFish->Seq();
     kf_rb_norming a;
     std::memset(&a, 0, sizeof(a));
     a.z = z, a.add = add, a.rows = rows, a.w = this->w->data, a.x_out = x_out, a.h_out = h_out, a.ld = ld, a.type = f->card.type, a.kind = f->card.norm_kind, a.dim = dim, a.n = n, a.eps = f->card.eps;
+    a.parts = parts, a.part_stride = (int64_t)n * ld;
     if (positions) a.pos_hi = F(f->pos_hi), a.pos_lo = F(f->pos_lo), a.meta = I(w.meta);
     return kf_rb_norm_rows(hFish->ctx, &a);
 }
@@ -59,8 +61,9 @@ int SeqFish::Enter(RowWork& w, int n) {
 }
 int SeqFish::Close(RowWork& w, RowProduct& proj, RowNorm& norm, const void* in, int64_t ldin, int n, bool defer) {
     if (card.add_norm) {
-        KF_TRY(proj.Forw(in, ldin, n, F(w.z), proj.m, KF_RB_STORE_F32));
-        return norm.Rows(w, F(w.z), n, F(w.x), F(w.x), P(w.h), nullptr, false);
+        const int parts = kf_rb_linear_parts(card.type, proj.m, proj.k, n); /* the norm adds them up */
+        KF_TRY(proj.Forw(in, ldin, n, F(w.z), proj.m, KF_RB_STORE_F32, 0, nullptr, 0, KF_RB_ALL, nullptr, nullptr, parts));
+        return norm.Rows(w, F(w.z), n, F(w.x), F(w.x), P(w.h), nullptr, false, parts);
     }
     KF_TRY(proj.Forw(in, ldin, n, F(w.z), proj.m, KF_RB_RESIDUAL, 0, F(w.x), card.alpha, KF_RB_ALL, nullptr, defer ? F(w.ssq) : nullptr));
     if (defer) {
@@ -512,7 +515,7 @@ int SeqFish::Ensure(RowWork& w, int rows, int n_seq, int head_rows, bool decode)
                 tiles = std::max(tiles, n), list = std::max(list, n * tile);
             }
         }
-        get(w.x, "x", KF_F32, (size_t)rows * W), get(w.z, "z", KF_F32, (size_t)rows * W), get(w.h, "h", T, (size_t)rows * W);
+        get(w.x, "x", KF_F32, (size_t)rows * W), get(w.z, "z", KF_F32, (size_t)std::max(rows, KF_RB_MAX_PARTS * std::min(rows, KF_RB_DECODE_MAX)) * W), get(w.h, "h", T, (size_t)rows * W);
         get(w.raw, "raw", T, need.raw), get(w.ao, "ao", T, need.ao), get(w.knew, "knew", T, need.knew);
         get(w.az, "az", KF_F32, need.az), get(w.gz, "gz", T, need.gz), get(w.recur, "recur", KF_F32, need.recur), get(w.act, "act", T, act), get(w.y, "y", T, y), get(w.rlogits, "rlogits", KF_F32, rl);
         get(w.meta, "meta", KF_F32, (size_t)rows * KF_RB_META), get(w.tok, "tok", KF_F32, rows), get(w.ids, "ids", KF_F32, pairs), get(w.weight, "weight", KF_F32, pairs);

@@ -101,14 +101,14 @@ struct RowProduct : GeNeuron {  // padded weight [m][k] (x experts)
     int m = 0, k = 0, experts = 0;
     int act_lo = 0, act_hi = 0, col_act = 0;  // KF_RB_STORE: columns [act_lo, act_hi) pass through col_act
     int Forw(const void* x, int64_t ldx, int n, void* y, int64_t ldy, int epilogue, int act = 0, const float* res = nullptr, float alpha = 0, int mode = KF_RB_ALL,
-             const kf_rb_experts* ex = nullptr, float* ssq = nullptr);
+             const kf_rb_experts* ex = nullptr, float* ssq = nullptr, int parts = 1);  // parts: y's planes lie n rows apart
     int ForwNormed(RowWork& w, int n, void* y, int64_t ldy, int epilogue, int act = 0);  // of w.h, the pending norm first
 };
 struct RowNorm : GeNeuron {
     hGTensor w;
     int dim = 0, ld = 0;
     int Forw(const void* z, int n, float* x_out, void* h_out, const float* res = nullptr, float alpha = 0, int top = 0, const int32_t* rows = nullptr);
-    int Rows(RowWork& w, const float* z, int n, const float* add, float* x_out, void* h_out, const int32_t* rows, bool positions);  // kf_rb_norm_rows, the design's kind of norm
+    int Rows(RowWork& w, const float* z, int n, const float* add, float* x_out, void* h_out, const int32_t* rows, bool positions, int parts = 1);  // kf_rb_norm_rows, the design's kind of norm; of `parts` planes of z, n rows apart
 };
 // a mixer: one product of h -> raw, what the kind does with raw -> ao, the product back, the sublayer's norm
 struct RowMixer : GeNeuron {

@@ -451,3 +451,34 @@ def test_attention_and_decayed_sum_in_one_launch(ctx, kind, sizes):
         L.check(ctx.hip.kf_rb_attention_decay_decode(ctx.h, C.byref(a.a), C.byref(b.a), ra[2].data_ptr(), n, ra[7]))
         ctx.sync()
         a.check(pa, results=a.compare(pa, ra[1])), b.check(pb, results=b.compare(pb, rb[1]))
+
+
+@pytest.mark.parametrize("n", [1, 5, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("m,k,parts", [(64, 64, 2), (192, 2048, 2), (448, 4160, 2), (256, 3136, 2)])
+def test_a_product_in_parts_and_the_norm_that_adds_them_up(ctx, n, m, k, parts):
+    """bf16, decode batches: every part of k in its own plane (fewer steps than waves, and parts that no wave count divides), their sum the product; the norm over the planes is the norm of the product"""
+    g = torch.Generator().manual_seed(n * m + k)
+    x, w = (torch.randn(n, k, generator=g)).bfloat16(), (torch.randn(m, k, generator=g) / k ** 0.5).bfloat16()
+    ws = w.reshape(m // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().cuda()
+    xd, z = x.cuda(), torch.full((parts + 1, n, m), 7.0, device="cuda")
+    p = L.RbProduct(w=ws.data_ptr(), x=xd.data_ptr(), y=z.data_ptr(), ldx=k, ldy=m, type=L.BF16, m=m, k=k, n=n, epilogue=L.RB_STORE_F32, mode=L.RB_ALL, parts=parts, part_stride=n * m)
+    L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+    ctx.sync()
+    steps = k // 32
+    for j in range(parts):
+        lo, hi = 32 * (steps * j // parts), 32 * (steps * (j + 1) // parts)
+        assert float((z[j].cpu().double() - x[:, lo:hi].double() @ w[:, lo:hi].double().t()).abs().max()) < 2e-5, j
+    assert bool((z[parts] == 7).all())
+    norm_w, h = torch.ones(m, device="cuda").bfloat16(), torch.zeros(n, m, device="cuda")
+    hb = torch.zeros(n, m, dtype=torch.bfloat16, device="cuda")
+    a = L.RbNorming(z=z.data_ptr(), w=norm_w.data_ptr(), x_out=h.data_ptr(), h_out=hb.data_ptr(), ld=m, type=L.BF16, kind=L.RB_LAYER, dim=m, n=n, eps=1e-5, parts=parts, part_stride=n * m)
+    L.check(ctx.hip.kf_rb_norm_rows(ctx.h, C.byref(a)))
+    ctx.sync()
+    y = x.double() @ w.double().t()
+    ref = torch.nn.functional.layer_norm(y, (m,), eps=1e-5)
+    assert float((h.cpu().double() - ref).abs().max()) < 1e-4
+    for bad in (dict(epilogue=L.RB_STORE), dict(parts=3), dict(part_stride=m // 2 if n == 1 else m)):
+        q = L.RbProduct.from_buffer_copy(p)
+        for f, v in bad.items():
+            setattr(q, f, v)
+        assert ctx.hip.kf_rb_linear(ctx.h, C.byref(q)) < 0, bad
