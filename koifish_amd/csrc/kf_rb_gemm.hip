@@ -11,14 +11,15 @@ namespace kf {
 using RbTiny = G3Cfg<64, 64, 4>;      /* 32-bit storage: five to a CU */
 using RbPairs = G3Cfg<128, 64, 4>;    /* experts of about a hundred pairs: half the padding of 128-pair tiles, each weight tile read about once; three to a CU (with three buffers, two: 64 experts of 3072 x 2048, 7884 pairs 259 -> 268 us) */
 
-// eight values from a multiple of 8 columns; rows of 16-bit values are at least 8-byte aligned
-__device__ __forceinline__ void rb_st8(uint16_t* p, const float (&v)[8], int64_t ld) {
+// eight values from a multiple of 8 columns; rows of 16-bit values are at least 8-byte aligned.  base: uniform, off: in elements.  In reach of 32 bits they are written through (g3_store16)
+__device__ __forceinline__ void rb_st8(uint16_t* base, size_t off, const float (&v)[8], int64_t ld, bool reach) {
     const u32x4 o = g3_pack8(v);
-    if ((ld & 7) == 0) *reinterpret_cast<u32x4*>(p) = o;
-    else reinterpret_cast<u32x2*>(p)[0] = u32x2{o.x, o.y}, reinterpret_cast<u32x2*>(p)[1] = u32x2{o.z, o.w};
+    if ((ld & 7) == 0 && reach) g3_store16(base, (uint32_t)off * 2, o);
+    else if ((ld & 7) == 0) *reinterpret_cast<u32x4*>(base + off) = o;
+    else reinterpret_cast<u32x2*>(base + off)[0] = u32x2{o.x, o.y}, reinterpret_cast<u32x2*>(base + off)[1] = u32x2{o.z, o.w};
 }
-__device__ __forceinline__ void rb_st8(float* p, const float (&v)[8], int64_t) {
-    reinterpret_cast<f32x4*>(p)[0] = f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p)[1] = f32x4{v[4], v[5], v[6], v[7]};
+__device__ __forceinline__ void rb_st8(float* base, size_t off, const float (&v)[8], int64_t, bool) {
+    reinterpret_cast<f32x4*>(base + off)[0] = f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(base + off)[1] = f32x4{v[4], v[5], v[6], v[7]};
 }
 
 // T: the storage, uint16_t (bf16: weights in MFMA tiles) or float (true 32-bit: weights in rows)
@@ -57,6 +58,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     // the tile by way of LDS (G3Out); rows of y: the token itself, or the pair in the token tile's place
     using Out = G3Out<C>;
     T* const y = reinterpret_cast<T*>(p.y);
+    const bool reach = !EXPERTS && (size_t)p.n * p.ldy < ((size_t)1 << 29); /* (experts' tiles leave at different times: 5.54 | 5.58 ms for 4 x 509 tokens) */
     auto row_of = [&](int tk) { return EXPERTS ? s_dst[EXPERTS ? tk : 0] : (t0 + tk < p.n ? t0 + tk : -1); };
     if (p.epilogue == KF_RB_GATED) {
         auto gated = [&](auto act) { /* a loop per activation: decided inside it costs a branch per value */
@@ -68,7 +70,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
                 Out::rows8(smem_raw, lt, c, tid, g), Out::rows8(smem_raw, lt, c + 2, tid, v);
 #pragma unroll
                 for (int j = 0; j < 8; j++) g[j] = scale * (rb_activate(act, g[j]) * v[j]);
-                rb_st8(y + (size_t)row * p.ldy + f, g, p.ldy);
+                rb_st8(y, (size_t)row * p.ldy + f, g, p.ldy, reach);
             });
         };
         if (p.act == KF_RB_SILU) gated(std::integral_constant<int, KF_RB_SILU>());
@@ -86,7 +88,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
                     v[j] = m + j >= p.act_lo && m + j < p.act_hi ? w : v[j];
                 }
             }
-            rb_st8(y + (size_t)row * p.ldy + m, v, p.ldy);
+            rb_st8(y, (size_t)row * p.ldy + m, v, p.ldy, reach);
         });
     } else {
         Out::template all<C::BM / 4>(acc, smem_raw, tid, [&](int tk, int lt, int u) {
@@ -103,7 +105,9 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
 #pragma unroll
                 for (int j = 0; j < 4; j++) d[j] = fmaf(p.alpha, r[j], d[j]);
             }
-            rb_st4(reinterpret_cast<float*>(p.y) + (size_t)row * p.ldy + m, d);
+            const size_t off = (size_t)row * p.ldy + m;
+            if (reach) g3_store16(p.y, (uint32_t)off * 4, __builtin_bit_cast(u32x4, d));
+            else rb_st4(reinterpret_cast<float*>(p.y) + off, d);
         });
     }
 }
