@@ -6,6 +6,7 @@
 //   * columns flattened over (token, head): any number of query heads per kv-head;
 //   * keys and values of the batch's own tokens read from the batch, older ones from the slot's ring: a prompt is attended to before its rows overwrite the ring;
 //   * only the tiles between a wave's first chunk start and its last position.
+// Heads of 64 or 128 whose values are as wide take the pipelined walk of kf_flash.h, tiles by loads into LDS (rb_attn_walk_kernel).
 // A decode row is one workgroup per (kv-head, key range): q and the new key are prepared in LDS, each of its four waves walks its own 32-key tiles (staged into LDS of its
 // own, no barrier in the walk) and the four partial softmaxes meet at the end.
 // fp32 storage, prompts with heads of multiples of 16 up to 128: the same scheme on 32-bit MFMAs.  Everything else: a plain form, one wave per (row, head), 32-bit throughout.
