@@ -12,13 +12,16 @@
 // workgroup owns (rows w, w + G, ... with G = min(rows, 512): fp64, in row order) and then over the G workgroups in a second launch (8 contiguous chunks of workgroups in index order, then the 8 chunk sums in order) -- a fixed
 // decomposition that oracle/kf_oracle.c kfo_norm_backward restates (the reference sums its blocks in index order too, in fp32).
 // HBM-bound: 3 reads + 1 write of rows*C bf16.  One workgroup owns whole rows: thread t holds the 8-column vectors t, t + 256, ... (C <= 8192).
+// Both launches together, us, with one row asked for ahead, factors by scalar loads and partials in column order | as it is now: LayerNorm 8192 x 1600 38.8 | 29.0 (in a training step 32.4 + 8.4 | 24.3 + 5.3;
+// 105 MB take about 20), 600 x 1600 23.7 | 14.2, 33100 x 1600 107 | 79, 8192 x 3072 55.0 | 42.5, 4096 x 5120 66.8 | 42.2, 4096 x 8192 95.6 | 68.8; RMS 8192 x 1600 27.2 | 23.7, 4096 x 8192 57.6 | 54.2.
 #include "kf_kernels.h"
 
 namespace kf {
 
+constexpr int NR_COLS = 32; /* sums of a workgroup of the second launch: weight and bias apart, 100 workgroups for 1600 columns (together, 50 of them with half the loads in flight took 8.4 us for 5.3) */
 constexpr int NB_MAXV = 4; /* 8-column vectors per thread: C <= 8192 */
 
-template <bool IS_LN, int NV>
+template <bool IS_LN, int NV, int DEPTH>
 __global__ void __launch_bounds__(256) norm_backward_kernel(uint16_t* __restrict__ dinp, const uint16_t* __restrict__ dout, const uint16_t* __restrict__ inp,
                                                             const uint16_t* __restrict__ weight, const float* __restrict__ mean, const float* __restrict__ rstd,
                                                             double* __restrict__ part, int rows, int C) {
@@ -40,10 +43,10 @@ __global__ void __launch_bounds__(256) norm_backward_kernel(uint16_t* __restrict
             dw[j][k] = 0.0;
             if (IS_LN) db[j][k] = 0.0;
         }
-    // the next row of this workgroup is requested (unconditionally: the last row re-reads itself) before the current one is reduced, so
-    // that a row costs its arithmetic and one barrier, not a memory round trip
-    u32x4 dov[NV], inv[NV], div[NV], ndo[NV], nin[NV], ndi[NV];
-    auto load_row = [&](int r, u32x4* a, u32x4* b, u32x4* c_) {
+    // DEPTH rows of this workgroup are on their way (unconditionally: past the last row the first one is read again) while one is reduced: two workgroups a CU with one row each ahead are 19 KB in flight,
+    // less than a memory round trip takes.  The rows' mean and 1/std stand in the lanes, 64 rows at a time: loaded per row they are scalar loads, whose wait is the LDS traffic's too, a round trip a row.
+    u32x4 ndo[DEPTH][NV], nin[DEPTH][NV], ndi[DEPTH][NV];
+    auto load_row = [&](int r, u32x4 (&a)[NV], u32x4 (&b)[NV], u32x4 (&c_)[NV]) {
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             const size_t o = (size_t)r * C + (size_t)(has[j] ? tid + 256 * j : 0) * 8;
@@ -52,23 +55,31 @@ __global__ void __launch_bounds__(256) norm_backward_kernel(uint16_t* __restrict
             c_[j] = *reinterpret_cast<const u32x4*>(dinp + o);
         }
     };
-    if ((int)blockIdx.x < rows) load_row(blockIdx.x, dov, inv, div);
+    float mean_l = 0.0f, rstd_l = 0.0f;
+    auto load_stats = [&](int r) { /* lane l: row r + l G */
+        const long rl = (long)r + (long)lane * G;
+        const int at = rl < rows ? (int)rl : r;
+        rstd_l = rstd[at];
+        if (IS_LN) mean_l = mean[at];
+        asm volatile("" ::"v"(rstd_l), "v"(mean_l)); /* waited for here, not at every row that reads them */
+    };
     int buf = 0;
-    for (int r = blockIdx.x; r < rows; r += G, buf ^= 1) {
+    auto row = [&](int r, int nth, u32x4 (&dov)[NV], u32x4 (&inv)[NV], u32x4 (&div)[NV]) {
         const size_t base = (size_t)r * C;
-        load_row(r + G < rows ? r + G : r, ndo, nin, ndi);
-        const float mean_r = IS_LN ? mean[r] : 0.0f, rstd_r = rstd[r];
+        const float mean_r = IS_LN ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mean_l), nth)) : 0.0f, rstd_r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, rstd_l), nth));
         double sa = 0.0, sb = 0.0;
 #pragma unroll
         for (int j = 0; j < NV; j++) {
-            if (!has[j]) continue;
+            if (NV > 2 && !has[j]) continue;
             const uint32_t wq[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w}, dq_[4] = {dov[j].x, dov[j].y, dov[j].z, dov[j].w}, iq[4] = {inv[j].x, inv[j].y, inv[j].z, inv[j].w};
+            double ta = sa, tb = sb;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const float d0 = bf_lo(wq[k]) * bf_lo(dq_[k]), d1 = bf_hi(wq[k]) * bf_hi(dq_[k]);
-                if (IS_LN) sa += (double)d0 + (double)d1;
-                sb += (double)(d0 * bf_lo(iq[k])) + (double)(d1 * bf_hi(iq[k]));
+                if (IS_LN) ta += (double)d0 + (double)d1;
+                tb += (double)(d0 * bf_lo(iq[k])) + (double)(d1 * bf_hi(iq[k]));
             }
+            if (has[j]) sa = ta, sb = tb; /* (lanes behind the last column hold the first ones: a branch round the arithmetic would make every load of the loop waited for at its end) */
         }
         sa = wave_sum_f64_fast(sa), sb = wave_sum_f64_fast(sb);
         if (lane == 0) red[buf][0][wave] = sa, red[buf][1][wave] = sb;
@@ -79,7 +90,7 @@ __global__ void __launch_bounds__(256) norm_backward_kernel(uint16_t* __restrict
         const float dnorm_norm_mean = IS_LN ? (float)B / (float)C * rstd_r - dnorm_mean * mean_r * rstd_r : (float)B / (float)C * rstd_r;
 #pragma unroll
         for (int j = 0; j < NV; j++) {
-            if (!has[j]) continue;
+            if (NV > 2 && !has[j]) continue;
             const uint32_t wq[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w}, dq_[4] = {dov[j].x, dov[j].y, dov[j].z, dov[j].w}, iq[4] = {inv[j].x, inv[j].y, inv[j].z, inv[j].w},
                            gq[4] = {div[j].x, div[j].y, div[j].z, div[j].w};
             uint32_t o[4];
@@ -101,20 +112,49 @@ __global__ void __launch_bounds__(256) norm_backward_kernel(uint16_t* __restrict
                 }
                 o[k] = pack_bf16x2(res[0], res[1]);
             }
-            *reinterpret_cast<u32x4*>(dinp + base + (size_t)(tid + 256 * j) * 8) = u32x4{o[0], o[1], o[2], o[3]};
+            if (has[j]) *reinterpret_cast<u32x4*>(dinp + base + (size_t)(tid + 256 * j) * 8) = u32x4{o[0], o[1], o[2], o[3]};
         }
+        buf ^= 1;
+    };
+    const int first = blockIdx.x; /* G <= rows */
+    const int mine = (rows - 1 - first) / G + 1; /* rows of this workgroup: first + i G */
+    auto ask = [&](int i, int u) { load_row(first + (i < mine ? i : 0) * G, ndo[u], nin[u], ndi[u]); };
+    load_stats(first);
+    if constexpr (NV > 2) { /* rows of that many registers: the next one is asked for before the present one is reduced (as below, 4096 x 5120 RMS took 42 us for 38: one workgroup a CU) */
+        ask(0, 0);
+        for (int i = 0; i < mine; i++) {
+            if (i && (i & 63) == 0) load_stats(first + i * G);
+            ask(i + 1, 1);
+            row(first + i * G, i & 63, ndo[0], nin[0], ndi[0]);
 #pragma unroll
-        for (int j = 0; j < NV; j++) dov[j] = ndo[j], inv[j] = nin[j], div[j] = ndi[j];
+            for (int j = 0; j < NV; j++) ndo[0][j] = ndo[1][j], nin[0][j] = nin[1][j], ndi[0][j] = ndi[1][j];
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < DEPTH; u++) ask(u, u);
+        int i = 0;
+        for (; i + DEPTH <= mine; i += DEPTH) {
+            if (i && (i & 63) == 0) load_stats(first + i * G);
+#pragma unroll
+            for (int u = 0; u < DEPTH; u++) {
+                row(first + (i + u) * G, (i + u) & 63, ndo[u], nin[u], ndi[u]);
+                ask(i + u + DEPTH, u); /* into the registers that the row has left: asked for earlier, it would land in others and wait to be moved */
+            }
+        }
+        if (i && i < mine && (i & 63) == 0) load_stats(first + i * G);
+#pragma unroll
+        for (int u = 0; u < DEPTH - 1; u++)
+            if (i + u < mine) row(first + (i + u) * G, (i + u) & 63, ndo[u], nin[u], ndi[u]);
     }
-    // this workgroup's column partials: part[blockIdx.x][{dw, db}][C] fp64
+    // this workgroup's column partials: part[blockIdx.x][{dw, db}][8][C / 8] fp64, column c = 8 v + k at [k][v]: a wave's stores are whole lines (in column order each lane's eight lie 64 bytes from its neighbour's)
     double* pw = part + (size_t)blockIdx.x * (IS_LN ? 2 : 1) * C;
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         if (!has[j]) continue;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            pw[(size_t)(tid + 256 * j) * 8 + k] = dw[j][k];
-            if (IS_LN) pw[C + (size_t)(tid + 256 * j) * 8 + k] = db[j][k];
+            pw[(size_t)k * nvec + tid + 256 * j] = dw[j][k];
+            if (IS_LN) pw[C + (size_t)k * nvec + tid + 256 * j] = db[j][k];
         }
     }
 }
@@ -203,8 +243,8 @@ __global__ void __launch_bounds__(256) norm_backward_narrow_kernel(uint16_t* __r
                 tw += red[w2][rr * LPR + l0][k];
                 if (IS_LN) tb += red[w2][rr * LPR + l0][8 + k];
             }
-        pw[c] = tw;
-        if (IS_LN) pw[C + c] = tb;
+        pw[k * (C >> 3) + l0] = tw;
+        if (IS_LN) pw[C + k * (C >> 3) + l0] = tb;
     }
 }
 
@@ -212,37 +252,32 @@ __global__ void __launch_bounds__(256) norm_backward_narrow_kernel(uint16_t* __r
 // sums added in chunk order -- then bf16(fp32 sum + old gradient).  (One thread walking all G partials is a chain of G dependent loads.)
 __global__ void __launch_bounds__(256) norm_backward_reduce_kernel(uint16_t* __restrict__ dweight, uint16_t* __restrict__ dbias, const double* __restrict__ part,
                                                                    int G, int C, int is_ln) {
-    __shared__ double sw_[8][32], sb_[8][32];
-    const int cl = threadIdx.x & 31, q = threadIdx.x >> 5;
-    const int c = blockIdx.x * 32 + cl;
-    const size_t stride = (size_t)(is_ln ? 2 : 1) * C;
+    __shared__ double s_[8][NR_COLS];
+    const int cl = threadIdx.x & (NR_COLS - 1), q = threadIdx.x / NR_COLS; /* place of the partials' order, chunk of workgroups */
+    const int at = blockIdx.x * NR_COLS + cl; /* places of dw, then (LayerNorm) of db */
+    const int all = is_ln ? 2 * C : C;
     const int chunk = (G + 7) / 8, g0 = q * chunk, g1 = g0 + chunk < G ? g0 + chunk : G;
-    double sw = 0.0, sbias = 0.0;
-    if (c < C) { /* the same index order, eight partials' loads in flight at a time (one at a time this launch took 24 us for 512 partials of 1600 columns) */
+    double s = 0.0;
+    if (at < all) { /* the same index order, 16 partials' loads in flight at a time */
         int g = g0;
-        for (; g + 8 <= g1; g += 8) {
-            double vw[8], vb[8];
+        for (; g + 16 <= g1; g += 16) {
+            double v[16];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                vw[u] = part[(g + u) * stride + c];
-                vb[u] = is_ln ? part[(g + u) * stride + C + c] : 0.0;
-            }
+            for (int u = 0; u < 16; u++) v[u] = part[(size_t)(g + u) * all + at];
 #pragma unroll
-            for (int u = 0; u < 8; u++) sw += vw[u], sbias += vb[u];
+            for (int u = 0; u < 16; u++) s += v[u];
         }
-        for (; g < g1; g++) {
-            sw += part[g * stride + c];
-            if (is_ln) sbias += part[g * stride + C + c];
-        }
+        for (; g < g1; g++) s += part[(size_t)g * all + at];
     }
-    sw_[q][cl] = sw, sb_[q][cl] = sbias;
+    s_[q][cl] = s;
     __syncthreads();
-    if (q == 0 && c < C) {
-        double tw = 0.0, tb = 0.0;
+    if (q == 0 && at < all) {
+        double t = 0.0;
 #pragma unroll
-        for (int k = 0; k < 8; k++) tw += sw_[k][cl], tb += sb_[k][cl];
-        dweight[c] = f2bf((float)tw + bf2f(dweight[c]));
-        if (is_ln && dbias) dbias[c] = f2bf((float)tb + bf2f(dbias[c]));
+        for (int k = 0; k < 8; k++) t += s_[k][cl];
+        const int p = at < C ? at : at - C, nvec = C >> 3, c = 8 * (p % nvec) + p / nvec;
+        uint16_t* const d = at < C ? dweight : dbias;
+        if (d) d[c] = f2bf((float)t + bf2f(d[c]));
     }
 }
 
@@ -257,13 +292,13 @@ int norm_backward_launch(hipStream_t st, uint16_t* dinp, uint16_t* dweight, uint
         const int lpr_log2 = __builtin_ctz(C) - 3;
         if (ln) hipLaunchKernelGGL((norm_backward_narrow_kernel<true>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C, lpr_log2);
         else hipLaunchKernelGGL((norm_backward_narrow_kernel<false>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C, lpr_log2);
-        hipLaunchKernelGGL(norm_backward_reduce_kernel, dim3((C + 31) / 32), dim3(256), 0, st, dweight, dbias, scratch, G, C, ln ? 1 : 0);
+        hipLaunchKernelGGL(norm_backward_reduce_kernel, dim3(((ln ? 2 : 1) * C + NR_COLS - 1) / NR_COLS), dim3(8 * NR_COLS), 0, st, dweight, dbias, scratch, G, C, ln ? 1 : 0);
         return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
     }
 #define KF_NB_GO(NV)                                                                                                                             \
     do {                                                                                                                                         \
-        if (ln) hipLaunchKernelGGL((norm_backward_kernel<true, NV>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C); \
-        else hipLaunchKernelGGL((norm_backward_kernel<false, NV>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C);   \
+        if (ln) hipLaunchKernelGGL((norm_backward_kernel<true, NV, NV == 1 ? 4 : 2>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C); \
+        else hipLaunchKernelGGL((norm_backward_kernel<false, NV, NV == 1 ? 4 : 2>), dim3(G), dim3(256), 0, st, dinp, dout, inp, weight, mean, rstd, scratch, rows, C);   \
     } while (0)
     switch (nv) {
         case 1: KF_NB_GO(1); break;
@@ -272,7 +307,7 @@ int norm_backward_launch(hipStream_t st, uint16_t* dinp, uint16_t* dweight, uint
         default: KF_NB_GO(4); break;
     }
 #undef KF_NB_GO
-    hipLaunchKernelGGL(norm_backward_reduce_kernel, dim3((C + 31) / 32), dim3(256), 0, st, dweight, dbias, scratch, G, C, ln ? 1 : 0);
+    hipLaunchKernelGGL(norm_backward_reduce_kernel, dim3(((ln ? 2 : 1) * C + NR_COLS - 1) / NR_COLS), dim3(8 * NR_COLS), 0, st, dweight, dbias, scratch, G, C, ln ? 1 : 0);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 
