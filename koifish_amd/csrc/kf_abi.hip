@@ -1506,7 +1506,8 @@ int kfdbg_set_knob(const char* name, long value) {
     else if (!strcmp(name, "attn_gq_split")) k.attn_gq_split = (int)value;
     else if (!strcmp(name, "g3_mid_min")) k.g3_mid_min = (int)value;
     else if (!strcmp(name, "resident_min")) k.resident_min = (int)value;
-    else if (!strcmp(name, "attn_parts_max")) k.attn_parts_max = (int)value;
+    else if (!strcmp(name, "attn_pair_min")) k.attn_pair_min = (int)value;
+    else if (!strcmp(name, "attn_walk_min")) k.attn_walk_min = (int)value;
     else return -1;
     return 0;
 }

@@ -3,8 +3,9 @@
 //   O^T[d][col]  += sum_key V^T[d][key] P^T[key][col]   the S^T registers, packed to bf16, ARE the B operand (slot (step s, half h, j) <-> key 16 s + (j & 3) + 8 (j >> 2) + 4 h on both operands);
 //      A = V^T fragments straight from the row-major V tile (ds_read_b64_tr_b16).  p enters as a bf16 pair (high part + remainder, ~16 significant bits), its sum stays fp32.
 // What bounds it: a tile's MFMAs take 768 cycles of a SIMD at dim 128, its vector instructions about as many, and one after the other they leave both pipes idle half the time -- a SIMD has two
-// waves at most here, often one.  So the walk is a pipeline: beside the exponentials of tile t run the MFMAs of the scores of tile t + 1, beside the P.V of tile t the scaling and the maximum of
-// tile t + 1 (order() below).  And the running maximum of a column is moved only when a tile's exceeds it by 8 (log2): up to there p just grows to 2^8, which costs no precision in
+// waves at most here, often one.  So a step holds a tile's exponentials and P.V beside the next tile's scores, their scaling and maximum: independent instructions that the compiler mixes.
+// A column's reference exponent M: NAT (scores in natural units, as they were stored) is the maximum of the keys seen so far, subtracted before the factor log2 e, so that the largest p is 1 whatever the scores'
+// size, and a sum does not depend on the tiles' way through LDS.  Otherwise (scores in log2 units) it is moved only when a tile's maximum exceeds it by 8: up to there p just grows to 2^8, which costs no precision in
 // fp32 and bf16 pairs, and the accumulator is rescaled a few times per column instead of at nearly every early tile.
 #pragma once
 #include "kf_device.h"
@@ -15,13 +16,13 @@ typedef __bf16 fl_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 fl_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr float FL_SLACK = 8.0f; /* log2 */
+constexpr float FL_SLACK = 8.0f, FL_LOG2E = 1.44269502162933349609375f;
 
-template <int HD>
+template <int HD, bool NAT>
 struct FlashWave {
     static constexpr int NS = HD / 16, NDB = HD / 32; /* MFMA steps over d of S^T; 32-row blocks of O^T */
     fl_f32x16 o[NDB];
-    float M, l; /* the column's reference exponent (log2 units; -inf: nothing seen) and this lane's half of the sum of p */
+    float M, l; /* the column's reference exponent (units of the scores; -inf: nothing seen) and this lane's half of the sum of p */
     u32x4 qf[NS];
     __device__ __forceinline__ void init() {
 #pragma unroll
@@ -65,10 +66,11 @@ struct FlashWave {
         }
         return mt;
     }
-    // mt: the column's maximum over the tile in log2 units (both lanes of the pair)
+    static __device__ __forceinline__ float power(float d) { return __builtin_amdgcn_exp2f(NAT ? d * FL_LOG2E : d); } /* of a difference of scores */
+    // mt: the column's maximum over the tile (both lanes of the pair)
     __device__ __forceinline__ void move(float mt) {
-        if (mt > M + FL_SLACK) {
-            const float alpha = __builtin_amdgcn_exp2f(M - mt); /* M = -inf on the first tile: 0 */
+        if (mt > (NAT ? M : M + FL_SLACK)) {
+            const float alpha = power(M - mt); /* M = -inf on the first tile: 0 */
             l *= alpha;
 #pragma unroll
             for (int db = 0; db < NDB; db++)
@@ -77,14 +79,12 @@ struct FlashWave {
             M = mt;
         }
     }
-    // p = 2^(LOG2E score - M) as bf16 pairs; scores in natural units where NAT, in log2 units otherwise.  A column that has seen nothing (M = -inf): p = 0
-    template <bool NAT>
+    // p = 2^(score - M) or e^(score - M) as bf16 pairs.  A column that has seen nothing (M = -inf): p = 0
     __device__ __forceinline__ void weights(const fl_f32x16& st, uint32_t (&ph)[8], uint32_t (&pl)[8]) {
         const float ref = M == -__builtin_inff() ? 0.f : M;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float a = st[2 * i], b = st[2 * i + 1];
-            const float p0 = __builtin_amdgcn_exp2f(NAT ? fmaf(a, 1.44269502162933349609375f, -ref) : a - ref), p1 = __builtin_amdgcn_exp2f(NAT ? fmaf(b, 1.44269502162933349609375f, -ref) : b - ref);
+            const float p0 = power(st[2 * i] - ref), p1 = power(st[2 * i + 1] - ref);
             l += p0;
             l += p1;
             ph[i] = pack_bf16x2(p0, p1);
@@ -105,16 +105,15 @@ struct FlashWave {
             }
         }
     }
-    // one tile of the pipeline: its scores are in `cur` (scaled, masked; mt their maximum in log2 units), those of the tile behind it come out in `nxt` (scaled; the result: this lane's maximum)
-    template <bool ROUND, bool NAT, class KF, class VF>
+    // one tile of the pipeline: its scores are in `cur` (scaled, masked; mt their maximum), those of the tile behind it come out in `nxt` (scaled; the result: this lane's maximum)
+    template <bool ROUND, class KF, class VF>
     __device__ __forceinline__ float tile(fl_f32x16& cur, float mt, fl_f32x16& nxt, float by, KF&& kfrag, VF&& vfrag) {
         move(mt);
         uint32_t ph[8], pl[8];
         scores(nxt, kfrag);
-        weights<NAT>(cur, ph, pl);
+        weights(cur, ph, pl);
         accumulate(ph, pl, vfrag);
-        const float m = scale<ROUND>(nxt, by);
-        return m;
+        return scale<ROUND>(nxt, by);
     }
 };
 

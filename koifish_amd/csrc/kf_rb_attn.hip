@@ -595,7 +595,7 @@ __global__ void __launch_bounds__(256 * KH, HD <= 128 ? 2 : 1) rb_attn_prefill_k
 // sequences of 300 25.9 | 22.6, of 509 with 20 heads on 4 52.4 | 43.0
 template <int HD>
 __global__ void __launch_bounds__(256, 2) rb_attn_walk_kernel(const kf_rb_attention a, const int32_t* __restrict__ seqs) {
-    using Wave = FlashWave<HD>;
+    using Wave = FlashWave<HD, false>;
     using Tile = ApTile<HD>;
     constexpr int NI = Tile::PART / 4096, SET = 2 * Tile::PART; /* load instructions per wave and part; bytes of a K and a V tile */
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(256, 2) rb_attn_walk_kernel(const kf_rb_attent
     };
     auto step = [&](int t, fl_f32x16& cur, fl_f32x16& nxt) {
         turn_to(t, [&](const unsigned char* k, const unsigned char* v) __attribute__((always_inline)) {
-            mt = W.template tile<false, false>(cur, mt, nxt, sc2, [&](int s) { return T.k(k, s); }, [&](int s2, int db) { return T.v(v, s2, db); });
+            mt = W.template tile<false>(cur, mt, nxt, sc2, [&](int s) { return T.k(k, s); }, [&](int s2, int db) { return T.v(v, s2, db); });
             mt = maximum(nxt, t + 1, mt);
         });
     };

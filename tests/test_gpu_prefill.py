@@ -155,35 +155,71 @@ def test_attn_prefill_long_prompt_form_vs_oracle(ctx, nh, nkv, hd, pos0, n):
     assert not (out == 0x4040).all(axis=1).any()
 
 
-@pytest.mark.parametrize("nh,nkv,hd,pos0,n", [(4, 2, 128, 0, 8), (4, 2, 128, 100, 33), (2, 2, 64, 90, 65), (8, 1, 128, 129, 127), (16, 4, 64, 0, 513), (4, 2, 128, 511, 130), (16, 2, 128, 3, 640)])
-@pytest.mark.parametrize("form", ["all keys", "halves", "quarters"])
-def test_every_split_of_the_keys_against_64_bits(ctx, form, nh, nkv, hd, pos0, n):
-    """Keys whose scores climb with the position, so that a column's running maximum moves past its slack again and again, some far below it; every dot is exact in fp32 (small multiples of 1/8), so the bf16
-    scores are the reference's own and only p (a bf16 pair, 2^-16), the sums (fp32) and one bf16 store of out differ: 2^-8 of a value, and half of that again for the sums"""
-    import ctypes as C
-    import torch
-    g = torch.Generator().manual_seed(7 * n + hd)
-    tot, GQ = pos0 + n, nh // nkv
-    q = torch.randint(-1, 2, (n, nh, hd), generator=g).float()
-    k = torch.randint(-1, 2, (tot, nkv, hd), generator=g).float() * 2
-    q[..., 0], k[..., 0] = 8.0, ((torch.arange(tot) % 251) / 8)[:, None]   # multiples of 1/8 below 32: eight bits
-    v = torch.randn(tot, nkv, hd, generator=g).bfloat16()
-    dots = torch.einsum("thd,skd->thsk", q.double(), k.double())
-    dots = torch.stack([dots[:, h, :, h // GQ] for h in range(nh)], 1)                            # [n, nh, tot]
-    s = (dots.float() * torch.tensor(1.0 / hd ** 0.5, dtype=torch.float32)).bfloat16().double()
-    s.masked_fill_(torch.arange(tot)[None, None] > (pos0 + torch.arange(n))[:, None, None], -float("inf"))
-    ref = torch.einsum("ths,shd->thd", torch.softmax(s, -1), v.double().repeat_interleave(GQ, 1))
-    wgs = (n * GQ + 127) // 128 * nkv
-    knob = {"all keys": 0, "halves": wgs // 2 if wgs > 1 else 0, "quarters": 4096}[form]
-    qd, kd, vd = (t.bfloat16().reshape(t.shape[0], -1).to(ctx.device) for t in (q, k, v))
-    buf = torch.full((n + 2, nh * hd), 3.0, dtype=torch.bfloat16, device=ctx.device)
+FORMS = {"registers": (1 << 30, 1 << 30), "loads into LDS": (1 << 30, 0), "halves": (0, 1 << 30)}   # all keys staged through registers, by loads into LDS; two key halves
+
+
+def _attention_in_form(ctx, form, q, k, v, out, pos0, n, n_seq, nh, nkv, hd):
+    pair, walk = FORMS[form]
     try:
-        assert ctx.hip.kfdbg_set_knob(b"attn_parts_max", knob) == 0
-        rc = ctx.hip.kf_attn_prefill(ctx.h, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), buf[1:].data_ptr(), pos0, n, nh * hd, nh, nkv, hd, nkv * hd)
+        assert ctx.hip.kfdbg_set_knob(b"attn_pair_min", pair) == 0 and ctx.hip.kfdbg_set_knob(b"attn_walk_min", walk) == 0
+        if n_seq == 1:
+            rc = ctx.hip.kf_attn_prefill(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), pos0, n, nh * hd, nh, nkv, hd, nkv * hd)
+        else:
+            rc = ctx.hip.kf_attn_prefill_batch(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n, nh * hd, nh, nkv, hd, nkv * hd, n_seq)
         assert rc == 0, ctx.hip.kf_last_error()
         ctx.sync()
     finally:
-        ctx.hip.kfdbg_set_knob(b"attn_parts_max", 256)
-    got = buf[1:n + 1].cpu().double().reshape(n, nh, hd)
+        ctx.hip.kfdbg_set_knob(b"attn_pair_min", 256), ctx.hip.kfdbg_set_knob(b"attn_walk_min", 512)
+
+
+# the last three: several sequences, every query head its own kv-head
+SPLITS = [(4, 2, 128, 0, 8, 1), (4, 2, 128, 100, 33, 1), (2, 2, 64, 90, 65, 1), (8, 1, 128, 129, 127, 1), (16, 4, 64, 0, 513, 1), (4, 2, 128, 511, 130, 1), (16, 2, 128, 3, 640, 1),
+          (2, 2, 64, 0, 515, 3), (2, 2, 128, 0, 600, 2), (4, 2, 64, 0, 70, 3)]
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,n,n_seq", SPLITS)
+@pytest.mark.parametrize("form", list(FORMS))
+def test_every_form_of_the_attention_against_64_bits(ctx, form, nh, nkv, hd, pos0, n, n_seq):
+    """Keys whose scores climb with the position, so that a column's running maximum moves again and again, some far below it; every dot is exact in fp32 (small multiples of 1/8), so the bf16
+    scores are the reference's own and only p (a bf16 pair, 2^-16), the sums (fp32) and one bf16 store of out differ: 2^-8 of a value, and half of that again for the sums.  Over all keys the two ways
+    of staging give the same bits."""
+    import torch
+    g = torch.Generator().manual_seed(7 * n + hd)
+    tot, GQ = pos0 + n, nh // nkv
+    q = torch.randint(-1, 2, (n_seq, n, nh, hd), generator=g).float()
+    k = torch.randint(-1, 2, (n_seq, tot, nkv, hd), generator=g).float() * 2
+    q[..., 0], k[..., 0] = 8.0, ((torch.arange(tot) % 251) / 8)[:, None]   # multiples of 1/8 below 32: eight bits
+    v = torch.randn(n_seq, tot, nkv, hd, generator=g).bfloat16()
+    dots = torch.einsum("zthd,zshd->zths", q.double(), k.double().repeat_interleave(GQ, 2))   # [n_seq, n, nh, tot]
+    s = (dots.float() * torch.tensor(1.0 / hd ** 0.5, dtype=torch.float32)).bfloat16().double()
+    s.masked_fill_(torch.arange(tot)[None, None] > (pos0 + torch.arange(n))[:, None, None], -float("inf"))
+    ref = torch.einsum("zths,zshd->zthd", torch.softmax(s, -1), v.double().repeat_interleave(GQ, 2))
+    qd, kd, vd = (t.bfloat16().reshape(n_seq * t.shape[1], -1).to(ctx.device) for t in (q, k, v))
+    buf = torch.full((n_seq * n + 2, nh * hd), 3.0, dtype=torch.bfloat16, device=ctx.device)
+    _attention_in_form(ctx, form, qd, kd, vd, buf[1:], pos0, n, n_seq, nh, nkv, hd)
+    got = buf[1:n_seq * n + 1].cpu().double().reshape(n_seq, n, nh, hd)
     assert float((got - ref).abs().max()) <= 1.5 * 2.0 ** -8 * float(ref.abs().max())
-    assert bool((buf[0] == 3).all()) and bool((buf[n + 1] == 3).all())
+    assert bool((buf[0] == 3).all()) and bool((buf[n_seq * n + 1] == 3).all())
+    if form == "loads into LDS":
+        again = torch.zeros_like(buf)
+        _attention_in_form(ctx, "registers", qd, kd, vd, again[1:], pos0, n, n_seq, nh, nkv, hd)
+        assert torch.equal(again[1:-1].view(torch.int16), buf[1:-1].view(torch.int16))
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("nh,nkv,hd,n", [(2, 1, 128, 300), (2, 2, 64, 530)])
+def test_attention_with_scores_far_beyond_the_exponents(ctx, form, nh, nkv, hd, n):
+    """scores of 1e4 to 1e14, each key's a bf16 of its own: the softmax is one-hot at the largest key that a query sees, whatever the size (the maximum is subtracted before anything is multiplied)"""
+    import torch
+    g = torch.Generator().manual_seed(n)
+    rank = torch.randperm(n, generator=g)
+    q = torch.zeros(n, nh, hd)
+    k = torch.zeros(n, nkv, hd)
+    q[..., 0] = 2.0 ** 20
+    k[..., 0] = ((128 + rank % 128).float() * 2.0 ** (4 * (rank // 128) - 7))[:, None]   # eight bits; climbs with the rank
+    v = torch.randn(n, nkv, hd, generator=g).bfloat16()
+    qd, kd, vd = (t.bfloat16().reshape(n, -1).to(ctx.device) for t in (q, k, v))
+    out = torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=ctx.device)
+    _attention_in_form(ctx, form, qd, kd, vd, out, 0, n, 1, nh, nkv, hd)
+    best = torch.stack([rank[:t + 1].argmax() for t in range(n)])
+    assert torch.equal(out.cpu().reshape(n, nh, hd), v[best].repeat_interleave(nh // nkv, 1))
