@@ -216,7 +216,7 @@ def test_attention_with_scores_far_beyond_the_exponents(ctx, form, nh, nkv, hd, 
     q = torch.zeros(n, nh, hd)
     k = torch.zeros(n, nkv, hd)
     q[..., 0] = 2.0 ** 20
-    k[..., 0] = ((128 + rank % 128).float() * 2.0 ** (4 * (rank // 128) - 7))[:, None]   # eight bits; climbs with the rank
+    k[..., 0] = ((64 + rank % 64).float() * 2.0 ** (4 * (rank // 64) - 6))[:, None]   # seven bits, so no two scores are one bf16; climbs with the rank
     v = torch.randn(n, nkv, hd, generator=g).bfloat16()
     qd, kd, vd = (t.bfloat16().reshape(n, -1).to(ctx.device) for t in (q, k, v))
     out = torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=ctx.device)
