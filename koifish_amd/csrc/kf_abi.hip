@@ -419,9 +419,10 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         kf_weight wb;
         memset(&wb, 0, sizeof(wb));
         wb.data = (char*)c->scratch + e.off, wb.type = KF_BF16, wb.ne0 = w->ne0, wb.ne1 = w->ne1;
-        // split-K slots behind the copies, from K = 6144: below it the copies, just written, are still in the caches, and whole tiles of one round are the faster ones (gemm3_launch has the figures)
+        // split-K slots behind the copies, from K = 3072.  Below it the copies, just written, are still in the caches, and pieces give less than on resident ones (0.6B, us per layer, whole | three pieces: 320
+        // rows 111 | 105, 1024 rows 134 | 130, 2047 rows 187 | 185; resident: kf_gemm3.hip) -- not enough to change the sums of every prompt
         const size_t slots = kf::gemm3_sk_ws_bytes();
-        void* const lent = w->ne1 >= 6144 ? c->scratch_end(slots) : nullptr;
+        void* const lent = w->ne1 >= 3072 ? c->scratch_end(slots) : nullptr;
         const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, lent, slots);
         if (rc < 0) return fail(rc, "kf_linear (bf16 tile GEMM on the layer's copy) failed with %d", rc);
         if (rc == KF_OK) return KF_OK;

@@ -349,6 +349,25 @@ void gemm3_sk_forget(void* ws) { /* something else was (or will be) written wher
         if (p == flags) p = nullptr;
 }
 
+// Whether nwg tiles of C go in k-pieces, and how (P, S, kp, R; the number of workgroups): when they are fewer than 4/5 of the resident workgroups and the pieces stay >= 512 deep in k; a K-contiguous product of
+// K < 3072 (KM: either operand k-major) only where three pieces of every tile find room.  us per layer of prompts on resident copies, never | from K = 3072 | three pieces: 0.6B 320 rows 134 | 116 | 106, 1024 rows
+// 149 | 143 | 137, 2047 rows 198 | 190 | 187; 1.7B 320 rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800 rows 325 -> 332 us.
+template <bool KM, class C>
+static bool g3_cut(long nwg, int nkt, G3SkArgs& s, int& nlaunch) {
+    const int G = 256 * C::WGS_PER_CU, min_steps = 512 / G3_BK;
+    if (5 * nwg >= 4 * G || !(KM || 3 * nwg <= G || nkt >= 48)) return false;
+    s.P = (int)nwg, s.S = G / s.P, s.kp = 0, s.R = 1;
+    if (s.S >= 2) {
+        while (s.S > 1 && nkt / s.S < min_steps) s.S--;
+        nlaunch = s.P * s.S;
+        return s.S >= 2;
+    }
+    s.kp = (int)(((long long)nkt * s.P + G / 2) / G);
+    nlaunch = G;
+    const long long T = (long long)s.P * (nkt - s.kp);
+    s.R = (int)((T + (G - s.P) - 1) / (G - s.P));
+    return nkt - s.kp >= 1 && nkt >= 4 * min_steps && T * 2 < (1LL << 31) && s.kp > 0;
+}
 // KF_OK launched, 1 = not for this kernel (the caller's other tile kernels take the shape), < 0 error.  bf16 "weights" only: quantised ones are dequantised first.
 // BK = 32 (4 LDS buffers, three steps in flight) was measured 8-10 % slower than BK = 64 (2 buffers) on every shape, forward and backward: the per-step costs
 // (barrier, counted wait, loop) double, and the loop is not waiting for memory.  Only BK = 64 is instantiated.
@@ -361,34 +380,16 @@ static int g3_go_c(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t
         if (hipFuncSetAttribute((const void*)gemm3_sk_kernel<AKM, BKM, BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
-    // split-K when the tiles are fewer than 4/5 of the resident workgroups, the caller lent the workspace, and the pieces stay >= 512 deep in k; a K-contiguous product of K < 3072 only where three pieces of
-    // every tile find room.  us per layer of prompts on resident copies, never | from K = 3072 | three pieces: 0.6B 320 rows 134 | 116 | 106, 1024 rows 149 | 143 | 137, 2047 rows 198 | 190 | 187; 1.7B 320
-    // rows 196 | 165 | 156.  Two pieces below K = 3072: 16 prompts of 131 tokens 6.12 -> 6.18 ms; a piece and tails: 1.7B at 1800 rows 325 -> 332 us.  Of one 128 x 128 tile to a CU a piece and tails pay up to two
-    // thirds of the CUs (K 6144: 144 tiles 64.9 -> 50.5 us; K 8192: 200 tiles 68.6 -> 78.9), beyond at K >= 16384 (25600: 200 tiles 227 -> 208)
-    const int G = 256 * C::WGS_PER_CU, nkt = a.K / BK, min_steps = 512 / BK;
-    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nwg < 4 * G && (AKM || BKM || 3 * nwg <= G || (nkt >= 48 && (C::WGS_PER_CU > 1 || 3 * nwg < 2 * G || nkt >= 256)))) {
-        G3SkArgs s;
+    G3SkArgs s;
+    int nlaunch;
+    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && g3_cut<AKM || BKM, C>(nwg, a.K / BK, s, nlaunch)) {
         // the flags live in the LAST 8 KiB of the lent workspace whatever the tile configuration (behind the partial tiles of THIS configuration they would move with it,
         // and another configuration's fp32 partials could overwrite words already marked "seen" with values that pass for an epoch)
         static_assert((size_t)256 * C::WGS_PER_CU * C::BM * C::BN * 4 <= (size_t)256 * G3_BM * G3_BN * 4 && 256 * C::WGS_PER_CU * 4 <= G3_SK_FLAG_BYTES, "partials and flags fit the lent workspace");
         s.ws = (float*)ws, s.flags = (uint32_t*)((char*)ws + gemm3_sk_ws_bytes() - G3_SK_FLAG_BYTES);
-        s.P = (int)nwg, s.S = G / s.P, s.kp = 0, s.R = 1;
-        int nlaunch;
-        if (s.S >= 2) {
-            while (s.S > 1 && nkt / s.S < min_steps) s.S--;
-            nlaunch = s.P * s.S;
-        } else {
-            s.kp = (int)(((long long)nkt * s.P + G / 2) / G);
-            nlaunch = G;
-            const long long T = (long long)s.P * (nkt - s.kp);
-            s.R = (int)((T + (G - s.P) - 1) / (G - s.P));
-            if (nkt - s.kp < 1 || nkt < 4 * min_steps || T * 2 >= (1LL << 31)) s.S = 0;
-        }
-        if (s.S >= 1 && (s.S >= 2 || s.kp > 0)) {
-            if (g3_sk_epoch(st, s.flags, G, &s.epoch) != KF_OK) return KF_HIP_CHECK;
-            hipLaunchKernelGGL((gemm3_sk_kernel<AKM, BKM, BK, C>), dim3(nlaunch), dim3(C::NTH), SMEM, st, a, s);
-            return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
-        }
+        if (g3_sk_epoch(st, s.flags, 256 * C::WGS_PER_CU, &s.epoch) != KF_OK) return KF_HIP_CHECK;
+        hipLaunchKernelGGL((gemm3_sk_kernel<AKM, BKM, BK, C>), dim3(nlaunch), dim3(C::NTH), SMEM, st, a, s);
+        return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
     }
     if (nwg < min_plain) return 1;
     hipLaunchKernelGGL((gemm3_kernel<AKM, BKM, BK, C>), dim3((unsigned)nwg), dim3(C::NTH), SMEM, st, a);
@@ -426,18 +427,20 @@ int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws
     const int nkt = a.K / G3_BK;
     const long n128 = g3_tiles_of(a.M, a.n, 128, 128), n64 = g3_tiles_of(a.M, a.n, 64, 64);
     if (n128 < 32 && n64 < 64) return 1;
-    // resident copies lend the workspace at every K: k-pieces of 64 x 64 and 64 x 128 tiles (g3_go_c says when; a partial is 16 or 32 KiB -- the 64 KiB ones of a 128 x 128 tile cost what they give at these K)
-    if (ws && nkt < 96 && n128 < 256) {
+    // Where the workspace is lent (resident copies, and a layer's own from K = 3072): k-pieces of 64 x 128 or 64 x 64 tiles, when g3_cut says so (a partial is 16 or 32 KiB; the 64 KiB ones of a 128 x 128 tile cost what
+    // they give at K <= 3072).  Which products are cut, and where, is part of their result, and stays: k-pieces of 128 x 128 tiles on 8 waves are faster from K = 6144 on (us at 515 rows, these | those: M 2048 x K 6144 35.5 | 28.6,
+    // 5120 x 8192 98 | 56, 5120 x 25600 344 | 191), but their sums are others, and a 1.7B or 32B prompt in 4 bits is then farther from itself than its error allows
+    if (ws && ws_bytes >= gemm3_sk_ws_bytes() && n128 < 256) {
         const long nmid = g3_tiles_of(a.M, a.n, 64, 128);
-        return nmid >= 192 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 64) : g3_go_c<false, false, G3Tiny>(st, a, n64, ws, ws_bytes, 64);
+        G3SkArgs s;
+        int nl;
+        if (nmid >= 192 ? g3_cut<false, G3Mid>(nmid, nkt, s, nl) : g3_cut<false, G3Tiny>(n64, nkt, s, nl))
+            return nmid >= 192 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 1) : g3_go_c<false, false, G3Tiny>(st, a, n64, ws, ws_bytes, 1);
     }
-    // Otherwise the smallest tile that makes ONE round of the CUs (g3_pick; in front of it 64 x 64: up to two side by side, from K = 6144 one, or k-pieces).  us with a residual, 64 x 64 | 64 x 128 (three buffers) | 128 x 128 on 8 waves |
+    // Otherwise the smallest tile that makes ONE round of the CUs (g3_pick; in front of it 64 x 64: up to two side by side, from K = 6144 one).  us with a residual, 64 x 64 | 64 x 128 (three buffers) | 128 x 128 on 8 waves |
     // 128 x 256 | 128 x 128 on 4 waves:  M 1024 x K 2048 at 515 rows 12.5 | 17.4 | 20.7 | 31.0 | 28.3, at 2047 rows 18.0 | 18.5 | 21.4 | 32.0 | 29.2, at 2608 rows (656 tiles) 22.8 | 23.9 | 21.8 | 32.3 | 29.4;
-    // M 2048 x K 6144 at 1540 rows 99 | 87 | 66 | 100 | 90, at 2608 rows (1312 | 672 | 336 | 176) 146 | 133 | 132 | 102 | 122.  K-pieces where the workspace is lent (K >= 6144), whole | pieces, 128 x 128 on 8 waves:
-    // M 2048 x K 6144 at 515 rows 60.6 | 36.0, at 1030 64.9 | 50.5 (a piece and tails), M 5120 x K 25600 at 330 rows 220 | 135; 64 x 64 tiles of M 2048 x K 6144 at 330 rows 32.9 | 27.3.  At K = 3072 pieces lose (2608
-    // rows 32.6 | 36.8)
-    if (n64 <= (nkt < 96 ? 512 : 256)) return g3_go_c<false, false, G3Few>(st, a, n64, ws, ws_bytes, 1);
-    if (n128 <= 256) return g3_go_c<false, false, G3Duo>(st, a, n128, ws, ws_bytes, 1);
+    // M 2048 x K 6144 at 1540 rows 99 | 87 | 66 | 100 | 90, at 2608 rows (1312 | 672 | 336 | 176) 146 | 133 | 132 | 102 | 122
+    if (n64 <= (nkt < 96 ? 512 : 256)) return g3_whole<G3Few>(st, a);
     return g3_picked(st, a, true);
 }
 // y[n, M] = alpha * sum_k B(k, tok) A(k, m) + beta * y (+ bias) with either operand stored K-MAJOR: akm: A = w[K][lda] (element (k, m) at k * lda + m), else w[M][K];

@@ -230,3 +230,31 @@ def test_flags_written_over_behind_the_copies_are_cleared(ctx):
         ctx.sync()
         ctx.hip.kf_set_dequant_arena(ctx.h, None, 0)
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+@pytest.mark.parametrize("dim,q,kv,ffn,n,pieces", [(1024, 2048, 1024, 3072, 515, 6), (2048, 2048, 1024, 6144, 515, 4)])
+def test_down_is_cut_into_the_same_pieces(ctx, dim, q, kv, ffn, n, pieces):
+    """The cuts of k are part of a product's result, so they are told apart here: two large terms that cancel take with them whatever stands in the same piece as they do and nothing else.  Every term is a small whole
+    number or 15 * 2^40 of either sign, the sums of the other pieces are whole numbers below 128: the result is exact."""
+    part = ffn // pieces
+    w = torch.randint(0, 16, (dim, ffn), device=ctx.device).float()
+    w[:, 64::128], w[:, 65::128] = 0.0, 15.0                     # a group's range is 0 .. 15: its 4-bit storage holds the numbers as they are
+    w[:, ::part], w[:, part - 1::part] = 15.0, 15.0
+    ws, _ = _layer(ctx, dim, q, kv, ffn)
+    ws[6] = ctx.quantize(w.bfloat16(), L.Q4)
+    assert torch.equal(ctx.dequant(ws[6]).float().view_as(w), w)
+    descs = [e.desc() for e in ws]
+    x, at = torch.zeros(n, ffn, device=ctx.device), torch.arange(n, device=ctx.device) % pieces
+    x[:, 200::part] = 1.0
+    x[torch.arange(n), at * part], x[torch.arange(n), at * part + part - 1] = 2.0 ** 40, -2.0 ** 40
+    small = w[:, 200::part].t()                                  # [pieces, dim]
+    want = small.sum(0) - small[at]
+    x, y = x.bfloat16(), torch.zeros(n, dim, device=ctx.device, dtype=torch.bfloat16)
+    try:
+        need, scratch = _copies(ctx, descs, n)
+        assert need and ctx.hip.kf_linear(ctx.h, C.byref(descs[6]), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+        ctx.sync()
+    finally:
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
+    assert torch.equal(y.float(), want)
