@@ -229,6 +229,9 @@ int swiglu_launch(hipStream_t st, const uint16_t* gate, const uint16_t* up, uint
 int add_launch(hipStream_t st, const uint16_t* a, const uint16_t* b, uint16_t* out, int n);
 int embed_launch(hipStream_t st, const kf_weight* w, int token, const int32_t* d_token, const int32_t* d_state, const int32_t* d_forced,
                  uint16_t* out, int n_tok = 1);
+// n8 pieces of 8 weights whose copy lies in `ilv_n` matrices' interleaved one: every piece's place is counted in 32 bits; its byte offset fits 32 bits
+static constexpr bool deq4_counted(size_t n8, int ilv_n) { return n8 <= 0x7FFFFFFFu && n8 * (ilv_n > 1 ? ilv_n : 1) <= 0xFFFFFFFFu; }
+static constexpr bool deq4_in_reach(size_t n8, int ilv_n) { return n8 * (ilv_n > 1 ? ilv_n : 1) <= 0x0FFFFFFFu; }
 int dequant4_layer_launch(hipStream_t st, int n, const kf_weight* const* w, uint16_t* const* out, const int* ilv_n, const int* ilv_i); /* up to 8 4-bit matrices (groups of 128) in one launch */
 int dequant_launch(hipStream_t st, const kf_weight* w, uint16_t* out, int ilv_n = 1, int ilv_i = 0); /* ilv_n > 1: rows interleaved with ilv_n - 1 other matrices in blocks of 16 (kf_ops.hip) */
 int adamw_launch(hipStream_t st, uint16_t* params, uint16_t* grads, void* gm, void* gv, size_t n, int mv_bf16, float lr, float beta1, float beta2, float b1c,

@@ -399,7 +399,7 @@ int dequant_launch(hipStream_t st, const kf_weight* w, uint16_t* out, int ilv_n,
         zero = w->gama + w->ne0 + w->ne1;
         step = zero + n / w->lGroup;
     }
-    if (fmt == FMT_Q4 && w->lGroup == 128 && n % 128 == 0 && n / 8 <= 0x0FFFFFFFu && (ilv_n < 2 || (w->ne0 % 16 == 0 && w->ne1 % 8 == 0))) /* 6400 x 1600: 13.1 -> 7.0 us */
+    if (fmt == FMT_Q4 && w->lGroup == 128 && n % 128 == 0 && deq4_counted(n / 8, ilv_n) && (ilv_n < 2 || (w->ne0 % 16 == 0 && w->ne1 % 8 == 0))) /* 6400 x 1600: 13.1 -> 7.0 us */
         return dequant4_layer_launch(st, 1, &w, &out, &ilv_n, &ilv_i);
     const size_t nb = n / epb;
     if (ilv_n > 1 && (w->ne1 % epb != 0 || w->ne0 % 16 != 0)) return KF_INVALID_ARGS;
@@ -418,6 +418,7 @@ struct DeqJob {
     uint32_t n8, row8; /* pieces of 8 weights: of the matrix, of a row */
     int ilv_n, ilv_i;
     float qBias;
+    bool reach; /* deq4_in_reach */
 };
 struct DeqJobs {
     int n;
@@ -448,7 +449,9 @@ __global__ void __launch_bounds__(256) dequant4_layer_kernel(const DeqJobs a) {
             o = ((r >> 4) * 16 * j.ilv_n + 16 * j.ilv_i + (r & 15)) * j.row8 + c;
         }
         const float s = bf2f(st[k]);
-        st_through(j.out, o * 16, frag_q4(d[k], s, s * 0.0625f, -j.qBias * s, bf2f(ze[k])));
+        const u32x4 v = frag_q4(d[k], s, s * 0.0625f, -j.qBias * s, bf2f(ze[k]));
+        if (j.reach) st_through(j.out, o * 16, v);
+        else j.out[o] = v;
     }
 }
 int dequant4_layer_launch(hipStream_t st, int n, const kf_weight* const* w, uint16_t* const* out, const int* ilv_n, const int* ilv_i) {
@@ -458,9 +461,9 @@ int dequant4_layer_launch(hipStream_t st, int n, const kf_weight* const* w, uint
     a.n = n;
     for (int i = 0; i < n; i++) {
         const size_t el = (size_t)w[i]->ne0 * w[i]->ne1;
-        if (el / 8 > 0x0FFFFFFFu || el % 128 || w[i]->type != KF_Q4 || w[i]->lGroup != 128 || !w[i]->gama || (ilv_n[i] > 1 && (w[i]->ne0 % 16 || w[i]->ne1 % 8))) return KF_INVALID_ARGS;
+        if (!deq4_counted(el / 8, ilv_n[i]) || el % 128 || w[i]->type != KF_Q4 || w[i]->lGroup != 128 || !w[i]->gama || (ilv_n[i] > 1 && (w[i]->ne0 % 16 || w[i]->ne1 % 8))) return KF_INVALID_ARGS;
         const uint16_t* const zero = w[i]->gama + w[i]->ne0 + w[i]->ne1;
-        a.j[i] = DeqJob{(const uint32_t*)w[i]->data, zero, zero + el / 128, (u32x4*)out[i], (uint32_t)(el / 8), (uint32_t)(w[i]->ne1 / 8), ilv_n[i], ilv_i[i], (float)w[i]->qBias};
+        a.j[i] = DeqJob{(const uint32_t*)w[i]->data, zero, zero + el / 128, (u32x4*)out[i], (uint32_t)(el / 8), (uint32_t)(w[i]->ne1 / 8), ilv_n[i], ilv_i[i], (float)w[i]->qBias, deq4_in_reach(el / 8, ilv_n[i])};
         a.first[i] = wg, wg += (uint32_t)((el / 8 + 256 * DEQ_PER - 1) / (256 * DEQ_PER));
     }
     a.first[n] = wg;

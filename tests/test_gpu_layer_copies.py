@@ -258,3 +258,23 @@ def test_down_is_cut_into_the_same_pieces(ctx, dim, q, kv, ffn, n, pieces):
     finally:
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
     assert torch.equal(y.float(), want)
+
+
+def test_copies_whose_offsets_pass_32_bits(ctx):
+    """gate | up of 65792 x 16384: the interleaved copy is 4 311 744 512 bytes long, rows from 65536 on lie past 2^32; every row against kf_dequant of its matrix"""
+    dim, ffn, n = 16384, 65792, 2047
+    gate, up = (ctx.quantize(torch.randn(ffn, dim, device=ctx.device, dtype=torch.bfloat16), L.Q4) for _ in range(2))
+    small = [ctx.quantize((torch.randn(*s, device=ctx.device) * 0.05).bfloat16(), L.Q4) for s in ((256, dim), (256, dim), (256, dim), (dim, 256), (dim, 512))]   # (the last stands for down: widths are not compared)
+    ws = small[:4] + [gate, up, small[4]]
+    descs = [w.desc() for w in ws]
+    try:
+        need, scratch = _copies(ctx, descs, n)
+        assert need > 2 ** 32
+        off = sum(w.ne0 * w.ne1 * 2 for w in small[:4])
+        rows = scratch[off:off + 4 * ffn * dim].view(torch.bfloat16).view(ffn // 16, 2, 16, dim)
+        for i, w in enumerate((gate, up)):
+            assert torch.equal(rows[:, i], ctx.dequant(w).view(ffn // 16, 16, dim))
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)

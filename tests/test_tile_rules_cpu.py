@@ -31,3 +31,16 @@ def test_one_round_of_tiles_is_taken_where_there_is_one(tmp_path):
     src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_pick(%d, %d, %d, true) == kf::G3_%s);\n" % (m, n, k, t) for m, n, k, t in PICKED))
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
+
+
+# (pieces of 8 weights, matrices interleaved, offsets of the copy in 32 bits): gate and up of 65552 x 16384 lie in 4 296 015 872 bytes
+REACH = [(65552 * 16384 // 8, 1, True), (65552 * 16384 // 8, 2, False), (65536 * 16384 // 8 - 1, 2, True), ((1 << 28) - 1, 1, True), (1 << 28, 1, False), ((1 << 31) - 1, 2, False)]
+
+
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_offsets_of_dequantised_copies_are_bounded_where_they_end(tmp_path):
+    src = tmp_path / "reach.hip"
+    src.write_text('#include "%s/kf_kernels.h"\n' % B.CSRC + "".join("static_assert(kf::deq4_in_reach(%dull, %d) == %s && kf::deq4_counted(%dull, %d));\n" % (n, i, "true" if r else "false", n, i) for n, i, r in REACH)
+                   + "static_assert(!kf::deq4_counted(1ull << 31, 1) && !kf::deq4_counted(0x7FFFFFFFull, 3));\n")
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
