@@ -23,6 +23,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+constexpr long long AB_NEAR = 1ll << 24; /* elements between rows of which 32 are in reach of a load's 32-bit offset */
 constexpr int AB_T = 32, AB_NB = 4; /* rows of a tile; buffers: two to three tiles are on their way */
 constexpr float AB_LOG2E = 1.44269502162933349609375f, AB_SLACK = 8.0f; /* the running reference of a column moves only past 2^8 (kf_flash.h) */
 
@@ -40,7 +41,7 @@ template <int HD>
 __device__ __forceinline__ int ab_swz(int r, int c) {
     return HD == 128 ? c ^ (((r & 3) << 2) | ((r >> 2) & 3)) : c ^ ((((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1));
 }
-template <int HD>
+template <int HD, bool FAR>
 struct AbTile {
     static constexpr int RB = 2 * HD, PART = AB_T * RB, RPI = 1024 / RB, NI = PART / 4096; /* bytes of a row, of a tile; rows per load instruction; instructions per wave (four to a workgroup) */
     int rf[HD / 16], tl[HD / 32], th[HD / 32]; /* this lane's offsets: row fragments per MFMA step, transposing reads per 32 columns (tile rows 4 h + (l16 >> 2), and 8 further) */
@@ -65,13 +66,23 @@ struct AbTile {
         const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(tile + th[db] + 16 * s2 * RB));
         return __builtin_bit_cast(u32x4, bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
     }
-    // 32 rows from `base` (rows `row_bytes` apart, `left` of them exist: the others become zeros) into LDS, this wave's share
-    __device__ __forceinline__ void load(const uint16_t* base, uint32_t row_bytes, int left, unsigned char* to, int wave) const {
+    // 32 rows from `base`, rows `row_bytes` apart, into LDS: this wave's share.  `left` of them exist (<= 0: the sequence ended that far in front of base).  The others become zeros, and so does everything unless
+    // `wanted`; FAR (a lane's offset does not fit 32 bits): rows of the sequence instead: nobody may look at what they hold
+    __device__ __forceinline__ void load(const uint16_t* base, long long row_bytes, int left, bool wanted, unsigned char* to, int wave) const {
 #ifdef __HIP_DEVICE_COMPILE__
-        const long long n = left <= 0 ? 0 : (long long)(left < AB_T ? left : AB_T) * row_bytes;
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (int)n, 0x00020000);
+        if constexpr (!FAR) {
+            const uint32_t rb = (uint32_t)row_bytes, n = left <= 0 || !wanted ? 0 : (uint32_t)(left < AB_T ? left : AB_T) * rb;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (int)n, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < NI; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(to + (wave * NI + i) * 1024), 16, (uint32_t)off_row[i] * row_bytes + off_chunk[i], 0, 0, 0);
+            for (int i = 0; i < NI; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(to + (wave * NI + i) * 1024), 16, (uint32_t)off_row[i] * rb + off_chunk[i], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int row = off_row[i] < left ? off_row[i] : left - 1;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(reinterpret_cast<const unsigned char*>(base) + row * row_bytes + off_chunk[i]),
+                                                 (__attribute__((address_space(3))) void*)(to + (wave * NI + i) * 1024), 16, 0, 0);
+            }
+        }
 #endif
     }
 };
@@ -87,10 +98,10 @@ __device__ __forceinline__ void ab_apart(const unsigned char* __restrict__ tile,
     f(tile, to);
 }
 
-template <int HD>
+template <int HD, bool FAR>
 __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o,
                                                                                  uint16_t* dq, long long ld_d, float* LD, int T, float scale, int gq, long long ld_kv) {
-    using Tile = AbTile<HD>;
+    using Tile = AbTile<HD, FAR>;
     constexpr int NS = HD / 16, NDB = HD / 32, SET = 2 * Tile::PART, LPS = 2 * Tile::NI; /* K and V of a tile; loads per wave and tile */
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
@@ -105,11 +116,9 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel
     const int tok_last = tok0 + 127 < T ? tok0 + 127 : T - 1, ntile = tok_last / AB_T + 1, first = tok0 + wave * 32; /* first: this wave's first column */
     Tile W;
     W.init(lane, wave);
-    const uint32_t rb = (uint32_t)(ld_kv * 2);
-    auto load = [&](int t, unsigned char* to) {
-        const int left = t < ntile ? T - t * AB_T : 0;
-        W.load(k + (size_t)t * AB_T * ld_kv, rb, left, to, wave);
-        W.load(v + (size_t)t * AB_T * ld_kv, rb, left, to + Tile::PART, wave);
+    auto load = [&](int t, unsigned char* to) { /* (keys past the sequence's end lie behind every column: masked) */
+        W.load(k + (size_t)t * AB_T * ld_kv, 2 * ld_kv, T - t * AB_T, t < ntile, to, wave);
+        W.load(v + (size_t)t * AB_T * ld_kv, 2 * ld_kv, T - t * AB_T, t < ntile, to + Tile::PART, wave);
     };
     int tok = first + r;
     const bool col_ok = tok < T;
@@ -200,10 +209,10 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel
         }
 }
 
-template <int HD>
+template <int HD, bool FAR>
 __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dkv_mfma_kernel(const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* dO, long long ld_o, uint16_t* dk,
                                                                                   uint16_t* dv, long long ld_d, const float* LD, int T, float scale, int gq, long long ld_kv, long long ld_dkv) {
-    using Tile = AbTile<HD>;
+    using Tile = AbTile<HD, FAR>;
     constexpr int NS = HD / 16, NDB = HD / 32, SET = 2 * Tile::PART + 1024, LPS = 2 * Tile::NI + 1; /* Q and dO of a tile, and each wave's own copy of its L | D; loads per wave and tile */
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
@@ -217,12 +226,11 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dkv_mfma_kerne
     const int ntq = (T + AB_T - 1) / AB_T, tg0 = (key0 / AB_T) * gq, tg1 = ntq * gq; /* (query tile, query head of the group) pairs */
     Tile W;
     W.init(lane, wave);
-    const uint32_t rbq = (uint32_t)(ld_qkv * 2), rbo = (uint32_t)(ld_o * 2);
     int lt = tg0 / gq, lh = 0; /* the pair loaded next */
     auto load = [&](unsigned char* to) {
-        const int left = lt < ntq ? T - lt * AB_T : 0, head = kvh * gq + lh;
-        W.load(q + (size_t)lt * AB_T * ld_qkv + (size_t)head * HD, rbq, left, to, wave);
-        W.load(dO + (size_t)lt * AB_T * ld_o + (size_t)head * HD, rbo, left, to + Tile::PART, wave);
+        const int left = T - lt * AB_T, head = kvh * gq + lh;
+        W.load(q + (size_t)lt * AB_T * ld_qkv + (size_t)head * HD, 2 * ld_qkv, left, true, to, wave);
+        W.load(dO + (size_t)lt * AB_T * ld_o + (size_t)head * HD, 2 * ld_o, left, true, to + Tile::PART, wave);
 #ifdef __HIP_DEVICE_COMPILE__
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(LD + ((size_t)head * T + lt * AB_T) * 2), 0, left < 0 ? 0 : left * 8, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(to + 2 * Tile::PART + wave * 256), 4, lane * 4, 0, 0, 0);
@@ -258,9 +266,12 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dkv_mfma_kerne
                 st = ab_mfma(W.rows(tile, s), kf_[s], st);
                 dpt = ab_mfma(W.rows(tile + Tile::PART, s), vf[s], dpt);
             }
-            if (t * AB_T < wave_key0 + 31) { /* else every query of the tile follows every key of this wave; rows past the sequence's end are zeros in Q, dO, L and D and add nothing */
+            if (t * AB_T < wave_key0 + 31 || t * AB_T + AB_T > T) { /* else every query of the tile exists and follows every key of this wave */
 #pragma unroll
-                for (int i = 0; i < 16; i++) st[i] = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2) >= key ? st[i] : -__builtin_inff();
+                for (int i = 0; i < 16; i++) {
+                    const int query = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2);
+                    st[i] = query >= key && query < T ? st[i] : -__builtin_inff();
+                }
             }
             uint32_t pw[8], dw[8];
             const f32x4* const ld = reinterpret_cast<const f32x4*>(tile + 2 * Tile::PART + wave * 256);
@@ -301,30 +312,30 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dkv_mfma_kerne
         }
 }
 
-template <int HD>
+template <int HD, bool FAR>
 static int ab_go(hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o, uint16_t* dq, uint16_t* dk, uint16_t* dv,
                  long long ld_d, int T, int n_head, int n_seq, float* LD, int n_kv, long long ld_kv, long long ld_dkv) {
-    constexpr int smem_q = AB_NB * 2 * AbTile<HD>::PART, smem_kv = AB_NB * (2 * AbTile<HD>::PART + 1024);
+    constexpr int smem_q = AB_NB * 2 * AbTile<HD, FAR>::PART, smem_kv = AB_NB * (2 * AbTile<HD, FAR>::PART + 1024);
     static int attr_set = 0;
     if (!attr_set && smem_kv > 64 * 1024) {
-        if (hipFuncSetAttribute((const void*)attn_bwd_dq_mfma_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q) != hipSuccess) return KF_HIP_CHECK;
-        if (hipFuncSetAttribute((const void*)attn_bwd_dkv_mfma_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv) != hipSuccess) return KF_HIP_CHECK;
+        if (hipFuncSetAttribute((const void*)attn_bwd_dq_mfma_kernel<HD, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_q) != hipSuccess) return KF_HIP_CHECK;
+        if (hipFuncSetAttribute((const void*)attn_bwd_dkv_mfma_kernel<HD, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, smem_kv) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
     const float scale = 1.0f / sqrtf((float)HD);
     const dim3 grid((T + 127) / 128, n_head, n_seq), grid_kv((T + 127) / 128, n_kv, n_seq);
-    hipLaunchKernelGGL((attn_bwd_dq_mfma_kernel<HD>), grid, dim3(256), smem_q, st, q, k, v, ld_qkv, o, dO, ld_o, dq, ld_d, LD, T, scale, n_head / n_kv, ld_kv);
-    hipLaunchKernelGGL((attn_bwd_dkv_mfma_kernel<HD>), grid_kv, dim3(256), smem_kv, st, q, k, v, ld_qkv, dO, ld_o, dk, dv, ld_d, LD, T, scale, n_head / n_kv, ld_kv, ld_dkv);
+    hipLaunchKernelGGL((attn_bwd_dq_mfma_kernel<HD, FAR>), grid, dim3(256), smem_q, st, q, k, v, ld_qkv, o, dO, ld_o, dq, ld_d, LD, T, scale, n_head / n_kv, ld_kv);
+    hipLaunchKernelGGL((attn_bwd_dkv_mfma_kernel<HD, FAR>), grid_kv, dim3(256), smem_kv, st, q, k, v, ld_qkv, dO, ld_o, dk, dv, ld_d, LD, T, scale, n_head / n_kv, ld_kv, ld_dkv);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 // KF_OK launched; 1 = shape not covered by the MFMA form
 int attn_backward_mfma_launch(hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v, long long ld_qkv, const uint16_t* o, const uint16_t* dO, long long ld_o,
                               uint16_t* dq, uint16_t* dk, uint16_t* dv, long long ld_d, int T, int n_head, int hd, int n_seq, float* scratch, int n_kv, long long ld_kv, long long ld_dkv) {
     if ((hd != 64 && hd != 128) || n_kv < 1 || n_head % n_kv != 0) return 1;
-    if ((ld_qkv | ld_o | ld_kv) >= (1 << 24)) return 1; /* 32 rows in reach of a load's 32-bit offset */
     float* const LD = scratch; /* [n_seq][n_head][T][2]: log-sum-exp and dO . O of a query */
-    return hd == 64 ? ab_go<64>(st, q, k, v, ld_qkv, o, dO, ld_o, dq, dk, dv, ld_d, T, n_head, n_seq, LD, n_kv, ld_kv, ld_dkv)
-                    : ab_go<128>(st, q, k, v, ld_qkv, o, dO, ld_o, dq, dk, dv, ld_d, T, n_head, n_seq, LD, n_kv, ld_kv, ld_dkv);
+    const bool far = ld_qkv >= AB_NEAR || ld_o >= AB_NEAR || ld_kv >= AB_NEAR;
+    const auto go = hd == 64 ? (far ? &ab_go<64, true> : &ab_go<64, false>) : (far ? &ab_go<128, true> : &ab_go<128, false>);
+    return go(st, q, k, v, ld_qkv, o, dO, ld_o, dq, dk, dv, ld_d, T, n_head, n_seq, LD, n_kv, ld_kv, ld_dkv);
 }
 
 }  // namespace kf

@@ -468,3 +468,27 @@ def test_attn_backward_where_references_move(ctx, T, H, G, hd, std):
         ref, y = x[i].grad, got[i].double().cpu()
         assert float((y[:, :n * hd] - ref).abs().max()) <= 2.0 ** -6 * max(float(ref.abs().max()), 2.0 ** -6 * (i < 2)), i
         assert bool((y[:, n * hd:] == 0).all())
+
+
+@pytest.mark.parametrize("hd,T", [(64, 70), (128, 33)])
+def test_attn_backward_of_rows_far_apart(ctx, hd, T):
+    """rows of q | k | v and of o | dO as far apart as no 32-bit offset reaches: the bits of the same rows side by side"""
+    H, G, far, dev = 2, 1, (1 << 24) + 64, ctx.device
+    near = 8 * hd
+    g = torch.Generator().manual_seed(T)
+    rows = torch.randn(5, T, H * hd, generator=g).bfloat16().to(dev)   # q, k, v, o, dO (k and v: their first head)
+    sc = torch.zeros(ctx.hip.kf_attn_backward_scratch_bytes(T, H, 1) // 4 + 1, dtype=torch.float32, device=dev)
+    got = []
+    big = torch.empty((T - 1) * far + near, dtype=torch.bfloat16, device=dev)
+    for ld in (near, far):
+        both = (big if ld == far else torch.empty(T * near, dtype=torch.bfloat16, device=dev)).as_strided((T, near), (ld, 1))
+        views = []
+        for i, (col, w) in enumerate(((0, H * hd), (2 * hd, hd), (3 * hd, hd), (4 * hd, H * hd), (6 * hd, H * hd))):
+            both[:, col:col + w] = rows[i][:, :w]
+            views.append(both[:, col:col + w])
+        d = torch.zeros(3, T, H * hd, dtype=torch.bfloat16, device=dev)
+        assert ctx.hip.kf_attn_backward(ctx.h, views[0].data_ptr(), views[1].data_ptr(), views[2].data_ptr(), ld, views[3].data_ptr(), views[4].data_ptr(), ld, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(),
+                                        H * hd, T, H, G, hd, 1, sc.data_ptr()) == 0, ctx.hip.kf_last_error()
+        ctx.sync()
+        got.append(d)
+    assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16)) and float(got[0][0].float().abs().max()) > 0
