@@ -504,7 +504,8 @@ int attn_prefill_mfma_launch(hipStream_t st, const uint16_t* q, const uint16_t* 
     // Otherwise the walk by loads into LDS from 512 keys on: its first tiles take longer to come, its step is shorter.  us, staged through registers | by loads: 16 / 8 heads x 128, 128 tokens 8.5 | 9.3, 255 13.6 | 14.1,
     // 16 prompts of 131 tokens 14.6 | 14.7; 64 / 8 heads, 700 tokens 32.9 | 31.5, 1024 47.4 | 43.4; 16 / 8 heads, 4095 tokens 163 | 152; 25 heads x 64, 8 x 1024 tokens 90.3 | 83.7
     const bool halves = (long)grid.x * grid.y * grid.z <= 320 && n_tok >= g_knobs.attn_pair_min; /* short prompts: the launch is a few microseconds either way */
-    const int kh = halves ? 2 : pos0 + n_tok >= g_knobs.attn_walk_min ? 0 : 1;
+    const bool near = kv_stride < (1 << 24); /* the 32 rows of its tiles in reach of a load's 32-bit offset; the others' are 64-bit */
+    const int kh = halves ? 2 : near && pos0 + n_tok >= g_knobs.attn_walk_min ? 0 : 1;
     if (kh == 2) grid.x = (nsb + 1) / 2;
     const int rc = hd == 128 ? ap_launch_gq<128>(st, a, GQ, grid, kh) : ap_launch_gq<64>(st, a, GQ, grid, kh);
     if (rc) return rc;

@@ -158,14 +158,15 @@ def test_attn_prefill_long_prompt_form_vs_oracle(ctx, nh, nkv, hd, pos0, n):
 FORMS = {"registers": (1 << 30, 1 << 30), "loads into LDS": (1 << 30, 0), "halves": (0, 1 << 30)}   # all keys staged through registers, by loads into LDS; two key halves
 
 
-def _attention_in_form(ctx, form, q, k, v, out, pos0, n, n_seq, nh, nkv, hd):
+def _attention_in_form(ctx, form, q, k, v, out, pos0, n, n_seq, nh, nkv, hd, kv_stride=None):
+    kv_stride = kv_stride or nkv * hd
     pair, walk = FORMS[form]
     try:
         assert ctx.hip.kfdbg_set_knob(b"attn_pair_min", pair) == 0 and ctx.hip.kfdbg_set_knob(b"attn_walk_min", walk) == 0
         if n_seq == 1:
-            rc = ctx.hip.kf_attn_prefill(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), pos0, n, nh * hd, nh, nkv, hd, nkv * hd)
+            rc = ctx.hip.kf_attn_prefill(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), pos0, n, nh * hd, nh, nkv, hd, kv_stride)
         else:
-            rc = ctx.hip.kf_attn_prefill_batch(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n, nh * hd, nh, nkv, hd, nkv * hd, n_seq)
+            rc = ctx.hip.kf_attn_prefill_batch(ctx.h, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), n, nh * hd, nh, nkv, hd, kv_stride, n_seq)
         assert rc == 0, ctx.hip.kf_last_error()
         ctx.sync()
     finally:
@@ -223,3 +224,20 @@ def test_attention_with_scores_far_beyond_the_exponents(ctx, form, nh, nkv, hd, 
     _attention_in_form(ctx, form, qd, kd, vd, out, 0, n, 1, nh, nkv, hd)
     best = torch.stack([rank[:t + 1].argmax() for t in range(n)])
     assert torch.equal(out.cpu().reshape(n, nh, hd), v[best].repeat_interleave(nh // nkv, 1))
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_over_cache_rows_far_apart(ctx, form, hd):
+    """K and V rows 80 MB apart, the last of a tile past 2^31 bytes: the bits of the same rows side by side"""
+    import torch
+    n, nh, nkv, far = 40, 4, 2, 5 << 23
+    g = torch.Generator().manual_seed(hd)
+    q, k, v = (torch.randn(n, h * hd, generator=g).bfloat16().to(ctx.device) for h in (nh, nkv, nkv))
+    big = torch.zeros((n - 1) * far + 2 * nkv * hd, dtype=torch.bfloat16, device=ctx.device)
+    kf, vf = (big.as_strided((n, nkv * hd), (far, 1), i * nkv * hd) for i in (0, 1))
+    kf.copy_(k), vf.copy_(v)
+    near, out = (torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=ctx.device) for _ in range(2))
+    _attention_in_form(ctx, form, q, k, v, near, 0, n, 1, nh, nkv, hd)
+    _attention_in_form(ctx, form, q, kf, vf, out, 0, n, 1, nh, nkv, hd, far)
+    assert torch.equal(near.view(torch.int16), out.view(torch.int16)) and float(near.float().abs().max()) > 0
