@@ -403,6 +403,7 @@ struct G3Out16 {
         }
     }
     static __device__ __forceinline__ u32x4 rows8(const unsigned char* smem, int tok, int chunk) { return *reinterpret_cast<const u32x4*>(smem + at(tok, chunk)); }
+    static __device__ __forceinline__ u32x2 rows4(const unsigned char* smem, int tok, int u) { return *reinterpret_cast<const u32x2*>(smem + at(tok, u >> 1) + 8 * (u & 1)); } /* rows 4 u .. + 3 */
     template <int U, class F>
     static __device__ __forceinline__ void each(int tid, F&& f) { /* f(token of the tile, unit) for this thread's share of BN tokens x U units, after a barrier */
         __syncthreads();

@@ -445,16 +445,16 @@ def test_tiles_of_one_round_and_more_against_fp32(ctx, M, K, n):
     assert bool((buf[0] == 7).all()) and bool((buf[n + 1] == 7).all())
 
 
-@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("alpha,beta,odd", [(0.5, 0.0, 0), (0.5, 1.0, 0), (1.0, 0.0, 0), (1.0, 0.0, 1), (1.0, 1.0, 1)])
 @pytest.mark.parametrize("M,K,n", [(1001, 128, 257), (1004, 192, 2047), (2050, 128, 1541), (2049, 320, 4001), (6148, 256, 2608), (1032, 128, 2600), (6152, 256, 2608)])
-def test_tiles_whose_rows_are_no_whole_chunks(ctx, M, K, n, beta):
-    """rows of y that no 16-byte store divides (and two that it does), added to what is there and scaled: the bound of the test above"""
+def test_tiles_whose_rows_are_no_whole_chunks(ctx, M, K, n, alpha, beta, odd):
+    """rows of y that no 16-byte store divides (and two that it does), added to what is there and scaled, as they are, and a bias at an odd address: the bound of the test above"""
     w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.BF16)
-    x, bias, res = torch.randn(n, K, device=ctx.device).bfloat16(), torch.randn(M, device=ctx.device).bfloat16(), torch.randn(n, M, device=ctx.device).bfloat16()
+    x, bias, res = torch.randn(n, K, device=ctx.device).bfloat16(), torch.randn(M + odd, device=ctx.device).bfloat16()[odd:], torch.randn(n, M, device=ctx.device).bfloat16()
     buf = torch.full((n + 2, M), 7.0, device=ctx.device, dtype=torch.bfloat16)
     d, y = w.desc(), buf[1:n + 1]
-    assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), bias.data_ptr(), n, 0.5, beta, L.KF_EPI_RESIDUAL, res.data_ptr()) == 0, ctx.hip.kf_last_error()
+    assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y.data_ptr(), bias.data_ptr(), n, alpha, beta, L.KF_EPI_RESIDUAL, res.data_ptr()) == 0, ctx.hip.kf_last_error()
     ctx.sync()
-    s = 0.5 * (x.float() @ ctx.dequant(w).float().reshape(M, K).t()) + 7.0 * beta + bias.float()
+    s = alpha * (x.float() @ ctx.dequant(w).float().reshape(M, K).t()) + 7.0 * beta + bias.float()
     assert float((y.float() - s - res.float()).abs().max()) <= 2.0 ** -8 * (float(s.abs().max()) + float((s + res.float()).abs().max()))
     assert bool((buf[0] == 7).all()) and bool((buf[n + 1] == 7).all())
