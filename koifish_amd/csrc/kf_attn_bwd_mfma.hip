@@ -1,11 +1,11 @@
 // kf_attn_bwd_mfma.hip -- causal multi-head attention backward on MFMA (flash form), gfx950 / wave64.  Same contract as kf_attn_bwd.hip (its
 // header has the mathematics and the reference), same two-launch split, the tile algebra of the forward kernel (kf_flash.h):
 //
-//   dQ launch, workgroup = 128 query columns (32 per wave), ONE walk over key tiles of 32:
+//   dQ launch, workgroup = 128 query columns (32 per wave), key tiles of 32, two walks:
 //              S^T[key][col] = K . Q^T, dP^T[key][col] = V . dO^T     A = K / V rows (ds_read_b128), B = Q / dO rows (registers, loaded once)
-//              p = exp(scale S^T - M), dS^T = p o (dP^T - D)          element-wise on the accumulators: a column lives in one lane pair; M the column's running reference as in the forward kernel
+//              first walk: the column's log-sum-exp L (running maximum and sum, a column lives in one lane pair); L and D = dO . O go to launch 2, side by side
+//              P = exp(scale S^T - L), dS^T = P o (dP^T - D)          element-wise on the accumulators
 //              dQ^T[d][col] += K^T[d][key] . dS^T[key][col]           the dS^T registers, packed to bf16, ARE the B operand (free contraction order)
-//              dQ is linear in p, so it is divided by the sum of p at the end; the column's log-sum-exp L and D = dO . O go to launch 2, side by side
 //   dK/dV launch, workgroup = 128 key columns, query tiles of 32 from the diagonal down (Q, dO, and L | D of the tile's queries):
 //              S[q][key] = Q . K^T, dP[q][key] = dO . V^T   A = Q / dO rows, B = K / V rows of the column (registers)
 //              P = exp(scale S - L_q), dS = P o (dP - D_q)  L, D per accumulator ROW: two ds_read_b128 per four rows
@@ -13,8 +13,8 @@
 // P and dS enter their products as single bf16 values (gradients are compared at 2^-7 of scale); everything else fp32.
 //
 // What bounds it: per 32 x 32 tile the two launches' MFMAs take 384 + 512 cycles of a SIMD at dim 64 and their vector instructions about as many.  A tile goes global -> LDS by buffer loads, AB_NB buffers, ONE barrier per
-// tile; it lies there once, under a swizzle that suits the row reads and the transposing reads of the same rows (ab_swz); two or three waves to a SIMD do the rest.  25 heads x 64, 8 x 1024 tokens: 430 us with tiles staged through
-// registers, twice each, two barriers a tile and a walk of its own for L; 164 (76 + 88) so.
+// tile (the first walk: per two); it lies there once, under a swizzle that suits the row reads and the transposing reads of the same rows (ab_swz); two or three waves to a SIMD do the rest.  25 heads x 64, 8 x 1024
+// tokens: 410 us with tiles staged through registers, twice each, two barriers a tile; 193 so, the same bits.  With one walk, dQ divided by the sum of p at its end, 165, but other roundings of every dS.
 #include "kf_kernels.h"
 
 namespace kf {
@@ -25,7 +25,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr long long AB_NEAR = 1ll << 24; /* elements between rows of which 32 are in reach of a load's 32-bit offset */
 constexpr int AB_T = 32, AB_NB = 4; /* rows of a tile; buffers: two to three tiles are on their way */
-constexpr float AB_LOG2E = 1.44269502162933349609375f, AB_SLACK = 8.0f; /* the running reference of a column moves only past 2^8 (kf_flash.h) */
+constexpr float AB_LOG2E = 1.44269502162933349609375f;
 
 __device__ __forceinline__ f32x16 ab_zero() {
     f32x16 z;
@@ -116,9 +116,13 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel
     const int tok_last = tok0 + 127 < T ? tok0 + 127 : T - 1, ntile = tok_last / AB_T + 1, first = tok0 + wave * 32; /* first: this wave's first column */
     Tile W;
     W.init(lane, wave);
-    auto load = [&](int t, unsigned char* to) { /* (keys past the sequence's end lie behind every column: masked) */
-        W.load(k + (size_t)t * AB_T * ld_kv, 2 * ld_kv, T - t * AB_T, t < ntile, to, wave);
-        W.load(v + (size_t)t * AB_T * ld_kv, 2 * ld_kv, T - t * AB_T, t < ntile, to + Tile::PART, wave);
+    const int n1 = (ntile + 1) / 2;
+    auto load = [&](int i, unsigned char* to) { /* step i: two K tiles of the first walk, then K and V of each of the second (keys past the sequence's end lie behind every column: masked) */
+        const bool one = i < n1;
+        const int ta = one ? 2 * i : i - n1, tb = one ? ta + 1 : ta;
+        const uint16_t* const second = one ? k : v;
+        W.load(k + (size_t)ta * AB_T * ld_kv, 2 * ld_kv, T - ta * AB_T, ta < ntile, to, wave);
+        W.load(second + (size_t)tb * AB_T * ld_kv, 2 * ld_kv, T - tb * AB_T, tb < ntile, to + Tile::PART, wave);
     };
     int tok = first + r;
     const bool col_ok = tok < T;
@@ -143,46 +147,64 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel
 #pragma unroll
     for (int b = 0; b < AB_NB - 1; b++) load(b, smem_raw + b * SET);
 
+    const float c1 = scale * AB_LOG2E;
+    int b = 0;
+    auto step = [&](int i, auto&& f) { /* step i is here; step i + NB - 1 goes where step i - 1 was */
+        ab_landed<(AB_NB - 2) * LPS>();
+        ab_apart(smem_raw + b * SET, smem_raw + (b ? b - 1 : AB_NB - 1) * SET, [&](const unsigned char* tile, unsigned char* to) __attribute__((always_inline)) {
+            load(i + AB_NB - 1, to);
+            f(tile);
+        });
+        b = b + 1 < AB_NB ? b + 1 : 0;
+    };
+    // the log-sum-exp of every column, in log2 units: running maximum and sum of 2^(s - M)
+    float M = -__builtin_inff(), l = 0.f;
+    for (int i = 0; i < n1; i++)
+        step(i, [&](const unsigned char* tile) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int t = 2 * i + u;
+                if (t * AB_T > first + 31) return; /* every key of the tile follows this wave's columns */
+                f32x16 st = ab_zero();
+#pragma unroll
+                for (int s = 0; s < NS; s++) st = ab_mfma(W.rows(tile + u * Tile::PART, s), qf[s], st);
+#pragma unroll
+                for (int e = 0; e < 16; e++) st[e] *= c1;
+                if (t * AB_T + AB_T - 1 > first) { /* else every key of the tile precedes every column of this wave */
+#pragma unroll
+                    for (int e = 0; e < 16; e++) st[e] = t * AB_T + 4 * h + (e & 3) + 8 * (e >> 2) <= tok ? st[e] : -__builtin_inff();
+                }
+                float mt = st[0];
+#pragma unroll
+                for (int e = 1; e < 16; e++) mt = fmaxf(mt, st[e]);
+                mt = xmax32(mt);
+                if (mt > M) l *= __builtin_amdgcn_exp2f(M - mt), M = mt; /* M = -inf on the first tile: 0 */
+#pragma unroll
+                for (int e = 0; e < 16; e++) l += __builtin_amdgcn_exp2f(st[e] - M);
+            }
+        });
+    const float L2 = (M + __log2f(xsum32(l))) * 0.693147182464599609375f * AB_LOG2E; /* (by way of natural units) */
+
     f32x16 acc[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; db++) acc[db] = ab_zero();
-    float M = -__builtin_inff(), l = 0.f; /* log2 units; this lane's half of the sum */
-    const float c1 = scale * AB_LOG2E;
-    int b = 0;
-    for (int t = 0; t < ntile; t++) {
-        ab_landed<(AB_NB - 2) * LPS>(); /* tile t; tile t + NB - 1 goes where tile t - 1 was */
-        ab_apart(smem_raw + b * SET, smem_raw + (b ? b - 1 : AB_NB - 1) * SET, [&](const unsigned char* tile, unsigned char* to) __attribute__((always_inline)) {
-            load(t + AB_NB - 1, to);
-            if (t * AB_T > first + 31) return; /* every key of the tile follows this wave's columns */
+    for (int t = 0; t < ntile; t++)
+        step(n1 + t, [&](const unsigned char* tile) __attribute__((always_inline)) {
+            if (t * AB_T > first + 31) return;
             f32x16 st = ab_zero(), dpt = ab_zero();
 #pragma unroll
             for (int s = 0; s < NS; s++) {
                 st = ab_mfma(W.rows(tile, s), qf[s], st);
                 dpt = ab_mfma(W.rows(tile + Tile::PART, s), dof[s], dpt);
             }
-            if (t * AB_T + AB_T - 1 > first) { /* else every key of the tile precedes every column of this wave */
+            if (t * AB_T + AB_T - 1 > first) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) st[i] = t * AB_T + 4 * h + (i & 3) + 8 * (i >> 2) <= tok ? st[i] : -__builtin_inff();
-            }
-            float mt = st[0];
-#pragma unroll
-            for (int i = 1; i < 16; i++) mt = fmaxf(mt, st[i]);
-            mt = xmax32(mt) * c1;
-            if (mt > M + AB_SLACK) {
-                const float alpha = __builtin_amdgcn_exp2f(M - mt); /* M = -inf on the first tile: 0 */
-                l *= alpha;
-#pragma unroll
-                for (int db = 0; db < NDB; db++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[db][i] *= alpha;
-                M = mt;
             }
             uint32_t dw[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(st[2 * i], c1, -M)), p1 = __builtin_amdgcn_exp2f(fmaf(st[2 * i + 1], c1, -M));
-                l += p0;
-                l += p1;
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(st[2 * i], c1, -L2)), p1 = __builtin_amdgcn_exp2f(fmaf(st[2 * i + 1], c1, -L2));
                 dw[i] = pack_bf16x2(p0 * (dpt[2 * i] - D), p1 * (dpt[2 * i + 1] - D));
             }
 #pragma unroll
@@ -192,20 +214,16 @@ __global__ void __launch_bounds__(256, HD == 64 ? 3 : 2) attn_bwd_dq_mfma_kernel
                 for (int db = 0; db < NDB; db++) acc[db] = ab_mfma(W.turned(tile, db, s2), B, acc[db]);
             }
         });
-        b = b + 1 < AB_NB ? b + 1 : 0;
-    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* loads past the last tile write zeros: none may be on its way when the workgroup's LDS goes to another */
-    l = xsum32(l);
     if (!col_ok) return;
-    if (h == 0) LD[((size_t)head * T + tok) * 2] = M + __log2f(l), LD[((size_t)head * T + tok) * 2 + 1] = D; /* log-sum-exp of the scaled scores, log2 units */
-    const float by = scale / l;
+    if (h == 0) LD[((size_t)head * T + tok) * 2] = L2, LD[((size_t)head * T + tok) * 2 + 1] = D; /* log-sum-exp of the scaled scores, log2 units */
     uint16_t* out = dq + (size_t)tok * ld_d + hoff;
 #pragma unroll
     for (int db = 0; db < NDB; db++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const int d = 32 * db + 8 * g + 4 * h;
-            *reinterpret_cast<u32x2*>(out + d) = u32x2{pack_bf16x2(acc[db][4 * g] * by, acc[db][4 * g + 1] * by), pack_bf16x2(acc[db][4 * g + 2] * by, acc[db][4 * g + 3] * by)};
+            *reinterpret_cast<u32x2*>(out + d) = u32x2{pack_bf16x2(acc[db][4 * g] * scale, acc[db][4 * g + 1] * scale), pack_bf16x2(acc[db][4 * g + 2] * scale, acc[db][4 * g + 3] * scale)};
         }
 }
 
