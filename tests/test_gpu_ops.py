@@ -428,3 +428,25 @@ def test_argmax_rows_by_wide_loads_and_the_ends_of_prompts(ctx, n, ld):
     ctx.sync()
     assert st[seq.long()].tolist() == [[at[i], 21 + i, 9, 0] for i in range(rows)]
     assert [int(out[int(seq[i]), 20 + i]) for i in range(rows)] == at
+
+
+@pytest.mark.parametrize("n,ld", [(9000, 9000), (70001, 70008), (1500, 1501)])
+def test_argmax_rows_with_values_that_are_not_numbers(ctx, O, n, ld):
+    """the pick of every row is the oracle's: NaNs first in what a thread reads and elsewhere, rows of -inf, NaN at the front, nothing but NaNs"""
+    rows, dev = 8, ctx.device
+    g = torch.Generator().manual_seed(n)
+    lg = torch.randn(rows, ld, generator=g).bfloat16()
+    lg[1, 1024], lg[1, 1029] = float("nan"), 50.0     # a 16-byte load's first value, the maximum behind it
+    lg[2, 8], lg[2, min(n - 1, 8200)] = float("nan"), 50.0
+    lg[3, :n:8] = float("nan")
+    lg[4, 0] = float("nan")
+    lg[5] = float("nan")
+    lg[6] = -float("inf")
+    lg[7, :n - 1] = float("nan")
+    lg[7, 0] = -float("inf")
+    want = [O.argmax_bf16(lg[i, :n].view(torch.int16).numpy().view(np.uint16)) for i in range(rows)]
+    seq = torch.arange(rows, dtype=torch.int32, device=dev)
+    st, out, d = torch.zeros(rows, 4, dtype=torch.int32, device=dev), torch.zeros(rows, 4, dtype=torch.int32, device=dev), lg.to(dev)
+    assert ctx.hip.kf_argmax_rows_state(ctx.h, d.data_ptr(), ld, n, rows, seq.data_ptr(), st.data_ptr(), out.data_ptr(), 4) == 0
+    ctx.sync()
+    assert st[:, 0].tolist() == want and out[:, 0].tolist() == want
