@@ -71,7 +71,7 @@ __device__ __forceinline__ void g3_epilogue_qkrope(const GemmArgs& a, int m0, in
         }
         if (t0 + tk < a.n) {
 #pragma unroll
-            for (int e = 0; e < 2; e++) g3_store16(ybase + (size_t)t0 * ldy + (m0 - mshift), (uint32_t)tk * (uint32_t)(2 * ldy) + 128 * e + 16 * u, g3_pack8(x[e]));
+            for (int e = 0; e < 2; e++) g3_store_row(ybase + (size_t)t0 * ldy + (m0 - mshift), tk, ldy, 128 * e + 16 * u, g3_pack8(x[e]));
         }
     });
 }
@@ -92,7 +92,7 @@ __device__ __forceinline__ void g3_epilogue(const GemmArgs& a, int m0, int t0, c
             g3_unpack8(Half::rows8(smem_raw, tk, c), g), g3_unpack8(Half::rows8(smem_raw, tk, c + 2), p);
 #pragma unroll
             for (int j = 0; j < 8; j++) g[j] = (g[j] * p[j]) / (1.0f + kf_expf(-g[j]));
-            g3_store16(a.y + (size_t)t0 * a.ldy + (m0 >> 1), (uint32_t)tk * (uint32_t)(2 * a.ldy) + 16 * u, g3_pack8(g));
+            g3_store_row(a.y + (size_t)t0 * a.ldy + (m0 >> 1), tk, a.ldy, 16 * u, g3_pack8(g));
         });
         return;
     }

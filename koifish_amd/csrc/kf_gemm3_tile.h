@@ -366,6 +366,11 @@ struct G3Out {
 };
 // 16 bytes to base + off (base: uniform), written through: left to the write-back of the XCDs' L2s at the launch's end a one-round product is 1.5 - 2.5 us longer
 __device__ __forceinline__ void g3_store16(void* base, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, g3_rsrc(base, G3_ALL), off, 0, 16 /* sc1 */); }
+/* the same to `byte` of token tk's row of a tile at `base`, rows ld values apart: out of a 32-bit offset's reach by its own address */
+__device__ __forceinline__ void g3_store_row(uint16_t* base, int tk, long long ld, int byte, u32x4 v) {
+    if (ld < (1 << 22)) g3_store16(base, (uint32_t)tk * (uint32_t)(2 * ld) + byte, v);
+    else *reinterpret_cast<u32x4*>(reinterpret_cast<unsigned char*>(base + tk * ld) + byte) = v;
+}
 __device__ __forceinline__ u32x4 g3_pack8(const float (&v)[8]) { return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])}; }
 __device__ __forceinline__ void g3_unpack8(u32x4 p, float (&v)[8]) {
 #pragma unroll

@@ -278,3 +278,24 @@ def test_copies_whose_offsets_pass_32_bits(ctx):
     finally:
         ctx.sync()
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
+
+
+def test_swiglu_rows_whose_offsets_pass_32_bits(ctx):
+    """gate | up with 2^23 + 65536 FFN rows: from token 254 of a tile on a row lies past 2^32 bytes; some columns of every token against fp32 on the dequantised values"""
+    dim, ffn, n = 128, (1 << 23) + 65536, 320
+    ws, descs = _layer(ctx, dim, 2048, 512, ffn)
+    try:
+        need, scratch = _copies(ctx, descs, n)
+        assert need
+        x = torch.randn(n, dim, device=ctx.device).bfloat16()
+        act, up = (torch.zeros(n, ffn, device=ctx.device, dtype=torch.bfloat16) for _ in range(2))
+        assert ctx.hip.kf_gateup_swiglu_batch(ctx.h, C.byref(descs[4]), C.byref(descs[5]), x.data_ptr(), act.data_ptr(), up.data_ptr(), n) == 0
+        ctx.sync()
+        at = torch.cat([torch.arange(64), torch.randint(0, ffn, (512,)), torch.arange(ffn - 64, ffn)]).to(ctx.device)
+        g, u = (x.float() @ ctx.dequant(w)[at].float().t() for w in (ws[4], ws[5]))
+        ref = torch.nn.functional.silu(g) * u
+        assert float((act[:, at].float() - ref).abs().max()) <= 2.0 ** -6 * float(ref.abs().max())
+        assert ctx.hip.kf_layer_copies_end(ctx.h) == 0
+    finally:
+        ctx.sync()
+        ctx.hip.kf_set_scratch(ctx.h, None, 0)
