@@ -1501,11 +1501,9 @@ int kfdbg_set_knob(const char* name, long value) {
     else if (!strcmp(name, "gemv_stream")) k.gemv_stream = (int)value;
     else if (!strcmp(name, "gemv_xf2")) k.gemv_xf2 = (int)value;
     else if (!strcmp(name, "gemm_min")) k.gemm_min = (int)value;
-    else if (!strcmp(name, "g3_tiles")) k.g3_tiles = (int)value;
     else if (!strcmp(name, "g3_first")) k.g3_first = (int)value;
     else if (!strcmp(name, "g3_wide")) k.g3_wide = (int)value;
     else if (!strcmp(name, "attn_gq_split")) k.attn_gq_split = (int)value;
-    else if (!strcmp(name, "g3_mid_min")) k.g3_mid_min = (int)value;
     else if (!strcmp(name, "resident_min")) k.resident_min = (int)value;
     else if (!strcmp(name, "attn_pair_min")) k.attn_pair_min = (int)value;
     else if (!strcmp(name, "attn_walk_min")) k.attn_walk_min = (int)value;

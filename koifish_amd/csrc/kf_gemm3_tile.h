@@ -15,7 +15,6 @@ template <int BM_, int BN_, int NW_, int NBUF_ = 2>
 struct G3Cfg {
     static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = NW_ / 2, MT = BM_ / 32, NT = BN_ / (16 * (NW_ / 2)), NBUF = NBUF_;
     static constexpr int NIA = BM_ / (8 * NW_), NIB = BN_ / (8 * NW_); /* global_load_lds instructions per wave, operand and k-step (8 rows of 128 bytes each) */
-    static constexpr __host__ __device__ int row_block(int wm, int mt) { return wm * MT + mt; } /* the 16-row block of the tile that is block mt of the waves wm */
     static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, SMEM = NBUF_ * STAGE, WGS_PER_CU = (160 * 1024) / SMEM;
 };
 using G3Big = G3Cfg<256, 256, 8>;      /* 128 KiB of LDS: one workgroup per CU */
@@ -215,9 +214,9 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
                 const int mt = half * HM + mh;
-                if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(tile + (C::row_block(wm, mt) * 2 + kk) * 1024 + lane * 16);
-                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(tile, km, C::row_block(wm, mt), kk);
-                else f[mh][kk] = g3_frag(tile, C::row_block(wm, mt) * 16 + r16, kk * 4 + q4);
+                if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(tile + ((wm * C::MT + mt) * 2 + kk) * 1024 + lane * 16);
+                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(tile, km, wm * C::MT + mt, kk);
+                else f[mh][kk] = g3_frag(tile, (wm * C::MT + mt) * 16 + r16, kk * 4 + q4);
             }
     };
     auto readB = [&](const unsigned char* tile, int half, bf16x8 (&f)[HN][2]) {
@@ -334,7 +333,7 @@ struct G3Out {
         unsigned char* const to = smem + (wn * (16 * HT) + r16) * (4 * C::BM); /* (16 tokens further the swizzle is the same) */
 #pragma unroll
         for (int mt = 0; mt < C::MT; mt++) {
-            unsigned char* const b = to + (((C::row_block(wm, mt) * 4 + q4) ^ r16) << 4);
+            unsigned char* const b = to + ((((wm * C::MT + mt) * 4 + q4) ^ r16) << 4);
 #pragma unroll
             for (int nt = 0; nt < HT; nt++) *reinterpret_cast<f32x4*>(b + nt * 16 * (4 * C::BM)) = PASSES == 2 && pass ? acc[mt][nt + C::NT - HT] : acc[mt][nt];
         }
@@ -388,7 +387,7 @@ struct G3Out16 {
         const int wid = tid >> 6, lane = tid & 63, wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
 #pragma unroll
         for (int mt = 0; mt < C::MT; mt++) {
-            const int blk = C::row_block(wm, mt);
+            const int blk = wm * C::MT + mt; /* the wave's 16-row block mt in the tile */
             float b[4] = {0.f, 0.f, 0.f, 0.f};
             if constexpr (BIAS) {
                 u32x2 b4 = u32x2{0, 0};

@@ -150,12 +150,10 @@ struct EngineHost;
 struct Knobs {
     int q4_perm = 1;      /* 4-bit mat-vec through the register-table lookup (0: the arithmetic form; same bits) */
     int q2_tab = 1;       /* 2-bit mat-vec through the LDS selector table (0: the arithmetic form; same bits) */
-    int g3_tiles = 3;     /* smallest bf16 tile gemm3_launch may pick: 0 = 128 x 128 only, 1 = + 64 x 128, 3 = + 64 x 64 (kf_gemm3.hip) */
     int resident_min = 320;  /* token rows from which the token-batch routes use RESIDENT dequantised copies (kf_set_dequant_arena) + the bf16 tile kernels; without an arena: 1024 */
     int attn_pair_min = 256;  /* prompt tokens from which kf_attn_prefill takes its paired two-key-half form (when there is about one workgroup per CU or fewer) */
     int attn_walk_min = 512;  /* keys from which it otherwise takes the walk whose tiles come by loads into LDS (same bits) */
-    int g3_wide = 1;      /* kf_gemm3.hip: 192 x 256 tiles where g3_prefer_wide says so (0: 256 x 256; same bits) */
-    int g3_mid_min = 192; /* 64 x 128 tiles from this many of them, 64 x 64 below */
+    int g3_wide = 1;      /* kf_gemm3.hip: tiles of 192 rows may be picked (0: the choice is among the others; same bits) */
     int attn_gq_split = 4; /* canonical decode attention of a GQA-8 model: workgroups per (kv-head, slice), 2 or 4 */
     int g3_first = 256;   /* token rows from which bf16 operands try the kf_gemm3.hip tile kernels before the 32 x 32 direct kernel */
     int q1_tab = 1;       /* 1-bit mat-vec through the LDS selector table (0: the per-bit select form; same bits) */
