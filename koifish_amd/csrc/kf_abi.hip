@@ -428,8 +428,8 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         if (rc == KF_OK) return KF_OK;
     }
     if (c->arena && nTok >= kf::g_knobs.resident_min && w->type != KF_BF16 && w->quant == KF_QUANT_GROUP && w->ne0 >= 128 && (w->ne1 % 64) == 0) {
-        // a resident copy (kf_set_dequant_arena): nothing to dequantise -- the bf16 tile kernels of kf_gemm3.hip from g_knobs.resident_min token rows (the 1024-row o_proj / down_proj of a
-        // long prompt as 256 tiles of 64 x 128 or 64 x 64)
+        // a resident copy (kf_set_dequant_arena): nothing to dequantise -- the bf16 tile kernels of kf_gemm3.hip from g_knobs.resident_min token rows (gemm3_launch: which
+        // of them go in k-pieces)
         const kf_weight* one[1] = {w};
         const uint16_t* W = nullptr;
         r = deq_copies(c, 1, one, DEQ_STACK, &W, nullptr, true);

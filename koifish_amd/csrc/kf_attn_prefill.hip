@@ -499,12 +499,12 @@ int attn_prefill_mfma_launch(hipStream_t st, const uint16_t* q, const uint16_t* 
     const int TQ = 128 / GQ;
     dim3 grid((n_tok + TQ - 1) / TQ, n_kv, n_seq);
     const int nsb = (n_tok + TQ / 2 - 1) / (TQ / 2); /* the paired form (kh = 2): half blocks of TQ / 2 tokens, one from the front and one from the back per workgroup */
-    // about one workgroup per CU or fewer: the launch lasts as long as its last query block -- two key halves per workgroup (2047 tokens, 16 / 8 heads x 128:
-    // 81 -> 67 us); with more workgroups than that the halves only compete for the CU (8 x 1024 x 25 x 64: 130 vs 143 us; 4095 tokens: 15.9 vs 16.4 ms per prompt)
+    // about one workgroup per CU or fewer: the launch lasts as long as its last query block -- two key halves per workgroup (us, all keys | halves: 16 / 8 heads x 128, 2047 tokens 80 | 46, 1000 tokens 41 | 25,
+    // 2 x 300 15.4 | 13.6; 64 / 8 heads, 512 tokens 23 | 17; 12 heads x 64, 4 x 513 17.2 | 13.2); with more workgroups than that the halves only compete for the CU (8 x 1024 x 25 x 64: 130 vs 143 us).
     // Otherwise the walk by loads into LDS from 512 keys on: its first tiles take longer to come, its step is shorter.  us, staged through registers | by loads: 16 / 8 heads x 128, 128 tokens 8.5 | 9.3, 255 13.6 | 14.1,
-    // 16 prompts of 131 tokens 14.6 | 14.7; 64 / 8 heads, 700 tokens 32.9 | 31.5, 1024 47.4 | 43.4; 16 / 8 heads, 4095 tokens 163 | 152; 25 heads x 64, 8 x 1024 tokens 90.3 | 83.7
-    const bool halves = (long)grid.x * grid.y * grid.z <= 320 && n_tok >= g_knobs.attn_pair_min; /* short prompts: the launch is a few microseconds either way */
+    // 16 prompts of 131 tokens 14.6 | 14.7, 4095 tokens 165 | 153; 64 / 8 heads, 700 tokens 32.5 | 30.8, 1024 47.4 | 43.4; 25 heads x 64, 8 x 1024 tokens 92.0 | 84.2; 12 heads x 64, 6 x 513 23.5 | 22.9
     const bool near = kv_stride < (1 << 24); /* the 32 rows of its tiles in reach of a load's 32-bit offset; the others' are 64-bit */
+    const bool halves = (long)grid.x * grid.y * grid.z <= 320 && n_tok >= g_knobs.attn_pair_min; /* short prompts: the launch is a few microseconds either way */
     const int kh = halves ? 2 : near && pos0 + n_tok >= g_knobs.attn_walk_min ? 0 : 1;
     if (kh == 2) grid.x = (nsb + 1) / 2;
     const int rc = hd == 128 ? ap_launch_gq<128>(st, a, GQ, grid, kh) : ap_launch_gq<64>(st, a, GQ, grid, kh);

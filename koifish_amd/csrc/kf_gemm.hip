@@ -680,7 +680,8 @@ int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long
         const int rc3 = gemm3_launch(st, g.fmt, a, ws, ws_bytes);
         if (rc3 != 1) return rc3;
     }
-    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide (us, staged | direct: 151936 x 1024 bf16 at 16 rows 157 | 100, at 32 160 | 108; 4-bit 80 | 50, 78 | 56)
+    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide.  us, staged | direct, at 8 rows, at 32: bf16 151936 x 1024 154 | 94, 159 | 108; x 2048 295 | 224, 302 | 240; x 5120 808 | 661, 825 | 705;
+    // 50304 x 768 51 | 31, 53 | 33; x 1600 91 | 71, 93 | 76; 65536 x 4096 224 | 176, 229 | 188; 4-bit 151936 x 1024 77 | 45, 76 | 56; 51200 x 5120 159 | 91, 164 | 120; 65536 x 4096 111 | 82, 112 | 113 (24 rows 111 | 108)
     if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max || n <= 32) {
         KS = 0;
         grid = dim3((M + 31) / 32, (n + 31) / 32);

@@ -1,19 +1,19 @@
-// kf_gemm3.hip -- large-batch bf16 GEMM on 256 x 256 x 64 (or 128 x 128 x 64) tiles: y[n, M] (+)= x[n, K] . W[M, K]^T (SLP::Forw's product for a dequantised or bf16
+// kf_gemm3.hip -- large-batch bf16 GEMM on tiles of 64 x 64 to 256 x 256 outputs, 64 deep: y[n, M] (+)= x[n, K] . W[M, K]^T (SLP::Forw's product for a dequantised or bf16
 // weight) and, with either operand stored K-MAJOR, both GEMMs of SLP::Back without a transpose of anything:
 //   * both operand tiles go global -> LDS by buffer loads (16 bytes per lane, no VGPR round trip; a scalar base and step, one lane offset, an empty descriptor past the last step).  The LDS image of
 //     such a load is lane-linear, so the bank-conflict-free layout is produced on the SOURCE side: a tile row is 128 bytes = 8 chunks of 16 bytes, chunk c of row r
 //     is stored at position c ^ ((r >> 1) & 7); a fragment read (16 rows x one chunk, ds_read_b128) then touches all 64 banks exactly once;
 //     a k-major operand's image is [64 k][rows], two-term swizzle, fragments by the transposing ds_read_b64_tr_b16 (g3_frag_km);
-//   * two LDS buffers: the loads of a later k-step are issued among the MFMAs of this one, the fragments of a quadrant are read while the one before is multiplied, and ONE raw s_barrier per
-//     step, behind a wait for everything that was issued a step earlier (in front of the loop only the first step's loads are waited for, by count);
-//   * 256 x 256: 8 waves as 2 (rows) x 4 (tokens), 128 x 64 outputs per wave = 32 accumulator tiles of v_mfma_f32_16x16x32_bf16, one workgroup per CU; 192 x 256 where those fill the chip's
-//     rounds better; 128 x 128: 4 waves as 2 x 2, 64 x 64 outputs per wave, two workgroups per CU -- for products with too few big tiles to fill the chip; 64 x 128 and 64 x 64 below that;
+//   * two or three LDS buffers (G3Cfg::NBUF): the loads of a later k-step are issued among the MFMAs of this one, the fragments of a quadrant are read while the one before is multiplied, and ONE raw
+//     s_barrier per step, behind a wait, by count, for the next step's loads;
+//   * 256 x 256: 8 waves as 2 (rows) x 4 (tokens), 128 x 64 outputs per wave = 32 accumulator tiles of v_mfma_f32_16x16x32_bf16, one workgroup per CU.  A product takes the smallest tile that makes one
+//     round of the CUs, of several rounds the cheaper one (g3_pick; kf_gemm3_tile.h lists the tiles).  All of them add up a k in the same order;
 //   * workgroup order remapped so that the blocks an XCD runs back to back share their W row-tile in that XCD's L2;
 //   * split-K forms (gemm3_sk_kernel) with an ordered in-kernel fix-up for launches with fewer tiles than resident workgroups: deterministic, no atomics on data;
 //   * up to three matrices stacked along M (Q | K | V, gate | up) in one launch, each tile's rows routed to its matrix's output (gemm3_multi_launch).
 // Measured: 8192 x 8192 x 8192 about 1.45 PFLOP/s (1.0 with the fragments of a step read behind its barrier and per-lane global pointers); the MFMAs alone, without a load, reach 2.0 - 2.06 at the card's
 // power limit.  BK = 32 with four buffers, stream-K ranges and 4 waves of 128 x 128 were slower.
-// The epilogue is gemm_epilogue's (alpha, beta, bias, one bf16 store, residual added to the rounded value).
+// The epilogue is gemm_epilogue's (alpha, beta, bias, one bf16 store, residual added to the rounded value), a loop over the tile in LDS (G3Out).
 #include <string.h>
 
 #include <type_traits>
@@ -515,8 +515,8 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
 
 // up to three bf16 matrices stacked along M in ONE contiguous buffer (the caller dequantised them back to back: Q | K | V, or gate | up), each a multiple of 256
 // rows, multiplied by the same x in one launch; matrix j's rows go to y[j] (row stride M[j]).  1 = shape not served.
-// rope != NULL (n_w == 3: Q | K | V, head_dim 128): q/k-norm + RoPE in the epilogue (GemmArgs::qkrope); served on the 128 x 128 tile only -- 1 otherwise, the caller then
-// runs the plain stacked launch and qknorm_rope_launch
+// rope != NULL (n_w == 3: Q | K | V, head_dim 128): q/k-norm + RoPE in the epilogue (GemmArgs::qkrope), on tiles of 128 rows: one head; 1 where Q and K are not whole heads
+// or a pointer is not 16-byte aligned: the caller then runs the plain stacked launch and qknorm_rope_launch
 int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int* M, int K, const uint16_t* x, long long ldx, int n, uint16_t* const* y, const G3Rope* rope) {
     if (n_w < 2 || n_w > 3 || K % G3_BK != 0 || K < G3_BK || n < G3_BN || (ldx & 7) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(Wcat) & 15)) return 1;
     GemmArgs a;
@@ -539,7 +539,8 @@ int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int*
         if (n_w != 3 || M[0] % 128 != 0 || M[1] % 128 != 0 || ((reinterpret_cast<uintptr_t>(y[0]) | reinterpret_cast<uintptr_t>(y[1]) | reinterpret_cast<uintptr_t>(rope->wq) | reinterpret_cast<uintptr_t>(rope->wk) | reinterpret_cast<uintptr_t>(rope->table)) & 15)) return 1;
         a.qkrope = 1, a.qk_norm[0] = rope->wq, a.qk_norm[1] = rope->wk, a.rope_table = rope->table, a.rope_pos0 = rope->pos0, a.rope_seq = rope->seq_len, a.qk_eps = rope->eps;
     }
-    // us, 16 + 8 + 8 heads x 128, K 1024, at 2608 rows: 128 x 128 on 4 waves (672 tiles) 36.7, 128 x 384 (224) 32.4
+    // us, 128 x 128 on 4 waves | 128 x 384 where that is one round: 16 + 8 + 8 heads x 128, K 1024, at 2100 rows 37.1 | 30.5, at 3000 36.5 | 31.0; K 2048, 2608 rows 57.7 | 47.9; 8 + 2 + 2 heads, K 1024, 7500 rows
+    // 36.5 | 31.4; 32 + 8 + 8, K 4096, 1600 rows 98.0 | 80.8; 64 + 8 + 8, K 5120, 1000 rows 127.8 | 96.4
     if (rope) return n128 <= 256 ? g3_whole<G3Duo>(st, a) : g3_tiles_of(tot, n, 128, 256) <= 256 ? g3_whole<G3Half>(st, a) : g3_tiles_of(tot, n, 128, 384) <= 256 ? g3_whole<G3Long>(st, a) : g3_whole<G3Small>(st, a);
     return g3_picked(st, a, false); /* a tile's rows are one matrix's: no 192-row ones */
 }

@@ -24,7 +24,7 @@ using G3Long = G3Cfg<128, 384, 8>;     /* 128 KiB: as many outputs as 192 x 256,
 using G3Duo = G3Cfg<128, 128, 8, 3>;   /* 96 KiB */
 using G3Small = G3Cfg<128, 128, 4>;    /* 64 KiB: two workgroups per CU; the split-K tile of the k-major products */
 using G3Few = G3Cfg<64, 64, 4, 3>;     /* 48 KiB: three */
-// k-pieces of resident copies (gemm3_launch)
+// k-pieces where a workspace is lent (gemm3_launch)
 using G3Mid = G3Cfg<64, 128, 4>;
 using G3Tiny = G3Cfg<64, 64, 4>;
 

@@ -36,7 +36,7 @@ struct GemmArgs {
     int xM[2];
     uint16_t* xy[2];
     long long xldy[2];
-    // kf_gemm3.hip only, the 128 x 128 tile, head_dim 128 (a tile = one head): ROPE::cuInfer (q/k-norm CU_rms_forward_v2 + rotate-half RoPE) in the epilogue of the stacked
+    // kf_gemm3.hip only, tiles of 128 rows, head_dim 128 (a tile = one head): ROPE::cuInfer (q/k-norm CU_rms_forward_v2 + rotate-half RoPE) in the epilogue of the stacked
     // Q | K | V launch -- job 0's rows normed with qk_norm[0], job 1's with qk_norm[1], job 2 (V) stored as it is; position of token t = rope_pos0 + t
     int qkrope;
     const uint16_t* qk_norm[2];

@@ -347,7 +347,8 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
 
 using namespace kf;
 // Up to half a workgroup per CU: two parts of k, a chip full of workgroups.  us per step of 8 recurrent / windowed layers behind 300 tokens, whole | two | four parts: 2048 wide, 32 rows 867 | 828 | 850, 8 rows 537 | 514 | 523, one
-// 473 | 457 | 467; 4096 wide (256 workgroups) 1 row 969 | 978, 16 rows 1238 | 1252
+// 473 | 457 | 467; 4096 wide (256 workgroups) 1 row 969 | 978, 16 rows 1238 | 1252.  A product and its norm, us, whole | two parts, one row, 32: 1024 x 2048 6.6 | 6.2, 8.8 | 7.6; 1024 x 6144 10.1 | 8.4, 15.2 | 11.0;
+// 1536 x 4096 9.2 | 8.2, 12.7 | 10.3; 2048 x 2048 7.7 | 7.6, 9.7 | 8.8; 2048 x 6144 11.4 | 9.9, 16.4 | 12.6
 extern "C" int kf_rb_linear_parts(int type, int m, int k, int n) { return type == KF_BF16 && n >= 1 && n <= KF_RB_DECODE_MAX && m >= 1 && m / 16 <= 128 && k >= 2048 ? 2 : 1; }
 extern "C" int kf_rb_linear_norms(int type, int n, int k) { return type == KF_BF16 && n >= 1 && n <= KF_RB_NORM_ROWS && k % KF_RB_PAD == 0; }
 extern "C" int kf_rb_linear(kf_ctx* c, const kf_rb_product* p) {

@@ -235,8 +235,8 @@ def test_training_size_batch_of_a_quantised_weight_takes_the_dequantise_then_til
 
 @pytest.mark.parametrize("nt,seq", [(1100, 0), (2047, 0), (1280, 160), (2200, 0), (2560, 160)])
 def test_fused_qkv_rope_epilogue_equals_the_two_launch_route(ctx, O, nt, seq):
-    """kf_qkv_rope_batch at >= 1024 tokens: Q | K | V stacked in ONE tile-GEMM launch with q/k-norm + RoPE in its epilogue (a 128-row tile is one head: the token's 128
-    squares meet through row swaps and LDS, a rotation pair's other element sits in the other wave at the same lane) against kf_linear_multi + kf_qknorm_rope_batch:
+    """kf_qkv_rope_batch at >= 1024 tokens: Q | K | V stacked in ONE tile-GEMM launch with q/k-norm + RoPE in its epilogue (a 128-row tile is one head: by way
+    of LDS a thread has eight rotation pairs of a token, the token's 128 squares meet over eight neighbouring threads) against kf_linear_multi + kf_qknorm_rope_batch:
     same tile kernel, same prep_head_cs arithmetic -- every bit of q, k (rotated) and v equal; plus the exact fp64 reference within the batch-GEMM tolerance.
     seq > 0: kf_qkv_rope_seqs -- the rows are sequences of `seq` tokens back to back (a batch of prompts), positions restart in each -- against kf_linear_multi +
     kf_qknorm_rope_train."""
