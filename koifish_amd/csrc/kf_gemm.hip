@@ -680,9 +680,12 @@ int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long
         const int rc3 = gemm3_launch(st, g.fmt, a, ws, ws_bytes);
         if (rc3 != 1) return rc3;
     }
-    // up to 32 rows whatever the matrix: the staged tiles are 128 rows wide.  us, staged | direct, at 8 rows, at 32: bf16 151936 x 1024 154 | 94, 159 | 108; x 2048 295 | 224, 302 | 240; x 5120 808 | 661, 825 | 705;
-    // 50304 x 768 51 | 31, 53 | 33; x 1600 91 | 71, 93 | 76; 65536 x 4096 224 | 176, 229 | 188; 4-bit 151936 x 1024 77 | 45, 76 | 56; 51200 x 5120 159 | 91, 164 | 120; 65536 x 4096 111 | 82, 112 | 113 (24 rows 111 | 108)
-    if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max || n <= 32) {
+    // up to 32 rows of any number of matrix rows in bf16 and 4 bits, up to 8 in the others: the staged tiles are 128 rows wide.  us, staged | direct, at 8 rows, at 32: bf16 151936 x 1024 154 | 94, 159 | 108; x 2048
+    // 295 | 224, 302 | 240; x 5120 808 | 661, 825 | 705; 50304 x 768 51 | 31, 53 | 33; x 1600 91 | 71, 93 | 76; 65536 x 4096 224 | 176, 229 | 188; x 8192 428 | 330, 438 | 360; 4-bit 151936 x 1024 77 | 45, 76 | 56; 51200 x
+    // 5120 159 | 91, 164 | 120; 65536 x 4096 111 | 82, 112 | 113; x 8192 243 | 176, 250 | 211; codebooks x 4096 132 | 85, 136 | 90; 8-bit 65536 x 2048 60 | 58, 62 | 68; x 8192 231 | 198, 240 | 258; 2-bit x 2048
+    // 49 | 41, 49 | 64; x 4096 96 | 79, 96 | 108; 1-bit x 2048 42 | 37, 41 | 56
+    const int few = g.fmt == FMT_BF16 || g.fmt == FMT_Q4 || g.fmt == FMT_Q4R ? 32 : 8;
+    if ((long)((M + 31) / 32) * ((n + 31) / 32) <= direct_max || n <= few) {
         KS = 0;
         grid = dim3((M + 31) / 32, (n + 31) / 32);
     } else {

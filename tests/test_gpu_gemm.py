@@ -458,3 +458,15 @@ def test_tiles_whose_rows_are_no_whole_chunks(ctx, M, K, n, alpha, beta, odd):
     s = alpha * (x.float() @ ctx.dequant(w).float().reshape(M, K).t()) + 7.0 * beta + bias.float()
     assert float((y.float() - s - res.float()).abs().max()) <= 2.0 ** -8 * (float(s.abs().max()) + float((s + res.float()).abs().max()))
     assert bool((buf[0] == 7).all()) and bool((buf[n + 1] == 7).all())
+
+
+@pytest.mark.parametrize("kind", [L.F8E5M2, L.T_SIGN, L.BOOL1])
+def test_few_rows_of_a_tall_narrow_matrix_are_staged(ctx, kind):
+    """8-, 2- and 1-bit matrices of many rows: 32 token rows go through the tiles that 33 go through (those that split k over a workgroup's waves are slower there, and add up in another order)"""
+    w = ctx.quantize((torch.randn(41600, 1024, device=ctx.device) * 0.05).bfloat16(), kind)
+    x, d = torch.randn(33, 1024, device=ctx.device).bfloat16(), w.desc()
+    y = [torch.zeros(33, 41600, device=ctx.device, dtype=torch.bfloat16) for _ in range(2)]
+    for out, n in zip(y, (32, 33)):
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), out.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    assert torch.equal(y[0][:32].view(torch.int16), y[1][:32].view(torch.int16)) and float(y[0].float().abs().max()) > 0
