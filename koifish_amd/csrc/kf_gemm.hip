@@ -526,15 +526,26 @@ static int gm_fmt_of(int type) {
 
 constexpr int GD_NW = 8, GD_UPG = 2; /* direct kernel: 8 waves, groups of two 64-element units, 32-token tiles */
 
-// Token rows by way of LDS, whole lines, from 17 rows (bf16: always): read as fragments a wave's load touches 64 pieces of 16 bytes.  us at 128 rows, fragments | LDS: 4-bit 1024 x 2048 9.6 | 8.5, 1024 x 3072 12.5 | 11.2,
-// 4096 x 1024 8.6 | 7.5, 2048 x 6144 24.6 | 20.6, gate and up 3072 x 1024 13.8 | 11.6; at 16 rows, where the padding repeats one row's lines, 8.1 | 8.3, 11.2 | 10.9, 5.2 | 5.5 (at 8: 7.7 | 8.4, 10.3 | 10.9, 5.0 | 6.0); bf16
-// 151936 x 1024 at 8 rows 115 | 94, at 32 137 | 108.  Same sums in the same order.
+// Token rows by way of LDS, whole lines: read as fragments a wave's load touches 64 pieces of 16 bytes.  Same sums in the same order.  From 17 rows on, below which the padding repeats one row's lines; in bf16, whose weights
+// take as many loads as the rows, also from 9 rows on at K >= 2048, and from K = 3072 or tall ones on always.  A wave's second group of columns takes a second slot, 128 KiB a workgroup: where the unpacking is long
+// (4-bit, 2-bit, 1-bit) two workgroups of a CU hide more than the rows' way gives, as long as a wave has but two groups.  us, fragments | LDS:
+//   128 rows, 4-bit: 1024 x 2048 10.1 | 8.9, 1024 x 3072 12.5 | 11.3, 5120 x 5120 55.6 | 49.9, gate and up 3072 x 1024 14.0 | 11.3; 2-bit 5120 x 5120 58.7 | 46.9; 1-bit 53.8 | 38.0; 8-bit 68.8 | 59.1; bf16 111.7 | 98.4
+//   16 rows: 4-bit 1024 x 2048 8.7 | 8.7, 5120 x 5120 17.7 | 17.6, 4096 x 1024 5.5 | 5.7; bf16 4096 x 1024 5.7 | 6.3, 1024 x 2048 8.3 | 7.8, 5120 x 5120 36.6 | 34.2
+//   8 rows, bf16: 3072 x 1024 6.5 | 6.9, 2048 x 2048 8.8 | 9.2, 1024 x 3072 18.1 | 17.7, 151936 x 1024 115 | 94
+//   K = 1536, 1600, 64 | 128 | 200 rows: 4-bit 4800 x 1600 13.4 18.8 26.3 | 14.8 21.8 33.8; 1-bit 4800 x 1536 11.9 16.5 22.3 | 11.8 17.3 26.4; 8-bit 6400 x 1600 16.3 29.4 | 15.1 26.9; bf16 18.7 31.2 | 16.3 27.0
+//   K = 2048, 200 rows, 4-bit: 448 workgroups 16.6 | 16.0, 896 28.1 | 30.8
+template <int FMT>
+static bool gd_rows_by_lds(const GemmArgs& a, long wgs) {
+    if (a.n <= 16) return FMT == FMT_BF16 && (a.M > 1280 * 32 || a.K >= (a.n > 8 ? 2048 : 3072));
+    constexpr bool unpacks = FMT == FMT_Q4 || FMT == FMT_Q2 || FMT == FMT_Q1;
+    return !(unpacks && a.K > GD_NW * GD_UPG * 64 && (a.K < 2048 || (a.K < 3072 && wgs > 768)));
+}
 template <int FMT, int TB, bool PAIRED>
 static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
     const size_t sums = (size_t)GD_NW * (PAIRED ? 2 : 1) * TB * 16 * 64 * 4;
     const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1; /* one group of a wave, or two in turn */
     const size_t rows = (size_t)GD_NW * slots * TB * 32 * 256;
-    if ((a.n > 16 || FMT == FMT_BF16) && rows <= 128 * 1024 && a.ldx < (1 << 24)) {
+    if (gd_rows_by_lds<FMT>(a, (long)grid.x * grid.y) && rows <= 128 * 1024 && a.ldx < (1 << 24)) {
         static int attr_set = 0;
         if (!attr_set) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024), attr_set = 1;
         hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), grid, dim3(GD_NW * 64), rows > sums ? rows : sums, st, a, slots);

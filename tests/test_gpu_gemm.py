@@ -470,3 +470,19 @@ def test_few_rows_of_a_tall_narrow_matrix_are_staged(ctx, kind):
         assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), out.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
     ctx.sync()
     assert torch.equal(y[0][:32].view(torch.int16), y[1][:32].view(torch.int16)) and float(y[0].float().abs().max()) > 0
+
+
+@pytest.mark.parametrize("kind", [L.BF16, L.F8E5M2, L.Q4, L.T_SIGN, L.BOOL1])
+@pytest.mark.parametrize("M,K", [(96, 1024), (40, 1536), (160, 2048), (33, 3072)])
+def test_rows_of_small_batches_do_not_depend_on_their_way(ctx, kind, M, K):
+    """up to 8, 16 and more token rows, read as fragments or by way of LDS (the rule differs by format and K): a row's sums are the same bits"""
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), kind)
+    x, d = torch.randn(40, K, device=ctx.device).bfloat16(), w.desc()
+    y = {n: torch.zeros(n + 1, M, device=ctx.device, dtype=torch.bfloat16) for n in (8, 9, 16, 17, 32, 40)}
+    for n, out in y.items():
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), out.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    for n, out in y.items():
+        assert torch.equal(out[:n].view(torch.int16), y[40][:n].view(torch.int16)) and bool((out[n] == 0).all()), n
+    ref = x.float() @ ctx.dequant(w).float().reshape(M, K).t()
+    assert float((y[40][:40].float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
