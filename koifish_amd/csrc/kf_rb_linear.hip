@@ -142,8 +142,9 @@ struct RbTokens {
     }
 };
 
-// TURN: the token rows go through RbTokens (rows in order, no experts); else every lane reads its fragments itself
-template <int NT, bool GATED, int NW, bool NORM, bool TURN>
+// TURN: the token rows go through RbTokens (rows in order, no experts); else every lane reads its fragments itself.  PARTS: blockIdx.y is a part of k (a form of its own: 1 % of a decode step of products
+// that have none)
+template <int NT, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
     constexpr int MG = GATED ? 2 : 1, U = NT >= 4 ? 2 : 4;
@@ -153,8 +154,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[RED > STAGE ? RED : STAGE];
     auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
-    const int m0 = blockIdx.x * (16 * MG), part = p.mode == KF_RB_ALL ? (int)blockIdx.y : 0, parts = p.parts > 1 ? p.parts : 1;
-    const int steps = p.k / 32, nstep = parts > 1 ? steps * (part + 1) / parts : steps; /* this part's steps end here */
+    const int m0 = blockIdx.x * (16 * MG), part = PARTS ? (int)blockIdx.y : 0, steps = p.k / 32, nstep = PARTS ? steps * (part + 1) / p.parts : steps; /* this part's steps end here */
     const uint16_t* W = reinterpret_cast<const uint16_t*>(p.w);
     const uint16_t* X = reinterpret_cast<const uint16_t*>(p.x);
     const int32_t* list = nullptr;
@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     }
     const uint16_t* wr = W + (size_t)m0 * p.k + 8 * lane;
     u32x4 a[U][MG], b[U][NT];
-    int s = (parts > 1 ? steps * part / parts : 0) + wid * U;
+    int s = (PARTS ? steps * part / p.parts : 0) + wid * U;
     rb_load_w<MG, U>(a, wr, p.k, s, nstep);
     const uint16_t* xp[NT];
     Tokens tok;
@@ -314,6 +314,8 @@ static void stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     if (p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
     else if (gated && turn) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
     else if (gated) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
+    else if (p.parts > 1 && turn) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, true, true>), grid, dim3(64 * NW), 0, st, q);
+    else if (p.parts > 1) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, false, true>), grid, dim3(64 * NW), 0, st, q);
     else if (turn) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
     else hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
 }
