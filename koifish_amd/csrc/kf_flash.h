@@ -4,9 +4,7 @@
 //      A = V^T fragments straight from the row-major V tile (ds_read_b64_tr_b16).  p enters as a bf16 pair (high part + remainder, ~16 significant bits), its sum stays fp32.
 // What bounds it: a tile's MFMAs take 768 cycles of a SIMD at dim 128, its vector instructions about as many, and one after the other they leave both pipes idle half the time -- a SIMD has two
 // waves at most here, often one.  So a step holds a tile's exponentials and P.V beside the next tile's scores, their scaling and maximum: independent instructions that the compiler mixes.
-// A column's reference exponent M: NAT (scores in natural units, as they were stored) is the maximum of the keys seen so far, subtracted before the factor log2 e, so that the largest p is 1 whatever the scores'
-// size, and a sum does not depend on the tiles' way through LDS.  Otherwise (scores in log2 units) it is moved only when a tile's maximum exceeds it by 8: up to there p just grows to 2^8, which costs no precision in
-// fp32 and bf16 pairs, and the accumulator is rescaled a few times per column instead of at nearly every early tile.
+// A column's reference exponent M is the maximum of the keys seen so far, subtracted before any factor: the largest p is 1 whatever the scores' size, and a sum does not depend on the tiles' way through LDS.
 #pragma once
 #include "kf_device.h"
 
@@ -16,9 +14,9 @@ typedef __bf16 fl_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 fl_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr float FL_SLACK = 8.0f, FL_LOG2E = 1.44269502162933349609375f;
+constexpr float FL_LOG2E = 1.44269502162933349609375f;
 
-template <int HD, bool NAT>
+template <int HD, bool NAT> /* NAT: scores in natural units; else in log2 units */
 struct FlashWave {
     static constexpr int NS = HD / 16, NDB = HD / 32; /* MFMA steps over d of S^T; 32-row blocks of O^T */
     fl_f32x16 o[NDB];
@@ -69,7 +67,7 @@ struct FlashWave {
     static __device__ __forceinline__ float power(float d) { return __builtin_amdgcn_exp2f(NAT ? d * FL_LOG2E : d); } /* of a difference of scores */
     // mt: the column's maximum over the tile (both lanes of the pair)
     __device__ __forceinline__ void move(float mt) {
-        if (mt > (NAT ? M : M + FL_SLACK)) {
+        if (mt > M) {
             const float alpha = power(M - mt); /* M = -inf on the first tile: 0 */
             l *= alpha;
 #pragma unroll

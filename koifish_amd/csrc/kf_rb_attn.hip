@@ -6,7 +6,7 @@
 //   * columns flattened over (token, head): any number of query heads per kv-head;
 //   * keys and values of the batch's own tokens read from the batch, older ones from the slot's ring: a prompt is attended to before its rows overwrite the ring;
 //   * only the tiles between a wave's first chunk start and its last position.
-// Heads of 64 or 128 whose values are as wide take the pipelined walk of kf_flash.h, tiles by loads into LDS (rb_attn_walk_kernel).
+// Heads of 64 or 128 whose values are as wide, a column's keys in one wave: the pipelined walk of kf_flash.h, tiles by loads into LDS (rb_attn_walk_kernel).
 // A decode row is one workgroup per (kv-head, key range): q and the new key are prepared in LDS, each of its four waves walks its own 32-key tiles (staged into LDS of its
 // own, no barrier in the walk) and the four partial softmaxes meet at the end.
 // fp32 storage, prompts with heads of multiples of 16 up to 128: the same scheme on 32-bit MFMAs.  Everything else: a plain form, one wave per (row, head), 32-bit throughout.
@@ -591,8 +591,9 @@ __global__ void __launch_bounds__(256 * KH, HD <= 128 ? 2 : 1) rb_attn_prefill_k
 }
 
 // The same for heads of exactly HD keys and values columns, four waves over all keys: tiles go global -> LDS by buffer loads, several on their way, and a wave's walk is the pipeline of kf_flash.h.
-// us, staged through registers (keys in two halves up to 512 workgroups) | so, 16 heads on 8 of 128: 300 tokens 22.1 | 20.0, 1500 58.7 | 51.0, 3000 109 | 99.5, windowed 4096, 8190 tokens 443 | 313; four
-// sequences of 300 25.9 | 22.6, of 509 with 20 heads on 4 52.4 | 43.0
+// The same sums in the same order as one wave's walk above.  us, staged through registers | so, 16 heads on 8 of 128: 60 tokens 15.7 | 15.2, 200 20.6 | 17.7, 8 x 200 25.3 | 21.4, 4 x 1200 in chunks 88 | 76, 8000 288 | 243;
+// windowed, 4 x 1500 111 | 94, 8190 408 | 322.  Launches of up to 512 workgroups from 256 tokens on are those of two key halves above: 300 tokens 22.1, 1500 58.7 (walked by one wave to a column, which adds up in
+// another order, 20.0 and 51.0)
 template <int HD>
 __global__ void __launch_bounds__(256, 2) rb_attn_walk_kernel(const kf_rb_attention a, const int32_t* __restrict__ seqs) {
     using Wave = FlashWave<HD, false>;
@@ -955,6 +956,7 @@ template <int HD>
 static int prefill_go(hipStream_t st, const kf_rb_attention& a, const int32_t* seqs, int n_seq, int max_n) {
     const dim3 grid((unsigned)(((long long)max_n * (a.n_head / a.n_kv) + 127) / 128), a.n_kv, n_seq);
     if constexpr (HD <= 128) {
+        if ((long)grid.x * grid.y * grid.z <= 512 && max_n >= 256) return prefill_kh<HD, 2>(st, a, seqs, grid);
         if constexpr (HD == 64 || HD == 128) {
             if (a.dim == HD && a.vdim == HD) {
                 constexpr size_t smem = AP_NB * 2 * ApTile<HD>::PART;
@@ -964,7 +966,6 @@ static int prefill_go(hipStream_t st, const kf_rb_attention& a, const int32_t* s
                 return KF_OK;
             }
         }
-        if ((long)grid.x * grid.y * grid.z <= 512 && max_n >= 256) return prefill_kh<HD, 2>(st, a, seqs, grid);
     }
     return prefill_kh<HD, 1>(st, a, seqs, grid);
 }
