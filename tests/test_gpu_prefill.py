@@ -241,3 +241,17 @@ def test_attention_over_cache_rows_far_apart(ctx, form, hd):
     _attention_in_form(ctx, form, q, k, v, near, 0, n, 1, nh, nkv, hd)
     _attention_in_form(ctx, form, q, kf, vf, out, 0, n, 1, nh, nkv, hd, far)
     assert torch.equal(near.view(torch.int16), out.view(torch.int16)) and float(near.float().abs().max()) > 0
+
+
+@pytest.mark.parametrize("form,kept", [("registers", 0.0), ("loads into LDS", 0.0), ("halves", 64.0)])
+def test_attention_adds_up_in_one_order(ctx, form, kept):
+    """the order of a column's keys is part of its sum: equal weights, two large values that cancel and take with them whatever the same walk added between.  Key halves are the even and the odd tiles of 64 keys"""
+    import torch
+    n, hd = 300, 128
+    q, k, v = torch.zeros(n, 2 * hd), torch.randn(n, hd), torch.zeros(n, hd)
+    v[0], v[64:128], v[128] = 2.0 ** 60, 1.0, -2.0 ** 60
+    qd, kd, vd = (t.bfloat16().to(ctx.device) for t in (q, k, v))
+    out = torch.zeros(n, 2 * hd, dtype=torch.bfloat16, device=ctx.device)
+    _attention_in_form(ctx, form, qd, kd, vd, out, 0, n, 1, 2, 1, hd)
+    want = kept / (1.0 + torch.arange(n))[:, None]
+    assert float((out.cpu().float() - want)[160:].abs().max()) <= 2.0 ** -8 * float(want[160:].max())

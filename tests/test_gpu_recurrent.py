@@ -398,6 +398,21 @@ def test_window_attention_scores_far_below_and_above_the_sink(ctx, kind, scale, 
         a.check({0: store_type(x[:1], a.dt)}, decode=True)
 
 
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 64), (48, 48)])
+def test_window_attention_adds_up_in_one_order(ctx, D, V):
+    """the order of a column's keys is part of its sum: equal weights, two large values that cancel and take with them whatever the same walk added between.  Prompts of 256 tokens and more in few workgroups are two
+    walks, over the even and the odd tiles of 32 keys; shorter ones one"""
+    for n, kept in ((300, 32.0), (200, 0.0)):
+        a = Window(ctx, (L.BF16, torch.bfloat16, 0), 2, 1, D, V, 600, 0.0, sink=0)
+        a.new(0)
+        x = a.rows(n)
+        x[:, a.a.v_col:] = 0.0
+        x[0, a.a.v_col:], x[32:64, a.a.v_col:], x[64, a.a.v_col:] = 2.0 ** 60, 1.0, -2.0 ** 60
+        (got, _), = a.feed({0: x}).values()
+        want = 0.6 * kept / (1.0 + np.arange(n))[:, None]
+        assert np.abs(got[96:] - want[96:]).max() <= 2.0 ** -8 * want[96:].max()
+
+
 @pytest.mark.parametrize("how", ["prompt", "portions", "decode"])
 @pytest.mark.parametrize("window", [20, 64, 150])
 def test_window_edges(ctx, kind, window, how):
