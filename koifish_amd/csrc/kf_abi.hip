@@ -423,7 +423,7 @@ int kf_linear(kf_ctx* c, const kf_weight* w, const kf_bf16* x, kf_bf16* y, const
         // rows 111 | 105, 1024 rows 134 | 130, 2047 rows 187 | 185; resident: kf_gemm3.hip) -- not enough to change the sums of every prompt
         const size_t slots = kf::gemm3_sk_ws_bytes();
         void* const lent = w->ne1 >= 3072 ? c->scratch_end(slots) : nullptr;
-        const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, lent, slots);
+        const int rc = kf::gemm_launch(c->stream, &wb, x, w->ne1, nTok, y, w->ne0, bias, alpha, beta, (epilogue & KF_EPI_RESIDUAL) ? residual : nullptr, w->ne0, lent, slots, true);
         if (rc < 0) return fail(rc, "kf_linear (bf16 tile GEMM on the layer's copy) failed with %d", rc);
         if (rc == KF_OK) return KF_OK;
     }

@@ -670,7 +670,7 @@ int gemm_paired_launch(hipStream_t st, const kf_weight* gate, const kf_weight* u
 
 // Returns KF_OK when launched, 1 when the shape is not eligible (the caller then loops the mat-vec), < 0 on error.
 int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long ldx, int n, uint16_t* y, long long ldy, const uint16_t* bias, float alpha,
-                float beta, const uint16_t* residual, long long ldr, void* ws, size_t ws_bytes) {
+                float beta, const uint16_t* residual, long long ldr, void* ws, size_t ws_bytes, bool own_pieces) {
     GmWeight g;
     const int rc = gm_weight(w, g);
     if (rc) return rc;
@@ -678,7 +678,7 @@ int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long
     const int M = g.M;
     GemmArgs a;
     gm_base(a, g, x, ldx, n, y, ldy);
-    a.bias = bias, a.residual = residual, a.ldr = ldr, a.alpha = alpha, a.beta = beta;
+    a.bias = bias, a.residual = residual, a.ldr = ldr, a.alpha = alpha, a.beta = beta, a.own_pieces = own_pieces;
     const int ttiles = (n + GM_TOK - 1) / GM_TOK;
     // prompt-sized batches on small matrices: the wave-independent kernel while its 32 x 32 workgroups fit ~2-3 rounds of the chip
     // (measured crossover against the staged tiles, scratch/ub_gemm.py: 1024 rows up to n ~ 1024, 2048 up to ~ 600, 3072 up to ~ 400)

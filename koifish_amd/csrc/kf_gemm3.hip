@@ -245,6 +245,37 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_kerne
     g3_epilogue<AKM, C>(a, m0, t0, acc, e, smem_raw);
 }
 
+// a tile by one workgroup, its k in S equal pieces that are added up in order: the sums of the S >= 2 split-K form below, bit for bit, where no workgroup is idle that would take a piece
+template <class C>
+__global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_pieces_kernel(const GemmArgs a, int S) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int tid = threadIdx.x, nbx = (a.M + C::BM - 1) / C::BM, nby = (a.n + C::BN - 1) / C::BN, nkt = a.K / G3_BK;
+    int bx, by;
+    g3_tile(g3_remap(blockIdx.x, nbx * nby), nbx, nby, bx, by);
+    const int m0 = bx * C::BM, t0 = by * C::BN;
+    f32x4 acc[C::MT][C::NT], sum[C::MT][C::NT];
+#pragma unroll
+    for (int i = 0; i < C::MT; i++)
+#pragma unroll
+        for (int j = 0; j < C::NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int piece = 1, next = nkt / S;
+    auto between = [&](int kt) __attribute__((always_inline)) {
+        if (kt != next) return;
+#pragma unroll
+        for (int i = 0; i < C::MT; i++)
+#pragma unroll
+            for (int j = 0; j < C::NT; j++) sum[i][j] = piece == 1 ? acc[i][j] : sum[i][j] + acc[i][j], acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        piece++, next = (int)((long long)nkt * piece / S);
+    };
+    g3_mainloop<false, false, G3_BK, C>(a, m0, t0, 0, nkt, acc, smem_raw, tid >> 6, tid & 63, G3Rows(), between);
+#pragma unroll
+    for (int i = 0; i < C::MT; i++)
+#pragma unroll
+        for (int j = 0; j < C::NT; j++) acc[i][j] = sum[i][j] + acc[i][j];
+    const int e = g3_opaque(tid);
+    g3_epilogue<false, C>(a, m0, t0, acc, e, smem_raw);
+}
+
 // SPLIT-K forms for launches with fewer tiles than CUs (a weight gradient [OC, IC] is 49 .. 175 tiles, its contraction 8192 token rows long).  The pieces are cut so
 // that the workgroups an XCD runs side by side stay at (nearly) the SAME k: they share operand strips in that XCD's L2.  (Ranges of a plain stream-K cut drift apart
 // in k and every workgroup then streams its own strips through the fabric -- measured: 496 TFLOP/s.)
@@ -455,6 +486,16 @@ static int g3_whole(hipStream_t st, const GemmArgs& a) { /* one workgroup per ti
     hipLaunchKernelGGL((gemm3_kernel<false, false, G3_BK, C>), dim3((unsigned)g3_tiles_of(a.M, a.n, C::BM, C::BN)), dim3(C::NTH), C::SMEM, st, a);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
+template <class C>
+static int g3_pieces(hipStream_t st, const GemmArgs& a, int S) {
+    static int attr_set = 0;
+    if (!attr_set && C::SMEM > 64 * 1024) {
+        if (hipFuncSetAttribute((const void*)gemm3_pieces_kernel<C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::SMEM) != hipSuccess) return KF_HIP_CHECK;
+        attr_set = 1;
+    }
+    hipLaunchKernelGGL((gemm3_pieces_kernel<C>), dim3((unsigned)g3_tiles_of(a.M, a.n, C::BM, C::BN)), dim3(C::NTH), C::SMEM, st, a, S);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
 static int g3_picked(hipStream_t st, const GemmArgs& a, bool wide) {
     switch (g3_pick(a.M, a.n, a.K, wide && g_knobs.g3_wide)) {
         case G3_DUO: return g3_whole<G3Duo>(st, a);
@@ -471,15 +512,21 @@ int gemm3_launch(hipStream_t st, int fmt, const GemmArgs& a, void* ws, size_t ws
     const int nkt = a.K / G3_BK;
     const long n128 = g3_tiles_of(a.M, a.n, 128, 128), n64 = g3_tiles_of(a.M, a.n, 64, 64);
     if (n128 < 32 && n64 < 64) return 1;
-    // Where the workspace is lent (resident copies, and a layer's own from K = 3072): k-pieces of 64 x 128 or 64 x 64 tiles, when g3_cut says so (a partial is 16 or 32 KiB; the 64 KiB ones of a 128 x 128 tile cost what
-    // they give at K <= 3072).  Which products are cut, and where, is part of their result, and stays: k-pieces of 128 x 128 tiles on 8 waves are faster from K = 6144 on (us at 515 rows, these | those: M 2048 x K 6144 35.5 | 28.6,
-    // 5120 x 8192 98 | 56, 5120 x 25600 344 | 191), but their sums are others, and a 1.7B or 32B prompt in 4 bits is then farther from itself than its error allows
+    // Where the workspace is lent (resident copies, and a layer's own from K = 3072) products go in k-pieces, cut as g3_cut says for 64 x 128 or 64 x 64 tiles.  Which products are cut, and where, is part of their result,
+    // and stays: other cuts are other sums in every layer of a prompt, and a 1.7B or 32B prompt in 4 bits is then farther from itself than its error allows.  Who adds the pieces up is free: other workgroups
+    // (gemm3_sk_kernel) or, of a layer's own copies (a.own_pieces), the tile's workgroup one after the other (gemm3_pieces_kernel), of 64 x 64 tiles or of 128 x 128 on 8 waves.  us, M x K at rows (64 x 64 tiles | 128 x 128): others' | 64 x 64 | 128 x 128:
+    //   1024 x 3072 at 515 rows (144 | 40) 17.8 | 16.4 | 28.0, at 1500 (384 | 96) 23.3 | 20.8 | 26.7, at 2047 (512 | 128) 25.7 | 21.6 | 26.2, at 2608 (656 | 168) 31.1 | 29.0 | 25.6; 1024 x 2048 at 2047 20.6 | 16.2 | 19.9;
+    //   2048 x 4096 at 1030 (544 | 144) 37.0 | 35.6 | 31.5; 2048 x 6144 at 330 (192) 28.7 | 27.3 | 46.8, at 700 (352 | 96) 34.2 | 38.7 | 46.0, at 1300 (672 | 176) 55.7 | 59.7 | 46.2; 2560 x 9728 at 330 (240) 46.7 | 40.2 |
+    //   65.4, at 515 (360) 52.0 | 56.7 | 64.2, at 900 (600 | 160) 71.9 | 85.9 | 64.3; 5120 x 8192 at 330 (480) 49.1 | 51.7 | 55.8, at 450 (640 | 160) 62.1 | 70.0 | 54.2
     if (ws && ws_bytes >= gemm3_sk_ws_bytes() && n128 < 256) {
         const long nmid = g3_tiles_of(a.M, a.n, 64, 128);
         G3SkArgs s;
         int nl;
-        if (nmid >= 192 ? g3_cut<false, G3Mid>(nmid, nkt, s, nl) : g3_cut<false, G3Tiny>(n64, nkt, s, nl))
+        if (nmid >= 192 ? g3_cut<false, G3Mid>(nmid, nkt, s, nl) : g3_cut<false, G3Tiny>(n64, nkt, s, nl)) {
+            if (a.own_pieces && s.S >= 2 && n64 <= (nkt < 96 ? 512 : 256)) return g3_pieces<G3Few>(st, a, s.S);
+            if (a.own_pieces && s.S >= 2 && n64 > 512) return g3_pieces<G3Duo>(st, a, s.S);
             return nmid >= 192 ? g3_go_c<false, false, G3Mid>(st, a, nmid, ws, ws_bytes, 1) : g3_go_c<false, false, G3Tiny>(st, a, n64, ws, ws_bytes, 1);
+        }
     }
     // Otherwise the smallest tile that makes ONE round of the CUs (g3_pick; in front of it 64 x 64: up to two side by side, from K = 6144 one).  us with a residual, 64 x 64 | 64 x 128 (three buffers) | 128 x 128 on 8 waves |
     // 128 x 256 | 128 x 128 on 4 waves:  M 1024 x K 2048 at 515 rows 12.5 | 17.4 | 20.7 | 31.0 | 28.3, at 2047 rows 18.0 | 18.5 | 21.4 | 32.0 | 29.2, at 2608 rows (656 tiles) 22.8 | 23.9 | 21.8 | 32.3 | 29.4;

@@ -135,8 +135,13 @@ template <class F>
 static __device__ void g3_told_apart(unsigned char* __restrict__ a0, unsigned char* __restrict__ a1, unsigned char* __restrict__ b0, unsigned char* __restrict__ b1, F&& f) {
     f(a0, a1, b0, b1);
 }
-template <bool AKM, bool BKM, int BK, class C, class ROWS = G3Rows>
-__device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, int kt0, int kt1, f32x4 (&acc)[C::MT][C::NT], unsigned char* smem_raw, int wid_, int lane, ROWS rows = ROWS()) {
+struct G3Nothing {
+    __device__ __forceinline__ void operator()(int) const {}
+};
+// between(kt): in front of step kt, behind all MFMAs of the step before
+template <bool AKM, bool BKM, int BK, class C, class ROWS = G3Rows, class BETWEEN = G3Nothing>
+__device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, int kt0, int kt1, f32x4 (&acc)[C::MT][C::NT], unsigned char* smem_raw, int wid_, int lane, ROWS rows = ROWS(),
+                                            BETWEEN between = BETWEEN()) {
     static_assert(BK == G3_BK && C::MT % 2 == 0 && C::NT % 2 == 0, "two k-halves of 32 per step, two halves of rows and of tokens per wave");
     constexpr int LPW = C::NIA + C::NIB, HM = C::MT / 2, HN = C::NT / 2; /* loads per wave and step; MFMA blocks per half */
     constexpr int BYTES_A = C::BM * BK * 2, BYTES_B = C::BN * BK * 2;
@@ -296,16 +301,18 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         readA(a_even, 0, a0), readB(b_even, 0, b0);
         if constexpr (C::NBUF == 2) {
             for (int kt = kt0; kt < kt1; kt += 2) {
+                between(kt);
                 step(kt, a_even, b_even, a_odd, b_odd, b0, b1);
-                if (kt + 1 < kt1) step(kt + 1, a_odd, b_odd, a_even, b_even, b1, b0);
+                if (kt + 1 < kt1) between(kt + 1), step(kt + 1, a_odd, b_odd, a_even, b_even, b1, b0);
             }
         } else {
             int cur = 0;
             auto behind = [](int b) { return b + 1 < C::NBUF ? b + 1 : 0; };
             for (int kt = kt0; kt < kt1; kt += 2) {
                 const int one = behind(cur), two = behind(one);
+                between(kt);
                 step(kt, bufA(cur), bufB(cur), bufA(one), bufB(one), b0, b1);
-                if (kt + 1 < kt1) step(kt + 1, bufA(one), bufB(one), bufA(two), bufB(two), b1, b0);
+                if (kt + 1 < kt1) between(kt + 1), step(kt + 1, bufA(one), bufB(one), bufA(two), bufB(two), b1, b0);
                 cur = two;
             }
         }

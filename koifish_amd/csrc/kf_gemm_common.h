@@ -44,6 +44,7 @@ struct GemmArgs {
     int rope_pos0;
     int rope_seq; /* > 0: the rows are sequences of rope_seq tokens back to back (a batch of prompts, a training batch): position of token t = rope_pos0 + t % rope_seq */
     float qk_eps;
+    int own_pieces; /* kf_gemm3.hip only: a product that goes in k-pieces may have a tile's added up by its own workgroup */
     int swiglu; /* kf_gemm3.hip only: W = gate | up interleaved in blocks of 16 rows (dequant_launch ilv_n = 2), M = 2 ffn; the epilogue stores SwiGLU(gate, up) of every FFN row: y[n, ffn] */
 };
 

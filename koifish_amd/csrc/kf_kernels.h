@@ -101,7 +101,7 @@ struct G3Rope { /* ROPE::cuInfer folded into the stacked Q | K | V launch's epil
 int gemm3_multi_launch(hipStream_t st, int n_w, const uint16_t* Wcat, const int* M, int K, const uint16_t* x, long long ldx, int n, uint16_t* const* y, const G3Rope* rope = nullptr);
 int gemm3_swiglu_launch(hipStream_t st, const uint16_t* Wilv, int ffn, int K, const uint16_t* x, long long ldx, int n, uint16_t* act); /* kf_gemm3.hip */
 int gemm_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, long long ldx, int n, uint16_t* y, long long ldy, const uint16_t* bias, float alpha,
-                float beta, const uint16_t* residual, long long ldr, void* ws = nullptr, size_t ws_bytes = 0); /* ws: split-K slots of the small bf16 tiles (gemm3_sk_ws_bytes) */
+                float beta, const uint16_t* residual, long long ldr, void* ws = nullptr, size_t ws_bytes = 0, bool own_pieces = false); /* ws: split-K slots of the small bf16 tiles (gemm3_sk_ws_bytes); own_pieces: GemmArgs::own_pieces */
 
 int gemm_multi_launch(hipStream_t st, int n_w, const kf_weight* const* w, const uint16_t* x, long long ldx, int n, uint16_t* const* y);
 int gemm_paired_launch(hipStream_t st, const kf_weight* gate, const kf_weight* up, const uint16_t* x, long long ldx, int n, uint16_t* act);

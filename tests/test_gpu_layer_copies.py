@@ -232,24 +232,29 @@ def test_flags_written_over_behind_the_copies_are_cleared(ctx):
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
 
 
-@pytest.mark.parametrize("dim,q,kv,ffn,n,pieces", [(1024, 2048, 1024, 3072, 515, 6), (2048, 2048, 1024, 6144, 515, 4)])
-def test_down_is_cut_into_the_same_pieces(ctx, dim, q, kv, ffn, n, pieces):
+# pieces that a tile's workgroup adds up itself, of 64 x 64 and of 128 x 128 tiles, and pieces of other workgroups; numbers of k-steps that the pieces do not divide
+@pytest.mark.parametrize("M,K,n,pieces", [(1024, 3072, 515, 6), (1024, 3072, 2047, 3), (1008, 3200, 700, 6), (656, 9856, 330, 19), (1024, 3072, 2300, 2), (2048, 6144, 1030, 2), (1040, 3200, 2201, 2),
+                                          (2048, 6144, 515, 4), (2064, 6272, 515, 4)])
+def test_down_is_cut_into_the_same_pieces(ctx, M, K, n, pieces):
     """The cuts of k are part of a product's result, so they are told apart here: two large terms that cancel take with them whatever stands in the same piece as they do and nothing else.  Every term is a small whole
-    number or 15 * 2^40 of either sign, the sums of the other pieces are whole numbers below 128: the result is exact."""
-    part = ffn // pieces
-    w = torch.randint(0, 16, (dim, ffn), device=ctx.device).float()
+    number or 15 * 2^40 of either sign, the sums of the other pieces are whole numbers below 512: the result is exact but for its rounding."""
+    steps = K // 64
+    cut = torch.tensor([steps * p // pieces * 64 for p in range(pieces + 1)], device=ctx.device)
+    w = torch.randint(0, 16, (M, K), device=ctx.device).float()
     w[:, 64::128], w[:, 65::128] = 0.0, 15.0                     # a group's range is 0 .. 15: its 4-bit storage holds the numbers as they are
-    w[:, ::part], w[:, part - 1::part] = 15.0, 15.0
-    ws, _ = _layer(ctx, dim, q, kv, ffn)
-    ws[6] = ctx.quantize(w.bfloat16(), L.Q4)
+    lo, hi = cut[:-1], cut[1:]
+    first, last, mid = lo + 32, hi - 32, lo + 200
+    w[:, first], w[:, last] = 15.0, 15.0
+    ws, _ = _layer(ctx, 1024, 2048, 1024, 3072)
+    ws[6] = ctx.quantize(w.bfloat16(), L.Q4)                     # (the last matrix: widths are not compared)
     assert torch.equal(ctx.dequant(ws[6]).float().view_as(w), w)
     descs = [e.desc() for e in ws]
-    x, at = torch.zeros(n, ffn, device=ctx.device), torch.arange(n, device=ctx.device) % pieces
-    x[:, 200::part] = 1.0
-    x[torch.arange(n), at * part], x[torch.arange(n), at * part + part - 1] = 2.0 ** 40, -2.0 ** 40
-    small = w[:, 200::part].t()                                  # [pieces, dim]
-    want = small.sum(0) - small[at]
-    x, y = x.bfloat16(), torch.zeros(n, dim, device=ctx.device, dtype=torch.bfloat16)
+    x, at = torch.zeros(n, K, device=ctx.device), torch.arange(n, device=ctx.device) % pieces
+    x[:, mid] = 1.0
+    x[torch.arange(n), first[at]], x[torch.arange(n), last[at]] = 2.0 ** 40, -2.0 ** 40
+    small = w[:, mid].t()                                        # [pieces, M]
+    want = (small.sum(0) - small[at]).bfloat16()
+    x, y = x.bfloat16(), torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
     try:
         need, scratch = _copies(ctx, descs, n)
         assert need and ctx.hip.kf_linear(ctx.h, C.byref(descs[6]), x.data_ptr(), y.data_ptr(), None, n, 1.0, 0.0, 0, None) == 0
@@ -257,7 +262,7 @@ def test_down_is_cut_into_the_same_pieces(ctx, dim, q, kv, ffn, n, pieces):
         ctx.sync()
     finally:
         ctx.hip.kf_set_scratch(ctx.h, None, 0)
-    assert torch.equal(y.float(), want)
+    assert torch.equal(y, want)
 
 
 def test_copies_whose_offsets_pass_32_bits(ctx):
