@@ -837,7 +837,7 @@ __global__ void __launch_bounds__(1024) argmax_rows_state_kernel(const uint16_t*
     float best = -__builtin_inff();
     int bi = 0x7fffffff;
     auto take = [&](float v, int i) { /* ascending i per thread: its first maximum.  No comparison with a NaN holds, so none is taken */
-        if (v > best || (v == best && i < bi)) best = v, bi = i;
+        if (v > best) best = v, bi = i;
     };
     // few workgroups, each a serial walk: eight 16-byte loads per thread at a time (16 rows of 151936: one 2-byte load at a time 50 us, so 8)
     const int n8 = (ld & 7) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0 ? n / 8 : 0;
@@ -866,7 +866,7 @@ __global__ void __launch_bounds__(1024) argmax_rows_state_kernel(const uint16_t*
         for (int w = 1; w < 16; w++)
             if (better(sv[w], si[w], best, bi)) best = sv[w], bi = si[w];
         const float v0 = bf2f(row[0]);
-        if (v0 != v0) bi = 0; /* nothing exceeds a NaN that stands first */
+        if (v0 != v0 || bi == 0x7fffffff) bi = 0; /* nothing exceeds a NaN that stands first, and nothing but -inf is there */
         const int seq = d_seq[blockIdx.x];
         int32_t* st = states + 4 * (size_t)seq;
         const int p = st[1];
