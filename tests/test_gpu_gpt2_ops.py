@@ -34,6 +34,23 @@ def test_layernorm_bit_exact(ctx, rows, dim, with_bias):
     assert np.array_equal(mean.cpu().numpy(), rm) and np.array_equal(rstd.cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("rows", [5119, 5120, 5121])
+@pytest.mark.parametrize("ln", [True, False])
+def test_norm_rows_written_through_and_not(ctx, rows, ln):
+    """results on both sides of 10 MB, where the stores change: every row is the oracle's, and nothing behind the last one is written"""
+    dim, dev = 1024, ctx.device
+    rng = np.random.default_rng(rows)
+    x = O.f32_to_bf16(rng.normal(0.3, 2.0, size=(rows, dim)).astype(np.float32))
+    w, b = O.f32_to_bf16((1 + rng.normal(0, 0.1, size=dim)).astype(np.float32)), O.f32_to_bf16(rng.normal(0, 0.1, size=dim).astype(np.float32))
+    xd, wd, bd = bf16_t(x, dev), bf16_t(w, dev), bf16_t(b, dev)
+    y = torch.full((rows + 1, dim), 7.0, dtype=torch.bfloat16, device=dev)
+    if ln: assert ctx.hip.kf_layernorm(ctx.h, xd.data_ptr(), wd.data_ptr(), bd.data_ptr(), y.data_ptr(), rows, dim, 1e-5, None, None) == 0
+    else: assert ctx.hip.kf_rmsnorm(ctx.h, xd.data_ptr(), wd.data_ptr(), y.data_ptr(), rows, dim, 1e-6, None) == 0
+    ctx.sync()
+    want = O.layernorm(x, w, b, 1e-5) if ln else O.rmsnorm(x, w, 1e-6)
+    assert np.array_equal(u16(y[:rows]), want) and bool((y[rows] == 7.0).all())
+
+
 def test_gelu_bit_exact(ctx):
     rng = np.random.default_rng(5)
     x = O.f32_to_bf16(np.concatenate([rng.normal(0, 3, 70000), [0.0, -0.0, 12.0, -12.0, 1e-30, 40.0, -40.0]]).astype(np.float32))
@@ -230,7 +247,8 @@ def test_activation_backward_bit_exact(ctx):
 
 
 @pytest.mark.parametrize("rows,dim", [(1, 768), (37, 1600), (300, 1024), (700, 5120), (5, 8192), (9, 8), (4100, 128), (8200, 64), (5000, 512), (4097, 256),
-                                      (2348, 72), (1800, 2056), (33100, 24)])  # 4 and 5 rows a workgroup; 3 and 4 of two vectors a thread; 64 and 65
+                                      (2348, 72), (1800, 2056), (33100, 24),   # 4 and 5 rows a workgroup; 3 and 4 of two vectors a thread; 64 and 65
+                                      (9, 136), (64, 2048), (121, 72), (128, 72), (130, 72), (255, 72)])  # partials a chunk: 2 and 1, 8, 16 and 9, 16, 17 and 11, 32 and 31
 @pytest.mark.parametrize("ln", [True, False])
 def test_norm_backward_bit_exact(ctx, rows, dim, ln):
     rng = np.random.default_rng(rows * dim + ln)
