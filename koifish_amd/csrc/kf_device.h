@@ -120,6 +120,10 @@ __device__ __forceinline__ float dpp_f(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
     const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
     const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xF, 0xF, true);
@@ -139,6 +143,30 @@ __device__ __forceinline__ float xsum16(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// v_mfma_f32_4x4x1_16b_f32: sixteen squares b of 4 rows x 4 columns; lane 4 b + i brings row i's and column i's operand, register r of lane 4 b + j holds row r, column j.  Every
+// element is ONE fused multiply-add, fmaf's result for every pair of operands (subnormal ones too): a chain of them is a chain of fmaf.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4_t mx_fma(float row, float col, f32x4_t acc) { return __builtin_amdgcn_mfma_f32_4x4x1f32(row, col, acc, 0, 0, 0); }
+// register c of lane 4 b + i: what register i of lane 4 b + c held
+__device__ __forceinline__ void quad_transpose(uint32_t (&r)[4], int lane) {
+    const bool o = lane & 1, h = lane & 2;
+    const uint32_t x0 = dpp_u<0xB1>(r[0]), x1 = dpp_u<0xB1>(r[1]), x2 = dpp_u<0xB1>(r[2]), x3 = dpp_u<0xB1>(r[3]); /* (every lane takes part: not inside the choices) */
+    const uint32_t n0 = o ? x1 : r[0], n1 = o ? r[1] : x0, n2 = o ? x3 : r[2], n3 = o ? r[3] : x2;
+    const uint32_t y0 = dpp_u<0x4E>(n0), y1 = dpp_u<0x4E>(n1), y2 = dpp_u<0x4E>(n2), y3 = dpp_u<0x4E>(n3);
+    r[0] = h ? y2 : n0, r[2] = h ? n2 : y0, r[1] = h ? y3 : n1, r[3] = h ? n3 : y1;
+}
+// the first two levels of the lane tree over such squares (neighbouring squares first: group_sum's order): lane 4 t + j of sixteen gets row t, column j, summed over their four squares
+__device__ __forceinline__ float mx_tree4(f32x4_t v, int lane) {
+    const bool t1 = lane & 4, t2 = lane & 8;
+    float m[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const float a = v[2 * p] + dpp_f<0x104>(v[2 * p]), b = v[2 * p + 1] + dpp_f<0x114>(v[2 * p + 1]); /* squares 0 + 1 and 2 + 3: in the even fours for a, in the odd ones for b */
+        m[p] = t1 ? b : a;
+    }
+    const float lo = m[0] + dpp_f<0x108>(m[0]), hi = m[1] + dpp_f<0x118>(m[1]);
+    return t2 ? hi : lo;
+}
 __device__ __forceinline__ double xsum32_d(double v) {
     const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
     const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);

@@ -169,6 +169,33 @@ struct XCfg {
                                   SH::P6::nBlk == SH::P6::iters * SH::P6::LPR;
     static constexpr int maxR = (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R) > (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R) ? (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R)
                                                                                                                                       : (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R);
+    // MF: the 4-bit phases of the batched form on the matrix cores (xe_unit_mf): a wave takes UNITS of 4 KiB, four loads of a whole KiB each
+    static constexpr bool MF = NB_ > 1 && FMT_ == FMT_Q4P && SH::P1::LPR >= 32 && SH::P4::LPR >= 32 && SH::P5::LPR >= 32 && SH::P6::LPR >= 32;
+    template <class P>
+    struct MG { /* a phase's figures (P: PlanT): units of CE block columns x RS rows, 64 / CE sets of four; a slot: RS rows, all its NIT units */
+        static constexpr int CE = P::nBlk % P::LPR == 0 ? P::LPR : 32, RS = 4 * (64 / CE), NIT = P::nBlk / CE, H = P::LPR / CE, SPG = P::R / RS;
+        static constexpr int ce_log2 = CE == 64 ? 6 : 5, rs_log2 = CE == 64 ? 2 : 3;
+        /* a row's lanes are walked CE at a time (H parts of them, in turn), a part's lanes through all their blocks: unit k of a slot is the column piece (order >> 4 k) & 15 = part + H j, j rising; bit k of `ends`:
+           the last unit of its part */
+        static constexpr unsigned long long order() {
+            unsigned long long o = 0;
+            int k = 0;
+            for (int h = 0; h < H; h++)
+                for (int it = h; it < NIT; it += H) o |= (unsigned long long)it << (4 * k++);
+            return o;
+        }
+        static constexpr uint32_t ends() {
+            uint32_t e = 0;
+            int k = 0;
+            for (int h = 0; h < H; h++)
+                for (int it = h; it < NIT; it += H, k++) e |= it + H >= NIT ? 1u << k : 0u;
+            return e;
+        }
+        static constexpr bool ok = (CE == 32 || CE == 64) && P::nBlk % CE == 0 && NIT >= H && NIT <= 16 && (H == 1 || H == 2) && P::R % RS == 0;
+    };
+    static constexpr int RING = MF ? (NWV_ == 8 ? 4 : 2) : DEPTH_; /* entries (MF: units) of a phase in flight per wave */
+    static_assert(!MF || !PREP, "sixteen bytes a lane");
+    static_assert(!MF || (MG<typename SH::P1>::ok && MG<typename SH::P4>::ok && MG<typename SH::P5>::ok && MG<typename SH::P6>::ok), "whole entries, whole slots");
     static_assert(NB_ >= 1 && NB_ <= 4, "sequences per decoder");
     static_assert(!COOP || NP == NB_, "cooperative staging: a merge / norm scratch per sequence");
     static_assert(NB_ == 1 || (!TP_ && WPC_ == 1 && !FUSED && NG == 1 && (FMT_ == FMT_Q4P || PREP) && DIM_ / 256 <= 12 && FFNP / 256 <= 24 && !COMB_IN_XS1),
@@ -183,8 +210,12 @@ struct XLay {
     static constexpr int xs_bytes = (maxK * 4 + 15) & ~15, xr_bytes = (C::DIM * 2 + 15) & ~15;
     static constexpr size_t o_attn = (size_t)2 * xs_bytes + 2 * xr_bytes;
     static constexpr size_t o_outb = (o_attn + sizeof(uint16_t) * ((size_t)2 * GQ * hd + 3 * hd) + 15) & ~(size_t)15;
-    static constexpr size_t o_wmax = o_outb + 4 * (size_t)((C::maxR + 63) & ~63);
-    static constexpr size_t seq_bytes = (o_wmax + 4 * 2 * 16 + 15) & ~(size_t)15;
+    /* MF: the head's maxima where the phases' rows were (between the two stand the barriers of the head), and the sequences' blocks 16 bytes apart modulo 64: sixteen lanes of xe_unit_mf read every fourth column of
+       each of four sequences */
+    static constexpr size_t outb_bytes = 4 * (size_t)((C::maxR + 63) & ~63), o_wmax = C::MF ? o_outb : o_outb + outb_bytes;
+    static constexpr size_t seq_apart = (o_outb + outb_bytes + 4 * 2 * 16 + 15) & ~(size_t)15, seq_tight = (o_outb + outb_bytes + 15) & ~(size_t)15, seq_even = ((seq_tight + 47) & ~(size_t)63) + 16;
+    static constexpr size_t seq_bytes = C::MF ? seq_even : seq_apart;
+    static_assert(seq_even <= seq_apart, "no more room than without");
     static constexpr size_t msc_bytes = (sizeof(double) * ((size_t)C::ME * C::SPK) + 4 * 64 + 4 * 128 + 15) & ~(size_t)15; /* the slice merge's scratch of ONE poller ([SPK][ME] fp64 + shifts + the merged granules; xe_coop_norm_stage: a slot per wave) */
     static constexpr size_t o_msc = (size_t)C::NB * seq_bytes;
     static constexpr size_t o_comb = o_msc + (size_t)C::NP * msc_bytes;
@@ -241,9 +272,9 @@ struct XSeq { /* this workgroup's place in its decoder, and the step's slice */
 // ---- ring of 16-byte blocks in flight (per lane), with their group's step / zero.  ONE ring serves every phase: entry e of a phase is the wave's block e (single-matrix
 // phases) or -- gate | up -- block e / 2 of gate_proj (e even) resp. up_proj (e odd), so a slot that falls idle in one phase's last round takes the next phase's entry of the
 // same index whatever the two phases are.
-template <int D>
+template <int D, bool MF = false>
 struct XRing {
-    u32x4 w[D];
+    u32x4 w[D * (MF ? 4 : 1)]; /* MF: unit d's rows 4 d .. */
     uint16_t st[D], ze[D];
 };
 // One mat-vec phase as RUN-TIME parameters of one wave (all wave-uniform: scalar registers).  The geometry figures are the compile-time constants of PlanT (the lanes per row,
@@ -259,6 +290,8 @@ struct XPhase {
     int n;           /* ring entries this wave walks: its slots x iters (x 2 paired) */
     int row0;        /* first row of the workgroup's piece, counted inside the matrix */
     uint32_t wbytes, gbytes;
+    unsigned long long order; /* XCfg::MF: XCfg::MG (slots of RS rows: rps_log2; units of CE columns: lpr_log2; iters = NIT; n counts units, a slot's gate units in front of its up units) */
+    uint32_t ends;
 };
 // Which of a workgroup's row slots a compute wave walks: slot sl_a + k * sl_b for k = 0 .. n - 1 (XPhase).  Waves w and w + 4 share a SIMD (measured: HW_ID of waves 0 .. 7 =
 // SIMD 1 3 0 2 1 3 0 2) and a SIMD's waves finish one after the other -- a phase lasts as long as the busiest SIMD.  The poller (wave NCW) sits on the SIMD of class NCW & 3,
@@ -343,11 +376,43 @@ __device__ __forceinline__ void xe_issue(const XPhase& P, const XLaneGeo& G, con
     R.ze[d] = __builtin_amdgcn_raw_buffer_load_b16(eng_rsrc((const void*)pz, gbytes), (vblk >> 2) * 2u, (ublk >> 2) * 2u, 0);
 }
 // a phase's first entries into an idle ring
-template <int NCW, int D, int WAUX, int FMT = FMT_Q4P>
-__device__ __forceinline__ void xe_fill(const XPhase& P, int cw, int lane, XRing<D>& R) {
-    const XLaneGeo G = xe_lane_geo(P, lane);
+// the same for unit e of an MF phase into ring slot d: four loads of one row each (of 64 / CE rows), the lane's 16 bytes beside its neighbours' -- with the lanes of a square of xe_unit_mf on four rows a load
+// took a whole cache line for every 16 bytes: the phases stood at 46 GB/s of those for a CU --, and zero / step of the row that the lane holds behind xe_unit_mf's transposition
+template <int D, int WAUX>
+__device__ __forceinline__ void xe_issue_mf(const XPhase& P, const XPhase& NX, bool use_nx, int e, int d, int lane, bool on, XRing<D, true>& R) {
+    auto pick = [](bool c, auto x, auto y) { return c ? x : y; };
+    const int paired = pick(use_nx, +NX.paired, +P.paired), iters = pick(use_nx, +NX.iters, +P.iters), s0 = pick(use_nx, +NX.s0, +P.s0), sl_b = pick(use_nx, +NX.sl_b, +P.sl_b);
+    const int rps_log2 = pick(use_nx, +NX.rps_log2, +P.rps_log2), lpr_log2 = pick(use_nx, +NX.lpr_log2, +P.lpr_log2), nBlk = pick(use_nx, +NX.nBlk, +P.nBlk);
+    const int k = e / iters, in = e - k * iters, sl = paired ? k >> 1 : k;
+    const int it = (int)(pick(use_nx, +NX.order, +P.order) >> (4 * in)) & 15;
+    const bool second = paired && (k & 1);
+    const uint32_t ublk = (uint32_t)(((s0 + sl * sl_b) << rps_log2) * nBlk + (it << lpr_log2));
+    const g_u32x4 w_a = P.m.w, w_b = P.m2.w, w_c = NX.m.w, w_d = NX.m2.w;
+    const g_u16 s_a = P.m.step, s_b = P.m2.step, s_c = NX.m.step, s_d = NX.m2.step;
+    const g_u16 z_a = P.m.zero, z_b = P.m2.zero, z_c = NX.m.zero, z_d = NX.m2.zero;
+    const g_u32x4 pw = pick(use_nx, pick(second, w_d, w_c), pick(second, w_b, w_a));
+    const g_u16 ps = pick(use_nx, pick(second, s_d, s_c), pick(second, s_b, s_a));
+    const g_u16 pz = pick(use_nx, pick(second, z_d, z_c), pick(second, z_b, z_a));
+    const uint32_t wbytes = on ? pick(use_nx, +NX.wbytes, +P.wbytes) : 0u, gbytes = on ? pick(use_nx, +NX.gbytes, +P.gbytes) : 0u;
+    const int set = lane >> lpr_log2, col = lane & ((1 << lpr_log2) - 1);
+    const uint32_t vblk = (uint32_t)(4 * set * nBlk + col), vgrp = (uint32_t)((4 * set + (lane & 3)) * (nBlk >> 2) + (col >> 2));
 #pragma unroll
-    for (int d = 0; d < D; d++) xe_issue<NCW, D, WAUX, FMT>(P, G, P, G, false, d, d, cw, d < P.n, R);
+    for (int r = 0; r < 4; r++) R.w[4 * d + r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(eng_rsrc((const void*)pw, wbytes), vblk * 16u, (ublk + (uint32_t)(r * nBlk)) * 16u, WAUX));
+    R.st[d] = __builtin_amdgcn_raw_buffer_load_b16(eng_rsrc((const void*)ps, gbytes), vgrp * 2u, (ublk >> 2) * 2u, 0);
+    R.ze[d] = __builtin_amdgcn_raw_buffer_load_b16(eng_rsrc((const void*)pz, gbytes), vgrp * 2u, (ublk >> 2) * 2u, 0);
+}
+// a phase's first entries into an idle ring
+template <class C>
+__device__ __forceinline__ void xe_fill(const XPhase& P, int cw, int lane, XRing<C::RING, C::MF>& R) {
+    constexpr int D = C::RING;
+    if constexpr (C::MF) {
+#pragma unroll
+        for (int d = 0; d < D; d++) xe_issue_mf<D, C::WAUX>(P, P, false, d, d, lane, d < P.n, R);
+    } else {
+        const XLaneGeo G = xe_lane_geo(P, lane);
+#pragma unroll
+        for (int d = 0; d < D; d++) xe_issue<C::NCW, D, C::WAUX, C::FMT>(P, G, P, G, false, d, d, cw, d < P.n, R);
+    }
 }
 // one block's 32 products into the lane's chain pair: BlockDotF<FMT> (kf_gemv_blocks.h) on the fp32 activation chunks in LDS, chunk j of block column c at xf[j * XS + c]
 // (XS: the chunk stride, a compile-time constant of the model shape -- the same for every phase, so the eight reads of a block are one address and immediate offsets)
@@ -439,9 +504,91 @@ __device__ __forceinline__ void xe_block_nb(u32x4 w, uint16_t st16, uint16_t ze1
         }
     }
 }
+// A unit's 128 weights a lane against the activations of up to four sequences (XCfg::MF).  As loaded, lane 4 b + i holds four rows' blocks of column 4 b + i; transposed among the four lanes, row i's blocks of the
+// columns 4 b .. 4 b + 3, which is ONE group of 128: the lane forms that group's table once.  The weights then go through mx_fma -- rows the lane's weight, columns the activation of sequence lane & 3 (xc: that
+// sequence's, column 4 b), squares the columns' fours -- as the chains of the canonical order: acc[c][e] = the even / odd chain of column 4 b + c, register r = row r, sequence lane & 3.
+// The vector ALU bounds a phase: 5 instructions a weight for all sequences together and one matrix instruction, a v_fma_f32 of each sequence and weight in its place made it 8.3 at four.  us per layer of Qwen3-0.6B, 32
+// sequences, q | k | v, o, gate | up, down: 14.1, 8.1, 20.6, 14.2 then, 9.2, 5.6, 13.1, 8.4 now (down as four slots of three units on four waves).  One lane's weights by themselves bound to squares (no transposition,
+// lanes of a square on four rows of memory): 11.2, 6.3, 16.8, 8.7.
+template <int XS>
+__device__ __forceinline__ void xe_unit_mf(const u32x4* w4, uint16_t st16, uint16_t ze16, float qb, const f32x4* xc, int lane, f32x4 (&acc)[4][2]) {
+    const float step = bf2f(st16), zero = bf2f(ze16), nb = -(qb * step);
+    uint32_t P[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const uint32_t r = pack_bf16x2(fmaf((float)(2 * k), step, nb), fmaf((float)(2 * k + 1), step, nb));
+        P[k] = pack_bf16x2(bf_lo(r) - zero, bf_hi(r) - zero);
+    }
+    PermLut t;
+#pragma unroll
+    for (int m = 0; m < 4; m++) t.tl[m] = __builtin_amdgcn_perm(P[2 * m + 1], P[2 * m], 0x06040200u), t.th[m] = __builtin_amdgcn_perm(P[2 * m + 1], P[2 * m], 0x07050301u);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t D[4] = {w4[0][3 - i], w4[1][3 - i], w4[2][3 - i], w4[3][3 - i]}; /* dword 3 holds a block's elements 0 .. 7 */
+        quad_transpose(D, lane);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            uint32_t le, he, lo, ho;
+            perm_lookup4(D[c] >> 4, t, le, he);
+            perm_lookup4(D[c], t, lo, ho);
+            const f32x4 X0 = xc[(2 * i) * XS + c], X1 = xc[(2 * i + 1) * XS + c];
+            auto mul = [&](uint32_t sel, float xe, float xo) { /* an even element and the odd one behind it */
+                acc[c][0] = mx_fma(__uint_as_float(__builtin_amdgcn_perm(he, le, sel)), xe, acc[c][0]);
+                acc[c][1] = mx_fma(__uint_as_float(__builtin_amdgcn_perm(ho, lo, sel)), xo, acc[c][1]);
+            };
+            mul(0x07030c0cu, X0.x, X0.y), mul(0x06020c0cu, X0.z, X0.w), mul(0x05010c0cu, X1.x, X1.y), mul(0x04000c0cu, X1.z, X1.w);
+        }
+    }
+}
 // One mat-vec phase of a compute wave: ONE copy of this loop serves every phase.  The ring holds the wave's first min(D, n) entries on entry (xe_fill / the previous phase's
 // last round); entry e + D is requested when entry e has been multiplied, and in the last round slot d takes entry d of the NEXT phase NX (nx_on; they do not depend on the
 // hand-off that separates the phases).  epi(row, v, v2) runs in the lane that owns a finished row (LDS only: no memory operation inside the loop but the refills).
+// the MF form of xe_mv_run (below): the same ring and refills, of units; a slot's parts one after the other.  epi runs in lane 4 t + j of every set for row t of the set's four and sequence j
+template <class C, typename Epi>
+__device__ __forceinline__ void xe_mv_run_mf(const XPhase& P, const XPhase& NX, bool nx_on, int lane, const u32x4* xs, XRing<C::RING, true>& R, Epi&& epi) {
+    constexpr int NB = C::NB, D = C::RING;
+    const int n = P.n;
+    const int t = (lane >> 2) & 3, j = lane & 3, set = lane >> P.lpr_log2, in_set = lane & ((1 << P.lpr_log2) - 1);
+    /* the activations of this lane's sequence (of two: columns 2 and 3 are the first two's again, not looked at) */
+    const f32x4* const xl = reinterpret_cast<const f32x4*>(reinterpret_cast<const unsigned char*>(xs) + (size_t)(NB == 4 ? j : j % NB) * XLay<C>::seq_bytes) + (in_set & ~3);
+    f32x4 acc[4][2];
+    auto clear = [&]() {
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[c][0] = acc[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
+    float sum = 0.f, gate = 0.f; /* of the parts so far; the slot's first matrix */
+#pragma unroll 1
+    for (int e = 0; e < n; e++) {
+        const int k = e / P.iters, in = e - k * P.iters;
+        const bool second = P.paired && (k & 1);
+        xe_unit_mf<C::XS>(R.w, R.st[0], R.ze[0], second ? P.qb2 : P.qb, xl + (((int)(P.order >> (4 * in)) & 15) << P.lpr_log2), lane, acc);
+#pragma unroll
+        for (int d = 0; d + 1 < D; d++) { /* the ring moves on (the unit behind is needed next anyway) */
+#pragma unroll
+            for (int r = 0; r < 4; r++) R.w[4 * d + r] = R.w[4 * d + 4 + r];
+            R.st[d] = R.st[d + 1], R.ze[d] = R.ze[d + 1];
+        }
+        xe_issue_mf<D, C::WAUX>(P, P, false, e + D < n ? e + D : 0, D - 1, lane, e + D < n, R);
+        if ((P.ends >> in) & 1u) { /* the part's chains joined, then the lane tree: a square's four columns, then squares, sixteens, halves */
+            f32x4 v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = acc[c][0] + acc[c][1];
+            float q = xsum16(mx_tree4((v[0] + v[1]) + (v[2] + v[3]), lane));
+            if (P.lpr_log2 == 6) q = xsum32(q);
+            sum = in == P.iters - 1 && (P.ends & ((1u << in) - 1u)) ? sum + q : q; /* (two parts at most: the second one's end is the slot's) */
+            clear();
+        }
+        if (in == P.iters - 1) {
+            if (P.paired && !second) gate = sum;
+            else if (in_set < 16 && j < NB) epi(j, ((P.s0 + (P.paired ? k >> 1 : k) * P.sl_b) << P.rps_log2) + 4 * set + t, P.paired ? gate : sum, sum);
+        }
+    }
+    if (nx_on) { /* the next phase's first units */
+#pragma unroll
+        for (int d = 0; d < D; d++) xe_issue_mf<D, C::WAUX>(NX, NX, false, d, d, lane, d < NX.n, R);
+    }
+}
 template <class C, int D, typename Epi>
 __device__ __forceinline__ void xe_mv_run(const XPhase& P, const XPhase& NX, bool nx_on, int cw, int lane, const u32x4* xs, XRing<D>& R, Epi&& epi, const u32x4* qtab = nullptr) {
     constexpr int NCW = C::NCW, XS = C::XS, NB = C::NB;
@@ -633,6 +780,39 @@ __device__ __forceinline__ void xe_attn_issue(const XArgs& a, const EngLayer& ly
         }
     }
 }
+// behind the barrier that closes the compute waves' sums: the slice's partials, by all of them
+template <class C>
+__device__ __forceinline__ void xe_attn_partials(const XArgs& a, const XLds& L, const XSeq& S, uint32_t gen, int tid) {
+    constexpr int GQ = C::GQW, hd = C::HD, hd_log2 = C::HD == 128 ? 7 : 6, NWA = C::NCW;
+    // the slice's partial {O[hd], L, m} per query head, as {32 bits, generation} granule pairs in this XCD's partial area (an empty slice: sums 0, exponent -inf)
+    constexpr int PSD = hd + 2, ME = C::ME, SPK = C::SPK;
+    unsigned long long* const pbase = reinterpret_cast<unsigned long long*>(reinterpret_cast<uint32_t*>(a.loc + (size_t)S.seq * a.loc_stride) + C::part);
+    const unsigned long long gg = (unsigned long long)gen << 32;
+    for (int i = tid; i < (S.act ? GQ * hd : 0); i += NWA * 64) {
+        const int hq = i >> hd_log2, d = i & (hd - 1);
+        double o = 0.0, Ls = 0.0;
+        float ms = -__builtin_inff();
+        if (!S.empty) {
+#pragma unroll
+            for (int sl = 0; sl < NWA; sl++) ms = fmaxf(ms, (float)L.comb[((size_t)sl * GQ + hq) * PSD + hd + 1]);
+#pragma unroll
+            for (int sl = 0; sl < NWA; sl++) {
+                const double* c = L.comb + ((size_t)sl * GQ + hq) * PSD;
+                const int e = canon_shift((float)c[hd + 1] - ms);
+                o += ldexp_d(c[d], e);
+                Ls += ldexp_d(c[hd], e);
+            }
+        }
+        unsigned long long* dst = pbase + (size_t)(S.h0 + hq) * C::PSH;
+        const size_t oi = ((size_t)(d / ME) * (SPK * ME) + (size_t)S.split * ME + (d & (ME - 1))) * 2, mi = (size_t)hd * SPK * 2 + (size_t)S.split * 4;
+        const unsigned long long ob = __builtin_bit_cast(unsigned long long, o), lb = __builtin_bit_cast(unsigned long long, Ls);
+        *reinterpret_cast<ulonglong2*>(dst + oi) = ulonglong2{gg | (ob & 0xffffffffull), gg | (ob >> 32)};
+        if (d == 0) {
+            *reinterpret_cast<ulonglong2*>(dst + mi) = ulonglong2{gg | __float_as_uint(ms), gg | (lb & 0xffffffffull)};
+            dst[mi + 2] = gg | (lb >> 32);
+        }
+    }
+}
 // compute waves only (the poller meets the three barriers in xe_poller_main).  p4_fill: requests the first o_proj blocks, called when the last batch's tiles are in registers
 // bi: the sub-sequence (XCfg::NB > 1: called once per sequence of the decoder, S and L being that sequence's views); p4_fill runs behind the key loop (the last sequence: the
 // first o_proj blocks; before that: the next sequence's first tiles)
@@ -708,34 +888,7 @@ __device__ __forceinline__ void xe_attn_phase(const XArgs& a, const XLds& L, con
     }
     p4_fill(); /* the first o_proj blocks: two hand-offs (slice partials, ao) lie between here and their use -- inside the key loop the ring would cost the loop 48 registers */
     __syncthreads(); /* the waves' sums in LDS */
-    // the slice's partial {O[hd], L, m} per query head, as {32 bits, generation} granule pairs in this XCD's partial area (an empty slice: sums 0, exponent -inf)
-    constexpr int PSD = hd + 2, ME = C::ME, SPK = C::SPK;
-    unsigned long long* const pbase = reinterpret_cast<unsigned long long*>(reinterpret_cast<uint32_t*>(a.loc + (size_t)S.seq * a.loc_stride) + C::part);
-    const unsigned long long gg = (unsigned long long)gen << 32;
-    for (int i = tid; i < (S.act ? GQ * hd : 0); i += NWA * 64) {
-        const int hq = i >> hd_log2, d = i & (hd - 1);
-        double o = 0.0, Ls = 0.0;
-        float ms = -__builtin_inff();
-        if (!S.empty) {
-#pragma unroll
-            for (int sl = 0; sl < NWA; sl++) ms = fmaxf(ms, (float)L.comb[((size_t)sl * GQ + hq) * PSD + hd + 1]);
-#pragma unroll
-            for (int sl = 0; sl < NWA; sl++) {
-                const double* c = L.comb + ((size_t)sl * GQ + hq) * PSD;
-                const int e = canon_shift((float)c[hd + 1] - ms);
-                o += ldexp_d(c[d], e);
-                Ls += ldexp_d(c[hd], e);
-            }
-        }
-        unsigned long long* dst = pbase + (size_t)(S.h0 + hq) * C::PSH;
-        const size_t oi = ((size_t)(d / ME) * (SPK * ME) + (size_t)S.split * ME + (d & (ME - 1))) * 2, mi = (size_t)hd * SPK * 2 + (size_t)S.split * 4;
-        const unsigned long long ob = __builtin_bit_cast(unsigned long long, o), lb = __builtin_bit_cast(unsigned long long, Ls);
-        *reinterpret_cast<ulonglong2*>(dst + oi) = ulonglong2{gg | (ob & 0xffffffffull), gg | (ob >> 32)};
-        if (d == 0) {
-            *reinterpret_cast<ulonglong2*>(dst + mi) = ulonglong2{gg | __float_as_uint(ms), gg | (lb & 0xffffffffull)};
-            dst[mi + 2] = gg | (lb >> 32);
-        }
-    }
+    xe_attn_partials<C>(a, L, S, gen, tid);
 }
 
 // ---- cooperative RMSNorm staging (XCfg::COOP): wave w owns the 1 KiB units w, w + NWV, ... of the vector.  Sweep until tagged; raw bf16 -> xraw (the residual of the phase
@@ -1038,7 +1191,7 @@ __device__ __forceinline__ void xe_poller_main(const XArgs& a, const XLds& L0, c
 
 // ---- the compute waves
 template <class C>
-__device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, const XSeq (&SS)[C::NB], int epoch, int cw, int lane, XRing<C::DEPTH>& R) {
+__device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, const XSeq (&SS)[C::NB], int epoch, int cw, int lane, XRing<C::RING, C::MF>& R) {
     constexpr int NB = C::NB;
     const XSeq& S = SS[0]; /* the workgroup's place (and, NB == 1, the sequence) */
     using SH = typename C::SH;
@@ -1046,7 +1199,7 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
     using P4 = typename SH::P4;
     using P5 = typename SH::P5;
     using P6 = typename SH::P6;
-    constexpr int NCW = C::NCW, D = C::DEPTH;
+    constexpr int NCW = C::NCW, D = C::RING;
     static_assert(P1::R % 4 == 0 && P4::R % 4 == 0 && P5::R % 4 == 0 && P6::R % 4 == 0, "16-byte pieces");
     static_assert(P1::total == C::P1W * P1::spg && P4::total == XE_NWG * P4::spg && P5::total == XE_NWG * P5::spg && P6::total == XE_NWG * P6::spg, "every workgroup owns rows of every phase");
     static_assert(C::FUSED || (P1::S1 % P1::spg == 0 && P1::S2 % P1::spg == 0), "a workgroup's P1 rows belong to one matrix");
@@ -1069,6 +1222,10 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
     // phase q of a layer (0: q | k | v, 1: o_proj, 2: gate | up, 3: down_proj) as scalars: every field by a chain of selects on q -- never a struct chosen among four (the
     // compiler keeps such a value in scratch memory and every later field read becomes an indexed scratch load, in front of which it drains the weight loads in flight)
     auto sel4 = [](int q, auto v0, auto v1, auto v2, auto v3) { return q == 0 ? v0 : (q == 1 ? v1 : (q == 2 ? v2 : v3)); };
+    auto slots_of = [&](int q) { /* row slots of the workgroup */
+        if constexpr (C::MF) return sel4(q, +C::template MG<P1>::SPG, +C::template MG<P4>::SPG, +C::template MG<P5>::SPG, +C::template MG<P6>::SPG);
+        else return sel4(q, +P1::spg, +P4::spg, +P5::spg, +P6::spg);
+    };
     auto phase_of = [&](int q, const EngLayer& ly) {
         auto uni = [](auto ptr) {
             const unsigned long long v = (unsigned long long)(uintptr_t)ptr;
@@ -1084,7 +1241,17 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
         P.iters = sel4(q, P1::iters, P4::iters, P5::iters, P6::iters), P.rps_log2 = 6 - P.lpr_log2, P.paired = q == 2 ? 1 : 0;
         P.s0 = sel4(q, S.s1, wg * P4::spg, wg * P5::spg, wg * P6::spg), P.Mj = sel4(q, S.M1, P4::M0, P5::M0, P6::M0);
         P.row0 = P.s0 << P.rps_log2;
-        const int spg = sel4(q, P1::spg, P4::spg, P5::spg, P6::spg);
+        if constexpr (C::MF) {
+            using M1 = typename C::template MG<P1>;
+            using M4 = typename C::template MG<P4>;
+            using M5 = typename C::template MG<P5>;
+            using M6 = typename C::template MG<P6>;
+            P.lpr_log2 = sel4(q, +M1::ce_log2, +M4::ce_log2, +M5::ce_log2, +M6::ce_log2), P.rps_log2 = sel4(q, +M1::rs_log2, +M4::rs_log2, +M5::rs_log2, +M6::rs_log2);
+            P.iters = sel4(q, +M1::NIT, +M4::NIT, +M5::NIT, +M6::NIT);
+            P.order = sel4(q, M1::order(), M4::order(), M5::order(), M6::order()), P.ends = sel4(q, M1::ends(), M4::ends(), M5::ends(), M6::ends());
+            P.s0 = P.row0 >> P.rps_log2;
+        }
+        const int spg = slots_of(q);
         const XDeal dl = xe_deal<NCW, C::DEAL_CONTIG, C::NP>(cw, spg, a.deal_wl);
         P.s0 += __builtin_amdgcn_readfirstlane(dl.a), P.sl_b = __builtin_amdgcn_readfirstlane(dl.b);
         P.n = __builtin_amdgcn_readfirstlane(dl.n) * P.iters * (P.paired ? 2 : 1);
@@ -1092,9 +1259,10 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
         P.wbytes = (uint32_t)P.Mj * (uint32_t)P.nBlk * (uint32_t)C::VBYTES, P.gbytes = (uint32_t)P.Mj * (uint32_t)(P.nBlk / 4) * 2u;
         return P;
     };
+    static_assert(!C::MF || P1::RPS * P1::spg % C::template MG<P1>::RS == 0, "a workgroup's rows start at a slot");
     static_assert(P1::nBlk % 4 == 0 && P4::nBlk % 4 == 0 && P5::nBlk % 4 == 0 && P6::nBlk % 4 == 0 && P1::LPR % 4 == 0 && P4::LPR % 4 == 0 && P5::LPR % 4 == 0 && P6::LPR % 4 == 0,
                   "a group's four blocks start at a multiple of four");
-    xe_fill<NCW, D, C::WAUX, C::FMT>(phase_of(0, L.lay[0]), cw, lane, R);
+    xe_fill<C>(phase_of(0, L.lay[0]), cw, lane, R);
     for (int l = 0; l < a.n_layer; l++) {
         const EngLayer& ly = L.lay[l];
         const uint32_t gen = (uint32_t)epoch * (uint32_t)a.n_layer + (uint32_t)l, tag = gen & 0xffffu, tag_next = (gen + 1u) & 0xffffu;
@@ -1113,7 +1281,7 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
             const bool nx_on = q == 0 ? false : (q == 3 ? !last : true); /* behind q | k | v comes the attention (its first tiles are requested instead); the ring is not carried through the head phase */
             const u32x4* xs = (q == 0 || q == 2) ? L.xs[0] : L.xs[1];
             const int nrows = q == 0 ? P1::R : (q == 1 ? P4::R : (q == 2 ? P5::R : P6::R));
-            const int spg = q == 0 ? P1::spg : (q == 1 ? P4::spg : (q == 2 ? P5::spg : P6::spg));
+            const int spg = slots_of(q);
             int nwp = 0; /* waves that own rows of the phase */
 #pragma unroll
             for (int w = 0; w < NCW; w++) nwp += xe_deal<NCW, C::DEAL_CONTIG, C::NP>(w, spg, a.deal_wl).n > 0 ? 1 : 0;
@@ -1124,26 +1292,25 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
             }
             __syncthreads(); /* the phase's activations are staged (B1 / B4 / B5 / B6) */
             if (cw == 0) XE_STAMP(16 + 2 * q);
-            xe_mv_run<C, D>(
-                P, NX, nx_on, cw, lane, xs, R,
-                [&](int b, int row, float v, float v2) {
-                    const XLds Lb = xe_lds_view<C>(L, b);
-                    uint32_t g;
-                    if (q == 0) {
-                        g = (tag << 16) | (uint32_t)f2bf(v);
-                    } else if (C::TP && (q == 1 || q == 3)) {
-                        g = __float_as_uint(v); /* a column shard's row: the un-rounded fp32 partial (xe_publish pushes it to every rank) */
-                    } else if (q == 1) {
-                        g = (tag << 16) | (uint32_t)f2bf(bf2f(Lb.xrawA[row]) + bf2f(f2bf(v))); /* CU_add3: bf16(x + bf16(W.x)) */
-                    } else if (q == 2) {
-                        g = pack_bf16x2(v, v2); /* the two bf16-rounded projections; CU_swiglu_v0 on them runs in xe_publish, once per row with every lane busy (here: the whole wave would walk
-                                                   the exponential and the division for two rows) */
-                    } else {
-                        g = (tag_next << 16) | (uint32_t)f2bf(bf2f(Lb.xrawB[row]) + bf2f(f2bf(v)));
-                    }
-                    Lb.outb[row - P.row0] = g;
-                },
-                L.qtab);
+            auto epi = [&](int b, int row, float v, float v2) {
+                const XLds Lb = xe_lds_view<C>(L, b);
+                uint32_t g;
+                if (q == 0) {
+                    g = (tag << 16) | (uint32_t)f2bf(v);
+                } else if (C::TP && (q == 1 || q == 3)) {
+                    g = __float_as_uint(v); /* a column shard's row: the un-rounded fp32 partial (xe_publish pushes it to every rank) */
+                } else if (q == 1) {
+                    g = (tag << 16) | (uint32_t)f2bf(bf2f(Lb.xrawA[row]) + bf2f(f2bf(v))); /* CU_add3: bf16(x + bf16(W.x)) */
+                } else if (q == 2) {
+                    g = pack_bf16x2(v, v2); /* the two bf16-rounded projections; CU_swiglu_v0 on them runs in xe_publish, once per row with every lane busy (here: the whole wave would walk
+                                               the exponential and the division for two rows) */
+                } else {
+                    g = (tag_next << 16) | (uint32_t)f2bf(bf2f(Lb.xrawB[row]) + bf2f(f2bf(v)));
+                }
+                Lb.outb[row - P.row0] = g;
+            };
+            if constexpr (C::MF) xe_mv_run_mf<C>(P, NX, nx_on, lane, xs, R, epi);
+            else xe_mv_run<C, D>(P, NX, nx_on, cw, lane, xs, R, epi, L.qtab);
             XE_STAMP(32 + 8 * q + (cw & 7)); /* this wave's rows of the phase are done */
             if (C::DBG && S.stamp && lane == 0 && q == 0) {
                 unsigned hw;
@@ -1171,7 +1338,7 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
                             if (b + 1 < NB) {
                                 if (SS[b + 1 < NB ? b + 1 : b].act) xe_attn_issue<C>(a, ly, SS[b + 1 < NB ? b + 1 : b], cw, lane, T, 0, 0);
                             } else {
-                                xe_fill<NCW, D, C::WAUX, C::FMT>(phase_of(1, ly), cw, lane, R);
+                                xe_fill<C>(phase_of(1, ly), cw, lane, R);
                             }
                         },
                         b);
@@ -1544,7 +1711,7 @@ __global__ void __launch_bounds__(C::NWV * 64, (C::NWV * C::WPC + 3) / 4 /* wave
             Sb.grp0 = grp == 0;
         }
     }
-    XRing<C::DEPTH> R;
+    XRing<C::RING, C::MF> R;
     for (int step = 0; step < nst; step++) {
         const int epoch = epoch0 + step;
 #pragma unroll
