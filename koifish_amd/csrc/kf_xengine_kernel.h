@@ -161,6 +161,9 @@ struct XCfg {
     // buffer is idle between the barrier in front of q | k | v (down_proj of the layer before has read it) and the staging of the attention output, which waits for every
     // slice partial of the XCD -- so for this workgroup's, written after the last read of the sums
     static constexpr bool COMB_IN_XS1 = (size_t)maxKc * 8 + (size_t)DIM_ * 4 + sizeof(double) * (size_t)(NWV_ - 1) * GQW * (HD_ + 2) > (size_t)(WPC_ > 1 ? 70 : 140) * 1024; /* (two workgroups per CU: half the LDS each -- the 1.7B shape) */
+    // several sequences: their attentions between ONE set of barriers (xe_attn_all), each with sums of its own, which lie where its activations do -- idle between the barrier behind q | k | v and the staging of the
+    // attention output, which waits for every partial made of them
+    static constexpr bool ALL = NB_ > 1 && sizeof(double) * (size_t)NCW * GQW * (HD_ + 2) <= 2 * (((size_t)maxKc * 4 + 15) & ~(size_t)15);
     static_assert(!COMB_IN_XS1 || sizeof(double) * (size_t)(NWV_ - 1) * GQW * (HD_ + 2) <= (size_t)maxKc * 4, "the sums fit the buffer");
     static constexpr int XS = maxKc / 32; /* chunk stride of the staged activations (16-byte units): chunk j of block column c at [j * XS + c], whatever the phase's width */
     // every phase in whole rows and whole iterations: no masks at the multiply
@@ -219,7 +222,7 @@ struct XLay {
     static constexpr size_t msc_bytes = (sizeof(double) * ((size_t)C::ME * C::SPK) + 4 * 64 + 4 * 128 + 15) & ~(size_t)15; /* the slice merge's scratch of ONE poller ([SPK][ME] fp64 + shifts + the merged granules; xe_coop_norm_stage: a slot per wave) */
     static constexpr size_t o_msc = (size_t)C::NB * seq_bytes;
     static constexpr size_t o_comb = o_msc + (size_t)C::NP * msc_bytes;
-    static constexpr size_t o_cnt = o_comb + (C::COMB_IN_XS1 ? 0 : sizeof(double) * (size_t)NCW * GQ * (hd + 2));
+    static constexpr size_t o_cnt = o_comb + (C::COMB_IN_XS1 || C::ALL ? 0 : sizeof(double) * (size_t)NCW * GQ * (hd + 2));
     static constexpr size_t o_tab = (o_cnt + 64 + 15) & ~(size_t)15; /* FMT_Q1T: the 256 x 16 B selector table of BlockPrep<FMT_Q1T> */
     static constexpr size_t fixed_bytes = o_tab + (C::FMT == FMT_Q1T ? 4096 : (C::FMT == FMT_Q2T ? 2048 : 0));
 };
@@ -255,6 +258,7 @@ __device__ __forceinline__ XLds xe_lds_view(const XLds& L, int b) {
         V.xs[0] = mv(L.xs[0]), V.xs[1] = mv(L.xs[1]), V.xrawA = mv(L.xrawA), V.xrawB = mv(L.xrawB);
         V.qraw = mv(L.qraw), V.kraw = mv(L.kraw), V.vraw = mv(L.vraw), V.qb = mv(L.qb), V.knew = mv(L.knew);
         V.wmax = mv(L.wmax), V.outb = mv(L.outb);
+        if constexpr (C::ALL) V.comb = reinterpret_cast<double*>(V.xs[0]);
         V.msc = reinterpret_cast<double*>(reinterpret_cast<unsigned char*>(L.msc) + (size_t)(b % C::NP) * XLay<C>::msc_bytes); /* the scratch of the sequence's poller */
         return V;
     }
@@ -268,6 +272,18 @@ struct XSeq { /* this workgroup's place in its decoder, and the step's slice */
     int j1, s1, M1, q_out0;
     long long kv_off; /* elements: this sequence's K/V cache behind sequence 0's */
 };
+// SS[b], b uniform and not a constant (an indexed array of them would lie in scratch memory)
+template <int NB>
+__device__ __forceinline__ XSeq xe_seq(const XSeq (&SS)[NB], int b) {
+    XSeq S = SS[0];
+#pragma unroll
+    for (int i = 1; i < NB; i++) {
+        const bool is = b == i;
+        S.seq = is ? SS[i].seq : S.seq, S.sq = is ? SS[i].sq : S.sq, S.pos = is ? SS[i].pos : S.pos, S.len = is ? SS[i].len : S.len, S.t0 = is ? SS[i].t0 : S.t0, S.t1 = is ? SS[i].t1 : S.t1;
+        S.empty = is ? SS[i].empty : S.empty, S.own_new = is ? SS[i].own_new : S.own_new, S.act = is ? SS[i].act : S.act, S.kv_off = is ? SS[i].kv_off : S.kv_off;
+    }
+    return S;
+}
 
 // ---- ring of 16-byte blocks in flight (per lane), with their group's step / zero.  ONE ring serves every phase: entry e of a phase is the wave's block e (single-matrix
 // phases) or -- gate | up -- block e / 2 of gate_proj (e even) resp. up_proj (e odd), so a slot that falls idle in one phase's last round takes the next phase's entry of the
@@ -813,17 +829,63 @@ __device__ __forceinline__ void xe_attn_partials(const XArgs& a, const XLds& L, 
         }
     }
 }
+// a wave's share of the slice's keys (its first batch is on its way): its sums to LDS
+template <class C>
+__device__ __forceinline__ void xe_attn_keys(const XArgs& a, const XLds& L, const XSeq& S, const EngLayer& ly, int cw, int lane, XAttn<C>& T) {
+    constexpr int GQ = C::GQW, hd = C::HD, hd_log2 = C::HD == 128 ? 7 : 6, LPK = hd >> 3, KPW = 64 / LPK, lpk_log2 = hd_log2 - 3, NWA = C::NCW, U = XAttn<C>::U;
+    const int pos = S.pos, t1 = S.t1, grp = lane >> lpk_log2, d0 = (lane & (LPK - 1)) * 8, tstride = NWA * KPW, tstart = S.t0 + cw * KPW + grp;
+    const int nbatch = S.empty ? 0 : (S.t1 - S.t0 + U * tstride - 1) / (U * tstride);
+    CanonAcc<GQ> A;
+    A.init();
+    float qf[GQ][8];
+#pragma unroll
+    for (int hq = 0; hq < GQ; hq++) {
+        const u32x4 qv = *reinterpret_cast<const u32x4*>(L.qb + hq * hd + d0);
+        const uint32_t q4[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) qf[hq][2 * i] = bf_lo(q4[i]), qf[hq][2 * i + 1] = bf_hi(q4[i]);
+    }
+    const float rden = 1.0f / sqrtf((float)hd);
+    auto batch = [&](int b, int buf) {
+        const int tb = tstart + b * U * tstride;
+        u32x4 ck[U], cv[U];
+        bool valid[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int t = tb + u * tstride;
+            valid[u] = t < t1;
+            ck[u] = T.kk[buf][u], cv[u] = T.vv[buf][u];
+            if (valid[u] && t == pos) ck[u] = *reinterpret_cast<const u32x4*>(L.knew + d0), cv[u] = *reinterpret_cast<const u32x4*>(L.vraw + d0);
+        }
+        canon_batch<GQ, LPK, U>(A, qf, ck, cv, valid, lpk_log2, rden);
+    };
+    for (int b = 0; b < nbatch; b += 2) { /* batch b sits in buffer 0 (requested by the phase before, or by the step below), b + 1 goes to buffer 1; requests past the slice are clamped */
+        xe_attn_issue<C>(a, ly, S, cw, lane, T, b + 1, 1);
+        batch(b, 0);
+        if (b + 1 >= nbatch) break;
+        xe_attn_issue<C>(a, ly, S, cw, lane, T, b + 2, 0);
+        batch(b + 1, 1);
+    }
+    canon_wave_to_lds<GQ, LPK>(A, L.comb + (size_t)cw * GQ * (hd + 2), hd, lane, d0);
+}
+// this position's cache rows: the prepared key, the raw value (K.out / V.out alias them in the reference)
+template <class C>
+__device__ __forceinline__ void xe_attn_new_rows(const XArgs& a, const XLds& L, const XSeq& S, const EngLayer& ly, int tid) {
+    if (S.own_new && S.grp0 && tid < C::HD / 8) {
+        g_u16w krow = ly.kcache + (size_t)S.kv_off + (size_t)S.pos * a.kv_stride + (size_t)S.kvh * C::HD;
+        g_u16w vrow = ly.vcache + (size_t)S.kv_off + (size_t)S.pos * a.kv_stride + (size_t)S.kvh * C::HD;
+        *reinterpret_cast<u32x4 KF_GLOBAL*>(const_cast<uint16_t KF_GLOBAL*>(krow) + 8 * tid) = *reinterpret_cast<const u32x4*>(L.knew + 8 * tid);
+        *reinterpret_cast<u32x4 KF_GLOBAL*>(const_cast<uint16_t KF_GLOBAL*>(vrow) + 8 * tid) = *reinterpret_cast<const u32x4*>(L.vraw + 8 * tid);
+    }
+}
 // compute waves only (the poller meets the three barriers in xe_poller_main).  p4_fill: requests the first o_proj blocks, called when the last batch's tiles are in registers
 // bi: the sub-sequence (XCfg::NB > 1: called once per sequence of the decoder, S and L being that sequence's views); p4_fill runs behind the key loop (the last sequence: the
 // first o_proj blocks; before that: the next sequence's first tiles)
 template <class C, typename Fill>
 __device__ __forceinline__ void xe_attn_phase(const XArgs& a, const XLds& L, const XSeq& S, const EngLayer& ly, uint32_t gen, int cw, int lane, XAttn<C>& T, int l, Fill&& p4_fill, int bi = 0) {
-    constexpr int GQ = C::GQW /* the heads of this workgroup's group */, hd = C::HD, hd_log2 = C::HD == 128 ? 7 : 6, LPK = hd >> 3, KPW = 64 / LPK, lpk_log2 = hd_log2 - 3, NWA = C::NCW, U = XAttn<C>::U;
+    constexpr int GQ = C::GQW /* the heads of this workgroup's group */, hd = C::HD, NWA = C::NCW;
     constexpr int NQ = (GQ + NWA - 1) / NWA;
-    const int tid = (cw << 6) | lane, pos = S.pos, t1 = S.t1;
-    const int grp = lane >> lpk_log2, d0 = (lane & (LPK - 1)) * 8;
-    const int tstride = NWA * KPW, tstart = S.t0 + cw * KPW + grp;
-    const int nbatch = S.empty ? 0 : (S.t1 - S.t0 + U * tstride - 1) / (U * tstride);
+    const int tid = (cw << 6) | lane;
     __syncthreads(); /* raw heads staged */
     if (!S.empty) {
         const bool rope = a.rope_table != nullptr, qnorm = ly.norm_q != nullptr;
@@ -847,48 +909,57 @@ __device__ __forceinline__ void xe_attn_phase(const XArgs& a, const XLds& L, con
     }
     __syncthreads(); /* heads prepared */
     if (!S.empty) {
-        if (S.own_new && S.grp0 && tid < hd / 8) { /* the cache rows of this position: the prepared key, the raw value (K.out / V.out alias them in the reference) */
-            g_u16w krow = ly.kcache + (size_t)S.kv_off + (size_t)pos * a.kv_stride + (size_t)S.kvh * hd;
-            g_u16w vrow = ly.vcache + (size_t)S.kv_off + (size_t)pos * a.kv_stride + (size_t)S.kvh * hd;
-            *reinterpret_cast<u32x4 KF_GLOBAL*>(const_cast<uint16_t KF_GLOBAL*>(krow) + 8 * tid) = *reinterpret_cast<const u32x4*>(L.knew + 8 * tid);
-            *reinterpret_cast<u32x4 KF_GLOBAL*>(const_cast<uint16_t KF_GLOBAL*>(vrow) + 8 * tid) = *reinterpret_cast<const u32x4*>(L.vraw + 8 * tid);
-        }
-        CanonAcc<GQ> A;
-        A.init();
-        float qf[GQ][8];
-#pragma unroll
-        for (int hq = 0; hq < GQ; hq++) {
-            const u32x4 qv = *reinterpret_cast<const u32x4*>(L.qb + hq * hd + d0);
-            const uint32_t q4[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) qf[hq][2 * i] = bf_lo(q4[i]), qf[hq][2 * i + 1] = bf_hi(q4[i]);
-        }
-        const float rden = 1.0f / sqrtf((float)hd);
-        auto batch = [&](int b, int buf) {
-            const int tb = tstart + b * U * tstride;
-            u32x4 ck[U], cv[U];
-            bool valid[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int t = tb + u * tstride;
-                valid[u] = t < t1;
-                ck[u] = T.kk[buf][u], cv[u] = T.vv[buf][u];
-                if (valid[u] && t == pos) ck[u] = *reinterpret_cast<const u32x4*>(L.knew + d0), cv[u] = *reinterpret_cast<const u32x4*>(L.vraw + d0);
-            }
-            canon_batch<GQ, LPK, U>(A, qf, ck, cv, valid, lpk_log2, rden);
-        };
-        for (int b = 0; b < nbatch; b += 2) { /* batch b sits in buffer 0 (requested by the phase before, or by the step below), b + 1 goes to buffer 1; requests past the slice are clamped */
-            xe_attn_issue<C>(a, ly, S, cw, lane, T, b + 1, 1);
-            batch(b, 0);
-            if (b + 1 >= nbatch) break;
-            xe_attn_issue<C>(a, ly, S, cw, lane, T, b + 2, 0);
-            batch(b + 1, 1);
-        }
-        canon_wave_to_lds<GQ, LPK>(A, L.comb + (size_t)cw * GQ * (hd + 2), hd, lane, d0);
+        xe_attn_new_rows<C>(a, L, S, ly, tid);
+        xe_attn_keys<C>(a, L, S, ly, cw, lane, T);
     }
     p4_fill(); /* the first o_proj blocks: two hand-offs (slice partials, ao) lie between here and their use -- inside the key loop the ring would cost the loop 48 registers */
     __syncthreads(); /* the waves' sums in LDS */
     xe_attn_partials<C>(a, L, S, gen, tid);
+}
+
+// XCfg::ALL: every sequence's heads, then every sequence's keys, then every sequence's partials, three barriers in all.  One sequence after the other, with barriers of its own, 3.5 us of a sequence's 11 (2 k keys, four
+// sequences) were three waves preparing its heads while the others waited.  ONE copy of the code for all sequences.
+template <class C>
+struct XHeadNorm { /* the lane's pair of the q / k-norm weights */
+    uint16_t q0, q1, k0, k1;
+};
+template <class C, typename Fill>
+__device__ __forceinline__ void xe_attn_all(const XArgs& a, const XLds& L0, const XSeq (&SS)[C::NB], const EngLayer& ly, uint32_t gen, int cw, int lane, XAttn<C>& T, const XHeadNorm<C>& W, Fill&& p4_fill) {
+    constexpr int GQ = C::GQW, hd = C::HD, NWA = C::NCW, NB = C::NB;
+    const int tid = (cw << 6) | lane;
+    __syncthreads(); /* raw heads staged */
+#pragma unroll 1
+    for (int i = cw; i < NB * (GQ + 1); i += NWA) { /* a query head of a sequence, or its new key */
+        const int b = i / (GQ + 1), h = i - b * (GQ + 1);
+        const XSeq S = xe_seq<NB>(SS, b);
+        if (S.empty || (h == GQ && !S.own_new)) continue;
+        const XLds L = xe_lds_view<C>(L0, b);
+        float rc = T.rc[0], rs = T.rs[0];
+#pragma unroll
+        for (int k = 1; k < NB; k++) rc = b == k ? T.rc[k] : rc, rs = b == k ? T.rs[k] : rs;
+        const int half = hd >> 1, j = lane < half ? lane : half - 1;
+        const bool key = h == GQ, norm = (key ? ly.norm_k : ly.norm_q) != nullptr;
+        const uint16_t* const src = key ? L.kraw : L.qraw + h * hd;
+        HeadRaw r;
+        r.x0 = src[j], r.x1 = src[j + half];
+        r.w0 = norm ? (key ? W.k0 : W.q0) : r.x0, r.w1 = norm ? (key ? W.k1 : W.q1) : r.x1;
+        prep_head_cs(r, norm, a.rope_table != nullptr, rc, rs, hd, a.qk_eps, key ? L.knew : L.qb + h * hd, nullptr, lane);
+    }
+    __syncthreads(); /* heads prepared */
+#pragma unroll 1
+    for (int b = 0; b < NB; b++) {
+        const XSeq S = xe_seq<NB>(SS, b), N = xe_seq<NB>(SS, b + 1 < NB ? b + 1 : b);
+        const XLds L = xe_lds_view<C>(L0, b);
+        if (!S.empty) {
+            xe_attn_new_rows<C>(a, L, S, ly, tid);
+            xe_attn_keys<C>(a, L, S, ly, cw, lane, T);
+        }
+        if (b + 1 < NB && N.act) xe_attn_issue<C>(a, ly, N, cw, lane, T, 0, 0); /* the next sequence's first tiles */
+    }
+    p4_fill();
+    __syncthreads(); /* the waves' sums in LDS */
+#pragma unroll 1
+    for (int b = 0; b < NB; b++) xe_attn_partials<C>(a, xe_lds_view<C>(L0, b), xe_seq<NB>(SS, b), gen, tid);
 }
 
 // ---- cooperative RMSNorm staging (XCfg::COOP): wave w owns the 1 KiB units w, w + NWV, ... of the vector.  Sweep until tagged; raw bf16 -> xraw (the residual of the phase
@@ -1153,7 +1224,7 @@ __device__ __forceinline__ void xe_poller_main(const XArgs& a, const XLds& L0, c
             if (!SS[PB + k * NP].empty) xe_ho_qkv<C>(a, xe_lds_view<C>(L0, PB + k * NP), SS[PB + k * NP], tag, lane, dead); /* only a slice with keys needs the heads (an inactive sequence is an empty one) */
         XE_STAMP(2);
 #pragma unroll
-        for (int b = 0; b < NB; b++) { /* the compute waves' attention, sequence after sequence (xe_attn_phase) */
+        for (int b = 0; b < (C::ALL ? 1 : NB); b++) { /* the compute waves' attention: of all sequences (xe_attn_all), or sequence after sequence (xe_attn_phase) */
             __syncthreads(); /* raw heads staged */
             __syncthreads(); /* heads prepared */
             __syncthreads(); /* the waves' sums in LDS */
@@ -1208,6 +1279,7 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
     const float qb1 = S.j1 == 0 ? a.qbias[0] : (S.j1 == 1 ? a.qbias[1] : a.qbias[2]);
     const int wg = S.r;
     XAttn<C> T;
+    [[maybe_unused]] XHeadNorm<C> W{0, 0, 0, 0};
     uint32_t actm = 0; /* bit b: sequence b of the decoder is active */
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -1270,9 +1342,15 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
         const EngLayer& lyn = L.lay[last ? l : l + 1];
         if (NB > 1 || !S.empty) { /* q-norm (waves that prepare a q head) / k-norm (the wave that prepares the new key) weights of this lane's pair */
             const int half = C::HD >> 1, j = lane < half ? lane : half - 1;
-            g_u16 np = cw < C::GQW ? ly.norm_q : ly.norm_k;
-            T.nw0 = T.nw1 = 0;
-            if (np) T.nw0 = np[j], T.nw1 = np[j + half];
+            if constexpr (C::ALL) {
+                W = XHeadNorm<C>{0, 0, 0, 0};
+                if (ly.norm_q) W.q0 = ly.norm_q[j], W.q1 = ly.norm_q[j + half];
+                if (ly.norm_k) W.k0 = ly.norm_k[j], W.k1 = ly.norm_k[j + half];
+            } else {
+                g_u16 np = cw < C::GQW ? ly.norm_q : ly.norm_k;
+                T.nw0 = T.nw1 = 0;
+                if (np) T.nw0 = np[j], T.nw1 = np[j + half];
+            }
         }
         for (int q = 0; q < 4; q++) {
             // q = 0: RMSNorm(x) -> q | k | v rows, then (below) the attention; 1: o_proj + residual -> xB; 2: RMSNorm + gate | up + SwiGLU -> act; 3: down_proj + residual -> next x
@@ -1330,6 +1408,8 @@ __device__ __forceinline__ void xe_compute_main(const XArgs& a, const XLds& L, c
             }
             if (cw == 0) XE_STAMP(17 + 2 * q);
             if (q == 0) { /* q/k-norm + RoPE + attention over the workgroup's key slice; the slice partial into the XCD's partial area; then the first o_proj blocks */
+                if constexpr (C::ALL) xe_attn_all<C>(a, L, SS, ly, gen, cw, lane, T, W, [&]() { xe_fill<C>(phase_of(1, ly), cw, lane, R); });
+                else
 #pragma unroll
                 for (int b = 0; b < NB; b++) { /* sequence after sequence (own positions, own slices, own K / V rows); behind a sequence's key loop the next one's first tiles are requested */
                     xe_attn_phase<C>(
@@ -1596,7 +1676,7 @@ __global__ void __launch_bounds__(C::NWV * 64, (C::NWV * C::WPC + 3) / 4 /* wave
     L.kraw = L.qraw + GQ * hd, L.vraw = L.kraw + hd, L.qb = L.vraw + hd, L.knew = L.qb + GQ * hd;
     L.outb = reinterpret_cast<uint32_t*>(smem + LY::o_outb);
     L.wmax = reinterpret_cast<float*>(smem + LY::o_wmax);
-    L.comb = reinterpret_cast<double*>(smem + (C::COMB_IN_XS1 ? (size_t)LY::xs_bytes : LY::o_comb));
+    L.comb = reinterpret_cast<double*>(smem + (C::ALL ? 0 : C::COMB_IN_XS1 ? (size_t)LY::xs_bytes : LY::o_comb));
     L.msc = reinterpret_cast<double*>(smem + LY::o_msc);
     L.cnt = reinterpret_cast<int*>(smem + LY::o_cnt);
     L.pub = L.cnt + 8;
