@@ -196,6 +196,7 @@ struct XCfg {
         }
         static constexpr bool ok = (CE == 32 || CE == 64) && P::nBlk % CE == 0 && NIT >= H && NIT <= 16 && (H == 1 || H == 2) && P::R % RS == 0;
     };
+    static constexpr bool MFH = MF && HLPR == 64 && HnBlk % 64 == 0; /* the head on the matrix cores too: slots of four rows */
     static constexpr int RING = MF ? (NWV_ == 8 ? 4 : 2) : DEPTH_; /* entries (MF: units) of a phase in flight per wave */
     static_assert(!MF || !PREP, "sixteen bytes a lane");
     static_assert(!MF || (MG<typename SH::P1>::ok && MG<typename SH::P4>::ok && MG<typename SH::P5>::ok && MG<typename SH::P6>::ok), "whole entries, whole slots");
@@ -1451,16 +1452,36 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
             if (r == S.seq) logits = a.logits_r[r], head_w = a.head_w_r[r], vocab = a.vocab_r[r], row0g = a.row0_r[r];
     }
     const int sub = lane >> C::Hlpr_log2, ll = lane & (LPR - 1);
-    const int total = (vocab + RPS - 1) / RPS, spg = (total + NWG - 1) / NWG;
+    constexpr int RPS4 = C::MFH ? 4 : RPS; /* rows of a slot */
+    const int total = (vocab + RPS4 - 1) / RPS4, spg = (total + NWG - 1) / NWG;
     const int s_wg = wg * spg;
     int s_end = s_wg + spg;
     s_end = s_end < total ? s_end : total;
     const int nmine = s_end > s_wg + wave ? (s_end - s_wg - wave + NWV - 1) / NWV : 0;
-    const int nbatch = (nmine + HG - 1) / HG;
-    u32x4 w[2][HG][ITERS];
+    const int nbatch = C::MFH ? nmine : (nmine + HG - 1) / HG;
+    /* the lane, formed where it is used: what is kept of it for every slot goes to scratch memory, and a reload waits for all rows in flight (activations kept for every slot, 64 registers, send the rows there) */
+    [[maybe_unused]] auto fresh_lane = []() {
+        int l;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+        return l;
+    };
+    u32x4 w[2][C::MFH ? 4 : HG][ITERS];
     auto issue = [&](int b, int buf) {
+        if constexpr (C::MFH) { /* four rows, each ITERS KiB: the lane's 16 bytes beside its neighbours' */
+            const int i = b < nmine ? b : (nmine > 0 ? nmine - 1 : 0), row0 = (s_wg + wave + NWV * i) * 4;
+            const unsigned long long at = (unsigned long long)(uintptr_t)(head_w + (size_t)row0 * nBlk);
+            const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at), hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
+            const int rows = __builtin_amdgcn_readfirstlane(vocab - row0 < 4 ? vocab - row0 : 4); /* rows past the last one: zeros */
+            const __amdgpu_buffer_rsrc_t rs = eng_rsrc((const void*)(uintptr_t)(((unsigned long long)hi << 32) | lo), (uint32_t)(rows > 0 ? rows : 0) * (uint32_t)(nBlk * 16));
+            const int ln = fresh_lane();
 #pragma unroll
-        for (int g = 0; g < HG; g++) {
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int it = 0; it < ITERS; it++) w[buf][r][it] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, ln * 16, r * (nBlk * 16) + it * 1024, 0));
+            return;
+        }
+#pragma unroll
+        for (int g = 0; g < (C::MFH ? 0 : HG); g++) {
             int i = b * HG + g;
             i = i < nmine ? i : (nmine > 0 ? nmine - 1 : 0);
             int row = (s_wg + wave + NWV * i) * RPS + sub;
@@ -1488,7 +1509,7 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
                 const XLds Lb = xe_lds_view<C>(L, b);
                 uint32_t* const loc = reinterpret_cast<uint32_t*>(a.loc + (size_t)SS[b].seq * a.loc_stride);
                 if constexpr (ND > 12) eng_poll_stage_norm_long<1, ND, nBlk, false, false, 8>(loc + C::xA, nullptr, tag, a.head_norm, a.eps, Lb.xs[0], Lb.xrawA, lane, a.ws, dead);
-                else eng_poll_stage<1, ND, nBlk, true, false, false>(loc + C::xA, nullptr, tag, a.head_norm, a.eps, Lb.xs[0], nullptr, lane, a.ws, dead, nullptr, L.pub + 3, (S.step + 1) * a.n_layer, 0);
+                else eng_poll_stage<C::MFH ? 2 : 1, ND, nBlk, true, false, C::MFH>(loc + C::xA, nullptr, tag, a.head_norm, a.eps, Lb.xs[0], nullptr, lane, a.ws, dead, nullptr, L.pub + 3, (S.step + 1) * a.n_layer, 0);
             }
         }
     } else {
@@ -1496,9 +1517,9 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
     }
     __syncthreads();
     if (wave >= C::NCW) issue(0, 0);
-    float xf[NB][ITERS][8];
+    float xf[C::MFH ? 1 : NB][ITERS][8];
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
+    for (int b = 0; b < (C::MFH ? 0 : NB); b++) {
         const XLds Lb = xe_lds_view<C>(L, b);
 #pragma unroll
         for (int it = 0; it < ITERS; it++) {
@@ -1514,9 +1535,53 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
     int best_i[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) best_v[b] = -__builtin_inff(), best_i[b] = 0x7fffffff;
-    auto compute = [&](int bt, int buf) {
+    [[maybe_unused]] uint32_t actm = 0;
 #pragma unroll
-        for (int g = 0; g < HG; g++) {
+    for (int b = 0; b < NB; b++) actm |= SS[b].act ? 1u << b : 0u;
+    actm = __builtin_amdgcn_readfirstlane(actm);
+    [[maybe_unused]] float mine_v = -__builtin_inff(); /* MFH: the lane's best, of sequence lane & 3 */
+    [[maybe_unused]] int mine_i = 0x7fffffff;
+    auto compute = [&](int bt, int buf) {
+        if constexpr (C::MFH) { /* four rows against every sequence, as xe_unit_mf: transposed among four lanes, row lane & 3 and the columns 4 (lane / 4) + c of each iteration are this lane's; each product one mx_fma */
+            const int ln = fresh_lane();
+            const int j = ln & 3;
+            const f32x4* const xl = reinterpret_cast<const f32x4*>(reinterpret_cast<const unsigned char*>(L.xs[0]) + (size_t)(NB == 4 ? j : j % NB) * XLay<C>::seq_bytes) + (ln & ~3);
+            f32x4 acc[4][2];
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[c][0] = acc[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int it = 0; it < ITERS; it++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) { /* elements 4 h .. of the columns' eight */
+                    uint32_t D[2][4];
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) D[k][r] = w[buf][r][it][2 * h + k];
+                        quad_transpose(D[k], ln);
+                    }
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const f32x4 X = xl[h * nBlk + it * 64 + c];
+                        acc[c][0] = mx_fma(bf_lo(D[0][c]), X.x, acc[c][0]), acc[c][1] = mx_fma(bf_hi(D[0][c]), X.y, acc[c][1]);
+                        acc[c][0] = mx_fma(bf_lo(D[1][c]), X.z, acc[c][0]), acc[c][1] = mx_fma(bf_hi(D[1][c]), X.w, acc[c][1]);
+                    }
+                }
+            f32x4 v4[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v4[c] = acc[c][0] + acc[c][1];
+            const float v = xsum32(xsum16(mx_tree4((v4[0] + v4[1]) + (v4[2] + v4[3]), ln)));
+            const int row = (s_wg + wave + NWV * bt) * 4 + ((ln >> 2) & 3);
+            if (ln < 16 && bt < nmine && row < vocab && j < NB && ((actm >> j) & 1u)) {
+                const uint16_t o = f2bf(v);
+                logits[(size_t)j * XE_NXCD * vocab + row] = o;
+                const float fv = bf2f(o);
+                if (fv > mine_v || (fv == mine_v && row < mine_i)) mine_v = fv, mine_i = row;
+            }
+            return;
+        }
+#pragma unroll
+        for (int g = 0; g < (C::MFH ? 0 : HG); g++) {
             const int i = bt * HG + g;
             const int row = (s_wg + wave + NWV * i) * RPS + sub;
 #pragma unroll
@@ -1547,10 +1612,20 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
         issue(b + 2, 0);
         compute(b + 1, 1);
     }
+    if constexpr (C::MFH) { /* the wave's maximum of every sequence: lane j, that of sequence j */
+#pragma unroll
+        for (int m = 8; m >= 4; m >>= 1) {
+            const float ov = __shfl_xor(mine_v, m, 64);
+            const int oi = __shfl_xor(mine_i, m, 64);
+            if (ov > mine_v || (ov == mine_v && oi < mine_i)) mine_v = ov, mine_i = oi;
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) best_v[b] = __shfl(mine_v, b, 64), best_i[b] = __shfl(mine_i, b, 64);
+    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
 #pragma unroll
-        for (int m = 32; m > 0; m >>= 1) {
+        for (int m = C::MFH ? 0 : 32; m > 0; m >>= 1) {
             const float ov = __shfl_xor(best_v[b], m, 64);
             const int oi = __shfl_xor(best_i[b], m, 64);
             if (ov > best_v[b] || (ov == best_v[b] && oi < best_i[b])) best_v[b] = ov, best_i[b] = oi;
