@@ -699,9 +699,31 @@ __device__ __forceinline__ void xe_publish(const XLds& L, int phase, uint32_t ta
         if (lane == 0) __hip_atomic_fetch_add(L.pub + phase, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         return;
     }
+    if constexpr (NB > 1) { /* four rows of a sequence a lane, all sequences side by side: piece after piece by one wave, the publication stood 3 - 5 us behind the last row */
+        const int n4 = nrows >> 2;
+        for (int c = lane; c < NB * n4; c += 64) {
+            int b = 0, i = c;
+#pragma unroll
+            for (int k = 1; k < NB; k++) b += c >= k * n4 ? 1 : 0;
+            i = 4 * (c - b * n4);
+            if (!((actm >> b) & 1u)) continue;
+            u32x4 g = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(L.outb) + (size_t)b * LBS + 4 * i);
+            if (phase == 2) { /* as below */
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float gt = bf_lo(g[k]), up = bf_hi(g[k]);
+                    const bool cold = hot != nullptr && hot[i + k] != 1;
+                    g[k] = (tag << 16) | (cold ? 0u : (uint32_t)f2bf((gt * up) / (1.0f + kf_expf(-gt))));
+                }
+            }
+            *reinterpret_cast<u32x4*>(dst + (size_t)b * dst_bs + i) = g;
+            if (plain) *reinterpret_cast<u32x2*>(plain + (size_t)b * plain_bs + i) = u32x2{(g.x & 0xffffu) | (g.y << 16), (g.z & 0xffffu) | (g.w << 16)};
+        }
+        if (lane == 0) __hip_atomic_fetch_add(L.pub + phase, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return;
+    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        if (NB > 1 && !((actm >> b) & 1u)) continue;
         uint32_t* const ob = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(L.outb) + (size_t)b * LBS);
         uint32_t* const db = dst + (size_t)b * dst_bs;
         uint16_t* const pb = plain ? plain + (size_t)b * plain_bs : nullptr;
