@@ -96,6 +96,9 @@ int kf_free(kf_ctx* ctx, void* p);
 int kf_memset(kf_ctx* ctx, void* p, int value, size_t bytes);
 /* `count` 32-bit words of `value`, on the context's stream, no host sync (kf_h2d synchronises: a flag or a seed set between launches goes through this) */
 int kf_memset32(kf_ctx* ctx, void* p, int32_t value, size_t count);
+/* a few 32-bit words (up to KF_PUT_WORDS) from the host, on the context's stream as a kernel's argument: no staging, no host sync, h_src is free on return */
+#define KF_PUT_WORDS 768
+int kf_put_words(kf_ctx* ctx, int32_t* dst, const int32_t* h_src, int count);
 int kf_h2d(kf_ctx* ctx, void* dst, const void* h_src, size_t bytes);
 int kf_d2h(kf_ctx* ctx, void* h_dst, const void* src, size_t bytes);
 int kf_d2d(kf_ctx* ctx, void* dst, const void* src, size_t bytes);
@@ -270,6 +273,8 @@ int kf_norm_lm_head(kf_ctx* ctx, const kf_bf16* x, const kf_bf16* norm_w_or_null
                     int32_t* d_state, int32_t* d_tokens_out, void* scratch);
 /* writes the decode state {token, pos} (a one-thread kernel: capturable, no host staging buffer) */
 int kf_set_state(kf_ctx* ctx, int32_t* d_state, int token, int pos);
+/* the same for a sequence of several, {token, pos, parked, status}: the status word becomes 0 */
+int kf_set_slot_state(kf_ctx* ctx, int32_t* d_state, int token, int pos);
 /* embed lookup driven by device state: token = (d_forced && d_forced[pos] >= 0) ? d_forced[pos] : d_state[0] */
 int kf_embed_state(kf_ctx* ctx, const kf_weight* w, const int32_t* d_state, const int32_t* d_forced, kf_bf16* out);
 

@@ -225,6 +225,8 @@ int kf_rb_list_tiles(int n, int top, int n_expert, int tile);
  * alone.  scratch: kf_rb_pick_scratch(n) bytes. */
 int kf_rb_pick(kf_ctx* ctx, const float* logits, int64_t ld, int vocab, int n, const int32_t* meta, int32_t* d_state, int32_t* d_tokens_out, int tokens_stride, void* scratch);
 size_t kf_rb_pick_scratch(int n);
+/* row j of fp32 logits [n][ld] to the slot meta[4 j + 1] of dst [.][ld]; that slot's status word (d_state[4 slot + 3]) becomes 0 */
+int kf_rb_slot_logits(kf_ctx* ctx, const float* logits, int64_t ld, int n, const int32_t* meta, float* dst, int32_t* d_state);
 /* fp32 logits row -> bf16 (what kf_sample reads) */
 int kf_rb_to_bf16(kf_ctx* ctx, const float* src, kf_bf16* dst, size_t n);
 

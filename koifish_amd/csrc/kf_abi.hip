@@ -208,6 +208,11 @@ int kf_memset32(kf_ctx* c, void* p, int32_t v, size_t count) {
     HIPCHK(hipMemsetD32Async((hipDeviceptr_t)p, v, count, c->stream));
     return KF_OK;
 }
+int kf_put_words(kf_ctx* c, int32_t* dst, const int32_t* src, int count) {
+    CHKCTX(c);
+    if (!dst || !src || count < 1 || count > KF_PUT_WORDS || ((uintptr_t)dst & 3)) return fail(KF_INVALID_ARGS, "kf_put_words: %d words", count);
+    RET(kf::put_words_launch(c->stream, dst, src, count));
+}
 int kf_h2d(kf_ctx* c, void* dst, const void* src, size_t bytes) {
     CHKCTX(c);
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
@@ -1032,6 +1037,11 @@ int kf_set_state(kf_ctx* c, int32_t* d_state, int token, int pos) {
     RET(kf::set_state_launch(c->stream, d_state, token, pos));
 }
 
+int kf_set_slot_state(kf_ctx* c, int32_t* d_state, int token, int pos) {
+    CHKCTX(c);
+    if (!d_state) return fail(KF_INVALID_ARGS, "kf_set_slot_state: null state");
+    RET(kf::set_slot_state_launch(c->stream, d_state, token, pos));
+}
 size_t kf_head_scratch_bytes(void) { return (sizeof(float) + sizeof(int)) * (size_t)kf::KF_MAX_ARGMAX_PARTIALS; }
 
 static int head_impl(kf_ctx* c, const kf_bf16* x, const kf_bf16* norm_w, float eps, const kf_weight* w, kf_bf16* logits, int32_t* d_argmax, int32_t* d_state,

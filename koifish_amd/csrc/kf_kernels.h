@@ -248,6 +248,8 @@ int awq_linear_launch(hipStream_t st, const kf_weight* w, const uint16_t* x, uin
 int awq_dequant_launch(hipStream_t st, const kf_weight* w, uint16_t* out);
 
 int set_state_launch(hipStream_t st, int32_t* d_state, int token, int pos);
+int set_slot_state_launch(hipStream_t st, int32_t* d_state, int token, int pos);
+int put_words_launch(hipStream_t st, int32_t* dst, const int32_t* h_src, int count);
 int hot_rows_launch(hipStream_t st, const int32_t* hot, int n, int32_t* rows, int32_t* count);
 int cold_fill_launch(hipStream_t st, uint16_t* y, const uint16_t* bias, int n);
 int tp_reduce_launch(hipStream_t st, const float* partials, int R, int n, const uint16_t* residual, uint16_t* out);

@@ -1,4 +1,6 @@
 // kf_ops.hip -- the small operators of the decode step and the (load-time) dequant / quantise kernels.
+#include <string.h>
+
 #include "kf_gemm_common.h"
 
 namespace kf {
@@ -1065,6 +1067,23 @@ int tp_reduce_launch(hipStream_t st, const float* partials, int R, int n, const 
 __global__ void set_state_kernel(int32_t* st, int token, int pos) { st[0] = token, st[1] = pos; }
 int set_state_launch(hipStream_t st, int32_t* d_state, int token, int pos) {
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, st, d_state, token, pos);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+__global__ void set_slot_state_kernel(int32_t* st, int token, int pos) { st[0] = token, st[1] = pos, st[3] = 0; }
+int set_slot_state_launch(hipStream_t st, int32_t* d_state, int token, int pos) {
+    hipLaunchKernelGGL(set_slot_state_kernel, dim3(1), dim3(1), 0, st, d_state, token, pos);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+struct PutWords {
+    int32_t v[KF_PUT_WORDS]; /* 3 KiB of the 4 that a launch's arguments may take */
+};
+__global__ void __launch_bounds__(256) put_words_kernel(int32_t* dst, const PutWords w, int count) {
+    for (int i = threadIdx.x; i < count; i += 256) dst[i] = w.v[i];
+}
+int put_words_launch(hipStream_t st, int32_t* dst, const int32_t* h_src, int count) {
+    PutWords w;
+    memcpy(w.v, h_src, (size_t)count * 4);
+    hipLaunchKernelGGL(put_words_kernel, dim3(1), dim3(256), 0, st, dst, w, count);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 

@@ -372,6 +372,18 @@ __global__ void __launch_bounds__(256) rb_pick_part_kernel(const float* __restri
         pv[blockIdx.y * PICK_PIECES + blockIdx.x] = m, pi[blockIdx.y * PICK_PIECES + blockIdx.x] = idx;
     }
 }
+// One launch for all slots (a copy and a fill of one word each: 64 launches for 32 slots, 2 - 4.6 us apiece)
+__global__ void __launch_bounds__(256) rb_slot_logits_kernel(const float* logits, long long ld, const int32_t* meta, float* dst, int32_t* d_state) {
+    const int j = blockIdx.y, slot = meta[4 * j + 1];
+    const u32x4* const from = reinterpret_cast<const u32x4*>(logits + j * ld);
+    u32x4* const to = reinterpret_cast<u32x4*>(dst + slot * ld);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const long long i = (long long)blockIdx.x * 1024 + k * 256 + threadIdx.x;
+        if (i < ld / 4) to[i] = from[i];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) d_state[4 * slot + 3] = 0;
+}
 __global__ void __launch_bounds__(64) rb_pick_finish_kernel(const float* __restrict__ pv, const int* __restrict__ pi, int pieces, int vocab, const int32_t* __restrict__ meta,
                                                             int32_t* __restrict__ state, int32_t* __restrict__ tokens_out, int tokens_stride) {
     const int r = blockIdx.x, pos = meta[KF_RB_META * r];
@@ -505,6 +517,13 @@ int kf_rb_pick(kf_ctx* c, const float* logits, int64_t ld, int vocab, int n, con
     hipLaunchKernelGGL(rb_pick_part_kernel, dim3(pieces, n), dim3(256), 0, c->stream, logits, (long long)ld, vocab, span, pv, pi);
     hipLaunchKernelGGL(rb_pick_finish_kernel, dim3(n), dim3(64), 0, c->stream, pv, pi, pieces, vocab, meta, d_state, d_tokens_out, tokens_stride);
     return launched("kf_rb_pick");
+}
+int kf_rb_slot_logits(kf_ctx* c, const float* logits, int64_t ld, int n, const int32_t* meta, float* dst, int32_t* d_state) {
+    CHKCTX(c);
+    if (!logits || !meta || !dst || !d_state || ld < 1 || ld % 4 || n < 1) return abi_fail(KF_INVALID_ARGS, "kf_rb_slot_logits: bad arguments");
+    if (!al16(logits) || !al16(dst)) return abi_fail(KF_BLAS_UNALIGN, "kf_rb_slot_logits: unaligned pointer");
+    hipLaunchKernelGGL(rb_slot_logits_kernel, dim3((unsigned)((ld / 4 + 1023) / 1024), n), dim3(256), 0, c->stream, logits, (long long)ld, meta, dst, d_state);
+    return launched("kf_rb_slot_logits");
 }
 int kf_rb_pack(kf_ctx* c, int type, const kf_bf16* src, int rows, int cols, void* dst, int64_t ld, int row0, int half, int tiled) {
     CHKCTX(c);

@@ -1084,9 +1084,8 @@ int XcdReplicas::SetForced(int seq, const int32_t* ids, int n) {
 }
 int XcdReplicas::SetState(int seq, int token, int pos) {
     if (seq < 0 || seq >= n_seq || pos < 0 || pos >= hFish->config.n_ctx || token < 0 || token >= hFish->config.vocab) return KF_INVALID_ARGS;
-    KF_TRY(kf_memset32(hFish->ctx, d_state + 4 * seq + 3, 0, 1)); /* the status word of the re-aimed sequence */
     if (slots) slots->pos[seq] = pos;
-    return kf_set_state(hFish->ctx, d_state + 4 * seq, token, pos);
+    return kf_set_slot_state(hFish->ctx, d_state + 4 * seq, token, pos); /* (and the status word of the re-aimed sequence) */
 }
 // CHAT_SAMPLER for Chat (greedy by default): one rng word per sequence, seeded per request
 int XcdReplicas::SetSampler(const CHAT_SAMPLER& sp) {

@@ -549,8 +549,14 @@ int SeqFish::Layers(RowWork& w, const KVCache& kv, const RowBatch& b) {
     }
     return KF_OK;
 }
+// words of a batch's tables: a few as a kernel's argument (a copy of three tables waited for all work in front of it, three times over), more by copy
+static int Upload(kf_ctx* ctx, void* dst, const std::vector<int32_t>& v) {
+    if (v.size() > 2 * KF_PUT_WORDS) return kf_h2d(ctx, dst, v.data(), v.size() * 4);
+    for (size_t i = 0; i < v.size(); i += KF_PUT_WORDS) KF_TRY(kf_put_words(ctx, static_cast<int32_t*>(dst) + i, v.data() + i, (int)std::min<size_t>(KF_PUT_WORDS, v.size() - i)));
+    return KF_OK;
+}
 int SeqFish::HeadRows(RowWork& w, const int32_t* h_rows, int n) {
-    if (h_rows) KF_TRY(kf_h2d(ctx, w.want->data, h_rows, (size_t)n * 4));
+    if (h_rows) KF_TRY(Upload(ctx, w.want->data, std::vector<int32_t>(h_rows, h_rows + n)));
     const int32_t* rows = h_rows ? I(w.want) : nullptr;
     KF_TRY(card.norm_kind == KF_RB_RMS ? seq_norm.Forw(F(w.x), n, nullptr, P(w.hl), nullptr, 0, 0, rows) : seq_norm.Rows(w, F(w.x), n, nullptr, nullptr, P(w.hl), rows, false));
     return seq_head.Forw(P(w.hl), seq_head.k, n, F(w.logits), seq_head.m, KF_RB_STORE_F32);
@@ -589,11 +595,26 @@ int SeqFish::Spans(SeqSlots& s, const SeqSpan* spans, int n_span, const int32_t*
         }
         if (!rows) break;
         KF_TRY(Ensure(pre, rows, n_span, 1, false));
-        KF_TRY(kf_h2d(ctx, pre.meta->data, meta.data(), meta.size() * 4));
-        KF_TRY(kf_h2d(ctx, pre.tok->data, tok.data(), tok.size() * 4));
-        KF_TRY(kf_h2d(ctx, pre.seqs->data, seqs.data(), seqs.size() * 4));
+        KF_TRY(Upload(ctx, pre.meta->data, meta));
+        KF_TRY(Upload(ctx, pre.tok->data, tok));
+        KF_TRY(Upload(ctx, pre.seqs->data, seqs));
         KF_TRY(kf_rb_embed(ctx, card.type, table->data, card.vocab, card.width, Width(card.width), I(pre.tok), rows, F(pre.x), P(pre.h)));
         KF_TRY(Layers(pre, s.kv, RowBatch{rows, (int)part.size(), max_n, 0}));
+        // the spans that end in this pass: their last rows' logits go into the slots', the greedy pick
+        std::vector<int32_t> end_rows, end_meta;
+        if (last)
+            for (int i : part)
+                if (done[i] == spans[i].n) {
+                    const int32_t m[4] = {spans[i].pos0 + spans[i].n - 1, spans[i].slot, 0, 0};
+                    end_rows.push_back(row0[i] + done[i] - from[i] - 1), end_meta.insert(end_meta.end(), m, m + 4);
+                }
+        auto pick = [&]() {
+            int32_t* d_meta = I(pre.want) + up(pre.head_rows, 4);
+            const int n = (int)end_rows.size();
+            KF_TRY(Upload(ctx, d_meta, end_meta));
+            KF_TRY(kf_rb_slot_logits(ctx, F(pre.logits), V, n, d_meta, F(s.dec.logits), s.d_state));
+            return kf_rb_pick(ctx, F(pre.logits), V, card.vocab, n, d_meta, s.d_state, s.d_tokens_out, card.n_ctx, s.pick_ws->data);
+        };
         // logits asked for, a block of rows at a time
         std::vector<int32_t> list, at;
         for (int i = 0; i < n_want; i++) {
@@ -605,30 +626,24 @@ int SeqFish::Spans(SeqSlots& s, const SeqSpan* spans, int n_span, const int32_t*
             const int n = (int)std::min<size_t>(block, list.size() - b);
             KF_TRY(Ensure(pre, rows, n_span, n, false));
             KF_TRY(HeadRows(pre, list.data() + b, n));
+            if (!end_rows.empty() && list == end_rows && n == (int)list.size()) { /* the rows asked for are the last ones: their logits are here already */
+                KF_TRY(pick());
+                end_rows.clear();
+            }
+            bool whole = V == card.vocab; /* the rows lie in `out` as they do here */
+            for (int j = 1; j < n; j++) whole = whole && at[b + j] == at[b] + j;
+            if (whole) {
+                KF_TRY(kf_d2h(ctx, out + (size_t)at[b] * card.vocab, pre.logits->data, (size_t)n * V * 4));
+                continue;
+            }
             std::vector<float> lg((size_t)n * V);
             KF_TRY(kf_d2h(ctx, lg.data(), pre.logits->data, lg.size() * 4));
             for (int j = 0; j < n; j++) std::memcpy(out + (size_t)at[b + j] * card.vocab, lg.data() + (size_t)j * V, (size_t)card.vocab * 4);
         }
-        if (last) { /* the spans that end in this pass: their last rows' logits into the slots', the greedy pick */
-            list.clear(), meta.clear();
-            std::vector<int> ends;
-            for (int i : part)
-                if (done[i] == spans[i].n) {
-                    const int32_t m[4] = {spans[i].pos0 + spans[i].n - 1, spans[i].slot, 0, 0};
-                    list.push_back(row0[i] + done[i] - from[i] - 1), meta.insert(meta.end(), m, m + 4), ends.push_back(i);
-                }
-            const int n = (int)list.size();
-            if (n) {
-                KF_TRY(Ensure(pre, rows, n_span, n, false));
-                KF_TRY(HeadRows(pre, list.data(), n));
-                int32_t* d_meta = I(pre.want) + up(pre.head_rows, 4);
-                KF_TRY(kf_h2d(ctx, d_meta, meta.data(), meta.size() * 4));
-                for (int j = 0; j < n; j++) {
-                    KF_TRY(kf_d2d(ctx, F(s.dec.logits) + (size_t)spans[ends[j]].slot * V, F(pre.logits) + (size_t)j * V, (size_t)V * 4));
-                    KF_TRY(kf_memset32(ctx, s.d_state + 4 * spans[ends[j]].slot + 3, 0, 1));
-                }
-                KF_TRY(kf_rb_pick(ctx, F(pre.logits), V, card.vocab, n, d_meta, s.d_state, s.d_tokens_out, card.n_ctx, s.pick_ws->data));
-            }
+        if (!end_rows.empty()) {
+            KF_TRY(Ensure(pre, rows, n_span, (int)end_rows.size(), false));
+            KF_TRY(HeadRows(pre, end_rows.data(), (int)end_rows.size()));
+            KF_TRY(pick());
         }
     }
     for (int i = 0; i < n_span; i++) s.pos[spans[i].slot] = spans[i].pos0 + spans[i].n;
