@@ -1,6 +1,6 @@
 // kf_rb_linear.hip -- row-batch products y[t][m] = W[m] . x[t] for few rows (decode batches) and in 32-bit, and the ABI entry that picks the form.
 //
-// Decode batches stream the weights: a workgroup owns 16 weight rows (GATED: 16 gate and the 16 up rows that follow them), its waves take runs of 32-deep k-steps -- a
+// Decode batches stream the weights: a workgroup owns one to four blocks of 16 weight rows (GATED: of 8 gate rows and their 8 up rows), its waves take runs of 32-deep k-steps -- a
 // step's 16 x 32 weights are one stored tile, a contiguous kilobyte -- and multiply them against up to 64 token columns by v_mfma_f32_16x16x32_bf16 (A = weight rows, B = token rows from
 // L2, where the activations of a decode batch stay: more than 8 rows by way of RbTokens), the next run's weights in flight.  The waves' partial tiles meet in LDS, one thread
 // per output finishes it.  The RMS norm in front of a product (NORM: few rows of the 32-bit residual sum) costs no pass: the product that formed the sum left its squares
@@ -13,19 +13,23 @@ namespace kf {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
+// k-steps of a run, loaded one run ahead: a wave of several weight blocks or of many token columns has its bytes in flight with two, and stays within 128 registers, two workgroups of eight waves to a CU
+// (us at four | two, two blocks: 32 rows of 32768 x 2048 27.7 | 25.4, of 6464 x 2048 8.8 | 8.2, three blocks of 12288 x 2048 13.2 | 11.9; with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
+constexpr int rb_run(int nt, int mg) { return nt >= 3 || mg >= 2 ? 2 : 4; }
+
 __device__ __forceinline__ f32x4 rb_mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-// the run of U k-steps from step s of the MG 16-row blocks at wr (this lane's piece of the first block's first tile; a tile per step)
+// the run of U k-steps from step s of MG blocks of 16 weight rows; wr[g]: this lane's piece of block g's first tile (a tile per step)
 template <int MG, int U>
-__device__ __forceinline__ void rb_load_w(u32x4 (&a)[U][MG], const uint16_t* __restrict__ wr, int k, int s, int s_end) {
+__device__ __forceinline__ void rb_load_w(u32x4 (&a)[U][MG], const uint16_t* const (&wr)[MG], int s, int s_end) {
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
         for (int g = 0; g < MG; g++) {
             a[u][g] = u32x4{0, 0, 0, 0};
-            if (s + u < s_end) a[u][g] = ld_nt(reinterpret_cast<const u32x4*>(wr + (size_t)g * 16 * k + 512 * (s + u))); /* wave-uniform */
+            if (s + u < s_end) a[u][g] = ld_nt(reinterpret_cast<const u32x4*>(wr[g] + 512 * (s + u))); /* wave-uniform */
         }
 }
 // token fragments of the same steps; xp[t]: this lane's token row + its k octet (NULLABLE: NULL is a zero column), steps past s_end read step s_end - 1 against zero weights
@@ -54,9 +58,9 @@ __device__ __forceinline__ void rb_multiply(const u32x4 (&a)[U][MG], const u32x4
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[g][t] = rb_mfma16(a[u][g], b[u][t], acc[g][t]);
 }
-// the waves' partial tiles -> outputs; list: the columns are pairs
-template <int NT, int MG, int NW>
-__device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4 (&acc)[MG][NT], float (&red)[NW][MG][16 * NT][17], const int32_t* list, int m0, int tid, int part = 0) {
+// the waves' partial tiles of the blocks from unit0 -> outputs; list: the columns are pairs; units: blocks past them repeat the last one.  GATED: a block is 8 gate rows and their 8 up rows
+template <int NT, int MG, int NW, bool GATED>
+__device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4 (&acc)[MG][NT], float (&red)[NW][MG][16 * NT][17], const int32_t* list, int unit0, int units, int tid, int part = 0) {
     const kf_rb_product& p = q.p;
     const int lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
 #pragma unroll
@@ -66,9 +70,11 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
 #pragma unroll
             for (int j = 0; j < 4; j++) red[wid][g][t * 16 + r16][4 * q4 + j] = acc[g][t][j];
     __syncthreads();
-    const int cols = list ? 16 * NT : p.n;
-    for (int i = tid; i < cols * 16; i += 64 * NW) {
-        const int row = i & 15, col = i >> 4;
+    constexpr int OUT = GATED ? 8 : 16, ROWS = MG * OUT; /* a block's outputs, the workgroup's */
+    const int cols = list ? 16 * NT : p.n, rows = (MG == 1 || units - unit0 >= MG ? MG : units - unit0) * OUT;
+    for (int i = tid; i < cols * ROWS; i += 64 * NW) {
+        const int row = i % ROWS, col = i / ROWS, g = row / OUT, rg = row % OUT, m = unit0 * OUT + row;
+        if (MG > 1 && row >= rows) continue;
         int yr = col;
         float scale = 1.f;
         if (list) {
@@ -78,27 +84,26 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
         }
         float d = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; w++) d += red[w][0][col][row];
-        if constexpr (MG == 2) {
+        for (int w = 0; w < NW; w++) d += red[w][g][col][rg];
+        if constexpr (GATED) {
             float u = 0.f;
 #pragma unroll
-            for (int w = 0; w < NW; w++) u += red[w][MG - 1][col][row];
-            reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + (m0 >> 1) + row] = f2bf(scale * (rb_activate(p.act, d) * u));
+            for (int w = 0; w < NW; w++) u += red[w][g][col][8 + rg];
+            reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + m] = f2bf(scale * (rb_activate(p.act, d) * u));
         } else if (p.epilogue == KF_RB_STORE) {
-            const int m = m0 + row;
             reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + m] = f2bf(m >= p.act_lo && m < p.act_hi ? rb_activate(p.act, d) : d);
         } else if (p.epilogue == KF_RB_STORE_F32) {
-            reinterpret_cast<float*>(p.y)[part * (size_t)p.part_stride + (size_t)yr * p.ldy + m0 + row] = d;
+            reinterpret_cast<float*>(p.y)[part * (size_t)p.part_stride + (size_t)yr * p.ldy + m] = d;
         } else {
-            const float z = fmaf(p.alpha, p.res[(size_t)yr * p.ldr + m0 + row], d);
-            reinterpret_cast<float*>(p.y)[(size_t)yr * p.ldy + m0 + row] = z;
+            const float z = fmaf(p.alpha, p.res[(size_t)yr * p.ldr + m], d);
+            reinterpret_cast<float*>(p.y)[(size_t)yr * p.ldy + m] = z;
             if (NT == 1 && p.ssq) { /* 16 lanes = the 16 columns of one row */
                 float ss = z * z;
                 ss += dpp_f<0xB1>(ss);
                 ss += dpp_f<0x4E>(ss);
                 ss += dpp_f<0x141>(ss);
                 ss += dpp_f<0x140>(ss);
-                if (row == 0) p.ssq[(size_t)(m0 / 16) * KF_RB_NORM_ROWS + yr] = ss;
+                if (rg == 0) p.ssq[(size_t)(unit0 + g) * KF_RB_NORM_ROWS + yr] = ss;
             }
         }
     }
@@ -144,17 +149,16 @@ struct RbTokens {
 
 // TURN: the token rows go through RbTokens (rows in order, no experts); else every lane reads its fragments itself.  PARTS: blockIdx.y is a part of k (a form of its own: 1 % of a decode step of products
 // that have none)
-template <int NT, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
+template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
-    constexpr int MG = GATED ? 2 : 1, U = NT >= 4 ? 2 : 4;
+    constexpr int U = rb_run(NT, MG);
     static_assert(!(NORM && TURN), "normed fragments are made from the residual sum");
     using Tokens = RbTokens<NT, U>;
-    constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * Tokens::LDS * 2 : 0;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[RED > STAGE ? RED : STAGE];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
-    const int m0 = blockIdx.x * (16 * MG), part = PARTS ? (int)blockIdx.y : 0, steps = p.k / 32, nstep = PARTS ? steps * (part + 1) / p.parts : steps; /* this part's steps end here */
+    const int unit0 = blockIdx.x * MG, units = p.m / 16, part = PARTS ? (int)blockIdx.y : 0, steps = p.k / 32, nstep = PARTS ? steps * (part + 1) / p.parts : steps; /* this part's steps end here */
     const uint16_t* W = reinterpret_cast<const uint16_t*>(p.w);
     const uint16_t* X = reinterpret_cast<const uint16_t*>(p.x);
     const int32_t* list = nullptr;
@@ -164,10 +168,16 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
         W += (size_t)ex * q.e.w_stride;
         list = q.e.list + (size_t)blockIdx.y * q.e.tile;
     }
-    const uint16_t* wr = W + (size_t)m0 * p.k + 8 * lane;
+    const uint16_t* wr[MG];
+#pragma unroll
+    for (int g = 0; g < MG; g++) {
+        const int unit = MG == 1 || unit0 + g < units ? unit0 + g : units - 1;
+        if (GATED) wr[g] = W + (size_t)(2 * (unit >> 1) + (r16 >> 3)) * 16 * p.k + 8 * (16 * q4 + 8 * (unit & 1) + (r16 & 7)); /* half of the gate's tile, half of the up rows': whole lines of both */
+        else wr[g] = W + (size_t)unit * 16 * p.k + 8 * lane;
+    }
     u32x4 a[U][MG], b[U][NT];
     int s = (PARTS ? steps * part / p.parts : 0) + wid * U;
-    rb_load_w<MG, U>(a, wr, p.k, s, nstep);
+    rb_load_w<MG, U>(a, wr, s, nstep);
     const uint16_t* xp[NT];
     Tokens tok;
     const float* zp = nullptr;   /* NORM: this lane's row of the residual sum, and 1 / its root mean square */
@@ -219,7 +229,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
                 const int k0 = 32 * (s + u < nstep ? s + u : nstep - 1);
                 z0[u] = rb_ld4(zp + k0), z1[u] = rb_ld4(zp + k0 + 4), g[u] = *reinterpret_cast<const u32x4*>(gp + k0);
             }
-            rb_load_w<MG, U>(an, wr, p.k, s + NW * U, nstep);
+            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const f32x4 o0 = f32x4{z0[u].x * rs * bf_lo(g[u].x), z0[u].y * rs * bf_hi(g[u].x), z0[u].z * rs * bf_lo(g[u].y), z0[u].w * rs * bf_hi(g[u].y)};
@@ -234,10 +244,10 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
         } else if constexpr (TURN) {
             tok.turn(b);
             if (s + NW * U < nstep) tok.load(s + NW * U, nstep); /* wave-uniform */
-            rb_load_w<MG, U>(an, wr, p.k, s + NW * U, nstep);
+            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
         } else {
             rb_load_x<NT, U, false>(b, xp, s, nstep);
-            rb_load_w<MG, U>(an, wr, p.k, s + NW * U, nstep);
+            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
         }
         rb_multiply<NT, MG, U>(a, b, acc);
 #pragma unroll
@@ -246,7 +256,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
             for (int g = 0; g < MG; g++) a[u][g] = an[u][g];
     }
     if constexpr (TURN) __syncthreads(); /* the token rows make way */
-    rb_stream_finish<NT, MG, NW>(q, acc, red, list, m0, tid, part);
+    rb_stream_finish<NT, MG, NW, GATED>(q, acc, red, list, unit0, units, tid, part);
 }
 
 // RESIDUAL with the rows' experts summed: (chosen expert, k-step) pairs as one list, cut evenly over the waves
@@ -281,9 +291,9 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
     while (at < end) { /* an expert's part of this wave's range (wave-uniform) */
         const int i = at / nstep, s0 = at - i * nstep, s1 = s0 + (end - at) < nstep ? s0 + (end - at) : nstep;
         const int ex = s_ex[i];
-        const uint16_t* wr = reinterpret_cast<const uint16_t*>(p.w) + (size_t)ex * q.e.w_stride + (size_t)m0 * p.k + 8 * lane;
+        const uint16_t* const wr[1] = {reinterpret_cast<const uint16_t*>(p.w) + (size_t)ex * q.e.w_stride + (size_t)m0 * p.k + 8 * lane};
         u32x4 a[U][1], b[U][NT];
-        rb_load_w<1, U>(a, wr, p.k, s0, s1);
+        rb_load_w<1, U>(a, wr, s0, s1);
         const uint16_t* xp[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -296,53 +306,80 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
         for (int s = s0; s < s1; s += U) {
             u32x4 an[U][1];
             rb_load_x<NT, U, true>(b, xp, s, s1);
-            rb_load_w<1, U>(an, wr, p.k, s + U, s1);
+            rb_load_w<1, U>(an, wr, s + U, s1);
             rb_multiply<NT, 1, U>(a, b, acc);
 #pragma unroll
             for (int u = 0; u < U; u++) a[u][0] = an[u][0];
         }
         at += s1 - s0;
     }
-    rb_stream_finish<NT, 1, NW>(q, acc, red, nullptr, m0, tid);
+    rb_stream_finish<NT, 1, NW, false>(q, acc, red, nullptr, blockIdx.x, p.m / 16, tid);
 }
-template <int NT, int NW>
-static void stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
+template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
+static int stream_form(hipStream_t st, const RbProduct& q, dim3 grid) {
+    constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * RbTokens<NT, rb_run(NT, MG)>::LDS * 2 : 0, SMEM = RED > STAGE ? RED : STAGE;
+    static_assert(SMEM <= 160 * 1024, "LDS");
+    const auto kernel = rb_stream_kernel<NT, MG, GATED, NW, NORM, TURN, PARTS>;
+    if constexpr (SMEM > 64 * 1024) {
+        static bool done = false;
+        if (!done && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
+        done = true;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), SMEM, st, q);
+    return KF_OK;
+}
+template <int NT, int MG, int NW>
+static int stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     const kf_rb_product& p = q.p;
     // whole lines for more than 8 rows in order: below, a fragment's 16 half lines are few distinct ones and the way round costs more than it saves (one token of a 2048-wide model: 1.79 -> 1.87 ms
-    // over four steps; 6 rows 2.04 -> 2.08; 14 rows 2.42 -> 2.35; 32 rows 4.62 -> 4.23); experts' tiles are mostly padding, which repeats row 0 (32 rows of 64 experts: 10.15 -> 10.36)
-    const bool turn = p.mode == KF_RB_ALL && p.n > 8 && p.ldx <= (1 << 24), gated = p.epilogue == KF_RB_GATED;
-    if (p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
-    else if (gated && turn) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
-    else if (gated) hipLaunchKernelGGL((rb_stream_kernel<NT, true, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
-    else if (p.parts > 1 && turn) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, true, true>), grid, dim3(64 * NW), 0, st, q);
-    else if (p.parts > 1) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, false, true>), grid, dim3(64 * NW), 0, st, q);
-    else if (turn) hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, true>), grid, dim3(64 * NW), 0, st, q);
-    else hipLaunchKernelGGL((rb_stream_kernel<NT, false, NW, false, false>), grid, dim3(64 * NW), 0, st, q);
+    // over four steps; 6 rows 2.04 -> 2.08; 14 rows 2.42 -> 2.35; 32 rows 4.62 -> 4.23)
+    const bool turn = p.n > 8 && p.ldx <= (1 << 24), gated = p.epilogue == KF_RB_GATED;
+    if constexpr (NT == 1) {
+        if (p.norm_z) return gated ? stream_form<1, MG, true, NW, true, false>(st, q, grid) : stream_form<1, MG, false, NW, true, false>(st, q, grid);
+    }
+    if constexpr (MG == 1) {
+        if (p.parts > 1) return turn ? stream_form<NT, 1, false, NW, false, true, true>(st, q, grid) : stream_form<NT, 1, false, NW, false, false, true>(st, q, grid);
+    }
+    if (gated) return turn ? stream_form<NT, MG, true, NW, false, true>(st, q, grid) : stream_form<NT, MG, true, NW, false, false>(st, q, grid);
+    return turn ? stream_form<NT, MG, false, NW, false, true>(st, q, grid) : stream_form<NT, MG, false, NW, false, false>(st, q, grid);
 }
-template <int NW>
-static void norm_stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
-    if (q.p.epilogue == KF_RB_GATED) hipLaunchKernelGGL((rb_stream_kernel<1, true, 4, true, false>), grid, dim3(256), 0, st, q);
-    else hipLaunchKernelGGL((rb_stream_kernel<1, false, NW, true, false>), grid, dim3(64 * NW), 0, st, q);
+// experts: one gate block and its up rows a workgroup; the tiles are mostly padding, which repeats row 0, and the way round by LDS does not pay (32 rows of 64 experts: 10.15 -> 10.36 ms)
+template <int NT, int NW>
+static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
+    if (q.p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
+    else if (q.p.epilogue == KF_RB_GATED) return stream_form<NT, 2, true, NW, false, false>(st, q, grid);
+    else return stream_form<NT, 1, false, NW, false, false>(st, q, grid);
+    return KF_OK;
+}
+// How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
+// one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
+// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.2 10.9 11.8 14.2; plain 10.1 11.4 14.4 19.5 -> 10.0 11.0 11.9 15.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.3 8.2 10.7.
+// More than that is bound by HBM while the rows are few: pairs of blocks, many workgroups that follow each other; else the least work for the busiest CU, by workgroups of four waves, several to a
+// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 22.3 22.2 25.5 29.3 (134 MB: 5.3 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 32.4 32.1 34.6 42.4.
+static int stream_blocks(int units, int n) {
+    if (units <= 1024) return (units + 255) / 256;
+    int best = 2;
+    long least = 0;
+    for (int mg = 2; n > 24 && mg <= 4; mg++) {
+        const long cost = ((units + mg - 1) / mg + 255) / 256 * (16 * mg + n);
+        if (mg == 2 || cost < least) best = mg, least = cost;
+    }
+    return best;
 }
 int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const kf_rb_product& p = q.p;
-    const bool tiles = p.mode == KF_RB_UP || p.mode == KF_RB_DOWN;
-    const int cols = tiles ? q.e.tile : p.n, nt = (cols + 15) / 16;
+    const bool tiles = p.mode == KF_RB_UP || p.mode == KF_RB_DOWN, all = p.mode == KF_RB_ALL;
+    const int cols = tiles ? q.e.tile : p.n, nt = (cols + 15) / 16, units = p.m / 16;
     if (nt > 4 || (tiles && q.e.tile % 16)) return 1;
     if (p.mode == KF_RB_SUM && ((long)p.n * q.e.top > KF_RB_SUM_PAIRS || q.e.tile < p.n)) return 1;
-    dim3 grid(p.m / (p.epilogue == KF_RB_GATED ? 32 : 16), tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
-    const bool wide = (long)grid.x * grid.y < 768 && p.k >= 512; /* few workgroups: more waves each, more loads in flight per CU */
-    if (p.norm_z) {
-        wide ? norm_stream_go<8>(st, q, grid) : norm_stream_go<4>(st, q, grid);
-        return KF_OK;
-    }
-    switch (nt) {
-        case 1: wide ? stream_go<1, 8>(st, q, grid) : stream_go<1, 4>(st, q, grid); break;
-        case 2: wide ? stream_go<2, 8>(st, q, grid) : stream_go<2, 4>(st, q, grid); break;
-        case 3: stream_go<3, 4>(st, q, grid); break;
-        default: stream_go<4, 4>(st, q, grid); break;
-    }
-    return KF_OK;
+    const int mg = !all ? (p.epilogue == KF_RB_GATED ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n);
+    const dim3 grid((units + mg - 1) / mg, tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
+    const bool wide = p.k >= 512 && (all ? units <= 1024 || p.n <= 24 : (long)grid.x * grid.y < 768); /* few workgroups: more waves each, more loads in flight per CU */
+#define RB_STREAM_MG(nt, nw) (mg == 1 ? stream_go<nt, 1, nw>(st, q, grid) : mg == 2 ? stream_go<nt, 2, nw>(st, q, grid) : mg == 3 ? stream_go<nt, 3, nw>(st, q, grid) : stream_go<nt, 4, nw>(st, q, grid))
+#define RB_STREAM(nt) (!all ? (wide && nt <= 2 ? expert_go<nt, 8>(st, q, grid) : expert_go<nt, 4>(st, q, grid)) : wide ? RB_STREAM_MG(nt, 8) : RB_STREAM_MG(nt, 4))
+    return nt == 1 ? RB_STREAM(1) : nt == 2 ? RB_STREAM(2) : nt == 3 ? RB_STREAM(3) : RB_STREAM(4);
+#undef RB_STREAM
+#undef RB_STREAM_MG
 }
 
 }  // namespace kf

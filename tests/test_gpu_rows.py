@@ -110,6 +110,31 @@ def test_product_epilogues(ctx, kind, n, m, k):
         assert np.abs(f64(y) - fn(gate) * upw).max() < tol * 8
 
 
+@pytest.mark.parametrize("m", [4096, 4160, 8320, 12352, 16448, 32768])  # one, two, three (and a rest), four blocks of 16 weight rows a workgroup; more than one round: two, three (a rest), four by the rows
+@pytest.mark.parametrize("n,k", [(1, 512), (4, 64), (9, 576), (24, 512), (25, 64), (33, 512), (64, 576)])
+def test_products_of_several_blocks(ctx, m, n, k):
+    """Against float64.  A sum of k products of normal numbers over sqrt(k) is about 1 and at most 6 here; in float32 its rounding is at most k 2^-24 of the sum of magnitudes (< 1.2 sqrt(k)): below 1e-4 where k <= 576 were they all of
+    one sign, a tenth of that as it is.  16-bit results add half of 2^-8."""
+    g = torch.Generator().manual_seed(m + n)
+    w, x, res = dev(torch.randn(m, k, generator=g) / k ** 0.5, torch.bfloat16), dev(torch.randn(n, k + 8, generator=g), torch.bfloat16), dev(torch.randn(n, m, generator=g))
+    ref, ws, ssq = f64(x)[:, :k] @ f64(w).T, stored(w), torch.full((m // 16, 4), 7.0, device="cuda")
+    for epi, y in ((L.RB_STORE, torch.zeros(n, m, dtype=torch.bfloat16, device="cuda")), (L.RB_STORE_F32, torch.zeros(n, m, device="cuda")), (L.RB_RESIDUAL, torch.zeros(n, m, device="cuda"))):
+        sums = ssq.data_ptr() if epi == L.RB_RESIDUAL and n <= 4 else None
+        p = L.RbProduct(ws.data_ptr(), x.data_ptr(), y.data_ptr(), res.data_ptr(), k + 8, m, m, L.BF16, m, k, n, epi, 0, L.RB_ALL, -0.75, None, sums)
+        L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+        want = ref + (-0.75 * f64(res) if epi == L.RB_RESIDUAL else 0)
+        assert (np.abs(f64(y) - want) <= 1e-5 + (np.abs(want) * 2.0 ** -8 if epi == L.RB_STORE else 0)).all(), epi
+        if sums:
+            assert np.allclose(f64(ssq)[:, :n], (f64(y) ** 2).reshape(n, m // 16, 16).sum(2).T, rtol=1e-5) and (ssq[:, n:] == 7.0).all()
+    il = f64(w).reshape(m // 32, 2, 16, k)
+    gate, upw = f64(x)[:, :k] @ il[:, 0].reshape(-1, k).T, f64(x)[:, :k] @ il[:, 1].reshape(-1, k).T
+    y = torch.full((n, m // 2 + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    p = L.RbProduct(ws.data_ptr(), x.data_ptr(), y.data_ptr(), None, k + 8, m // 2 + 8, 0, L.BF16, m, k, n, L.RB_GATED, L.RB_SILU, L.RB_ALL, 0.0, None)
+    L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+    want = P.silu(gate) * upw
+    assert (np.abs(f64(y)[:, :m // 2] - want) <= 2e-4 + np.abs(want) * 2.0 ** -8).all() and (y[:, m // 2:] == 7.0).all()
+
+
 @pytest.mark.parametrize("n,m,k,dim", [(1, 64, 64, 50), (3, 192, 320, 300), (4, 448, 1024, 1024), (2, 256, 4096, 4090)])
 def test_norm_in_front_of_a_product(ctx, n, m, k, dim):
     assert ctx.hip.kf_rb_linear_norms(L.BF16, n, k) and not ctx.hip.kf_rb_linear_norms(L.F32, n, k) and not ctx.hip.kf_rb_linear_norms(L.BF16, 5, k)
@@ -136,6 +161,11 @@ def test_norm_in_front_of_a_product(ctx, n, m, k, dim):
             full = P.silu(f64(h) @ il[:, 0].reshape(-1, k).T) * (f64(h) @ il[:, 1].reshape(-1, k).T)
         got = f64(y).reshape(-1)[:n * m].reshape(n, m)[:, :full.shape[1]]
         assert np.abs(got - full).max() < (2e-5 if epi == L.RB_STORE_F32 else 0.04)
+
+
+@pytest.mark.parametrize("n,m,k,dim", [(1, 8320, 512, 500), (4, 16448, 64, 64)])
+def test_norm_in_front_of_several_blocks(ctx, n, m, k, dim):
+    test_norm_in_front_of_a_product(ctx, n, m, k, dim)
 
 
 def test_product_many_tiles(ctx):
