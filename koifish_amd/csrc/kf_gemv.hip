@@ -41,6 +41,32 @@ struct Batch {
     uint16_t st2[PAIRED ? G : 1], ze2[PAIRED ? G : 1];
 };
 
+// a row's dot into its place; o: the bf16 result (true), if there is one
+__device__ __forceinline__ bool gemv_put(const GemvArgs& a, uint16_t* y, int r, float v, uint16_t& o) {
+    if (a.tp) { /* tensor-parallel push: one 8-byte {value | tag} granule into this rank's slot of every rank's receive area (kf_tp.hip) */
+        const TpPushDev& t = *a.tp;
+        const unsigned long long gr = ((unsigned long long)(*t.step * t.per_step + t.index + 1u) << 32) | __float_as_uint(v);
+        for (int p = 0; p < t.world; p++) __hip_atomic_store(t.peer[p] + r, gr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return false;
+    }
+    if (a.yf) { /* un-rounded fp32 row dots: tensor-parallel partial sums (column-split o_proj / down_proj) */
+        a.yf[r] = v;
+        return false;
+    }
+    if (a.alpha != 1.0f) v = a.alpha * v;
+    if (a.beta != 0.0f) v = v + a.beta * bf2f(y[r]);
+    if (a.bias) v = v + bf2f(a.bias[r]);
+    o = f2bf(v);
+    if (a.residual) o = f2bf(bf2f(a.residual[r]) + bf2f(o)); /* CU_add3: bf16(x + bf16(W.x)) */
+    y[r] = o;
+    return true;
+}
+// SwiGLU of the two bf16-rounded projections (CU_swiglu_v0, Activation.cu:85-93)
+__device__ __forceinline__ uint16_t gemv_swiglu(float gate, float up) {
+    const float gt = round_bf16(gate);
+    return f2bf((gt * round_bf16(up)) / (1.0f + kf_expf(-gt)));
+}
+
 // LDS: x as u32x4 chunks [XCH][nBlk] (K*2 bytes) | 256 B reduction scratch.
 // Each wave keeps two batches of G blocks in flight: the first batch is issued BEFORE the x prologue so that the
 // weight stream's HBM latency overlaps the (dependent) activation load + norm.
@@ -364,27 +390,11 @@ __global__ void __launch_bounds__(256) gemv_kernel(const GemvArgs a) {
                     uint16_t* y = jy + (size_t)pos * jystride;
                     float v = sum[g];
                     if (PAIRED) {
-                        // SwiGLU of the two bf16-rounded projections (CU_swiglu_v0, Activation.cu:85-93)
-                        const float gt = round_bf16(v), up = round_bf16(sum2[g]);
-                        y[r] = f2bf((gt * up) / (1.0f + kf_expf(-gt)));
+                        y[r] = gemv_swiglu(v, sum2[g]);
                         continue;
                     }
-                    if (a.tp) { /* tensor-parallel push: one 8-byte {value | tag} granule into this rank's slot of every rank's receive area (kf_tp.hip) */
-                        const TpPushDev& t = *a.tp;
-                        const unsigned long long gr = ((unsigned long long)(*t.step * t.per_step + t.index + 1u) << 32) | __float_as_uint(v);
-                        for (int p = 0; p < t.world; p++) __hip_atomic_store(t.peer[p] + r, gr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                        continue;
-                    }
-                    if (a.yf) { /* un-rounded fp32 row dots: tensor-parallel partial sums (column-split o_proj / down_proj) */
-                        a.yf[r] = v;
-                        continue;
-                    }
-                    if (a.alpha != 1.0f) v = a.alpha * v;
-                    if (a.beta != 0.0f) v = v + a.beta * bf2f(y[r]);
-                    if (a.bias) v = v + bf2f(a.bias[r]);
-                    uint16_t o = f2bf(v);
-                    if (a.residual) o = f2bf(bf2f(a.residual[r]) + bf2f(o)); /* CU_add3: bf16(x + bf16(W.x)) */
-                    y[r] = o;
+                    uint16_t o = 0;
+                    if (!gemv_put(a, y, r, v, o)) continue;
                     if (MODE == GEMV_ARGMAX) {
                         const float fv = bf2f(o);
                         if (fv > best_v || (fv == best_v && r < best_i)) best_v = fv, best_i = r;
@@ -463,6 +473,142 @@ __global__ void __launch_bounds__(256) gemv_kernel(const GemvArgs a) {
         }
     }
 }
+
+#if KF_GEMV_CANON
+// Large 4-bit matrices in the canonical order.  Bound by the vector pipe, not by memory (131 MB take 26 us at the rate of a copy): the lookup and the two chains are 5.2 instructions per weight, four in seven of
+// them of half rate (v_perm; fma, and, or, add, shifts right are of full rate), so what counts is that every SIMD always has a wave that can issue and that nothing else is issued.  One workgroup of 16 waves to a CU,
+// which takes an even share of the row slots: x is normed, widened and staged once per CU instead of once per four waves and eight to sixteen slots; waves take slots in turn, four blocks in flight through the
+// slots' ends (six, or 24 waves to a CU: no difference); a block column's 32 activations lie side by side in LDS (nine 16-byte pieces apart: 16 lanes' equal pieces in different banks), so one address serves a block's
+// eight reads; the quad exchanges its table through the LDS crossbar; no masks (rows and columns divide evenly, or the kernel above takes the matrix).  Same chains, same tree, same bits.  us, the kernel above | this
+// one: gate and up 25600 x 5120 63.2 | 50.2, 5120 x 25600 38.1 | 28.9, 5120 x 8192 14.6 | 11.2, 8192 + 1024 + 1024 x 5120 18.0 | 15.9.
+constexpr int GQ_WAVES = 16, GQ_RING = 4, GQ_XCH = 4; /* GQ_XCH x 1024 threads x 8 elements: the longest x */
+template <bool PAIRED, bool ONEJOB>
+__global__ void __launch_bounds__(64 * GQ_WAVES) gemv_q4_kernel(const GemvArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    f32x4* const xs = reinterpret_cast<f32x4*>(smem_raw);
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), nBlk = a.nBlk, iters = a.iters, lg = a.lpr_log2, LPR = 1 << lg, RPS = 64 >> lg;
+    double* const red = reinterpret_cast<double*>(smem_raw + (size_t)nBlk * 144);
+    const int sub = lane >> lg, ll = lane & (LPR - 1);
+    const long lo = (long)a.total_slots * blockIdx.x / gridDim.x, hi = (long)a.total_slots * (blockIdx.x + 1) / gridDim.x;
+    const int s0 = (int)lo + wid, n_slot = s0 < (int)hi ? ((int)hi - s0 + GQ_WAVES - 1) / GQ_WAVES : 0, n_step = n_slot * iters * (PAIRED ? 2 : 1);
+    // ---- x and the norm weight first: their staging overlaps the first blocks' way
+    const int nch = a.K >> 3;
+    const bool has_norm = a.norm_w != nullptr;
+    const uint16_t* const nw = has_norm ? a.norm_w : a.x;
+    u32x4 xr[GQ_XCH], xn[GQ_XCH];
+#pragma unroll
+    for (int i = 0; i < GQ_XCH; i++) {
+        const int c = tid + 64 * GQ_WAVES * i, at = c < nch ? c : tid & 7; /* nch >= 16 */
+        xr[i] = *reinterpret_cast<const u32x4*>(a.x + (size_t)at * 8), xn[i] = *reinterpret_cast<const u32x4*>(nw + (size_t)at * 8);
+    }
+    // ---- the weight stream: (slot, matrix, iteration) steps; the slot's job by constant indices into the kernel arguments
+    struct Block {
+        u32x4 w;
+        uint16_t st, ze;
+    };
+    struct Place {
+        int slot, mat, it;
+    };
+    auto job_of = [&](int slot) { return ONEJOB || PAIRED ? 0 : (int)(a.njobs > 1 && slot >= a.job[1].slot0) + (int)(a.njobs > 2 && slot >= a.job[2].slot0); };
+#define JF(j, f) (ONEJOB ? a.job[0].f : PAIRED ? ((j) ? a.job[1].f : a.job[0].f) : ((j) == 0 ? a.job[0].f : ((j) == 1 ? a.job[1].f : a.job[2].f)))
+    const uint32_t lane_w = (uint32_t)(sub * nBlk + ll) * 16u, lane_g = (uint32_t)((sub * nBlk + ll) >> 2) * 2u; /* a group: four blocks of a row, an aligned quad of lanes */
+    auto next = [&](Place& p) {
+        if (++p.it == iters) {
+            p.it = 0;
+            if (PAIRED) p.mat ^= 1;
+            if (!PAIRED || p.mat == 0) p.slot += GQ_WAVES;
+        }
+    };
+    auto load = [&](const Place& p, Block& b) {
+        const int j = PAIRED ? p.mat : job_of(p.slot);
+        const size_t block = (size_t)(p.slot - (PAIRED ? 0 : JF(j, slot0))) * (size_t)(RPS * nBlk) + (size_t)(p.it << lg);
+        b.w = ld_nt(reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(JF(j, w)) + block * 16 + lane_w));
+        b.st = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const unsigned char*>(JF(j, step)) + block / 2 + lane_g);
+        b.ze = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const unsigned char*>(JF(j, zero)) + block / 2 + lane_g);
+    };
+    Block ring[GQ_RING];
+    Place at{s0, 0, 0}, here = at; /* the step being loaded, being multiplied */
+    int ahead = 0;
+    auto fetch = [&](Block& b) { /* unconditional: past the last step it reads that step again */
+        load(at, b);
+        if (ahead + 1 < n_step) next(at);
+        ahead++;
+    };
+    if (n_step > 0) {
+#pragma unroll
+        for (int d = 0; d < GQ_RING; d++) fetch(ring[d]);
+    }
+    const int pos = a.d_pos ? *a.d_pos : a.pos;
+    {
+        float mul = 1.0f;
+        if (has_norm) { /* RMSNorm (rms_norm_kernel, layernorm.cuh:800-847): sum of squares in fp64 */
+            double ss = 0.0;
+#pragma unroll
+            for (int i = 0; i < GQ_XCH; i++) {
+                if (tid + 64 * GQ_WAVES * i >= nch) continue;
+                const uint32_t w[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const double l = (double)bf_lo(w[k]), h = (double)bf_hi(w[k]);
+                    ss = fma(l, l, ss), ss = fma(h, h, ss);
+                }
+            }
+            ss = wave_sum_f64_fast(ss);
+            if (lane == 0) red[wid] = ss;
+            __syncthreads();
+            double tot = 0.0;
+#pragma unroll
+            for (int w = 0; w < GQ_WAVES; w++) tot += red[w];
+            mul = 1.0f / sqrtf(fmaf((float)tot, a.inv_dim, a.eps));
+        }
+#pragma unroll
+        for (int i = 0; i < GQ_XCH; i++) {
+            const int c = tid + 64 * GQ_WAVES * i;
+            if (c >= nch) continue;
+            uint32_t w[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
+            const uint32_t g[4] = {xn[i].x, xn[i].y, xn[i].z, xn[i].w};
+            if (has_norm) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) w[k] = pack_bf16x2((bf_lo(w[k]) * mul) * bf_lo(g[k]), (bf_hi(w[k]) * mul) * bf_hi(g[k]));
+            }
+            f32x4* const o = xs + (c >> 2) * 9 + (c & 3) * 2; /* block column c / 4 */
+            o[0] = f32x4{bf_lo(w[0]), bf_hi(w[0]), bf_lo(w[1]), bf_hi(w[1])}, o[1] = f32x4{bf_lo(w[2]), bf_hi(w[2]), bf_lo(w[3]), bf_hi(w[3])};
+        }
+    }
+    __syncthreads();
+    // ---- multiply
+    const f32x4* const xs_lane = xs + ll * 9;
+    f32x2_t acc = f32x2_t{0.f, 0.f};
+    float gate = 0.f;
+    auto compute = [&](const Block& b) {
+        const float st = bf2f(b.st);
+        const int j = PAIRED ? here.mat : job_of(here.slot);
+        acc = BlockDotF<FMT_Q4P>::run_side(b.w, xs_lane + (here.it << lg) * 9, st, bf2f(b.ze), -((float)JF(j, qBias) * st), acc);
+        if (here.it == iters - 1) {
+            const float sum = group_sum(acc_join(acc), lg);
+            acc = f32x2_t{0.f, 0.f};
+            if (PAIRED && here.mat == 0) {
+                gate = sum;
+            } else if (ll == 0) {
+                const int r = (here.slot - (PAIRED ? 0 : JF(j, slot0))) * RPS + sub;
+                uint16_t* const y = (PAIRED ? a.job[0].y : JF(j, y)) + (size_t)pos * (PAIRED ? a.job[0].y_pos_stride : JF(j, y_pos_stride));
+                uint16_t o;
+                if (PAIRED) y[r] = gemv_swiglu(gate, sum);
+                else gemv_put(a, y, r, sum, o);
+            }
+        }
+        next(here);
+    };
+    for (int k = 0; k < n_step; k += GQ_RING) {
+#pragma unroll
+        for (int d = 0; d < GQ_RING; d++) {
+            if (k + d < n_step) compute(ring[d]);
+            fetch(ring[d]);
+        }
+    }
+#undef JF
+}
+#endif
 
 #if !KF_GEMV_CANON
 // Final pick over the per-workgroup partial maxima, then the decode-state update for graph replay.
@@ -615,6 +761,16 @@ static void launch_g(const GemvArgs& a, int G, dim3 grid, size_t smem, hipStream
             launch_j<FMT, MODE, SPARSE, false>(a, G, grid, smem, st);
     }
 }
+#if KF_GEMV_CANON
+template <bool PAIRED, bool ONEJOB>
+static int launch_q4(const GemvArgs& a, hipStream_t st) {
+    static bool done = false;
+    if (!done && hipFuncSetAttribute((const void*)gemv_q4_kernel<PAIRED, ONEJOB>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return KF_HIP_CHECK;
+    done = true;
+    hipLaunchKernelGGL((gemv_q4_kernel<PAIRED, ONEJOB>), dim3(256), dim3(64 * GQ_WAVES), (size_t)a.nBlk * 144 + 256, st, a);
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+#endif
 template <int FMT>
 static void launch_m(const GemvArgs& a, int mode, int G, dim3 grid, size_t smem, hipStream_t st) {
     if (a.row_map) { /* the sparse forward: kf_linear_masked (plain) and kf_norm_gateup_swiglu_masked (paired) */
@@ -691,6 +847,21 @@ int gemv_launch_dot2(hipStream_t st, GemvLaunch& L) {
     // memory waits of one wave are covered by the dequant arithmetic of the others (measured: 25600x5120 q4 41 -> 33 us; the Qwen3-32B
     // q/k/v and o_proj launches, 22-28 MB each, 21.8 -> 19.1 and 16.1 -> 13.2 us; the 0.6B launches stay below the threshold)
     const long blocks_all = raw_slots * (long)nBlk * (64 / (1 << lpr_log2));
+#if KF_GEMV_CANON
+    // a workgroup per CU from 2^20 blocks: below, its one prologue of all 16 waves costs more than it saves.  us, the kernel of small workgroups | one per CU: 4096 x 4096 6.4 | 8.3, 6144 x 4096 7.3 | 8.9, gate and up
+    // 9728 x 2560 (2^20.6) 14.7 | 14.6, 12288 x 4096 23.7 | 22.4, 17408 x 5120 42.7 | 33.2; 7168 x 5120 12.0 | 11.3, 4096 x 12288 16.5 | 14.1
+    if (fmt == FMT_Q4 && g_knobs.q4_perm != 0 && g_knobs.gemv_waves == 0 && L.target_waves <= 0 && L.mode != GEMV_ARGMAX && !a.row_map && blocks_all * (L.mode == GEMV_PAIRED ? 2 : 1) >= (1L << 20) && raw_slots >= 2048 && a.lGroup == 128 && K % 128 == 0 &&
+        lpr_log2 >= 2 && nBlk % LPR == 0 && K <= 8 * 64 * GQ_WAVES * GQ_XCH) {
+        bool even = true;
+        for (int j = 0; j < L.n; j++) even = even && L.w[j]->ne0 % RPS == 0;
+        if (even) {
+            int slots = 0;
+            for (int j = 0; j < a.njobs; j++) a.job[j].slot0 = slots, slots += (int)rows_slots[j];
+            a.total_slots = slots, L.blocks = 256;
+            return L.mode == GEMV_PAIRED ? launch_q4<true, false>(a, st) : a.njobs == 1 ? launch_q4<false, true>(a, st) : launch_q4<false, false>(a, st);
+        }
+    }
+#endif
     long target_waves = L.target_waves > 0 ? L.target_waves : (blocks_all >= (1L << 19) ? 16384 : 4096);
     // the largest launches (>= 4 M blocks: the 25600-row FFN matrices of Qwen3-32B): two slots per wave through the buffer-load form, half the workgroups to
     // start and half the x staging (25600 x 5120: 27.6 -> 26.4 us, A/B in one run; smaller launches lose more from the coarser tail than they gain)

@@ -370,7 +370,14 @@ template <>
 struct BlockDotF<FMT_Q4P> {
     static constexpr int EPB = 32, XCH = 8;
     static constexpr bool HAS_GAMA = true;
-    __device__ static __forceinline__ f32x2_t run(u32x4 w, const f32x4* xs, int col, int nBlk, float step, float zero, float nb, f32x2_t acc) {
+    __device__ static __forceinline__ f32x2_t run(u32x4 w, const f32x4* xs, int col, int nBlk, float step, float zero, float nb, f32x2_t acc) { return dot<false>(w, xs + col, nBlk, step, zero, nb, acc); }
+    /* a block column's chunks side by side */
+    __device__ static __forceinline__ f32x2_t run_side(u32x4 w, const f32x4* xs, float step, float zero, float nb, f32x2_t acc) { return dot<true>(w, xs, 1, step, zero, nb, acc); }
+    template <int K>
+    __device__ static __forceinline__ uint32_t swizzle(uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x8000 | K | (K << 2) | (K << 4) | (K << 6)); }
+    // SWIZZLE: the quad exchanges its table words through the LDS crossbar instead of by DPP moves, each two vector-pipe slots
+    template <bool SWIZZLE>
+    __device__ static __forceinline__ f32x2_t dot(u32x4 w, const f32x4* xs, int stride, float step, float zero, float nb, f32x2_t acc) {
         const float q0 = (float)((threadIdx.x & 3) << 2);
         uint32_t r = pack_bf16x2(fmaf(q0, step, nb), fmaf(q0 + 1.0f, step, nb));
         const uint32_t P0 = pack_bf16x2(bf_lo(r) - zero, bf_hi(r) - zero);
@@ -378,12 +385,17 @@ struct BlockDotF<FMT_Q4P> {
         const uint32_t P1 = pack_bf16x2(bf_lo(r) - zero, bf_hi(r) - zero);
         const uint32_t tlm = __builtin_amdgcn_perm(P1, P0, 0x06040200u), thm = __builtin_amdgcn_perm(P1, P0, 0x07050301u);
         PermLut t;
-        t.tl[0] = quad_bcast<0>(tlm), t.tl[1] = quad_bcast<1>(tlm), t.tl[2] = quad_bcast<2>(tlm), t.tl[3] = quad_bcast<3>(tlm);
-        t.th[0] = quad_bcast<0>(thm), t.th[1] = quad_bcast<1>(thm), t.th[2] = quad_bcast<2>(thm), t.th[3] = quad_bcast<3>(thm);
-        acc = perm_fma_dword(w.w, xs[col], xs[nBlk + col], t, acc);
-        acc = perm_fma_dword(w.z, xs[2 * nBlk + col], xs[3 * nBlk + col], t, acc);
-        acc = perm_fma_dword(w.y, xs[4 * nBlk + col], xs[5 * nBlk + col], t, acc);
-        acc = perm_fma_dword(w.x, xs[6 * nBlk + col], xs[7 * nBlk + col], t, acc);
+        if constexpr (SWIZZLE) {
+            t.tl[0] = swizzle<0>(tlm), t.tl[1] = swizzle<1>(tlm), t.tl[2] = swizzle<2>(tlm), t.tl[3] = swizzle<3>(tlm);
+            t.th[0] = swizzle<0>(thm), t.th[1] = swizzle<1>(thm), t.th[2] = swizzle<2>(thm), t.th[3] = swizzle<3>(thm);
+        } else {
+            t.tl[0] = quad_bcast<0>(tlm), t.tl[1] = quad_bcast<1>(tlm), t.tl[2] = quad_bcast<2>(tlm), t.tl[3] = quad_bcast<3>(tlm);
+            t.th[0] = quad_bcast<0>(thm), t.th[1] = quad_bcast<1>(thm), t.th[2] = quad_bcast<2>(thm), t.th[3] = quad_bcast<3>(thm);
+        }
+        acc = perm_fma_dword(w.w, xs[0], xs[stride], t, acc);
+        acc = perm_fma_dword(w.z, xs[2 * stride], xs[3 * stride], t, acc);
+        acc = perm_fma_dword(w.y, xs[4 * stride], xs[5 * stride], t, acc);
+        acc = perm_fma_dword(w.x, xs[6 * stride], xs[7 * stride], t, acc);
         return acc;
     }
 };

@@ -72,6 +72,41 @@ def test_long_4bit_rows_through_two_fp32_windows_are_bit_exact(cctx, canon, m, k
     assert np.array_equal(y0, ref)
 
 
+@pytest.mark.parametrize("m,k", [(262160, 128), (65552, 512), (6562, 5120), (2056, 32768), (2048, 33792)])  # 4 lanes a row and one step, 16, an odd number of row slots, the longest x of a workgroup per CU, one longer
+def test_large_4bit_matrices_are_bit_exact(cctx, canon, m, k):
+    """2^20 blocks and more: one workgroup per CU (gemv_q4_kernel)"""
+    ctx = cctx
+    rng = np.random.default_rng(m + k)
+    w = O.f32_to_bf16(rng.standard_normal(size=(m, k), dtype=np.float32) * np.float32(0.05))
+    x = O.f32_to_bf16(rng.normal(0, 1.0, size=k).astype(np.float32))
+    ow = O.quantize(w, m, k, L.Q4)
+    y = u16(ctx.linear(ctx.upload_blob(L.Q4, m, k, ow.blob()), bf16_t(x, ctx.device)))
+    ref = O.linear(ow, x)
+    assert np.array_equal(y, ref), "%dx%d: %d of %d outputs differ" % (m, k, int((y != ref).sum()), m)
+
+
+def test_large_fused_entries_are_bit_exact(cctx, canon):
+    """the same form behind a norm: three matrices, gate and up"""
+    ctx = cctx
+    rng = np.random.default_rng(6)
+    k = 5120
+    x = O.f32_to_bf16(rng.normal(0, 1.0, size=k).astype(np.float32))
+    nw = O.f32_to_bf16((1 + rng.normal(0, 0.1, size=k)).astype(np.float32))
+    xn = O.rmsnorm(x, nw, 1e-6)
+    made = lambda m: O.quantize(O.f32_to_bf16(rng.standard_normal(size=(m, k), dtype=np.float32) * np.float32(0.05)), m, k, L.Q4)
+    ms = [5000, 1026, 1034]
+    ows = [made(m) for m in ms]
+    ys = ctx.norm_linear(bf16_t(x, ctx.device), bf16_t(nw, ctx.device), [ctx.upload_blob(L.Q4, m, k, ow.blob()) for m, ow in zip(ms, ows)], 1e-6)
+    with O.canonical(rows=sum(ms)):
+        for y, ow in zip(ys, ows):
+            assert np.array_equal(u16(y), O.linear(ow, xn))
+    f = 4102
+    og, ou = made(f), made(f)
+    act = u16(ctx.norm_gateup_swiglu(bf16_t(x, ctx.device), bf16_t(nw, ctx.device), ctx.upload_blob(L.Q4, f, k, og.blob()), ctx.upload_blob(L.Q4, f, k, ou.blob()), 1e-6))
+    with O.canonical(rows=f):
+        assert np.array_equal(act, O.swiglu(O.linear(og, xn), O.linear(ou, xn)))
+
+
 def test_fused_entries_are_bit_exact(cctx, canon):
     """fused RMSNorm + Q|K|V (rows of the launch = all three matrices), paired gate / up + SwiGLU, LM head + arg-max"""
     ctx = cctx
