@@ -20,6 +20,8 @@
 // nsp-1 reads every partial with agent-scope relaxed atomic loads (`sc1`) after a barrier, and re-zeroes the counter.
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "kf_attn_common.h"
 
 namespace kf {
@@ -123,7 +125,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(const AttnArgs a) {
                 if (has_new && valid[u] && t == pos) ck[u] = *reinterpret_cast<const u32x4*>(knew + d0);
             }
             if (tb - grp - wave * KPW + ATTN_U * tstride < t1) issue(tb + ATTN_U * tstride, t1);
-            canon_batch<GQ, LPK>(A, qf, ck, cv, valid, lpk_log2, rden);
+            canon_batch<GQ, LPK, ATTN_U, GQ == 4>(A, qf, ck, cv, valid, lpk_log2, rden);
         }
         // ---- the wave's key groups summed (reduce-scatter by row swaps), the waves through LDS: exact rescales to the slice's maximum exponent
         canon_wave_to_lds<GQ, LPK>(A, comb + (size_t)wave * GQ * PS, hd, lane, d0);
@@ -171,27 +173,38 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(const AttnArgs a) {
     if (!flag[0]) return;
 
     // Every thread merges its output elements over the slices: the head is the same for the whole wave (64 | hd), lane sp of the wave fetches (m, L) of slice sp,
-    // the maximum exponent and the rescaled L are formed in registers; the element's own chain walks the slices in order (fp64: the order does not matter).
+    // the maximum exponent and the rescaled L are formed in registers; the element's own chain walks the slices in order (fp64: the order does not matter).  All loads set out before the
+    // first is waited for: each takes the way to memory, and one after the other 32 slices' took 6 of the kernel's 26 us.
     constexpr int NT = NW * 64;
     constexpr int NV = (GQ * 128 + NT - 1) / NT; /* output elements per thread (hd <= 128) */
+    constexpr int NE = NV <= 2 ? NV : 1;         /* of them at a time: 64 registers each */
 #pragma unroll
-    for (int e = 0; e < NV; e++) {
-        const int i = tid + e * NT;
-        const bool in = i < GQ * hd;
-        const int hq = in ? (i >> hd_log2) : 0, d = i & (hd - 1);
-        const double* p = part + (size_t)(h0 + hq) * nsp * PS;
-        const bool mine = in && lane < nsp;
-        const float ms = mine ? (float)__hip_atomic_load(p + (size_t)lane * PS + hd + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -__builtin_inff();
-        const double ls = mine ? __hip_atomic_load(p + (size_t)lane * PS + hd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-        const float Mx = wave_max(ms);
-        const int sh = canon_shift(ms - Mx);
-        const double L = wave_sum_f64_fast(ldexp_d(ls, sh));
-        double o = 0.0;
-        for (int sp = 0; sp < nsp; sp++) {
-            const double v = in ? __hip_atomic_load(p + (size_t)sp * PS + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-            o += ldexp_d(v, __builtin_amdgcn_readlane(sh, sp));
+    for (int e0 = 0; e0 < NV; e0 += NE) {
+        float ms[NE];
+        double ls[NE], v[NE][KF_ATTN_MAX_SPLITS];
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const int i = tid + (e0 + e) * NT, hq = i < GQ * hd ? i >> hd_log2 : 0, d = i & (hd - 1); /* a thread past the last element: head 0's */
+            const double* p = part + (size_t)(h0 + hq) * nsp * PS;
+            const int mine = lane < nsp ? lane : nsp - 1;
+            ms[e] = (float)__hip_atomic_load(p + (size_t)mine * PS + hd + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ls[e] = __hip_atomic_load(p + (size_t)mine * PS + hd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int sp = 0; sp < KF_ATTN_MAX_SPLITS; sp++) v[e][sp] = __hip_atomic_load(p + (size_t)(sp < nsp ? sp : nsp - 1) * PS + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (in) odst[(size_t)(h0 + hq) * hd + d] = f2bf((float)(o / L));
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const int i = tid + (e0 + e) * NT;
+            const float mv = lane < nsp ? ms[e] : -__builtin_inff();
+            const float Mx = wave_max(mv);
+            const int sh = canon_shift(mv - Mx);
+            const double L = wave_sum_f64_fast(ldexp_d(lane < nsp ? ls[e] : 0.0, sh));
+            double o = 0.0;
+#pragma unroll
+            for (int sp = 0; sp < KF_ATTN_MAX_SPLITS; sp++)
+                if (sp < nsp) o += ldexp_d(v[e][sp], __builtin_amdgcn_readlane(sh, sp));
+            if (i < GQ * hd) odst[(size_t)(h0 + (i >> hd_log2)) * hd + (i & (hd - 1))] = f2bf((float)(o / L));
+        }
     }
     if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -496,18 +509,25 @@ int attn_launch(hipStream_t st, AttnArgs& a) {
     if (a.n_tok < 1) a.n_tok = 1;
     if (!batch) a.n_tok = 1, a.q_stride = 0;
     const int pos_max = a.pos + a.n_tok - 1;
-    const int nsp = batch ? 1 : attn_splits(a.pos, a.n_kv);
+    int nsp = batch ? 1 : attn_splits(a.pos, a.n_kv);
+    a.inv_sqrt_hd_den = sqrtf((float)hd);
+    // Canonical order, hd 128, GQA-8 and -4: short contexts by workgroups of two heads, four waves and 64 keys (a short chain each); above 1024 keys by workgroups of four heads and eight waves, one
+    // to a CU, whose slices grow with the context: two to four times fewer partials to leave, count in and merge, K and V unpacked once for four heads, and all of them resident at once (of two heads and
+    // 145 registers, 768 of 1024 were).  us, 64 heads on 8, two heads | four, at 512 keys 7.4 | 10.1, 1024 9.6 | 10.2, 1344 12.4 | 10.7, 1664 13.2 | 10.9,
+    // 4000 19.6 | 13.4 (26.5 with the merge's loads one after the other); four heads and four waves at 4000 with 32 | 16 slices 16.9 | 15.9, eight waves with 32 (two rounds) 21.5.
+    const int knob = g_knobs.attn_gq_split;
+    const bool fours = a.canon && (GQ == 8 || GQ == 4) && hd == 128 && !batch && knob <= 2 && a.pos >= 1024;
+    a.gq_split = !a.canon ? 1 : GQ == 8 ? (knob ? knob : fours ? 2 : 4) : GQ == 4 && !fours && knob != 2 ? 2 : 1;
+    const int gq_wg = GQ / a.gq_split; /* query heads per workgroup */
+    if (fours) nsp = std::max(1, std::min({nsp, 256 / (a.n_kv * a.gq_split), (a.pos + 128) / 128}));
     a.n_splits = nsp;
     a.chunk = (pos_max + 1 + nsp - 1) / nsp;
-    a.inv_sqrt_hd_den = sqrtf((float)hd);
-    a.gq_split = (a.canon && GQ == 8) ? (g_knobs.attn_gq_split == 8 ? 8 : (g_knobs.attn_gq_split == 4 ? 4 : 2)) : ((a.canon && GQ == 4 && g_knobs.attn_gq_split >= 4) ? 2 : 1);
     a.cnt_stride = KF_ATTN_CNT_BYTES / 4 / (a.n_kv * a.gq_split); /* arrival counters of different kv-heads in different cache lines: atomics on one line serialise */
     if (a.cnt_stride > 64) a.cnt_stride = 64;
     if (a.cnt_stride < 1) return KF_INVALID_ARGS;
     // one 64-key batch per 4-wave workgroup (one wave per SIMD: the kernel is bound by VALU issue inside a latency chain, so
     // spreading the keys over more CUs beats more waves per CU); 8 waves once the slices have to grow past 128 keys
-    int NW = (GQ <= 2 && a.chunk > 128) ? 8 : 4;
-    const int gq_wg = GQ / a.gq_split; /* query heads per workgroup */
+    int NW = fours || (GQ <= 2 && a.chunk > 128) ? 8 : 4;
     size_t smem = sizeof(double) * ((size_t)NW * gq_wg * (hd + 2)) + sizeof(uint16_t) * ((size_t)gq_wg * hd + hd) + 16;
     const size_t smem_fast = sizeof(uint16_t) * ((size_t)GQ * hd + hd) + sizeof(float) * (NW * GQ + 4 + (size_t)NW * GQ * (hd + 4));
     if (!a.canon) smem = smem_fast;
@@ -526,13 +546,15 @@ int attn_launch(hipStream_t st, AttnArgs& a) {
         case 1: if (NW == 8) KF_ATTN_GO(1, 8); else KF_ATTN_GO(1, 4); break;
         case 2: if (NW == 8) KF_ATTN_GO(2, 8); else KF_ATTN_GO(2, 4); break;
         case 4:
-            if (a.gq_split == 2) KF_ATTN_GO(2, 4); /* canonical order: two workgroups of two heads each, as for GQA-8 */
+            if (a.gq_split == 2) KF_ATTN_GO(2, 4);
+            else if (NW == 8) KF_ATTN_GO(4, 8);
             else KF_ATTN_GO(4, 4);
             break;
         case 8:
             if (a.gq_split == 8) KF_ATTN_GO(1, 4); /* one head per workgroup */
             else if (a.gq_split == 4) KF_ATTN_GO(2, 4); /* four workgroups of two heads each */
-            else if (a.gq_split == 2) KF_ATTN_GO(4, 4); /* two workgroups of four heads each (canonical order) */
+            else if (a.gq_split == 2 && NW == 8) KF_ATTN_GO(4, 8); /* two workgroups of four heads each (canonical order) */
+            else if (a.gq_split == 2) KF_ATTN_GO(4, 4);
             else KF_ATTN_GO(8, 4);
             break;
         default: return KF_INVALID_ARGS;

@@ -174,18 +174,14 @@ __device__ __forceinline__ void canon_apply_items(CanonAcc<GQ>& A, double p, con
 // (Measured and removed: two query heads per v_pk_fma_f32 / v_pk_mul_f32 / v_pk_add_f32 in the score chain and in the exponential's polynomial -- bit-identical (179
 //  canonical tests), half the vector instructions of those two parts, and slower: the single-sequence engine 2304 -> 2103 tokens/s, 32 batched sequences 7770 -> 7410: the operand
 //  pairs have to be assembled in even-aligned register pairs per use.)
-#ifndef KF_CANON_ITEMS
-#define KF_CANON_ITEMS 0 /* scratch/build_variant.py A/B.  1 = the item-per-lane form below: bit for bit the same (194 canonical tests), a quarter fewer vector instructions per key
-                            tile on paper -- and SLOWER on the part: 32 sequences 7770 -> 6360 tokens/s, 16: 6240 -> 5710, 8: 4625 -> 4450, the single-sequence engine unchanged (each
-                            broadcast is a DPP move with its wait states in front of a dependent fp64 chain; the replicated form keeps sixteen independent lanes busy instead).  Off. */
-#endif
 // one batch of U key tiles of this lane's key group: k / v tiles (8 elements of this lane), validity per tile; q as 8 floats per head
-// KF_CANON_ITEMS (measured and left off): hd = 128, a key group is a row of 16 lanes -- the U * GQ dots of a group stand in all of its 16 lanes after the tree; the
-// score's scale and rounding, the exponential's parts and the exact power-of-two weight p worked out ONCE, item i = u * GQ + hq in lane i of the group, p_i handed to the
-// group's lanes by a row broadcast: the same operations on the same values as the per-lane form.
-template <int GQ, int LPK, int U = ATTN_U>
+// ITEMS (hd = 128: a key group is a row of 16 lanes; bit for bit the same): the U * GQ dots of a group stand in all of its 16 lanes after the tree; the score's scale and rounding, the exponential's parts and the
+// exact power-of-two weight p are worked out ONCE, item i = u * GQ + hq in lane i of the group, p_i handed to the group's lanes by a row broadcast.  A quarter fewer vector instructions, but each broadcast is a DPP
+// move with its wait states in front of a dependent fp64 chain: worth it where several waves share a SIMD and four heads fill the row (kf_attn.hip), not in the persistent engines (32 batched sequences 7770 ->
+// 6360 tokens/s, one unchanged).
+template <int GQ, int LPK, int U = ATTN_U, bool ITEMS = false>
 __device__ __forceinline__ void canon_batch(CanonAcc<GQ>& A, const float (&qf)[GQ][8], const u32x4 (&kk)[U], const u32x4 (&vv)[U], const bool (&valid)[U], int lpk_log2, float rden) {
-    if constexpr (KF_CANON_ITEMS && LPK == 16 && U * GQ <= 16 && (GQ & (GQ - 1)) == 0 && (U & (U - 1)) == 0) {
+    if constexpr (ITEMS && LPK == 16 && U * GQ <= 16 && (GQ & (GQ - 1)) == 0 && (U & (U - 1)) == 0) {
         constexpr int NI = U * GQ;
         const int lig = (int)(threadIdx.x & 15);
         float d[U][GQ];

@@ -154,7 +154,7 @@ struct Knobs {
     int attn_pair_min = 256;  /* prompt tokens from which kf_attn_prefill takes its paired two-key-half form (when there is about one workgroup per CU or fewer) */
     int attn_walk_min = 512;  /* keys from which it otherwise takes the walk whose tiles come by loads into LDS (same bits) */
     int g3_wide = 1;      /* kf_gemm3.hip: tiles of 192 rows may be picked (0: the choice is among the others; same bits) */
-    int attn_gq_split = 4; /* canonical decode attention of a GQA-8 model: workgroups per (kv-head, slice), 2 or 4 */
+    int attn_gq_split = 0; /* canonical decode attention of a GQA-8 model: workgroups per (kv-head, slice), 2 (four heads each), 4 or 8 (0: attn_launch's rule) */
     int g3_first = 256;   /* token rows from which bf16 operands try the kf_gemm3.hip tile kernels before the 32 x 32 direct kernel */
     int q1_tab = 1;       /* 1-bit mat-vec through the LDS selector table (0: the per-bit select form; same bits) */
     long gemv_waves = 0;  /* > 0: waves a mat-vec launch aims for (0: the launcher's rule) */

@@ -150,6 +150,12 @@ def test_decode_attention_is_bit_exact(cctx, n_head, n_kv, hd, pos):
     assert np.array_equal(out, ref), "%d of %d outputs differ" % (int((out != ref).sum()), out.size)
 
 
+@pytest.mark.parametrize("n_head,n_kv,hd,pos", [(64, 8, 128, 1023), (64, 8, 128, 1024), (64, 8, 128, 1101), (4, 1, 128, 4095), (32, 8, 128, 1030), (64, 64, 128, 1500)])
+def test_decode_attention_by_fours_is_bit_exact(cctx, n_head, n_kv, hd, pos):
+    """four heads and eight waves a workgroup above 1024 keys: the last position of two heads, the first of four, uneven slices, most slices, GQA-4; no GQA"""
+    test_decode_attention_is_bit_exact(cctx, n_head, n_kv, hd, pos)
+
+
 def _steps(m, om, cfg, n, forced, use_graph):
     m.set_forced(forced)
     m.set_state(int(forced[0]), 0)
