@@ -172,8 +172,10 @@ struct XCfg {
                                   SH::P6::nBlk == SH::P6::iters * SH::P6::LPR;
     static constexpr int maxR = (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R) > (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R) ? (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R)
                                                                                                                                       : (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R);
-    // MF: the 4-bit phases of the batched form on the matrix cores (xe_unit_mf): a wave takes UNITS of 4 KiB, four loads of a whole KiB each
-    static constexpr bool MF = NB_ > 1 && FMT_ == FMT_Q4P && SH::P1::LPR >= 32 && SH::P4::LPR >= 32 && SH::P5::LPR >= 32 && SH::P6::LPR >= 32;
+    // MF: the 4-bit phases on the matrix cores (xe_unit_mf): a wave takes UNITS of 4 KiB, four loads of a whole KiB each.  For several sequences, and for one where a phase's rows are long and many: there the
+    // products cost what the vector pipe's did and the whole-KiB units are the gain (28 layers of 2048 x 6144, 8 decoders of one sequence at 2 k
+    // keys 5202 -> 4940 us a step, two decoders 4988 -> 4849; of 1024 x 3072, short rows, 8 decoders 1776 -> 1971)
+    static constexpr bool MF = (NB_ > 1 || (DIM_ >= 2048 && !TP_ && WPC_ == 1 && !FUSED && NG == 1)) && FMT_ == FMT_Q4P && SH::P1::LPR >= 32 && SH::P4::LPR >= 32 && SH::P5::LPR >= 32 && SH::P6::LPR >= 32;
     template <class P>
     struct MG { /* a phase's figures (P: PlanT): units of CE block columns x RS rows, 64 / CE sets of four; a slot: RS rows, all its NIT units */
         static constexpr int CE = P::nBlk % P::LPR == 0 ? P::LPR : 32, RS = 4 * (64 / CE), NIT = P::nBlk / CE, H = P::LPR / CE, SPG = P::R / RS;
@@ -196,7 +198,7 @@ struct XCfg {
         }
         static constexpr bool ok = (CE == 32 || CE == 64) && P::nBlk % CE == 0 && NIT >= H && NIT <= 16 && (H == 1 || H == 2) && P::R % RS == 0;
     };
-    static constexpr bool MFH = MF && HLPR == 64 && HnBlk % 64 == 0; /* the head on the matrix cores too: slots of four rows */
+    static constexpr bool MFH = MF && NB_ > 1 && HLPR == 64 && HnBlk % 64 == 0; /* the head on the matrix cores too: slots of four rows */
     static constexpr int RING = MF ? (NWV_ == 8 ? 4 : 2) : DEPTH_; /* entries (MF: units) of a phase in flight per wave */
     static_assert(!MF || !PREP, "sixteen bytes a lane");
     static_assert(!MF || (MG<typename SH::P1>::ok && MG<typename SH::P4>::ok && MG<typename SH::P5>::ok && MG<typename SH::P6>::ok), "whole entries, whole slots");
