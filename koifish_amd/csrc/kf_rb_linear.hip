@@ -14,7 +14,7 @@ namespace kf {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 // k-steps of a run, loaded one run ahead: a wave of several weight blocks or of many token columns has its bytes in flight with two, and stays within 128 registers, two workgroups of eight waves to a CU
-// (us at four | two, two blocks: 32 rows of 32768 x 2048 27.7 | 25.4, of 6464 x 2048 8.8 | 8.2, three blocks of 12288 x 2048 13.2 | 11.9; with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
+// (us at four | two, 32 rows, two blocks of 32768 x 2048 27.7 | 26.3, three of 12288 x 2048 12.9 | 12.1; with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
 constexpr int rb_run(int nt, int mg) { return nt >= 3 || mg >= 2 ? 2 : 4; }
 
 __device__ __forceinline__ f32x4 rb_mfma16(u32x4 a, u32x4 b, f32x4 c) {
@@ -111,7 +111,7 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
 
 // A run's token rows on their way to the fragments: loaded in whole lines (a row's U x 64 bytes by neighbouring lanes) a run ahead, turned round in this wave's own LDS, no barrier.  A fragment read
 // straight from memory takes half a line of each of 16 rows, and a workgroup of 32 rows reads twice as many token bytes as weight bytes: the CU's way to its L2 was the bound, not HBM.  32 rows,
-// 2048 x 6144 (128 workgroups): 16.9 -> 12.4 us; gate and up 12288 x 2048: 17.8 -> 15.5; 32768 x 2048: 43.2 -> 32.6 (134 MB: 4.1 TB/s).  Prefetching alone, without the lines, gave 1 %, and 16 waves
+// 2048 x 6144 (128 workgroups): 16.9 -> 12.4 us; gate and up 12288 x 2048: 17.8 -> 15.5; 32768 x 2048: 43.2 -> 32.6 (each with one block of weight rows, or two gated, to a workgroup).  Prefetching alone, without the lines, gave 1 %, and 16 waves
 // instead of 8 where workgroups are few cost 10 %.
 template <int NT, int U>
 struct RbTokens {
@@ -152,12 +152,13 @@ struct RbTokens {
 template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
-    constexpr int U = rb_run(NT, MG);
+    constexpr int U = rb_run(NT, MG), DEAL = NT >= 4 ? 2 : 4; /* steps on the way at a time; steps a wave takes in a row, whatever U: part of the result's last bits */
+    static_assert(DEAL == U || DEAL == 2 * U, "a deal is a run or two");
     static_assert(!(NORM && TURN), "normed fragments are made from the residual sum");
     using Tokens = RbTokens<NT, U>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, q4 = lane >> 4;
     const int unit0 = blockIdx.x * MG, units = p.m / 16, part = PARTS ? (int)blockIdx.y : 0, steps = p.k / 32, nstep = PARTS ? steps * (part + 1) / p.parts : steps; /* this part's steps end here */
     const uint16_t* W = reinterpret_cast<const uint16_t*>(p.w);
     const uint16_t* X = reinterpret_cast<const uint16_t*>(p.x);
@@ -176,7 +177,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
         else wr[g] = W + (size_t)unit * 16 * p.k + 8 * lane;
     }
     u32x4 a[U][MG], b[U][NT];
-    int s = (PARTS ? steps * part / p.parts : 0) + wid * U;
+    int s = (PARTS ? steps * part / p.parts : 0) + wid * DEAL, half = 0;
     rb_load_w<MG, U>(a, wr, s, nstep);
     const uint16_t* xp[NT];
     Tokens tok;
@@ -219,7 +220,8 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     for (int g = 0; g < MG; g++)
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (; s < nstep; s += NW * U) {
+    for (int s1; s < nstep; s = s1) {
+        s1 = DEAL > U && half == 0 ? s + U : s + U + (NW - 1) * DEAL, half ^= 1; /* the wave's next run */
         u32x4 an[U][MG];
         if constexpr (NORM) {
             f32x4 z0[U], z1[U];
@@ -229,7 +231,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
                 const int k0 = 32 * (s + u < nstep ? s + u : nstep - 1);
                 z0[u] = rb_ld4(zp + k0), z1[u] = rb_ld4(zp + k0 + 4), g[u] = *reinterpret_cast<const u32x4*>(gp + k0);
             }
-            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
+            rb_load_w<MG, U>(an, wr, s1, nstep);
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const f32x4 o0 = f32x4{z0[u].x * rs * bf_lo(g[u].x), z0[u].y * rs * bf_hi(g[u].x), z0[u].z * rs * bf_lo(g[u].y), z0[u].w * rs * bf_hi(g[u].y)};
@@ -243,11 +245,11 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
             }
         } else if constexpr (TURN) {
             tok.turn(b);
-            if (s + NW * U < nstep) tok.load(s + NW * U, nstep); /* wave-uniform */
-            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
+            if (s1 < nstep) tok.load(s1, nstep); /* wave-uniform */
+            rb_load_w<MG, U>(an, wr, s1, nstep);
         } else {
             rb_load_x<NT, U, false>(b, xp, s, nstep);
-            rb_load_w<MG, U>(an, wr, s + NW * U, nstep);
+            rb_load_w<MG, U>(an, wr, s1, nstep);
         }
         rb_multiply<NT, MG, U>(a, b, acc);
 #pragma unroll
@@ -353,11 +355,13 @@ static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
 }
 // How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
 // one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
-// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.2 10.9 11.8 14.2; plain 10.1 11.4 14.4 19.5 -> 10.0 11.0 11.9 15.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.3 8.2 10.7.
+// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.6 11.3 12.1 14.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.8 8.7 10.5.
 // More than that is bound by HBM while the rows are few: pairs of blocks, many workgroups that follow each other; else the least work for the busiest CU, by workgroups of four waves, several to a
-// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 22.3 22.2 25.5 29.3 (134 MB: 5.3 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 32.4 32.1 34.6 42.4.
-static int stream_blocks(int units, int n) {
-    if (units <= 1024) return (units + 255) / 256;
+// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 23.0 23.9 26.3 28.8 (134 MB: 5.1 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 33.0 33.7 35.7 42.1.
+// The number of waves is part of a result's last bits (each adds up a part of k), and up to 32 rows stays what it was with the smaller workgroups: four waves also for 768 to 1024 blocks of one matrix, from 17 rows in pairs
+// (12288 x 2048 plain 10.1 11.4 14.4 19.5 -> 10.1 11.4 13.6 14.7; eight waves of three blocks: 10.0 11.0 11.9 15.0).
+static int stream_blocks(int units, int n, bool wide) {
+    if (units <= 1024) return wide ? (units + 255) / 256 : n > 16 ? 2 : 1;
     int best = 2;
     long least = 0;
     for (int mg = 2; n > 24 && mg <= 4; mg++) {
@@ -372,9 +376,11 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const int cols = tiles ? q.e.tile : p.n, nt = (cols + 15) / 16, units = p.m / 16;
     if (nt > 4 || (tiles && q.e.tile % 16)) return 1;
     if (p.mode == KF_RB_SUM && ((long)p.n * q.e.top > KF_RB_SUM_PAIRS || q.e.tile < p.n)) return 1;
-    const int mg = !all ? (p.epilogue == KF_RB_GATED ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n);
+    const bool gated = p.epilogue == KF_RB_GATED;
+    const long small = (long)units / (gated ? 2 : 1) * (tiles ? q.e.n_tile : p.parts > 1 ? p.parts : 1); /* workgroups of 16 rows, of 16 gates and 16 ups */
+    const bool wide = p.k >= 512 && (all && p.n > 32 ? units <= 1024 : small < 768);                        /* few workgroups: more waves each, more loads in flight per CU */
+    const int mg = !all ? (gated ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n, wide);
     const dim3 grid((units + mg - 1) / mg, tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
-    const bool wide = p.k >= 512 && (all ? units <= 1024 || p.n <= 24 : (long)grid.x * grid.y < 768); /* few workgroups: more waves each, more loads in flight per CU */
 #define RB_STREAM_MG(nt, nw) (mg == 1 ? stream_go<nt, 1, nw>(st, q, grid) : mg == 2 ? stream_go<nt, 2, nw>(st, q, grid) : mg == 3 ? stream_go<nt, 3, nw>(st, q, grid) : stream_go<nt, 4, nw>(st, q, grid))
 #define RB_STREAM(nt) (!all ? (wide && nt <= 2 ? expert_go<nt, 8>(st, q, grid) : expert_go<nt, 4>(st, q, grid)) : wide ? RB_STREAM_MG(nt, 8) : RB_STREAM_MG(nt, 4))
     return nt == 1 ? RB_STREAM(1) : nt == 2 ? RB_STREAM(2) : nt == 3 ? RB_STREAM(3) : RB_STREAM(4);

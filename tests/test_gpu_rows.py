@@ -543,3 +543,32 @@ def test_embed_and_pack(ctx, kind):
     L.check(ctx.hip.kf_rb_embed_state(ctx.h, typ, tab.data_ptr(), V, dim, ld, state.data_ptr(), forced.data_ptr(), 8, 8, 4, x.data_ptr(), h.data_ptr(), meta.data_ptr()))
     assert meta[:, 0].tolist() == [2, -1, -1, 7] and meta[:, 1].tolist() == [0, 1, 2, 3] and state[:, 3].tolist() == [0, 0, 64, 0]
     assert torch.equal(x[0, :dim], src[1].float()) and torch.equal(x[3, :dim], src[9].float())
+
+
+@pytest.mark.parametrize("count", [1, 5, 767, 768])
+def test_put_words(ctx, count):
+    """words of the host as kernel arguments: nothing behind them is touched; none, too many or an odd address are refused"""
+    src = np.arange(7, 7 + count, dtype=np.int32) * -3
+    dst = torch.full((800,), 11, dtype=torch.int32, device="cuda")
+    L.check(ctx.hip.kf_put_words(ctx.h, C.c_void_p(dst.data_ptr()), src.ctypes.data_as(C.c_void_p), count))
+    got = dst.cpu().numpy()
+    assert np.array_equal(got[:count], src) and (got[count:] == 11).all()
+    for bad in (0, -1, 769):
+        assert ctx.hip.kf_put_words(ctx.h, C.c_void_p(dst.data_ptr()), src.ctypes.data_as(C.c_void_p), bad) < 0
+    assert ctx.hip.kf_put_words(ctx.h, C.c_void_p(dst.data_ptr() + 2), src.ctypes.data_as(C.c_void_p), 1) < 0
+
+
+@pytest.mark.parametrize("ld,slots", [(4, [2, 0]), (4096, [1]), (4100, [3, 5, 0, 4])])
+def test_slot_logits(ctx, ld, slots):
+    """rows to their slots' places and nowhere else, the slots' status words cleared"""
+    n = len(slots)
+    src, dst = torch.randn(n, ld, device="cuda"), torch.full((6, ld), 7.0, device="cuda")
+    meta = torch.tensor([[9, s, 0, 0] for s in slots], dtype=torch.int32, device="cuda")
+    state = torch.full((6, 4), 5, dtype=torch.int32, device="cuda")
+    L.check(ctx.hip.kf_rb_slot_logits(ctx.h, C.c_void_p(src.data_ptr()), C.c_int64(ld), n, C.c_void_p(meta.data_ptr()), C.c_void_p(dst.data_ptr()), C.c_void_p(state.data_ptr())))
+    for s in range(6):
+        assert torch.equal(dst[s], src[slots.index(s)]) if s in slots else (dst[s] == 7.0).all()
+        assert state[s].tolist() == [5, 5, 5, 0 if s in slots else 5]
+    for bad in (dict(ld=0), dict(ld=6), dict(n=0)):
+        k = dict(dict(ld=ld, n=n), **bad)
+        assert ctx.hip.kf_rb_slot_logits(ctx.h, C.c_void_p(src.data_ptr()), C.c_int64(k["ld"]), k["n"], C.c_void_p(meta.data_ptr()), C.c_void_p(dst.data_ptr()), C.c_void_p(state.data_ptr())) < 0
