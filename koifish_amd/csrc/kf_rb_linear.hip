@@ -13,8 +13,10 @@ namespace kf {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-// k-steps of a run, loaded one run ahead: a wave of several weight blocks or of many token columns has its bytes in flight with two, and stays within 128 registers, two workgroups of eight waves to a CU
-// (us at four | two, 32 rows, two blocks of 32768 x 2048 27.7 | 26.3, three of 12288 x 2048 12.9 | 12.1; with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
+// k-steps a wave takes in a row (part of a result's last bits: which steps a wave adds up), its token rows' run in LDS
+constexpr int rb_deal(int nt) { return nt >= 4 ? 2 : 4; }
+// k-steps of weights loaded at a time, one run ahead: a wave of several weight blocks has its bytes in flight with two (us at four | two, 32 rows, two blocks of 32768 x 2048 27.7 | 26.0, three of 12288 x 2048 12.9 | 12.3;
+// with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
 constexpr int rb_run(int nt, int mg) { return nt >= 3 || mg >= 2 ? 2 : 4; }
 
 __device__ __forceinline__ f32x4 rb_mfma16(u32x4 a, u32x4 b, f32x4 c) {
@@ -49,14 +51,14 @@ __device__ __forceinline__ void rb_load_x(u32x4 (&b)[U][NT], const uint16_t* con
         }
     }
 }
-template <int NT, int MG, int U>
-__device__ __forceinline__ void rb_multiply(const u32x4 (&a)[U][MG], const u32x4 (&b)[U][NT], f32x4 (&acc)[MG][NT]) {
+template <int NT, int MG, int U, int B>
+__device__ __forceinline__ void rb_multiply(const u32x4 (&a)[U][MG], const u32x4 (&b)[B][NT], int first, f32x4 (&acc)[MG][NT]) {
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
         for (int g = 0; g < MG; g++)
 #pragma unroll
-            for (int t = 0; t < NT; t++) acc[g][t] = rb_mfma16(a[u][g], b[u][t], acc[g][t]);
+            for (int t = 0; t < NT; t++) acc[g][t] = rb_mfma16(a[u][g], b[first + u][t], acc[g][t]);
 }
 // the waves' partial tiles of the blocks from unit0 -> outputs; list: the columns are pairs; units: blocks past them repeat the last one.  GATED: a block is 8 gate rows and their 8 up rows
 template <int NT, int MG, int NW, bool GATED>
@@ -152,10 +154,10 @@ struct RbTokens {
 template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
-    constexpr int U = rb_run(NT, MG), DEAL = NT >= 4 ? 2 : 4; /* steps on the way at a time; steps a wave takes in a row, whatever U: part of the result's last bits */
-    static_assert(DEAL == U || DEAL == 2 * U, "a deal is a run or two");
+    constexpr int U = rb_run(NT, MG), DEAL = rb_deal(NT);
+    static_assert(DEAL % U == 0, "a deal is whole runs");
     static_assert(!(NORM && TURN), "normed fragments are made from the residual sum");
-    using Tokens = RbTokens<NT, U>;
+    using Tokens = RbTokens<NT, DEAL>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     auto& red = *reinterpret_cast<float(*)[NW][MG][16 * NT][17]>(smem); /* [wave][block][column][row], padded; after the waves' token rows */
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, q4 = lane >> 4;
@@ -176,8 +178,8 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
         if (GATED) wr[g] = W + (size_t)(2 * (unit >> 1) + (r16 >> 3)) * 16 * p.k + 8 * (16 * q4 + 8 * (unit & 1) + (r16 & 7)); /* half of the gate's tile, half of the up rows': whole lines of both */
         else wr[g] = W + (size_t)unit * 16 * p.k + 8 * lane;
     }
-    u32x4 a[U][MG], b[U][NT];
-    int s = (PARTS ? steps * part / p.parts : 0) + wid * DEAL, half = 0;
+    u32x4 a[U][MG], b[TURN ? DEAL : U][NT];
+    int s = (PARTS ? steps * part / p.parts : 0) + wid * DEAL;
     rb_load_w<MG, U>(a, wr, s, nstep);
     const uint16_t* xp[NT];
     Tokens tok;
@@ -198,7 +200,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     } else if constexpr (TURN) {
         tok.x = X, tok.lds = reinterpret_cast<uint16_t*>(smem) + wid * Tokens::LDS, tok.lane = lane;
 #pragma unroll
-        for (int i = 0; i < NT * U; i++) {
+        for (int i = 0; i < NT * DEAL; i++) {
             const int row = tok.row(i);
             tok.off[i] = (uint32_t)(row < p.n ? row : p.n - 1) * (uint32_t)p.ldx; /* <= 64 rows: below 2^32 (the launch sees to it) */
         }
@@ -220,42 +222,45 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     for (int g = 0; g < MG; g++)
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s1; s < nstep; s = s1) {
-        s1 = DEAL > U && half == 0 ? s + U : s + U + (NW - 1) * DEAL, half ^= 1; /* the wave's next run */
-        u32x4 an[U][MG];
-        if constexpr (NORM) {
-            f32x4 z0[U], z1[U];
-            u32x4 g[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int k0 = 32 * (s + u < nstep ? s + u : nstep - 1);
-                z0[u] = rb_ld4(zp + k0), z1[u] = rb_ld4(zp + k0 + 4), g[u] = *reinterpret_cast<const u32x4*>(gp + k0);
-            }
-            rb_load_w<MG, U>(an, wr, s1, nstep);
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const f32x4 o0 = f32x4{z0[u].x * rs * bf_lo(g[u].x), z0[u].y * rs * bf_hi(g[u].x), z0[u].z * rs * bf_lo(g[u].y), z0[u].w * rs * bf_hi(g[u].y)};
-                const f32x4 o1 = f32x4{z1[u].x * rs * bf_lo(g[u].z), z1[u].y * rs * bf_hi(g[u].z), z1[u].z * rs * bf_lo(g[u].w), z1[u].w * rs * bf_hi(g[u].w)};
-                b[u][0] = u32x4{pack_bf16x2(o0.x, o0.y), pack_bf16x2(o0.z, o0.w), pack_bf16x2(o1.x, o1.y), pack_bf16x2(o1.z, o1.w)};
-                if (blockIdx.x == 0 && r16 < p.n && s + u < nstep) { /* the normed rows themselves, once */
-                    const size_t at = (size_t)r16 * p.ldx + 32 * (s + u) + 8 * q4;
-                    rb_st4(p.norm_x + at, o0), rb_st4(p.norm_x + at + 4, o1);
-                    *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(const_cast<void*>(p.x)) + at) = b[u][0];
-                }
-            }
-        } else if constexpr (TURN) {
+    for (; s < nstep; s += NW * DEAL) {
+        if constexpr (TURN) {
             tok.turn(b);
-            if (s1 < nstep) tok.load(s1, nstep); /* wave-uniform */
-            rb_load_w<MG, U>(an, wr, s1, nstep);
-        } else {
-            rb_load_x<NT, U, false>(b, xp, s, nstep);
-            rb_load_w<MG, U>(an, wr, s1, nstep);
+            if (s + NW * DEAL < nstep) tok.load(s + NW * DEAL, nstep); /* wave-uniform */
         }
-        rb_multiply<NT, MG, U>(a, b, acc);
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int run = 0; run < DEAL; run += U) { /* (one that begins past the end meets zero weights) */
+            const int s0 = s + run, s1 = run + U < DEAL ? s0 + U : s + NW * DEAL;
+            u32x4 an[U][MG];
+            if constexpr (NORM) {
+                f32x4 z0[U], z1[U];
+                u32x4 g[U];
 #pragma unroll
-            for (int g = 0; g < MG; g++) a[u][g] = an[u][g];
+                for (int u = 0; u < U; u++) {
+                    const int k0 = 32 * (s0 + u < nstep ? s0 + u : nstep - 1);
+                    z0[u] = rb_ld4(zp + k0), z1[u] = rb_ld4(zp + k0 + 4), g[u] = *reinterpret_cast<const u32x4*>(gp + k0);
+                }
+                rb_load_w<MG, U>(an, wr, s1, nstep);
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const f32x4 o0 = f32x4{z0[u].x * rs * bf_lo(g[u].x), z0[u].y * rs * bf_hi(g[u].x), z0[u].z * rs * bf_lo(g[u].y), z0[u].w * rs * bf_hi(g[u].y)};
+                    const f32x4 o1 = f32x4{z1[u].x * rs * bf_lo(g[u].z), z1[u].y * rs * bf_hi(g[u].z), z1[u].z * rs * bf_lo(g[u].w), z1[u].w * rs * bf_hi(g[u].w)};
+                    b[u][0] = u32x4{pack_bf16x2(o0.x, o0.y), pack_bf16x2(o0.z, o0.w), pack_bf16x2(o1.x, o1.y), pack_bf16x2(o1.z, o1.w)};
+                    if (blockIdx.x == 0 && r16 < p.n && s0 + u < nstep) { /* the normed rows themselves, once */
+                        const size_t at = (size_t)r16 * p.ldx + 32 * (s0 + u) + 8 * q4;
+                        rb_st4(p.norm_x + at, o0), rb_st4(p.norm_x + at + 4, o1);
+                        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(const_cast<void*>(p.x)) + at) = b[u][0];
+                    }
+                }
+            } else {
+                if constexpr (!TURN) rb_load_x<NT, U, false>(b, xp, s0, nstep);
+                rb_load_w<MG, U>(an, wr, s1, nstep);
+            }
+            rb_multiply<NT, MG, U>(a, b, TURN ? run : 0, acc);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int g = 0; g < MG; g++) a[u][g] = an[u][g];
+        }
     }
     if constexpr (TURN) __syncthreads(); /* the token rows make way */
     rb_stream_finish<NT, MG, NW, GATED>(q, acc, red, list, unit0, units, tid, part);
@@ -309,7 +314,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
             u32x4 an[U][1];
             rb_load_x<NT, U, true>(b, xp, s, s1);
             rb_load_w<1, U>(an, wr, s + U, s1);
-            rb_multiply<NT, 1, U>(a, b, acc);
+            rb_multiply<NT, 1, U>(a, b, 0, acc);
 #pragma unroll
             for (int u = 0; u < U; u++) a[u][0] = an[u][0];
         }
@@ -319,7 +324,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
 }
 template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
 static int stream_form(hipStream_t st, const RbProduct& q, dim3 grid) {
-    constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * RbTokens<NT, rb_run(NT, MG)>::LDS * 2 : 0, SMEM = RED > STAGE ? RED : STAGE;
+    constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * RbTokens<NT, rb_deal(NT)>::LDS * 2 : 0, SMEM = RED > STAGE ? RED : STAGE;
     static_assert(SMEM <= 160 * 1024, "LDS");
     const auto kernel = rb_stream_kernel<NT, MG, GATED, NW, NORM, TURN, PARTS>;
     if constexpr (SMEM > 64 * 1024) {
@@ -355,9 +360,9 @@ static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
 }
 // How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
 // one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
-// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.6 11.3 12.1 14.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.8 8.7 10.5.
+// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.5 11.2 12.3 14.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.6 8.6 10.5.
 // More than that is bound by HBM while the rows are few: pairs of blocks, many workgroups that follow each other; else the least work for the busiest CU, by workgroups of four waves, several to a
-// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 23.0 23.9 26.3 28.8 (134 MB: 5.1 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 33.0 33.7 35.7 42.1.
+// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 23.0 23.5 26.0 28.8 (134 MB: 5.1 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 33.0 33.0 36.5 42.0.
 // The number of waves is part of a result's last bits (each adds up a part of k), and up to 32 rows stays what it was with the smaller workgroups: four waves also for 768 to 1024 blocks of one matrix, from 17 rows in pairs
 // (12288 x 2048 plain 10.1 11.4 14.4 19.5 -> 10.1 11.4 13.6 14.7; eight waves of three blocks: 10.0 11.0 11.9 15.0).
 static int stream_blocks(int units, int n, bool wide) {
