@@ -34,21 +34,14 @@ __device__ __forceinline__ void rb_load_w(u32x4 (&a)[U][MG], const uint16_t* con
             if (s + u < s_end) a[u][g] = ld_nt(reinterpret_cast<const u32x4*>(wr[g] + 512 * (s + u))); /* wave-uniform */
         }
 }
-// token fragments of the same steps; xp[t]: this lane's token row + its k octet (NULLABLE: NULL is a zero column), steps past s_end read step s_end - 1 against zero weights
-template <int NT, int U, bool NULLABLE>
+// token fragments of the same steps; xp[t]: this lane's token row + its k octet; steps past s_end read step s_end - 1 against zero weights
+template <int NT, int U>
 __device__ __forceinline__ void rb_load_x(u32x4 (&b)[U][NT], const uint16_t* const (&xp)[NT], int s, int s_end) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int st = s + u < s_end ? s + u : s_end - 1;
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            if (NULLABLE) {
-                b[u][t] = u32x4{0, 0, 0, 0};
-                if (xp[t]) b[u][t] = *reinterpret_cast<const u32x4*>(xp[t] + 32 * st);
-            } else {
-                b[u][t] = *reinterpret_cast<const u32x4*>(xp[t] + 32 * st);
-            }
-        }
+        for (int t = 0; t < NT; t++) b[u][t] = *reinterpret_cast<const u32x4*>(xp[t] + 32 * st);
     }
 }
 template <int NT, int MG, int U, int B>
@@ -60,8 +53,9 @@ __device__ __forceinline__ void rb_multiply(const u32x4 (&a)[U][MG], const u32x4
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[g][t] = rb_mfma16(a[u][g], b[first + u][t], acc[g][t]);
 }
-// the waves' partial tiles of the blocks from unit0 -> outputs; list: the columns are pairs; units: blocks past them repeat the last one.  GATED: a block is 8 gate rows and their 8 up rows
-template <int NT, int MG, int NW, bool GATED>
+// the waves' partial tiles of the blocks from unit0 -> outputs; list: the columns are pairs; units: blocks past them repeat the last one.  GATED: a block is 8 gate rows and their 8 up rows; WHOLE: two blocks,
+// 16 gate rows and their 16 up rows
+template <int NT, int MG, int NW, bool GATED, bool WHOLE = false>
 __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4 (&acc)[MG][NT], float (&red)[NW][MG][16 * NT][17], const int32_t* list, int unit0, int units, int tid, int part = 0) {
     const kf_rb_product& p = q.p;
     const int lane = tid & 63, wid = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
@@ -86,11 +80,11 @@ __device__ __forceinline__ void rb_stream_finish(const RbProduct& q, const f32x4
         }
         float d = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; w++) d += red[w][g][col][rg];
+        for (int w = 0; w < NW; w++) d += red[w][WHOLE ? 0 : g][col][WHOLE ? row : rg];
         if constexpr (GATED) {
             float u = 0.f;
 #pragma unroll
-            for (int w = 0; w < NW; w++) u += red[w][g][col][8 + rg];
+            for (int w = 0; w < NW; w++) u += red[w][WHOLE ? 1 : g][col][WHOLE ? row : 8 + rg];
             reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + m] = f2bf(scale * (rb_activate(p.act, d) * u));
         } else if (p.epilogue == KF_RB_STORE) {
             reinterpret_cast<uint16_t*>(p.y)[(size_t)yr * p.ldy + m] = f2bf(m >= p.act_lo && m < p.act_hi ? rb_activate(p.act, d) : d);
@@ -151,11 +145,11 @@ struct RbTokens {
 
 // TURN: the token rows go through RbTokens (rows in order, no experts); else every lane reads its fragments itself.  PARTS: blockIdx.y is a part of k (a form of its own: 1 % of a decode step of products
 // that have none)
-template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
+template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false, bool WHOLE = false, int U = rb_run(NT, MG)>
 __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
     const kf_rb_product& p = q.p;
-    constexpr int U = rb_run(NT, MG), DEAL = rb_deal(NT);
-    static_assert(DEAL % U == 0, "a deal is whole runs");
+    constexpr int DEAL = rb_deal(NT);
+    static_assert(DEAL % U == 0 && (!WHOLE || (GATED && MG == 2)), "a deal is whole runs; a gate block and its up block");
     static_assert(!(NORM && TURN), "normed fragments are made from the residual sum");
     using Tokens = RbTokens<NT, DEAL>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -175,7 +169,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
 #pragma unroll
     for (int g = 0; g < MG; g++) {
         const int unit = MG == 1 || unit0 + g < units ? unit0 + g : units - 1;
-        if (GATED) wr[g] = W + (size_t)(2 * (unit >> 1) + (r16 >> 3)) * 16 * p.k + 8 * (16 * q4 + 8 * (unit & 1) + (r16 & 7)); /* half of the gate's tile, half of the up rows': whole lines of both */
+        if (GATED && !WHOLE) wr[g] = W + (size_t)(2 * (unit >> 1) + (r16 >> 3)) * 16 * p.k + 8 * (16 * q4 + 8 * (unit & 1) + (r16 & 7)); /* half of the gate's tile, half of the up rows': whole lines of both */
         else wr[g] = W + (size_t)unit * 16 * p.k + 8 * lane;
     }
     u32x4 a[U][MG], b[TURN ? DEAL : U][NT];
@@ -252,7 +246,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
                     }
                 }
             } else {
-                if constexpr (!TURN) rb_load_x<NT, U, false>(b, xp, s0, nstep);
+                if constexpr (!TURN) rb_load_x<NT, U>(b, xp, s0, nstep);
                 rb_load_w<MG, U>(an, wr, s1, nstep);
             }
             rb_multiply<NT, MG, U>(a, b, TURN ? run : 0, acc);
@@ -263,7 +257,7 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_kernel(const RbProduct q) {
         }
     }
     if constexpr (TURN) __syncthreads(); /* the token rows make way */
-    rb_stream_finish<NT, MG, NW, GATED>(q, acc, red, list, unit0, units, tid, part);
+    rb_stream_finish<NT, MG, NW, GATED, WHOLE>(q, acc, red, list, unit0, units, tid, part);
 }
 
 // RESIDUAL with the rows' experts summed: (chosen expert, k-step) pairs as one list, cut evenly over the waves
@@ -298,35 +292,49 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
     while (at < end) { /* an expert's part of this wave's range (wave-uniform) */
         const int i = at / nstep, s0 = at - i * nstep, s1 = s0 + (end - at) < nstep ? s0 + (end - at) : nstep;
         const int ex = s_ex[i];
-        const uint16_t* const wr[1] = {reinterpret_cast<const uint16_t*>(p.w) + (size_t)ex * q.e.w_stride + (size_t)m0 * p.k + 8 * lane};
-        u32x4 a[U][1], b[U][NT];
-        rb_load_w<1, U>(a, wr, s0, s1);
+        const uint16_t* wr = reinterpret_cast<const uint16_t*>(p.w) + (size_t)ex * q.e.w_stride + (size_t)m0 * p.k + 8 * lane;
+        // every load is unconditional and no run is copied from one set of registers to another: either makes the wave wait for what it has just asked for.  Past the range its last step is read again, and columns of
+        // another expert read row 0, both against zeros.  us per call of four tokens, 2048 wide, 64 experts, 1, 4, 8, 14, 32 sequences: 2565 4089 5414 6853 9913 -> 2469 3723 4769 5965 8399
         const uint16_t* xp[NT];
+        bool on[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const int row = t * 16 + r16;
-            xp[t] = nullptr;
+            xp[t] = X + 8 * q4, on[t] = false;
             if (row < p.n)
                 for (int j = 0; j < q.e.top; j++)
-                    if (s_ids[row * q.e.top + j] == ex) xp[t] = X + (size_t)(row * q.e.top + j) * p.ldx + 8 * q4;
+                    if (s_ids[row * q.e.top + j] == ex) xp[t] = X + (size_t)(row * q.e.top + j) * p.ldx + 8 * q4, on[t] = true;
         }
-        for (int s = s0; s < s1; s += U) {
-            u32x4 an[U][1];
-            rb_load_x<NT, U, true>(b, xp, s, s1);
-            rb_load_w<1, U>(an, wr, s + U, s1);
-            rb_multiply<NT, 1, U>(a, b, 0, acc);
+        auto weights = [&](u32x4 (&w)[U][1], int s) {
 #pragma unroll
-            for (int u = 0; u < U; u++) a[u][0] = an[u][0];
+            for (int u = 0; u < U; u++) w[u][0] = ld_nt(reinterpret_cast<const u32x4*>(wr + 512 * (s + u < s1 ? s + u : s1 - 1)));
+        };
+        auto run = [&](const u32x4 (&w)[U][1], u32x4 (&next)[U][1], int s) {
+            u32x4 b[U][NT];
+            rb_load_x<NT, U>(b, xp, s, s1);
+            weights(next, s + U);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    if (!(on[t] && s + u < s1)) b[u][t] = u32x4{0, 0, 0, 0};
+            rb_multiply<NT, 1, U>(w, b, 0, acc);
+        };
+        u32x4 w0[U][1], w1[U][1];
+        weights(w0, s0);
+        for (int s = s0; s < s1; s += 2 * U) {
+            run(w0, w1, s);
+            if (s + U < s1) run(w1, w0, s + U);
         }
         at += s1 - s0;
     }
     rb_stream_finish<NT, 1, NW, false>(q, acc, red, nullptr, blockIdx.x, p.m / 16, tid);
 }
-template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false>
+template <int NT, int MG, bool GATED, int NW, bool NORM, bool TURN, bool PARTS = false, bool WHOLE = false, int U = rb_run(NT, MG)>
 static int stream_form(hipStream_t st, const RbProduct& q, dim3 grid) {
     constexpr int RED = NW * MG * 16 * NT * 17 * 4, STAGE = TURN ? NW * RbTokens<NT, rb_deal(NT)>::LDS * 2 : 0, SMEM = RED > STAGE ? RED : STAGE;
     static_assert(SMEM <= 160 * 1024, "LDS");
-    const auto kernel = rb_stream_kernel<NT, MG, GATED, NW, NORM, TURN, PARTS>;
+    const auto kernel = rb_stream_kernel<NT, MG, GATED, NW, NORM, TURN, PARTS, WHOLE, U>;
     if constexpr (SMEM > 64 * 1024) {
         static bool done = false;
         if (!done && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) return KF_HIP_CHECK;
@@ -354,7 +362,7 @@ static int stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
 template <int NT, int NW>
 static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     if (q.p.mode == KF_RB_SUM) hipLaunchKernelGGL((rb_stream_sum_kernel<NT, NW>), grid, dim3(64 * NW), 0, st, q);
-    else if (q.p.epilogue == KF_RB_GATED) return stream_form<NT, 2, true, NW, false, false>(st, q, grid);
+    else if (q.p.epilogue == KF_RB_GATED) return stream_form<NT, 2, true, NW, false, false, false, true, rb_deal(NT)>(st, q, grid);
     else return stream_form<NT, 1, false, NW, false, false>(st, q, grid);
     return KF_OK;
 }
