@@ -89,7 +89,7 @@ template <int FMT_, int GQ_, int HD_, int NWV_, int DIM_, int QD_, int KVD_, int
 struct XCfg {
     // NB: sequences per decoder.  The decoders of a launch unpack the SAME 4-bit blocks; with NB > 1 a decoder multiplies every unpacked block against the
     // activations of NB sequences (xcc + 8 b, b = 0 .. NB - 1) staged side by side in LDS -- the exact bf16-stepwise unpack (7 vector instructions per weight with its
-    // bookkeeping) is paid once, each sequence adds its half-instruction per weight (v_pk_fma_f32) and keeps its own canonical chain, lane tree and rounding: every id, logit
+    // bookkeeping) is paid once, each sequence adds its chains' products (4-bit: on the matrix cores, MF below) and keeps its own canonical chain, lane tree and rounding: every id, logit
     // and K / V row of every sequence stays bit for bit what the sequence alone produces.  Hand-offs carry NB vectors (one wait, NB sweeps), the attention, the K / V caches
     // and the decode state stay per sequence, the head's bf16 rows are read once for the NB sequences.
     static constexpr int NB = NB_;
@@ -463,7 +463,7 @@ __device__ __forceinline__ f32x2_t xe_block(u32x4 w, uint16_t st16, uint16_t ze1
     return acc;
 }
 // Storages without a register-table form (1-bit): the block's 16 bf16 pair words by BlockPrep<FMT> (kf_gemv_blocks.h: the words kf_engine.hip multiplies), widened ONCE to the
-// fp32 operand pairs, then every sequence's chain pair takes its sixteen v_pk_fma_f32 -- pairs_dot<true>'s products, element after element
+// fp32 operand pairs, then every sequence's chain pair takes its sixteen pairs of fused multiply-adds -- pairs_dot<true>'s products, element after element
 template <int FMT, int XS, int NB, size_t SEQB>
 __device__ __forceinline__ void xe_block_prep_nb(u32x4 w, uint16_t st16, uint16_t ze16, float qb, const f32x4* xc0, int lane, const u32x4* tab, f32x2_t (&acc)[NB]) {
     const float step = bf2f(st16), zero = bf2f(ze16), nb = -(qb * step);
@@ -487,7 +487,7 @@ __device__ __forceinline__ void xe_block_prep_nb(u32x4 w, uint16_t st16, uint16_
     }
 }
 // The same block against the activations of NB sequences (XCfg::NB > 1): the group's table and the block's 32 weights are formed ONCE (the byte-plane lookups and the fp32
-// assembly of perm_fma_dword), then every sequence's chain pair takes its sixteen v_pk_fma_f32 -- element after element of the block, as xe_block does for one sequence
+// assembly of perm_fma_dword), then every sequence's chain pair takes its sixteen pairs of fused multiply-adds -- element after element of the block, as xe_block does for one sequence
 template <int XS, int NB, size_t SEQB>
 __device__ __forceinline__ void xe_block_nb(u32x4 w, uint16_t st16, uint16_t ze16, float qb, const f32x4* xc0, int lane, f32x2_t (&acc)[NB]) {
     const float step = bf2f(st16), zero = bf2f(ze16), nb = -(qb * step);
