@@ -368,11 +368,11 @@ static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
 }
 // How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
 // one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
-// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.5 11.2 12.3 14.0; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.6 8.6 10.5.
+// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.5 11.2 12.3 17.2; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.6 8.6 12.5.
 // More than that is bound by HBM while the rows are few: pairs of blocks, many workgroups that follow each other; else the least work for the busiest CU, by workgroups of four waves, several to a
 // CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 23.0 23.5 26.0 28.8 (134 MB: 5.1 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 33.0 33.0 36.5 42.0.
-// The number of waves is part of a result's last bits (each adds up a part of k), and up to 32 rows stays what it was with the smaller workgroups: four waves also behind a norm where gated, and for 768 to 1024 blocks of one matrix, from 17 rows in pairs
-// (12288 x 2048 plain 10.1 11.4 14.4 19.5 -> 10.1 11.4 13.6 14.7; eight waves of three blocks: 10.0 11.0 11.9 15.0).
+// The number of waves is part of a result's last bits (each adds up a part of k) and stays what it was with the smaller workgroups: four waves for more than 32 rows, behind a norm where gated, and for 768 to 1024 blocks of one matrix, from 17 rows in pairs
+// (12288 x 2048 plain 10.1 11.4 14.4 19.5 -> 10.1 11.4 13.6 17.4; eight waves of three blocks: 10.0 11.0 11.9 15.0).
 static int stream_blocks(int units, int n, bool wide) {
     if (units <= 1024) return wide ? (units + 255) / 256 : n > 16 ? 2 : 1;
     int best = 2;
@@ -391,11 +391,11 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     if (p.mode == KF_RB_SUM && ((long)p.n * q.e.top > KF_RB_SUM_PAIRS || q.e.tile < p.n)) return 1;
     const bool gated = p.epilogue == KF_RB_GATED;
     const long small = (long)units / (gated ? 2 : 1) * (tiles ? q.e.n_tile : p.parts > 1 ? p.parts : 1); /* workgroups of 16 rows, of 16 gates and 16 ups */
-    const bool wide = p.k >= 512 && !(p.norm_z && gated) && (all && p.n > 32 ? units <= 1024 : small < 768);                        /* few workgroups: more waves each, more loads in flight per CU */
+    const bool wide = p.k >= 512 && nt <= 2 && !(p.norm_z && gated) && small < 768;                        /* few workgroups: more waves each, more loads in flight per CU */
     const int mg = !all ? (gated ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n, wide);
     const dim3 grid((units + mg - 1) / mg, tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
 #define RB_STREAM_MG(nt, nw) (mg == 1 ? stream_go<nt, 1, nw>(st, q, grid) : mg == 2 ? stream_go<nt, 2, nw>(st, q, grid) : mg == 3 ? stream_go<nt, 3, nw>(st, q, grid) : stream_go<nt, 4, nw>(st, q, grid))
-#define RB_STREAM(nt) (!all ? (wide && nt <= 2 ? expert_go<nt, 8>(st, q, grid) : expert_go<nt, 4>(st, q, grid)) : wide ? RB_STREAM_MG(nt, 8) : RB_STREAM_MG(nt, 4))
+#define RB_STREAM(nt) (!all ? (wide ? expert_go<nt, 8>(st, q, grid) : expert_go<nt, 4>(st, q, grid)) : wide ? RB_STREAM_MG(nt, 8) : RB_STREAM_MG(nt, 4))
     return nt == 1 ? RB_STREAM(1) : nt == 2 ? RB_STREAM(2) : nt == 3 ? RB_STREAM(3) : RB_STREAM(4);
 #undef RB_STREAM
 #undef RB_STREAM_MG
