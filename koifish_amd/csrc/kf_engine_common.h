@@ -49,6 +49,8 @@ constexpr int pow2_ceil(int v) {
     return p;
 }
 
+// A raw buffer of `bytes`.  A load's scalar offset is part of the hardware's bounds check here (1 KiB, scalar offset 512: the upper 32 of 64 lanes read zeros; 1024 and more, or no bytes at all: every lane); the
+// compiler's description of the builtin leaves it out, so an address that only the scalar offset carries past the end is better not formed.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t eng_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }

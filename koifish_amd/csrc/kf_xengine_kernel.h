@@ -1492,16 +1492,16 @@ __device__ __forceinline__ void xe_head_main(const XArgs& a, const XLds& L, cons
     u32x4 w[2][C::MFH ? 4 : HG][ITERS];
     auto issue = [&](int b, int buf) {
         if constexpr (C::MFH) { /* four rows, each ITERS KiB: the lane's 16 bytes beside its neighbours' */
-            const int i = b < nmine ? b : (nmine > 0 ? nmine - 1 : 0), row0 = (s_wg + wave + NWV * i) * 4;
+            const int i = b < nmine ? b : (nmine > 0 ? nmine - 1 : 0), slot0 = (s_wg + wave + NWV * i) * 4, row0 = slot0 < vocab ? slot0 : vocab - 1;
             const unsigned long long at = (unsigned long long)(uintptr_t)(head_w + (size_t)row0 * nBlk);
             const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at), hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
-            const int rows = __builtin_amdgcn_readfirstlane(vocab - row0 < 4 ? vocab - row0 : 4); /* rows past the last one: zeros */
-            const __amdgpu_buffer_rsrc_t rs = eng_rsrc((const void*)(uintptr_t)(((unsigned long long)hi << 32) | lo), (uint32_t)(rows > 0 ? rows : 0) * (uint32_t)(nBlk * 16));
+            const int last = __builtin_amdgcn_readfirstlane(vocab - row0 < 4 ? vocab - row0 - 1 : 3); /* the head's last row once more in the place of rows past it: `compute` stores none of them */
+            const __amdgpu_buffer_rsrc_t rs = eng_rsrc((const void*)(uintptr_t)(((unsigned long long)hi << 32) | lo), 4u * (uint32_t)(nBlk * 16));
             const int ln = fresh_lane();
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int it = 0; it < ITERS; it++) w[buf][r][it] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, ln * 16, r * (nBlk * 16) + it * 1024, 0));
+                for (int it = 0; it < ITERS; it++) w[buf][r][it] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, ln * 16, (r < last ? r : last) * (nBlk * 16) + it * 1024, 0));
             return;
         }
 #pragma unroll

@@ -96,6 +96,29 @@ def test_every_sequence_equals_the_oracle(canon, cfg_name, max_seq, n_steps, n_s
     m.close()
 
 
+@pytest.mark.parametrize("n_seq,vocab", [(16, 4093), (32, 4094), (16, 4095), (32, 131)])
+def test_head_rows_that_are_no_multiple_of_four(canon, n_seq, vocab):
+    """the batched decoders' head takes rows by fours: one, two and three rows in the last four, waves and whole workgroups without any (33 fours on 32 workgroups) -- ids and logits against the oracle"""
+    cfg, n = dict(synth.CONFIGS["small"], vocab=vocab, max_seq=32), 8
+    raw = synth.raw_weights_numpy(cfg, 97, w_std=0.1)
+    m = synth.build_from_raw(cfg, raw, L.Q4, L.BF16)
+    m.set_canonical(True)
+    xr = XcdReplicas(m, n_seq)
+    forced = np.full((n_seq, cfg["max_seq"]), -1, dtype=np.int32)
+    for s in range(n_seq):
+        forced[s, :4] = prompt_ids(cfg, 4, seed=30 + s)
+        xr.set_forced(s, forced[s])
+        xr.set_state(s, int(forced[s, 0]), 0)
+    xr.run_steps(n)
+    m.sync()
+    xr.check()
+    for s in (0, 5, 9, n_seq - 1):
+        o_ids, o_logits, _, _ = _oracle_run(cfg, raw, forced[s], n)
+        assert xr.tokens_out(s, n).tolist() == o_ids and np.array_equal(xr.logits(s), o_logits), "sequence %d" % s
+    xr.close()
+    m.close()
+
+
 @pytest.mark.parametrize("layer_type,cfg_name,max_seq,n_steps,n_seq,check", [
     (L.BOOL1, "tiny", 200, 150, 8, None), (L.BOOL1, "small", 320, 100, 16, (0, 5, 9, 14)), (L.BOOL1, "small", 320, 100, 32, (0, 7, 13, 18, 24, 31)), (L.BOOL1, "tiny", 200, 150, 27, (1, 6, 10, 15, 19, 24)),
     (L.T_SIGN, "tiny", 200, 150, 8, None), (L.T_SIGN, "small", 320, 100, 32, (0, 7, 13, 18, 24, 31)), (L.T_SIGN, "tiny", 200, 100, 11, None)])
