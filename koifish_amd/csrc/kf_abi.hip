@@ -1513,7 +1513,10 @@ int kfdbg_set_knob(const char* name, long value) {
     else if (!strcmp(name, "gemm_min")) k.gemm_min = (int)value;
     else if (!strcmp(name, "g3_first")) k.g3_first = (int)value;
     else if (!strcmp(name, "g3_wide")) k.g3_wide = (int)value;
-    else if (!strcmp(name, "attn_gq_split")) k.attn_gq_split = (int)value;
+    else if (!strcmp(name, "attn_gq_split")) {
+        if (value != 0 && value != 2 && value != 4 && value != 8) return -1; /* attn_launch has kernels for these and no others */
+        k.attn_gq_split = (int)value;
+    }
     else if (!strcmp(name, "resident_min")) k.resident_min = (int)value;
     else if (!strcmp(name, "attn_pair_min")) k.attn_pair_min = (int)value;
     else if (!strcmp(name, "attn_walk_min")) k.attn_walk_min = (int)value;

@@ -108,3 +108,14 @@ def test_kf_weight_struct_matches_the_ctypes_mirror(tmp_path):
     nums = [int(x) for x in subprocess.check_output([str(exe)]).decode().split()]
     assert nums[:-1] == [getattr(L.Weight, f).offset for f in fields]
     assert nums[-1] == C.sizeof(L.Weight)
+
+
+def test_the_attention_knob_takes_its_forms_and_no_others():
+    """kfdbg_set_knob("attn_gq_split"): the workgroups per kv-head that attn_launch has a kernel for; the value divides a GQA-8 model's heads, so anything else would address heads that do not exist"""
+    from koifish_amd import lib as L
+    hip, _ = L.load()
+    hip.kfdbg_set_knob.argtypes = [C.c_char_p, C.c_long]
+    for bad in (-8, -1, 1, 3, 5, 6, 7, 9, 16):
+        assert hip.kfdbg_set_knob(b"attn_gq_split", bad) == -1, bad
+    for good in (2, 4, 8, 0):
+        assert hip.kfdbg_set_knob(b"attn_gq_split", good) == 0, good
