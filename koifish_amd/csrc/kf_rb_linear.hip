@@ -293,8 +293,8 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
         const int i = at / nstep, s0 = at - i * nstep, s1 = s0 + (end - at) < nstep ? s0 + (end - at) : nstep;
         const int ex = s_ex[i];
         const uint16_t* wr = reinterpret_cast<const uint16_t*>(p.w) + (size_t)ex * q.e.w_stride + (size_t)m0 * p.k + 8 * lane;
-        // every load is unconditional and no run is copied from one set of registers to another: either makes the wave wait for what it has just asked for.  Past the range its last step is read again, and columns of
-        // another expert read row 0, both against zeros.  us per call of four tokens, 2048 wide, 64 experts, 1, 4, 8, 14, 32 sequences: 2565 4089 5414 6853 9913 -> 2469 3723 4769 5965 8399
+        // every load is unconditional and no run is copied from one set of registers to another: either makes the wave wait for what it has just asked for.  Past the range its last step is read again and columns of
+        // another expert read row 0, and zeros are multiplied instead.  us per call of four tokens, 2048 wide, 64 experts, 1, 4, 8, 14, 32 sequences: 2565 4089 5414 6853 9913 -> 2469 3723 4769 5965 8399
         const uint16_t* xp[NT];
         bool on[NT];
 #pragma unroll
@@ -309,15 +309,17 @@ __global__ void __launch_bounds__(64 * NW) rb_stream_sum_kernel(const RbProduct 
 #pragma unroll
             for (int u = 0; u < U; u++) w[u][0] = ld_nt(reinterpret_cast<const u32x4*>(wr + 512 * (s + u < s1 ? s + u : s1 - 1)));
         };
-        auto run = [&](const u32x4 (&w)[U][1], u32x4 (&next)[U][1], int s) {
+        auto run = [&](u32x4 (&w)[U][1], u32x4 (&next)[U][1], int s) {
             u32x4 b[U][NT];
             rb_load_x<NT, U>(b, xp, s, s1);
             weights(next, s + U);
 #pragma unroll
-            for (int u = 0; u < U; u++)
+            for (int u = 0; u < U; u++) {
+                if (s + u >= s1) w[u][0] = u32x4{0, 0, 0, 0}; /* (both factors: the other one may be an infinity) */
 #pragma unroll
                 for (int t = 0; t < NT; t++)
                     if (!(on[t] && s + u < s1)) b[u][t] = u32x4{0, 0, 0, 0};
+            }
             rb_multiply<NT, 1, U>(w, b, 0, acc);
         };
         u32x4 w0[U][1], w1[U][1];

@@ -276,6 +276,26 @@ def test_experts(ctx, kind, n, E, top, tile):
         assert rc == 0 and np.abs(f64(z) - (1.25 * f64(res) + y.reshape(n, top, C_).sum(1))).max() < 2e-5
 
 
+@pytest.mark.parametrize("n", [1, 20])  # one block of columns, two
+@pytest.mark.parametrize("at", [63, 191])  # the last k of a wave's two steps (it multiplies in fours), the last of all
+@pytest.mark.parametrize("what", ["weight", "token"])
+def test_infinities_in_the_sum_of_experts(ctx, what, at, n):
+    """an infinite weight or activation makes its own products infinite and no others: steps past a wave's range add nothing"""
+    C_, ff, g = 64, 192, torch.Generator().manual_seed(at)
+    dn, act, res = torch.randn(1, C_, ff, generator=g), torch.randn(n, ff, generator=g), torch.randn(n, C_, generator=g)
+    (dn[0, 3] if what == "weight" else act[0])[at] = float("inf")
+    dn, act, res = dev(dn, torch.bfloat16), dev(act, torch.bfloat16), dev(res)
+    e, b = route(ctx, pad(dev(torch.zeros(n, 1)), n, up(1)), None, n, 1, 1, 16 if n <= 16 else 32, L.BF16, w_stride=C_ * ff)
+    dns, z = stored(dn), torch.zeros(n, C_, device="cuda")
+    p = L.RbProduct(dns.data_ptr(), act.data_ptr(), z.data_ptr(), res.data_ptr(), ff, C_, C_, L.BF16, C_, ff, n, L.RB_RESIDUAL, 0, L.RB_SUM, 1.0, C.pointer(e))
+    L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+    want = f64(res) + f64(act) @ f64(dn)[0].T
+    got = f64(z)
+    assert np.isinf(want).any() and np.array_equal(np.isinf(want), np.isinf(got)) and np.array_equal(want[np.isinf(want)], got[np.isinf(want)])
+    fin = np.isfinite(want)
+    assert (np.abs(got[fin] - want[fin]) < 1.5e-3).all()  # 192 additions in float32: at most 192 2^-24 of the sum of magnitudes, about 125
+
+
 # ---- attention
 def mix(H, G, D, chunk, rot, scale=None):
     return {"heads": H, "kv_heads": G, "dim": D, "mask": {"size": chunk} if chunk else None, "scale": D ** -0.5 if scale is None else scale,
