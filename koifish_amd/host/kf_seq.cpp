@@ -600,21 +600,6 @@ int SeqFish::Spans(SeqSlots& s, const SeqSpan* spans, int n_span, const int32_t*
         KF_TRY(Upload(ctx, pre.seqs->data, seqs));
         KF_TRY(kf_rb_embed(ctx, card.type, table->data, card.vocab, card.width, Width(card.width), I(pre.tok), rows, F(pre.x), P(pre.h)));
         KF_TRY(Layers(pre, s.kv, RowBatch{rows, (int)part.size(), max_n, 0}));
-        // the spans that end in this pass: their last rows' logits go into the slots', the greedy pick
-        std::vector<int32_t> end_rows, end_meta;
-        if (last)
-            for (int i : part)
-                if (done[i] == spans[i].n) {
-                    const int32_t m[4] = {spans[i].pos0 + spans[i].n - 1, spans[i].slot, 0, 0};
-                    end_rows.push_back(row0[i] + done[i] - from[i] - 1), end_meta.insert(end_meta.end(), m, m + 4);
-                }
-        auto pick = [&]() {
-            int32_t* d_meta = I(pre.want) + up(pre.head_rows, 4);
-            const int n = (int)end_rows.size();
-            KF_TRY(Upload(ctx, d_meta, end_meta));
-            KF_TRY(kf_rb_slot_logits(ctx, F(pre.logits), V, n, d_meta, F(s.dec.logits), s.d_state));
-            return kf_rb_pick(ctx, F(pre.logits), V, card.vocab, n, d_meta, s.d_state, s.d_tokens_out, card.n_ctx, s.pick_ws->data);
-        };
         // logits asked for, a block of rows at a time
         std::vector<int32_t> list, at;
         for (int i = 0; i < n_want; i++) {
@@ -626,10 +611,6 @@ int SeqFish::Spans(SeqSlots& s, const SeqSpan* spans, int n_span, const int32_t*
             const int n = (int)std::min<size_t>(block, list.size() - b);
             KF_TRY(Ensure(pre, rows, n_span, n, false));
             KF_TRY(HeadRows(pre, list.data() + b, n));
-            if (!end_rows.empty() && list == end_rows && n == (int)list.size()) { /* the rows asked for are the last ones: their logits are here already */
-                KF_TRY(pick());
-                end_rows.clear();
-            }
             bool whole = V == card.vocab; /* the rows lie in `out` as they do here */
             for (int j = 1; j < n; j++) whole = whole && at[b + j] == at[b] + j;
             if (whole) {
@@ -640,10 +621,21 @@ int SeqFish::Spans(SeqSlots& s, const SeqSpan* spans, int n_span, const int32_t*
             KF_TRY(kf_d2h(ctx, lg.data(), pre.logits->data, lg.size() * 4));
             for (int j = 0; j < n; j++) std::memcpy(out + (size_t)at[b + j] * card.vocab, lg.data() + (size_t)j * V, (size_t)card.vocab * 4);
         }
-        if (!end_rows.empty()) {
-            KF_TRY(Ensure(pre, rows, n_span, (int)end_rows.size(), false));
-            KF_TRY(HeadRows(pre, end_rows.data(), (int)end_rows.size()));
-            KF_TRY(pick());
+        if (!last) continue;
+        // the spans that end in this pass: their last rows' logits into the slots', the greedy pick
+        std::vector<int32_t> end_rows, end_meta;
+        for (int i : part)
+            if (done[i] == spans[i].n) {
+                const int32_t m[4] = {spans[i].pos0 + spans[i].n - 1, spans[i].slot, 0, 0};
+                end_rows.push_back(row0[i] + done[i] - from[i] - 1), end_meta.insert(end_meta.end(), m, m + 4);
+            }
+        if (const int n = (int)end_rows.size()) {
+            KF_TRY(Ensure(pre, rows, n_span, n, false));
+            KF_TRY(HeadRows(pre, end_rows.data(), n));
+            int32_t* d_meta = I(pre.want) + up(pre.head_rows, 4);
+            KF_TRY(Upload(ctx, d_meta, end_meta));
+            KF_TRY(kf_rb_slot_logits(ctx, F(pre.logits), V, n, d_meta, F(s.dec.logits), s.d_state));
+            KF_TRY(kf_rb_pick(ctx, F(pre.logits), V, card.vocab, n, d_meta, s.d_state, s.d_tokens_out, card.n_ctx, s.pick_ws->data));
         }
     }
     for (int i = 0; i < n_span; i++) s.pos[spans[i].slot] = spans[i].pos0 + spans[i].n;
