@@ -351,14 +351,25 @@ static int stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     // whole lines for more than 8 rows in order: below, a fragment's 16 half lines are few distinct ones and the way round costs more than it saves (one token of a 2048-wide model: 1.79 -> 1.87 ms
     // over four steps; 6 rows 2.04 -> 2.08; 14 rows 2.42 -> 2.35; 32 rows 4.62 -> 4.23)
     const bool turn = p.n > 8 && p.ldx <= (1 << 24), gated = p.epilogue == KF_RB_GATED;
-    if constexpr (NT == 1) {
-        if (p.norm_z) return gated ? stream_form<1, MG, true, NW, true, false>(st, q, grid) : stream_form<1, MG, false, NW, true, false>(st, q, grid);
+    // what stream_blocks gives: four waves take one block or two of up to 16 rows and two to four of more; eight take four only where gated; a norm goes in front of gated products of four waves and of any plain ones
+    constexpr bool GATED = NW == 8 || (NT == 1 ? MG <= 2 : MG >= 2), PLAIN = GATED && !(NW == 8 && MG == 4);
+    if constexpr (NT == 1 && GATED && NW == 4) {
+        if (p.norm_z && gated) return stream_form<1, MG, true, 4, true, false>(st, q, grid);
     }
+    if constexpr (NT == 1 && PLAIN) {
+        if (p.norm_z && !gated) return stream_form<1, MG, false, NW, true, false>(st, q, grid);
+    }
+    if (p.norm_z) return KF_INTERNAL_ERR;
     if constexpr (MG == 1) {
         if (p.parts > 1) return turn ? stream_form<NT, 1, false, NW, false, true, true>(st, q, grid) : stream_form<NT, 1, false, NW, false, false, true>(st, q, grid);
     }
-    if (gated) return turn ? stream_form<NT, MG, true, NW, false, true>(st, q, grid) : stream_form<NT, MG, true, NW, false, false>(st, q, grid);
-    return turn ? stream_form<NT, MG, false, NW, false, true>(st, q, grid) : stream_form<NT, MG, false, NW, false, false>(st, q, grid);
+    if constexpr (GATED) {
+        if (gated) return turn ? stream_form<NT, MG, true, NW, false, true>(st, q, grid) : stream_form<NT, MG, true, NW, false, false>(st, q, grid);
+    }
+    if constexpr (PLAIN) {
+        if (!gated) return turn ? stream_form<NT, MG, false, NW, false, true>(st, q, grid) : stream_form<NT, MG, false, NW, false, false>(st, q, grid);
+    }
+    return KF_INTERNAL_ERR;
 }
 // experts: one gate block and its up rows a workgroup; the tiles are mostly padding, which repeats row 0, and the way round by LDS does not pay (32 rows of 64 experts: 10.15 -> 10.36 ms)
 template <int NT, int NW>
@@ -367,6 +378,11 @@ static int expert_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     else if (q.p.epilogue == KF_RB_GATED) return stream_form<NT, 2, true, NW, false, false, false, true, rb_deal(NT)>(st, q, grid);
     else return stream_form<NT, 1, false, NW, false, false>(st, q, grid);
     return KF_OK;
+}
+template <int NT, int NW>
+static int stream_any(hipStream_t st, const RbProduct& q, dim3 grid, int mg) {
+    if (q.p.mode != KF_RB_ALL) return expert_go<NT, NW>(st, q, grid);
+    return mg == 1 ? stream_go<NT, 1, NW>(st, q, grid) : mg == 2 ? stream_go<NT, 2, NW>(st, q, grid) : mg == 3 ? stream_go<NT, 3, NW>(st, q, grid) : stream_go<NT, 4, NW>(st, q, grid);
 }
 // How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
 // one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
@@ -396,11 +412,8 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const bool wide = p.k >= 512 && nt <= 2 && !(p.norm_z && gated) && small < 768;                        /* few workgroups: more waves each, more loads in flight per CU */
     const int mg = !all ? (gated ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n, wide);
     const dim3 grid((units + mg - 1) / mg, tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
-#define RB_STREAM_MG(nt, nw) (mg == 1 ? stream_go<nt, 1, nw>(st, q, grid) : mg == 2 ? stream_go<nt, 2, nw>(st, q, grid) : mg == 3 ? stream_go<nt, 3, nw>(st, q, grid) : stream_go<nt, 4, nw>(st, q, grid))
-#define RB_STREAM(nt) (!all ? (wide ? expert_go<nt, 8>(st, q, grid) : expert_go<nt, 4>(st, q, grid)) : wide ? RB_STREAM_MG(nt, 8) : RB_STREAM_MG(nt, 4))
-    return nt == 1 ? RB_STREAM(1) : nt == 2 ? RB_STREAM(2) : nt == 3 ? RB_STREAM(3) : RB_STREAM(4);
-#undef RB_STREAM
-#undef RB_STREAM_MG
+    if (nt > 2) return nt == 3 ? stream_any<3, 4>(st, q, grid, mg) : stream_any<4, 4>(st, q, grid, mg);
+    return nt == 1 ? (wide ? stream_any<1, 8>(st, q, grid, mg) : stream_any<1, 4>(st, q, grid, mg)) : (wide ? stream_any<2, 8>(st, q, grid, mg) : stream_any<2, 4>(st, q, grid, mg));
 }
 
 }  // namespace kf
