@@ -1500,6 +1500,12 @@ int kfdbg_engine_set_delays(kf_engine* e, const int* d6) {
     kf::engine_set_delays(e->h, d6);
     return 0;
 }
+// the matrix instruction of the batched decoders on given operands (kf_device.h mx_fma): `waves` x 64 lanes, acc and out 16-byte aligned
+int kfdbg_mx_fma(kf_ctx* c, const float* row, const float* col, const float* acc, float* out, int waves) {
+    CHKCTX(c);
+    if (!row || !col || !acc || !out || !al16(acc) || !al16(out) || waves < 1) return fail(KF_INVALID_ARGS, "kfdbg_mx_fma: bad arguments");
+    RET(kf::mx_fma_launch(c->stream, row, col, acc, out, waves));
+}
 // development knobs (kf::Knobs): a kernel form against the form it replaces, inside one process
 int kfdbg_set_knob(const char* name, long value) {
     if (!name) return -1;

@@ -249,6 +249,7 @@ int awq_dequant_launch(hipStream_t st, const kf_weight* w, uint16_t* out);
 
 int set_state_launch(hipStream_t st, int32_t* d_state, int token, int pos);
 int set_slot_state_launch(hipStream_t st, int32_t* d_state, int token, int pos);
+int mx_fma_launch(hipStream_t st, const float* row, const float* col, const float* acc, float* out, int waves);
 int put_words_launch(hipStream_t st, int32_t* dst, const int32_t* h_src, int count);
 int hot_rows_launch(hipStream_t st, const int32_t* hot, int n, int32_t* rows, int32_t* count);
 int cold_fill_launch(hipStream_t st, uint16_t* y, const uint16_t* bias, int n);

@@ -1087,6 +1087,16 @@ int put_words_launch(hipStream_t st, int32_t* dst, const int32_t* h_src, int cou
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 
+// mx_fma on given operands: lane l of wave b brings row[64 b + l], col[64 b + l] and acc[4 (64 b + l) ..]; its four sums to the same place of out
+__global__ void __launch_bounds__(64) mx_fma_kernel(const float* row, const float* col, const f32x4_t* acc, f32x4_t* out) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    out[i] = mx_fma(row[i], col[i], acc[i]);
+}
+int mx_fma_launch(hipStream_t st, const float* row, const float* col, const float* acc, float* out, int waves) {
+    hipLaunchKernelGGL(mx_fma_kernel, dim3(waves), dim3(64), 0, st, row, col, reinterpret_cast<const f32x4_t*>(acc), reinterpret_cast<f32x4_t*>(out));
+    return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
+}
+
 // ---- hot-row lists for the sparse forward (CS_Picker's `hot` array, SparseNeuron.cpp:20-29; D_matmul_sparse, GST_float.cpp:306-318)
 // rows[0 .. count) = the indices i with hot[i] == 1, ascending; one workgroup walks the mask in chunks of 1024 with a ballot-ordered compaction
 __global__ void __launch_bounds__(1024) hot_rows_kernel(const int32_t* hot, int n, int32_t* rows, int32_t* count) {

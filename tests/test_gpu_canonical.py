@@ -33,6 +33,42 @@ def cctx(ctx):
     ctx.set_canonical(False)
 
 
+def test_the_matrix_instruction_is_fmaf(ctx):
+    """kf_device.h mx_fma: register r of lane 4 b + j = fmaf(lane 4 b + r's row operand, lane 4 b + j's column operand, its own sum) -- against the C library's fmaf bit for bit (NaN as NaN): ordinary values, subnormal
+    operands, products and sums, results on both sides of the smallest normal and the largest number, halfway cases, signed zeros, infinities"""
+    import ctypes as C
+    import ctypes.util
+    waves, rng = 96, np.random.default_rng(12)
+    bits = lambda lo, hi, n: (rng.integers(lo, hi, size=n, dtype=np.uint32) << np.uint32(23)) | rng.integers(0, 1 << 23, size=n, dtype=np.uint32) | (rng.integers(0, 2, size=n, dtype=np.uint32) << np.uint32(31))
+    edge = np.array([0, 0x80000000, 1, 0x80000001, 0x007fffff, 0x00800000, 0x3f800000, 0xbf800000, 0x3f800001, 0x33800000, 0x7f7fffff, 0xff7fffff, 0x7f800000, 0xff800000, 0x7fc00000, 0x1fffffff], dtype=np.uint32)
+    row, col, acc = (np.empty(n, dtype=np.uint32) for n in (64 * waves, 64 * waves, 256 * waves))
+    for w in range(waves):  # exponents: anything; around 1; tiny; products near the subnormals; sums that nearly cancel; edges
+        a, b = row[64 * w:64 * w + 64], col[64 * w:64 * w + 64]
+        c = acc[256 * w:256 * w + 256].reshape(64, 4)
+        kind = w % 6
+        span = ((0, 255), (120, 134), (0, 3), (58, 70), (125, 129), (0, 255))[kind]
+        a[:], b[:], c[:] = bits(*span, 64), bits(*span, 64), bits(*((0, 255), (120, 134), (0, 3), (0, 12), (0, 1), (0, 255))[kind], 256).reshape(64, 4)
+        if kind == 4:  # minus the rounded product, a few last places off
+            p = (a.view(np.float32).reshape(16, 1, 4) * b.view(np.float32).reshape(16, 4, 1)).reshape(64, 4)
+            c[:] = ((-p).view(np.uint32).astype(np.int64) + rng.integers(-2, 3, size=(64, 4))).astype(np.uint32)
+        if kind == 5:
+            a[:], b[:], c[:] = rng.choice(edge, 64), rng.choice(edge, 64), rng.choice(edge, (64, 4))
+    dev = lambda a: torch.from_numpy(a.view(np.float32).copy()).to(ctx.device)
+    r_d, c_d, a_d, out = dev(row), dev(col), dev(acc), torch.zeros(256 * waves, device=ctx.device)
+    L.check(ctx.hip.kfdbg_mx_fma(ctx.h, *[C.c_void_p(t.data_ptr()) for t in (r_d, c_d, a_d, out)], waves))
+    got = out.cpu().numpy()
+    fmaf = C.CDLL(ctypes.util.find_library("m")).fmaf
+    fmaf.argtypes, fmaf.restype = [C.c_float] * 3, C.c_float
+    q = row.view(np.float32).reshape(-1, 1, 4), col.view(np.float32).reshape(-1, 4, 1), acc.view(np.float32).reshape(-1, 4, 4)  # [square][lane j][register r]
+    want = np.array([fmaf(*map(float, t)) for t in zip(*(v.ravel() for v in np.broadcast_arrays(*q)))], dtype=np.float32)
+    nan = np.isnan(want)
+    same = np.where(nan, np.isnan(got), want.view(np.uint32) == got.view(np.uint32))
+    tiny = (np.abs(want) > 0) & (np.abs(want) < 2.0 ** -126)
+    assert nan.sum() > 100 and tiny.sum() > 1000 and np.isinf(want).sum() > 100
+    bad = np.flatnonzero(~same)
+    assert not len(bad), "%d differ, the first at %d: %r, fmaf %r" % (len(bad), bad[0], got[bad[0]], want[bad[0]])
+
+
 @pytest.mark.parametrize("type_name", ["Q4", "BF16", "F8E5M2", "T_SIGN", "BOOL1"])
 @pytest.mark.parametrize("m,k", [(1024, 1024), (1024, 3072), (4096, 2048), (96, 256), (1536, 5120)])
 def test_matvec_is_bit_exact(cctx, canon, type_name, m, k):
