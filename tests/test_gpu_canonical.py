@@ -143,6 +143,63 @@ def test_large_fused_entries_are_bit_exact(cctx, canon):
         assert np.array_equal(act, O.swiglu(O.linear(og, xn), O.linear(ou, xn)))
 
 
+def test_large_4bit_matrices_every_epilogue_is_bit_exact(cctx, canon):
+    """the same form with a residual, with bias and alpha / beta, with fp32 results, and pushing them (this rank's slot of two ranks' areas, tagged)"""
+    import ctypes as C
+    ctx, m, k = cctx, 6562, 5120
+    rng = np.random.default_rng(8)
+    ow = O.quantize(O.f32_to_bf16(rng.standard_normal(size=(m, k), dtype=np.float32) * np.float32(0.05)), m, k, L.Q4)
+    w = ctx.upload_blob(L.Q4, m, k, ow.blob())
+    x, res, bias, y0 = (O.f32_to_bf16(rng.normal(0, 1.0, size=n).astype(np.float32)) for n in (k, m, m, m))
+    xd = bf16_t(x, ctx.device)
+    assert np.array_equal(u16(ctx.linear(w, xd, residual=bf16_t(res, ctx.device))), O.add(res, O.linear(ow, x)))
+    got = u16(ctx.linear(w, xd, bias=bf16_t(bias, ctx.device), alpha=1.5, beta=-0.5, y=bf16_t(y0, ctx.device)))
+    assert np.array_equal(got, O.linear(ow, x, bias=bias, alpha=1.5, beta=-0.5, y=y0))
+    ref = O.linear_f32(ow, x).view(np.uint32)
+    yf, d = torch.full((m + 8,), 7.0, device=ctx.device), w.desc()
+    L.check(ctx.hip.kf_linear_f32(ctx.h, C.byref(d), xd.data_ptr(), yf.data_ptr()))
+    got = yf.cpu().numpy()
+    assert np.array_equal(got[:m].view(np.uint32), ref) and (got[m:] == 7.0).all()
+
+    class Comm(C.Structure):
+        _fields_ = [("rank", C.c_int32), ("world", C.c_int32), ("n_max", C.c_int32), ("per_step", C.c_uint32), ("recv", C.c_void_p), ("peer", C.c_void_p * 8), ("d_step", C.c_void_p), ("d_err", C.c_void_p), ("d_push", C.c_void_p)]
+    n_max, per_step, index, step = m + 6, 3, 1, 5
+    areas = torch.zeros(2, 2 * 2 * n_max + 4, dtype=torch.int64, device=ctx.device)  # [exchange buffer][rank][row], then the picks
+    words = torch.tensor([step, 0], dtype=torch.int32, device=ctx.device)
+    ctx.hip.kf_tp_push_bytes.restype = C.c_size_t
+    push = torch.zeros(ctx.hip.kf_tp_push_bytes(C.c_uint32(per_step)), dtype=torch.uint8, device=ctx.device)
+    t = Comm(1, 2, n_max, per_step, areas[1].data_ptr(), (C.c_void_p * 8)(areas[0].data_ptr(), areas[1].data_ptr()), words.data_ptr(), words[1:].data_ptr(), push.data_ptr())
+    L.check(ctx.hip.kf_tp_commit(ctx.h, C.byref(t)))
+    L.check(ctx.hip.kf_linear_f32_push(ctx.h, C.byref(d), C.c_void_p(xd.data_ptr()), C.byref(t), C.c_uint32(index)))
+    want = np.zeros((2, 2, n_max), dtype=np.uint64)  # index is odd: buffer 1; rank 1's slot
+    want[1, 1, :m] = (np.uint64(step * per_step + index + 1) << np.uint64(32)) | ref.astype(np.uint64)
+    for a in areas.cpu().numpy().view(np.uint64):
+        assert np.array_equal(a[:-4].reshape(2, 2, n_max), want) and not a[-4:].any()
+
+
+@pytest.mark.parametrize("device_position", [False, True])
+def test_large_projections_into_the_cache_are_bit_exact(cctx, canon, device_position):
+    """the same form as q | k | v of a decode step: k and v rows at a position of their caches, nothing else written"""
+    import ctypes as C
+    ctx, k, ms, pos, eps = cctx, 5120, [5000, 1026, 1034], 3, 1e-6
+    rng = np.random.default_rng(9)
+    x = O.f32_to_bf16(rng.normal(0, 1.0, size=k).astype(np.float32))
+    nw = O.f32_to_bf16((1 + rng.normal(0, 0.1, size=k)).astype(np.float32))
+    ows = [O.quantize(O.f32_to_bf16(rng.standard_normal(size=(m, k), dtype=np.float32) * np.float32(0.05)), m, k, L.Q4) for m in ms]
+    ws = [ctx.upload_blob(L.Q4, m, k, ow.blob()) for m, ow in zip(ms, ows)]
+    ds, xd, nd, at = [w.desc() for w in ws], bf16_t(x, ctx.device), bf16_t(nw, ctx.device), torch.tensor([pos], dtype=torch.int32, device=ctx.device)
+    ys = [torch.full((r, 1040), 7.0, dtype=torch.bfloat16, device=ctx.device) for r in (5, 5, 5)]
+    ys[0] = torch.full((1, 5000), 7.0, dtype=torch.bfloat16, device=ctx.device)
+    args = (3, (C.c_void_p * 3)(*[C.addressof(d) for d in ds]), (C.c_void_p * 3)(*[y.data_ptr() for y in ys]), (C.c_int64 * 3)(0, 1040, 1040))
+    L.check(ctx.hip.kf_norm_linear(ctx.h, xd.data_ptr(), nd.data_ptr(), eps, *args, 0 if device_position else pos, at.data_ptr() if device_position else None))
+    xn = O.rmsnorm(x, nw, eps)
+    with O.canonical(rows=sum(ms)):
+        for j, (y, ow, m) in enumerate(zip(ys, ows, ms)):
+            want = np.full(tuple(y.shape), O.f32_to_bf16(np.float32([7.0]))[0], dtype=np.uint16)
+            want[pos if j else 0, :m] = O.linear(ow, xn)
+            assert np.array_equal(u16(y), want), j
+
+
 def test_fused_entries_are_bit_exact(cctx, canon):
     """fused RMSNorm + Q|K|V (rows of the launch = all three matrices), paired gate / up + SwiGLU, LM head + arg-max"""
     ctx = cctx
