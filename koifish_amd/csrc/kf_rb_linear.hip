@@ -17,7 +17,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int rb_deal(int nt) { return nt >= 4 ? 2 : 4; }
 // k-steps of weights loaded at a time, one run ahead: a wave of several weight blocks has its bytes in flight with two (us at four | two, 32 rows, two blocks of 32768 x 2048 27.7 | 26.0, three of 12288 x 2048 12.9 | 12.3;
 // with one block two are the slower: one row of 2048 x 6144 6.2 | 7.0)
-constexpr int rb_run(int nt, int mg) { return nt >= 3 || mg >= 2 ? 2 : 4; }
+constexpr int rb_run(int nt, int mg) { return nt >= 4 || mg >= 2 ? 2 : 4; }
 
 __device__ __forceinline__ f32x4 rb_mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
@@ -351,9 +351,16 @@ static int stream_go(hipStream_t st, const RbProduct& q, dim3 grid) {
     // whole lines for more than 8 rows in order: below, a fragment's 16 half lines are few distinct ones and the way round costs more than it saves (one token of a 2048-wide model: 1.79 -> 1.87 ms
     // over four steps; 6 rows 2.04 -> 2.08; 14 rows 2.42 -> 2.35; 32 rows 4.62 -> 4.23)
     const bool turn = p.n > 8 && p.ldx <= (1 << 24), gated = p.epilogue == KF_RB_GATED;
-    // what stream_blocks gives: four waves take one block or two of up to 16 rows and two to four of more; eight take four only where gated; a norm goes in front of gated products of four waves and of any plain ones
-    constexpr bool GATED = NW == 8 || (NT == 1 ? MG <= 2 : MG >= 2), PLAIN = GATED && !(NW == 8 && MG == 4);
+    // what stream_blocks gives, and nothing else.  Four waves: one block or two of up to 16 rows; any of more, but one only where not gated and four not of 33 to 48 rows.  Eight: four only where gated.  In front of a
+    // gated product a norm has four waves.
+    constexpr bool THREE = NT == 3 && MG == 4, GATED = NW == 8 || (NT == 1 ? MG <= 2 : MG >= 2 && !THREE), PLAIN = NW == 8 ? MG <= 3 : NT == 1 ? MG <= 2 : !THREE;
     if constexpr (NT == 1 && GATED && NW == 4) {
+        // a pair as a gate block and its up block of 16 rows each, four k-steps at a time, instead of two blocks of 8 and 8 (the same sums): behind a norm (768 blocks x 2048, 4 rows, us 15.5 | 16.6) up to 1024 blocks, and
+        // for rows that go through LDS from there (6144 x 512, 12 rows, 20.3 | 21.7)
+        if constexpr (MG == 2) {
+            if (gated && p.norm_z && p.m <= 16 * 1024) return stream_form<1, 2, true, 4, true, false, false, true, rb_deal(1)>(st, q, grid);
+            if (gated && turn && p.m > 16 * 1024) return stream_form<1, 2, true, 4, false, true, false, true, rb_deal(1)>(st, q, grid);
+        }
         if (p.norm_z && gated) return stream_form<1, MG, true, 4, true, false>(st, q, grid);
     }
     if constexpr (NT == 1 && PLAIN) {
@@ -384,18 +391,34 @@ static int stream_any(hipStream_t st, const RbProduct& q, dim3 grid, int mg) {
     if (q.p.mode != KF_RB_ALL) return expert_go<NT, NW>(st, q, grid);
     return mg == 1 ? stream_go<NT, 1, NW>(st, q, grid) : mg == 2 ? stream_go<NT, 2, NW>(st, q, grid) : mg == 3 ? stream_go<NT, 3, NW>(st, q, grid) : stream_go<NT, 4, NW>(st, q, grid);
 }
-// How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounded products of
-// one block each: with 32 rows two bytes of tokens to one of weights.  Up to four blocks a CU: as many as make one round of the CUs, eight waves each.  us before (16 weight rows, gated 32) -> now, n = 1, 16, 32, 64 rows:
-// 12288 x 2048 gated 11.1 12.1 15.6 17.2 -> 10.5 11.2 12.3 17.2; 6464 x 2048 7.0 8.7 11.3 13.7 -> 6.8 7.6 8.6 12.5.
-// More than that is bound by HBM while the rows are few: pairs of blocks, many workgroups that follow each other; else the least work for the busiest CU, by workgroups of four waves, several to a
-// CU.  32768 x 2048 22.8 25.5 33.4 45.8 -> 23.0 23.5 26.0 28.8 (134 MB: 5.1 TB/s with 32 rows); 24576 x 4096 gated 33.0 33.2 41.9 47.3 -> 33.0 33.0 36.5 42.0.
-// The number of waves is part of a result's last bits (each adds up a part of k) and stays what it was with the smaller workgroups: four waves for more than 32 rows, behind a norm where gated, and for 768 to 1024 blocks of one matrix, from 17 rows in pairs
-// (12288 x 2048 plain 10.1 11.4 14.4 19.5 -> 10.1 11.4 13.6 17.4; eight waves of three blocks: 10.0 11.0 11.9 15.0).
-static int stream_blocks(int units, int n, bool wide) {
-    if (units <= 1024) return wide ? (units + 255) / 256 : n > 16 ? 2 : 1;
+// How many 16-row blocks a workgroup takes.  A workgroup takes in its weight rows and, once, all of the batch's token rows by its CU's way to the L2 (about 46 bytes a ns), which, and not HBM, bounds products of
+// one block each: with 32 rows two bytes of tokens to one of weights.  More blocks: fewer token bytes, fewer and longer workgroups.  us, one block (gated: 8 gate rows and their 8 up rows) | two | three | four, by blocks of
+// the matrix x k:
+//  - one round of the CUs (eight waves each, up to 1024 blocks): as many as fill it.  12 rows 640 x 2048 plain 11.4 | 11.6 | 10.2 | 10.8; 32 rows 12288 x 2048 gated 15.6 before, three 12.3.  Not where the tokens are
+//    few: plain, 4 rows or fewer (1 row 512 x 1024 5.0 | 5.5), up to 12 where k is short too; gated, 1024 x 512 8 rows two 5.5, four 6.0, 1024 x 4096 9 rows two 27.2, four 28.7.
+//  - up to 10 rows of more than 1024 blocks, plain: one.  1 row 2048 x 1024 13.6 | 14.9; 9 14.4 | 14.7; 12 14.7 | 14.8; 16 rows 2048 x 2048 28.3 | 26.1.  Behind a norm, which every workgroup makes for itself: two.
+//  - a norm in front of a gated product: one up to 256 blocks (128 x 2048 7.9 | 9.3), then pairs: 768 x 2048 4 rows 16.4 | 15.5.
+//  - more than 16 rows of up to 1024 blocks, four waves: two where the CUs still get one workgroup each.  128 x 2048 33 rows 8.4 | 9.8, 320 x 1024 48 rows 7.5 | 7.5, 1024 x 256 24 rows 6.3 | 5.0; short k moves the line up
+//    (40 x 256 3.1 | 4.1, 512 x 256 3.8 | 4.4), since the products are over before the tokens are in.
+//  - more than 1024 blocks: pairs, many workgroups that follow each other, up to 24 rows; then the least work for the busiest CU.  32 rows 32768 weight rows x 2048 33.4 | 26.0, 64 rows 45.8 | 28.8 with four.  33 to 48
+//    rows: three, two workgroups to a CU (four need registers of which only one goes): 3072 x 1024 gated 33.3 | 28.0 | 25.9 | 31.5, but two where the second round of them would be nearly empty: 2048 x 1024 25.6 | 21.1 |
+//    22.8 | 23.4.  49 rows and more of a short k: two (3072 x 256 gated 15.4 | 13.7 | 15.1 | 15.3).
+// The number of waves is part of a result's last bits (each adds up a part of k) and the same for every count: four for more than 32 rows, behind a norm where gated, and for 768 to 1024 blocks of one matrix.
+static int stream_blocks(const kf_rb_product& p, bool wide) {
+    const bool gated = p.epilogue == KF_RB_GATED, norm = p.norm_z != nullptr;
+    const int units = p.m / 16, n = p.n, k = p.k, round = (units + 255) / 256;
+    if (units <= 1024) {
+        if (wide && gated) return units > 768 && n <= 16 && (n > 8 || k < 1024) ? 2 : round;
+        if (wide) return !norm && (n <= 4 || (n <= 12 && k <= 1024 && units <= 512)) ? 1 : round;
+        if (gated) return n > 16 || (norm && units > 256) ? 2 : 1;
+        return n > 16 && units >= (k >= 1024 ? 257 : n > 32 && n <= 48 ? 513 : 768) ? 2 : 1;
+    }
+    if (n <= 16) return gated || norm || n > 10 ? 2 : 1;
+    if (n <= 24 || (n > 48 && k < 512)) return 2;
+    if (n > 32 && n <= 48) return units > 1536 && units <= 2048 ? 2 : 3;
     int best = 2;
     long least = 0;
-    for (int mg = 2; n > 24 && mg <= 4; mg++) {
+    for (int mg = 2; mg <= 4; mg++) {
         const long cost = ((units + mg - 1) / mg + 255) / 256 * (16 * mg + n);
         if (mg == 2 || cost < least) best = mg, least = cost;
     }
@@ -410,7 +433,7 @@ int rb_stream_launch(hipStream_t st, const RbProduct& q) {
     const bool gated = p.epilogue == KF_RB_GATED;
     const long small = (long)units / (gated ? 2 : 1) * (tiles ? q.e.n_tile : p.parts > 1 ? p.parts : 1); /* workgroups of 16 rows, of 16 gates and 16 ups */
     const bool wide = p.k >= 512 && nt <= 2 && !(p.norm_z && gated) && small < 768;                        /* few workgroups: more waves each, more loads in flight per CU */
-    const int mg = !all ? (gated ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(units, p.n, wide);
+    const int mg = !all ? (gated ? 2 : 1) : p.parts > 1 ? 1 : stream_blocks(p, wide);
     const dim3 grid((units + mg - 1) / mg, tiles ? q.e.n_tile : (p.parts > 1 ? p.parts : 1));
     if (nt > 2) return nt == 3 ? stream_any<3, 4>(st, q, grid, mg) : stream_any<4, 4>(st, q, grid, mg);
     return nt == 1 ? (wide ? stream_any<1, 8>(st, q, grid, mg) : stream_any<1, 4>(st, q, grid, mg)) : (wide ? stream_any<2, 8>(st, q, grid, mg) : stream_any<2, 4>(st, q, grid, mg));

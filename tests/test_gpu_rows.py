@@ -110,11 +110,11 @@ def test_product_epilogues(ctx, kind, n, m, k):
         assert np.abs(f64(y) - fn(gate) * upw).max() < tol * 8
 
 
-@pytest.mark.parametrize("m", [4096, 4160, 8320, 12352, 16448, 32768])  # one, two, three (and a rest), four blocks of 16 weight rows a workgroup; more than one round: two, three (a rest), four by the rows
-@pytest.mark.parametrize("n,k", [(1, 512), (4, 64), (9, 576), (24, 512), (25, 64), (33, 512), (64, 576)])
+@pytest.mark.parametrize("m", [4096, 4160, 8320, 12352, 16448, 32768])  # both sides of 256, 513, 768 and 1024 blocks of 16 weight rows, no multiples of three and four; 2048, the last of two rounds of three
+@pytest.mark.parametrize("n,k", [(1, 512), (4, 64), (8, 1024), (9, 576), (12, 64), (24, 512), (25, 64), (33, 512), (48, 64), (64, 576)])
 def test_products_of_several_blocks(ctx, m, n, k):
-    """Against float64.  A sum of k products of normal numbers over sqrt(k) is about 1 and at most 6 here; in float32 its rounding is at most k 2^-24 of the sum of magnitudes (< 1.2 sqrt(k)): below 1e-4 where k <= 576 were they all of
-    one sign, a tenth of that as it is.  16-bit results add half of 2^-8."""
+    """Against float64.  A sum of k products of normal numbers over sqrt(k) is about 1 and at most 6 here; in float32 each of its k additions rounds by at most 2^-24 of a partial sum, either way: about sqrt(k) 2^-24 of 3, below
+    6e-6 for k <= 1024.  16-bit results add half of 2^-8."""
     g = torch.Generator().manual_seed(m + n)
     w, x, res = dev(torch.randn(m, k, generator=g) / k ** 0.5, torch.bfloat16), dev(torch.randn(n, k + 8, generator=g), torch.bfloat16), dev(torch.randn(n, m, generator=g))
     ref, ws, ssq = f64(x)[:, :k] @ f64(w).T, stored(w), torch.full((m // 16, 4), 7.0, device="cuda")
