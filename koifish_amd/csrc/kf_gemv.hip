@@ -848,9 +848,13 @@ int gemv_launch_dot2(hipStream_t st, GemvLaunch& L) {
     // q/k/v and o_proj launches, 22-28 MB each, 21.8 -> 19.1 and 16.1 -> 13.2 us; the 0.6B launches stay below the threshold)
     const long blocks_all = raw_slots * (long)nBlk * (64 / (1 << lpr_log2));
 #if KF_GEMV_CANON
-    // a workgroup per CU from 2^20 blocks: below, its one prologue of all 16 waves costs more than it saves.  us, the kernel of small workgroups | one per CU: 4096 x 4096 6.4 | 8.3, 6144 x 4096 7.3 | 8.9, gate and up
-    // 9728 x 2560 (2^20.6) 14.7 | 14.6, 12288 x 4096 23.7 | 22.4, 17408 x 5120 42.7 | 33.2; 7168 x 5120 12.0 | 11.3, 4096 x 12288 16.5 | 14.1
-    if (fmt == FMT_Q4 && g_knobs.q4_perm != 0 && g_knobs.gemv_waves == 0 && L.target_waves <= 0 && L.mode != GEMV_ARGMAX && !a.row_map && blocks_all * (L.mode == GEMV_PAIRED ? 2 : 1) >= (1L << 20) && raw_slots >= 2048 && a.lGroup == 128 && K % 128 == 0 &&
+    // A workgroup per CU from 2^20 blocks: below, its one prologue of all 16 waves costs more than it saves.  us, the kernel of small workgroups | one per CU: 4096 x 4096 6.4 | 8.3, 6144 x 4096 7.3 | 8.9, 6592 x 5120
+    // 11.9 | 11.4, 4096 x 8192 11.4 | 10.3, gate and up 2752 x 6144 14.9 | 11.8.  Short rows leave the small workgroups little to stage, and with one slot a wave they are the faster up to 2^21 blocks (11520 x 4096
+    // 11.9 | 12.9, 13120 12.6 | 13.6, 16384 15.5 | 15.4; 13696 x 3072 10.3 | 11.8, 21888 15.0 | 15.1), of several matrices to 2^20.6 (gate and up 4096 x 4096 10.2 | 11.0, 5120 12.0 | 12.2, 6592 15.1 | 14.4; q, k and v 11520 x 4096
+    // 15.1 | 15.3, 14784 18.0 | 16.8); from 16384 slots on their waves take two (16384 x 2048 9.2 | 10.4, 18368 11.6 | 11.1; 32768 x 1024 9.5 | 10.9, 36736 11.5 | 11.3).
+    const long blocks_read = blocks_all * (L.mode == GEMV_PAIRED ? 2 : 1);
+    const bool per_cu = blocks_read >= (1L << 20) && (K > 4096 || raw_slots > 16384 || blocks_read >= (L.n > 1 ? 3L << 19 : 1L << 21));
+    if (fmt == FMT_Q4 && g_knobs.q4_perm != 0 && g_knobs.gemv_waves == 0 && L.target_waves <= 0 && L.mode != GEMV_ARGMAX && !a.row_map && per_cu && raw_slots >= 2048 && a.lGroup == 128 && K % 128 == 0 &&
         lpr_log2 >= 2 && nBlk % LPR == 0 && K <= 8 * 64 * GQ_WAVES * GQ_XCH) {
         bool even = true;
         for (int j = 0; j < L.n; j++) even = even && L.w[j]->ne0 % RPS == 0;

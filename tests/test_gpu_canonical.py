@@ -108,9 +108,9 @@ def test_long_4bit_rows_through_two_fp32_windows_are_bit_exact(cctx, canon, m, k
     assert np.array_equal(y0, ref)
 
 
-@pytest.mark.parametrize("m,k", [(262160, 128), (65552, 512), (6562, 5120), (2056, 32768), (2048, 33792)])  # 4 lanes a row and one step, 16, an odd number of row slots, the longest x of a workgroup per CU, one longer
+@pytest.mark.parametrize("m,k", [(262160, 128), (65552, 512), (16384, 4096), (6562, 5120), (2056, 32768), (2048, 33792)])  # 4 lanes a row and one step, 16, 64 (short rows), an odd number of row slots, the longest x of a workgroup per CU, one longer
 def test_large_4bit_matrices_are_bit_exact(cctx, canon, m, k):
-    """2^20 blocks and more: one workgroup per CU (gemv_q4_kernel)"""
+    """one workgroup per CU (gemv_q4_kernel): 2^20 blocks of long rows, of more than 16384 row slots, 2^21 of others"""
     ctx = cctx
     rng = np.random.default_rng(m + k)
     w = O.f32_to_bf16(rng.standard_normal(size=(m, k), dtype=np.float32) * np.float32(0.05))
