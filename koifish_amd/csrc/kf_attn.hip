@@ -511,12 +511,13 @@ int attn_launch(hipStream_t st, AttnArgs& a) {
     const int pos_max = a.pos + a.n_tok - 1;
     int nsp = batch ? 1 : attn_splits(a.pos, a.n_kv);
     a.inv_sqrt_hd_den = sqrtf((float)hd);
-    // Canonical order, hd 128, GQA-8 and -4: short contexts by workgroups of two heads, four waves and 64 keys (a short chain each); above 1024 keys by workgroups of four heads and eight waves, one
-    // to a CU, whose slices grow with the context: two to four times fewer partials to leave, count in and merge, K and V unpacked once for four heads, and all of them resident at once (of two heads and
-    // 145 registers, 768 of 1024 were).  us, 64 heads on 8, two heads | four, at 512 keys 7.4 | 10.1, 1024 9.6 | 10.2, 1344 12.4 | 10.7, 1664 13.2 | 10.9,
-    // 4000 19.6 | 13.4 (26.5 with the merge's loads one after the other); four heads and four waves at 4000 with 32 | 16 slices 16.9 | 15.9, eight waves with 32 (two rounds) 21.5.
-    const int knob = g_knobs.attn_gq_split;
-    const bool fours = a.canon && (GQ == 8 || GQ == 4) && hd == 128 && !batch && knob <= 2 && a.pos >= 1024;
+    // Canonical order, hd 128, GQA-8 and -4: workgroups of two heads, four waves and 64 keys (a short chain each) as long as they are no more than two to a CU; above, workgroups of four heads and eight waves, one to
+    // a CU, whose slices grow with the context: two to four times fewer partials to leave, count in and merge, K and V unpacked once for four heads, and all of them resident at once (of two heads and 145 registers, 768
+    // of 1024 were).  us, heads on kv-heads, two | four: 64 on 8 1024 keys 9.6 | 10.2, 1030 11.3 | 10.2, 2040 14.3 | 10.8, 4000 18.3 | 13.9; 64 on 16 1030 11.5 | 10.6; 16 on 4 (at most one to a CU) 1030 7.2 | 9.4, 4000
+    // 9.2 | 11.1, 16000 17.6 | 19.5.  At exactly two to a CU the slices grow with the context too, and four heads are the faster from 192 keys a slice: 32 on 8 4000 keys 12.1 | 12.4, 6100 14.5 | 15.5, 6200
+    // 16.4 | 15.9, 16000 25.9 | 22.4; 32 on 4 6100 13.3 | 13.8, 6200 15.2 | 13.8.
+    const int knob = g_knobs.attn_gq_split, two_heads = a.n_head / 2 * nsp; /* workgroups of two heads */
+    const bool fours = a.canon && (GQ == 8 || GQ == 4) && hd == 128 && !batch && knob <= 2 && (two_heads > 512 || (two_heads == 512 && pos_max >= 192 * nsp));
     a.gq_split = !a.canon ? 1 : GQ == 8 ? (knob ? knob : fours ? 2 : 4) : GQ == 4 && !fours && knob != 2 ? 2 : 1;
     const int gq_wg = GQ / a.gq_split; /* query heads per workgroup */
     if (fours) nsp = std::max(1, std::min({nsp, 256 / (a.n_kv * a.gq_split), (a.pos + 128) / 128}));

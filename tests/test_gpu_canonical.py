@@ -243,9 +243,11 @@ def test_decode_attention_is_bit_exact(cctx, n_head, n_kv, hd, pos):
     assert np.array_equal(out, ref), "%d of %d outputs differ" % (int((out != ref).sum()), out.size)
 
 
-@pytest.mark.parametrize("n_head,n_kv,hd,pos", [(64, 8, 128, 1023), (64, 8, 128, 1024), (64, 8, 128, 1101), (4, 1, 128, 4095), (32, 8, 128, 1030), (64, 64, 128, 1500)])
+@pytest.mark.parametrize("n_head,n_kv,hd,pos", [(64, 8, 128, 1023), (64, 8, 128, 1024), (64, 8, 128, 1101), (4, 1, 128, 4095), (32, 8, 128, 1030), (64, 64, 128, 1500),
+                                                (128, 16, 128, 511), (128, 16, 128, 512), (32, 8, 128, 6143), (32, 8, 128, 6144), (64, 16, 128, 1200)])
 def test_decode_attention_by_fours_is_bit_exact(cctx, n_head, n_kv, hd, pos):
-    """four heads and eight waves a workgroup above 1024 keys: the last position of two heads, the first of four, uneven slices, most slices, GQA-4; no GQA"""
+    """four heads and eight waves a workgroup: the last position at which workgroups of two heads are two to a CU, the first of four (8 and 16 kv-heads), uneven slices, the longest slices of two heads and one key more, GQA-4;
+    few kv-heads (two heads at any length); no GQA"""
     test_decode_attention_is_bit_exact(cctx, n_head, n_kv, hd, pos)
 
 
