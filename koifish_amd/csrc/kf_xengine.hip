@@ -158,9 +158,9 @@ int xengine_build(const kf_engine_desc* d, int n_seq, long long kv_seq_stride, v
     if (sc == 2 && xe_shape_smem<XC2>(n_seq, d->n_layer, false) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
     if (sc == 4 && xe_smem<XC4W>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
     if (sc == 5 && xe_smem<XC5W>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
-    if (sc == 3 && n_seq <= XE_NXCD && xe_smem<XC3<12, 6, false, 1>>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
+    if (sc == 3 && n_seq <= XE_NXCD && xe_smem<XC3<12, 2, false, 1>>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
     *why = "two decoders per XCD (more than 8 sequences) do not fit this shape and depth: two workgroups per CU need 2 x the activations + the layer table in 160 KB of LDS";
-    if (sc == 3 && n_seq > XE_NXCD && 2 * xe_smem_class3_two(d->n_layer) > 160 * 1024 && xe_smem<XC3<8, 8, false, 1, 2, 2>>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
+    if (sc == 3 && n_seq > XE_NXCD && 2 * xe_smem_class3_two(d->n_layer) > 160 * 1024 && xe_smem<XC3<8, 4, false, 1, 2, 2>>(d->n_layer) > 160 * 1024) return KF_UNSUPPORTED_DATATYPE;
     if (!dry && (ws_bytes < xengine_ws_bytes(d) || ((uintptr_t)ws & 255) != 0)) {
         *why = "workspace too small or not 256-byte aligned";
         return KF_INVALID_ARGS;
@@ -359,41 +359,19 @@ static int xengine_go_shape(XEngineHost* E, hipStream_t st) {
 #ifndef XE_ONLY_DEFAULT
     const bool dbg = E->args.dbg != nullptr;
     if (dbg && nb == 4) return xengine_go<XF<XC, 12, 2, true, 1, 2, 4>>(E, st);
-    if (dbg && nb == 2) return xengine_go<XF<XC, 12, 4, true, 1, 2, 2>>(E, st);
+    if (dbg && nb == 2) return xengine_go<XF<XC, 12, 2, true, 1, 2, 2>>(E, st);
     if (dbg && nb == 1) return two ? xengine_go<XF<XC, 8, 4, true, 2, 1, 1>>(E, st) : xengine_go<XF<XC, 12, 2, true, 1, 2, 1>>(E, st);
 #endif
     if (nb == 4) { /* 8 compute waves + the four sequences' pollers (168 registers), where the four sequences' activations + the layer table fit the LDS; else 4 + 4 waves */
-#ifdef XE_NB4_VARIANTS /* tuning builds only */
-        if (E->variant_set && E->nwv == 12 && E->depth == 8) return xengine_go<XF<XC, 12, 8, false, 1, 2, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 4) return xengine_go<XF<XC, 12, 4, false, 1, 2, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 61) return xengine_go<XF<XC, 12, 6, false, 1, 1, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 41) return xengine_go<XF<XC, 12, 4, false, 1, 1, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 21) return xengine_go<XF<XC, 12, 2, false, 1, 1, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 6) return xengine_go<XF<XC, 12, 6, false, 1, 2, 4>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 22) return xengine_go<XF<XC, 12, 2, false, 1, 2, 4, 2>>(E, st); /* two pollers for the four sequences */
-        if (E->variant_set && E->nwv == 12 && E->depth == 12) return xengine_go<XF<XC, 12, 2, false, 1, 2, 4, 1>>(E, st); /* one */
-        if (E->variant_set && E->nwv == 12 && E->depth == 44) return xengine_go<XF<XC, 12, 4, false, 1, 2, 4, 4>>(E, st);
-#endif
-        // ring depth 2 (measured, 32 sequences at 2 k keys, tokens/s: depth 8 5320 -- spills --, 6 6970, 4 7360, 2 7815; one key tile per attention batch 7480 / 7720 at depth 6 / 2): with
-        // four sequences' chain pairs and activation chunks live, every register the ring does not hold is worth more than a deeper queue -- twelve waves hide the latency
+        // A ring of two units (the 0.6B shape, 32 sequences at 2 k keys, us a step: 12 waves with 1 / 2 / 3 / 4 units 2993 / 3021 / 3315 / 3614, 8 waves with 2 / 3 / 4 / 6 3216 / 3263 / 3313 / 3396): every register the
+        // ring does not hold is worth more than a deeper queue -- twelve waves hide the latency
         if (!(E->variant_set && E->nwv == 8) && xe_smem<XF<XC, 12, 2, false, 1, 2, 4>>(E->args.n_layer) <= 160 * 1024) return xengine_go<XF<XC, 12, 2, false, 1, 2, 4>>(E, st);
-        return xengine_go<XF<XC, 8, 8, false, 1, 2, 4>>(E, st);
+        return xengine_go<XF<XC, 8, 4, false, 1, 2, 4>>(E, st);
     }
     if (nb == 2) {
-#ifdef XE_NB4_VARIANTS /* tuning builds only */
-        if (E->variant_set && E->nwv == 12 && E->depth == 61) return xengine_go<XF<XC, 12, 6, false, 1, 1, 2>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 6) return xengine_go<XF<XC, 12, 6, false, 1, 2, 2>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 41) return xengine_go<XF<XC, 12, 4, false, 1, 1, 2>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 2) return xengine_go<XF<XC, 12, 2, false, 1, 2, 2>>(E, st);
-        if (E->variant_set && E->nwv == 12 && E->depth == 14) return xengine_go<XF<XC, 12, 4, false, 1, 2, 2, 1>>(E, st); /* one poller for the two sequences */
-        if (E->variant_set && E->nwv == 12 && E->depth == 12) return xengine_go<XF<XC, 12, 2, false, 1, 2, 2, 1>>(E, st);
-#endif
-        if (E->variant_set && E->nwv == 8) return xengine_go<XF<XC, 8, 8, false, 1, 2, 2>>(E, st);
-        return xengine_go<XF<XC, 12, 4, false, 1, 2, 2>>(E, st); /* (16 sequences: depth 6 5990, 4 6250, 2 6200 tokens/s) */
+        if (E->variant_set && E->nwv == 8) return xengine_go<XF<XC, 8, 4, false, 1, 2, 2>>(E, st);
+        return xengine_go<XF<XC, 12, 2, false, 1, 2, 2>>(E, st); /* (16 sequences, us a step: 1 / 2 / 3 / 4 units 2333 / 2358 / 2605 / 2787; 8 waves with 2 / 3 / 4 / 6 2603 / 2630 / 2662 / 2782) */
     }
-#ifdef XE_NB4_VARIANTS
-    if (!two && E->variant_set && E->nwv == 12 && E->depth == 4) return xengine_go<XF<XC, 12, 4, false, 1, 2, 1>>(E, st);
-#endif
     if (!two && E->variant_set && E->nwv == 12 && E->depth == 6) return xengine_go<XF<XC, 12, 6, false, 1, 2, 1>>(E, st);
     if (!two && E->variant_set && E->nwv == 9) return xengine_go<XF<XC, 9, 8, false, 1, 2, 1>>(E, st);
     return two ? xengine_go<XF<XC, 8, 4, false, 2, 1, 1>>(E, st) : xengine_go<XF<XC, 12, 2, false, 1, 2, 1>>(E, st); /* (8 sequences: depth 6 4370, 4 4570, 2 4630 tokens/s) */
@@ -402,8 +380,8 @@ static int xengine_go_shape(XEngineHost* E, hipStream_t st) {
 template <template <int, int, bool, int, int, int, int> class XC>
 static size_t xe_shape_smem(int n_seq, int n_layer, bool two_wpc) {
     if (n_seq <= XE_NXCD) return xe_smem<XF<XC, 12, 2, false, 1, 2, 1>>(n_layer);
-    if (n_seq <= 2 * XE_NXCD) return two_wpc ? 2 * (xe_smem<XF<XC, 8, 4, false, 2, 1, 1>>(n_layer) < 54 * 1024 ? (size_t)54 * 1024 : xe_smem<XF<XC, 8, 4, false, 2, 1, 1>>(n_layer)) : xe_smem<XF<XC, 12, 4, false, 1, 2, 2>>(n_layer);
-    const size_t s12 = xe_smem<XF<XC, 12, 2, false, 1, 2, 4>>(n_layer), s8 = xe_smem<XF<XC, 8, 8, false, 1, 2, 4>>(n_layer);
+    if (n_seq <= 2 * XE_NXCD) return two_wpc ? 2 * (xe_smem<XF<XC, 8, 4, false, 2, 1, 1>>(n_layer) < 54 * 1024 ? (size_t)54 * 1024 : xe_smem<XF<XC, 8, 4, false, 2, 1, 1>>(n_layer)) : xe_smem<XF<XC, 12, 2, false, 1, 2, 2>>(n_layer);
+    const size_t s12 = xe_smem<XF<XC, 12, 2, false, 1, 2, 4>>(n_layer), s8 = xe_smem<XF<XC, 8, 4, false, 1, 2, 4>>(n_layer);
     return s12 < s8 ? s12 : s8;
 }
 // n_steps decode steps of every sequence in ONE launch; with_head: 0 layers only (x_out), 1 + logits, 2 + greedy pick and state update (needed for n_steps > 1)
@@ -418,28 +396,17 @@ int xengine_steps(XEngineHost* E, hipStream_t st, int32_t* d_state, uint16_t* x_
     int rc;
     if (E->fmt != FMT_Q4P) rc = xengine_go_lowbit(E, st);
     else
-#ifdef XE_NB4_VARIANTS /* tuning builds: the ring depth of the other shapes */
-    if (E->shape_class == 3 && a.n_seq <= XE_NXCD && E->variant_set && E->depth == 4) rc = xengine_go<XC3<12, 4, false, 1>>(E, st);
-    else if (E->shape_class == 3 && a.n_seq <= XE_NXCD && E->variant_set && E->depth == 2) rc = xengine_go<XC3<12, 2, false, 1>>(E, st);
-    else if (E->shape_class == 4 && E->variant_set && E->depth == 4) rc = xengine_go<XCfg<FMT_Q4P, 4, 128, 12, 2560, 4096, 1024, 9728, 4, false, 1, 1>>(E, st);
+#ifdef XE_GQ4_VARIANTS /* tuning builds: the ring depth of the GQA-4 shapes */
+    if (E->shape_class == 4 && E->variant_set && E->depth == 4) rc = xengine_go<XCfg<FMT_Q4P, 4, 128, 12, 2560, 4096, 1024, 9728, 4, false, 1, 1>>(E, st);
     else if (E->shape_class == 4 && E->variant_set && E->depth == 2) rc = xengine_go<XCfg<FMT_Q4P, 4, 128, 12, 2560, 4096, 1024, 9728, 2, false, 1, 1>>(E, st);
     else if (E->shape_class == 5 && E->variant_set && E->depth == 2) rc = xengine_go<XCfg<FMT_Q4P, 4, 128, 12, 4096, 4096, 1024, 12288, 2, false, 1, 1>>(E, st);
     else
 #endif
     if (E->shape_class == 3) { /* the default instantiations only (no tuning variants, no stamps) */
-#ifdef XE_C3_VARIANTS /* tuning builds: the two-sequences-per-decoder form of the 1.7B shape */
-        if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 12 && E->depth == 2) rc = xengine_go<XC3<12, 2, false, 1, 2, 2>>(E, st);
-        else if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 12 && E->depth == 21) rc = xengine_go<XC3<12, 2, false, 1, 1, 2>>(E, st);
-        else if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 12 && E->depth == 4) rc = xengine_go<XC3<12, 4, false, 1, 2, 2>>(E, st);
-        else if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 8 && E->depth == 4) rc = xengine_go<XC3<8, 4, false, 1, 2, 2>>(E, st);
-        else if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 8 && E->depth == 6) rc = xengine_go<XC3<8, 6, false, 1, 2, 2>>(E, st);
-        else if (a.n_seq > XE_NXCD && E->variant_set && E->nwv == 8 && E->depth == 2) rc = xengine_go<XC3<8, 2, false, 1, 2, 2>>(E, st);
-        else
-#endif
-        // two sequences per decoder: 6 compute waves + 2 pollers at 256 registers (measured at 2 k keys, 16 sequences: 2180 tokens/s; 12 waves at 168 registers spill in the
-        // streaming loops: 1650 - 1690; two decoders per XCD 1600; eight sequences, one per decoder: 1940)
-        if (a.n_seq > XE_NXCD && !E->two_wpc && xe_smem<XC3<8, 8, false, 1, 2, 2>>(a.n_layer) <= 160 * 1024) rc = xengine_go<XC3<8, 8, false, 1, 2, 2>>(E, st); /* (ring depth 4 / 6 / 8: 2180 / 2230 / 2240) */
-        else rc = a.n_seq > XE_NXCD ? xengine_go<XC3<8, 4, false, 2, 1>>(E, st) : xengine_go<XC3<12, 6, false, 1>>(E, st);
+        // two sequences per decoder: 6 compute waves + 2 pollers at 256 registers (16 sequences at 2 k keys, us a step: 8 waves with 2 / 3 / 4 / 6 units 5191 / 5184 / 5284 / 5472, 12 at 168 registers with 1 / 2 / 3 / 4 4969 /
+        // 5105 / 5201 / 5717); one per decoder, 8 sequences: 12 waves 5000 / 4961 / 5218 / 4918, 8 waves 4703 / 4797 / 4816 / 4949
+        if (a.n_seq > XE_NXCD && !E->two_wpc && xe_smem<XC3<8, 4, false, 1, 2, 2>>(a.n_layer) <= 160 * 1024) rc = xengine_go<XC3<8, 4, false, 1, 2, 2>>(E, st);
+        else rc = a.n_seq > XE_NXCD ? xengine_go<XC3<8, 4, false, 2, 1>>(E, st) : xengine_go<XC3<12, 2, false, 1>>(E, st);
     }
     else if (E->shape_class == 4)
         rc = E->nwv == 8 ? xengine_go<XC4>(E, st) : xengine_go<XC4W>(E, st);

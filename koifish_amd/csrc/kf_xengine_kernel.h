@@ -11,7 +11,7 @@
 //   * every hand-off vector of a decoder lives in cached memory that only its XCD touches: producers write tagged granules with PLAIN stores (they land in that XCD's
 //     L2), the poller wave sweeps them with sc1 loads -- "the data is the flag" exactly as in kf_engine.hip, but an edge costs ~0.7 us instead of 1.2-2.3.
 //   * 32 CUs cannot hold a layer in registers (261 KB of blocks per workgroup and layer), so the mat-vec phases STREAM: each compute wave walks its row slots with a ring
-//     of DEPTH 16-byte blocks in flight, and in the last round of a phase the ring is refilled with the first blocks of the NEXT phase -- they do not depend on the
+//     of RING 16-byte blocks in flight, and in the last round of a phase the ring is refilled with the first blocks of the NEXT phase -- they do not depend on the
 //     hand-off, so HBM latency stays off the chain.  The attention phase streams its K/V rows the same way (two batches of tiles in flight).
 //
 // The arithmetic is the canonical order of oracle/kf_oracle.c sections 4c and 6 (the library default): the same lanes per row, chain pairs and lane tree as
@@ -116,7 +116,7 @@ struct XCfg {
     // ten of twelve waves to the arithmetic (the mat-vec phases and the attention are 86 % of the NB = 4 layer period; the hand-offs 12 %)
     static constexpr int NP = NP_ > 0 ? NP_ : NB_;
     static_assert(NB_ % NP == 0, "every poller the same number of sequences");
-    static constexpr int FMT = FMT_, GQ = GQ_, HD = HD_, NWV = NWV_, NCW = NWV_ - NP, DIM = DIM_, QD = QD_, KVD = KVD_, FFN = FFN_, DEPTH = DEPTH_, NWG = XE_NWG;
+    static constexpr int FMT = FMT_, GQ = GQ_, HD = HD_, NWV = NWV_, NCW = NWV_ - NP, DIM = DIM_, QD = QD_, KVD = KVD_, FFN = FFN_, RING = DEPTH_, NWG = XE_NWG; /* RING: entries (MF, below: units of 4 KiB) of a phase in flight per wave */
     static constexpr bool DBG = DBG_;
     static_assert(FMT_ == FMT_Q4 || FMT_ == FMT_Q4P || FMT_ == FMT_Q1T || FMT_ == FMT_Q2T,
                   "4-bit PackedQ layers (arithmetic or register-table unpack), or 1-bit / 2-bit: one dword of a 128-element block, resp. one 8-byte half of a 64-element block per lane");
@@ -172,9 +172,9 @@ struct XCfg {
                                   SH::P6::nBlk == SH::P6::iters * SH::P6::LPR;
     static constexpr int maxR = (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R) > (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R) ? (SH::P1::R > SH::P5::R ? SH::P1::R : SH::P5::R)
                                                                                                                                       : (SH::P4::R > SH::P6::R ? SH::P4::R : SH::P6::R);
-    // MF: the 4-bit phases on the matrix cores (xe_unit_mf): a wave takes UNITS of 4 KiB, four loads of a whole KiB each.  For several sequences, and for one where a phase's rows are long and many: there the
-    // products cost what the vector pipe's did and the whole-KiB units are the gain (28 layers of 2048 x 6144, 8 decoders of one sequence at 2 k
-    // keys 5202 -> 4940 us a step, two decoders 4988 -> 4849; of 1024 x 3072, short rows, 8 decoders 1776 -> 1971)
+    // MF: the 4-bit phases on the matrix cores (xe_unit_mf): a wave takes UNITS of 4 KiB, four loads of a whole KiB each.  For several sequences, and for one sequence of the 2048-wide shape: there the products cost what
+    // the vector pipe's did and the whole-KiB units are the gain (28 layers of 2048 x 6144, 8 decoders of one sequence at 2 k keys 5202 -> 4940 us a step, two decoders 4988 -> 4849).  Not for one sequence of the other shapes:
+    // 1024 wide the rows are short (8 decoders 1776 -> 1971); 2560 wide a row has 16 lanes, less than a unit's 32; 4096 wide and the tensor-parallel ranks, whose q | k | v are one matrix (FUSED), were not tried.
     static constexpr bool MF = (NB_ > 1 || (DIM_ >= 2048 && !TP_ && WPC_ == 1 && !FUSED && NG == 1)) && FMT_ == FMT_Q4P && SH::P1::LPR >= 32 && SH::P4::LPR >= 32 && SH::P5::LPR >= 32 && SH::P6::LPR >= 32;
     template <class P>
     struct MG { /* a phase's figures (P: PlanT): units of CE block columns x RS rows, 64 / CE sets of four; a slot: RS rows, all its NIT units */
@@ -199,7 +199,6 @@ struct XCfg {
         static constexpr bool ok = (CE == 32 || CE == 64) && P::nBlk % CE == 0 && NIT >= H && NIT <= 16 && (H == 1 || H == 2) && P::R % RS == 0;
     };
     static constexpr bool MFH = MF && NB_ > 1 && HLPR == 64 && HnBlk % 64 == 0; /* the head on the matrix cores too: slots of four rows */
-    static constexpr int RING = MF ? (NWV_ == 8 ? 4 : 2) : DEPTH_; /* entries (MF: units) of a phase in flight per wave */
     static_assert(!MF || !PREP, "sixteen bytes a lane");
     static_assert(!MF || (MG<typename SH::P1>::ok && MG<typename SH::P4>::ok && MG<typename SH::P5>::ok && MG<typename SH::P6>::ok), "whole entries, whole slots");
     static_assert(NB_ >= 1 && NB_ <= 4, "sequences per decoder");
@@ -298,7 +297,7 @@ struct XRing {
 };
 // One mat-vec phase as RUN-TIME parameters of one wave (all wave-uniform: scalar registers).  The geometry figures are the compile-time constants of PlanT (the lanes per row,
 // rows per wave step and steps per row gemv_launch picks for the matrices: the canonical summation order), handed to ONE copy of the streaming loop: four typed copies of the
-// DEPTH-times unrolled block code were 150 KB of instructions.
+// RING-times unrolled block code were 150 KB of instructions.
 struct XPhase {
     EngMat m, m2;    /* m2: up_proj beside gate_proj (paired) */
     float qb, qb2;
