@@ -476,11 +476,13 @@ __global__ void __launch_bounds__(256) gemv_kernel(const GemvArgs a) {
 
 #if KF_GEMV_CANON
 // Large 4-bit matrices in the canonical order.  Bound by the vector pipe, not by memory (131 MB take 26 us at the rate of a copy): the lookup and the two chains are 5.2 instructions per weight, four in seven of
-// them of half rate (v_perm; fma, and, or, add, shifts right are of full rate), so what counts is that every SIMD always has a wave that can issue and that nothing else is issued.  One workgroup of 16 waves to a CU,
+// them of half rate (v_perm; fma, and, or, add, shifts right are of full rate), so what counts is that a SIMD has a wave that can issue and that nothing else is issued.  One workgroup of 16 waves to a CU,
 // which takes an even share of the row slots: x is normed, widened and staged once per CU instead of once per four waves and eight to sixteen slots; waves take slots in turn, four blocks in flight through the
 // slots' ends (six, or 24 waves to a CU: no difference); a block column's 32 activations lie side by side in LDS (nine 16-byte pieces apart: 16 lanes' equal pieces in different banks), so one address serves a block's
 // eight reads; the quad exchanges its table through the LDS crossbar; no masks (rows and columns divide evenly, or the kernel above takes the matrix).  Same chains, same tree, same bits.  us, the kernel above | this
 // one: gate and up 25600 x 5120 63.2 | 50.2, 5120 x 25600 38.1 | 28.9, 5120 x 8192 14.6 | 11.2, 8192 + 1024 + 1024 x 5120 18.0 | 15.9.
+// Counted, vector instructions a cycle of a CU that has a wave: 0.92, 0.73, 0.63, 0.62 of these.  Slots are dealt whole: 5120 x 25600 is ten of them for a workgroup's sixteen waves, three on two of the SIMDs and two on the
+// others, which run out (at most 0.83 of the longest); 20 slots of four and five steps (the last two) leave the second turn to one wave a SIMD, beside the staging of x.
 constexpr int GQ_WAVES = 16, GQ_RING = 4, GQ_XCH = 4; /* GQ_XCH x 1024 threads x 8 elements: the longest x */
 template <bool PAIRED, bool ONEJOB>
 __global__ void __launch_bounds__(64 * GQ_WAVES) gemv_q4_kernel(const GemvArgs a) {
