@@ -985,11 +985,11 @@ def xcd_replicas(m, cfg, forced, timed_positions, warmup, n_seq, ids_main, jump=
     K = len(timed_positions)
     first = timed_positions[0]
     traffic, traffic_src, valu = None, None, None
-    try:   # counter passes of scratch/gpu_r05_profile.sh / gpu_r06_pmc.sh (not re-collected by this run: --pmc around bench.py itself crashes the profiler on this pool)
+    try:   # counter passes around scratch/ub_xengine.py (not re-collected by this run: a --pmc pass slows it many times over)
         if cfg["dim"] != 1024:
             raise KeyError("the passes were taken on Qwen3-0.6B")
         ns = 32 if n_seq > 16 else (16 if n_seq > 8 else 8)
-        pf = "r06_pmc_xengine_%d.json" % ns if ns > 8 else "r05_pmc_xengine_8.json"
+        pf = "pmc_xengine_%d.json" % ns
         pj = json.load(open(os.path.join(ROOT, "profiles", pf)))
         traffic = int(pj["hbm_bytes_per_launch"] / (ns * 4))
         traffic_src = "profiles/%s: FETCH_SIZE / WRITE_SIZE passes of scratch/ub_xengine.py (4 steps per launch at positions 2037..2040), per sequence and step" % pf
