@@ -286,7 +286,7 @@ def main():
                     out["cpu_baseline"] = {"error": repr(e)[:300]}
             if args.lean_xcd > 0 and world == 1:
                 try:
-                    out["xcd_replicas"] = xcd_replicas(m, cfg, forced, timed_positions, W, args.lean_xcd, ids_timed_run, jump=args.jump)
+                    out["xcd_replicas"] = xcd_replicas(m, cfg, forced, timed_positions, W, args.lean_xcd, ids_timed_run, jump=args.jump, counted=args.layers == "q4" and args.sparse == 0.0)
                 except Exception as e:
                     out["xcd_replicas"] = {"error": repr(e)[:300]}
             if args.lean_prefill > 0 and world == 1:
@@ -971,7 +971,7 @@ def concurrent_streams(cfg, layer_type, head_type, dev, S, forced, n_prompt, mea
             "note": "independent decoders, separate weight copies and HIP streams, positions %d..%d each" % (n_prompt, S_len - 1)}
 
 
-def xcd_replicas(m, cfg, forced, timed_positions, warmup, n_seq, ids_main, jump=False, queue=False):
+def xcd_replicas(m, cfg, forced, timed_positions, warmup, n_seq, ids_main, jump=False, queue=False, counted=True):
     """The chip's aggregate rate on INDEPENDENT sequences (never `value`, which stays the single-sequence rate): n_seq decoders inside one launch, one per XCD (32 workgroups
     each, every hand-off in that XCD's L2: koifish_amd/csrc/kf_xengine.hip), sharing this model's weights; own K / V cache, state, prompt and logits per sequence.  The
     reference decodes one sequence per process (GoPT.cpp:1139-1180) and scales a small model with more processes -- these are the processes, moved inside the package.
@@ -986,8 +986,8 @@ def xcd_replicas(m, cfg, forced, timed_positions, warmup, n_seq, ids_main, jump=
     first = timed_positions[0]
     traffic, traffic_src, valu = None, None, None
     try:   # counter passes around scratch/ub_xengine.py (not re-collected by this run: a --pmc pass slows it many times over)
-        if cfg["dim"] != 1024:
-            raise KeyError("the passes were taken on Qwen3-0.6B")
+        if cfg["dim"] != 1024 or not counted:
+            raise KeyError("the passes were taken on Qwen3-0.6B with 4-bit layers, all rows")
         ns = 32 if n_seq > 16 else (16 if n_seq > 8 else 8)
         pf = "pmc_xengine_%d.json" % ns
         pj = json.load(open(os.path.join(ROOT, "profiles", pf)))
