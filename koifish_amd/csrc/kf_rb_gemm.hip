@@ -22,6 +22,24 @@ __device__ __forceinline__ void rb_st8(float* base, size_t off, const float (&v)
     reinterpret_cast<f32x4*>(base + off)[0] = f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(base + off)[1] = f32x4{v[4], v[5], v[6], v[7]};
 }
 
+// The list's tiles up to the last that holds pairs: those at its end are empty (-1).  Only these are dealt to the XCDs, in equal runs of neighbours; dealt with the others an XCD that the list's end falls to, once per band of row tiles,
+// has little to do.  us, 128 experts of 15768 pairs, about 300 of 374 tiles filled, dealt all | filled: gated 1536 x 2048 252 | 220 (1.08 GB from memory, 0.8 of it weights: 4.9 TB/s), 2048 x 768 145 | 131; bands of all 12 or 16 row tiles
+// instead of g3_tile's, the token rows read once by an XCD, 229 and 131; bands of 4 the same as of 6 and 8.
+__device__ __forceinline__ int rb_filled(const int32_t* tile_expert, int n, int lane) {
+    int c = 0;
+    for (int i0 = 0; i0 < n; i0 += 512) {
+        int v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = tile_expert[i0 + 64 * j + lane < n ? i0 + 64 * j + lane : 0];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const unsigned long long b = __ballot(i0 + 64 * j + lane < n && v[j] >= 0);
+            if (b) c = i0 + 64 * j + 64 - __builtin_clzll(b);
+        }
+    }
+    return c;
+}
+
 // T: the storage, uint16_t (bf16: weights in MFMA tiles) or float (true 32-bit: weights in rows)
 template <class C, bool EXPERTS, class T>
 __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_kernel(const RbProduct q) {
@@ -30,8 +48,15 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
     const kf_rb_product& p = q.p;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int nbx = (p.m + C::BM - 1) / C::BM;
-    int bx, by;
-    g3_tile(g3_remap(blockIdx.x, gridDim.x), nbx, (int)gridDim.x / nbx, bx, by);
+    int bx, by, ex = 0;
+    if constexpr (EXPERTS) {
+        const int n_act = rb_filled(q.e.tile_expert, (int)gridDim.x / nbx, lane);
+        if ((int)blockIdx.x / 8 >= (nbx * n_act + 7 - (int)blockIdx.x % 8) / 8) return; /* workgroup-uniform */
+        g3_tile(g3_remap(blockIdx.x, nbx * n_act), nbx, n_act, bx, by);
+        ex = q.e.tile_expert[by];
+        if (ex < 0) return; /* workgroup-uniform */
+    } else
+        g3_tile(g3_remap(blockIdx.x, gridDim.x), nbx, (int)gridDim.x / nbx, bx, by);
     const int m0 = bx * C::BM, t0 = by * C::BN;
     GemmArgs a; /* what the main loop reads */
     constexpr int U = sizeof(T) / 2, KT = G3_BK / U; /* 16-bit units of an element, elements of a step */
@@ -42,8 +67,6 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) rb_gemm_ker
 #pragma unroll
         for (int j = 0; j < C::NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (EXPERTS) {
-        const int ex = q.e.tile_expert[by];
-        if (ex < 0) return; /* workgroup-uniform */
         a.w += (size_t)ex * q.e.w_stride * sizeof(T);
         for (int i = tid; i < C::BN; i += C::NTH) {
             const int pair = q.e.list[(size_t)by * C::BN + i];

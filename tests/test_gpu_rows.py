@@ -276,6 +276,28 @@ def test_experts(ctx, kind, n, E, top, tile):
         assert rc == 0 and np.abs(f64(z) - (1.25 * f64(res) + y.reshape(n, top, C_).sum(1))).max() < 2e-5
 
 
+# few and many row tiles, filled tiles in front of, behind and far behind empty ones, none at all
+@pytest.mark.parametrize("m", [64, 448, 1600])
+@pytest.mark.parametrize("filled", [(0,), (1, 3), (0, 2, 511, 512, 530), (7, 599), ()])
+def test_tiles_of_experts_among_empty_ones(ctx, kind, m, filled):
+    typ, dt, tol = kind
+    E, tile, k, nt, g = 3, 64, 128, 600, torch.Generator().manual_seed(m)
+    n = 65 + sum(1 + 9 * i for i in range(len(filled)))   # (more than 64 rows: not a decode batch)
+    w, x = dev(torch.randn(E, m, k, generator=g) / k ** 0.5, dt), dev(torch.randn(n, k, generator=g), dt)
+    ws, y = stored(w), torch.full((n, m), 3.0, dtype=dt, device="cuda")
+    e, b = experts_of(n, E, 1, tile, m * k)
+    te, li, ref, at = torch.full((nt,), -1, dtype=torch.int32), torch.full((nt, tile), -1, dtype=torch.int32), np.full((n, m), 3.0), 0
+    for i, t in enumerate(filled):
+        te[t], li[t, :1 + 9 * i] = i % E, torch.arange(at, at + 1 + 9 * i, dtype=torch.int32)
+        ref[at:at + 1 + 9 * i] = f64(x)[at:at + 1 + 9 * i] @ f64(w)[i % E].T
+        at += 1 + 9 * i
+    te, li = te.cuda(), li.cuda()
+    e.n_tile, e.tile_expert, e.list = nt, te.data_ptr(), li.data_ptr()
+    p = L.RbProduct(ws.data_ptr(), x.data_ptr(), y.data_ptr(), None, k, m, 0, typ, m, k, n, L.RB_STORE, 0, L.RB_DOWN, 0.0, C.pointer(e))
+    L.check(ctx.hip.kf_rb_linear(ctx.h, C.byref(p)))
+    assert np.abs(f64(y) - ref).max() < tol * 4   # as test_experts': a bf16 rounding of values up to 4
+
+
 @pytest.mark.parametrize("n", [1, 20])  # one block of columns, two
 @pytest.mark.parametrize("at", [63, 191])  # the last k of a wave's two steps (it multiplies in fours), the last of all
 @pytest.mark.parametrize("what", ["weight", "token"])
