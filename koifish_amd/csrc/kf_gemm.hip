@@ -58,6 +58,11 @@ struct WTile<FMT_Q4, KS> {
         const float s = in[p] ? bf2f(st[p]) : 0.f, z = in[p] ? bf2f(ze[p]) : 0.f;
         return frag_q4(D, s, s * 0.0625f, -a.qBias * s, z);
     }
+    __device__ __forceinline__ void table(PermLut& t, const GemmArgs& a) const { /* KS 2: the block's */
+        const float s = in[0] ? bf2f(st[0]) : 0.f, z = in[0] ? bf2f(ze[0]) : 0.f;
+        build_perm_lut(t, s, z, -a.qBias * s);
+    }
+    __device__ __forceinline__ u32x4 frag_t(int sl, const PermLut& t) const { return frag_q4t(sl == 0 ? b[0].w : (sl == 1 ? b[0].z : (sl == 2 ? b[0].y : b[0].x)), t); }
 };
 // 4-bit row codebook: the same block ranges as the Packed128 form; the row's 16-entry table rides along (two 16-byte loads through the cache)
 template <int KS>
@@ -418,9 +423,36 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
         if constexpr (XL) return *reinterpret_cast<const u32x4*>(xs + slot * XG + (tb * 32 + r) * 256 + (((WTile<FMT, 2>::koff(sl, h, j) >> 3) ^ (r & 15)) << 4));
         else return g.x[j][sl][tb];
     };
+    // 4-bit: the weights come from a table of their quantisation group's 16, one for both units of a group of columns where these lie in one.  Two tables at a time (PAIRED), or the registers that the rows' fragments take
+    // without LDS, leave one workgroup to a CU where there were two (gate and up 3072 x 1024, 128 rows: 12.2 -> 14.6 us): these keep the arithmetic form.  us a prompt of 28 layers of 1024 x 2048 and 1024 x 3072, so | by
+    // the table: 24 rows 1475 | 1438, 128 rows 1786 | 1760, 319 rows 3032 | 2964
+    constexpr bool TABLE = FMT == FMT_Q4 && !PAIRED && XL;
+    const bool one_table = a.gshift >= 2 && (a.nBlk & 3) == 0;
+    [[maybe_unused]] PermLut lut, lut2;
+    auto wfrag = [&](const WTile<FMT, 2>& w, [[maybe_unused]] PermLut& t, const GemmArgs& m, int j, int sl, int ks) {
+        if constexpr (TABLE) {
+            if (sl == 0 && (j == 0 || !one_table)) w.table(t, m);
+            return w.frag_t(sl, t);
+        } else
+            return get_frag<FMT, 2>(w, sl, m, ks);
+    };
     Group gc, gn;
     int u0 = wave * UPG, slot = 0;
     if (u0 < nunit) gload(u0, gc, 0);
+    // the residual's values for this thread's two rows of a token, behind the first loads: asked for in the epilogue they are a memory latency of their own (us, the prompts above: 128 rows 1822 | 1786, 16 rows 1446 | 1421)
+    constexpr int RPW = 16 / NW; /* registers per wave */
+    static_assert(NW == 8 || NW == 4, "registers per wave: pairs of adjacent rows");
+    const bool res_early = !PAIRED && a.residual && ((a.ldr | a.M) & 1) == 0 && (reinterpret_cast<uintptr_t>(a.residual) & 3) == 0;
+    uint32_t res[TB][RPW / 2];
+    if (res_early) {
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+            for (int q = 0; q < RPW; q += 2) {
+                const int i0 = wave * RPW + q, rg = row_base + 8 * (i0 >> 2) + 4 * h + (i0 & 3), tok = tok0 + tb * 32 + r;
+                res[tb][q / 2] = *reinterpret_cast<const uint32_t*>(a.residual + (size_t)(tok < a.n ? tok : a.n - 1) * a.ldr + (rg < a.M ? rg : 0));
+            }
+    }
     for (; u0 < nunit; u0 += NW * UPG) {
         const bool more = u0 + NW * UPG < nunit;
         if (more) gload(u0 + NW * UPG, gn, slot ^ 1);
@@ -432,7 +464,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
             if (u0 + j < nunit) {
 #pragma unroll
                 for (int sl = 0; sl < 4; sl++) {
-                    const bf16x8 A = __builtin_bit_cast(bf16x8, get_frag<FMT, 2>(gc.w[j], sl, a, (u0 + j) & 1));
+                    const bf16x8 A = __builtin_bit_cast(bf16x8, wfrag(gc.w[j], lut, a, j, sl, (u0 + j) & 1));
                     u32x4 X[TB];
 #pragma unroll
                     for (int tb = 0; tb < TB; tb++) X[tb] = xfrag(gc, slot, j, sl, tb);
@@ -440,7 +472,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
                     for (int tb = 0; tb < TB; tb++)
                         acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(bf16x8, X[tb]), acc[tb], 0, 0, 0);
                     if (PAIRED) {
-                        const bf16x8 A2 = __builtin_bit_cast(bf16x8, get_frag<FMT, 2>(gc.w2[j], sl, b, (u0 + j) & 1));
+                        const bf16x8 A2 = __builtin_bit_cast(bf16x8, wfrag(gc.w2[j], lut2, b, j, sl, (u0 + j) & 1));
 #pragma unroll
                         for (int tb = 0; tb < TB; tb++)
                             acc2[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A2, __builtin_bit_cast(bf16x8, X[tb]), acc2[tb], 0, 0, 0);
@@ -455,8 +487,6 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     // fixed-order sum over the k-slices, ((w0 + w1) + w2) + ..., and the epilogue, spread over the waves: every wave leaves its 16 sums per token block in LDS and
     // wave w adds and stores accumulator registers 16 w / NW .. (two adjacent output rows per lane with 8 waves) -- the same additions in the same order as one wave
     // doing all of it, at an eighth of the serial work behind the barrier (measured on the 0.6B shapes at 128 tokens: reduce 0.65 us + epilogue 1.3-1.7 us by wave 0)
-    constexpr int RPW = 16 / NW; /* registers per wave */
-    static_assert(NW == 8 || NW == 4, "registers per wave: pairs of adjacent rows");
 #pragma unroll
     for (int tb = 0; tb < TB; tb++)
 #pragma unroll
@@ -496,7 +526,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
                     if (a.beta != 0.0f) x = x + a.beta * bf2f(yp[j]);
                     if (a.bias) x = x + bf2f(a.bias[rg + j]);
                     uint16_t qv = f2bf(x);
-                    if (a.residual) qv = f2bf(bf2f(a.residual[(size_t)tok * a.ldr + rg + j]) + bf2f(qv));
+                    if (res_early) qv = f2bf((j ? bf_hi(res[tb][q / 2]) : bf_lo(res[tb][q / 2])) + bf2f(qv));
+                    else if (a.residual) qv = f2bf(bf2f(a.residual[(size_t)tok * a.ldr + rg + j]) + bf2f(qv));
                     o[j] = qv;
                 } else { /* act = silu(gate) * up on the bf16-rounded gate / up (Relu::Forw SWIG, Activation.cu:85-93; the expression of kf_swiglu) */
                     const float g = round_bf16(v[j]), u = round_bf16(v2[j]);

@@ -486,3 +486,23 @@ def test_rows_of_small_batches_do_not_depend_on_their_way(ctx, kind, M, K):
         assert torch.equal(out[:n].view(torch.int16), y[40][:n].view(torch.int16)) and bool((out[n] == 0).all()), n
     ref = x.float() @ ctx.dequant(w).float().reshape(M, K).t()
     assert float((y[40][:40].float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("M,K", [(64, 128), (34, 192), (33, 1600), (96, 2048)])
+def test_tables_of_4_bit_groups_and_the_residual_of_a_small_batch(ctx, M, K, group):
+    """groups of one, two and four blocks, rows whose groups begin in the row before, odd and even rows: 20 rows by way of LDS (weights from tables, the residual loaded early where rows pair) equal 16 read as
+    fragments (arithmetic) bit for bit, and the product in 32 bits to a bf16 rounding of the sum and one of the residual's"""
+    if M * K % group:
+        pytest.skip("whole groups only")
+    w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4, lGroup=group)
+    x, res, d = torch.randn(20, K, device=ctx.device).bfloat16(), torch.randn(20, M, device=ctx.device).bfloat16(), w.desc()
+    ref = x.float() @ ctx.dequant(w).float().reshape(M, K).t()
+    for r in (None, res):
+        y = {n: torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16) for n in (16, 20)}
+        for n, out in y.items():
+            assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), out.data_ptr(), None, n, 1.0, 0.0, 0 if r is None else 1, None if r is None else r.data_ptr()) == 0, ctx.hip.kf_last_error()
+        ctx.sync()
+        assert torch.equal(y[16].view(torch.int16), y[20][:16].view(torch.int16))
+        want = ref if r is None else ref + res.float()
+        assert float((y[20].float() - want).abs().max()) <= 2.0 ** -8 * (float(ref.abs().max()) + float(want.abs().max()))
