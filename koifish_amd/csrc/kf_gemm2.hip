@@ -51,18 +51,19 @@ __global__ void __launch_bounds__(512) gemm2_kernel(const GemmArgs a) {
         auto issue = [&](int kt, int q) { /* tile kt (clamped to the last one) -> register set q */
             if (kt >= nkt) kt = nkt - 1;
             const int e0 = kt * G2_BK + whalf * 32; /* first element of this thread's 32 */
+            // (plain loads, as in kf_gemm.hip: a thread's piece is 16 bytes to 64 of a line.  us a prompt of six layers of the 32B shape in 4 bits, with the non-temporal hint | without: 256 rows 4820 | 4668, 319 rows 6556 | 6184)
             if constexpr (FMT == FMT_Q4) {
                 const uint32_t bidx = (uint32_t)wrow * (uint32_t)a.nBlk + (uint32_t)(e0 >> 5);
-                wreg[q][0] = ld_nt(reinterpret_cast<const u32x4*>(a.w) + bidx);
+                wreg[q][0] = reinterpret_cast<const u32x4*>(a.w)[bidx];
                 const uint32_t gi = bidx >> a.gshift;
                 wst[q] = a.step[gi], wze[q] = a.zero[gi];
             } else if constexpr (FMT == FMT_BF16) {
                 const u32x4* src = reinterpret_cast<const u32x4*>(a.w + ((size_t)wrow * a.K + e0) * 2);
 #pragma unroll
-                for (int c = 0; c < 4; c++) wreg[q][c] = ld_nt(src + c);
+                for (int c = 0; c < 4; c++) wreg[q][c] = src[c];
             } else { /* f8e5m2: 32 bytes */
                 const u32x4* src = reinterpret_cast<const u32x4*>(a.w + (size_t)wrow * a.K + e0);
-                wreg[q][0] = ld_nt(src), wreg[q][1] = ld_nt(src + 1);
+                wreg[q][0] = src[0], wreg[q][1] = src[1];
             }
 #pragma unroll
             for (int i = 0; i < 8; i++) {
