@@ -547,6 +547,142 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     }
 }
 
+// The same for 4-bit matrices of which blocks of 32 rows are too few workgroups: 16 rows a workgroup, twice as many of them, each with half of the unpacking.  v_mfma_f32_16x16x32_bf16 adds up a step's 32 products as
+// two v_mfma_f32_32x32x16_bf16 do one behind the other (the same bits, compared over 10^8 sums), so lane group q holds what lane half q & 1 holds there in step 2 m + (q >> 1).
+template <int TB, bool PAIRED>
+__global__ void __launch_bounds__(512) gemm_direct16_kernel(const GemmArgs a0, int slots) {
+    constexpr int NW = 8, UPG = 2, XG = TB * 16 * 256;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    float* const red = reinterpret_cast<float*>(smem_raw); /* [PAIRED ? 2 : 1][NW][TB][4][64] */
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, q = lane >> 4, h = q & 1, hi = q >> 1;
+    GemmArgs a = a0, b = a0;
+    int rb = blockIdx.x; /* 16-row blocks, one job's behind another's */
+    if (!PAIRED && a0.njobs > 1 && rb >= 2 * a0.rb_end[0]) {
+        const int j = a0.njobs > 2 && rb >= 2 * a0.rb_end[1] ? 1 : 0;
+        rb -= 2 * (j ? a0.rb_end[1] : a0.rb_end[0]);
+        a.w = j ? a0.xw[1] : a0.xw[0], a.zero = j ? a0.xzero[1] : a0.xzero[0], a.step = j ? a0.xstep[1] : a0.xstep[0], a.qBias = j ? a0.xqBias[1] : a0.xqBias[0];
+        a.M = j ? a0.xM[1] : a0.xM[0], a.y = j ? a0.xy[1] : a0.xy[0], a.ldy = j ? a0.xldy[1] : a0.xldy[0];
+    }
+    if (PAIRED) b.w = a0.xw[0], b.zero = a0.xzero[0], b.step = a0.xstep[0], b.qBias = a0.xqBias[0];
+    const int row0 = rb * 16, tok0 = blockIdx.y * (TB * 16), nunit = a.K / 64, row = row0 + r < a.M ? row0 + r : a.M - 1;
+    unsigned char* const xs = smem_raw + wave * slots * XG;
+    const uint32_t ldb = (uint32_t)a.ldx * 2;
+    struct Group {
+        WTile<FMT_Q4, 2> w[UPG], w2[PAIRED ? UPG : 1];
+    };
+    auto gload = [&](int u0, Group& g, int slot) { /* as gemm_direct_kernel's: the token rows first, whole lines to this wave's own LDS; units past the end repeat the last one */
+#ifdef __HIP_DEVICE_COMPILE__
+        const long long left = ((long long)a.n - tok0) * ldb - (long long)u0 * 128;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x) + (size_t)tok0 * a.ldx + (size_t)u0 * 64, 0, (int)(left < 0x7FFFFFFFll ? left : 0x7FFFFFFFll), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < TB * 4; i++) {
+            const int t = 4 * i + q;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(xs + slot * XG + i * 1024), 16, (uint32_t)t * ldb + ((r ^ (t & 15)) << 4), 0, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+#endif
+#pragma unroll
+        for (int j = 0; j < UPG; j++) {
+            const int u = u0 + j < nunit ? u0 + j : nunit - 1;
+            g.w[j].load(a, row, u >> 1, h, u & 1);
+            if (PAIRED) g.w2[j].load(b, row, u >> 1, h, u & 1);
+        }
+    };
+    f32x4 acc[TB], acc2[PAIRED ? TB : 1];
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++) {
+        acc[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (PAIRED) acc2[tb] = acc[tb];
+    }
+    const bool one_table = a.gshift >= 2 && (a.nBlk & 3) == 0;
+    PermLut lut, lut2;
+    auto frag = [&](const WTile<FMT_Q4, 2>& w, const PermLut& t, int m) { return __builtin_bit_cast(bf16x8, frag_q4t(m == 0 ? (hi ? w.b[0].z : w.b[0].w) : (hi ? w.b[0].x : w.b[0].y), t)); };
+    Group gc, gn;
+    int u0 = wave * UPG, slot = 0;
+    if (u0 < nunit) gload(u0, gc, 0);
+    // the first TB * 2 waves store: two rows (2 p, 2 p + 1 of a lane group's four) of a token a thread; their residual sets out behind the first loads
+    const int otb = wave >> 1, orow = row0 + 4 * q + 2 * (wave & 1), otok = tok0 + otb * 16 + r;
+    const bool stores = wave < 2 * TB, res_early = !PAIRED && a.residual && ((a.ldr | a.M) & 1) == 0 && (reinterpret_cast<uintptr_t>(a.residual) & 3) == 0;
+    uint32_t res = 0;
+    if (res_early && stores) res = *reinterpret_cast<const uint32_t*>(a.residual + (size_t)(otok < a.n ? otok : a.n - 1) * a.ldr + (orow < a.M ? orow : 0));
+    for (; u0 < nunit; u0 += NW * UPG) {
+        const bool more = u0 + NW * UPG < nunit;
+        if (more) gload(u0 + NW * UPG, gn, slot ^ 1);
+        asm volatile("" ::"v"(gm_first(gc.w[0].b)) : "memory"); /* a weight of the group has come: its token rows have */
+#pragma unroll
+        for (int j = 0; j < UPG; j++) {
+            if (u0 + j < nunit) {
+                if (j == 0 || !one_table) {
+                    gc.w[j].table(lut, a);
+                    if (PAIRED) gc.w2[j].table(lut2, b);
+                }
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    bf16x8 X[TB];
+#pragma unroll
+                    for (int tb = 0; tb < TB; tb++) X[tb] = *reinterpret_cast<const bf16x8*>(xs + slot * XG + (tb * 16 + r) * 256 + ((((2 * j + h) * 4 + 2 * m + hi) ^ r) << 4));
+                    const bf16x8 A = frag(gc.w[j], lut, m);
+#pragma unroll
+                    for (int tb = 0; tb < TB; tb++) acc[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, X[tb], acc[tb], 0, 0, 0);
+                    if constexpr (PAIRED) {
+                        const bf16x8 A2 = frag(gc.w2[j], lut2, m);
+#pragma unroll
+                        for (int tb = 0; tb < TB; tb++) acc2[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A2, X[tb], acc2[tb], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        if (more) gc = gn;
+        slot ^= 1;
+    }
+    __syncthreads(); /* the sums go where the token rows were */
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            red[((wave * TB + tb) * 4 + i) * 64 + lane] = acc[tb][i];
+            if (PAIRED) red[(((NW + wave) * TB + tb) * 4 + i) * 64 + lane] = acc2[tb][i];
+        }
+    __syncthreads();
+    if (!stores || otok >= a.n || orow >= a.M) return;
+    float v[2], v2[2];
+#pragma unroll
+    for (int w = 0; w < NW; w++) /* ((w0 + w1) + w2) + ... */
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float p = red[((w * TB + otb) * 4 + 2 * (wave & 1) + j) * 64 + lane];
+            v[j] = w == 0 ? p : v[j] + p;
+            if (PAIRED) {
+                const float p2 = red[(((NW + w) * TB + otb) * 4 + 2 * (wave & 1) + j) * 64 + lane];
+                v2[j] = w == 0 ? p2 : v2[j] + p2;
+            }
+        }
+    uint16_t* const yp = a.y + (size_t)otok * a.ldy + orow;
+    uint16_t o[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (orow + j >= a.M) continue;
+        if (!PAIRED) { /* gemm_epilogue's expression */
+            float x = v[j];
+            if (a.alpha != 1.0f) x = a.alpha * x;
+            if (a.beta != 0.0f) x = x + a.beta * bf2f(yp[j]);
+            if (a.bias) x = x + bf2f(a.bias[orow + j]);
+            uint16_t qv = f2bf(x);
+            if (res_early) qv = f2bf((j ? bf_hi(res) : bf_lo(res)) + bf2f(qv));
+            else if (a.residual) qv = f2bf(bf2f(a.residual[(size_t)otok * a.ldr + orow + j]) + bf2f(qv));
+            o[j] = qv;
+        } else { /* act = silu(gate) * up, as in gemm_direct_kernel */
+            const float g = round_bf16(v[j]), u = round_bf16(v2[j]);
+            o[j] = f2bf((g * u) / (1.0f + kf_expf(-g)));
+        }
+    }
+    if (((a.ldy & 1) == 0) && ((reinterpret_cast<uintptr_t>(a.y) & 3) == 0) && orow + 1 < a.M) *reinterpret_cast<uint32_t*>(yp) = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+    else {
+        yp[0] = o[0];
+        if (orow + 1 < a.M) yp[1] = o[1];
+    }
+}
+
 static int gm_fmt_of(int type) {
     switch (type) {
         case KF_BF16: return FMT_BF16;
@@ -574,8 +710,26 @@ static bool gd_rows_by_lds(const GemmArgs& a, long wgs) {
     constexpr bool unpacks = FMT == FMT_Q4 || FMT == FMT_Q2 || FMT == FMT_Q1;
     return !(unpacks && a.K > GD_NW * GD_UPG * 64 && (a.K < 2048 || (a.K < 3072 && wgs > 768)));
 }
+template <int TB, bool PAIRED>
+static void gm_direct16(const GemmArgs& a, int nrb, hipStream_t st) {
+    const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1;
+    const size_t sums = (size_t)8 * (PAIRED ? 2 : 1) * TB * 4 * 64 * 4, rows = (size_t)8 * slots * TB * 16 * 256;
+    static int attr_set = 0;
+    if (!attr_set) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_direct16_kernel<TB, PAIRED>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024), attr_set = 1;
+    hipLaunchKernelGGL((gemm_direct16_kernel<TB, PAIRED>), dim3(2 * nrb, (a.n + 16 * TB - 1) / (16 * TB)), dim3(512), rows > sums ? rows : sums, st, a, slots);
+}
 template <int FMT, int TB, bool PAIRED>
 static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
+    if constexpr (FMT == FMT_Q4 && TB == 1) {
+        // 16 weight rows a workgroup where that makes no more than one of them for a CU, and then 16 token rows instead of 32 where it still does: a workgroup's time is its unpacking and the token rows that it takes in.
+        // us a 0.6B prompt, 32 weight rows | 16 from 64 | 128 | 192 workgroups of 32 down: 16 token rows 1414 | 1282 | 1219 | 1230, 32 1449 | 1396 | 1355 | 1374, 128 1741 | 1737 | 1693 | 1700; 1.7B, 16 rows 2107 | 1862 |
+        // 1805 | 1903; with 32 token rows always | 16 up to 128 | 256 | 512 workgroups: 24 rows 1346 | 1280 | 1269 | 1311, 64 rows 1486 | 1481 | 1397 | 1400, 128 rows 1704 | 1698 | 1694 | 1808
+        if ((long)grid.x * grid.y <= 128 && a.ldx < (1 << 24)) {
+            if (a.n <= 16 || 2l * grid.x * ((a.n + 15) / 16) <= 256) gm_direct16<1, PAIRED>(a, (int)grid.x, st);
+            else gm_direct16<2, PAIRED>(a, (int)grid.x, st);
+            return;
+        }
+    }
     const size_t sums = (size_t)GD_NW * (PAIRED ? 2 : 1) * TB * 16 * 64 * 4;
     const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1; /* one group of a wave, or two in turn */
     const size_t rows = (size_t)GD_NW * slots * TB * 32 * 256;

@@ -506,3 +506,33 @@ def test_tables_of_4_bit_groups_and_the_residual_of_a_small_batch(ctx, M, K, gro
         assert torch.equal(y[16].view(torch.int16), y[20][:16].view(torch.int16))
         want = ref if r is None else ref + res.float()
         assert float((y[20].float() - want).abs().max()) <= 2.0 ** -8 * (float(ref.abs().max()) + float(want.abs().max()))
+
+
+@pytest.mark.parametrize("K", [128, 192, 1024, 2048, 3072])
+@pytest.mark.parametrize("n,M", [(8, 4096), (16, 4096), (17, 2048), (32, 4096), (33, 1024), (50, 2048), (100, 1024)])
+def test_blocks_of_16_and_of_32_weight_rows_give_the_same_bits(ctx, n, M, K):
+    """4-bit products whose 32-row blocks are at most 128 workgroups go in blocks of 16 rows, by 16 or 32 token rows: their rows are the first ones of a taller product that does not, one by one, three stacked and as gate | up"""
+    tall = M + 32 if M * ((n + 31) // 32) >= 4096 else 4096 // ((n + 31) // 32) // 32 * 32 + 64
+    assert (M // 32) * ((n + 31) // 32) <= 128 < (tall // 32) * ((n + 31) // 32)
+    g = torch.Generator(device=ctx.device).manual_seed(n + K)
+    x = torch.randn(n, K, device=ctx.device, generator=g).bfloat16()
+    W = [(torch.randn(tall, K, device=ctx.device, generator=g) * 0.05).bfloat16() for _ in range(2)]
+    big, small = [ctx.quantize(w, L.Q4) for w in W], [ctx.quantize(w[:M].contiguous(), L.Q4) for w in W]
+    y = {}
+    for rows, ws in ((tall, big), (M, small)):
+        d, res, out = [w.desc() for w in ws], torch.ones(n, rows, device=ctx.device).bfloat16(), [torch.zeros(n, rows, device=ctx.device, dtype=torch.bfloat16) for _ in range(4)]
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d[0]), x.data_ptr(), out[0].data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d[1]), x.data_ptr(), out[1].data_ptr(), None, n, 1.0, 0.0, 1, res.data_ptr()) == 0, ctx.hip.kf_last_error()
+        assert ctx.hip.kf_gateup_swiglu_batch(ctx.h, C.byref(d[0]), C.byref(d[1]), x.data_ptr(), out[2].data_ptr(), out[3].data_ptr(), n) == 0, ctx.hip.kf_last_error()
+        ctx.sync()
+        y[rows] = out
+    for a, b in zip(y[tall][:3], y[M][:3]):
+        assert torch.equal(a[:, :M].contiguous().view(torch.int16), b.view(torch.int16)) and float(b.float().abs().max()) > 0
+    # three matrices of a launch: 32 + 16 + 16 blocks of 32 rows at most
+    part = [ctx.quantize(W[0][:r].contiguous(), L.Q4) for r in (256, 96, 64)]
+    d, out = [w.desc() for w in part], [torch.zeros(n, r, device=ctx.device, dtype=torch.bfloat16) for r in (256, 96, 64)]
+    ws, ys = (C.POINTER(L.Weight) * 3)(*[C.pointer(v) for v in d]), (C.c_void_p * 3)(*[t.data_ptr() for t in out])
+    assert ctx.hip.kf_linear_multi(ctx.h, 3, ws, x.data_ptr(), ys, n) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    for t in out:
+        assert torch.equal(t.view(torch.int16), y[tall][0][:, :t.shape[1]].contiguous().view(torch.int16))
