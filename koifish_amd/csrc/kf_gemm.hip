@@ -403,8 +403,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
         asm volatile("" ::: "memory");
 #endif
     };
-    auto gload = [&](int u0, Group& g, int slot) { /* units u0 .. u0+UPG-1; units past the end repeat the last one and are skipped in the arithmetic */
-        if constexpr (XL) xload(u0, slot);
+    auto gload = [&](int u0, Group& g, int slot, bool rows) { /* units u0 .. u0+UPG-1; units past the end repeat the last one and are skipped in the arithmetic */
+        if constexpr (XL)
+            if (rows) xload(u0, slot);
 #pragma unroll
         for (int j = 0; j < UPG; j++) {
             int u = u0 + j;
@@ -441,7 +442,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     };
     Group gc, gn;
     int u0 = wave * UPG, slot = 0;
-    if (u0 < nunit) gload(u0, gc, 0);
+    if (u0 < nunit) gload(u0, gc, 0, true);
     // the residual's values for this thread's two rows of a token, behind the first loads: asked for in the epilogue they are a memory latency of their own (us, the prompts above: 128 rows 1822 | 1786, 16 rows 1446 | 1421)
     constexpr int RPW = 16 / NW; /* registers per wave */
     static_assert(NW == 8 || NW == 4, "registers per wave: pairs of adjacent rows");
@@ -458,9 +459,10 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     }
     for (; u0 < nunit; u0 += NW * UPG) {
         const bool more = u0 + NW * UPG < nunit;
-        if (more) gload(u0 + NW * UPG, gn, slot ^ 1);
+        if (more) gload(u0 + NW * UPG, gn, XL && slots == 1 ? 0 : slot ^ 1, !XL || slots == 2);
         if constexpr (XL) { /* a weight of the group has come: its token rows have */
-            asm volatile("" ::"v"(gm_first(gc.w[0].b)) : "memory");
+            if (slots == 1 && u0 >= NW * UPG) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* (these set out behind it) */
+            else asm volatile("" ::"v"(gm_first(gc.w[0].b)) : "memory");
         }
 #pragma unroll
         for (int j = 0; j < UPG; j++) {
@@ -483,8 +485,11 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
                 }
             }
         }
+        if (XL && slots == 1) {
+            if (more) xload(u0 + NW * UPG, 0);
+        } else
+            slot ^= 1;
         if (more) gc = gn;
-        slot ^= 1;
     }
     if constexpr (XL) __syncthreads(); /* the sums go where the token rows were */
     // fixed-order sum over the k-slices, ((w0 + w1) + w2) + ..., and the epilogue, spread over the waves: every wave leaves its 16 sums per token block in LDS and
@@ -697,19 +702,15 @@ static int gm_fmt_of(int type) {
 constexpr int GD_NW = 8, GD_UPG = 2; /* direct kernel: 8 waves, groups of two 64-element units, 32-token tiles */
 
 // Token rows by way of LDS, whole lines: read as fragments a wave's load touches 64 pieces of 16 bytes.  Same sums in the same order.  From 17 rows on, below which the padding repeats one row's lines; in bf16, whose weights
-// take as many loads as the rows, also from 9 rows on at K >= 2048, and from K = 3072 or tall ones on always.  A wave's second group of columns takes a second slot, 128 KiB a workgroup: where the unpacking is long
-// (4-bit, 2-bit, 1-bit) two workgroups of a CU hide more than the rows' way gives, as long as a wave has but two groups.  us, fragments | LDS:
-//   128 rows, 4-bit: 1024 x 2048 10.1 | 8.9, 1024 x 3072 12.5 | 11.3, 5120 x 5120 55.6 | 49.9, gate and up 3072 x 1024 14.0 | 11.3; 2-bit 5120 x 5120 58.7 | 46.9; 1-bit 53.8 | 38.0; 8-bit 68.8 | 59.1; bf16 111.7 | 98.4
+// take as many loads as the rows, also from 9 rows on at K >= 2048, and from K = 3072 or tall ones on always.  us, fragments | LDS (with a second slot, where the products took these ways):
+//   128 rows, 4-bit: 1024 x 2048 10.1 | 8.9, 1024 x 3072 12.5 | 11.3, 5120 x 5120 55.6 | 49.9; 8-bit 68.8 | 59.1; bf16 111.7 | 98.4
 //   16 rows: 4-bit 1024 x 2048 8.7 | 8.7, 5120 x 5120 17.7 | 17.6, 4096 x 1024 5.5 | 5.7; bf16 4096 x 1024 5.7 | 6.3, 1024 x 2048 8.3 | 7.8, 5120 x 5120 36.6 | 34.2
 //   8 rows, bf16: 3072 x 1024 6.5 | 6.9, 2048 x 2048 8.8 | 9.2, 1024 x 3072 18.1 | 17.7, 151936 x 1024 115 | 94
-//   K = 1536, 1600, 64 | 128 | 200 rows: 4-bit 4800 x 1600 13.4 18.8 26.3 | 14.8 21.8 33.8; 1-bit 4800 x 1536 11.9 16.5 22.3 | 11.8 17.3 26.4; 8-bit 6400 x 1600 16.3 29.4 | 15.1 26.9; bf16 18.7 31.2 | 16.3 27.0
-//   K = 2048, 200 rows, 4-bit: 448 workgroups 16.6 | 16.0, 896 28.1 | 30.8
+// A wave's second group of columns takes a second slot of LDS, loaded ahead, where a CU has no more than one workgroup anyhow; else it waits for the first one's, and two workgroups of a CU hide that wait (a second slot is
+// 128 KiB a workgroup).  us, two slots | one: 128 rows, 4-bit 6144 x 2048 22.6 | 18.1, 2-bit 24.5 | 19.0, 8-bit 19.1 | 15.0, bf16 23.9 | 20.2, 4-bit 2048 x 2048 at 200 rows 15.0 | 12.3; K = 1536, where two slots did not pay
+// against the fragments, fragments | one slot: 4-bit 4800 x 1536 at 64 | 128 | 200 rows 12.2 17.6 25.8 | 8.9 12.4 17.7, 1-bit 10.0 13.8 19.6 | 8.5 11.7 16.3; 1.7B prompts, 128 rows 3079 | 2743, 256 rows 5215 | 4275
 template <int FMT>
-static bool gd_rows_by_lds(const GemmArgs& a, long wgs) {
-    if (a.n <= 16) return FMT == FMT_BF16 && (a.M > 1280 * 32 || a.K >= (a.n > 8 ? 2048 : 3072));
-    constexpr bool unpacks = FMT == FMT_Q4 || FMT == FMT_Q2 || FMT == FMT_Q1;
-    return !(unpacks && a.K > GD_NW * GD_UPG * 64 && (a.K < 2048 || (a.K < 3072 && wgs > 768)));
-}
+static bool gd_rows_by_lds(const GemmArgs& a) { return a.n > 16 || (FMT == FMT_BF16 && (a.M > 1280 * 32 || a.K >= (a.n > 8 ? 2048 : 3072))); }
 template <int TB, bool PAIRED>
 static void gm_direct16(const GemmArgs& a, int nrb, hipStream_t st) {
     const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1;
@@ -731,9 +732,9 @@ static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
         }
     }
     const size_t sums = (size_t)GD_NW * (PAIRED ? 2 : 1) * TB * 16 * 64 * 4;
-    const int slots = a.K > GD_NW * GD_UPG * 64 ? 2 : 1; /* one group of a wave, or two in turn */
+    const int slots = TB == 1 && a.K > GD_NW * GD_UPG * 64 && (long)grid.x * grid.y <= 256 ? 2 : 1;
     const size_t rows = (size_t)GD_NW * slots * TB * 32 * 256;
-    if (gd_rows_by_lds<FMT>(a, (long)grid.x * grid.y) && rows <= 128 * 1024 && a.ldx < (1 << 24)) {
+    if (gd_rows_by_lds<FMT>(a) && a.ldx < (1 << 24)) {
         static int attr_set = 0;
         if (!attr_set) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024), attr_set = 1;
         hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), grid, dim3(GD_NW * 64), rows > sums ? rows : sums, st, a, slots);

@@ -489,9 +489,9 @@ def test_rows_of_small_batches_do_not_depend_on_their_way(ctx, kind, M, K):
 
 
 @pytest.mark.parametrize("group", [32, 64, 128])
-@pytest.mark.parametrize("M,K", [(64, 128), (34, 192), (33, 1600), (96, 2048)])
+@pytest.mark.parametrize("M,K", [(4160, 128), (4130, 192), (4129, 1600), (4192, 2048), (33, 1600), (34, 192)])
 def test_tables_of_4_bit_groups_and_the_residual_of_a_small_batch(ctx, M, K, group):
-    """groups of one, two and four blocks, rows whose groups begin in the row before, odd and even rows: 20 rows by way of LDS (weights from tables, the residual loaded early where rows pair) equal 16 read as
+    """groups of one, two and four blocks, rows whose groups begin in the row before, odd and even rows (the last two: blocks of 16 rows): 20 rows by way of LDS (weights from tables, the residual loaded early where rows pair) equal 16 read as
     fragments (arithmetic) bit for bit, and the product in 32 bits to a bf16 rounding of the sum and one of the residual's"""
     if M * K % group:
         pytest.skip("whole groups only")
@@ -536,3 +536,30 @@ def test_blocks_of_16_and_of_32_weight_rows_give_the_same_bits(ctx, n, M, K):
     ctx.sync()
     for t in out:
         assert torch.equal(t.view(torch.int16), y[tall][0][:, :t.shape[1]].contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("kind,K", [(k, K) for k in (L.BF16, L.F8E5M2, L.Q4, L.T_SIGN, L.BOOL1) for K in (1152, 1600, 2048, 3072) if K != 1600 or k in (L.BF16, L.F8E5M2, L.Q4)])
+@pytest.mark.parametrize("n", [33, 64])
+def test_rows_with_one_and_two_slots_of_lds_give_the_same_bits(ctx, kind, K, n):
+    """more workgroups than CUs: a wave's token rows take turns in one slot; up to one for a CU: two.  The first rows of a taller product, and (64 rows) those of three matrices in a launch, by 64 token rows a workgroup"""
+    g = torch.Generator(device=ctx.device).manual_seed(n + K)
+    x, W = torch.randn(n, K, device=ctx.device, generator=g).bfloat16(), (torch.randn(4224, K, device=ctx.device, generator=g) * 0.05).bfloat16()
+    y = {}
+    for M in (4224, 4096):
+        w = ctx.quantize(W[:M].contiguous(), kind)
+        d, y[M] = w.desc(), torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y[M].data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    assert torch.equal(y[4224][:, :4096].contiguous().view(torch.int16), y[4096].view(torch.int16))
+    ref = x.float() @ ctx.dequant(w).float().reshape(4096, K).t()
+    assert float((y[4096].float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+    if K % 128 or (n >= 64 and kind == L.BF16):
+        return   # (bf16 matrices of 64 rows and more take the tile kernels)
+    rows = (4096, 2048, 2048 + 128)   # 256 blocks and more: 64 token rows a workgroup
+    part = [ctx.quantize(W[:r].contiguous(), kind) for r in rows]
+    d, out = [w.desc() for w in part], [torch.zeros(n, r, device=ctx.device, dtype=torch.bfloat16) for r in rows]
+    ws, ys = (C.c_void_p * 3)(*[C.addressof(v) for v in d]), (C.c_void_p * 3)(*[t.data_ptr() for t in out])
+    assert ctx.hip.kf_linear_multi(ctx.h, 3, ws, x.data_ptr(), ys, n) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    for t in out:
+        assert torch.equal(t.view(torch.int16), y[4224][:, :t.shape[1]].contiguous().view(torch.int16))
