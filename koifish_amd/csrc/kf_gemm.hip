@@ -734,19 +734,27 @@ static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
     const size_t sums = (size_t)GD_NW * (PAIRED ? 2 : 1) * TB * 16 * 64 * 4;
     const int slots = TB == 1 && a.K > GD_NW * GD_UPG * 64 && (long)grid.x * grid.y <= 256 ? 2 : 1;
     const size_t rows = (size_t)GD_NW * slots * TB * 32 * 256;
-    if (gd_rows_by_lds<FMT>(a) && a.ldx < (1 << 24)) {
+    if (TB == 2 || (gd_rows_by_lds<FMT>(a) && a.ldx < (1 << 24))) {
         static int attr_set = 0;
         if (!attr_set) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024), attr_set = 1;
         hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, true>), grid, dim3(GD_NW * 64), rows > sums ? rows : sums, st, a, slots);
         return;
     }
-    hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, false>), grid, dim3(GD_NW * 64), sums, st, a, 0);
+    if constexpr (TB == 1) hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, false>), grid, dim3(GD_NW * 64), sums, st, a, 0);
+}
+// 64 token rows a workgroup: every weight is unpacked for twice as many, but a workgroup has a CU to itself.  Taken where the rounds that the launch takes of such workgroups are the shorter: 1.4 a round, against 1.8 for a
+// round of 512 of the others, two to a CU, and 1 for a last one of at most 256.  us a prompt, 32 | 64 where the rule takes them: o and down, 0.6B 319 rows 2732 | 2592, 1.7B 192 rows 3949 | 3736, 256 rows 4270 | 4020, six layers
+// of the 32B shape at 256 rows 4640 | 4370; gate | up, 0.6B 128 rows 1718 | 1667, 1.7B 256 rows 4270 | 4057, 32B 64 rows 2446 | 2340; where it does not: 0.6B 256 rows 2162 | 2217, 1.7B 128 rows 2765 | 2785, 2765 | 2984
+static bool gd_wide(const GemmArgs& a, long row_blocks) {
+    const long one = row_blocks * ((a.n + 31) / 32), two = row_blocks * ((a.n + 63) / 64), last = one % 512;
+    return a.n > 32 && a.ldx < (1 << 24) && 14 * ((two + 255) / 256) < 18 * (one / 512) + (last == 0 ? 0 : last <= 256 ? 10 : 18);
 }
 template <int FMT>
 static void gm_launch(const GemmArgs& a, int KS, dim3 grid, size_t smem, hipStream_t st) {
-    if (KS == 0) gm_direct<FMT, 1, false>(a, grid, st);
-    else if (KS == -2) gm_direct<FMT, 2, false>(a, grid, st); /* 64-token tiles: every weight block is unpacked for two token blocks */
-    else if (KS == -1) gm_direct<FMT, 1, true>(a, grid, st); /* paired SwiGLU */
+    const bool wide = KS <= 0 && gd_wide(a, grid.x);
+    const dim3 half(grid.x, (a.n + 63) / 64);
+    if (KS == 0) wide ? gm_direct<FMT, 2, false>(a, half, st) : gm_direct<FMT, 1, false>(a, grid, st);
+    else if (KS == -1) wide && FMT == FMT_Q4 ? gm_direct<FMT == FMT_Q4 ? FMT : FMT_BF16, 2, FMT == FMT_Q4>(a, half, st) : gm_direct<FMT, 1, true>(a, grid, st); /* paired SwiGLU */
     else if (KS == 2)
         hipLaunchKernelGGL((gemm_kernel<FMT, 2>), grid, dim3(256), smem, st, a);
     else
@@ -833,10 +841,7 @@ int gemm_multi_launch(hipStream_t st, int n_w, const kf_weight* const* w, const 
             a.xw[i - 1] = g[i].w, a.xzero[i - 1] = g[i].zero, a.xstep[i - 1] = g[i].step, a.xqBias[i - 1] = g[i].qBias, a.xM[i - 1] = g[i].M, a.xy[i - 1] = y[i],
                      a.xldy[i - 1] = g[i].M;
     }
-    if (n >= 64 && (long)end * ((n + 63) / 64) >= 256)
-        gm_dispatch(g[0].fmt, a, -2, dim3(end, (n + 63) / 64), 0, st);
-    else
-        gm_dispatch(g[0].fmt, a, 0, dim3(end, (n + 31) / 32), 0, st);
+    gm_dispatch(g[0].fmt, a, 0, dim3(end, (n + 31) / 32), 0, st);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 

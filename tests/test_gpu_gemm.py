@@ -541,21 +541,22 @@ def test_blocks_of_16_and_of_32_weight_rows_give_the_same_bits(ctx, n, M, K):
 @pytest.mark.parametrize("kind,K", [(k, K) for k in (L.BF16, L.F8E5M2, L.Q4, L.T_SIGN, L.BOOL1) for K in (1152, 1600, 2048, 3072) if K != 1600 or k in (L.BF16, L.F8E5M2, L.Q4)])
 @pytest.mark.parametrize("n", [33, 64])
 def test_rows_with_one_and_two_slots_of_lds_give_the_same_bits(ctx, kind, K, n):
-    """more workgroups than CUs: a wave's token rows take turns in one slot; up to one for a CU: two.  The first rows of a taller product, and (64 rows) those of three matrices in a launch, by 64 token rows a workgroup"""
+    """32 token rows a workgroup, up to one of them for a CU (two slots of LDS a wave: 4096 rows) and more (one slot: 9216), and 64 token rows (4224; three matrices in a launch): the same rows, the same bits"""
     g = torch.Generator(device=ctx.device).manual_seed(n + K)
-    x, W = torch.randn(n, K, device=ctx.device, generator=g).bfloat16(), (torch.randn(4224, K, device=ctx.device, generator=g) * 0.05).bfloat16()
+    x, W = torch.randn(n, K, device=ctx.device, generator=g).bfloat16(), (torch.randn(9216, K, device=ctx.device, generator=g) * 0.05).bfloat16()
     y = {}
-    for M in (4224, 4096):
+    for M in (9216, 4224, 4096):
         w = ctx.quantize(W[:M].contiguous(), kind)
         d, y[M] = w.desc(), torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
         assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y[M].data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
     ctx.sync()
-    assert torch.equal(y[4224][:, :4096].contiguous().view(torch.int16), y[4096].view(torch.int16))
+    for M in (9216, 4224):
+        assert n >= 64 and kind == L.BF16 or torch.equal(y[M][:, :4096].contiguous().view(torch.int16), y[4096].view(torch.int16))
     ref = x.float() @ ctx.dequant(w).float().reshape(4096, K).t()
     assert float((y[4096].float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
     if K % 128 or (n >= 64 and kind == L.BF16):
         return   # (bf16 matrices of 64 rows and more take the tile kernels)
-    rows = (4096, 2048, 2048 + 128)   # 256 blocks and more: 64 token rows a workgroup
+    rows = (4096, 2048, 2048)   # 512 blocks of 32 rows and tokens
     part = [ctx.quantize(W[:r].contiguous(), kind) for r in rows]
     d, out = [w.desc() for w in part], [torch.zeros(n, r, device=ctx.device, dtype=torch.bfloat16) for r in rows]
     ws, ys = (C.c_void_p * 3)(*[C.addressof(v) for v in d]), (C.c_void_p * 3)(*[t.data_ptr() for t in out])
