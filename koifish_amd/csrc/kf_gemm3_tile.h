@@ -135,6 +135,11 @@ template <class F>
 static __device__ void g3_told_apart(unsigned char* __restrict__ a0, unsigned char* __restrict__ a1, unsigned char* __restrict__ b0, unsigned char* __restrict__ b1, F&& f) {
     f(a0, a1, b0, b1);
 }
+template <class F>
+static __device__ void g3_told_apart(unsigned char* __restrict__ a0, unsigned char* __restrict__ a1, unsigned char* __restrict__ a2, unsigned char* __restrict__ b0, unsigned char* __restrict__ b1,
+                                     unsigned char* __restrict__ b2, F&& f) {
+    f(a0, a1, a2, b0, b1, b2);
+}
 struct G3Nothing {
     __device__ __forceinline__ void operator()(int) const {}
 };
@@ -292,33 +297,45 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         order(rb, lb);
     };
     // the steps are unrolled by two: the two token halves' registers swap roles with them, and of two buffers every LDS address of a step is base + an immediate
-    auto all = [&](unsigned char* a_even, unsigned char* a_odd, unsigned char* b_even, unsigned char* b_odd) {
-#pragma unroll
-        for (int b = 0; b < C::NBUF; b++) stageA(kt0 + b, b == 0 ? a_even : b == 1 ? a_odd : bufA(b)), stageB(kt0 + b, b == 0 ? b_even : b == 1 ? b_odd : bufB(b));
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((C::NBUF - 1) * LPW) : "memory");
+    [[maybe_unused]] auto two = [&](unsigned char* a_even, unsigned char* a_odd, unsigned char* b_even, unsigned char* b_odd) {
+        stageA(kt0, a_even), stageB(kt0, b_even), stageA(kt0 + 1, a_odd), stageB(kt0 + 1, b_odd);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory"); /* no read moves up */
         readA(a_even, 0, a0), readB(b_even, 0, b0);
-        if constexpr (C::NBUF == 2) {
-            for (int kt = kt0; kt < kt1; kt += 2) {
-                between(kt);
-                step(kt, a_even, b_even, a_odd, b_odd, b0, b1);
-                if (kt + 1 < kt1) between(kt + 1), step(kt + 1, a_odd, b_odd, a_even, b_even, b1, b0);
-            }
-        } else {
-            int cur = 0;
-            auto behind = [](int b) { return b + 1 < C::NBUF ? b + 1 : 0; };
-            for (int kt = kt0; kt < kt1; kt += 2) {
-                const int one = behind(cur), two = behind(one);
-                between(kt);
-                step(kt, bufA(cur), bufB(cur), bufA(one), bufB(one), b0, b1);
-                if (kt + 1 < kt1) between(kt + 1), step(kt + 1, bufA(one), bufB(one), bufA(two), bufB(two), b1, b0);
-                cur = two;
-            }
+        for (int kt = kt0; kt < kt1; kt += 2) {
+            between(kt);
+            step(kt, a_even, b_even, a_odd, b_odd, b0, b1);
+            if (kt + 1 < kt1) between(kt + 1), step(kt + 1, a_odd, b_odd, a_even, b_even, b1, b0);
         }
     };
-    if constexpr (AKM || BKM) g3_told_apart(bufA(0), bufA(1), bufB(0), bufB(1), all);
-    else all(bufA(0), bufA(1), bufB(0), bufB(1));
+    // three buffers: by six, so that every buffer is a name too.  With the buffer's number in a register a step had 14 - 21 vector additions for its LDS addresses in front of its MFMAs: us, numbered | named,
+    // 128 x 256 tiles: 5120 x 5120 at 1000 rows 65 | 60, 6400 x 1600 at 8192 rows 188 | 180; 128 x 128 on 8 waves: 2048 x 2048 at 2047 rows 22.6 | 20.7, 1024 x 2048 at 2608 19.0 | 18.0; 64 x 64: 1024 x 2048 at 2047 14.7 | 14.6
+    [[maybe_unused]] auto three = [&](unsigned char* a_0, unsigned char* a_1, unsigned char* a_2, unsigned char* b_0, unsigned char* b_1, unsigned char* b_2) {
+        stageA(kt0, a_0), stageB(kt0, b_0), stageA(kt0 + 1, a_1), stageB(kt0 + 1, b_1), stageA(kt0 + 2, a_2), stageB(kt0 + 2, b_2);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory"); /* no read moves up */
+        readA(a_0, 0, a0), readB(b_0, 0, b0);
+        for (int kt = kt0;;) {
+            between(kt), step(kt, a_0, b_0, a_1, b_1, b0, b1);
+            if (++kt >= kt1) break;
+            between(kt), step(kt, a_1, b_1, a_2, b_2, b1, b0);
+            if (++kt >= kt1) break;
+            between(kt), step(kt, a_2, b_2, a_0, b_0, b0, b1);
+            if (++kt >= kt1) break;
+            between(kt), step(kt, a_0, b_0, a_1, b_1, b1, b0);
+            if (++kt >= kt1) break;
+            between(kt), step(kt, a_1, b_1, a_2, b_2, b0, b1);
+            if (++kt >= kt1) break;
+            between(kt), step(kt, a_2, b_2, a_0, b_0, b1, b0);
+            if (++kt >= kt1) break;
+        }
+    };
+    static_assert(C::NBUF == 2 || C::NBUF == 3, "two or three buffers");
+    if constexpr (C::NBUF == 3) g3_told_apart(bufA(0), bufA(1), bufA(2), bufB(0), bufB(1), bufB(2), three);
+    else if constexpr (AKM || BKM) g3_told_apart(bufA(0), bufA(1), bufB(0), bufB(1), two);
+    else two(bufA(0), bufA(1), bufB(0), bufB(1));
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier(); /* the buffers are free: for a following segment's first loads, for an epilogue's exchange */
     asm volatile("" ::: "memory");
