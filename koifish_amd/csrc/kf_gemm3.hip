@@ -476,14 +476,14 @@ static int g3_go(hipStream_t st, const GemmArgs& a, long nwg, void* ws, size_t w
 }
 size_t gemm3_sk_ws_bytes() { return (size_t)256 * G3_BM * G3_BN * 4 + G3_SK_FLAG_BYTES; }
 static long g3_tiles_of(int M, int n, int bm, int bn) { return (long)((M + bm - 1) / bm) * ((n + bn - 1) / bn); }
-template <class C>
+template <class C, bool AKM = false, bool BKM = false>
 static int g3_whole(hipStream_t st, const GemmArgs& a) { /* one workgroup per tile */
     static int attr_set = 0;
     if (!attr_set && C::SMEM > 64 * 1024) {
-        if (hipFuncSetAttribute((const void*)gemm3_kernel<false, false, G3_BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::SMEM) != hipSuccess) return KF_HIP_CHECK;
+        if (hipFuncSetAttribute((const void*)gemm3_kernel<AKM, BKM, G3_BK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::SMEM) != hipSuccess) return KF_HIP_CHECK;
         attr_set = 1;
     }
-    hipLaunchKernelGGL((gemm3_kernel<false, false, G3_BK, C>), dim3((unsigned)g3_tiles_of(a.M, a.n, C::BM, C::BN)), dim3(C::NTH), C::SMEM, st, a);
+    hipLaunchKernelGGL((gemm3_kernel<AKM, BKM, G3_BK, C>), dim3((unsigned)g3_tiles_of(a.M, a.n, C::BM, C::BN)), dim3(C::NTH), C::SMEM, st, a);
     return hipGetLastError() == hipSuccess ? KF_OK : KF_HIP_CHECK;
 }
 template <class C>
@@ -554,6 +554,11 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
     const long nws = (long)((M + 127) / 128) * ((n + 127) / 128), rounds = (nws + 511) / 512;
     const bool small = 5 * nwg < 4 * 256 && akm && (20 * nws >= 17 * rounds * 512 || (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nws < 4 * 512));
     if (small) return bkm ? g3_go_c<true, true, G3Small>(st, a, nws, ws, ws_bytes, 1) : g3_go_c<true, false, G3Small>(st, a, nws, ws, ws_bytes, 1);
+    switch (akm ? g3_km_pick(M, n, bkm) : G3_BIG) {
+        case G3_SLIM: return bkm ? g3_whole<G3Slim, true, true>(st, a) : g3_whole<G3Slim, true, false>(st, a);
+        case G3_FLAT: return bkm ? g3_whole<G3Flat, true, true>(st, a) : g3_whole<G3Flat, true, false>(st, a);
+        default: break;
+    }
     if (akm && bkm) return g3_go<true, true>(st, a, nwg, ws, ws_bytes);
     if (akm) return g3_go<true, false>(st, a, nwg, ws, ws_bytes);
     if (bkm) return g3_go<false, true>(st, a, nwg, ws, ws_bytes);

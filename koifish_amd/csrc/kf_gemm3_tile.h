@@ -8,14 +8,25 @@
 namespace kf {
 
 constexpr int G3_BM = 256, G3_BN = 256, G3_BK = 64;
-// the workgroup tile: BM rows x BN tokens, NW waves as 2 (rows) x NW / 2 (tokens), NBUF LDS buffers: the loads of NBUF - 1 later k-steps are in flight under the step that is multiplied.
+// the workgroup tile: BM rows x BN tokens, NW waves as NW / WN_ (rows; 2 by default) x WN_ (tokens), NBUF LDS buffers: the loads of NBUF - 1 later k-steps are in flight under the step that is multiplied.
 // A step is bound by those loads, not by its MFMAs (loads alone take 85 - 95 % of every configuration's time), and with two buffers a lone workgroup of a CU waits out their latency: us per
 // step with one workgroup on every CU, two buffers | more: 64 x 64 0.41 | 0.23 (3), 128 x 128 on 8 waves 0.89 | 0.58 (3), 128 x 256 0.82 (3) against 1.26 of 192 x 256 (2: three do not fit).
-template <int BM_, int BN_, int NW_, int NBUF_ = 2>
+// Where an operand's instructions are no multiple of the waves (EVEN false: 160 rows are 20) the first waves issue one more; the others' last one has an empty descriptor and
+// a KiB of its own behind the buffers (SPARE), so that every wave counts the same loads.  SMEM then is the whole LDS: the tile in 32 bits fits.
+template <int BM_, int BN_, int NW_, int NBUF_ = 2, int WN_ = NW_ / 2>
 struct G3Cfg {
-    static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = NW_ / 2, MT = BM_ / 32, NT = BN_ / (16 * (NW_ / 2)), NBUF = NBUF_;
-    static constexpr int NIA = BM_ / (8 * NW_), NIB = BN_ / (8 * NW_); /* global_load_lds instructions per wave, operand and k-step (8 rows of 128 bytes each) */
-    static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, SMEM = NBUF_ * STAGE, WGS_PER_CU = (160 * 1024) / SMEM;
+    static constexpr int BM = BM_, BN = BN_, NW = NW_, WN = WN_, MT = BM_ / (16 * (NW_ / WN_)), NT = BN_ / (16 * WN_), NBUF = NBUF_;
+    static constexpr int NIA = (BM_ / 8 + NW_ - 1) / NW_, NIB = (BN_ / 8 + NW_ - 1) / NW_; /* global_load_lds instructions per wave, operand and k-step (8 rows of 128 bytes each) */
+    static constexpr bool EVEN = BM_ % (8 * NW_) == 0 && BN_ % (8 * NW_) == 0;
+    static constexpr int STAGE = (BM_ + BN_) * G3_BK * 2, NTH = 64 * NW_, SPARE = NBUF_ * STAGE, SMEM = EVEN ? SPARE : 160 * 1024, WGS_PER_CU = (160 * 1024) / SMEM;
+    static_assert(EVEN || SPARE + 1024 <= SMEM, "the spare KiB");
+};
+// an operand of ROWS rows: the first of wave `wid`'s load instructions, and whether it has an i-th one
+template <int ROWS, int NW>
+struct G3Share {
+    static constexpr int ALL = ROWS / 8, Q = ALL / NW, REST = ALL % NW;
+    static __device__ __forceinline__ int first(int wid) { return Q * wid + (REST == 0 || wid < REST ? (REST ? wid : 0) : REST); }
+    static __device__ __forceinline__ bool has(int wid, int i) { return i < Q || wid < REST; }
 };
 using G3Big = G3Cfg<256, 256, 8>;      /* 128 KiB of LDS: one workgroup per CU */
 using G3Wide = G3Cfg<192, 256, 8>;
@@ -25,6 +36,8 @@ using G3Duo = G3Cfg<128, 128, 8, 3>;   /* 96 KiB */
 using G3Small = G3Cfg<128, 128, 4>;    /* 64 KiB: two workgroups per CU; the split-K tile of the k-major products */
 using G3Few = G3Cfg<64, 64, 4, 3>;     /* 48 KiB: three */
 // k-pieces where a workspace is lent (gemm3_launch)
+using G3Slim = G3Cfg<160, 256, 8, 3>;  /* 156 KiB: three buffers where 192 rows leave two, five eighths of the big tile's outputs */
+using G3Flat = G3Cfg<256, 160, 8, 3, 2>;
 using G3Mid = G3Cfg<64, 128, 4>;
 using G3Tiny = G3Cfg<64, 64, 4>;
 
@@ -42,16 +55,15 @@ constexpr uint32_t G3_ALL = 0x7FFFFFF0u; /* a descriptor's size that no lane par
 struct G3Src {
     const unsigned char* base; /* uniform: the tile's origin at k-step 0 */
     long long left, step, inst; /* bytes from there to the operand's end (< 0: no row past the end); bytes per k-step; bytes per instruction */
-    uint32_t lane[2];
+    uint32_t lane[3]; /* [2]: 160-row k-major images */
 };
-template <int NI>
-__device__ __forceinline__ G3Src g3_src(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int wid, int lane) {
+__device__ __forceinline__ G3Src g3_src(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int first, int lane) { /* first: the wave's first instruction */
     G3Src s;
-    s.base = reinterpret_cast<const unsigned char*>(src + ((size_t)row0 + (size_t)wid * NI * 8) * ld);
-    s.left = ((long long)nrows - row0 - (long long)wid * NI * 8) * ld * 2, s.step = G3_BK * 2, s.inst = ld * 16;
+    s.base = reinterpret_cast<const unsigned char*>(src + ((size_t)row0 + (size_t)first * 8) * ld);
+    s.left = ((long long)nrows - row0 - (long long)first * 8) * ld * 2, s.step = G3_BK * 2, s.inst = ld * 16;
 #pragma unroll
     for (int v = 0; v < 2; v++) {
-        const int r = (wid * NI + v) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        const int r = (first + v) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
         s.lane[v] = (uint32_t)(lane >> 3) * (uint32_t)(ld * 2) + c * 16;
     }
     return s;
@@ -65,13 +77,27 @@ __device__ __forceinline__ bf16x8 g3_frag(const unsigned char* tile, int row, in
 // both GEMMs of SLP::Back): the LDS image is [BK k][ROWS rows] (512- or 256-byte k-rows), one wave instruction = two or four k-rows; its 32-byte blocks are XOR-swizzled by k & 3 and
 // its 128-byte quarters by bit 3 of k, so that the transposing fragment read below (per 32 lanes: k-rows k .. k+3 and k+8 .. k+11, 32 bytes of each) touches all 64
 // banks once (without the second term the two 16-lane halves meet in the same 32 banks: SQ_LDS_BANK_CONFLICT = 50 % of the LDS cycles, measured).
-// ROWS = the tile's rows (256 or 128): a k-row of the image is 2 ROWS bytes = CPK chunks of 16 bytes, one wave instruction covers 64 / CPK k-rows, wave `wid` issues
+// A k-row of 160 rows is 20 chunks, 64 bytes past whole turns of the banks, so four k-rows meet in no bank as they are and only bit 3 of k moves a block, to its neighbour; five instructions are 16 k-rows.
+// ROWS = the tile's rows (256, 160 or 128): a k-row of the image is 2 ROWS bytes = CPK chunks of 16 bytes, one wave instruction covers 64 / CPK k-rows, wave `wid` issues
 // instructions NI wid .. NI wid + NI - 1 of the ROWS / 8
 template <int ROWS, int NI>
 __device__ __forceinline__ G3Src g3_src_km(const uint16_t* __restrict__ src, long long ld, int row0, int nrows, int wid, int lane) {
     constexpr int CPK = ROWS / 8, KPI = 64 / CPK, UNIT = ROWS == 256 ? 1 : 2; /* 256: the swizzle tells even from odd instructions, 128: pairs of them */
-    static_assert((ROWS == 256 || ROWS == 128) && NI == 4, "two lane parts per wave");
     G3Src s;
+    if constexpr (ROWS == 160) {
+        static_assert(NI == 3, "a lane part per instruction");
+        const int first = G3Share<160, 8>::first(wid);
+        s.base = reinterpret_cast<const unsigned char*>(src), s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = 32 * ld; /* (inst: 16 k-rows, five instructions) */
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+            const int at = (first + v) % 5 * 64 + lane, kr = at / CPK, p = at % CPK, c = p ^ (((kr >> 3) & 1) << 1);
+            int col = row0 + c * 8;
+            col = col + 8 <= nrows ? col : (nrows - 8 > 0 ? nrows - 8 : 0); /* as below */
+            s.lane[v] = G3Share<160, 8>::has(wid, v) ? (uint32_t)kr * (uint32_t)(ld * 2) + col * 2 : G3_ALL; /* (none: past the descriptor's end) */
+        }
+        return s;
+    }
+    static_assert(ROWS == 160 || ((ROWS == 256 || ROWS == 128) && NI == 4), "two lane parts per wave");
     s.base = reinterpret_cast<const unsigned char*>(src + (size_t)wid * NI * KPI * ld);
     s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = (long long)KPI * ld * 2; /* every k-row of the steps exists; chunks past a row's end are clamped here */
 #pragma unroll
@@ -87,6 +113,11 @@ __device__ __forceinline__ G3Src g3_src_km(const uint16_t* __restrict__ src, lon
 // (lane i of the 16 receives D[(i >> 2) + 4 j][i & 3], scratch/dbg/ds_read_tr_probe.hip): lane l16 reads k-row kbase + (l16 >> 2), 8-byte piece l16 & 3 of the 16-row block
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 // The row block only flips three bits of a lane's offset (the swizzle's), so one register serves all blocks.
+// 160 rows: the swizzle puts a block behind or in front of its place by the block's parity, one offset for each (odd: of the blocks 1, 3, .. of a wave whose first block is odd or even, `odd` says which)
+__device__ __forceinline__ int g3_km_lane160(int l16, int q4, int odd) {
+    const int k = 8 * q4 + (l16 >> 2);
+    return k * 320 + ((l16 & 3) >> 1) * 16 + 8 * (l16 & 1) + ((q4 & 1) ? (odd ? -32 : 32) : 0);
+}
 __device__ __forceinline__ int g3_km_lane(int rows, int l16, int q4) { /* the lane's offset in a tile at row block 0, k 0 */
     const int k = 8 * q4 + (l16 >> 2), swz = ((k & 3) << 1) ^ (((k >> 3) & 1) << 3);
     return k * (2 * rows) + ((((l16 & 3) >> 1) ^ swz) << 4) + 8 * (l16 & 1);
@@ -94,7 +125,7 @@ __device__ __forceinline__ int g3_km_lane(int rows, int l16, int q4) { /* the la
 template <int ROWS>
 __device__ __forceinline__ bf16x8 g3_frag_km(const unsigned char* tile, int km_lane, int rowblk16, int kk) {
     bf16x4 h[2];
-    const unsigned char* const at = tile + ((km_lane ^ ((rowblk16 & 7) << 5)) + ((rowblk16 >> 3) << 8));
+    const unsigned char* const at = tile + (ROWS == 160 ? km_lane + rowblk16 * 32 : (km_lane ^ ((rowblk16 & 7) << 5)) + ((rowblk16 >> 3) << 8));
 #pragma unroll
     for (int t = 0; t < 2; t++) h[t] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(at + (kk * 32 + 4 * t) * (2 * ROWS)));
     return bf16x8{h[0][0], h[0][1], h[0][2], h[0][3], h[1][0], h[1][1], h[1][2], h[1][3]};
@@ -140,6 +171,14 @@ static __device__ void g3_told_apart(unsigned char* __restrict__ a0, unsigned ch
                                      unsigned char* __restrict__ b2, F&& f) {
     f(a0, a1, a2, b0, b1, b2);
 }
+template <int M, int N, int V, int I>
+__device__ __forceinline__ void g3_issue() { /* an MFMA, then its share of N reads and of V loads among M MFMAs */
+    constexpr int P = N < M ? N : M, Q = V < M - 1 ? V : M - 1;
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if constexpr (I < P) __builtin_amdgcn_sched_group_barrier(0x100, N * (I + 1) / P - N * I / P, 0);
+    if constexpr (I < Q) __builtin_amdgcn_sched_group_barrier(0x010, V * (I + 1) / Q - V * I / Q, 0);
+    if constexpr (I + 1 < (P > Q ? P : Q)) g3_issue<M, N, V, I + 1>();
+}
 struct G3Nothing {
     __device__ __forceinline__ void operator()(int) const {}
 };
@@ -147,12 +186,17 @@ struct G3Nothing {
 template <bool AKM, bool BKM, int BK, class C, class ROWS = G3Rows, class BETWEEN = G3Nothing>
 __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, int kt0, int kt1, f32x4 (&acc)[C::MT][C::NT], unsigned char* smem_raw, int wid_, int lane, ROWS rows = ROWS(),
                                             BETWEEN between = BETWEEN()) {
-    static_assert(BK == G3_BK && C::MT % 2 == 0 && C::NT % 2 == 0, "two k-halves of 32 per step, two halves of rows and of tokens per wave");
-    constexpr int LPW = C::NIA + C::NIB, HM = C::MT / 2, HN = C::NT / 2; /* loads per wave and step; MFMA blocks per half */
+    static_assert(BK == G3_BK && C::MT > 1 && C::NT > 1, "two k-halves of 32 per step, two halves of rows and of tokens per wave");
+    constexpr int LPW = C::NIA + C::NIB, HM = (C::MT + 1) / 2, HN = (C::NT + 1) / 2; /* loads per wave and step; MFMA blocks of the first half (five: three and two) */
+    constexpr std::integral_constant<int, 0> lo{};
+    constexpr std::integral_constant<int, 1> hi{};
+    using ShareA = G3Share<C::BM, C::NW>;
+    using ShareB = G3Share<C::BN, C::NW>;
     constexpr int BYTES_A = C::BM * BK * 2, BYTES_B = C::BN * BK * 2;
     const int wid = __builtin_amdgcn_readfirstlane(wid_), wm = wid / C::WN, wn = wid % C::WN;
     auto bufA = [&](int b) { return smem_raw + b * BYTES_A; }; /* an operand's two buffers side by side: both in reach of an LDS instruction's 16-bit offset */
     auto bufB = [&](int b) { return smem_raw + C::NBUF * BYTES_A + b * BYTES_B; };
+    [[maybe_unused]] const int firstA = ShareA::first(wid), firstB = ShareB::first(wid);
     // AKM: W is [K][M] with row stride a.ldr (re-used field: the residual is not served by the k-major forms); BKM: x is [K][n] with row stride a.ldx.
     G3Src sa, sb;
     const uint16_t* gat[ROWS::GATHER ? C::NIB : 1];
@@ -165,40 +209,42 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     } else if constexpr (AKM)
         sa = g3_src_km<C::BM, C::NIA>(W, a.ldr, m0, a.M, wid, lane);
     else
-        sa = g3_src<C::NIA>(W, a.K, m0, a.M, wid, lane);
+        sa = g3_src(W, a.K, m0, a.M, firstA, lane);
     if constexpr (ROWS::GATHER) {
-        static_assert(!BKM, "gathered rows: K-contiguous operands");
+        static_assert(!BKM && ShareB::REST == 0, "gathered rows: K-contiguous operands, every load has a row");
 #pragma unroll
         for (int i = 0; i < C::NIB; i++) {
-            const int r = (wid * C::NIB + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+            const int r = (firstB + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
             gat[i] = a.x + (size_t)rows.map[r] * a.ldx + c * 8;
         }
     } else if constexpr (BKM)
         sb = g3_src_km<C::BN, C::NIB>(a.x, a.ldx, t0, a.n, wid, lane);
     else
-        sb = g3_src<C::NIB>(a.x, a.ldx, t0, a.n, wid, lane);
+        sb = g3_src(a.x, a.ldx, t0, a.n, firstB, lane);
     // K-contiguous operands: one descriptor per instruction for the whole tile, a step is the scalar offset (a row past the end lies past the descriptor's end at every
-    // step, whether or not the check counts that offset; a row inside never does).  k-major: every step has a base of its own, of any size.
+    // step, whether or not the check counts that offset; a row inside never does).  k-major: every step has a base of its own, of any size, and an instruction the scalar offset.
     // Past the last step the descriptors are empty: the load moves nothing and puts zeros where nobody reads, and the steps need no branch.
     uint32_t restA[C::NIA], restB[C::NIB];
     auto rest = [](long long left) { return (uint32_t)(left < 0 ? 0 : (left > 0xFFFFFFFFll ? 0xFFFFFFFFll : left)); };
     auto atA = [&](int i) {
-        const int j = wid * C::NIA + i; /* tile (row block j / 2, k-half j % 2) of the workgroup's */
-        return ROWS::TILED ? sa.inst * (j >> 1) + (j & 1) * 1024 : sa.inst * i;
+        const int j = firstA + i; /* tile (row block j / 2, k-half j % 2) of the workgroup's */
+        return ROWS::TILED ? sa.inst * (j >> 1) + (j & 1) * 1024 : AKM && C::BM == 160 ? sa.inst * (j / 5) : sa.inst * i;
     };
+    [[maybe_unused]] auto atB = [&](int i) { return BKM && C::BN == 160 ? sb.inst * ((firstB + i) / 5) : sb.inst * i; };
 #pragma unroll
-    for (int i = 0; i < C::NIA; i++) restA[i] = AKM ? G3_ALL : rest(sa.left - atA(i));
+    for (int i = 0; i < C::NIA; i++) restA[i] = !ShareA::has(wid, i) ? 0 : AKM ? G3_ALL : rest(sa.left - atA(i));
 #pragma unroll
-    for (int i = 0; i < C::NIB; i++) restB[i] = BKM || ROWS::GATHER ? G3_ALL : rest(sb.left - sb.inst * i);
+    for (int i = 0; i < C::NIB; i++) restB[i] = !ShareB::has(wid, i) ? 0 : BKM || ROWS::GATHER ? G3_ALL : rest(sb.left - atB(i));
+    [[maybe_unused]] auto to = [&](unsigned char* tile, int i, bool has) { return (__attribute__((address_space(3))) void*)(has ? tile + i * 1024 : smem_raw + C::SPARE); };
     [[maybe_unused]] const unsigned char *nextA = sa.base + (AKM ? sa.step * kt0 : 0), *nextB = BKM ? sb.base + sb.step * kt0 : nullptr; /* k-major: the base of the step staged next */
     auto stageA = [&](int kt, unsigned char* tile) {
 #ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
         for (int i = 0; i < C::NIA; i++) {
-            const auto to = (__attribute__((address_space(3))) void*)(tile + (wid * C::NIA + i) * 1024);
-            const uint32_t n = kt < kt1 ? restA[i] : 0;
-            if constexpr (AKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextA + sa.inst * i, n), to, 16, sa.lane[C::BM == 128 ? i >> 1 : i & 1], 0, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sa.base + atA(i), n), to, 16, sa.lane[ROWS::TILED ? 0 : i & 1], (int)sa.step * kt, 0, 0);
+            [[maybe_unused]] const auto at = to(tile, firstA + i, ShareA::has(wid, i));
+            [[maybe_unused]] const uint32_t n = kt < kt1 ? restA[i] : 0;
+            if constexpr (AKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextA, kt < kt1 ? G3_ALL : 0), at, 16, sa.lane[C::BM == 160 ? i : C::BM == 128 ? i >> 1 : i & 1], (int)atA(i), 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sa.base + atA(i), n), at, 16, sa.lane[ROWS::TILED ? 0 : i & 1], (int)sa.step * kt, 0, 0);
         }
         if constexpr (AKM) nextA += sa.step;
 #endif
@@ -207,68 +253,75 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
 #ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
         for (int i = 0; i < C::NIB; i++) {
-            const auto to = (__attribute__((address_space(3))) void*)(tile + (wid * C::NIB + i) * 1024);
-            const uint32_t n = kt < kt1 ? restB[i] : 0;
-            if constexpr (ROWS::GATHER) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gat[i] + (size_t)(kt < kt1 ? kt : kt1 - 1) * BK), to, 16, 0, 0); /* (past the end: the last step again) */
-            else if constexpr (BKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextB + sb.inst * i, n), to, 16, sb.lane[C::BN == 128 ? i >> 1 : i & 1], 0, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sb.base + sb.inst * i, n), to, 16, sb.lane[i & 1], (int)sb.step * kt, 0, 0);
+            [[maybe_unused]] const auto at = to(tile, firstB + i, ShareB::has(wid, i));
+            [[maybe_unused]] const uint32_t n = kt < kt1 ? restB[i] : 0;
+            if constexpr (ROWS::GATHER) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gat[i] + (size_t)(kt < kt1 ? kt : kt1 - 1) * BK), at, 16, 0, 0); /* (past the end: the last step again) */
+            else if constexpr (BKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextB, kt < kt1 ? G3_ALL : 0), at, 16, sb.lane[C::BN == 160 ? i : C::BN == 128 ? i >> 1 : i & 1], (int)atB(i), 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sb.base + atB(i), n), at, 16, sb.lane[i & 1], (int)sb.step * kt, 0, 0);
         }
         if constexpr (BKM) nextB += sb.step;
 #endif
     };
-    const int r16 = lane & 15, q4 = lane >> 4, kmA = g3_km_lane(C::BM, r16, q4), kmB = g3_km_lane(C::BN, r16, q4);
-    auto readA = [&](const unsigned char* tile, int half, bf16x8 (&f)[HM][2]) {
-        const int km = AKM && HM > 2 ? g3_opaque(kmA) : kmA; /* eight blocks' addresses kept would not leave room for the fragments */
+    const int r16 = lane & 15, q4 = lane >> 4;
+    int kmA[2], kmB[2]; /* [1]: odd blocks of a 160-row operand */
 #pragma unroll
-        for (int mh = 0; mh < HM; mh++)
+    for (int odd = 0; odd < 2; odd++) {
+        kmA[odd] = C::BM == 160 ? g3_km_lane160(r16, q4, (wm * C::MT + odd) & 1) : g3_km_lane(C::BM, r16, q4);
+        kmB[odd] = C::BN == 160 ? g3_km_lane160(r16, q4, (wn * C::NT + odd) & 1) : g3_km_lane(C::BN, r16, q4);
+    }
+    auto readA = [&](const unsigned char* tile, auto half, bf16x8 (&f)[HM][2]) {
+        constexpr int H = decltype(half)::value, BLOCKS = H ? C::MT - HM : HM;
+        const int km = AKM && C::BM != 160 && HM > 2 ? g3_opaque(kmA[0]) : kmA[0]; /* eight blocks' addresses kept would not leave room for the fragments */
+#pragma unroll
+        for (int mh = 0; mh < BLOCKS; mh++)
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
-                const int mt = half * HM + mh;
+                const int mt = H * HM + mh;
                 if constexpr (ROWS::TILED) f[mh][kk] = *reinterpret_cast<const bf16x8*>(tile + ((wm * C::MT + mt) * 2 + kk) * 1024 + lane * 16);
-                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(tile, km, wm * C::MT + mt, kk);
+                else if constexpr (AKM) f[mh][kk] = g3_frag_km<C::BM>(tile, C::BM == 160 && (mt & 1) ? kmA[1] : km, wm * C::MT + mt, kk);
                 else f[mh][kk] = g3_frag(tile, (wm * C::MT + mt) * 16 + r16, kk * 4 + q4);
             }
     };
-    auto readB = [&](const unsigned char* tile, int half, bf16x8 (&f)[HN][2]) {
-        const int km = BKM && C::BN > 128 ? g3_opaque(kmB) : kmB;
+    auto readB = [&](const unsigned char* tile, auto half, bf16x8 (&f)[HN][2]) {
+        constexpr int H = decltype(half)::value, BLOCKS = H ? C::NT - HN : HN;
+        const int km = BKM && C::BN != 160 && C::BN > 128 ? g3_opaque(kmB[0]) : kmB[0];
 #pragma unroll
-        for (int nh = 0; nh < HN; nh++)
+        for (int nh = 0; nh < BLOCKS; nh++)
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
-                const int nt = half * HN + nh;
-                if constexpr (BKM) f[nh][kk] = g3_frag_km<C::BN>(tile, km, wn * C::NT + nt, kk);
+                const int nt = H * HN + nh;
+                if constexpr (BKM) f[nh][kk] = g3_frag_km<C::BN>(tile, C::BN == 160 && (nt & 1) ? kmB[1] : km, wn * C::NT + nt, kk);
                 else f[nh][kk] = g3_frag(tile, wn * (16 * C::NT) + nt * 16 + r16, kk * 4 + q4);
             }
     };
     constexpr int PIECES = ROWS::F32 ? 4 : 1; /* MFMAs per pair of fragments */
-    auto mul = [&](int mh0, int nh0, const bf16x8 (&fa)[HM][2], const bf16x8 (&fb)[HN][2]) {
+    auto mul = [&](auto mh0, auto nh0, const bf16x8 (&fa)[HM][2], const bf16x8 (&fb)[HN][2]) {
+        constexpr int I0 = decltype(mh0)::value * HM, J0 = decltype(nh0)::value * HN;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++)
 #pragma unroll
             for (int e = 0; e < PIECES; e++)
 #pragma unroll
-                for (int i = 0; i < HM; i++)
+                for (int i = 0; i < (I0 ? C::MT - HM : HM); i++)
 #pragma unroll
-                    for (int j = 0; j < HN; j++) {
-                        f32x4& d = acc[mh0 * HM + i][nh0 * HN + j];
+                    for (int j = 0; j < (J0 ? C::NT - HN : HN); j++) {
+                        f32x4& d = acc[I0 + i][J0 + j];
                         if constexpr (ROWS::F32) d = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4, fa[i][kk])[e], __builtin_bit_cast(f32x4, fb[j][kk])[e], d, 0, 0, 0);
                         else d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][kk], fb[j][kk], d, 0, 0, 0);
                     }
     };
-    // a quadrant's issue order: its LDS reads and its loads one by one among its first MFMAs, the rest of the MFMAs behind them
-    auto order = [&](auto n_reads, auto n_loads) {
-        constexpr int N = decltype(n_reads)::value, V = decltype(n_loads)::value, M = HM * HN * 2 * PIECES, P = N < M ? N : M, Q = V < M - 1 ? V : M - 1, X = P > Q ? P : Q;
-#pragma unroll
-        for (int i = 0; i < X; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < P) __builtin_amdgcn_sched_group_barrier(0x100, N / P, 0);
-            if (i < Q) __builtin_amdgcn_sched_group_barrier(0x010, V / (Q ? Q : 1), 0);
-        }
+    // the issue order of quadrant (row half, token half): its LDS reads and its loads one by one among its first MFMAs, the rest of the MFMAs behind them
+    auto order = [&](auto mh, auto nh, auto n_reads, auto n_loads) {
+        constexpr int N = decltype(n_reads)::value, V = decltype(n_loads)::value, M = (decltype(mh)::value ? C::MT - HM : HM) * (decltype(nh)::value ? C::NT - HN : HN) * 2 * PIECES;
+        constexpr int P = N < M ? N : M, Q = V < M - 1 ? V : M - 1, X = P > Q ? P : Q;
+        g3_issue<M, N, V, 0>();
         if (M > X) __builtin_amdgcn_sched_group_barrier(0x008, M - X, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    constexpr std::integral_constant<int, HM * 2 * (AKM ? 2 : 1)> ra{};
-    constexpr std::integral_constant<int, HN * 2 * (BKM ? 2 : 1)> rb{};
+    constexpr std::integral_constant<int, HM * 2 * (AKM ? 2 : 1)> ra0{};
+    constexpr std::integral_constant<int, (C::MT - HM) * 2 * (AKM ? 2 : 1)> ra1{};
+    constexpr std::integral_constant<int, HN * 2 * (BKM ? 2 : 1)> rb0{};
+    constexpr std::integral_constant<int, (C::NT - HN) * 2 * (BKM ? 2 : 1)> rb1{};
     bf16x8 a0[HM][2], a1[HM][2], b0[HN][2], b1[HN][2];
     if (kt0 >= kt1) return;
     constexpr std::integral_constant<int, 0> none{};
@@ -277,24 +330,24 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     // step kt on the tiles ca, cb (which hold the step's loads, and then those of step kt + NBUF); those of step kt + 1 are at na, nb.  Behind the last step the reads of "step kt + 1" take what lies there: never used
     auto step = [&](int kt, unsigned char* ca, unsigned char* cb, const unsigned char* na, const unsigned char* nb, bf16x8 (&bx)[HN][2], bf16x8 (&by)[HN][2]) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
-        readB(cb, 1, by);
-        mul(0, 0, a0, bx);
-        order(rb, none);
-        readA(ca, 1, a1);
-        mul(0, 1, a0, by);
-        order(ra, none);
+        readB(cb, hi, by);
+        mul(lo, lo, a0, bx);
+        order(lo, lo, rb1, none);
+        readA(ca, hi, a1);
+        mul(lo, hi, a0, by);
+        order(lo, hi, ra1, none);
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((C::NBUF - 2) * LPW) : "memory");
         __builtin_amdgcn_s_barrier(); /* step kt + 1 has landed for every wave, and every wave has read all of step kt: its buffer may be filled again */
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         stageA(kt + C::NBUF, ca);
-        readA(na, 0, a0);
-        mul(1, 1, a1, by);
-        order(ra, la);
+        readA(na, lo, a0);
+        mul(hi, hi, a1, by);
+        order(hi, hi, ra0, la);
         stageB(kt + C::NBUF, cb);
-        readB(nb, 0, by);
-        mul(1, 0, a1, bx);
-        order(rb, lb);
+        readB(nb, lo, by);
+        mul(hi, lo, a1, bx);
+        order(hi, lo, rb0, lb);
     };
     // the steps are unrolled by two: the two token halves' registers swap roles with them, and of two buffers every LDS address of a step is base + an immediate
     [[maybe_unused]] auto two = [&](unsigned char* a_even, unsigned char* a_odd, unsigned char* b_even, unsigned char* b_odd) {
@@ -302,7 +355,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory"); /* no read moves up */
-        readA(a_even, 0, a0), readB(b_even, 0, b0);
+        readA(a_even, lo, a0), readB(b_even, lo, b0);
         for (int kt = kt0; kt < kt1; kt += 2) {
             between(kt);
             step(kt, a_even, b_even, a_odd, b_odd, b0, b1);
@@ -316,7 +369,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory"); /* no read moves up */
-        readA(a_0, 0, a0), readB(b_0, 0, b0);
+        readA(a_0, lo, a0), readB(b_0, lo, b0);
         for (int kt = kt0;;) {
             between(kt), step(kt, a_0, b_0, a_1, b_1, b0, b1);
             if (++kt >= kt1) break;
@@ -349,15 +402,17 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
 template <class C>
 struct G3Out {
     static constexpr int PASSES = (C::BM * C::BN * 4 + C::SMEM - 1) / C::SMEM, TN = C::BN / PASSES, HT = C::NT / PASSES; /* tokens, and 16-token blocks of a wave, per pass */
-    static_assert(PASSES <= 2 && C::NT % PASSES == 0 && C::BM % 64 == 0, "a token is whole turns of the banks");
-    static __device__ __forceinline__ int at(int lt, int chunk) { return lt * (4 * C::BM) + ((chunk ^ (lt & 15)) << 4); } /* rows 4 chunk .. + 3 of the pass's token lt */
+    static constexpr int P = C::BM % 64 == 0 ? 1 : 2; /* tokens whose rows start at different banks */
+    static_assert(PASSES <= 2 && C::NT % PASSES == 0 && C::BM % 32 == 0, "a token is whole or half turns of the banks");
+    static __device__ __forceinline__ int swz(int lt) { return (lt / P) & (16 / P - 1); }
+    static __device__ __forceinline__ int at(int lt, int chunk) { return lt * (4 * C::BM) + ((chunk ^ swz(lt)) << 4); } /* rows 4 chunk .. + 3 of the pass's token lt */
     static __device__ __forceinline__ int token(int pass, int lt) { return PASSES == 1 ? lt : lt / (16 * HT) * (16 * C::NT) + pass * (16 * HT) + lt % (16 * HT); } /* its place in the tile */
     static __device__ __forceinline__ void spill(const f32x4 (&acc)[C::MT][C::NT], unsigned char* smem, int pass, int wid, int lane) {
         const int wm = wid / C::WN, wn = wid % C::WN, r16 = lane & 15, q4 = lane >> 4;
         unsigned char* const to = smem + (wn * (16 * HT) + r16) * (4 * C::BM); /* (16 tokens further the swizzle is the same) */
 #pragma unroll
         for (int mt = 0; mt < C::MT; mt++) {
-            unsigned char* const b = to + ((((wm * C::MT + mt) * 4 + q4) ^ r16) << 4);
+            unsigned char* const b = to + ((((wm * C::MT + mt) * 4 + q4) ^ swz(r16)) << 4);
 #pragma unroll
             for (int nt = 0; nt < HT; nt++) *reinterpret_cast<f32x4*>(b + nt * 16 * (4 * C::BM)) = PASSES == 2 && pass ? acc[mt][nt + C::NT - HT] : acc[mt][nt];
         }
@@ -403,8 +458,8 @@ __device__ __forceinline__ void g3_unpack8(u32x4 p, float (&v)[8]) {
 // at 8192 rows 125.7 | 120.3
 template <class C>
 struct G3Out16 {
-    static constexpr int ROW = (C::BM / 2) % 64, P = ROW == 0 ? 1 : 2; /* tokens whose rows start at different banks */
-    static_assert(C::BM * C::BN * 2 <= C::SMEM && C::BM % 64 == 0, "the tile fits, its chunks of eight rows in eights");
+    static constexpr int ROW = (C::BM / 2) % 64, P = ROW == 0 ? 1 : ROW == 32 ? 2 : 4; /* tokens whose rows start at different banks */
+    static_assert(C::BM * C::BN * 2 <= C::SMEM && C::BM % 32 == 0, "the tile fits, its chunks of eight rows in eights");
     static __device__ __forceinline__ int at(int tok, int chunk) { return tok * (2 * C::BM) + ((chunk ^ ((tok / P) & (16 / P - 1))) << 4); } /* rows 8 chunk .. + 7 of a token */
     template <bool BIAS>
     static __device__ __forceinline__ void spill(const f32x4 (&acc)[C::MT][C::NT], unsigned char* smem, int tid, const uint16_t* bias, int rows) { /* bias: of the tile's rows, `rows` of them exist */
@@ -453,7 +508,7 @@ static constexpr bool g3_prefer_wide(int M, int n, int K) {
 //   4096 x 1024   at 2047 rows 22.6 | 18.9 | 19.7 | 22.9 | 28.3, at 2608 32.6 | 34.5 | 31.1 | 24.6 | 30.1, at 4096 48.0 | 39.3 | 38.5 | 48.1 | 33.3
 //   6144 x 1024 with SwiGLU at 2047 rows 36.9 | 40.0 | 35.1 | 29.2 | 36.0, at 2608 47.5 | 58.3 | 39.9 | 53.5 | 67.9
 //   6400 x 1600 at 8192 rows 191 | 174 | 169 | 164 | 169, 12288 x 2048 with SwiGLU at 8190 rows 448 | 372 | 368 | 339 | 327
-enum G3Pick { G3_DUO, G3_HALF, G3_SMALL, G3_WIDE, G3_BIG };
+enum G3Pick { G3_DUO, G3_HALF, G3_SMALL, G3_WIDE, G3_BIG, G3_SLIM, G3_FLAT };
 static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
     const long r128 = (M + 127) / 128, c128 = (n + 127) / 128, c256 = (n + 255) / 256, n128 = r128 * c128, nw = (M + 191) / 192 * c256, nb = (M + 255) / 256 * c256;
     if (n128 <= 256) return G3_DUO;
@@ -465,6 +520,17 @@ static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
     const double k = K / 64, rs = n128 / 512.0, rb = (w ? nw : nb) / 256.0, Rs = 3.7 + k, Rb = w ? 9.0 + 1.26 * k : 10.1 + 1.45 * k;
     const double ts = Rs * ((n128 + 511) / 512 + 0.8 * rs + 0.55), tb = Rb * (((w ? nw : nb) + 255) / 256 + 0.8 * rb + 0.55);
     return ts < 0.97 * tb ? G3_SMALL : w ? G3_WIDE : G3_BIG;
+}
+// Products with a k-major W (both GEMMs of a backward pass): 160 x 256 or 256 x 160 instead of 256 x 256 where they need no more rounds.  A big tile's round on three quarters of the CUs was cut in k-pieces over all of
+// them, whose partial tiles (256 KiB each, written and read) took what the idle CUs had been worth and more; five eighths of a tile on nearly all CUs needs none.  us, pieces | 256 x 256 whole | 160 x 256 | 256 x 160:
+//   weight gradients (bkm)  1600 x 6400 from 8192 tokens 167 | 166 | 136 | 241, 6400 x 1600 166 | 170 | 233 | 147, 1600 x 6400 from 2560 80 | 62 | 51 | 88, 4096 x 2560 from 8192 154 | 167 | 236 | 150,
+//                           3000 x 3000 from 4096 95 | 90 | 75 | 72, 2400 x 3600 from 2048 63 | 52 | 42 | 41
+//   input gradients         1600 x 5120 rows, K 6400: 112 | 119 | 93 | 99, 1600 x 6000, K 1600: 37 | 37 | 29 | 53, 6400 x 3000, K 1600 (two rounds each) - | 75 | 59 | 61
+// One round more for four big ones gains at most 3 % (6400 x 8192, K 1600: - | 158 | 155 | 171) and is not taken.  Of both with as many rounds: us of weight gradients 75 | 72, of input gradients 92 | 97.
+static constexpr G3Pick g3_km_pick(int M, int n, bool bkm) {
+    const long nb = (long)((M + 255) / 256) * ((n + 255) / 256), rb = (nb + 255) / 256, rs = ((long)((M + 159) / 160) * ((n + 255) / 256) + 255) / 256, rf = ((long)((M + 255) / 256) * ((n + 159) / 160) + 255) / 256;
+    if (nb <= 128 || (rs < rf ? rs : rf) > rb) return G3_BIG; /* (up to 128: two and more pieces of a tile, or tiles of 128 x 128) */
+    return rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
 }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {

@@ -113,6 +113,15 @@ def test_linear_backward_large_k_major(ctx, t, shape, accumulate):
     _run(ctx, t, OC, IC, n, accumulate)
 
 
+@pytest.mark.parametrize("shape", [(6336, 1592, 128), (6400, 1600, 192), (3008, 3000, 320), (1600, 6400, 448), (128, 1592, 5056), (192, 2048, 5120), (448, 6392, 2944)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_linear_backward_tiles_of_160(ctx, shape, accumulate):
+    """160 x 256 and 256 x 160 tiles of k-major operands: weight gradients (the first four: rows of either side past the last whole tile, K of two, three, five and seven steps, fewer than the three
+    buffers' turns and not) and input gradients (160 x 256 of one round, 256 x 160, 160 x 256 of two rounds)"""
+    OC, IC, n = shape
+    _run(ctx, L.BF16, OC, IC, n, accumulate)
+
+
 def test_linear_backward_split_k_is_deterministic(ctx):
     """the split-K forms add a tile's partial sums in slot order, not in arrival order: two runs give the same bits (49-tile weight gradient = 5 pieces per
     tile; 133 tiles = owners + helpers on tails)"""

@@ -33,6 +33,19 @@ def test_one_round_of_tiles_is_taken_where_there_is_one(tmp_path):
     assert r.returncode == 0, r.stderr[-3000:]
 
 
+# (rows, token rows, either operand k-major or one, the tile): as timed, and at the edges of the rule
+KM_PICKED = [(1600, 6400, True, "SLIM"), (6400, 1600, True, "FLAT"), (4096, 2560, True, "FLAT"), (3000, 3000, True, "FLAT"), (1600, 5120, False, "SLIM"), (6400, 3000, False, "SLIM"), (2048, 5120, False, "FLAT"),
+             (1600, 8192, False, "BIG"), (6400, 8192, False, "BIG"), (4800, 5120, False, "BIG"), (2048, 4096, True, "BIG"), (2049, 4096, True, "FLAT"), (1608, 6400, True, "BIG")]
+
+
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_tiles_of_160_are_taken_where_they_need_no_more_rounds(tmp_path):
+    src = tmp_path / "rules.hip"
+    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_pick(%d, %d, %s) == kf::G3_%s);\n" % (m, n, str(b).lower(), t) for m, n, b, t in KM_PICKED))
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+
 # (pieces of 8 weights, matrices interleaved, offsets of the copy in 32 bits): gate and up of 65552 x 16384 lie in 4 296 015 872 bytes
 REACH = [(65552 * 16384 // 8, 1, True), (65552 * 16384 // 8, 2, False), (65536 * 16384 // 8 - 1, 2, True), ((1 << 28) - 1, 1, True), (1 << 28, 1, False), ((1 << 31) - 1, 2, False)]
 
