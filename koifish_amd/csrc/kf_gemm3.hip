@@ -542,6 +542,7 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
                     const uint16_t* bias, float alpha, float beta, void* ws, size_t ws_bytes) {
     if (K % G3_BK != 0 || K < G3_BK || n < G3_BN || M < G3_BM || (M & 7) || (n & 7) || (lda & 7) || (ldb & 7)) return 1;
     if ((reinterpret_cast<uintptr_t>(A) & 15) || (reinterpret_cast<uintptr_t>(B) & 15)) return 1;
+    if ((akm && lda >= (1 << 24)) || (bkm && ldb >= (1 << 24))) return 1; /* up to 64 k-rows of an operand are a load's scalar and lane offsets: 31 bits */
     const long nwg = (long)((M + G3_BM - 1) / G3_BM) * ((n + G3_BN - 1) / G3_BN);
     GemmArgs a;
     memset(&a, 0, sizeof(a));
