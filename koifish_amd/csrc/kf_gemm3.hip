@@ -7,7 +7,7 @@
 //   * two or three LDS buffers (G3Cfg::NBUF): the loads of a later k-step are issued among the MFMAs of this one, the fragments of a quadrant are read while the one before is multiplied, and ONE raw
 //     s_barrier per step, behind a wait, by count, for the next step's loads;
 //   * 256 x 256: 8 waves as 2 (rows) x 4 (tokens), 128 x 64 outputs per wave = 32 accumulator tiles of v_mfma_f32_16x16x32_bf16, one workgroup per CU.  A product takes the smallest tile that makes one
-//     round of the CUs, of several rounds the cheaper one (g3_pick; kf_gemm3_tile.h lists the tiles).  All of them add up a k in the same order;
+//     round of the CUs, of several rounds the cheaper one (g3_pick; of k-major operands g3_km_pick; kf_gemm3_tile.h lists the tiles).  All of them add up a k in the same order;
 //   * workgroup order remapped so that the blocks an XCD runs back to back share their W row-tile in that XCD's L2;
 //   * split-K forms (gemm3_sk_kernel) with an ordered in-kernel fix-up for launches with fewer tiles than resident workgroups: deterministic, no atomics on data;
 //   * up to three matrices stacked along M (Q | K | V, gate | up) in one launch, each tile's rows routed to its matrix's output (gemm3_multi_launch).
@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(C::NTH, C::WGS_PER_CU * C::NW / 4) gemm3_piece
     g3_epilogue<false, C>(a, m0, t0, acc, e, smem_raw);
 }
 
-// SPLIT-K forms for launches with fewer tiles than CUs (a weight gradient [OC, IC] is 49 .. 175 tiles, its contraction 8192 token rows long).  The pieces are cut so
+// SPLIT-K forms for launches with fewer tiles than CUs (a weight gradient [OC, IC] of 49 tiles, its contraction 8192 token rows long; where tiles of 160 make one round they are taken instead).  The pieces are cut so
 // that the workgroups an XCD runs side by side stay at (nearly) the SAME k: they share operand strips in that XCD's L2.  (Ranges of a plain stream-K cut drift apart
 // in k and every workgroup then streams its own strips through the fabric -- measured: 496 TFLOP/s.)
 //   S >= 2 (2 P <= 256):  every tile's k-steps are cut in S equal pieces, P S workgroups; piece 0 owns the tile;
@@ -431,6 +431,7 @@ template <bool KM, class C>
 static bool g3_cut(long nwg, int nkt, G3SkArgs& s, int& nlaunch) {
     const int G = 256 * C::WGS_PER_CU, min_steps = 512 / G3_BK;
     if (5 * nwg >= 4 * G || !(KM || 3 * nwg <= G || nkt >= 48)) return false;
+    if (2 * nwg > G && nkt < g3_tails_from(C::BM)) return false;
     s.P = (int)nwg, s.S = G / s.P, s.kp = 0, s.R = 1;
     if (s.S >= 2) {
         while (s.S > 1 && nkt / s.S < min_steps) s.S--;
@@ -441,7 +442,7 @@ static bool g3_cut(long nwg, int nkt, G3SkArgs& s, int& nlaunch) {
     nlaunch = G;
     const long long T = (long long)s.P * (nkt - s.kp);
     s.R = (int)((T + (G - s.P) - 1) / (G - s.P));
-    return nkt - s.kp >= 1 && nkt >= 4 * min_steps && T * 2 < (1LL << 31) && s.kp > 0;
+    return nkt - s.kp >= 1 && T * 2 < (1LL << 31) && s.kp > 0;
 }
 // KF_OK launched, 1 = not for this kernel (the caller's other tile kernels take the shape), < 0 error.  bf16 "weights" only: quantised ones are dequantised first.
 // BK = 32 (4 LDS buffers, three steps in flight) was measured 8-10 % slower than BK = 64 (2 buffers) on every shape, forward and backward: the per-step costs

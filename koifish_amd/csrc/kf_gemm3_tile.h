@@ -10,7 +10,7 @@ namespace kf {
 constexpr int G3_BM = 256, G3_BN = 256, G3_BK = 64;
 // the workgroup tile: BM rows x BN tokens, NW waves as NW / WN_ (rows; 2 by default) x WN_ (tokens), NBUF LDS buffers: the loads of NBUF - 1 later k-steps are in flight under the step that is multiplied.
 // A step is bound by those loads, not by its MFMAs (loads alone take 85 - 95 % of every configuration's time), and with two buffers a lone workgroup of a CU waits out their latency: us per
-// step with one workgroup on every CU, two buffers | more: 64 x 64 0.41 | 0.23 (3), 128 x 128 on 8 waves 0.89 | 0.58 (3), 128 x 256 0.82 (3) against 1.26 of 192 x 256 (2: three do not fit).
+// step with one workgroup on every CU, two buffers | more: 64 x 64 0.41 | 0.23 (3), 128 x 128 on 8 waves 0.89 | 0.58 (3), 128 x 256 0.75 (3) against 1.26 of 192 x 256 (2: three do not fit).
 // Where an operand's instructions are no multiple of the waves (EVEN false: 160 rows are 20) the first waves issue one more; the others' last one has an empty descriptor and
 // a KiB of its own behind the buffers (SPARE), so that every wave counts the same loads.  SMEM then is the whole LDS: the tile in 32 bits fits.
 template <int BM_, int BN_, int NW_, int NBUF_ = 2, int WN_ = NW_ / 2>
@@ -532,6 +532,9 @@ static constexpr G3Pick g3_km_pick(int M, int n, bool bkm) {
     if (nb <= 128 || (rs < rf ? rs : rf) > rb) return G3_BIG; /* (up to 128: two and more pieces of a tile, or tiles of 128 x 128) */
     return rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
 }
+// Where a launch of more than half a round may be cut in owners and tails (gemm3_sk_kernel, S = 1): k-steps.  The tails of 256 x 256 tiles are 256 KiB each, and up to K = 8192 they take what the idle CUs are worth
+// or more; us, cut | whole: 1600 x 6400 (175 tiles) from 8192 tokens 167 | 166, from 2560 80 | 62; 3000 x 3000 (144) from 4096 95 | 90; 2400 x 3600 (150) from 2048 63 | 52; 1600 x 5120, K 6400 (140) 112 | 119
+static constexpr int g3_tails_from(int bm) { return bm == 256 ? 129 : 32; }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {
     const int q = nwg / 8, rr = nwg % 8, xcd = orig % 8;

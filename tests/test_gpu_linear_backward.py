@@ -122,6 +122,11 @@ def test_linear_backward_tiles_of_160(ctx, shape, accumulate):
     _run(ctx, L.BF16, OC, IC, n, accumulate)
 
 
+def test_linear_backward_tails_of_big_tiles(ctx):
+    """a weight gradient of 175 big tiles (tiles of 160 would be two rounds) from 8256 tokens: owners and helpers on tails"""
+    _run(ctx, L.BF16, 6400, 1608, 8256, False)
+
+
 def test_linear_backward_split_k_is_deterministic(ctx):
     """the split-K forms add a tile's partial sums in slot order, not in arrival order: two runs give the same bits (49-tile weight gradient = 5 pieces per
     tile; 133 tiles = owners + helpers on tails)"""

@@ -46,6 +46,14 @@ def test_tiles_of_160_are_taken_where_they_need_no_more_rounds(tmp_path):
     assert r.returncode == 0, r.stderr[-3000:]
 
 
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_big_tiles_have_tails_cut_off_behind_k_8192_only(tmp_path):
+    src = tmp_path / "rules.hip"
+    src.write_text('#include "%s/kf_gemm3_tile.h"\nstatic_assert(8192 / 64 < kf::g3_tails_from(256) && 8192 / 64 + 1 >= kf::g3_tails_from(256) && kf::g3_tails_from(128) == 2048 / 64);\n' % B.CSRC)
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+
 # (pieces of 8 weights, matrices interleaved, offsets of the copy in 32 bits): gate and up of 65552 x 16384 lie in 4 296 015 872 bytes
 REACH = [(65552 * 16384 // 8, 1, True), (65552 * 16384 // 8, 2, False), (65536 * 16384 // 8 - 1, 2, True), ((1 << 28) - 1, 1, True), (1 << 28, 1, False), ((1 << 31) - 1, 2, False)]
 
