@@ -393,6 +393,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     [[maybe_unused]] const uint32_t ldb = (uint32_t)a.ldx * 2;
     auto xload = [&](int u0, int slot) {
 #ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the slot's reads have their values: nothing else orders a load into LDS behind them */
         const long long left = ((long long)a.n - tok0) * ldb - (long long)u0 * 128;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x) + (size_t)tok0 * a.ldx + (size_t)u0 * 64, 0, (int)(left < 0x7FFFFFFFll ? left : 0x7FFFFFFFll), 0x00020000);
 #pragma unroll
@@ -577,6 +578,7 @@ __global__ void __launch_bounds__(512) gemm_direct16_kernel(const GemmArgs a0, i
     };
     auto gload = [&](int u0, Group& g, int slot) { /* as gemm_direct_kernel's: the token rows first, whole lines to this wave's own LDS; units past the end repeat the last one */
 #ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the slot's reads have their values */
         const long long left = ((long long)a.n - tok0) * ldb - (long long)u0 * 128;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.x) + (size_t)tok0 * a.ldx + (size_t)u0 * 64, 0, (int)(left < 0x7FFFFFFFll ? left : 0x7FFFFFFFll), 0x00020000);
 #pragma unroll
