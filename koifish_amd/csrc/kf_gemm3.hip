@@ -543,7 +543,7 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
                     const uint16_t* bias, float alpha, float beta, void* ws, size_t ws_bytes) {
     if (K % G3_BK != 0 || K < G3_BK || n < G3_BN || M < G3_BM || (M & 7) || (n & 7) || (lda & 7) || (ldb & 7)) return 1;
     if ((reinterpret_cast<uintptr_t>(A) & 15) || (reinterpret_cast<uintptr_t>(B) & 15)) return 1;
-    if ((akm && lda >= (1 << 24)) || (bkm && ldb >= (1 << 24))) return 1; /* up to 64 k-rows of an operand are a load's scalar and lane offsets: 31 bits */
+    if ((akm && !g3_km_reach<G3_BM>(lda)) || (bkm && !g3_km_reach<G3_BN>(ldb))) return 1;
     const long nwg = (long)((M + G3_BM - 1) / G3_BM) * ((n + G3_BN - 1) / G3_BN);
     GemmArgs a;
     memset(&a, 0, sizeof(a));
@@ -554,9 +554,9 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
     // workspace -- their split-K form (partials of 64 KiB instead of 256 KiB, twice the workgroups)
     // (measured: Qwen3-0.6B training step 99.3 -> 95.7 ms with the first rule alone, -> 87.2 ms with both; GPT2-1558M 166.0 -> 163.7 -> 161.2 ms)
     const long nws = (long)((M + 127) / 128) * ((n + 127) / 128), rounds = (nws + 511) / 512;
-    const bool small = 5 * nwg < 4 * 256 && akm && (20 * nws >= 17 * rounds * 512 || (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nws < 4 * 512));
+    const bool small = 5 * nwg < 4 * 256 && akm && g3_km_reach<128>(lda) && (!bkm || g3_km_reach<128>(ldb)) && (20 * nws >= 17 * rounds * 512 || (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nws < 4 * 512));
     if (small) return bkm ? g3_go_c<true, true, G3Small>(st, a, nws, ws, ws_bytes, 1) : g3_go_c<true, false, G3Small>(st, a, nws, ws, ws_bytes, 1);
-    switch (akm ? g3_km_pick(M, n, bkm) : G3_BIG) {
+    switch (akm ? g3_km_pick(M, n, bkm, lda, bkm ? ldb : 0) : G3_BIG) {
         case G3_SLIM: return bkm ? g3_whole<G3Slim, true, true>(st, a) : g3_whole<G3Slim, true, false>(st, a);
         case G3_FLAT: return bkm ? g3_whole<G3Flat, true, true>(st, a) : g3_whole<G3Flat, true, false>(st, a);
         default: break;

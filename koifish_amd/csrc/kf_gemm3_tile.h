@@ -78,6 +78,16 @@ __device__ __forceinline__ bf16x8 g3_frag(const unsigned char* tile, int row, in
 // its 128-byte quarters by bit 3 of k, so that the transposing fragment read below (per 32 lanes: k-rows k .. k+3 and k+8 .. k+11, 32 bytes of each) touches all 64
 // banks once (without the second term the two 16-lane halves meet in the same 32 banks: SQ_LDS_BANK_CONFLICT = 50 % of the LDS cycles, measured).
 // A k-row of 160 rows is 20 chunks, 64 bytes past whole turns of the banks, so four k-rows meet in no bank as they are and only bit 3 of k moves a block, to its neighbour; five instructions are 16 k-rows.
+// A base serves the loads of a wave and step (of a step, 160 rows): the k-rows between them are scalar offsets, a lane's own k-row and column the lane part, all below the descriptor's end, G3_ALL.
+template <int ROWS>
+struct G3Km {
+    static constexpr int INST = ROWS == 160 ? 16 : 512 / ROWS;      /* k-rows of a scalar step: of an instruction, of five (160) */
+    static constexpr int SPAN = 4 * INST;                            /* k-rows that a base's offsets lie in */
+    static constexpr int part(int i) { return ROWS == 160 ? i : ROWS == 128 ? i >> 1 : i & 1; }        /* which lane part instruction i of a wave takes */
+    static constexpr int steps(int first, int i) { return ROWS == 160 ? (first + i) / 5 : i; }        /* and how many scalar steps */
+};
+template <int ROWS>
+static constexpr bool g3_km_reach(long long ld) { return 2 * ld * G3Km<ROWS>::SPAN <= (long long)G3_ALL; } /* a row of ld values in reach: up to 2^24 - 8 (160), 2^26 - 8 (128), 2^27 - 8 (256) */
 // ROWS = the tile's rows (256, 160 or 128): a k-row of the image is 2 ROWS bytes = CPK chunks of 16 bytes, one wave instruction covers 64 / CPK k-rows, wave `wid` issues
 // instructions NI wid .. NI wid + NI - 1 of the ROWS / 8
 template <int ROWS, int NI>
@@ -87,7 +97,7 @@ __device__ __forceinline__ G3Src g3_src_km(const uint16_t* __restrict__ src, lon
     if constexpr (ROWS == 160) {
         static_assert(NI == 3, "a lane part per instruction");
         const int first = G3Share<160, 8>::first(wid);
-        s.base = reinterpret_cast<const unsigned char*>(src), s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = 32 * ld; /* (inst: 16 k-rows, five instructions) */
+        s.base = reinterpret_cast<const unsigned char*>(src), s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = (long long)G3Km<ROWS>::INST * ld * 2;
 #pragma unroll
         for (int v = 0; v < 3; v++) {
             const int at = (first + v) % 5 * 64 + lane, kr = at / CPK, p = at % CPK, c = p ^ (((kr >> 3) & 1) << 1);
@@ -99,7 +109,7 @@ __device__ __forceinline__ G3Src g3_src_km(const uint16_t* __restrict__ src, lon
     }
     static_assert(ROWS == 160 || ((ROWS == 256 || ROWS == 128) && NI == 4), "two lane parts per wave");
     s.base = reinterpret_cast<const unsigned char*>(src + (size_t)wid * NI * KPI * ld);
-    s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = (long long)KPI * ld * 2; /* every k-row of the steps exists; chunks past a row's end are clamped here */
+    s.left = -1, s.step = (long long)G3_BK * ld * 2, s.inst = (long long)G3Km<ROWS>::INST * ld * 2; /* every k-row of the steps exists; chunks past a row's end are clamped here */
 #pragma unroll
     for (int v = 0; v < 2; v++) {
         const int kr = (wid * NI + v * UNIT) * KPI + lane / CPK, p = lane % CPK, c = p ^ ((kr & 3) << 1) ^ (((kr >> 3) & 1) << 3);
@@ -228,9 +238,9 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
     auto rest = [](long long left) { return (uint32_t)(left < 0 ? 0 : (left > 0xFFFFFFFFll ? 0xFFFFFFFFll : left)); };
     auto atA = [&](int i) {
         const int j = firstA + i; /* tile (row block j / 2, k-half j % 2) of the workgroup's */
-        return ROWS::TILED ? sa.inst * (j >> 1) + (j & 1) * 1024 : AKM && C::BM == 160 ? sa.inst * (j / 5) : sa.inst * i;
+        return ROWS::TILED ? sa.inst * (j >> 1) + (j & 1) * 1024 : AKM ? sa.inst * G3Km<C::BM>::steps(firstA, i) : sa.inst * i;
     };
-    [[maybe_unused]] auto atB = [&](int i) { return BKM && C::BN == 160 ? sb.inst * ((firstB + i) / 5) : sb.inst * i; };
+    [[maybe_unused]] auto atB = [&](int i) { return BKM ? sb.inst * G3Km<C::BN>::steps(firstB, i) : sb.inst * i; };
 #pragma unroll
     for (int i = 0; i < C::NIA; i++) restA[i] = !ShareA::has(wid, i) ? 0 : AKM ? G3_ALL : rest(sa.left - atA(i));
 #pragma unroll
@@ -243,7 +253,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
         for (int i = 0; i < C::NIA; i++) {
             [[maybe_unused]] const auto at = to(tile, firstA + i, ShareA::has(wid, i));
             [[maybe_unused]] const uint32_t n = kt < kt1 ? restA[i] : 0;
-            if constexpr (AKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextA, kt < kt1 ? G3_ALL : 0), at, 16, sa.lane[C::BM == 160 ? i : C::BM == 128 ? i >> 1 : i & 1], (int)atA(i), 0, 0);
+            if constexpr (AKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextA, kt < kt1 ? G3_ALL : 0), at, 16, sa.lane[G3Km<C::BM>::part(i)], (int)atA(i), 0, 0);
             else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sa.base + atA(i), n), at, 16, sa.lane[ROWS::TILED ? 0 : i & 1], (int)sa.step * kt, 0, 0);
         }
         if constexpr (AKM) nextA += sa.step;
@@ -256,7 +266,7 @@ __device__ __forceinline__ void g3_mainloop(const GemmArgs& a, int m0, int t0, i
             [[maybe_unused]] const auto at = to(tile, firstB + i, ShareB::has(wid, i));
             [[maybe_unused]] const uint32_t n = kt < kt1 ? restB[i] : 0;
             if constexpr (ROWS::GATHER) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gat[i] + (size_t)(kt < kt1 ? kt : kt1 - 1) * BK), at, 16, 0, 0); /* (past the end: the last step again) */
-            else if constexpr (BKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextB, kt < kt1 ? G3_ALL : 0), at, 16, sb.lane[C::BN == 160 ? i : C::BN == 128 ? i >> 1 : i & 1], (int)atB(i), 0, 0);
+            else if constexpr (BKM) __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(nextB, kt < kt1 ? G3_ALL : 0), at, 16, sb.lane[G3Km<C::BN>::part(i)], (int)atB(i), 0, 0);
             else __builtin_amdgcn_raw_ptr_buffer_load_lds(g3_rsrc(sb.base + atB(i), n), at, 16, sb.lane[i & 1], (int)sb.step * kt, 0, 0);
         }
         if constexpr (BKM) nextB += sb.step;
@@ -527,10 +537,12 @@ static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
 //                           3000 x 3000 from 4096 95 | 90 | 75 | 72, 2400 x 3600 from 2048 63 | 52 | 42 | 41
 //   input gradients         1600 x 5120 rows, K 6400: 112 | 119 | 93 | 99, 1600 x 6000, K 1600: 37 | 37 | 29 | 53, 6400 x 3000, K 1600 (two rounds each) - | 75 | 59 | 61
 // One round more for four big ones gains at most 3 % (6400 x 8192, K 1600: - | 158 | 155 | 171) and is not taken.  Of both with as many rounds: us of weight gradients 75 | 72, of input gradients 92 | 97.
-static constexpr G3Pick g3_km_pick(int M, int n, bool bkm) {
+// 160-row tiles of an operand whose rows are in their reach (ldw: of W, ldx: of x where it is k-major too, else 0); a row beyond it is 2^24 values and more, and the big tiles reach to 2^27.
+static constexpr G3Pick g3_km_pick(int M, int n, bool bkm, long long ldw, long long ldx) {
     const long nb = (long)((M + 255) / 256) * ((n + 255) / 256), rb = (nb + 255) / 256, rs = ((long)((M + 159) / 160) * ((n + 255) / 256) + 255) / 256, rf = ((long)((M + 255) / 256) * ((n + 159) / 160) + 255) / 256;
     if (nb <= 128 || (rs < rf ? rs : rf) > rb) return G3_BIG; /* (up to 128: two and more pieces of a tile, or tiles of 128 x 128) */
-    return rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
+    const G3Pick p = rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
+    return g3_km_reach<160>(p == G3_SLIM ? ldw : ldx) ? p : G3_BIG;
 }
 // Where a launch of more than half a round may be cut in owners and tails (gemm3_sk_kernel, S = 1): k-steps.  The tails of 256 x 256 tiles are 256 KiB each, and up to K = 8192 they take what the idle CUs are worth
 // or more; us, cut | whole: 1600 x 6400 (175 tiles) from 8192 tokens 167 | 166, from 2560 80 | 62; 3000 x 3000 (144) from 4096 95 | 90; 2400 x 3600 (150) from 2048 63 | 52; 1600 x 5120, K 6400 (140) 112 | 119

@@ -41,9 +41,38 @@ KM_PICKED = [(1600, 6400, True, "SLIM"), (6400, 1600, True, "FLAT"), (4096, 2560
 @pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
 def test_tiles_of_160_are_taken_where_they_need_no_more_rounds(tmp_path):
     src = tmp_path / "rules.hip"
-    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_pick(%d, %d, %s) == kf::G3_%s);\n" % (m, n, str(b).lower(), t) for m, n, b, t in KM_PICKED))
+    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_pick(%d, %d, %s, %d, %d) == kf::G3_%s);\n" % (m, n, str(b).lower(), m, n if b else 0, t) for m, n, b, t in KM_PICKED))
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
+
+
+# (rows of the image, the longest k-row in reach): the last byte that a base's scalar and lane offsets name lies below the descriptor's end, with eight values more it does not
+KM_REACH = [(128, 2 ** 26 - 8), (160, 2 ** 24 - 8), (256, 2 ** 27 - 8)]
+
+
+def _last_byte(rows, ld):
+    """of the loads that share a base, as g3_src_km deals them: chunk by chunk along the k-rows, 64 lanes an instruction, eight waves of 160 rows (20 instructions), else four instructions a wave"""
+    chunks, end = rows // 8, 0
+    for i in range(20 if rows == 160 else 4):
+        scalar = (i // 5) * 16 if rows == 160 else i * (64 // chunks)
+        for lane in range(64):
+            kr = ((i % 5) * 64 + lane) // chunks if rows == 160 else lane // chunks
+            assert scalar + kr == (i * 64 + lane) // chunks
+            end = max(end, scalar * 2 * ld + kr * 2 * ld + (ld - 8) * 2 + 16)
+    return end
+
+
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_k_rows_are_in_reach_of_the_offsets_of_their_tile(tmp_path):
+    """and a longer row than the 160-row tiles reach takes the big tiles: transposed it would be a product that the other kernels refuse (2^24 x 2048: 2^32 pieces of eight)"""
+    src = tmp_path / "rules.hip"
+    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_reach<%d>(%d) && !kf::g3_km_reach<%d>(%d));\n" % (r, ld, r, ld + 8) for r, ld in KM_REACH)
+                   + "static_assert(kf::g3_km_pick(1600, 6400, true, 1600, 6400) == kf::G3_SLIM && kf::g3_km_pick(1600, 6400, true, 1 << 24, 6400) == kf::G3_BIG && kf::g3_km_pick(6400, 1600, true, 6400, 1 << 24) == kf::G3_BIG);\n"
+                   + "static_assert(kf::g3_km_pick(1 << 24, 300, true, 1 << 24, 300) == kf::G3_FLAT);\n")
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    for rows, ld in KM_REACH:
+        assert _last_byte(rows, ld) <= 0x7FFFFFF0 < _last_byte(rows, ld + 8)
 
 
 @pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
