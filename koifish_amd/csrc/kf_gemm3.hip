@@ -556,7 +556,7 @@ int gemm3_km_launch(hipStream_t st, const uint16_t* A, long long lda, bool akm, 
     const long nws = (long)((M + 127) / 128) * ((n + 127) / 128), rounds = (nws + 511) / 512;
     const bool small = 5 * nwg < 4 * 256 && akm && g3_km_reach<128>(lda) && (!bkm || g3_km_reach<128>(ldb)) && (20 * nws >= 17 * rounds * 512 || (ws && ws_bytes >= gemm3_sk_ws_bytes() && 5 * nws < 4 * 512));
     if (small) return bkm ? g3_go_c<true, true, G3Small>(st, a, nws, ws, ws_bytes, 1) : g3_go_c<true, false, G3Small>(st, a, nws, ws, ws_bytes, 1);
-    switch (akm ? g3_km_pick(M, n, bkm, lda, bkm ? ldb : 0) : G3_BIG) {
+    switch (akm ? g3_km_pick(M, n, K, bkm, lda, bkm ? ldb : 0) : G3_BIG) {
         case G3_SLIM: return bkm ? g3_whole<G3Slim, true, true>(st, a) : g3_whole<G3Slim, true, false>(st, a);
         case G3_FLAT: return bkm ? g3_whole<G3Flat, true, true>(st, a) : g3_whole<G3Flat, true, false>(st, a);
         default: break;

@@ -538,9 +538,12 @@ static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
 //   input gradients         1600 x 5120 rows, K 6400: 112 | 119 | 93 | 99, 1600 x 6000, K 1600: 37 | 37 | 29 | 53, 6400 x 3000, K 1600 (two rounds each) - | 75 | 59 | 61
 // One round more for four big ones gains at most 3 % (6400 x 8192, K 1600: - | 158 | 155 | 171) and is not taken.  Of both with as many rounds: us of weight gradients 75 | 72, of input gradients 92 | 97.
 // 160-row tiles of an operand whose rows are in their reach (ldw: of W, ldx: of x where it is k-major too, else 0); a row beyond it is 2^24 values and more, and the big tiles reach to 2^27.
-static constexpr G3Pick g3_km_pick(int M, int n, bool bkm, long long ldw, long long ldx) {
+// Up to K = 8192, the longest of these rows.  Behind it nothing was timed, and pieces gain there: their partial tiles cost the same at any K, while a round of 160 x 256 takes five eighths of a big tile's steps and 133 big
+// tiles in pieces 133 / 256 of them.  By the steps above the two are even at K = 8192 (119 | 118 us), and the input gradient of a 50304-wide head, 786 steps at 5120 rows, would take about 620 | 735.
+static constexpr int G3_KM_160_MAX_K = 8192;
+static constexpr G3Pick g3_km_pick(int M, int n, int K, bool bkm, long long ldw, long long ldx) {
     const long nb = (long)((M + 255) / 256) * ((n + 255) / 256), rb = (nb + 255) / 256, rs = ((long)((M + 159) / 160) * ((n + 255) / 256) + 255) / 256, rf = ((long)((M + 255) / 256) * ((n + 159) / 160) + 255) / 256;
-    if (nb <= 128 || (rs < rf ? rs : rf) > rb) return G3_BIG; /* (up to 128: two and more pieces of a tile, or tiles of 128 x 128) */
+    if (K > G3_KM_160_MAX_K || nb <= 128 || (rs < rf ? rs : rf) > rb) return G3_BIG; /* (up to 128: two and more pieces of a tile, or tiles of 128 x 128) */
     const G3Pick p = rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
     return g3_km_reach<160>(p == G3_SLIM ? ldw : ldx) ? p : G3_BIG;
 }

@@ -37,11 +37,15 @@ def test_one_round_of_tiles_is_taken_where_there_is_one(tmp_path):
 KM_PICKED = [(1600, 6400, True, "SLIM"), (6400, 1600, True, "FLAT"), (4096, 2560, True, "FLAT"), (3000, 3000, True, "FLAT"), (1600, 5120, False, "SLIM"), (6400, 3000, False, "SLIM"), (2048, 5120, False, "FLAT"),
              (1600, 8192, False, "BIG"), (6400, 8192, False, "BIG"), (4800, 5120, False, "BIG"), (2048, 4096, True, "BIG"), (2049, 4096, True, "FLAT"), (1608, 6400, True, "BIG")]
 
+# the same with K: up to the longest that was timed
+KM_PICKED_LONG = [(1600, 6400, 8192, True, "SLIM"), (1600, 4800, 8256, True, "BIG"), (3000, 3000, 16384, True, "BIG"), (1600, 5120, 8192, False, "SLIM"), (1600, 5120, 50304, False, "BIG"), (6400, 3000, 8256, False, "BIG")]
+
 
 @pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
 def test_tiles_of_160_are_taken_where_they_need_no_more_rounds(tmp_path):
     src = tmp_path / "rules.hip"
-    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_pick(%d, %d, %s, %d, %d) == kf::G3_%s);\n" % (m, n, str(b).lower(), m, n if b else 0, t) for m, n, b, t in KM_PICKED))
+    src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_pick(%d, %d, 1600, %s, %d, %d) == kf::G3_%s);\n" % (m, n, str(b).lower(), m, n if b else 0, t) for m, n, b, t in KM_PICKED)
+                   + "".join("static_assert(kf::g3_km_pick(%d, %d, %d, %s, %d, %d) == kf::G3_%s);\n" % (m, n, k, str(b).lower(), m, n if b else 0, t) for m, n, k, b, t in KM_PICKED_LONG))
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
 
@@ -67,8 +71,8 @@ def test_k_rows_are_in_reach_of_the_offsets_of_their_tile(tmp_path):
     """and a longer row than the 160-row tiles reach takes the big tiles: transposed it would be a product that the other kernels refuse (2^24 x 2048: 2^32 pieces of eight)"""
     src = tmp_path / "rules.hip"
     src.write_text('#include "%s/kf_gemm3_tile.h"\n' % B.CSRC + "".join("static_assert(kf::g3_km_reach<%d>(%d) && !kf::g3_km_reach<%d>(%d));\n" % (r, ld, r, ld + 8) for r, ld in KM_REACH)
-                   + "static_assert(kf::g3_km_pick(1600, 6400, true, 1600, 6400) == kf::G3_SLIM && kf::g3_km_pick(1600, 6400, true, 1 << 24, 6400) == kf::G3_BIG && kf::g3_km_pick(6400, 1600, true, 6400, 1 << 24) == kf::G3_BIG);\n"
-                   + "static_assert(kf::g3_km_pick(1 << 24, 300, true, 1 << 24, 300) == kf::G3_FLAT);\n")
+                   + "static_assert(kf::g3_km_pick(1600, 6400, 1600, true, 1600, 6400) == kf::G3_SLIM && kf::g3_km_pick(1600, 6400, 1600, true, 1 << 24, 6400) == kf::G3_BIG && kf::g3_km_pick(6400, 1600, 1600, true, 6400, 1 << 24) == kf::G3_BIG);\n"
+                   + "static_assert(kf::g3_km_pick(1 << 24, 300, 1600, true, 1 << 24, 300) == kf::G3_FLAT);\n")
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
     for rows, ld in KM_REACH:
