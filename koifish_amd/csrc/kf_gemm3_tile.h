@@ -547,9 +547,10 @@ static constexpr G3Pick g3_km_pick(int M, int n, int K, bool bkm, long long ldw,
     const G3Pick p = rs < rf || (rs == rf && !bkm) ? G3_SLIM : G3_FLAT;
     return g3_km_reach<160>(p == G3_SLIM ? ldw : ldx) ? p : G3_BIG;
 }
-// Where a launch of more than half a round may be cut in owners and tails (gemm3_sk_kernel, S = 1): k-steps.  The tails of 256 x 256 tiles are 256 KiB each, and up to K = 8192 they take what the idle CUs are worth
-// or more; us, cut | whole: 1600 x 6400 (175 tiles) from 8192 tokens 167 | 166, from 2560 80 | 62; 3000 x 3000 (144) from 4096 95 | 90; 2400 x 3600 (150) from 2048 63 | 52; 1600 x 5120, K 6400 (140) 112 | 119
-static constexpr int g3_tails_from(int bm) { return bm == 256 ? 129 : 32; }
+// Where a launch of more than half a round may be cut in owners and tails (gemm3_sk_kernel, S = 1): k-steps.  The tails of 256 x 256 tiles are 256 KiB each, about 50 us of writing and reading at any K; up to K = 4096 that is
+// what the idle CUs are worth or more.  us, cut | whole, tiles in brackets: from 2048 tokens 2400 x 3600 (150) 64 | 52, from 2560 1600 x 6400 (175) 80 | 62, from 4096 3000 x 3000 (144) 95 | 90, 3072 x 3072 (144) 89 | 88, 5120 x
+// 2048 (160) 94 | 91; K 6400, 1600 x 5120 (140) 112 | 119; from 8192 4096 x 2560 (160) 154 | 167, 2560 x 4096 149 | 161, 1600 x 6400 (175) 167 | 166, 1600 x 4800 (133) 119 | 118.  Between 4096 and 6400 nothing was timed: cut.
+static constexpr int g3_tails_from(int bm) { return bm == 256 ? 65 : 32; }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {
     const int q = nwg / 8, rr = nwg % 8, xcd = orig % 8;
