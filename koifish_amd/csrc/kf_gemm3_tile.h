@@ -538,8 +538,9 @@ static constexpr G3Pick g3_pick(int M, int n, int K, bool wide) {
 //   input gradients         1600 x 5120 rows, K 6400: 112 | 119 | 93 | 99, 1600 x 6000, K 1600: 37 | 37 | 29 | 53, 6400 x 3000, K 1600 (two rounds each) - | 75 | 59 | 61
 // One round more for four big ones gains at most 3 % (6400 x 8192, K 1600: - | 158 | 155 | 171) and is not taken.  Of both with as many rounds: us of weight gradients 75 | 72, of input gradients 92 | 97.
 // 160-row tiles of an operand whose rows are in their reach (ldw: of W, ldx: of x where it is k-major too, else 0); a row beyond it is 2^24 values and more, and the big tiles reach to 2^27.
-// Up to K = 8192, the longest of these rows.  Behind it nothing was timed, and pieces gain there: their partial tiles cost the same at any K, while a round of 160 x 256 takes five eighths of a big tile's steps and 133 big
-// tiles in pieces 133 / 256 of them.  By the steps above the two are even at K = 8192 (119 | 118 us), and the input gradient of a 50304-wide head, 786 steps at 5120 rows, would take about 620 | 735.
+// Up to K = 8192, the longest of these rows.  Behind it nothing was timed, and pieces gain there: their partial tiles cost the same at any K, and T big tiles then take T / 256 of a big tile's time where
+// 160 x 256 takes five eighths of it.  By the steps of the rows above 4096 x 2560 from 16384 tokens would be about 260 us in pieces and 290 whole (154 | 150 from 8192), the input gradient of a 50304-wide head at 5120
+// rows, 786 steps, about 560 and 700 (112 | 93 with 100).
 static constexpr int G3_KM_160_MAX_K = 8192;
 static constexpr G3Pick g3_km_pick(int M, int n, int K, bool bkm, long long ldw, long long ldx) {
     const long nb = (long)((M + 255) / 256) * ((n + 255) / 256), rb = (nb + 255) / 256, rs = ((long)((M + 159) / 160) * ((n + 255) / 256) + 255) / 256, rf = ((long)((M + 255) / 256) * ((n + 159) / 160) + 255) / 256;
@@ -549,7 +550,7 @@ static constexpr G3Pick g3_km_pick(int M, int n, int K, bool bkm, long long ldw,
 }
 // Where a launch of more than half a round may be cut in owners and tails (gemm3_sk_kernel, S = 1): k-steps.  The tails of 256 x 256 tiles are 256 KiB each, about 50 us of writing and reading at any K; up to K = 4096 that is
 // what the idle CUs are worth or more.  us, cut | whole, tiles in brackets: from 2048 tokens 2400 x 3600 (150) 64 | 52, from 2560 1600 x 6400 (175) 80 | 62, from 4096 3000 x 3000 (144) 95 | 90, 3072 x 3072 (144) 89 | 88, 5120 x
-// 2048 (160) 94 | 91; K 6400, 1600 x 5120 (140) 112 | 119; from 8192 4096 x 2560 (160) 154 | 167, 2560 x 4096 149 | 161, 1600 x 6400 (175) 167 | 166, 1600 x 4800 (133) 119 | 118.  Between 4096 and 6400 nothing was timed: cut.
+// 2048 (160) 94 | 91; K 6400, 1600 x 5120 (140) 112 | 119; from 8192 4096 x 2560 (160) 154 | 167, 2560 x 4096 149 | 161, 1600 x 6400 (175) 167 | 166.  Between 4096 and 6400 nothing was timed: cut.
 static constexpr int g3_tails_from(int bm) { return bm == 256 ? 65 : 32; }
 // workgroup number -> tile number: workgroups go to the 8 XCDs round robin, so the tiles an XCD runs back to back are made neighbours
 __device__ __forceinline__ int g3_remap(int orig, int nwg) {

@@ -38,7 +38,7 @@ KM_PICKED = [(1600, 6400, True, "SLIM"), (6400, 1600, True, "FLAT"), (4096, 2560
              (1600, 8192, False, "BIG"), (6400, 8192, False, "BIG"), (4800, 5120, False, "BIG"), (2048, 4096, True, "BIG"), (2049, 4096, True, "FLAT"), (1608, 6400, True, "BIG")]
 
 # the same with K: up to the longest that was timed
-KM_PICKED_LONG = [(1600, 6400, 8192, True, "SLIM"), (1600, 4800, 8256, True, "BIG"), (3000, 3000, 16384, True, "BIG"), (1600, 5120, 8192, False, "SLIM"), (1600, 5120, 50304, False, "BIG"), (6400, 3000, 8256, False, "BIG")]
+KM_PICKED_LONG = [(1600, 6400, 8192, True, "SLIM"), (4096, 2560, 8256, True, "BIG"), (3000, 3000, 16384, True, "BIG"), (1600, 5120, 8192, False, "SLIM"), (1600, 5120, 50304, False, "BIG"), (6400, 3000, 8256, False, "BIG")]
 
 
 @pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
@@ -81,7 +81,7 @@ def test_k_rows_are_in_reach_of_the_offsets_of_their_tile(tmp_path):
 
 # (big tiles of the launch, K, us cut in owners and tails, us whole)
 TAILS = [(150, 2048, 63.6, 52.0), (150, 2048, 64.4, 53.1), (175, 2560, 80.1, 61.9), (144, 4096, 95.3, 90.0), (144, 4096, 88.6, 88.3), (160, 4096, 94.6, 90.8), (160, 4096, 93.3, 92.3), (140, 6400, 112.1, 119.1),
-         (160, 8192, 154.7, 167.7), (160, 8192, 149.6, 161.1), (175, 8192, 167.0, 166.2), (133, 8192, 119.6, 118.5)]
+         (160, 8192, 154.7, 167.7), (160, 8192, 149.6, 161.1), (175, 8192, 167.0, 166.2)]
 
 
 @pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
@@ -89,6 +89,7 @@ def test_tails_of_big_tiles_are_cut_off_where_that_was_the_faster(tmp_path):
     """within 1.5 %, what two runs of one side differ by"""
     src = tmp_path / "rules.hip"
     src.write_text('#include "%s/kf_gemm3_tile.h"\nstatic_assert(kf::g3_tails_from(128) == 2048 / 64);\n' % B.CSRC
+                   + "static_assert(kf::g3_km_pick(1608, 6400, 4160, true, 1608, 6400) == kf::G3_BIG && 4160 / 64 >= kf::g3_tails_from(256));\n"   # the GPU test of repeated runs has this shape for its tails
                    + "".join("static_assert(%d / 64 %s kf::g3_tails_from(256));\n" % (k, ">=" if cut < whole else "<") for _, k, cut, whole in TAILS if abs(cut - whole) > 0.015 * whole))
     r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
