@@ -744,19 +744,21 @@ static void gm_direct(const GemmArgs& a, dim3 grid, hipStream_t st) {
     }
     if constexpr (TB == 1) hipLaunchKernelGGL((gemm_direct_kernel<FMT, TB, GD_UPG, GD_NW, PAIRED, false>), grid, dim3(GD_NW * 64), sums, st, a, 0);
 }
-// 64 token rows a workgroup: every weight is unpacked for twice as many, but a workgroup has a CU to itself.  Taken where the rounds that the launch takes of such workgroups are the shorter: 1.4 a round, against 1.8 for a
+// 64 token rows a workgroup: every weight is unpacked for twice as many, but a workgroup has a CU to itself.  In 4 bits taken where the rounds that the launch takes of such workgroups are the shorter: 1.4 a round, against 1.8 for a
 // round of 512 of the others, two to a CU, and 1 for a last one of at most 256.  us a prompt, 32 | 64 where the rule takes them: o and down, 0.6B 319 rows 2732 | 2592, 1.7B 192 rows 3949 | 3736, 256 rows 4270 | 4020, six layers
 // of the 32B shape at 256 rows 4640 | 4370; gate | up, 0.6B 128 rows 1718 | 1667, 1.7B 256 rows 4270 | 4057, 32B 64 rows 2446 | 2340; where it does not: 0.6B 256 rows 2162 | 2217, 1.7B 128 rows 2765 | 2785, 2765 | 2984
-static bool gd_wide(const GemmArgs& a, long row_blocks) {
-    const long one = row_blocks * ((a.n + 31) / 32), two = row_blocks * ((a.n + 63) / 64), last = one % 512;
-    return a.n > 32 && a.ldx < (1 << 24) && 14 * ((two + 255) / 256) < 18 * (one / 512) + (last == 0 ? 0 : last <= 256 ? 10 : 18);
+// The other storages' rounds were not timed: only several matrices in a launch go by 64 there, from one workgroup for every CU on.
+static constexpr bool gd_wide(int fmt, int njobs, int n, long row_blocks) {
+    const long one = row_blocks * ((n + 31) / 32), two = row_blocks * ((n + 63) / 64), last = one % 512;
+    if (fmt != FMT_Q4) return njobs > 1 && n >= 64 && two >= 256;
+    return n > 32 && 14 * ((two + 255) / 256) < 18 * (one / 512) + (last == 0 ? 0 : last <= 256 ? 10 : 18);
 }
 template <int FMT>
 static void gm_launch(const GemmArgs& a, int KS, dim3 grid, size_t smem, hipStream_t st) {
-    const bool wide = KS <= 0 && gd_wide(a, grid.x);
+    const bool wide = KS <= 0 && a.ldx < (1 << 24) && gd_wide(FMT, a.njobs, a.n, grid.x);
     const dim3 half(grid.x, (a.n + 63) / 64);
     if (KS == 0) wide ? gm_direct<FMT, 2, false>(a, half, st) : gm_direct<FMT, 1, false>(a, grid, st);
-    else if (KS == -1) wide && FMT == FMT_Q4 ? gm_direct<FMT == FMT_Q4 ? FMT : FMT_BF16, 2, FMT == FMT_Q4>(a, half, st) : gm_direct<FMT, 1, true>(a, grid, st); /* paired SwiGLU */
+    else if (KS == -1) wide ? gm_direct<FMT == FMT_Q4 ? FMT : FMT_BF16, 2, FMT == FMT_Q4>(a, half, st) : gm_direct<FMT, 1, true>(a, grid, st); /* paired SwiGLU (one job: by 64 in 4 bits only) */
     else if (KS == 2)
         hipLaunchKernelGGL((gemm_kernel<FMT, 2>), grid, dim3(256), smem, st, a);
     else

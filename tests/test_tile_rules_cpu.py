@@ -95,6 +95,19 @@ def test_tails_of_big_tiles_are_cut_off_where_that_was_the_faster(tmp_path):
     assert r.returncode == 0, r.stderr[-3000:]
 
 
+# (storage, matrices in the launch, token rows, blocks of 32 weight rows, 64 token rows a workgroup): 4 bits as timed in prompts; the others, whose rounds were not timed, only several matrices from 256 such workgroups on
+WIDE = [("Q4", 1, 128, 96, True), ("Q4", 1, 256, 96, False), ("Q4", 1, 256, 64, True), ("Q4", 3, 64, 256, True), ("Q4", 1, 32, 1280, False)] + \
+       [(f, *c) for f in ("BF16", "F8", "Q4R", "Q2", "Q1") for c in ((1, 64, 132, False), (1, 256, 160, False), (3, 192, 128, True), (3, 64, 256, True), (3, 63, 512, False), (2, 64, 255, False))]
+
+
+@pytest.mark.skipif(not shutil.which(B.HIPCC), reason="no hipcc")
+def test_64_token_rows_a_workgroup_where_that_was_timed(tmp_path):
+    src = tmp_path / "rules.hip"
+    src.write_text('#include "%s/kf_gemm.hip"\n' % B.CSRC + "".join("static_assert(kf::gd_wide(kf::FMT_%s, %d, %d, %d) == %s);\n" % (f, j, n, rb, str(w).lower()) for f, j, n, rb, w in WIDE))
+    r = subprocess.run([B.HIPCC, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-w", str(src)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+
 # (pieces of 8 weights, matrices interleaved, offsets of the copy in 32 bits): gate and up of 65552 x 16384 lie in 4 296 015 872 bytes
 REACH = [(65552 * 16384 // 8, 1, True), (65552 * 16384 // 8, 2, False), (65536 * 16384 // 8 - 1, 2, True), ((1 << 28) - 1, 1, True), (1 << 28, 1, False), ((1 << 31) - 1, 2, False)]
 
