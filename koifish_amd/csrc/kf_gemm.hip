@@ -433,11 +433,11 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
     // the table: 24 rows 1475 | 1438, 128 rows 1786 | 1760, 319 rows 3032 | 2964
     constexpr bool TABLE = FMT == FMT_Q4 && !PAIRED && XL;
     const bool one_table = a.gshift >= 2 && (a.nBlk & 3) == 0;
-    [[maybe_unused]] PermLut lut, lut2;
-    auto wfrag = [&](const WTile<FMT, 2>& w, [[maybe_unused]] PermLut& t, const GemmArgs& m, int j, int sl, int ks) {
+    [[maybe_unused]] PermLut lut;
+    auto wfrag = [&](const WTile<FMT, 2>& w, const GemmArgs& m, int j, int sl, int ks) {
         if constexpr (TABLE) {
-            if (sl == 0 && (j == 0 || !one_table)) w.table(t, m);
-            return w.frag_t(sl, t);
+            if (sl == 0 && (j == 0 || !one_table)) w.table(lut, m);
+            return w.frag_t(sl, lut);
         } else
             return get_frag<FMT, 2>(w, sl, m, ks);
     };
@@ -462,7 +462,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
         const bool more = u0 + NW * UPG < nunit;
         if (more) gload(u0 + NW * UPG, gn, XL && slots == 1 ? 0 : slot ^ 1, !XL || slots == 2);
         if constexpr (XL) { /* a weight of the group has come: its token rows have */
-            if (slots == 1 && u0 >= NW * UPG) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* (these set out behind it) */
+            if (slots == 1 && u0 >= NW * UPG) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* (the token rows set out behind it; the next group's weights, asked for a moment ago, are waited for as well) */
             else asm volatile("" ::"v"(gm_first(gc.w[0].b)) : "memory");
         }
 #pragma unroll
@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
             if (u0 + j < nunit) {
 #pragma unroll
                 for (int sl = 0; sl < 4; sl++) {
-                    const bf16x8 A = __builtin_bit_cast(bf16x8, wfrag(gc.w[j], lut, a, j, sl, (u0 + j) & 1));
+                    const bf16x8 A = __builtin_bit_cast(bf16x8, wfrag(gc.w[j], a, j, sl, (u0 + j) & 1));
                     u32x4 X[TB];
 #pragma unroll
                     for (int tb = 0; tb < TB; tb++) X[tb] = xfrag(gc, slot, j, sl, tb);
@@ -478,7 +478,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
                     for (int tb = 0; tb < TB; tb++)
                         acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, __builtin_bit_cast(bf16x8, X[tb]), acc[tb], 0, 0, 0);
                     if (PAIRED) {
-                        const bf16x8 A2 = __builtin_bit_cast(bf16x8, wfrag(gc.w2[j], lut2, b, j, sl, (u0 + j) & 1));
+                        const bf16x8 A2 = __builtin_bit_cast(bf16x8, wfrag(gc.w2[j], b, j, sl, (u0 + j) & 1));
 #pragma unroll
                         for (int tb = 0; tb < TB; tb++)
                             acc2[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A2, __builtin_bit_cast(bf16x8, X[tb]), acc2[tb], 0, 0, 0);
@@ -554,7 +554,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_direct_kernel(const GemmArgs a0,
 }
 
 // The same for 4-bit matrices of which blocks of 32 rows are too few workgroups: 16 rows a workgroup, twice as many of them, each with half of the unpacking.  v_mfma_f32_16x16x32_bf16 adds up a step's 32 products as
-// two v_mfma_f32_32x32x16_bf16 do one behind the other (the same bits, compared over 10^8 sums), so lane group q holds what lane half q & 1 holds there in step 2 m + (q >> 1).
+// two v_mfma_f32_32x32x16_bf16 do one behind the other (the same bits over 10^8 sums of normally distributed values; infinities and sums in the subnormal range were not compared), so lane group q holds what lane half q & 1 holds there in step 2 m + (q >> 1).
 template <int TB, bool PAIRED>
 __global__ void __launch_bounds__(512) gemm_direct16_kernel(const GemmArgs a0, int slots) {
     constexpr int NW = 8, UPG = 2, XG = TB * 16 * 256;

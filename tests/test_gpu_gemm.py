@@ -491,8 +491,8 @@ def test_rows_of_small_batches_do_not_depend_on_their_way(ctx, kind, M, K):
 @pytest.mark.parametrize("group", [32, 64, 128])
 @pytest.mark.parametrize("M,K", [(4160, 128), (4130, 192), (4129, 1600), (4192, 2048), (33, 1600), (34, 192)])
 def test_tables_of_4_bit_groups_and_the_residual_of_a_small_batch(ctx, M, K, group):
-    """groups of one, two and four blocks, rows whose groups begin in the row before, odd and even rows (the last two: blocks of 16 rows): 20 rows by way of LDS (weights from tables, the residual loaded early where rows pair) equal 16 read as
-    fragments (arithmetic) bit for bit, and the product in 32 bits to a bf16 rounding of the sum and one of the residual's"""
+    """groups of one, two and four blocks, rows whose groups begin in the row before, odd and even rows: 20 rows by way of LDS (weights from tables, the residual loaded early where rows pair) equal 16 read as
+    fragments (arithmetic) bit for bit, and the product in 32 bits to a bf16 rounding of the sum and one of the residual's.  The last two shapes go in blocks of 16 rows at 16 and at 20 rows, so there only the second says something"""
     if M * K % group:
         pytest.skip("whole groups only")
     w = ctx.quantize((torch.randn(M, K, device=ctx.device) * 0.05).bfloat16(), L.Q4, lGroup=group)
@@ -538,6 +538,25 @@ def test_blocks_of_16_and_of_32_weight_rows_give_the_same_bits(ctx, n, M, K):
         assert torch.equal(t.view(torch.int16), y[tall][0][:, :t.shape[1]].contiguous().view(torch.int16))
 
 
+@pytest.mark.parametrize("n,M,K", [(16, 2048, 1024), (33, 1024, 2048), (50, 2048, 192)])
+def test_blocks_of_16_and_of_32_weight_rows_add_up_values_that_cancel_alike(ctx, n, M, K):
+    """the two matrix instructions on products 2^48 apart, an eighth of which cancel but for a part in 128 of them: which products meet before a rounding decides the last bits there"""
+    g = torch.Generator(device=ctx.device).manual_seed(n + K)
+    e = torch.randint(-24, 25, (n, K), device=ctx.device, generator=g).float()
+    x = (torch.randn(n, K, device=ctx.device, generator=g) * torch.exp2(e)).bfloat16()
+    x[:, 1::16] = (-x[:, 0::16].float() * (1 + 2.0 ** -7)).bfloat16()
+    W = (torch.randn(4160, K, device=ctx.device, generator=g) * 0.05).bfloat16()
+    W[:, 1::16] = W[:, 0::16]
+    y = {}
+    for rows in (4160, M):
+        w = ctx.quantize(W[:rows].contiguous(), L.Q4)
+        d, y[rows] = w.desc(), torch.zeros(n, rows, device=ctx.device, dtype=torch.bfloat16)
+        assert ctx.hip.kf_linear(ctx.h, C.byref(d), x.data_ptr(), y[rows].data_ptr(), None, n, 1.0, 0.0, 0, None) == 0, ctx.hip.kf_last_error()
+    ctx.sync()
+    assert bool(torch.isfinite(y[M].float()).all()) and float(y[M].float().abs().max()) > 0
+    assert torch.equal(y[4160][:, :M].contiguous().view(torch.int16), y[M].view(torch.int16))
+
+
 @pytest.mark.parametrize("kind,K", [(k, K) for k in (L.BF16, L.F8E5M2, L.Q4, L.T_SIGN, L.BOOL1) for K in (1152, 1600, 2048, 3072) if K != 1600 or k in (L.BF16, L.F8E5M2, L.Q4)])
 @pytest.mark.parametrize("n", [33, 64])
 def test_rows_with_one_and_two_slots_of_lds_give_the_same_bits(ctx, kind, K, n):
@@ -555,6 +574,17 @@ def test_rows_with_one_and_two_slots_of_lds_give_the_same_bits(ctx, kind, K, n):
         assert torch.equal(y[M][:, :4096].contiguous().view(torch.int16), y[4096].view(torch.int16))
     ref = x.float() @ ctx.dequant(w).float().reshape(4096, K).t()
     assert float((y[4096].float() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+    if kind == L.Q4:   # gate | up in the same three forms
+        U, act = (torch.randn(9216, K, device=ctx.device, generator=g) * 0.05).bfloat16(), {}
+        for M in (9216, 4224, 4096):
+            ws = [ctx.quantize(m[:M].contiguous(), kind) for m in (W, U)]
+            d, up = [w.desc() for w in ws], torch.zeros(n, M, device=ctx.device, dtype=torch.bfloat16)
+            act[M] = torch.zeros_like(up)
+            assert ctx.hip.kf_gateup_swiglu_batch(ctx.h, C.byref(d[0]), C.byref(d[1]), x.data_ptr(), act[M].data_ptr(), up.data_ptr(), n) == 0, ctx.hip.kf_last_error()
+            ctx.sync()
+        assert float(act[4096].float().abs().max()) > 0
+        for M in (9216, 4224):
+            assert torch.equal(act[M][:, :4096].contiguous().view(torch.int16), act[4096].view(torch.int16))
     if K % 128:
         return
     rows = (4096, 2048, 2048)   # 512 blocks of 32 rows and tokens

@@ -96,7 +96,7 @@ def test_tails_of_big_tiles_are_cut_off_where_that_was_the_faster(tmp_path):
 
 
 # (storage, matrices in the launch, token rows, blocks of 32 weight rows, 64 token rows a workgroup): 4 bits as timed in prompts; the others, whose rounds were not timed, only several matrices from 256 such workgroups on
-WIDE = [("Q4", 1, 128, 96, True), ("Q4", 1, 256, 96, False), ("Q4", 1, 256, 64, True), ("Q4", 3, 64, 256, True), ("Q4", 1, 32, 1280, False)] + \
+WIDE = [("Q4", 1, 128, 96, True), ("Q4", 1, 256, 96, False), ("Q4", 1, 256, 64, True), ("Q4", 3, 64, 256, True), ("Q4", 1, 32, 1280, False), ("Q4", 1, 33, 132, True), ("Q4", 1, 64, 132, True), ("Q4", 1, 64, 128, False), ("Q4", 1, 64, 288, False)] + \
        [(f, *c) for f in ("BF16", "F8", "Q4R", "Q2", "Q1") for c in ((1, 64, 132, False), (1, 256, 160, False), (3, 192, 128, True), (3, 64, 256, True), (3, 63, 512, False), (2, 64, 255, False))]
 
 
